@@ -17,5 +17,7 @@ def load():
         raise RuntimeError(
             "pypto_amd: the native HIP extension is not built or not loadable "
             f"({exc}); build it in-tree with `python -m pypto_amd.build`") from exc
+    from .converter import Tensor
+    mod.set_wrapper(Tensor, "_t")
     _C = mod
     return _C

@@ -47,11 +47,20 @@ def build_library(verbose: bool = False) -> str:
 
 def build_extension(verbose: bool = False) -> str:
     import pybind11
+    import torch
     cxx = os.environ.get("CXX", "g++")
-    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+    torch_dir = os.path.dirname(os.path.abspath(torch.__file__))
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    # torch_calls.cpp reads torch tensors directly; torch's libraries are in the process before this module is loaded
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
            "-I" + INCLUDE, "-I" + pybind11.get_include(), "-I" + sysconfig.get_paths()["include"],
-           os.path.join(CSRC, "pybind.cpp"), "-o", EXT_PATH,
-           "-L" + HERE, "-l:" + LIB_NAME, "-Wl,-rpath,$ORIGIN"]
+           "-isystem", os.path.join(torch_dir, "include"),
+           "-isystem", os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
+           "-isystem", os.path.join(rocm, "include"),
+           os.path.join(CSRC, "pybind.cpp"), os.path.join(CSRC, "torch_calls.cpp"), "-o", EXT_PATH,
+           "-L" + HERE, "-l:" + LIB_NAME, "-Wl,-rpath,$ORIGIN",
+           "-L" + os.path.join(torch_dir, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
     out = _run(cmd)
     if verbose and out:
         print(out)

@@ -1,6 +1,7 @@
 // pybind11 face of the C ABI.  Tensors cross as raw device addresses (torch's data_ptr()) and the
 // HIP stream as an integer handle; no torch types appear here.  Argument errors raise ValueError,
-// everything else RuntimeError, carrying the library's own message.
+// everything else RuntimeError, carrying the library's own message.  The calls that take torch tensors
+// themselves, which the operators try first, are in torch_calls.cpp.
 #include <pybind11/pybind11.h>
 #include <pybind11/stl.h>
 
@@ -12,6 +13,7 @@
 #include <string>
 
 #include "pypto_amd_sfa.h"
+#include "torch_calls.h"
 
 namespace py = pybind11;
 
@@ -99,6 +101,7 @@ PYBIND11_MODULE(_C, m)
     m.attr("DT_FP16") = PTO_DT_FP16;
     m.attr("DT_FP32") = PTO_DT_FP32;
     m.attr("DT_BF16") = PTO_DT_BF16;
+    if (pto::add_torch_calls(m.ptr()) != 0) throw py::error_already_set();
     m.def("version", []() { return std::string(pto_version()); });
 
     m.def("sfa_quant_workspace_bytes",

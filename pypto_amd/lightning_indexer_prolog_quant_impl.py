@@ -116,6 +116,11 @@ def lightning_indexer_prolog_quant(x_in, q_norm_in, q_norm_scale_in, w_qb_in, w_
     attrs = attrs if attrs is not None else IndexerPrologQuantAttr()
     if getattr(attrs, "layerout_query", "TND") != "TND" or getattr(attrs, "layerout_key", "PA_BSND") != "PA_BSND":
         raise ValueError("lightning_indexer_prolog_quant: only layerout_query='TND' and layerout_key='PA_BSND' exist")
+    if _collect is None and C.li_prolog_call(
+            x_in, q_norm_in, q_norm_scale_in, w_qb_in, w_qb_scale_in, wk_in, w_proj_in, ln_gamma_k_in, ln_beta_k_in,
+            cos_idx_rope_in, sin_idx_rope_in, hadamard_q_in, hadamard_k_in, k_int8_in, k_scale_in, k_cache_index_in,
+            q_int8_out, q_scale_out, k_int8_out, k_scale_out, weights_out, attrs.eps, _sum_mode()):
+        return None
     names = ("x_in", "q_norm_in", "q_norm_scale_in", "w_qb_in", "w_qb_scale_in", "wk_in", "w_proj_in", "ln_gamma_k_in",
              "ln_beta_k_in", "cos_idx_rope_in", "sin_idx_rope_in", "hadamard_q_in", "hadamard_k_in", "k_int8_in",
              "k_scale_in", "k_cache_index_in", "q_int8_out", "q_scale_out", "k_int8_out", "k_scale_out", "weights_out")

@@ -53,6 +53,10 @@ def lightning_indexer_decode(idx_query, idx_query_scale, idx_key_cache, idx_key_
     q_scale, times k_scale (both products rounded to fp16), ReLU, times weight in fp16, fp32 head sum.  It takes
     fp16 scales and weights only."""
     C = _native.load()
+    if arith_variant in ("scaled_sum", "fp16_dequant") and C.li_decode_call(
+            idx_query, idx_query_scale, idx_key_cache, idx_key_scale, idx_weight, act_seq_key, block_table, topk_res,
+            selected_count, 1 if arith_variant == "fp16_dequant" else 0, MAX_LI_S1, MAX_LI_S2):
+        return None
     q = as_torch(idx_query, "idx_query")
     qs = as_torch(idx_query_scale, "idx_query_scale")
     kc = as_torch(idx_key_cache, "idx_key_cache")

@@ -14,6 +14,8 @@ from __future__ import annotations
 import torch
 
 from . import _native
+from . import lightning_indexer_prolog_quant_impl as _lip
+from . import mla_prolog_quant_impl as _mla
 from .converter import as_torch
 from .lightning_indexer_prolog_quant_impl import lightning_indexer_prolog_quant
 from .mla_prolog_quant_impl import mla_prolog_quant_d, mla_prolog_quant_p
@@ -67,11 +69,25 @@ def _fused(mla_op, token_x, mla_w_dq, mla_w_uq_qr, mla_dequant_scale, mla_w_uk, 
     return None
 
 
+def _native_call(args, kwargs) -> bool:
+    """The call as it usually comes -- 41 positional arguments, the caches updated in place -- in one native call."""
+    if kwargs or len(args) != 41 or args[36] not in ("PA_BSND", "PA_NZ"):
+        return False
+    attrs = args[38] if args[38] is not None else _lip.IndexerPrologQuantAttr()
+    if getattr(attrs, "layerout_query", "TND") != "TND" or getattr(attrs, "layerout_key", "PA_BSND") != "PA_BSND":
+        return False
+    return _native.load().fused_prolog_call(*args[:36], bool(_mla.EXACT_ABSORB), attrs.eps, _lip._sum_mode())
+
+
 def mla_indexer_prolog_quant_d(*args, **kwargs):
     """Decode entry point (reference :141-256); 41 positional arguments in the reference's order."""
+    if _native_call(args, kwargs):
+        return None
     return _fused(mla_prolog_quant_d, *args, **kwargs)
 
 
 def mla_indexer_prolog_quant_p(*args, **kwargs):
     """Prefill entry point (reference :49-138); the same kernels."""
+    if _native_call(args, kwargs):
+        return None
     return _fused(mla_prolog_quant_p, *args, **kwargs)

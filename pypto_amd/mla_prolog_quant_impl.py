@@ -103,6 +103,11 @@ def _mla_prolog_quant(token_x, w_dq, w_uq_qr, dequant_scale, w_uk, w_dkv_kr, gam
         raise ValueError(f"mla_prolog_quant: cache_mode must be 'PA_BSND' or 'PA_NZ', got {cache_mode!r}")
     if dequant_scale is None:
         raise ValueError("mla_prolog_quant: dequant_scale is None (the non-quantized w_uq_qr variant is not built)")
+    if _collect is None and C.mla_prolog_call(
+            token_x, w_dq, w_uq_qr, dequant_scale, w_uk, w_dkv_kr, gamma_cq, gamma_ckv, cos, sin, cache_index, kv_cache,
+            kr_cache, k_scale_cache, q_norm_out, q_norm_scale_out, query_nope_out, query_rope_out, kv_cache_out, kr_cache_out,
+            k_scale_cache_out, epsilon_cq, epsilon_ckv, bool(EXACT_ABSORB)):
+        return None
     names = ("token_x", "w_dq", "w_uq_qr", "dequant_scale", "w_uk", "w_dkv_kr", "gamma_cq", "gamma_ckv", "cos", "sin",
              "cache_index", "kv_cache", "kr_cache", "k_scale_cache", "q_norm_out", "q_norm_scale_out", "query_nope_out",
              "query_rope_out", "kv_cache_out", "kr_cache_out", "k_scale_cache_out")

@@ -89,6 +89,9 @@ def sparse_attention_antiquant_d(query_nope, query_rope, nope_cache, topk_indice
     topk_indices (t, n_kv*topk) int32; block_table (b, max_blocknum_perbatch) int32; kv_act_seqs (b,) int32;
     attention_out (b, s, n_q, 512) bf16, written in place.
     """
+    if _native.load().sa_antiquant_call(query_nope, query_rope, nope_cache, topk_indices, block_table, kv_act_seqs,
+                                        attention_out, nq, n_kv, softmax_scale, topk, block_size, max_blocknum_perbatch):
+        return None
     return _launch(query_nope, query_rope, nope_cache, topk_indices, block_table, kv_act_seqs, attention_out, nq, n_kv,
                    softmax_scale, topk, block_size, max_blocknum_perbatch)
 
@@ -98,5 +101,8 @@ def sparse_attention_antiquant_p(query_nope, query_rope, nope_cache, topk_indice
                                  nq, n_kv, softmax_scale, topk, block_size,
                                  max_blocknum_perbatch, tile_config=None):
     """Prefill entry point (:322-359); same computation and arguments as the decode one."""
+    if _native.load().sa_antiquant_call(query_nope, query_rope, nope_cache, topk_indices, block_table, kv_act_seqs,
+                                        attention_out, nq, n_kv, softmax_scale, topk, block_size, max_blocknum_perbatch):
+        return None
     return _launch(query_nope, query_rope, nope_cache, topk_indices, block_table, kv_act_seqs, attention_out, nq, n_kv,
                    softmax_scale, topk, block_size, max_blocknum_perbatch)

@@ -10,7 +10,8 @@ returns ``None`` and runs asynchronously on the current stream.
 
 What changes underneath: instead of tracing a tile graph and compiling it for an NPU, the call
 validates the arguments and launches the hand-written gfx950 kernels through the C ABI
-(include/pypto_amd_sfa.h).  ``tile_config`` carries NPU tiling hints and is accepted and ignored.
+(include/pypto_amd_sfa.h): in one native call (csrc/torch_calls.cpp) where the arguments are as they should
+be, and through the checks below, which name what is wrong, where they are not.  ``tile_config`` carries NPU tiling hints and is accepted and ignored.
 """
 from __future__ import annotations
 
@@ -122,6 +123,9 @@ def sparse_flash_attention_quant_d(query_nope, query_rope, key_nope_2d, key_rope
     topk_indices (t, n_kv*topk) int32; block_table (b, max_blocknum_perbatch) int32; kv_act_seqs (b,)
     int32; attention_out (b, s, n_q, 512) bf16, written in place.
     """
+    if _native.load().sfa_call(query_nope, query_rope, key_nope_2d, key_rope_2d, k_nope_scales, topk_indices, block_table,
+                               kv_act_seqs, attention_out, nq, n_kv, softmax_scale, topk, block_size, max_blocknum_perbatch):
+        return None
     return _launch(query_nope, query_rope, key_nope_2d, key_rope_2d, k_nope_scales, topk_indices, block_table,
                    kv_act_seqs, attention_out, nq, n_kv, softmax_scale, topk, block_size, max_blocknum_perbatch)
 
@@ -131,5 +135,8 @@ def sparse_flash_attention_quant_p(query_nope, query_rope, key_nope_2d, key_rope
                                    attention_out, nq, n_kv, softmax_scale, topk,
                                    block_size, max_blocknum_perbatch, tile_config=None):
     """Prefill entry point (:499-538); same computation and arguments as the decode one."""
+    if _native.load().sfa_call(query_nope, query_rope, key_nope_2d, key_rope_2d, k_nope_scales, topk_indices, block_table,
+                               kv_act_seqs, attention_out, nq, n_kv, softmax_scale, topk, block_size, max_blocknum_perbatch):
+        return None
     return _launch(query_nope, query_rope, key_nope_2d, key_rope_2d, k_nope_scales, topk_indices, block_table,
                    kv_act_seqs, attention_out, nq, n_kv, softmax_scale, topk, block_size, max_blocknum_perbatch)
