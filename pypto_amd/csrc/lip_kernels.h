@@ -42,7 +42,7 @@ struct LipParams {
     float eps, w_mul0, w_mul1;   // weights = fp16((bf16(x.w_proj) * w_mul0) * w_mul1)
     int sum_mode;                // LIP_SUMS_*
     int x_in_groups;             // 1: xpart already holds one row per group of eight blocks, left there by another
-                                 // operator's launch (the fused prolog at decode sizes); set by that launcher only
+                                 // operator's launch (the fused prolog); set by that launcher only
 };
 
 // How the fp32 sums are taken from LIP_MFMA_MIN_TOKENS tokens on (below that every sum has its fixed order):
@@ -63,11 +63,15 @@ __host__ __device__ inline bool lip_x_on_matrix_cores(const LipParams &p)
 }
 // the fixed-order sums over the hidden axis at prefill sizes leave one row per group of eight blocks (the group sums)
 // instead of one per block; the staging of that form needs w_proj rows of a power of two of 16-byte pieces
-__host__ __device__ inline bool lip_x_group_rows(const LipParams &p)
+__host__ __device__ inline bool lip_x_group_width(const LipParams &p)
 {
     const int wb = p.n_heads * 2;
+    return wb >= 16 && (wb & (wb - 1)) == 0;
+}
+__host__ __device__ inline bool lip_x_group_rows(const LipParams &p)
+{
     if (p.x_in_groups) return true;
-    return p.T >= LIP_MFMA_MIN_TOKENS && !lip_x_on_matrix_cores(p) && wb >= 16 && (wb & (wb - 1)) == 0;
+    return p.T >= LIP_MFMA_MIN_TOKENS && !lip_x_on_matrix_cores(p) && lip_x_group_width(p);
 }
 // partial rows [T, LIP_XCOLS] the first launch leaves per token: the blocks of 64 of the fixed-order form, or the
 // ranges of the matrix-core form (enough of them for about 512 workgroups of 128 tokens x 128 columns: two per compute unit)

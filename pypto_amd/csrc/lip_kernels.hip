@@ -12,8 +12,8 @@
 // The orders used here: sums over the hidden axis are cut into blocks of 64 (a block ascending from
 // 0.0), eight consecutive block sums are added ascending into a group sum, group sums are added
 // ascending; the Hadamard sums run over i ascending; the two layer-norm means
-// are balanced binary trees over neighbouring channels.  No matrix-core instruction touches these
-// sums (its internal order is not specified); only the exact integer projection uses one.
+// are balanced binary trees over neighbouring channels.  No matrix-core instruction that adds more than
+// one product touches these sums (its internal order is not specified).
 //
 // Two launches; below LIP_MFMA_MIN_TOKENS tokens (decode):
 //   lip_linear_kernel   workgroups of four independent waves.  Two of them share a query job (head,
@@ -33,8 +33,8 @@
 // which sums may leave their fixed order):
 //   lip_qproj_prefill_kernel, lip_qproj_prefill256_kernel   the query projection unsplit (prolog_common.h), a
 //                       workgroup per 128 x 128 or 256 x 256 tile over the whole reduction axis; exact.
-//   lip_xlinear_group_kernel   the fixed-order sums over the hidden axis, a group of eight blocks per workgroup and 16
-//                       tokens per weight block, hidden states broadcast by DPP (xlinear_fixed.h); or
+//   lip_xlinear_group_kernel   the fixed-order sums over the hidden axis on the matrix cores, one hidden row per
+//                       instruction (xlinear_fixed.h); or
 //   lip_xlinear_mfma_kernel    the same sums on the matrix cores (xlinear_mfma.h), if asked for.
 //   lip_finish_query_prefill_kernel   query rows with the Hadamard sums on the matrix cores, 32 rows per pass of a
 //                       wave (prolog_finish.h), unless every sum is to keep its fixed order.
@@ -97,24 +97,15 @@ __global__ __launch_bounds__(256) void lip_qproj_prefill_kernel(const QProj p, c
     q_prefill_body<TB>(p, q_prefill_job_of((int)blockIdx.x, njobs), lds);
 }
 
-// The fixed-order sums over the hidden axis at prefill sizes (xlinear_fixed.h, the form that broadcasts the hidden
-// states through DPP): workgroup = (wk or w_proj, group of eight blocks, 16 tokens); only the group sums reach memory,
-// an eighth of the rows the decode form leaves, and a block of weights serves sixteen tokens instead of two.
+// The fixed-order sums over the hidden axis at prefill sizes (xlinear_fixed.h, the matrix-core form of the sequential
+// sums); only the group sums reach memory, an eighth of the rows the decode form leaves.
 static_assert(XL_BLOCK == LIP_XBLOCK && XL_GROUP == LIP_XGROUP, "the second launch adds groups of eight blocks of 64");
-__global__ __launch_bounds__(64 * XL_WAVES) void lip_xlinear_group_kernel(const LipParams p, const int ngroups)
+__global__ __launch_bounds__(64 * XF_WAVES) void lip_xlinear_group_kernel(const LipParams p, const int ngroups)
 {
-    __shared__ __attribute__((aligned(16))) uint8_t smem[XD_LDS];
-    const int slab = blockIdx.x & 1;
-    const int g = (blockIdx.x >> 1) % ngroups;
-    const int t0 = ((blockIdx.x >> 1) / ngroups) * XD_TOK;
-    XlSlab sl;
-    sl.w = reinterpret_cast<const uint8_t *>(slab ? p.w_proj : p.wk);
-    sl.pitch = (slab ? p.n_heads : LIP_DIM) * 2;
-    sl.wbytes = sl.pitch;
-    sl.out = p.xpart + (size_t)g * p.T * LIP_XCOLS + slab * LIP_DIM;
-    sl.out_pitch = LIP_XCOLS;
-    if (slab) xd_body<false>(sl, p.x, p.T, p.h, g, t0, smem);      // w_proj: one column per lane
-    else xd_body<true>(sl, p.x, p.T, p.h, g, t0, smem);
+    __shared__ __attribute__((aligned(16))) uint8_t smem[XF_LDS];
+    const XfJob j = xf_job((int)blockIdx.x, LIP_XF_SETS, ngroups, p.T);
+    if (j.g < 0) return;
+    xf_body(lip_xf_slab(p, j.set, j.g), p.x, p.T, p.h, j.g, j.t0, smem);
 }
 
 // The sums over the hidden axis on the matrix cores (xlinear_mfma.h): workgroup = (wk or w_proj, one of nsplit
@@ -169,6 +160,7 @@ int lip_finish_query_wgs(const LipParams &p) { return lip_q_on_matrix_cores(p) ?
 
 hipError_t lip_launch_linear(const LipParams &p, hipStream_t stream)
 {
+    const bool x_done = p.x_in_groups != 0;           // the sums over the hidden axis rode in another launch
     const int steps = p.q_lora / LIP_KSPLIT / 32;
     const int tblocks = (p.T + 31) / 32;
     const bool unsplit = qproj_splits(p.T) == 1;      // prefill sizes: the query projection as a launch of its own
@@ -188,7 +180,7 @@ hipError_t lip_launch_linear(const LipParams &p, hipStream_t stream)
             else hipLaunchKernelGGL(lip_qproj_prefill_kernel<4>, g, b, 0, stream, qp, njobs);
         }
         const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
+        if (e != hipSuccess || x_done) return e;
     }
     if (lip_x_on_matrix_cores(p)) {
         const int nsplit = lip_xrows(p);
@@ -198,8 +190,7 @@ hipError_t lip_launch_linear(const LipParams &p, hipStream_t stream)
     }
     if (lip_x_group_rows(p)) {
         const int ngroups = lip_xrows(p);
-        const int tgroups = (p.T + XD_TOK - 1) / XD_TOK;
-        hipLaunchKernelGGL(lip_xlinear_group_kernel, dim3((unsigned)(2 * ngroups * tgroups)), dim3(64 * XL_WAVES), 0, stream, p, ngroups);
+        hipLaunchKernelGGL(lip_xlinear_group_kernel, dim3((unsigned)xf_jobs(LIP_XF_SETS, ngroups, p.T)), dim3(64 * XF_WAVES), 0, stream, p, ngroups);
         return hipGetLastError();
     }
     const int xtok = lip_xtok(p.T);

@@ -1,8 +1,10 @@
-// The lightning-indexer prolog's fixed-order sums over the hidden axis as wave jobs (decode forms): shared by the
-// indexer prolog's first launch and by the fused prolog, whose matrix-core launch takes them along as riders.
+// The lightning-indexer prolog's fixed-order sums over the hidden axis: as wave jobs (decode forms), and as column sets
+// of the matrix-core form, for the indexer prolog's own launch and for the fused prolog, whose first launch takes them
+// along.
 #pragma once
 #include "lip_kernels.h"
 #include "prolog_common.h"
+#include "xlinear_fixed.h"
 
 namespace pto {
 namespace {
@@ -109,16 +111,18 @@ __device__ __forceinline__ void x_linear_job(const LipParams &p, uint8_t *region
 __host__ __device__ inline int lip_xtok(const int T) { return T <= 8 ? 2 : (T <= 16 ? 4 : 8); }
 __host__ __device__ inline int lip_x_jobs(const LipParams &p, const int xtok) { return 2 * (p.h / LIP_XBLOCK) * ((p.T + xtok - 1) / xtok); }
 
-// jobs first, first + stride, ... of a wave, xtok tokens per job (uniform)
-__device__ __forceinline__ void x_linear_jobs(const LipParams &p, uint8_t *region, const int first, const int stride, const int x_jobs, const int xtok)
+// Column sets of the matrix-core form of these sums (xf_body): two halves of wk, then w_proj.
+constexpr int LIP_XF_SETS = 3;
+__device__ __forceinline__ XlSlab lip_xf_slab(const LipParams &p, const int set, const int g)
 {
-    if (xtok == 2) {
-        for (int j = first; j < x_jobs; j += stride) x_linear_job<2>(p, region, j);
-    } else if (xtok == 4) {
-        for (int j = first; j < x_jobs; j += stride) x_linear_job<4>(p, region, j);
-    } else {
-        for (int j = first; j < x_jobs; j += stride) x_linear_job<8>(p, region, j);
-    }
+    XlSlab sl;
+    const bool proj = set == 2;
+    sl.w = reinterpret_cast<const uint8_t *>(proj ? p.w_proj : p.wk) + (proj ? 0 : set * 2 * XF_COLS);
+    sl.pitch = (proj ? p.n_heads : LIP_DIM) * 2;
+    sl.wbytes = proj ? sl.pitch : 2 * XF_COLS;
+    sl.out = p.xpart + (size_t)g * p.T * LIP_XCOLS + set * XF_COLS;
+    sl.out_pitch = LIP_XCOLS;
+    return sl;
 }
 
 }  // namespace

@@ -31,7 +31,7 @@
 //   mlap_xlinear_mfma_kernel   the sums over the hidden axis on the matrix cores (xlinear_mfma.h) unless the fixed
 //                        order is asked for: per workgroup a 128-column slab x 128 tokens x a range of the hidden
 //                        axis, v_mfma_f32_32x32x16_bf16 with the row-major weight chunk as the transposed operand.
-//                        The launch's first workgroups take the 64 rope columns of w_dkv_kr in their fixed order
+//                        The launch's last workgroups take the 64 rope columns of w_dkv_kr in their fixed order
 //                        instead (the rotated key allows no outlier under the reference's acceptance rule).
 //   qproj_prefill_kernel, qproj_prefill256_kernel   the projection unsplit (prolog_common.h), a workgroup per
 //                        128 x 128 or 256 x 256 tile over the whole reduction axis; results leave de-quantised.
@@ -98,48 +98,40 @@ __global__ __launch_bounds__(64 * XL_WAVES) void mlap_xlinear_kernel(const MlapP
 // one of nsplit ranges of the hidden axis, 128 tokens); the 64 rope columns are a narrow slab of their own.
 static_assert(XM_KC == MLAP_XBLOCK, "the workspace is sized in chunks of the hidden axis");
 
-// The first rope_wgs workgroups of the launch (a multiple of eight, so that the XCD-wise order of the others keeps)
-// take the 64 rope columns of w_dkv_kr instead, in their fixed order at every size (xlinear_fixed.h, the four-wave DPP
-// form; workgroup = (group of eight blocks, 16 tokens)): the reference's acceptance rule allows the rotated key no
-// outlier at all (deepseekv32_mla_prolog_quant.py:688: atol 1e-4, rtol 2^-7 per element, ratio 0), and a sum that
-// lands next to a bf16 rounding boundary in another order moves a small rotated value by more than that.
-// The fused prolog's rider: workgroups past the launch's own run the indexer prolog's fixed-order sums over the
-// hidden axis (lip_xjob.h), a wave per job, beside the matrix-core workgroups (two workgroups fit a compute unit).
-struct MlapXRider {
-    LipParams lip;
-    int wgs;        // rider workgroups (0: none)
-    int x_jobs;
-    int xtok;
-};
-constexpr int XM_RIDER_LDS = 4 * X_REGION_BYTES;
-constexpr int XM_KERNEL_LDS = XM_LDS > XM_RIDER_LDS ? XM_LDS : XM_RIDER_LDS;
-static_assert(XR_LDS <= XM_LDS, "the rope jobs fit the launch's LDS");
-static_assert(2 * XM_KERNEL_LDS <= 160 * 1024, "two workgroups share a compute unit");
-__global__ __launch_bounds__(256) void mlap_xlinear_mfma_kernel(const MlapParams p, const int nslabs, const int nsplit, const int rope_wgs,
-                                                                const int rope_groups, const int own_wgs, const MlapXRider rider)
+// The workgroups past the first own_wgs take sums in their fixed order (xlinear_fixed.h, the matrix-core form of the
+// sequential sums), 64 columns each: the rope columns of w_dkv_kr at every size -- the reference's acceptance rule allows
+// the rotated key no outlier at all (deepseekv32_mla_prolog_quant.py:688: atol 1e-4, rtol 2^-7 per element, ratio 0), and
+// a sum that lands next to a bf16 rounding boundary in another order moves a small rotated value by more than that --
+// and, in the fused prolog from 64 tokens on, the indexer prolog's wk and w_proj.  They are short and follow the long workgroups of the
+// other slabs, so they fill the launch's last round; two workgroups fit a compute unit.  (1000 tokens: 69 us here and 79
+// in a launch of the indexer's own before they shared it.)
+// TB: at most 32 * TB tokens (xm_small_body), 0 for more.
+template <int TB> constexpr int XM_FORM_LDS = TB == 0 ? XM_LDS : XMS_LDS<TB == 0 ? 1 : TB>;
+template <int TB> constexpr int XM_KERNEL_LDS = XM_FORM_LDS<TB> > XF_LDS ? XM_FORM_LDS<TB> : XF_LDS;
+static_assert(2 * XM_KERNEL_LDS<0> <= 160 * 1024, "two workgroups share a compute unit");
+template <int TB>
+__global__ __launch_bounds__(256) void mlap_xlinear_mfma_kernel(const MlapParams p, const int nslabs, const int nsplit, const int own_wgs,
+                                                                const int fixed_sets, const int fixed_groups, const LipParams lip)
 {
-    __shared__ __attribute__((aligned(16))) uint8_t smem[XM_KERNEL_LDS];
+    __shared__ __attribute__((aligned(16))) uint8_t smem[XM_KERNEL_LDS<TB>];
     if ((int)blockIdx.x >= own_wgs) {
-        const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-        x_linear_jobs(rider.lip, smem + w * X_REGION_BYTES, ((int)blockIdx.x - own_wgs) * 4 + w, rider.wgs * 4, rider.x_jobs, rider.xtok);
-        return;
-    }
-    if ((int)blockIdx.x < rope_wgs) {
-        const int j = blockIdx.x;
-        const int g = j % rope_groups;
-        const int t0 = (j / rope_groups) * XD_TOK;
-        if (t0 >= p.T) return;                         // padding of the count to a multiple of eight
-        const int nc = p.q_lora + MLAP_KV + MLAP_ROPE;
+        const XfJob j = xf_job((int)blockIdx.x - own_wgs, fixed_sets, fixed_groups, p.T);
+        if (j.g < 0) return;
         XlSlab sl;
-        sl.w = reinterpret_cast<const uint8_t *>(p.w_dkvkr) + MLAP_KV * 2;
-        sl.pitch = (MLAP_KV + MLAP_ROPE) * 2;
-        sl.wbytes = MLAP_ROPE * 2;
-        sl.out = p.xpart + (size_t)g * p.T * nc + p.q_lora + MLAP_KV;
-        sl.out_pitch = nc;
-        xr_body(sl, p.x, p.T, p.h, g, t0, smem);
+        if (j.set == 0) {
+            const int nc = p.q_lora + MLAP_KV + MLAP_ROPE;
+            sl.w = reinterpret_cast<const uint8_t *>(p.w_dkvkr) + MLAP_KV * 2;
+            sl.pitch = (MLAP_KV + MLAP_ROPE) * 2;
+            sl.wbytes = MLAP_ROPE * 2;
+            sl.out = p.xpart + (size_t)j.g * p.T * nc + p.q_lora + MLAP_KV;
+            sl.out_pitch = nc;
+        } else {
+            sl = lip_xf_slab(lip, j.set - 1, j.g);
+        }
+        xf_body(sl, p.x, p.T, p.h, j.g, j.t0, smem);
         return;
     }
-    const int bid = (int)blockIdx.x - rope_wgs;
+    const int bid = (int)blockIdx.x;
     // Workgroups go round the eight XCDs, each with an L2 of its own, and the working set (hidden states + weights)
     // is several times one L2: the jobs of a slab (its ranges of h x token tiles) all run on XCD slab % 8, so a slab's
     // weights cross into one L2 only and every XCD reads the hidden states once for its two or so slabs.  The slabs
@@ -169,7 +161,9 @@ __global__ __launch_bounds__(256) void mlap_xlinear_mfma_kernel(const MlapParams
     sl.out = p.xpart + (size_t)sp * p.T * nc + slab * 128;
     sl.out_pitch = nc;
     const int nchunks = p.h / XM_KC;
-    xm_body(sl, p.x, p.T, p.h, t0, (int)((long long)sp * nchunks / nsplit), (int)((long long)(sp + 1) * nchunks / nsplit), smem);
+    const int c_begin = (int)((long long)sp * nchunks / nsplit), c_end = (int)((long long)(sp + 1) * nchunks / nsplit);
+    if constexpr (TB == 0) xm_body(sl, p.x, p.T, p.h, t0, c_begin, c_end, smem);
+    else xm_small_body<TB>(sl, p.x, p.T, p.h, c_begin, c_end, smem);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -337,21 +331,31 @@ __global__ __launch_bounds__(128) void qproj_kernel(const QProj pa, const int nj
     }
 }
 
-// TB: token blocks per tile (prolog_common.h).  HS > 0: workgroups past the launch's own run the fused prolog's
-// rider, the indexer prolog's split int8 projection (one job of a wave pair each, HS steps of 32 rows per half; the
-// other two waves only keep the barrier company), beside the tiles' workgroups (two workgroups fit a compute unit).
+// TB: token blocks per tile (prolog_common.h).  HS > 0: the fused prolog's riders.  The first fixed_wgs workgroups (a
+// multiple of eight) run the indexer prolog's fixed-order sums over the hidden axis, which nothing before the last launch
+// needs: in the first launch they would share compute units, and the matrix cores, with the workgroups every later
+// stage waits for (32 tokens: 16.3 us there against 12.7).  Workgroups past the launch's own run the indexer prolog's
+// split int8 projection (one job of a wave pair each, HS steps of 32 rows per half; the other two waves only keep the
+// barrier company), beside the tiles' workgroups (two workgroups fit a compute unit).
 template <int TB, int HS>
-__global__ __launch_bounds__(256) void qproj_prefill_kernel(const QProj p, const int njobs, const QProj rider)
+__global__ __launch_bounds__(256) void qproj_prefill_kernel(const QProj p, const int njobs, const QProj rider, const LipParams lip,
+                                                            const int fixed_groups, const int fixed_wgs)
 {
-    constexpr int RIDER_LDS = HS > 0 ? 2 * lin_region_bytes<(HS > 0 ? HS : 1)>() : 0;
+    constexpr int RIDER_LDS = HS > 0 ? (2 * lin_region_bytes<(HS > 0 ? HS : 1)>() > XF_LDS ? 2 * lin_region_bytes<(HS > 0 ? HS : 1)>() : XF_LDS) : 0;
     constexpr int LDS = QPF_LDS > RIDER_LDS ? QPF_LDS : RIDER_LDS;
     static_assert(2 * LDS <= 160 * 1024, "two workgroups share a compute unit");
     __shared__ __attribute__((aligned(16))) uint8_t lds[LDS];
-    if (HS > 0 && (int)blockIdx.x >= njobs) {
+    const int bid = (int)blockIdx.x - fixed_wgs;
+    if (HS > 0 && bid < 0) {
+        const XfJob j = xf_job((int)blockIdx.x, LIP_XF_SETS, fixed_groups, p.T);
+        if (j.g >= 0) xf_body(lip_xf_slab(lip, j.set, j.g), lip.x, lip.T, lip.h, j.g, j.t0, lds);
+        return;
+    }
+    if (HS > 0 && bid >= njobs) {
         constexpr int H = HS > 0 ? HS : 1;
         const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
         const int l = threadIdx.x & 63;
-        const int job = (int)blockIdx.x - njobs;
+        const int job = bid - njobs;
         i32x16 acc[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -366,7 +370,7 @@ __global__ __launch_bounds__(256) void qproj_prefill_kernel(const QProj p, const
         if (w == 0) q_pair_store<H>(rider, lds, job, l, acc);
         return;
     }
-    q_prefill_body<TB>(p, q_prefill_job_of((int)blockIdx.x, njobs), lds);
+    q_prefill_body<TB>(p, q_prefill_job_of(bid, njobs), lds);
 }
 
 __global__ __launch_bounds__(512) void qproj_prefill256_kernel(const QProj p, const int njobs)
@@ -424,6 +428,9 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
     const int nslabs = p.q_lora / 128 + 5;
     if (rider != nullptr && !mlap_takes_rider(p)) return hipErrorInvalidValue;
     if (lip_rider != nullptr && !mlap_takes_lip_rider(p)) return hipErrorInvalidValue;
+    LipParams lip;
+    std::memset(&lip, 0, sizeof lip);
+    if (lip_rider != nullptr) lip = *lip_rider;
     const MlapRider rd = rider != nullptr ? *rider : MlapRider{nullptr, nullptr, nullptr, nullptr, nullptr, 0};
     if (mlap_prefill_forms(p)) {
         // prefill sizes: the sums over the hidden axis on the matrix cores, in as many ranges of the hidden axis
@@ -435,26 +442,18 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
         ngroups = 2 * cus / (nslabs * ttiles);
         ngroups = ngroups < 1 ? 1 : ngroups;
         ngroups = ngroups > MLAP_XM_MAX_SPLITS ? MLAP_XM_MAX_SPLITS : ngroups;
-        ngroups = ngroups > nchunks ? nchunks : ngroups;
         // every slab but the last, the rope columns, which keep their fixed-order sums
         const int mslabs = nslabs - 1;
+        ngroups = ngroups > nchunks ? nchunks : ngroups;
         const int per_slab = ngroups * ttiles;
         const int wgs = 8 * ((mslabs >> 3) * per_slab + ((mslabs & 7) * per_slab + 7) / 8);   // the kernel's XCD-wise job order
-        const int rope_wgs = (ngroups_fixed * ((p.T + XD_TOK - 1) / XD_TOK) + 7) / 8 * 8;
-        MlapXRider xr;
-        xr.wgs = 0;
-        xr.x_jobs = xr.xtok = 0;
-        if (lip_rider != nullptr) {
-            xr.lip = *lip_rider;
-            xr.xtok = lip_xtok(lip_rider->T);
-            xr.x_jobs = lip_x_jobs(*lip_rider, xr.xtok);
-            xr.wgs = (xr.x_jobs + 3) / 4;
-            xr.wgs = xr.wgs > 2 * cus ? 2 * cus : xr.wgs;
-        } else {
-            std::memset(&xr.lip, 0, sizeof xr.lip);
-        }
-        hipLaunchKernelGGL(mlap_xlinear_mfma_kernel, dim3((unsigned)(rope_wgs + wgs + xr.wgs)), dim3(256), 0, stream, p, mslabs, ngroups, rope_wgs,
-                           ngroups_fixed, rope_wgs + wgs, xr);
+        const int sets = 1 + (lip_rider != nullptr && p.T >= QPROJ_PREFILL_TOKENS ? LIP_XF_SETS : 0);
+        const dim3 g((unsigned)(wgs + xf_jobs(sets, ngroups_fixed, p.T)));
+#define XM_LAUNCH(TBV) hipLaunchKernelGGL(mlap_xlinear_mfma_kernel<TBV>, g, dim3(256), 0, stream, p, mslabs, ngroups, wgs, sets, ngroups_fixed, lip)
+        if (p.T <= 32) XM_LAUNCH(1);
+        else if (p.T <= 64) XM_LAUNCH(2);
+        else XM_LAUNCH(0);
+#undef XM_LAUNCH
     } else {
         const int tgroups = (p.T + MLAP_XTOK - 1) / MLAP_XTOK;
         const int xslabs = nslabs + (rider != nullptr ? 1 : 0);
@@ -478,18 +477,19 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
         const int njobs = q_prefill_jobs(qp);
         const dim3 g((unsigned)njobs), b(256);
         const int tbk = q_prefill_token_blocks(p.T);
-        if (lip_rider != nullptr) {
+        if (lip_rider != nullptr && p.T < QPROJ_PREFILL_TOKENS) {
             // the indexer prolog's split projection rides along: one more workgroup per job of a wave pair
             const LipParams &lp = *lip_rider;
             const QProj qr = {lp.q_norm, lp.w_qb, lp.qpart, lp.T, lp.q_lora, lp.n_heads, lp.q_norm_scale, lp.w_qb_scale};
             const int rjobs = lp.n_heads * QPROJ_KSPLIT * ((lp.T + 31) / 32);
-            const dim3 gr((unsigned)(njobs + rjobs));
+            const int fixed_wgs = xf_jobs(LIP_XF_SETS, ngroups_fixed, p.T);
+            const dim3 gr((unsigned)(fixed_wgs + njobs + rjobs));
             const int steps = lp.q_lora / QPROJ_KSPLIT / 32;
 #define QPF_RIDER(TBV)                                                                                       \
     switch (steps) {                                                                                         \
-    case 4: hipLaunchKernelGGL((qproj_prefill_kernel<TBV, 2>), gr, b, 0, stream, qp, njobs, qr); break;     \
-    case 8: hipLaunchKernelGGL((qproj_prefill_kernel<TBV, 4>), gr, b, 0, stream, qp, njobs, qr); break;     \
-    case 12: hipLaunchKernelGGL((qproj_prefill_kernel<TBV, 6>), gr, b, 0, stream, qp, njobs, qr); break;    \
+    case 4: hipLaunchKernelGGL((qproj_prefill_kernel<TBV, 2>), gr, b, 0, stream, qp, njobs, qr, lip, ngroups_fixed, fixed_wgs); break;     \
+    case 8: hipLaunchKernelGGL((qproj_prefill_kernel<TBV, 4>), gr, b, 0, stream, qp, njobs, qr, lip, ngroups_fixed, fixed_wgs); break;     \
+    case 12: hipLaunchKernelGGL((qproj_prefill_kernel<TBV, 6>), gr, b, 0, stream, qp, njobs, qr, lip, ngroups_fixed, fixed_wgs); break;    \
     default: return hipErrorInvalidValue;                                                                    \
     }
             if (tbk == 1) { QPF_RIDER(1) } else { QPF_RIDER(2) }
@@ -497,9 +497,9 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
             return hipGetLastError();
         }
         switch (tbk) {
-        case 1: hipLaunchKernelGGL((qproj_prefill_kernel<1, 0>), g, b, 0, stream, qp, njobs, qp); break;
-        case 2: hipLaunchKernelGGL((qproj_prefill_kernel<2, 0>), g, b, 0, stream, qp, njobs, qp); break;
-        default: hipLaunchKernelGGL((qproj_prefill_kernel<4, 0>), g, b, 0, stream, qp, njobs, qp);
+        case 1: hipLaunchKernelGGL((qproj_prefill_kernel<1, 0>), g, b, 0, stream, qp, njobs, qp, lip, 0, 0); break;
+        case 2: hipLaunchKernelGGL((qproj_prefill_kernel<2, 0>), g, b, 0, stream, qp, njobs, qp, lip, 0, 0); break;
+        default: hipLaunchKernelGGL((qproj_prefill_kernel<4, 0>), g, b, 0, stream, qp, njobs, qp, lip, 0, 0);
         }
         return hipGetLastError();
     }

@@ -6,9 +6,9 @@
 // workgroups that finish the attention query (absorb product, 70 KB of LDS, four waves) and those that finish the
 // indexer's query rows, key row and weights (54 KB, eight waves) do not depend on each other and fit a compute
 // unit together, so they run side by side instead of one launch after the other.  Where the indexer prolog cannot
-// ride (other than 64 indexer heads) its first launch follows the MLA prolog's third.  Between 9 and 63 tokens the
-// MLA prolog's prefill forms take the jobs of the indexer prolog's first launch along as riders (five launches;
-// four up to 32 tokens, where the two last stages share one); from 64 tokens on every stage has a launch of its own.
+// ride (other than 64 indexer heads) its first launch follows the MLA prolog's third.  From 9 tokens on the MLA
+// prolog's prefill forms take the indexer prolog's fixed-order sums along, up to 63 tokens its projection too (five
+// launches; four up to 32 tokens, where the two last stages share one).
 #include "prolog_finish.h"
 
 #include "prolog_fused.h"
@@ -70,38 +70,40 @@ hipError_t prolog_fused_launch(const MlapParams &pm, const LipParams &pl, hipStr
                            mla_wgs, q_wgs);
         return hipGetLastError();
     }
-    // A batch of 9 to 63 tokens: the MLA prolog runs its prefill forms, the indexer prolog its decode forms, and the
-    // jobs of the indexer prolog's first launch (wave jobs with no kind of workgroup of their own) ride in the MLA
-    // prolog's first and third launch, whose workgroups leave half of every compute unit free, and up to 32 tokens the
-    // finishing stages of the two halves share the last launch: four launches, five above.
+    // From 9 tokens on the MLA prolog runs its prefill forms, which take the indexer prolog's fixed-order sums along in
+    // the first launch or, up to 63 tokens, in the third with its split projection (the third launch's workgroups leave
+    // half of every compute unit free); up to 32 tokens the finishing stages of the two halves share the last launch:
+    // four launches, five up to 63 tokens.
     const bool lip_rides = mlap_takes_lip_rider(pm) && pl.T == pm.T && pl.h == pm.h && pl.q_lora == pm.q_lora && pl.x == pm.x &&
-                           pl.q_norm == pm.q_norm && pl.q_norm_scale == pm.q_norm_scale && !lip_q_on_matrix_cores(pl) &&
-                           !lip_x_on_matrix_cores(pl) && !lip_x_group_rows(pl) && pl.n_heads <= LIP_MAX_HEADS;
-    hipError_t e = mlap_launch_front(pm, stream, nullptr, lip_rides ? &pl : nullptr);
+                           pl.q_norm == pm.q_norm && pl.q_norm_scale == pm.q_norm_scale && !lip_x_on_matrix_cores(pl) &&
+                           lip_x_group_width(pl) && pl.n_heads <= LIP_MAX_HEADS;
+    LipParams px = pl;
+    if (lip_rides) px.x_in_groups = 1;
+    hipError_t e = mlap_launch_front(pm, stream, nullptr, lip_rides ? &px : nullptr);
     if (e != hipSuccess) return e;
-    if (!lip_rides) {
-        e = lip_launch_linear(pl, stream);
+    if (!lip_rides || px.T >= QPROJ_PREFILL_TOKENS) {
+        e = lip_launch_linear(px, stream);
         if (e != hipSuccess) return e;
     }
     int per = 0, pf_wgs = 0;
     if (mlap_finish_is_prefill(pm)) mlap_finish_prefill_shape(pm, per, pf_wgs);
     // up to 32 tokens: one workgroup per head, the indexer half's take the other compute units (more would queue one
     // to a compute unit behind a full chip, slower than their own launch at two)
-    if (mlap_finish_is_prefill(pm) && !lip_q_on_matrix_cores(pl) && pf_wgs <= 128) {
-        const int q_wgs = lip_finish_query_wgs(pl);
-        hipLaunchKernelGGL(prolog_fused_finish_prefill_kernel, dim3((unsigned)(pf_wgs + q_wgs + pl.T)), dim3(64 * FIN_WAVES), 0, stream, pm, per,
-                           pl, pf_wgs, q_wgs);
+    if (mlap_finish_is_prefill(pm) && !lip_q_on_matrix_cores(px) && pf_wgs <= 128) {
+        const int q_wgs = lip_finish_query_wgs(px);
+        hipLaunchKernelGGL(prolog_fused_finish_prefill_kernel, dim3((unsigned)(pf_wgs + q_wgs + px.T)), dim3(64 * FIN_WAVES), 0, stream, pm, per,
+                           px, pf_wgs, q_wgs);
         return hipGetLastError();
     }
-    if (mlap_finish_is_prefill(pm) || lip_q_on_matrix_cores(pl)) {
+    if (mlap_finish_is_prefill(pm) || lip_q_on_matrix_cores(px)) {
         // prefill sizes: the last stages have forms of their own (the attention query's: one workgroup per compute unit)
         e = mlap_launch_finish(pm, stream);
         if (e != hipSuccess) return e;
-        return lip_launch_finish(pl, stream);
+        return lip_launch_finish(px, stream);
     }
     const int mla_wgs = mlap_finish_wgs(pm);
-    const int q_wgs = lip_finish_query_wgs(pl);
-    hipLaunchKernelGGL(prolog_fused_finish_kernel, dim3((unsigned)(mla_wgs + q_wgs + pl.T)), dim3(64 * FIN_WAVES), 0, stream, pm, pl,
+    const int q_wgs = lip_finish_query_wgs(px);
+    hipLaunchKernelGGL(prolog_fused_finish_kernel, dim3((unsigned)(mla_wgs + q_wgs + px.T)), dim3(64 * FIN_WAVES), 0, stream, pm, px,
                        mla_wgs, q_wgs);
     return hipGetLastError();
 }

@@ -1,6 +1,7 @@
 // Fixed-order sums over the hidden axis, one group of eight blocks of 64 rows per workgroup: x [T, h] bf16 times a
-// slab of up to 128 columns of a row-major bf16 weight matrix.  Shared by the MLA prolog (w_dq, w_dkv_kr; every
-// size) and the lightning-indexer prolog (wk, w_proj; prefill sizes); included after prolog_common.h.
+// slab of columns of a row-major bf16 weight matrix.  Two forms: xl_body on the vector ALU, 8 tokens per workgroup (the
+// MLA prolog's fixed-order launches), and xf_body on the matrix cores, 32 tokens (the rope columns and the indexer
+// prolog's wk and w_proj from 9 or 64 tokens on); included after prolog_common.h.
 //
 // Every product of two bf16 values is exact in fp32; a block is summed ascending from 0.0 by fp32 FMAs, the
 // workgroup's eight block sums (one per wave) meet in LDS and are added ascending into the group sum, which is all
@@ -125,255 +126,133 @@ __device__ __forceinline__ void xl_body(const XlSlab &sl, const uint16_t *x, con
 }
 
 // ---------------------------------------------------------------------------------------------
-// The same sums for prefill-sized token counts with the hidden states broadcast by the multiply-add itself: a lane
-// keeps x[t][k0 + 2*(l % 16)] and x[t][k0 + 2*(l % 16) + 1] of a 32-row half block in two registers per token (every
-// row of 16 lanes holds the same 32 values), and v_fmac_f32 with the DPP control row_newbcast:n reads lane n of the
-// row, i.e. hidden row k0 + 2n (or + 1), in all lanes -- no LDS read and no extra instruction per hidden state, where
-// the form above spends an LDS broadcast of 16 bytes per four multiply-adds.  Same products, same order (a block
-// ascending from 0.0, the eight block sums ascending), so the same bits.
-//   workgroup = (slab, group of 512 hidden rows, XD_TOK tokens), eight waves, wave w takes block 8*group + w.
-//   PAIR: lane l holds columns 2l, 2l+1 (a slab of 128 columns); otherwise column l (a slab of up to 64).
-constexpr int XD_TOK = 16;
-constexpr int XD_LDS = XL_WAVES * XL_W_BYTES;
+// The same sums for larger token counts on the matrix cores: v_mfma_f32_32x32x1_2b_f32 multiplies one hidden row at a
+// time, so each of its results is one product (exact: both factors are bf16 values) added to the accumulator with one
+// rounding -- an fp32 FMA -- and a chain of them is the sequential sum of the form above, bit for bit, whatever order
+// the cores have inside an instruction of more rows.  (Subnormal products and sums, signed zeros included: checked
+// against fmaf chains.)
+//   workgroup = (slab of up to 64 columns, group of 512 hidden rows, 32 tokens), four waves; wave w takes blocks 2w and
+//   2w + 1 of the group as the two independent products of the instruction (lanes 0..31 supply block 2w, lanes 32..63
+//   block 2w + 1).  Row i of the first operand is column 2i (accumulator 0) or 2i + 1 (accumulator 1) of the slab: one
+//   dword of LDS per lane and hidden row feeds both.  The hidden states go from memory to registers, 64 consecutive
+//   ones per lane.  The eight block sums meet in LDS and are chained ascending into the group sum.
+// Bound: the matrix cores' fp32 rate (64 clocks per instruction, 139 TFLOP/s reached by a bare loop); per two
+// instructions there are one LDS read and three conversions.  The multiply-add form of the vector ALU this replaced
+// (hidden states broadcast through DPP) ran at a quarter of that: 192 columns x 1000 tokens x 7168 rows took 79 us.
+constexpr int XF_TOK = 32;                                               // tokens per workgroup
+constexpr int XF_COLS = 64;                                              // columns per workgroup, at most
+constexpr int XF_WAVES = 4;
+constexpr int XF_BLOCK_PITCH = XL_BLOCK * 2 * XF_COLS + 128;             // a wave's second block lies 32 banks off the first
+constexpr int XF_STAGE = 2 * XF_BLOCK_PITCH;
+constexpr int XF_TOK_PITCH = XF_COLS * 4 + 16;                           // bytes between token rows of a block sum
+constexpr int XF_SUMS = XF_TOK * XF_TOK_PITCH;
+constexpr int XF_LDS = XF_WAVES * XF_STAGE > XL_GROUP * XF_SUMS ? XF_WAVES * XF_STAGE : XL_GROUP * XF_SUMS;   // 69 632 bytes
+static_assert(XL_GROUP == 2 * XF_WAVES, "two blocks per wave");
 
-// acc[t] += bcast_N(x[t]) * w for eight tokens (and a second column with w1), as one statement: nothing the compiler
-// emits can sit between the multiply-adds, and the statement opens with the two wait states a DPP read wants after a
-// write of its operand, whatever the compiler did to these registers just before.
-#define XD_F "v_fmac_f32_dpp %"
-#define XD_B " row_newbcast:%[n] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-template <int N>
-__device__ __forceinline__ void fmac8_pair(float *a0, float *a1, const float *x, const float w0, const float w1)
-{
-    asm("s_nop 1\n\t"
-        XD_F "0, %16, %[w0]" XD_B XD_F "8, %16, %[w1]" XD_B XD_F "1, %17, %[w0]" XD_B XD_F "9, %17, %[w1]" XD_B
-        XD_F "2, %18, %[w0]" XD_B XD_F "10, %18, %[w1]" XD_B XD_F "3, %19, %[w0]" XD_B XD_F "11, %19, %[w1]" XD_B
-        XD_F "4, %20, %[w0]" XD_B XD_F "12, %20, %[w1]" XD_B XD_F "5, %21, %[w0]" XD_B XD_F "13, %21, %[w1]" XD_B
-        XD_F "6, %22, %[w0]" XD_B XD_F "14, %22, %[w1]" XD_B XD_F "7, %23, %[w0]" XD_B XD_F "15, %23, %[w1]" XD_B
-        : "+v"(a0[0]), "+v"(a0[1]), "+v"(a0[2]), "+v"(a0[3]), "+v"(a0[4]), "+v"(a0[5]), "+v"(a0[6]), "+v"(a0[7]),
-          "+v"(a1[0]), "+v"(a1[1]), "+v"(a1[2]), "+v"(a1[3]), "+v"(a1[4]), "+v"(a1[5]), "+v"(a1[6]), "+v"(a1[7])
-        : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]), "v"(x[7]), [w0] "v"(w0), [w1] "v"(w1), [n] "n"(N));
-}
-template <int N>
-__device__ __forceinline__ void fmac8_single(float *a0, const float *x, const float w0)
-{
-    asm("s_nop 1\n\t"
-        XD_F "0, %8, %[w0]" XD_B XD_F "1, %9, %[w0]" XD_B XD_F "2, %10, %[w0]" XD_B XD_F "3, %11, %[w0]" XD_B
-        XD_F "4, %12, %[w0]" XD_B XD_F "5, %13, %[w0]" XD_B XD_F "6, %14, %[w0]" XD_B XD_F "7, %15, %[w0]" XD_B
-        : "+v"(a0[0]), "+v"(a0[1]), "+v"(a0[2]), "+v"(a0[3]), "+v"(a0[4]), "+v"(a0[5]), "+v"(a0[6]), "+v"(a0[7])
-        : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]), "v"(x[7]), [w0] "v"(w0), [n] "n"(N));
-}
-#undef XD_F
-#undef XD_B
+__host__ __device__ inline int xf_token_tiles(const int T) { return (T + XF_TOK - 1) / XF_TOK; }
 
-template <bool PAIR, int N>
-__device__ __forceinline__ void xd_pair_of_rows(const uint8_t *wrow, const int rowbytes, const int lane_off, float (&xe)[XD_TOK],
-                                                float (&xo)[XD_TOK], float (&a0)[XD_TOK], float (&a1)[XD_TOK])
+// The jobs of a launch: sets of columns x groups x token tiles.  Workgroups go round the eight XCDs; the sets of one
+// (group, tile) are consecutive workgroups of one XCD, so its hidden states cross into that L2 once.
+__host__ __device__ inline int xf_jobs(const int nsets, const int ngroups, const int T)
 {
-#pragma unroll
-    for (int odd = 0; odd < 2; ++odd) {
-        float *xs = odd ? xo : xe;
-        if (PAIR) {
-            const uint32_t wv = *reinterpret_cast<const uint32_t *>(wrow + (2 * N + odd) * rowbytes + lane_off);
-            const float w0 = __uint_as_float(wv << 16), w1 = __uint_as_float(wv & 0xffff0000u);
-#pragma unroll
-            for (int t = 0; t < XD_TOK; t += 8) fmac8_pair<N>(a0 + t, a1 + t, xs + t, w0, w1);
-        } else {
-            const float w0 = __uint_as_float((uint32_t) * reinterpret_cast<const uint16_t *>(wrow + (2 * N + odd) * rowbytes + lane_off) << 16);
-#pragma unroll
-            for (int t = 0; t < XD_TOK; t += 8) fmac8_single<N>(a0 + t, xs + t, w0);
-        }
-    }
+    return 8 * nsets * ((ngroups * xf_token_tiles(T) + 7) / 8);
+}
+struct XfJob {
+    int set, g, t0;       // g < 0: padding of the job count
+};
+__device__ __forceinline__ XfJob xf_job(const int j, const int nsets, const int ngroups, const int T)
+{
+    const int q = j >> 3;
+    const int c = (q / nsets) * 8 + (j & 7);
+    XfJob r;
+    r.set = q % nsets;
+    r.g = c < ngroups * xf_token_tiles(T) ? c % ngroups : -1;
+    r.t0 = (c / ngroups) * XF_TOK;
+    return r;
 }
 
-template <bool PAIR>
-__device__ __forceinline__ void xd_body(const XlSlab &sl, const uint16_t *x, const int T, const int h, const int g, const int t0, uint8_t *smem)
+// group g of the hidden axis, tokens t0 .. t0 + 31 (rows past T - 1 repeat it and are not stored); sl.wbytes <= 128
+__device__ __forceinline__ void xf_body(const XlSlab &sl, const uint16_t *x, const int T, const int h, const int g, const int t0, uint8_t *smem)
 {
+    typedef __attribute__((ext_vector_type(32))) float f32x32;
     const int l = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int half = l >> 5, i = l & 31;
     const int nblk = h / XL_BLOCK;
+    const int nb = nblk - g * XL_GROUP < XL_GROUP ? nblk - g * XL_GROUP : XL_GROUP;
     const int wbytes = sl.wbytes;
-    const int ncols = wbytes >> 1;
-    uint8_t *region = smem + w * XL_W_BYTES;
-    const int c = g * XL_GROUP + w;                                       // this wave's block
-    const int nb = nblk - g * XL_GROUP < XL_GROUP ? nblk - g * XL_GROUP : XL_GROUP;
-    float a0[XD_TOK], a1[XD_TOK];
+    f32x32 a0, a1;
 #pragma unroll
-    for (int t = 0; t < XD_TOK; ++t) a0[t] = a1[t] = 0.f;
-
-    if (w < nb) {
-        const int k0 = c * XL_BLOCK;
-        const uint32_t wdst = (uint32_t)(uintptr_t)(lds_byte_t *)region;
-        {   // rows of wbytes bytes: wbytes/16 lanes per row
-            const int lpr = wbytes >> 4;
-            const int rpi = 64 / lpr;                                     // rows per request
-            const uint8_t *src = sl.w + (size_t)(k0 + l / lpr) * sl.pitch + 16 * (l % lpr);
+    for (int r = 0; r < 32; ++r) a0[r] = a1[r] = 0.f;
+    if (2 * w < nb) {
+        // a group's last wave may have one block only: both halves then work on it, and the second result is dropped
+        const int second = 2 * w + 1 < nb ? 2 * w + 1 : 2 * w;
+        uint8_t *region = smem + w * XF_STAGE;
+        {   // eight rows per request, 128 bytes apart in LDS (lanes past a narrow slab's row repeat its first piece)
+            const int piece = (l & 7) < (wbytes >> 4) ? l & 7 : 0;
 #pragma unroll 1
-            for (int i = 0; i < XL_BLOCK / rpi; ++i) dma16(src + (size_t)i * rpi * sl.pitch, wdst + 1024 * i);
-        }
-        // hidden states of both half blocks: lane l holds rows k0 + 32*hb + 2*(l%16), +1 of every token
-        uint32_t xr[2][XD_TOK];
-#pragma unroll
-        for (int hb = 0; hb < 2; ++hb)
-#pragma unroll
-            for (int t = 0; t < XD_TOK; ++t) {
-                const int tt = t0 + t < T ? t0 + t : T - 1;
-                xr[hb][t] = reinterpret_cast<const uint32_t *>(x + (size_t)tt * h + k0 + 32 * hb)[l & 15];
+            for (int b = 0; b < 2; ++b) {
+                const int k0 = (g * XL_GROUP + (b ? second : 2 * w)) * XL_BLOCK;
+                const uint8_t *src = sl.w + (size_t)(k0 + (l >> 3)) * sl.pitch + 16 * piece;
+                const uint32_t dst = (uint32_t)(uintptr_t)(lds_byte_t *)(region + b * XF_BLOCK_PITCH);
+#pragma unroll 1
+                for (int q = 0; q < XL_BLOCK / 8; ++q) dma16(src + (size_t)q * 8 * sl.pitch, dst + 1024 * q);
             }
+        }
+        const int t = t0 + i < T ? t0 + i : T - 1;
+        const u32x4 *xp = reinterpret_cast<const u32x4 *>(x + (size_t)t * h + (g * XL_GROUP + (half ? second : 2 * w)) * XL_BLOCK);
+        u32x4 xv[XL_BLOCK / 8];
+#pragma unroll
+        for (int q = 0; q < XL_BLOCK / 8; ++q) xv[q] = xp[q];
         VM_WAIT(0);
-        const int lane_off = PAIR ? 4 * (2 * l < ncols ? l : 0) : 2 * (l < ncols ? l : 0);
+        asm volatile("" ::: "memory");
+        const uint8_t *wl = region + half * XF_BLOCK_PITCH + 4 * i;
 #pragma unroll
-        for (int hb = 0; hb < 2; ++hb) {
-            float xe[XD_TOK], xo[XD_TOK];
-#pragma unroll
-            for (int t = 0; t < XD_TOK; ++t) {
-                xe[t] = __uint_as_float(xr[hb][t] << 16);
-                xo[t] = __uint_as_float(xr[hb][t] & 0xffff0000u);
-            }
-            const uint8_t *wrow = region + 32 * hb * wbytes;
-            xd_pair_of_rows<PAIR, 0>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-            xd_pair_of_rows<PAIR, 1>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-            xd_pair_of_rows<PAIR, 2>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-            xd_pair_of_rows<PAIR, 3>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-            xd_pair_of_rows<PAIR, 4>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-            xd_pair_of_rows<PAIR, 5>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-            xd_pair_of_rows<PAIR, 6>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-            xd_pair_of_rows<PAIR, 7>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-            xd_pair_of_rows<PAIR, 8>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-            xd_pair_of_rows<PAIR, 9>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-            xd_pair_of_rows<PAIR, 10>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-            xd_pair_of_rows<PAIR, 11>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-            xd_pair_of_rows<PAIR, 12>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-            xd_pair_of_rows<PAIR, 13>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-            xd_pair_of_rows<PAIR, 14>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-            xd_pair_of_rows<PAIR, 15>(wrow, wbytes, lane_off, xe, xo, a0, a1);
+        for (int k = 0; k < XL_BLOCK; ++k) {
+            const uint32_t wv = *reinterpret_cast<const uint32_t *>(wl + k * 2 * XF_COLS);
+            const uint32_t xw = xv[k >> 3][(k >> 1) & 3];
+            const float xf = __uint_as_float((k & 1) ? xw & 0xffff0000u : xw << 16);
+            a0 = __builtin_amdgcn_mfma_f32_32x32x1f32(__uint_as_float(wv << 16), xf, a0, 0, 0, 0);
+            a1 = __builtin_amdgcn_mfma_f32_32x32x1f32(__uint_as_float(wv & 0xffff0000u), xf, a1, 0, 0, 0);
         }
     }
-    __syncthreads();                                   // every wave is done with its block of weights
-    // block sums into this wave's own (consumed) region: [XD_TOK tokens][128 columns]
-    if (w < nb) {
-        float *bs = reinterpret_cast<float *>(region);
+    __syncthreads();                                                     // every wave is done with its weights
+    if (2 * w < nb) {
+        // register 16*b + 4*q + j of lane (token, half) is row 8*q + 4*half + j of block b's product
 #pragma unroll
-        for (int t = 0; t < XD_TOK; ++t) {
-            if (PAIR) {
-                f32x2 v = {a0[t], a1[t]};
-                *reinterpret_cast<f32x2 *>(bs + t * 128 + 2 * l) = v;
-            } else {
-                bs[t * 128 + l] = a0[t];
-            }
+        for (int b = 0; b < 2; ++b) {
+            uint8_t *row = smem + (2 * w + b) * XF_SUMS + i * XF_TOK_PITCH + 32 * half;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const int r = 16 * b + 4 * q + 2 * e;
+                    const f32x4 v = {a0[r], a1[r], a0[r + 1], a1[r + 1]};
+                    *reinterpret_cast<f32x4 *>(row + 64 * q + 16 * e) = v;
+                }
         }
     }
     __syncthreads();
-    // group sums: wave w chains the block sums of tokens w and w + 8 in ascending order
-#pragma unroll
-    for (int u = 0; u < XD_TOK / XL_WAVES; ++u) {
-        const int tl = w + XL_WAVES * u;
+    {   // thread (token, eight columns) chains the block sums in ascending order
+        const int tl = threadIdx.x >> 3, c8 = 8 * (threadIdx.x & 7);
         const int t = t0 + tl;
-        if (t < T) {
-            if (PAIR) {
-                if (2 * l < ncols) {
-                    float s0 = 0.f, s1 = 0.f;
-                    for (int i = 0; i < nb; ++i) {
-                        const f32x2 v = *reinterpret_cast<const f32x2 *>(reinterpret_cast<const float *>(smem + i * XL_W_BYTES) + tl * 128 + 2 * l);
-                        s0 = __fadd_rn(s0, v[0]);
-                        s1 = __fadd_rn(s1, v[1]);
-                    }
-                    f32x2 v = {s0, s1};
-                    *reinterpret_cast<f32x2 *>(sl.out + (size_t)t * sl.out_pitch + 2 * l) = v;
+        if (t < T && 2 * c8 < wbytes) {
+            float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            for (int b = 0; b < nb; ++b) {
+                const f32x4 *src = reinterpret_cast<const f32x4 *>(smem + b * XF_SUMS + tl * XF_TOK_PITCH + 4 * c8);
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const f32x4 v = src[e];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) s[4 * e + j] = __fadd_rn(s[4 * e + j], v[j]);
                 }
-            } else if (l < ncols) {
-                float s0 = 0.f;
-                for (int i = 0; i < nb; ++i) s0 = __fadd_rn(s0, reinterpret_cast<const float *>(smem + i * XL_W_BYTES)[tl * 128 + l]);
-                sl.out[(size_t)t * sl.out_pitch + l] = s0;
             }
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------------------------
-// The DPP form for a slab of 64 columns in a workgroup of FOUR waves, so that its jobs can ride in a launch whose
-// workgroups have 256 threads: wave w takes blocks w and w + 4 of the group one after the other (the same 64
-// sequential multiply-adds per block from 0.0), the eight block sums are parked in LDS beside the staging areas and
-// chained ascending into the group sum -- product by product and sum by sum what xd_body<false> computes, so the
-// same bits.  LDS: four staging areas of 64 rows x 128 bytes, then eight block-sum areas of [XD_TOK][64] floats.
-constexpr int XR_WAVES = 4;
-constexpr int XR_STAGE = XL_BLOCK * 128;                                 // a block of the slab: 64 rows x 128 bytes
-constexpr int XR_SUMS = XD_TOK * 64 * 4;
-constexpr int XR_LDS = XR_WAVES * XR_STAGE + XL_GROUP * XR_SUMS;
-
-__device__ __forceinline__ void xr_body(const XlSlab &sl, const uint16_t *x, const int T, const int h, const int g, const int t0, uint8_t *smem)
-{
-    const int l = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int nblk = h / XL_BLOCK;
-    constexpr int wbytes = 128;
-    uint8_t *region = smem + w * XR_STAGE;
-    const int nb = nblk - g * XL_GROUP < XL_GROUP ? nblk - g * XL_GROUP : XL_GROUP;
-#pragma unroll 1
-    for (int pass = 0; pass < XL_GROUP / XR_WAVES; ++pass) {
-        const int bi = w + XR_WAVES * pass;                               // this wave's block of the group
-        if (bi < nb) {
-            float a0[XD_TOK], a1[XD_TOK];
+            f32x4 *dst = reinterpret_cast<f32x4 *>(sl.out + (size_t)t * sl.out_pitch + c8);
 #pragma unroll
-            for (int t = 0; t < XD_TOK; ++t) a0[t] = a1[t] = 0.f;
-            const int k0 = (g * XL_GROUP + bi) * XL_BLOCK;
-            const uint32_t wdst = (uint32_t)(uintptr_t)(lds_byte_t *)region;
-            {   // rows of 128 bytes: eight lanes per row, eight rows per request
-                const uint8_t *src = sl.w + (size_t)(k0 + (l >> 3)) * sl.pitch + 16 * (l & 7);
-#pragma unroll 1
-                for (int i = 0; i < XL_BLOCK / 8; ++i) dma16(src + (size_t)i * 8 * sl.pitch, wdst + 1024 * i);
+            for (int e = 0; e < 2; ++e) {
+                const f32x4 v = {s[4 * e], s[4 * e + 1], s[4 * e + 2], s[4 * e + 3]};
+                dst[e] = v;
             }
-            uint32_t xr[2][XD_TOK];
-#pragma unroll
-            for (int hb = 0; hb < 2; ++hb)
-#pragma unroll
-                for (int t = 0; t < XD_TOK; ++t) {
-                    const int tt = t0 + t < T ? t0 + t : T - 1;
-                    xr[hb][t] = reinterpret_cast<const uint32_t *>(x + (size_t)tt * h + k0 + 32 * hb)[l & 15];
-                }
-            VM_WAIT(0);
-            const int lane_off = 2 * l;
-#pragma unroll
-            for (int hb = 0; hb < 2; ++hb) {
-                float xe[XD_TOK], xo[XD_TOK];
-#pragma unroll
-                for (int t = 0; t < XD_TOK; ++t) {
-                    xe[t] = __uint_as_float(xr[hb][t] << 16);
-                    xo[t] = __uint_as_float(xr[hb][t] & 0xffff0000u);
-                }
-                const uint8_t *wrow = region + 32 * hb * wbytes;
-                xd_pair_of_rows<false, 0>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-                xd_pair_of_rows<false, 1>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-                xd_pair_of_rows<false, 2>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-                xd_pair_of_rows<false, 3>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-                xd_pair_of_rows<false, 4>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-                xd_pair_of_rows<false, 5>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-                xd_pair_of_rows<false, 6>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-                xd_pair_of_rows<false, 7>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-                xd_pair_of_rows<false, 8>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-                xd_pair_of_rows<false, 9>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-                xd_pair_of_rows<false, 10>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-                xd_pair_of_rows<false, 11>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-                xd_pair_of_rows<false, 12>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-                xd_pair_of_rows<false, 13>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-                xd_pair_of_rows<false, 14>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-                xd_pair_of_rows<false, 15>(wrow, wbytes, lane_off, xe, xo, a0, a1);
-            }
-            // (the LDS reads of the weights above are complete: their results were consumed by the multiply-adds)
-            float *bs = reinterpret_cast<float *>(smem + XR_WAVES * XR_STAGE + bi * XR_SUMS);
-#pragma unroll
-            for (int t = 0; t < XD_TOK; ++t) bs[t * 64 + l] = a0[t];
-        }
-    }
-    __syncthreads();
-    // group sums: wave w chains the block sums of tokens w, w + 4, w + 8, w + 12 in ascending order
-#pragma unroll
-    for (int u = 0; u < XD_TOK / XR_WAVES; ++u) {
-        const int tl = w + XR_WAVES * u;
-        const int t = t0 + tl;
-        if (t < T) {
-            float s0 = 0.f;
-            for (int i = 0; i < nb; ++i) s0 = __fadd_rn(s0, reinterpret_cast<const float *>(smem + XR_WAVES * XR_STAGE + i * XR_SUMS)[tl * 64 + l]);
-            sl.out[(size_t)t * sl.out_pitch + l] = s0;
         }
     }
 }

@@ -161,5 +161,107 @@ __device__ __forceinline__ void xm_body(const XmSlab &sl, const uint16_t *x, con
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// The same for at most 32 * TB tokens (TB = 1 or 2), where the slab's weights are nearly all a workgroup reads and a
+// compute unit holds one workgroup: what counts is that every compute unit has its requests on their way from the start
+// and keeps them coming.  The staged tokens are the launch's own (the form above stages 128 rows whatever T is), which
+// leaves room for a ring of seven (six) chunks instead of two buffers, and one barrier per chunk.  At 32 tokens
+// (29 MB of weights) the launch takes 12.1 us; with the form above, at most two chunks in flight per compute unit, 14.1.
+// Wave w takes token block w % TB and, of the slab's four blocks of 32 columns, the TB blocks from TB * (w / TB) on.
+template <int TB> constexpr int XMS_CHUNK = XM_W_BYTES + TB * 32 * XM_KC * 2;
+template <int TB> constexpr int XMS_RING = TB == 1 ? 7 : 6;
+template <int TB> constexpr int XMS_LDS = XMS_RING<TB> * XMS_CHUNK<TB>;      // 143 360, 147 456 bytes
+
+template <int TB>
+__device__ __forceinline__ void xm_small_body(const XmSlab &sl, const uint16_t *x, const int T, const int h, const int c_begin, const int c_end,
+                                              uint8_t *smem)
+{
+    static_assert(TB == 1 || TB == 2, "token blocks");
+    constexpr int RING = XMS_RING<TB>, CHUNK = XMS_CHUNK<TB>, PER = 4 + TB;    // requests of a wave per chunk
+    const int l = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tb = w % TB, cb0 = TB * (w / TB);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_byte_t *)smem;
+    const int wrow = l >> 4, wpos = l & 15, xrow = l >> 3, xpos = l & 7;
+    const uint8_t *wreq = sl.w + (size_t)(16 * w + wrow) * sl.pitch + 16 * (wpos ^ (4 * wrow));
+    const uint8_t *xreq[TB];
+#pragma unroll
+    for (int j = 0; j < TB; ++j) {
+        const int tl = 8 * (TB * w + j) + xrow;
+        xreq[j] = reinterpret_cast<const uint8_t *>(x) + (size_t)(tl < T ? tl : T - 1) * h * 2 + 16 * (xpos ^ ((tl >> 1) & 7));
+    }
+    auto request_chunk = [&](const int c, const int buf) {
+        const uint32_t dst = lds0 + (uint32_t)(buf * CHUNK);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dma16(wreq + ((size_t)c * XM_KC + 4 * j) * sl.pitch, dst + 1024u * (4 * w + j));
+#pragma unroll
+        for (int j = 0; j < TB; ++j) dma16(xreq[j] + (size_t)c * (XM_KC * 2), dst + XM_W_BYTES + 1024u * (TB * w + j));
+    };
+    f32x16 acc[TB];
+#pragma unroll
+    for (int i = 0; i < TB; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][r] = 0.f;
+    const int arow = 8 * (l >> 5) + ((l & 15) >> 2), aswz = 4 * ((l & 15) >> 2);
+    uint32_t aoff[TB];
+#pragma unroll
+    for (int i = 0; i < TB; ++i) aoff[i] = (uint32_t)(arow * 256 + 16 * ((4 * (cb0 + i) + 2 * ((l >> 4) & 1) + ((l & 3) >> 1)) ^ aswz) + 8 * (l & 1));
+    const int brow = 32 * tb + (l & 31), bswz = (brow >> 1) & 7;
+    const int n = c_end - c_begin;
+#pragma unroll 1
+    for (int c = 0; c < RING - 1 && c < n; ++c) request_chunk(c_begin + c, c);
+    int buf = 0;
+#pragma unroll 1
+    for (int c = 0; c < n; ++c) {
+        // chunk c has landed when at most the younger chunks' requests are outstanding (uniform)
+        const int younger = n - 1 - c < RING - 2 ? n - 1 - c : RING - 2;
+        switch (younger) {
+        case 5: VM_WAIT(5 * PER); break;
+        case 4: VM_WAIT(4 * PER); break;
+        case 3: VM_WAIT(3 * PER); break;
+        case 2: VM_WAIT(2 * PER); break;
+        case 1: VM_WAIT(PER); break;
+        default: VM_WAIT(0); break;
+        }
+        static_assert(RING <= 7, "the cases above");
+        __syncthreads();                               // every wave's part has landed; every wave is done with chunk c - 1
+        if (c + RING - 1 < n) request_chunk(c_begin + c + RING - 1, buf == 0 ? RING - 1 : buf - 1);
+        const uint8_t *wb = smem + buf * CHUNK;
+        const uint8_t *xb = wb + XM_W_BYTES;
+#pragma unroll
+        for (int ks = 0; ks < XM_KC / 16; ++ks) {
+            const bf16x8 b = *reinterpret_cast<const bf16x8 *>(xb + brow * 128 + 16 * ((2 * ks + (l >> 5)) ^ bswz));
+#pragma unroll
+            for (int i = 0; i < TB; ++i) {
+                const uint16_t *ap = reinterpret_cast<const uint16_t *>(wb + aoff[i] + 16 * ks * 256);
+                const s16x4 lo = lds_read_tr16(ap), hi = lds_read_tr16(ap + 4 * 128);
+                const bf16x8 a = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[i], 0, 0, 0);
+            }
+        }
+        buf = buf + 1 == RING ? 0 : buf + 1;
+    }
+    __syncthreads();                                   // every wave is done with the last chunk: the ring becomes staging areas
+    // 32 tokens x 32 * TB columns per wave leave as whole row segments (as above)
+    constexpr int SPITCH = 128 * TB + 16;
+    uint8_t *stg = smem + w * (32 * SPITCH);
+#pragma unroll
+    for (int i = 0; i < TB; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const f32x4 v = {acc[i][4 * q], acc[i][4 * q + 1], acc[i][4 * q + 2], acc[i][4 * q + 3]};
+            *reinterpret_cast<f32x4 *>(stg + (l & 31) * SPITCH + 16 * (l >> 5) + 128 * i + 32 * q) = v;
+        }
+    // the wave reads back what it wrote itself: LDS operations of a wave stay in order
+    constexpr int LPR = 8 * TB, RPI = 64 / LPR;        // lanes per row, rows per store
+#pragma unroll
+    for (int k = 0; k < 32 / RPI; ++k) {
+        const int r = RPI * k + l / LPR;
+        const f32x4 v = *reinterpret_cast<const f32x4 *>(stg + r * SPITCH + 16 * (l % LPR));
+        const int t = 32 * tb + r;
+        if (t < T) *reinterpret_cast<f32x4 *>(sl.out + (size_t)t * sl.out_pitch + 32 * cb0 + 4 * (l % LPR)) = v;
+    }
+}
+
 }  // namespace
 }  // namespace pto

@@ -218,6 +218,33 @@ def run_fused(dm, dl, t, n, n_idx, op=None):
     return q_nope, q_rope, q_int8, q_scale, weights
 
 
+@pytest.mark.parametrize("t,n_idx", [(9, 64), (32, 8), (33, 64), (64, 64), (65, 16), (130, 64)])
+def test_fused_prolog_fixed_order_sums_at_tile_edges(t, n_idx):
+    """The sums that keep their fixed order while the others run on the matrix cores -- the rope columns of w_dkv_kr, wk
+    and w_proj -- at the edges of the token tiles (32 tokens per job) and of the forms (32, 64 tokens), with 15 blocks
+    of the hidden axis (a second group of seven, so that a wave has one block) and narrow w_proj rows: the rotated key,
+    the indexer's key rows and its weights have the sequential statement's bits; the MLA half meets its rule."""
+    from oracle import lip_oracle as lo
+    from pypto_amd import mla_prolog_quant_impl as impl
+    from pypto_amd.synthetic import gen_indexer_prolog_inputs
+    impl.EXACT_ABSORB = False
+    kw = dict(h=960, q_lora_rank=512)
+    mla = gen_mla_prolog_inputs(1, t, [t + 30], seed=t, n_heads=2, **kw)
+    lip = gen_indexer_prolog_inputs(1, t, [t + 30], seed=t + 1, n_heads=n_idx, **kw)
+    ref = mo.mla_prolog_ref(*mla.input_tensors(), epsilon_cq=1e-5, epsilon_ckv=1e-5)
+    lip.x, lip.cos_idx_rope, lip.sin_idx_rope, lip.k_cache_index = mla.token_x, mla.cos, mla.sin, mla.cache_index
+    want = lo.indexer_prolog_ref(*lip.input_tensors())
+    dm, dl = mla.to(torch.device("cuda:0")), lip.to(torch.device("cuda:0"))
+    weights = run_fused(dm, dl, t, 2, n_idx)[4]
+    rows = mla.cache_index.numpy()
+    assert torch.equal(dm.kr_cache.cpu().reshape(-1, 64)[rows].float(), torch.from_numpy(ref["kr_cache"].reshape(-1, 64)[rows]).float())
+    assert np.array_equal(dl.k_cache.cpu().numpy(), want["k_cache"])
+    assert np.array_equal(dl.k_cache_scale.cpu().numpy().view(np.uint16), want["k_cache_scale"].view(np.uint16))
+    assert np.array_equal(weights.cpu().numpy().view(np.uint16), want["weights"].view(np.uint16))
+    gk, rk = dm.kv_cache.cpu().reshape(-1, 512)[rows].int(), torch.from_numpy(ref["kv_cache"].reshape(-1, 512)[rows]).int()
+    assert (gk - rk).abs().max() <= 1 and (gk != rk).float().mean() <= 0.01
+
+
 @pytest.mark.parametrize("mode,shape", [("default", "small"), ("exact", "small"), ("matrix_cores", "small"), ("default", "t_512"),
                                         ("default", "t_11_idx_64"), ("exact", "t_11_idx_64"), ("default", "t_3_idx_32"),
                                         ("default", "t_40_idx_64"), ("exact", "t_40_idx_64"), ("default", "t_7_idx_64"),
