@@ -88,8 +88,8 @@ void *scratch_of(int dev, hipError_t *err)
 }
 
 struct SfaPlan {
-    int waves;
-    int hgroups;
+    int head_groups;      // groups of 32 heads per workgroup: 1, 2 or 4
+    int hgroups;          // workgroups that share a row's heads
     int nsplit;
     int whole_slots;      // rows 0 .. 8 * whole_slots - 1 are not split
     size_t part_o_bytes;
@@ -122,77 +122,72 @@ int sfa_check(const PtoSfaQuantArgs *a)
 SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
 {
     SfaPlan pl;
-    pl.waves = a->nq > 64 ? 4 : (a->nq > 32 ? 2 : 1);
-    const int heads_per_wg = 32 * pl.waves;
-    pl.hgroups = (int)((a->nq + heads_per_wg - 1) / heads_per_wg);
     const long long rows = a->b * a->s1;
     const int tiles = (int)((a->topk + pto::SFA_KEY_TILE - 1) / pto::SFA_KEY_TILE);
     const int min_split = (int)((a->topk + pto::SFA_MAX_CHUNK - 1) / pto::SFA_MAX_CHUNK);
+    // (a size query on a host without a device plans for the 256 CUs of an MI355X; a launch there fails)
+    const int cus = cu_count() > 0 ? cu_count() : 256;
+    auto shares = [&](const int hg) { return (int)((a->nq + 32 * hg - 1) / (32 * hg)); };
+    auto partial_bytes = [&](const long long r, const int ns) {
+        return ns > 1 ? (size_t)r * ns * a->nq * (512 * sizeof(uint16_t) + 2 * sizeof(float)) : (size_t)0;
+    };
+    // The schedule model, in microseconds: what a launch pair took over 1 to 128 rows x 16 to 128 heads x 1 to 64 splits
+    // (fitted to within 10 %; neighbouring choices differ by less).  A compute unit holds one workgroup; a round of them
+    // is as long as a split's tiles; starting, staging the query and the first tile and the merge launch are `fixed`, and
+    // the partial results cost with the number of workgroups that write them.  Fewer head groups per workgroup make
+    // a tile shorter, and the prologue, but the tiles of a row are de-quantised once per workgroup: that pays while the
+    // chip is not full (128 heads, 1 row: 22.0 us as 16 splits of four groups, 14.3 as 32 splits of one; 4 rows: 22.5, 20.0).
+    auto round_us = [&](const int hg, const int ns) { return (tiles + ns - 1) / ns * (hg == 4 ? 1.75 : (hg == 2 ? 1.58 : 1.47)); };
+    auto tail_us = [&](const int hg, const long long wgs, const int ns) {
+        if (ns == 1) return 6.0;
+        const double fixed = hg == 4 ? 10.5 : (hg == 2 ? 9.5 : 9.3), per_wg = hg == 4 ? 0.045 : (hg == 2 ? 0.032 : 0.018);
+        return fixed + per_wg * (double)wgs + (ns > 8 ? (hg == 1 ? 0.5 : 1.5) : 0.0);       // (more than eight splits: the wide merge)
+    };
+    auto rounds = [&](const long long wgs) { return cus % 8 == 0 ? ((wgs + 7) / 8 + cus / 8 - 1) / (cus / 8) : (wgs + cus - 1) / cus; };
+    const int hg_max = a->nq > 64 ? 4 : (a->nq > 32 ? 2 : 1);
+    pl.head_groups = hg_max;
     int ns = a->num_splits;
+    double best = -1.0;
     if (ns == 0) {
-        // The split count with the shortest schedule.  The workgroups of a row share an XCD (row t on XCD t % 8,
-        // for the row's queries in that XCD's L2) and a compute unit holds one workgroup, so the fullest XCD runs
-        // ceil(its workgroups / its CUs) rounds, each as long as a split's tiles plus the fixed cost of a workgroup
-        // (query staging, row table, first tile, writing the partial results: about five and a half tiles' time;
-        // three when nothing is split); the merge launch costs about a tile plus a tile per hundred partial rows.
-        // Filling every XCD exactly once wins where the batch allows it; a batch that does not divide the CUs
-        // gets fewer, longer splits rather than a second round that is nearly empty, and a batch of more rows
-        // than CUs is split where shorter workgroups fill its last round better (300 rows: three rounds of half
-        // rows instead of two of whole ones).  A split shorter than four tiles is all prologue.
-        // (a size query on a host without a device plans for the 256 CUs of an MI355X; a launch there fails)
-        const int cus = cu_count() > 0 ? cu_count() : 256;
-        const long long xcd_cus = cus / 8 > 0 ? cus / 8 : 1;
-        const long long xcd_rows = (rows + 7) / 8;
-        const int max_split = tiles / 4 > 0 ? tiles / 4 : 1;
-        double best = -1.0;
-        if (cus % 8 != 0) {
-            // not the layout the schedule model describes (a partitioned device, another part): one workgroup per
-            // compute unit, as many splits as that takes
-            const long long per_split = rows * pl.hgroups;
-            ns = (int)((cus + per_split - 1) / per_split);
-            ns = ns > max_split ? max_split : ns;
-            while (ns > 1 && ns > min_split && (size_t)rows * ns * a->nq * (512 * sizeof(uint16_t) + 2 * sizeof(float)) > max_bytes) --ns;
-        }
-        for (int s = 1; s <= max_split && cus % 8 == 0; ++s) {
-            if (s > 1 && s >= min_split && (size_t)rows * s * a->nq * (512 * sizeof(uint16_t) + 2 * sizeof(float)) > max_bytes) break;
-            const long long rounds = (xcd_rows * pl.hgroups * s + xcd_cus - 1) / xcd_cus;
-            const double merge = s == 1 ? 0.0 : 1.0 + 0.01 * (double)rows * s * pl.hgroups;
-            const double cost = (double)rounds * ((tiles + s - 1) / s + (s == 1 ? 3.0 : 5.5)) + merge;
-            if (best < 0.0 || cost < best) {
-                best = cost;
-                ns = s;
+        for (int hg = hg_max; hg >= 1; hg /= 2)
+            // (of the split counts with equally long splits the smallest is the one to take)
+            for (int s = min_split, len = 0; s <= tiles; s = len > 1 ? (tiles + len - 2) / (len - 1) : tiles + 1) {
+                len = (tiles + s - 1) / s;
+                const long long wgs = rows * shares(hg) * s;
+                if (s > min_split && (partial_bytes(rows, s) > max_bytes || wgs > 4ll * cus)) break;
+                const double cost = (double)rounds(wgs) * round_us(hg, s) + tail_us(hg, wgs, s);
+                if (best < 0.0 || cost < best) {
+                    best = cost;
+                    ns = s;
+                    pl.head_groups = hg;
+                }
             }
-        }
     }
     ns = ns < min_split ? min_split : ns;
     ns = ns > tiles ? tiles : ns;
     ns = ns < 1 ? 1 : ns;
+    pl.hgroups = shares(pl.head_groups);
     pl.nsplit = ns;
     pl.whole_slots = 0;
     long long split_rows = rows;
-    if (a->num_splits == 0 && min_split == 1) {
+    if (a->num_splits == 0 && min_split == 1 && cus % 8 == 0) {
         // More rows than compute units: the full rounds of whole rows first, then the rows left over dealt out in
         // as many pieces as fill one more round (300 rows on 256 CUs: 32 whole rows per XCD, the other five or
         // six in five pieces each), where that beats the best uniform split above.
-        const int cus = cu_count() > 0 ? cu_count() : 256;
-        const long long xcd_cus = cus / 8 > 0 ? cus / 8 : 1;
         const long long xcd_rows = (rows + 7) / 8;
-        const long long per_round = cus % 8 == 0 ? xcd_cus / pl.hgroups : 0;   // rows of an XCD that one round holds
+        const long long per_round = cus / 8 / shares(hg_max);                 // rows of an XCD that one round holds
         const long long full = per_round > 0 ? xcd_rows / per_round : 0;
-        const long long rem = per_round > 0 ? xcd_rows - full * per_round : 0;
-        if (full >= 1 && rem >= 1) {
-            int sb = (int)(per_round / rem);
-            const int max_split = tiles / 4 > 0 ? tiles / 4 : 1;
+        const long long rows_b = rows - 8 * full * per_round;                 // rows 8 * whole_slots and up
+        if (full >= 1 && rows_b >= 1) {
+            int sb = (int)(cus / (rows_b * shares(hg_max)));
+            const int max_split = tiles / 4 > 0 ? tiles / 4 : 1;              // (a last round shorter than four tiles is all prologue)
             sb = sb > max_split ? max_split : sb;
-            const long long rows_b = rows - 8 * full * per_round;         // rows 8 * whole_slots and up
-            if (sb >= 2 && rows_b > 0 &&
-                (size_t)rows_b * sb * a->nq * (512 * sizeof(uint16_t) + 2 * sizeof(float)) <= max_bytes) {
-                const double merge = 1.0 + 0.01 * (double)rows_b * sb * pl.hgroups;
-                const double cost = (double)full * (tiles + 3.0) + ((tiles + sb - 1) / sb + 5.5) + merge;
-                const long long rounds_u = (xcd_rows * pl.hgroups * ns + xcd_cus - 1) / xcd_cus;
-                const double cost_u = (double)rounds_u * ((tiles + ns - 1) / ns + (ns == 1 ? 3.0 : 5.5)) +
-                                      (ns == 1 ? 0.0 : 1.0 + 0.01 * (double)rows * ns * pl.hgroups);
-                if (cost < cost_u) {
+            if (sb >= 2 && partial_bytes(rows_b, sb) <= max_bytes) {
+                const double cost = (double)full * round_us(hg_max, 1) + round_us(hg_max, sb) +
+                                    tail_us(hg_max, rows_b * shares(hg_max) * sb, sb);
+                if (cost < best) {
+                    pl.head_groups = hg_max;
+                    pl.hgroups = shares(hg_max);
                     pl.nsplit = sb;
                     pl.whole_slots = (int)(full * per_round);
                     split_rows = rows_b;
@@ -256,7 +251,7 @@ int sfa_enqueue(const PtoSfaQuantArgs *a, const int8_t *kn, int kn_pitch, const 
 {
     if (cu_count() <= 0) return fail(PTO_E_NO_DEVICE, "sfa: no usable device is current");
     const SfaPlan pl = sfa_plan(a, plan_limit);
-    if (((long long)(a->b * a->s1) + 7) / 8 * 8 * pl.hgroups * pl.nsplit > 0x7fffffffll)     // (an upper bound of the grid)
+    if (((long long)(a->b * a->s1) + 7) / 8 * 8 * pl.hgroups * pl.nsplit > 0x7ffffff0ll)     // (an upper bound of the grid)
         return fail(PTO_E_INVALID_ARG, "sfa: rows x head groups x key splits exceeds the largest launch");
     {
         const void *al16[] = {a->query_nope, a->query_rope, kn, kr, ksc, a->attention_out, a->workspace};
@@ -307,7 +302,7 @@ int sfa_enqueue(const PtoSfaQuantArgs *a, const int8_t *kn, int kn_pitch, const 
     p.nsplit = pl.nsplit;
     p.whole_slots = pl.whole_slots;
     p.hgroups = pl.hgroups;
-    p.waves = pl.waves;
+    p.head_groups = pl.head_groups;
     p.scale_log2 = a->softmax_scale * 1.4426950408889634f;
     hipError_t e = pto::sfa_launch(p, static_cast<hipStream_t>(hip_stream));
     if (e == hipErrorNoBinaryForGpu || e == hipErrorInvalidDeviceFunction)

@@ -8,8 +8,9 @@
 // products accumulated in fp32 over 576 dims, softmax runs in fp32, P is rounded to bf16
 // un-normalised, PV accumulates in fp32 over 512 dims and the result is divided by the fp32 row sum.
 //
-// Work decomposition: one workgroup = (query row, group of 32*NW heads, key split).  Each of the NW
-// waves owns 32 heads for both matrix products, so probabilities never leave registers:
+// Work decomposition: one workgroup of four waves = (query row, 32*HG heads, key split).  With HG = 4 each
+// wave owns 32 heads for both matrix products, so probabilities never leave registers (HG = 1 and 2: see the
+// kernel):
 //   S^T[key][head] = K[key][:] . Q^T        v_mfma_f32_32x32x16_bf16, A = K tile rows from LDS,
 //                                            B = Q^T fragments resident in registers
 //   O^T[dv][head] += V^T[dv][key] . P^T     A = V^T read from the same LDS tile with the
@@ -17,7 +18,7 @@
 //                                            accumulator registers of the first product
 // (the accumulator layout of a 32x32 product gives lane (head, half) the keys 8*(r/4)+4*half+r%4;
 // the transposed V read uses the same key order, so no cross-lane movement is needed).
-// All NW waves gather and de-quantise the tile cooperatively: each selected row is read once per
+// All waves gather and de-quantise the tile cooperatively: each selected row is read once per
 // workgroup (512 B int8 + 128 B rope + 16 B scales, from three arrays or from one packed 656-byte row)
 // and written to LDS as 576 bf16.
 #include <type_traits>
@@ -132,9 +133,20 @@ constexpr float RESCALE_TAU = 8.0f;   // log2 units: the reference max moves onl
 
 // QUANT: the latent part of a cache row is int8 with four fp32 scales and is de-quantised on the way into
 // LDS; otherwise it is bf16 already (1024 bytes) and travels cache -> LDS tile directly by LDS-DMA.
-template <int NW, bool QUANT>
-__global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
+// HG: groups of 32 heads in the workgroup, which always has four waves.  With HG = 4 a wave owns its 32 heads.  With fewer
+// groups the SP = 4 / HG waves ("parts") of a group share it: part q takes an SP-th of the score contraction and of the
+// value channels, the partial scores meet in LDS (one more barrier per tile) and every part does the softmax of the
+// group's heads for itself, on the same bits.  Bound by a wave's instruction stream (de-quantisation, LDS accesses), not
+// by the matrix cores: a tile takes 1.47 us with HG = 1, 1.58 with 2, 1.75 with 4.  (One wave per 32 heads and so one or
+// two waves per compute unit, as before: 40 rows x 64 heads over a bf16 cache 41.7 us, now 34.8; 4 rows x 16 heads over
+// 8 K keys 41.8, now 24.0.)
+template <int HG, bool QUANT>
+__global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
 {
+    constexpr int NW = 4;
+    constexpr int SP = NW / HG;
+    constexpr int KSP = KSTEPS / SP;                                   // contraction steps of a part
+    constexpr int DVP = DVB / SP;                                      // value blocks of a part
     // One LDS pool.  Prologue: per-wave query staging regions (QREGION bytes each).  Loop: tile
     // buffers of KT rows -- while tile n is consumed from one, tile n+1 is de-quantised into the other
     // (int8 cache: out of a staging ring of raw rows above the tile buffers, filled by LDS-DMA two tiles
@@ -149,7 +161,8 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
     constexpr int STG_BYTES = STG_NOPE + STG_SCALE + STG_ROPE;
     constexpr int STG_SLOTS = 2;
     constexpr int STG_BASE = TILES_BYTES > WAVE_BYTES ? TILES_BYTES : WAVE_BYTES;   // above everything else in the pool
-    constexpr int POOL_BYTES = STG_BASE + (QUANT ? STG_SLOTS * STG_BYTES : 0);
+    constexpr int XCH_BASE = STG_BASE + (QUANT ? STG_SLOTS * STG_BYTES : 0);        // partial scores, 4 KiB per wave
+    constexpr int POOL_BYTES = XCH_BASE + (SP > 1 ? NW * 4096 : 0);
     static_assert(STG_BASE % 16 == 0 && STG_BYTES % 16 == 0, "LDS-DMA destinations are 16-byte aligned");
     __shared__ __attribute__((aligned(16))) uint16_t pool[POOL_BYTES / 2];
     __shared__ int rows_lds[SFA_MAX_CHUNK + 3 * KT];
@@ -161,26 +174,29 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
     const int l = tid & 63;
     const int half = l >> 5;
     const int col = l & 31;
+    const int hgw = SP == 1 ? w : w % HG;                              // this wave's head group and part
+    const int part = SP == 1 ? 0 : w / HG;
 
-    // Workgroups of one query row share an XCD (consecutive workgroup ids rotate over the 8 XCDs): row t is row
-    // slot t / 8 of XCD t % 8.  The first whole_slots row slots of every XCD are rows taken by one workgroup each
-    // (per head group), the others are split over nsplit workgroups: a launch of more rows than compute units
-    // runs its full rounds of whole rows first and deals the rows left over out in pieces.
+    // Consecutive workgroup ids rotate over the 8 XCDs.  The first whole_slots row slots of every XCD are rows taken by
+    // one workgroup each (per head group), the others are split over nsplit workgroups: a launch of more rows than
+    // compute units runs its full rounds of whole rows first and deals the rows left over out in pieces.  The pieces
+    // are dealt to the XCDs in equal runs of consecutive ones, so that most of a row's workgroups share an XCD (for the
+    // row's queries in its L2) while a launch of a few rows still reaches every XCD.
     const int xcd = blockIdx.x & 7;
     const int slot = blockIdx.x >> 3;
     const int wslots = p.whole_slots * p.hgroups;
-    int rslot, within, nsplit;
+    int t, within, nsplit;
     if (slot < wslots) {
-        rslot = slot / p.hgroups;
-        within = slot - rslot * p.hgroups;
+        t = (slot / p.hgroups) * 8 + xcd;
+        within = slot % p.hgroups;
         nsplit = 1;
     } else {
         const int per_row = p.hgroups * p.nsplit;
-        rslot = p.whole_slots + (slot - wslots) / per_row;
-        within = (slot - wslots) % per_row;
+        const int piece = xcd * p.xcd_pieces + (slot - wslots);
+        t = 8 * p.whole_slots + piece / per_row;
+        within = piece % per_row;
         nsplit = p.nsplit;
     }
-    const int t = rslot * 8 + xcd;
     if (t >= p.T) return;
     const int hg = within / nsplit;
     const int sp = within % nsplit;
@@ -199,7 +215,7 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
         ke = ke > n ? n : ke;
     };
 
-    const int head = hg * (32 * NW) + w * 32 + col;
+    const int head = hg * (32 * HG) + hgw * 32 + col;
     const bool head_ok = head < p.NQ;
 
     // Q^T fragments: lane (head, half) holds q[head][16*ks + 8*half .. +8].  Read straight from global
@@ -211,10 +227,11 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
     // conflict-free.  The cache address is a wave-uniform base plus a per-lane offset.  Heads past NQ
     // read the last head and are never stored.  The second pass stays in flight while the row table
     // below is built.
-    bf16x8 qf[KSTEPS];
+    // (HG < 4: a wave holds a half or a quarter of its heads' fragments only, 18 or 9 loads straight from memory.)
+    bf16x8 qf[KSP];
     uint8_t *const qreg = reinterpret_cast<uint8_t *>(pool) + w * QREGION;
     const uint32_t qdst = (uint32_t)(uintptr_t)(lds_byte_t *)qreg;
-    const int q_head0 = hg * (32 * NW) + w * 32;
+    const int q_head0 = hg * (32 * HG) + hgw * 32;
     auto request_q = [&](const int pass) {
         if (q_head0 + 32 <= p.NQ) {                               // wave-uniform: all 32 heads exist
             const size_t qrow0 = (size_t)t * p.NQ + q_head0;
@@ -250,6 +267,7 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
     };
     // pending: the number of younger requests of this wave that may still be in flight
     auto collect_q = [&](const int pass, auto pending) {
+        if constexpr (SP == 1) {
         __builtin_amdgcn_s_waitcnt(vmcnt_imm(decltype(pending)::value));   // the pass has landed
         asm volatile("" ::: "memory");
 #pragma unroll
@@ -262,6 +280,25 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
         }
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_waitcnt(0xC07F);                       // lgkmcnt(0): the slice may be overwritten
+        }
+    };
+    auto load_q = [&]() {
+        if constexpr (SP > 1) {
+            const size_t row = (size_t)t * p.NQ + (head_ok ? head : p.NQ - 1);
+            const bf16x8 *qn = reinterpret_cast<const bf16x8 *>(p.q_nope + row * DN + 8 * half);
+            const bf16x8 *qr = reinterpret_cast<const bf16x8 *>(p.q_rope + row * DR + 8 * half);
+#pragma unroll
+            for (int i = 0; i < KSP; ++i) {
+                const int ks = part * KSP + i;
+                qf[i] = *(ks < DN / 16 ? qn + 2 * ks : qr + 2 * (ks - DN / 16));
+            }
+        }
+    };
+    auto land_q = [&]() {
+        if constexpr (SP > 1) {
+#pragma unroll
+            for (int i = 0; i < KSP; ++i) asm volatile("" : "+v"(qf[i]));
+        }
     };
     // logical position -> physical cache row for this split's keys.  The table is padded to an even
     // number of tiles plus two with the row of the split's first key: keys past k_end are then loaded
@@ -302,7 +339,8 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
     const int nv_s = ke_s - kb_s;
     const bool fast_s = nv_s > 0 && padded(nv_s) <= FAST_ENTRIES;              // uniform
     if (fast_s) request_positions(kb_s, nv_s);
-    request_q(0);                                                             // 16 requests
+    if constexpr (SP == 1) request_q(0);                                      // 16 requests
+    else load_q();
     int cur = act_b - p.S1 + 1 + s1i;
     cur = cur < 0 ? 0 : (cur > p.topk ? p.topk : cur);
     int k_begin, k_end;
@@ -313,7 +351,8 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
     const bool as_assumed = fast_s && k_begin == kb_s && n_valid == nv_s;     // uniform
     if (fast) {
         if (as_assumed) {
-            __builtin_amdgcn_s_waitcnt(vmcnt_imm(16));                        // the positions have landed
+            land_q();
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(SP == 1 ? 16 : 0));          // the positions have landed
         } else {
             request_positions(k_begin, n_valid);
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
@@ -329,9 +368,9 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
     } else {
         collect_q(0, std::integral_constant<int, 0>{});
     }
-    request_q(1);                                                             // 20 requests
+    if constexpr (SP == 1) request_q(1);                                      // 20 requests
     if (fast) {
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(20));                            // the pages have landed
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(SP == 1 ? 20 : 0));              // the pages have landed
         asm volatile("" ::: "memory");
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -347,10 +386,10 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
 
     // the first tile's products start the accumulators from zero (acc_mfma_first); they are cleared beforehand
     // only when there is no first tile
-    f32x16 o[DVB];
+    f32x16 o[DVP];
     if (k_begin >= k_end) {
 #pragma unroll
-        for (int i = 0; i < DVB; ++i)
+        for (int i = 0; i < DVP; ++i)
 #pragma unroll
             for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
         valu_to_mfma_fence();
@@ -597,6 +636,7 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
     } else {
         collect_q(1, std::integral_constant<int, 0>{});
     }
+    land_q();
     __syncthreads();                       // every wave holds its Q^T fragments: the tile buffers are free
     if (n_valid > 0) {
         if (QUANT) {
@@ -621,7 +661,7 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
     if (sc_log2 < 0.f) {
         sc_log2 = -sc_log2;
 #pragma unroll
-        for (int i = 0; i < KSTEPS; ++i) {
+        for (int i = 0; i < KSP; ++i) {
             u32x4 v = __builtin_bit_cast(u32x4, qf[i]);
             v ^= 0x80008000u;
             qf[i] = __builtin_bit_cast(bf16x8, v);
@@ -639,22 +679,46 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
         // ---- S^T = K . Q^T, LDS reads running one group of four contraction steps ahead
         f32x16 s;
         {
-            const uint16_t *arow = cur_tile + tile_row_of(col) * PITCH + 8 * half;
+            const uint16_t *arow = cur_tile + tile_row_of(col) * PITCH + 8 * half + part * (16 * KSP);
             // operand reads run four products ahead, in a ring of eight fragments
             bf16x8 fa[8];
 #pragma unroll
             for (int e = 0; e < 4; ++e) fa[e] = *reinterpret_cast<const bf16x8 *>(arow + 16 * e);
 #pragma unroll
-            for (int m = 0; m < KSTEPS; ++m) {
+            for (int m = 0; m < KSP; ++m) {
                 if (m == 0) s_mfma_first(s, fa[0], qf[0]);
                 else s_mfma(s, fa[m & 7], qf[m]);
                 __builtin_amdgcn_sched_barrier(0);          // the product leads its slot
-                if (m + 4 < KSTEPS) fa[(m + 4) & 7] = *reinterpret_cast<const bf16x8 *>(arow + 16 * (m + 4));
-                slot_work(m, (it + 1) & 1, (it + 1) & 1, kt + 2 * KT, it & 1);
+                if (m + 4 < KSP) fa[(m + 4) & 7] = *reinterpret_cast<const bf16x8 *>(arow + 16 * (m + 4));
+#pragma unroll
+                for (int j = 0; j < SP; ++j) slot_work(SP * m + j, (it + 1) & 1, (it + 1) & 1, kt + 2 * KT, it & 1);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
         s_chain_done(s);
+        if constexpr (SP > 1) {
+            // the parts' scores meet: own + neighbour's (+ the other pair's sum), the same bits in every part
+            uint8_t *const xch = pool_b + XCH_BASE + 16 * l;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const f32x4 v = {s[4 * j], s[4 * j + 1], s[4 * j + 2], s[4 * j + 3]};
+                *reinterpret_cast<f32x4 *>(xch + (w * 4 + j) * 1024) = v;
+            }
+            __syncthreads();
+            auto theirs = [&](const int q, const int j) { return *reinterpret_cast<const f32x4 *>(xch + ((q * HG + hgw) * 4 + j) * 1024); };
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const f32x4 a = theirs(part ^ 1, j);
+                f32x4 b = {0.f, 0.f, 0.f, 0.f};
+                if (SP == 4) {
+                    const f32x4 c = theirs(part ^ 2, j), d = theirs(part ^ 3, j);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) b[e] = c[e] + d[e];
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[4 * j + e] = SP == 4 ? (s[4 * j + e] + a[e]) + b[e] : s[4 * j + e] + a[e];
+            }
+        }
 
         // ---- online softmax; lane (head, half) holds keys kt + 8*(r/4) + 4*half + r%4
         float mx = -INFINITY;
@@ -689,7 +753,7 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
         m_run = m_new;
         if (!FIRST && __builtin_expect(__any(rescale), 0)) {     // rare: laid out away from the loop body
             mfma_to_valu_fence();
-            AccLoop<0, DVB>::scale(o, alpha);
+            AccLoop<0, DVP>::scale(o, alpha);
             valu_to_mfma_fence();
         }
         // P^T of the first sixteen keys is packed here; the exponentials of the other sixteen (needed by the
@@ -715,7 +779,7 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
         // ---- O^T += V^T . P^T: product mp = 16*kk + dvb, V^T reads four products ahead in a ring of eight;
         // each product carries its share of the work for the following tiles (slot_work)
         {
-            const uint16_t *vbase = cur_tile + (half + 4 * ((l & 15) >> 2)) * PITCH + 16 * ((l >> 4) & 1) + 4 * (l & 3);
+            const uint16_t *vbase = cur_tile + (half + 4 * ((l & 15) >> 2)) * PITCH + 16 * ((l >> 4) & 1) + 4 * (l & 3) + part * (32 * DVP);
             s16x4 va[8][2];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -723,19 +787,22 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
                 va[e][1] = lds_read_tr16(vbase + 32 * e + 2 * PITCH);
             }
 #pragma unroll
-            for (int mp = 0; mp < 2 * DVB; ++mp) {
+            for (int mp = 0; mp < 2 * DVP; ++mp) {
                 const s16x8 a = __builtin_shufflevector(va[mp & 7][0], va[mp & 7][1], 0, 1, 2, 3, 4, 5, 6, 7);
-                if (FIRST && mp < DVB) acc_mfma_first(o[mp], __builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, pk0));
-                else acc_mfma(o[mp & 15], __builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, mp < DVB ? pk0 : pk1));
+                if (FIRST && mp < DVP) acc_mfma_first(o[mp], __builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, pk0));
+                else acc_mfma(o[mp % DVP], __builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, mp < DVP ? pk0 : pk1));
                 __builtin_amdgcn_sched_barrier(0);          // the product leads its slot
-                if (mp + 4 < 2 * DVB) {
+                if (mp + 4 < 2 * DVP) {
                     const int m2 = mp + 4;
-                    const uint16_t *a0 = vbase + (16 * (m2 >> 4)) * PITCH + 32 * (m2 & 15);
+                    const uint16_t *a0 = vbase + (16 * (m2 / DVP)) * PITCH + 32 * (m2 % DVP);
                     va[m2 & 7][0] = lds_read_tr16(a0);
                     va[m2 & 7][1] = lds_read_tr16(a0 + 2 * PITCH);
                 }
-                softmax_slice(mp);
-                slot_work(KSTEPS + mp, (it + 1) & 1, (it + 1) & 1, kt + 2 * KT, it & 1);
+#pragma unroll
+                for (int j = 0; j < SP; ++j) {              // (complete before product DVP takes the other half of P^T)
+                    softmax_slice(SP * mp + j);
+                    slot_work(KSTEPS + SP * mp + j, (it + 1) & 1, (it + 1) & 1, kt + 2 * KT, it & 1);
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -743,17 +810,17 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
         __syncthreads();
     };
     {
-        // an odd number of tiles is rounded up: the extra tile holds padding rows only, all of them masked
         if (k_begin < k_end) {
             tile_step(std::integral_constant<int, 0>{}, std::true_type{}, k_begin);
-            tile_step(std::integral_constant<int, 1>{}, std::false_type{}, k_begin + KT);
+            if (k_begin + KT < k_end) tile_step(std::integral_constant<int, 1>{}, std::false_type{}, k_begin + KT);
         }
         for (int kt = k_begin + 2 * KT; kt < k_end; kt += 2 * KT) {
             tile_step(std::integral_constant<int, 0>{}, std::false_type{}, kt);
+            if (kt + KT >= k_end) break;
             tile_step(std::integral_constant<int, 1>{}, std::false_type{}, kt + KT);
         }
     }
-    __builtin_amdgcn_s_waitcnt(0x0F70);                 // the padding tiles' requests have landed: the pool is quiet
+    __builtin_amdgcn_s_waitcnt(0x0F70);                 // requests for tiles past the last have landed: the pool is quiet
 
     // ---- epilogue.  Lane (head, half) holds value channels 32*dvb + 8*(r/4) + 4*half + r%4 of its head;
     // written from there each store instruction would touch 32 rows with 8 bytes each.  Each wave
@@ -766,7 +833,7 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
         // of head h is stored at chunk c ^ h: the column-wise writes (32 heads, one chunk) and the
         // row-wise reads (two heads, 16 even or odd chunks each) both touch every bank once.
         uint8_t *stage = reinterpret_cast<uint8_t *>(pool) + w * (32 * 256);
-        const int head_base = hg * (32 * NW) + w * 32;
+        const int head_base = hg * (32 * HG) + hgw * 32;
         const size_t prow_base = ((size_t)(t - 8 * p.whole_slots) * nsplit + sp) * p.NQ;    // split rows only
         const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
         // FINAL: bf16 result rows; otherwise fp16 partial of a key split (O / l of the split, merged by
@@ -778,10 +845,10 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
             constexpr bool FINAL = decltype(final_tag)::value;
             constexpr bool ALL = decltype(all_tag)::value;
             const int hsub = l >> 4, j = l & 15;          // on the way out: head 4*e + hsub, channels 8*j .. 8*j+7
-            uint16_t *dst0 = FINAL ? p.out + ((size_t)t * p.NQ + head_base + hsub) * DN + 8 * j
-                                   : p.part_o + (prow_base + head_base + hsub) * DN + 8 * j;
+            uint16_t *dst0 = FINAL ? p.out + ((size_t)t * p.NQ + head_base + hsub) * DN + part * (32 * DVP) + 8 * j
+                                   : p.part_o + (prow_base + head_base + hsub) * DN + part * (32 * DVP) + 8 * j;
 #pragma unroll
-            for (int gq = 0; gq < DVB / 4; ++gq) {
+            for (int gq = 0; gq < DVP / 4; ++gq) {
 #pragma unroll
                 for (int b4 = 0; b4 < 4; ++b4)
 #pragma unroll
@@ -832,7 +899,7 @@ __global__ __launch_bounds__(NW * 64) void sfa_decode_kernel(const SfaParams p)
             if (all_heads) drain(std::false_type{}, std::true_type{});
             else drain(std::false_type{}, std::false_type{});
         }
-        if (nsplit > 1 && half == 0 && head_ok) {
+        if (nsplit > 1 && part == 0 && half == 0 && head_ok) {
             p.part_ml[(prow_base + head) * 2] = m_run;
             p.part_ml[(prow_base + head) * 2 + 1] = l_run;
         }
@@ -888,56 +955,78 @@ __global__ __launch_bounds__(256) void sfa_combine_kernel(const SfaParams p)
     *reinterpret_cast<u32x4 *>(p.out + ((size_t)t_first * p.NQ + th) * DN + 8 * lane) = outv;
 }
 
-// The same merge for any number of splits, eight at a time (rows with more than eight key splits).
-__global__ __launch_bounds__(256) void sfa_combine_many_kernel(const SfaParams p)
+// The same merge for more than eight splits: a workgroup of four waves per (row, head), wave w takes splits w, w + 4, ..,
+// NS of them in flight at a time (NS = 4: up to 16 splits in one round, 8: up to 32, further rounds beyond), and the four
+// partial merges meet in LDS.
+template <int NS>
+__global__ __launch_bounds__(256) void sfa_combine_wide_kernel(const SfaParams p)
 {
-    constexpr int NS = 8;
-    const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ float acc_lds[4][DN];
+    __shared__ float ml_lds[4][2];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int t_first = 8 * p.whole_slots;                         // the split rows are rows t_first and up
-    const size_t total = (size_t)(p.T - t_first) * p.NQ * (DN / 8);
-    if (gid >= total) return;
-    const int c8 = (int)(gid % (DN / 8));
-    const size_t th = gid / (DN / 8);
-    const int head = (int)(th % p.NQ);
-    const int ts = (int)(th / p.NQ);
-    const int t = t_first + ts;
+    const int th = (int)blockIdx.x;
+    const int ts = th / p.NQ, head = th - ts * p.NQ;
     const size_t prow0 = (size_t)ts * p.nsplit * p.NQ + head;      // split s: prow0 + s * NQ
     const f32x2 *ml = reinterpret_cast<const f32x2 *>(p.part_ml);
-
-    float m = -INFINITY;
-    for (int s0 = 0; s0 < p.nsplit; s0 += NS) {
-        f32x2 v[NS];
-#pragma unroll
-        for (int e = 0; e < NS; ++e) v[e] = ml[prow0 + (size_t)(s0 + e < p.nsplit ? s0 + e : p.nsplit - 1) * p.NQ];
-#pragma unroll
-        for (int e = 0; e < NS; ++e)
-            if (v[e][1] > 0.f) m = fmaxf(m, v[e][0]);
-    }
+    float m = -INFINITY, wsum = 0.f;
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    float wsum = 0.f;
-    for (int s0 = 0; s0 < p.nsplit; s0 += NS) {
+    for (int s0 = w; s0 < p.nsplit; s0 += 4 * NS) {
         f32x2 v[NS];
         f16x8 hv[NS];
 #pragma unroll
         for (int e = 0; e < NS; ++e) {
-            const size_t prow = prow0 + (size_t)(s0 + e < p.nsplit ? s0 + e : p.nsplit - 1) * p.NQ;
+            const size_t prow = prow0 + (size_t)(s0 + 4 * e < p.nsplit ? s0 + 4 * e : s0) * p.NQ;
             v[e] = ml[prow];
-            hv[e] = *reinterpret_cast<const f16x8 *>(p.part_o + prow * DN + 8 * c8);
+            hv[e] = *reinterpret_cast<const f16x8 *>(p.part_o + prow * DN + 8 * lane);
         }
+        float mn = m;
+#pragma unroll
+        for (int e = 0; e < NS; ++e)
+            if (s0 + 4 * e < p.nsplit && v[e][1] > 0.f) mn = fmaxf(mn, v[e][0]);
+        const float scale = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
+        wsum *= scale;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) acc[c] *= scale;
 #pragma unroll
         for (int e = 0; e < NS; ++e) {
-            const bool live = s0 + e < p.nsplit && v[e][1] > 0.f;
-            const float wgt = live ? v[e][1] * __builtin_amdgcn_exp2f(v[e][0] - m) : 0.f;
+            const bool live = s0 + 4 * e < p.nsplit && v[e][1] > 0.f;
+            const float wgt = live ? v[e][1] * __builtin_amdgcn_exp2f(v[e][0] - mn) : 0.f;
 #pragma unroll
             for (int c = 0; c < 8; ++c) acc[c] += wgt * (float)hv[e][c];
             wsum += wgt;
         }
+        m = mn;
     }
-    const float inv = wsum > 0.f ? 1.0f / wsum : 0.f;
-    u32x4 outv;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) outv[e] = pack_bf16x2(acc[2 * e] * inv, acc[2 * e + 1] * inv);
-    *reinterpret_cast<u32x4 *>(p.out + ((size_t)t * p.NQ + head) * DN + 8 * c8) = outv;
+    for (int q = 0; q < 2; ++q) {
+        const f32x4 v = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+        *reinterpret_cast<f32x4 *>(&acc_lds[w][4 * (lane + 64 * q)]) = v;
+    }
+    if (lane == 0) {
+        ml_lds[w][0] = m;
+        ml_lds[w][1] = wsum;
+    }
+    __syncthreads();
+    // thread i: channels 2i, 2i + 1; channel 8*lane + 4*q + j lies at 4*(lane + 64*q) + j
+    const int c = 2 * (int)threadIdx.x;
+    const int at = 4 * ((c >> 3) + 64 * ((c >> 2) & 1)) + (c & 3);
+    float mm = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (ml_lds[e][1] > 0.f) mm = fmaxf(mm, ml_lds[e][0]);
+    float a0 = 0.f, a1 = 0.f, ws = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float f = ml_lds[e][1] > 0.f ? __builtin_amdgcn_exp2f(ml_lds[e][0] - mm) : 0.f;
+        const f32x2 v = *reinterpret_cast<const f32x2 *>(&acc_lds[e][at]);
+        a0 += f * v[0];
+        a1 += f * v[1];
+        ws += f * ml_lds[e][1];
+    }
+    const float inv = ws > 0.f ? 1.0f / ws : 0.f;
+    *reinterpret_cast<uint32_t *>(p.out + ((size_t)t_first * p.NQ + th) * DN + c) = pack_bf16x2(a0 * inv, a1 * inv);
 }
 
 // De-quantises whole cache rows once: out[row][c] = bf16_rne(float(int8) * scale[c / 128]), the values the attention
@@ -960,30 +1049,28 @@ __global__ __launch_bounds__(256) void sfa_dequant_cache_kernel(const int8_t *kn
 
 }  // namespace
 
-hipError_t sfa_launch(const SfaParams &p, hipStream_t stream)
+hipError_t sfa_launch(const SfaParams &pa, hipStream_t stream)
 {
-    const int rslots = (p.T + 7) / 8;                      // row slots per XCD
-    const unsigned grid = (unsigned)(8 * p.hgroups * (p.whole_slots + (rslots - p.whole_slots) * p.nsplit));
-    if (p.kn_bf16) {
-        switch (p.waves) {
-        case 1: hipLaunchKernelGGL((sfa_decode_kernel<1, false>), dim3(grid), dim3(64), 0, stream, p); break;
-        case 2: hipLaunchKernelGGL((sfa_decode_kernel<2, false>), dim3(grid), dim3(128), 0, stream, p); break;
-        default: hipLaunchKernelGGL((sfa_decode_kernel<4, false>), dim3(grid), dim3(256), 0, stream, p); break;
-        }
-    } else {
-        switch (p.waves) {
-        case 1: hipLaunchKernelGGL((sfa_decode_kernel<1, true>), dim3(grid), dim3(64), 0, stream, p); break;
-        case 2: hipLaunchKernelGGL((sfa_decode_kernel<2, true>), dim3(grid), dim3(128), 0, stream, p); break;
-        default: hipLaunchKernelGGL((sfa_decode_kernel<4, true>), dim3(grid), dim3(256), 0, stream, p); break;
-        }
+    SfaParams p = pa;
+    if (p.nsplit == 1) p.whole_slots = (p.T + 7) / 8;
+    const int split_rows = p.T > 8 * p.whole_slots ? p.T - 8 * p.whole_slots : 0;
+    p.xcd_pieces = (int)(((long long)split_rows * p.hgroups * p.nsplit + 7) / 8);
+    const unsigned grid = (unsigned)(8 * (p.hgroups * p.whole_slots + p.xcd_pieces));
+#define SFA_LAUNCH(Q)                                                                                                       \
+    switch (p.head_groups) {                                                                                                \
+    case 1: hipLaunchKernelGGL((sfa_decode_kernel<1, Q>), dim3(grid), dim3(256), 0, stream, p); break;                      \
+    case 2: hipLaunchKernelGGL((sfa_decode_kernel<2, Q>), dim3(grid), dim3(256), 0, stream, p); break;                      \
+    default: hipLaunchKernelGGL((sfa_decode_kernel<4, Q>), dim3(grid), dim3(256), 0, stream, p); break;                     \
     }
+    if (p.kn_bf16) { SFA_LAUNCH(false) } else { SFA_LAUNCH(true) }
+#undef SFA_LAUNCH
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (p.nsplit > 1 && p.T > 8 * p.whole_slots) {
         const int n_th = (p.T - 8 * p.whole_slots) * p.NQ;
         if (p.nsplit > 8) {
-            const size_t total = (size_t)n_th * (DN / 8);
-            hipLaunchKernelGGL(sfa_combine_many_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, p);
+            if (p.nsplit <= 16) hipLaunchKernelGGL(sfa_combine_wide_kernel<4>, dim3((unsigned)n_th), dim3(256), 0, stream, p);
+            else hipLaunchKernelGGL(sfa_combine_wide_kernel<8>, dim3((unsigned)n_th), dim3(256), 0, stream, p);
         } else {
             // one wave per (row, head), four waves per workgroup
             const dim3 cgrid((unsigned)((n_th + 3) / 4));

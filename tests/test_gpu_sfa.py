@@ -105,6 +105,23 @@ def test_key_splits_agree_with_single_workgroup(splits):
     assert max_abs <= 2 ** -6
 
 
+@pytest.mark.parametrize("n_q", [1, 16, 32, 33, 64, 65, 96, 128])
+@pytest.mark.parametrize("splits", [0, 1, 3, 9, 20, 40])
+def test_head_groups_and_odd_tile_counts(n_q, splits):
+    """One, two and four groups of 32 heads per workgroup (the library's own choice: small batches take fewer), splits of
+    odd and even numbers of tiles, empty splits, both merge kernels; the bf16 cache gives the int8 cache's bits."""
+    from oracle import sfa_oracle as so
+    inp = gen_sfa_inputs(2, 2, n_q, [1500, 33], topk=1280, seed=n_q + splits)
+    out = run_op(inp, num_splits=splits)
+    check(out, oracle(inp), f"nq={n_q} splits={splits}")
+    d = inp.to(torch.device("cuda:0"))
+    out_bf = torch.full_like(out, float("nan"), device="cuda:0")
+    impl._launch(d.query_nope, d.query_rope, so.dequant_kn(inp.key_nope_2d, inp.k_nope_scales).cuda(), d.key_rope_2d, None,
+                 d.topk_indices, d.block_table, d.kv_act_seqs, out_bf, n_q, 1, inp.softmax_scale, inp.topk, inp.block_size,
+                 inp.max_blocknum_perbatch, num_splits=splits)
+    assert torch.equal(out_bf.cpu().view(torch.int16), out.view(torch.int16))
+
+
 @pytest.mark.parametrize("b", [20, 44])
 def test_batches_that_do_not_divide_the_compute_units(b):
     """Batches whose rows do not spread evenly over the eight XCDs (20 rows: three on some, two on others; 44: six and
