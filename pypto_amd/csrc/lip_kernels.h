@@ -56,6 +56,7 @@ __host__ __device__ inline bool lip_q_on_matrix_cores(const LipParams &p)
 {
     return p.T >= LIP_MFMA_MIN_TOKENS && p.sum_mode != LIP_SUMS_EXACT;
 }
+// (those rows are finished where the projection makes them: prolog_prefill.h)
 // the hidden-axis form needs w_proj rows made of whole 16-byte pieces
 __host__ __device__ inline bool lip_x_on_matrix_cores(const LipParams &p)
 {

@@ -32,13 +32,13 @@
 // From LIP_MFMA_MIN_TOKENS tokens on (prefill chunks) the stages take forms of their own (LipParams::sum_mode says
 // which sums may leave their fixed order):
 //   lip_qproj_prefill_kernel, lip_qproj_prefill256_kernel   the query projection unsplit (prolog_common.h), a
-//                       workgroup per 128 x 128 or 256 x 256 tile over the whole reduction axis; exact.
+//                       workgroup per 128 x 128 or 256 x 256 tile over the whole reduction axis; exact.  Only where every
+//                       sum is to keep its fixed order: otherwise the query rows are finished where the projection makes
+//                       them, the Hadamard sums on the matrix cores, in one launch with the key rows and weights
+//                       (prolog_prefill.h).
 //   lip_xlinear_group_kernel   the fixed-order sums over the hidden axis on the matrix cores, one hidden row per
 //                       instruction (xlinear_fixed.h); or
 //   lip_xlinear_mfma_kernel    the same sums on the matrix cores (xlinear_mfma.h), if asked for.
-//   lip_finish_query_prefill_kernel   query rows with the Hadamard sums on the matrix cores, 32 rows per pass of a
-//                       wave (prolog_finish.h), unless every sum is to keep its fixed order.
-//   lip_finish_tokens_prefill_kernel  key rows and weights, eight tokens per workgroup.
 #include "lip_kernels.h"
 #include "prolog_common.h"
 #include "prolog_finish.h"
@@ -127,22 +127,10 @@ __global__ __launch_bounds__(256) void lip_xlinear_mfma_kernel(const LipParams p
     xm_body(sl, p.x, p.T, p.h, t0, (int)((long long)sp * nchunks / nsplit), (int)((long long)(sp + 1) * nchunks / nsplit), smem);
 }
 
-__global__ __launch_bounds__(64 * QFP_WAVES) void lip_finish_query_prefill_kernel(const LipParams p)
-{
-    __shared__ __attribute__((aligned(16))) uint8_t lds[LIP_QFP_LDS];
-    lip_finish_query_prefill_body(p, (int)blockIdx.x, (int)gridDim.x, lds);
-}
-
 __global__ __launch_bounds__(512) void lip_qproj_prefill256_kernel(const QProj p, const int njobs)
 {
     __shared__ __attribute__((aligned(16))) uint8_t lds[QP2_LDS];
     q_prefill256_body(p, q_prefill_job_of((int)blockIdx.x, njobs), lds);
-}
-
-__global__ __launch_bounds__(64 * FIN_WAVES) void lip_finish_tokens_prefill_kernel(const LipParams p)
-{
-    __shared__ __attribute__((aligned(16))) uint8_t lds[LIP_FINT_LDS];
-    lip_finish_tokens_prefill_body(p, (int)blockIdx.x, lds);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -165,7 +153,9 @@ hipError_t lip_launch_linear(const LipParams &p, hipStream_t stream)
     const int tblocks = (p.T + 31) / 32;
     const bool unsplit = qproj_splits(p.T) == 1;      // prefill sizes: the query projection as a launch of its own
     const int q_jobs = unsplit ? 0 : p.n_heads * LIP_KSPLIT * tblocks;
-    if (unsplit) {
+    if (unsplit && lip_q_on_matrix_cores(p)) {
+        if (x_done) return hipSuccess;                // the projection is part of the last launch
+    } else if (unsplit) {
         if (p.q_lora % (32 * QPF_STEPS)) return hipErrorInvalidValue;
         const QProj qp = {p.q_norm, p.w_qb, p.qpart, p.T, p.q_lora, p.n_heads, p.q_norm_scale, p.w_qb_scale};
         const int cus = cu_count();
@@ -225,22 +215,8 @@ hipError_t lip_launch(const LipParams &p, hipStream_t stream)
 
 hipError_t lip_launch_finish(const LipParams &p, hipStream_t stream)
 {
+    if (lip_q_on_matrix_cores(p)) return prolog_prefill_launch(nullptr, &p, stream);
     const int q_wgs = lip_finish_query_wgs(p);
-    if (lip_q_on_matrix_cores(p)) {
-        // the query rows on the matrix cores, in passes of 32 rows per wave, as many workgroups as are resident at once
-        const int npass = (p.T * p.n_heads + 31) / 32;
-        const int cus = cu_count();
-        if (cus <= 0) return hipErrorNoDevice;
-        int wgs = (npass + QFP_WAVES - 1) / QFP_WAVES;
-        const int resident = cus * (160 * 1024 / LIP_QFP_LDS);
-        wgs = wgs > resident ? resident : wgs;
-        hipLaunchKernelGGL(lip_finish_query_prefill_kernel, dim3((unsigned)wgs), dim3(64 * QFP_WAVES), 0, stream, p);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        // key rows and weights: eight tokens per workgroup
-        hipLaunchKernelGGL(lip_finish_tokens_prefill_kernel, dim3((unsigned)((p.T + FIN_WAVES - 1) / FIN_WAVES)), dim3(64 * FIN_WAVES), 0, stream, p);
-        return hipGetLastError();
-    }
     hipLaunchKernelGGL(lip_finish_kernel, dim3((unsigned)(q_wgs + p.T)), dim3(64 * FIN_WAVES), 0, stream, p, q_wgs);
     return hipGetLastError();
 }

@@ -33,10 +33,13 @@
 //                        axis, v_mfma_f32_32x32x16_bf16 with the row-major weight chunk as the transposed operand.
 //                        The launch's last workgroups take the 64 rope columns of w_dkv_kr in their fixed order
 //                        instead (the rotated key allows no outlier under the reference's acceptance rule).
-//   qproj_prefill_kernel, qproj_prefill256_kernel   the projection unsplit (prolog_common.h), a workgroup per
-//                        128 x 128 or 256 x 256 tile over the whole reduction axis; results leave de-quantised.
+//   mlap_mid_prefill_kernel    the middle stage as a wave per token and latent (64 tokens and more)
+//   qproj_prefill_kernel   the projection unsplit (prolog_common.h), a workgroup per tile over the whole reduction axis;
+//                        results leave de-quantised (up to 63 tokens, and in the fixed-order mode, which has
+//                        qproj_prefill256_kernel for more).
 //   mlap_finish_prefill_kernel   per (head, run of 32-token blocks): the head's whole w_uk staged once
-//                        (prolog_finish.h), absorb product on the matrix cores.
+//                        (prolog_finish.h), absorb product on the matrix cores (up to 63 tokens).
+// From 64 tokens on the projection and the last stage are one launch (prolog_prefill.h).
 #include <cstring>
 
 #include "mlap_kernels.h"
@@ -105,8 +108,9 @@ static_assert(XM_KC == MLAP_XBLOCK, "the workspace is sized in chunks of the hid
 // and, in the fused prolog from 64 tokens on, the indexer prolog's wk and w_proj.  They are short and follow the long workgroups of the
 // other slabs, so they fill the launch's last round; two workgroups fit a compute unit.  (1000 tokens: 69 us here and 79
 // in a launch of the indexer's own before they shared it.)
-// TB: at most 32 * TB tokens (xm_small_body), 0 for more.
-template <int TB> constexpr int XM_FORM_LDS = TB == 0 ? XM_LDS : XMS_LDS<TB == 0 ? 1 : TB>;
+// TB: at most 32 * TB tokens (xm_small_body), 0 for tiles of 128 tokens (xm_body), XM_BIG for tiles of 256 (xb_body).
+constexpr int XM_BIG = 8;
+template <int TB> constexpr int XM_FORM_LDS = TB == 0 ? XM_LDS : (TB == XM_BIG ? XB_LDS : XMS_LDS<TB == 1 ? 1 : 2>);
 template <int TB> constexpr int XM_KERNEL_LDS = XM_FORM_LDS<TB> > XF_LDS ? XM_FORM_LDS<TB> : XF_LDS;
 static_assert(2 * XM_KERNEL_LDS<0> <= 160 * 1024, "two workgroups share a compute unit");
 template <int TB>
@@ -132,6 +136,25 @@ __global__ __launch_bounds__(256) void mlap_xlinear_mfma_kernel(const MlapParams
         return;
     }
     const int bid = (int)blockIdx.x;
+    if constexpr (TB == XM_BIG) {
+        // every XCD takes a run of the jobs in the order (range of h, token tile, slab): a range's weights and the hidden
+        // states of a tile or two cross into its L2 once, chunk by chunk, as the run's workgroups walk the range together
+        const int ttiles = (p.T + XB_TOK - 1) / XB_TOK;
+        const int idx = (bid & 7) * (own_wgs >> 3) + (bid >> 3);
+        if (idx >= nslabs * ttiles * nsplit) return;
+        const int slab = idx % nslabs, sp = (idx / nslabs) / ttiles, t0 = ((idx / nslabs) % ttiles) * XB_TOK;
+        const int qslabs = p.q_lora / 128;
+        const int nc = p.q_lora + MLAP_KV + MLAP_ROPE;
+        XmSlab sl;
+        sl.w = slab < qslabs ? reinterpret_cast<const uint8_t *>(p.w_dq) + slab * 256 : reinterpret_cast<const uint8_t *>(p.w_dkvkr) + (slab - qslabs) * 256;
+        sl.pitch = (slab < qslabs ? p.q_lora : MLAP_KV + MLAP_ROPE) * 2;
+        sl.pieces = 16;
+        sl.out = p.xpart + (size_t)sp * p.T * nc + slab * 128;
+        sl.out_pitch = nc;
+        const int nchunks = p.h / XB_KC;
+        xb_body(sl, p.x, p.T, p.h, t0, (int)((long long)sp * nchunks / nsplit), (int)((long long)(sp + 1) * nchunks / nsplit), smem);
+        return;
+    } else {
     // Workgroups go round the eight XCDs, each with an L2 of its own, and the working set (hidden states + weights)
     // is several times one L2: the jobs of a slab (its ranges of h x token tiles) all run on XCD slab % 8, so a slab's
     // weights cross into one L2 only and every XCD reads the hidden states once for its two or so slabs.  The slabs
@@ -164,6 +187,7 @@ __global__ __launch_bounds__(256) void mlap_xlinear_mfma_kernel(const MlapParams
     const int c_begin = (int)((long long)sp * nchunks / nsplit), c_end = (int)((long long)(sp + 1) * nchunks / nsplit);
     if constexpr (TB == 0) xm_body(sl, p.x, p.T, p.h, t0, c_begin, c_end, smem);
     else xm_small_body<TB>(sl, p.x, p.T, p.h, c_begin, c_end, smem);
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -274,6 +298,110 @@ __global__ __launch_bounds__(64 * MID_WAVES) void mlap_mid_kernel(const MlapPara
             reinterpret_cast<uint16_t *>(p.kv_cache + (size_t)dst * MLAP_KV)[w * 64 + l] = q;
             if (l == 0) p.k_scale_cache[(size_t)dst * 4 + w] = deq;
         }
+    }
+}
+
+// The same at prefill sizes, a wave per token and latent (waves 2t: the query latent, 2t + 1: the key latent and key rope):
+// no barriers, and the slabs' loads and reductions run side by side in one wave.  (The form above, a workgroup of twelve
+// waves per latent that waits for memory once and meets twice, is all latency once the chip has run out of room for more
+// workgroups: 1000 tokens 22.0 us.)
+constexpr int MIDP_WAVES = 4;
+constexpr int MIDP_MIN_TOKENS = 64;
+
+// NS slabs of 128 columns at src (lane: columns 2l, 2l + 1 of each): the partial sums added ascending, rounded to bf16
+template <int NS>
+__device__ __forceinline__ void mid_sum_slabs(const float *src, const int ngroups, const size_t gstride, float (&v)[NS][2])
+{
+    constexpr int FLY = NS > 4 ? 3 : 8;                // groups in flight
+#pragma unroll
+    for (int j = 0; j < NS; ++j) v[j][0] = v[j][1] = 0.f;
+    for (int g0 = 0; g0 < ngroups; g0 += FLY) {
+        f32x2 x[FLY][NS];
+#pragma unroll
+        for (int g = 0; g < FLY; ++g)
+#pragma unroll
+            for (int j = 0; j < NS; ++j)
+                x[g][j] = *reinterpret_cast<const f32x2 *>(src + (size_t)(g0 + g < ngroups ? g0 + g : ngroups - 1) * gstride + 128 * j);
+#pragma unroll
+        for (int g = 0; g < FLY; ++g)
+            if (g0 + g < ngroups) {
+#pragma unroll
+                for (int j = 0; j < NS; ++j) {
+                    v[j][0] = __fadd_rn(v[j][0], x[g][j][0]);
+                    v[j][1] = __fadd_rn(v[j][1], x[g][j][1]);
+                }
+            }
+    }
+#pragma unroll
+    for (int j = 0; j < NS; ++j) {
+        v[j][0] = bf16_round_f32(v[j][0]);
+        v[j][1] = bf16_round_f32(v[j][1]);
+    }
+}
+// RMS norm over the NS slabs in place; amax: largest magnitude of each slab
+template <int NS>
+__device__ __forceinline__ void mid_norm_slabs(float (&v)[NS][2], const uint16_t *gamma, const float eps, const int l, float (&amax)[NS])
+{
+    constexpr float coef = (float)(1.0 / (double)(NS * 128));
+    uint32_t gm[NS];
+#pragma unroll
+    for (int j = 0; j < NS; ++j) gm[j] = reinterpret_cast<const uint32_t *>(gamma)[64 * j + l];
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < NS; ++j) s = __fadd_rn(s, slab_square_sum(v[j][0], v[j][1], coef));
+    const float d = __builtin_sqrtf(__fadd_rn(s, eps));          // correctly rounded
+#pragma unroll
+    for (int j = 0; j < NS; ++j) {
+        v[j][0] = bf16_round_f32(__fmul_rn(__fdiv_rn(v[j][0], d), __uint_as_float(gm[j] << 16)));
+        v[j][1] = bf16_round_f32(__fmul_rn(__fdiv_rn(v[j][1], d), __uint_as_float(gm[j] & 0xffff0000u)));
+        amax[j] = wave_max_f32(fmaxf(fabsf(v[j][0]), fabsf(v[j][1])));
+    }
+}
+
+template <int QS>
+__global__ __launch_bounds__(64 * MIDP_WAVES) void mlap_mid_prefill_kernel(const MlapParams p, const int ngroups, const int ngroups_rope)
+{
+    const int l = threadIdx.x & 63;
+    const int job = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * MIDP_WAVES + (threadIdx.x >> 6)));
+    const int t = job >> 1;
+    if (t >= p.T) return;
+    const int nc = QS * 128 + MLAP_KV + MLAP_ROPE;
+    const size_t gstride = (size_t)p.T * nc;
+    const float *row = p.xpart + (size_t)t * nc + 2 * l;
+    if ((job & 1) == 0) {
+        float v[QS][2], amax[QS];
+        mid_sum_slabs<QS>(row, ngroups, gstride, v);
+        mid_norm_slabs<QS>(v, p.gamma_cq, p.eps_cq, l, amax);
+        float m = amax[0];
+#pragma unroll
+        for (int j = 1; j < QS; ++j) m = fmaxf(m, amax[j]);
+        float deq;
+#pragma unroll
+        for (int j = 0; j < QS; ++j)
+            reinterpret_cast<uint16_t *>(p.q_norm + (size_t)t * p.q_lora)[64 * j + l] = quant_pair_amax(v[j][0], v[j][1], m, deq);
+        if (l == 0) p.q_norm_scale[t] = deq;
+        return;
+    }
+    const long long dst = p.cache_index[t];
+    const bool dst_ok = dst >= 0 && dst < p.cache_rows;
+    float r[1][2], v[4][2], amax[4];
+    mid_sum_slabs<1>(row + QS * 128 + MLAP_KV - 2 * (l & 32), ngroups_rope, gstride, r);         // lanes 32.. repeat lanes 0..
+    mid_sum_slabs<4>(row + QS * 128, ngroups, gstride, v);
+    mid_norm_slabs<4>(v, p.gamma_ckv, p.eps_ckv, l, amax);
+    if (!dst_ok) return;
+    if (l < 32) {
+        // channels 2l, 2l + 1 become channels l, 32 + l: the two partners of one rotation
+        const uint16_t *c = p.cos + (size_t)t * MLAP_ROPE + l, *s = p.sin + (size_t)t * MLAP_ROPE + l;
+        const float r0 = __builtin_fmaf(r[0][0], bf16_bits_to_f32(c[0]), (-r[0][1]) * bf16_bits_to_f32(s[0]));      // products exact: one rounding
+        const float r1 = __builtin_fmaf(r[0][1], bf16_bits_to_f32(c[32]), r[0][0] * bf16_bits_to_f32(s[32]));
+        p.kr_cache[(size_t)dst * MLAP_ROPE + l] = (uint16_t)(pack_bf16x2(r0, 0.f) & 0xffffu);
+        p.kr_cache[(size_t)dst * MLAP_ROPE + 32 + l] = (uint16_t)(pack_bf16x2(r1, 0.f) & 0xffffu);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float deq;
+        reinterpret_cast<uint16_t *>(p.kv_cache + (size_t)dst * MLAP_KV)[64 * j + l] = quant_pair_amax(v[j][0], v[j][1], amax[j], deq);
+        if (l == 0) p.k_scale_cache[(size_t)dst * 4 + j] = deq;
     }
 }
 
@@ -408,6 +536,7 @@ void mlap_finish_prefill_shape(const MlapParams &p, int &per, int &wgs)
 
 hipError_t mlap_launch_finish(const MlapParams &p, hipStream_t stream)
 {
+    if (mlap_fused_projection(p)) return prolog_prefill_launch(&p, nullptr, stream);
     if (mlap_finish_is_prefill(p)) {
         int per, wgs;
         mlap_finish_prefill_shape(p, per, wgs);
@@ -445,13 +574,23 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
         // every slab but the last, the rope columns, which keep their fixed-order sums
         const int mslabs = nslabs - 1;
         ngroups = ngroups > nchunks ? nchunks : ngroups;
+        const bool big = p.T > XM_TOK;       // 130 tokens: 60.9 us per pass, 66.7 with tiles of 128; 1500: 282 and 293; 4096: 700 and 724
+        if (big) {
+            // one workgroup per compute unit (the other half of each is for the fixed-order sums)
+            const int tiles = mslabs * ((p.T + XB_TOK - 1) / XB_TOK);
+            ngroups = cus / tiles;
+            ngroups = ngroups < 1 ? 1 : ngroups;
+            ngroups = ngroups > MLAP_XM_MAX_SPLITS ? MLAP_XM_MAX_SPLITS : ngroups;
+            ngroups = ngroups > nchunks ? nchunks : ngroups;
+        }
         const int per_slab = ngroups * ttiles;
-        const int wgs = 8 * ((mslabs >> 3) * per_slab + ((mslabs & 7) * per_slab + 7) / 8);   // the kernel's XCD-wise job order
+        const int wgs = big ? 8 * ((mslabs * ((p.T + XB_TOK - 1) / XB_TOK) * ngroups + 7) / 8) : 8 * ((mslabs >> 3) * per_slab + ((mslabs & 7) * per_slab + 7) / 8);   // the kernel's XCD-wise job order
         const int sets = 1 + (lip_rider != nullptr && p.T >= QPROJ_PREFILL_TOKENS ? LIP_XF_SETS : 0);
         const dim3 g((unsigned)(wgs + xf_jobs(sets, ngroups_fixed, p.T)));
 #define XM_LAUNCH(TBV) hipLaunchKernelGGL(mlap_xlinear_mfma_kernel<TBV>, g, dim3(256), 0, stream, p, mslabs, ngroups, wgs, sets, ngroups_fixed, lip)
         if (p.T <= 32) XM_LAUNCH(1);
         else if (p.T <= 64) XM_LAUNCH(2);
+        else if (big) XM_LAUNCH(XM_BIG);
         else XM_LAUNCH(0);
 #undef XM_LAUNCH
     } else {
@@ -461,9 +600,19 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(mlap_mid_kernel, dim3((unsigned)(2 * p.T)), dim3(64 * MID_WAVES), 0, stream, p, ngroups, ngroups_fixed);
+    if (p.T >= MIDP_MIN_TOKENS) {
+        const dim3 g((unsigned)((2 * p.T + MIDP_WAVES - 1) / MIDP_WAVES)), b(64 * MIDP_WAVES);
+        switch (p.q_lora / 128) {
+        case 4: hipLaunchKernelGGL(mlap_mid_prefill_kernel<4>, g, b, 0, stream, p, ngroups, ngroups_fixed); break;
+        case 8: hipLaunchKernelGGL(mlap_mid_prefill_kernel<8>, g, b, 0, stream, p, ngroups, ngroups_fixed); break;
+        case 12: hipLaunchKernelGGL(mlap_mid_prefill_kernel<12>, g, b, 0, stream, p, ngroups, ngroups_fixed); break;
+        default: return hipErrorInvalidValue;
+        }
+    } else {
+        hipLaunchKernelGGL(mlap_mid_kernel, dim3((unsigned)(2 * p.T)), dim3(64 * MID_WAVES), 0, stream, p, ngroups, ngroups_fixed);
+    }
     e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess || mlap_fused_projection(p)) return e;
     const QProj qp = {p.q_norm, p.w_uqqr, p.qpart, p.T, p.q_lora, p.n_heads * MLAP_QHEAD / 128, p.q_norm_scale, p.w_qb_scale};
     if (mlap_qsplits(p) == 1) {
         if (p.q_lora % (32 * QPF_STEPS)) return hipErrorInvalidValue;

@@ -111,12 +111,13 @@ __device__ __forceinline__ uint16_t quant_pair(const float y0, const float y1, u
 
 constexpr int FIN_WAVES = 8;
 
-// the 128x128 bf16 matrix into LDS, as it is (2048 pieces of 16 bytes over the workgroup's FIN_WAVES waves)
+// the 128x128 bf16 matrix into LDS, as it is (2048 pieces of 16 bytes over the workgroup's waves)
+template <int WAVES>
 __device__ __forceinline__ void stage_matrix(uint16_t *dst, const uint16_t *src)
 {
     const u32x4 *s = reinterpret_cast<const u32x4 *>(src);
     u32x4 *d = reinterpret_cast<u32x4 *>(dst);
-    constexpr int NT = 64 * FIN_WAVES;
+    constexpr int NT = 64 * WAVES;
 #pragma unroll
     for (int i = 0; i < 2048 / NT; ++i) d[i * NT + threadIdx.x] = s[i * NT + threadIdx.x];
 }
@@ -168,7 +169,7 @@ __device__ __forceinline__ void lip_finish_body(const LipParams &p, const int q_
     const int ncols = p.n_heads * LIP_DIM;
 
     if (wg < q_wgs) {
-        stage_matrix(hmat, p.hq);
+        stage_matrix<FIN_WAVES>(hmat, p.hq);
         const int row = wg * FIN_WAVES + w;            // (token, head)
         const bool live = row < p.T * p.n_heads;
         const int t = live ? row / p.n_heads : 0;
@@ -198,7 +199,7 @@ __device__ __forceinline__ void lip_finish_body(const LipParams &p, const int q_
     const bool group_rows = lip_x_group_rows(p);       // the rows are group sums already
     const int nblk = group_rows ? 0 : lip_xrows(p);
     const int ngroups = group_rows ? lip_xrows(p) : (nblk + LIP_XGROUP - 1) / LIP_XGROUP;
-    stage_matrix(hmat, p.hk);
+    stage_matrix<FIN_WAVES>(hmat, p.hk);
     const bool pl = l < p.n_heads;
     // everything wave 0 needs later is requested now
     const uint32_t rc = rope_coef(p.cos, t, l), rs = rope_coef(p.sin, t, l);
@@ -263,11 +264,12 @@ __device__ __forceinline__ void lip_finish_body(const LipParams &p, const int q_
     }
 }
 
-// The key rows and weights at prefill sizes: a workgroup of FIN_WAVES waves takes FIN_WAVES tokens, one per wave (the
+// The key rows and weights at prefill sizes: a workgroup of FINT_WAVES waves takes FINT_WAVES tokens, one per wave (the
 // matrix is staged once for all of them instead of once per token, and the rows are finished side by side instead of
 // by one wave per workgroup).  A wave adds its token's partial rows in registers, in the order of the form they come
 // in: group sums ascending, or blocks / ranges ascending into groups of eight and the groups ascending.
-constexpr int LIP_FINT_LDS = LIP_DIM * LIP_DIM * 2 + FIN_WAVES * LIP_DIM * 4;
+constexpr int FINT_WAVES = 4;
+constexpr int LIP_FINT_LDS = LIP_DIM * LIP_DIM * 2 + FINT_WAVES * LIP_DIM * 4;
 
 __device__ __forceinline__ void lip_finish_tokens_prefill_body(const LipParams &p, const int wg, uint8_t *lds)
 {
@@ -275,10 +277,10 @@ __device__ __forceinline__ void lip_finish_tokens_prefill_body(const LipParams &
     float(*arow)[LIP_DIM] = reinterpret_cast<float(*)[LIP_DIM]>(lds + LIP_DIM * LIP_DIM * 2);
     const int l = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int t = wg * FIN_WAVES + w;
+    const int t = wg * FINT_WAVES + w;
     const bool live = t < p.T;
     const int tt = live ? t : p.T - 1;
-    stage_matrix(hmat, p.hk);
+    stage_matrix<FINT_WAVES>(hmat, p.hk);
     const bool pl = l < p.n_heads;
     const uint32_t rc = rope_coef(p.cos, tt, l), rs = rope_coef(p.sin, tt, l);
     const uint32_t gm = reinterpret_cast<const uint32_t *>(p.gamma)[l];
@@ -329,135 +331,40 @@ __device__ __forceinline__ void lip_finish_tokens_prefill_body(const LipParams &
 }
 
 
-// The query rows at prefill sizes with the Hadamard sums on the matrix cores: a workgroup of four waves stages the
-// matrix once (rows padded to 272 bytes so that the four rows of a transposing read fall into different banks),
-// then each wave walks passes of 32 rows (token, head): it de-quantises and rotates its rows, eight at a time, into
-// its own bf16 operand buffer, takes O^T[j][row] = sum_i H^T[j][i] a^T[i][row] as 32 products
-// (v_mfma_f32_32x32x16_bf16, A = the matrix read transposed, B = the rows), rounds to bf16, quantises each row
-// (lanes l and l + 32 hold one row between them) and sends the int8 rows through its buffer so that they leave as
-// whole 16-byte pieces.  All products are exact; the sums run in the cores' order instead of i ascending.
-constexpr int QFP_WAVES = 4;
-constexpr int QFP_HPITCH = 136;                        // elements between matrix rows in LDS
-constexpr int QFP_APITCH = 136;                        // elements between operand rows
-constexpr int QFP_OPITCH = 144;                        // bytes between int8 rows on their way out
-constexpr int QFP_WAVE_BYTES = 32 * QFP_APITCH * 2;
-constexpr int LIP_QFP_LDS = LIP_DIM * QFP_HPITCH * 2 + QFP_WAVES * QFP_WAVE_BYTES;   // 69 632 bytes
-static_assert(32 * QFP_OPITCH <= QFP_WAVE_BYTES, "the int8 rows reuse the operand buffer");
-static_assert(LIP_QFP_LDS <= 160 * 1024, "one workgroup fits a compute unit");
-
-__device__ __forceinline__ void lip_finish_query_prefill_body(const LipParams &p, const int wg, const int nwg, uint8_t *lds)
+// A block of 32 query rows out of the Hadamard product (lane (row, half) holds channels 32*cb + 8*(r/4) + 4*half + r%4 of its
+// row): rounded to bf16, quantised per row and left as int8 rows QFP_OPITCH bytes apart in the wave's staging area, from where
+// they leave as whole 16-byte pieces.  Returns the row's de-quantisation scale.
+constexpr int QFP_OPITCH = 144;
+__device__ __forceinline__ float lip_quant_rows(f32x16 (&c)[4], uint8_t *mine, const int l)
 {
-    uint16_t *hmat = reinterpret_cast<uint16_t *>(lds);
-    const int l = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    uint8_t *mine = lds + LIP_DIM * QFP_HPITCH * 2 + w * QFP_WAVE_BYTES;
-    uint16_t *abf = reinterpret_cast<uint16_t *>(mine);
+    float amax = 0.f;
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            c[cb][r] = bf16_round_f32(c[cb][r]);
+            amax = fmaxf(amax, fabsf(c[cb][r]));
+        }
     {
-        const u32x4 *s = reinterpret_cast<const u32x4 *>(p.hq);
-        for (int i = threadIdx.x; i < LIP_DIM * LIP_DIM / 8; i += 64 * QFP_WAVES)
-            *reinterpret_cast<u32x4 *>(hmat + (i >> 4) * QFP_HPITCH + (i & 15) * 8) = s[i];
+        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(amax), __float_as_uint(amax), false, false);
+        amax = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
     }
-    __syncthreads();
-    const int ncols = p.n_heads * LIP_DIM;
-    const int nrows = p.T * p.n_heads;
-    const int npass = (nrows + 31) / 32;
-    const uint16_t *at = abf + (l & 31) * QFP_APITCH + 4 * (l >> 5);
-    const uint16_t *wt = hmat + (4 * (l >> 5) + ((l & 15) >> 2)) * QFP_HPITCH + 16 * ((l >> 4) & 1) + 4 * (l & 3);
-    // Eight rows at a time; the loads of the next eight (of this pass or of the wave's next one) are on their way
-    // while the current eight are rotated: a pass would otherwise wait out four memory round trips.
-    struct Rows8 {
-        uint32_t raw[8], rc[8], rs[8];
-    };
-    auto load_rows = [&](Rows8 &r, const int pass, const int b8) {
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int row = pass * 32 + b8 * 8 + u;
-            const int rr = row < nrows ? row : nrows - 1;
-            const int t = rr / p.n_heads;
-            const int col = (rr - t * p.n_heads) * LIP_DIM + 2 * l;
-            r.raw[u] = *reinterpret_cast<const uint32_t *>(reinterpret_cast<const uint16_t *>(p.qpart) + (size_t)t * ncols + col);
-            r.rc[u] = rope_coef(p.cos, t, l);
-            r.rs[u] = rope_coef(p.sin, t, l);
-        }
-    };
-    auto rotate_rows = [&](const Rows8 &r, const int b8) {
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            float v0 = __uint_as_float(r.raw[u] << 16);        // the unsplit projection leaves its results de-quantised
-            float v1 = __uint_as_float(r.raw[u] & 0xffff0000u);
-            rope_pair(v0, v1, r.rc[u], r.rs[u], l);
-            *reinterpret_cast<uint32_t *>(abf + (b8 * 8 + u) * QFP_APITCH + 2 * l) = pack_bf16x2(v0, v1);
-        }
-    };
-    const int stride = nwg * QFP_WAVES;
-    Rows8 ra, rb;
-    if (wg * QFP_WAVES + w < npass) load_rows(ra, wg * QFP_WAVES + w, 0);
-#pragma unroll 1
-    for (int pass = wg * QFP_WAVES + w; pass < npass; pass += stride) {
-        load_rows(rb, pass, 1);
-        rotate_rows(ra, 0);
-        load_rows(ra, pass, 2);
-        rotate_rows(rb, 1);
-        load_rows(rb, pass, 3);
-        rotate_rows(ra, 2);
-        if (pass + stride < npass) load_rows(ra, pass + stride, 0);
-        rotate_rows(rb, 3);
-        // the wave reads back what it wrote itself: LDS operations of a wave stay in order
-        f32x16 c[4];
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) c[cb][r] = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < LIP_DIM / 16; ++ks) {
-            const u32x2 b0 = *reinterpret_cast<const u32x2 *>(at + 16 * ks);
-            const u32x2 b1 = *reinterpret_cast<const u32x2 *>(at + 16 * ks + 8);
-            const u32x4 bq = {b0[0], b0[1], b1[0], b1[1]};
-#pragma unroll
-            for (int cb = 0; cb < 4; ++cb) {
-                const s16x4 a0 = lds_read_tr16(wt + (16 * ks) * QFP_HPITCH + 32 * cb);
-                const s16x4 a1 = lds_read_tr16(wt + (16 * ks + 8) * QFP_HPITCH + 32 * cb);
-                const s16x8 a = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
-                c[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, bq), c[cb], 0, 0, 0);
-            }
-        }
-        // lane (row, half) holds channels 32*cb + 8*(r/4) + 4*half + r%4 of its row
-        float amax = 0.f;
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                c[cb][r] = bf16_round_f32(c[cb][r]);
-                amax = fmaxf(amax, fabsf(c[cb][r]));
-            }
-        {
-            const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(amax), __float_as_uint(amax), false, false);
-            amax = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-        }
-        float s = 0.f, deq = 0.f;
-        if (amax > 0.f) {
-            s = __fdiv_rn(127.0f, amax);
-            deq = __fdiv_rn(1.0f, s);
-        }
-        uint8_t *orow = mine + (l & 31) * QFP_OPITCH + 4 * (l >> 5);
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                uint32_t v = 0;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) v |= (uint32_t)((int)rintf(__fmul_rn(c[cb][4 * g + j], s)) & 0xff) << (8 * j);
-                *reinterpret_cast<uint32_t *>(orow + 32 * cb + 8 * g) = v;
-            }
-        const int row = pass * 32 + (l & 31);
-        if (l < 32 && row < nrows) p.q_scale[row] = (uint16_t)(pack_f16x2(deq, 0.f) & 0xffffu);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int r = 8 * k + (l >> 3);
-            const u32x4 v = *reinterpret_cast<const u32x4 *>(mine + r * QFP_OPITCH + 16 * (l & 7));
-            if (pass * 32 + r < nrows) *reinterpret_cast<u32x4 *>(p.q_int8 + (size_t)(pass * 32 + r) * LIP_DIM + 16 * (l & 7)) = v;
-        }
+    float s = 0.f, deq = 0.f;
+    if (amax > 0.f) {
+        s = __fdiv_rn(127.0f, amax);
+        deq = __fdiv_rn(1.0f, s);
     }
+    uint8_t *orow = mine + (l & 31) * QFP_OPITCH + 4 * (l >> 5);
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            uint32_t v = 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v |= (uint32_t)((int)rintf(__fmul_rn(c[cb][4 * g + j], s)) & 0xff) << (8 * j);
+            *reinterpret_cast<uint32_t *>(orow + 32 * cb + 8 * g) = v;
+        }
+    return deq;
 }
 
 // ---------------------------------------------------------------------------------- MLA prolog

@@ -8,10 +8,12 @@
 // unit together, so they run side by side instead of one launch after the other.  Where the indexer prolog cannot
 // ride (other than 64 indexer heads) its first launch follows the MLA prolog's third.  From 9 tokens on the MLA
 // prolog's prefill forms take the indexer prolog's fixed-order sums along, up to 63 tokens its projection too (five
-// launches; four up to 32 tokens, where the two last stages share one).
-#include "prolog_finish.h"
+// launches; four up to 32 tokens, where the two last stages share one); from 64 tokens on both projections and all that
+// follows them are one launch (three in all).
+#include <cstring>
 
 #include "prolog_fused.h"
+#include "prolog_prefill.h"
 
 namespace pto {
 namespace {
@@ -50,7 +52,46 @@ __global__ __launch_bounds__(64 * FIN_WAVES) void prolog_fused_finish_prefill_ke
     else lip_finish_body(pl, q_wgs, (int)blockIdx.x - mla_wgs, lds);
 }
 
+// Projections and last stages at prefill sizes (prolog_prefill.h): [0, mla_wgs) the attention query, then lip_wgs of the
+// indexer query, then the indexer's key rows and weights, a token per wave.  64 * TB tokens per workgroup of a head.
+template <int XC, int TB> constexpr int PF_LDS2 = PFA_LDS<XC, TB> > PFI_LDS<XC, TB / 2> ? PFA_LDS<XC, TB> : PFI_LDS<XC, TB / 2>;
+template <int XC, int TB> constexpr int PF_LDS = PF_LDS2<XC, TB> > LIP_FINT_LDS ? PF_LDS2<XC, TB> : LIP_FINT_LDS;
+template <int XC, int TB>
+__global__ __launch_bounds__(256, 2) void prolog_prefill_kernel(const MlapParams pm, const LipParams pl, const int mla_wgs, const int lip_wgs)
+{
+    static_assert(2 * PF_LDS<XC, TB> <= 160 * 1024, "two workgroups share a compute unit");
+    static_assert(FINT_WAVES == 4, "one block size for the three bodies");
+    __shared__ __attribute__((aligned(16))) uint8_t lds[PF_LDS<XC, TB>];
+    const int wg = (int)blockIdx.x;
+    if (wg < mla_wgs) mlap_prefill_body<XC, TB>(pm, q_prefill_job_of(wg, mla_wgs), lds);
+    else if (wg < mla_wgs + lip_wgs) lip_prefill_body<XC, TB / 2>(pl, q_prefill_job_of(wg - mla_wgs, lip_wgs), lds);
+    else lip_finish_tokens_prefill_body(pl, wg - mla_wgs - lip_wgs, lds);
+}
+
 }  // namespace
+
+hipError_t prolog_prefill_launch(const MlapParams *pm, const LipParams *pl, hipStream_t stream)
+{
+    const int T = pm ? pm->T : pl->T;
+    MlapParams m;
+    LipParams p;
+    std::memset(&m, 0, sizeof m);
+    std::memset(&p, 0, sizeof p);
+    if (pm) m = *pm;
+    if (pl) p = *pl;
+    // 256-token tiles take 12 % less time per (padded) token than 128-token ones where both fill the chip, which up to 256
+    // tokens they do not (256 tokens: 79.6 us per pass against 77.5; 600: 150.4 against 140.3; 1000: 188.5 against 206.6)
+    const bool small = T <= 256 || 100 * ((T + 127) / 128) <= 176 * ((T + 255) / 256);
+    const int tok = small ? 128 : 256;
+    const int tiles = (T + tok - 1) / tok;
+    const int mla_wgs = pm ? m.n_heads * tiles : 0;
+    const int lip_wgs = pl ? p.n_heads * tiles : 0;
+    const int tok_wgs = pl ? (T + FINT_WAVES - 1) / FINT_WAVES : 0;
+    const dim3 g((unsigned)(mla_wgs + lip_wgs + tok_wgs));
+    if (small) hipLaunchKernelGGL((prolog_prefill_kernel<2, 2>), g, dim3(256), 0, stream, m, p, mla_wgs, lip_wgs);
+    else hipLaunchKernelGGL((prolog_prefill_kernel<1, 4>), g, dim3(256), 0, stream, m, p, mla_wgs, lip_wgs);
+    return hipGetLastError();
+}
 
 hipError_t prolog_fused_launch(const MlapParams &pm, const LipParams &pl, hipStream_t stream)
 {
@@ -85,6 +126,7 @@ hipError_t prolog_fused_launch(const MlapParams &pm, const LipParams &pl, hipStr
         e = lip_launch_linear(px, stream);
         if (e != hipSuccess) return e;
     }
+    if (mlap_fused_projection(pm) && lip_q_on_matrix_cores(px)) return prolog_prefill_launch(&pm, &px, stream);
     int per = 0, pf_wgs = 0;
     if (mlap_finish_is_prefill(pm)) mlap_finish_prefill_shape(pm, per, pf_wgs);
     // up to 32 tokens: one workgroup per head, the indexer half's take the other compute units (more would queue one

@@ -245,6 +245,31 @@ def test_fused_prolog_fixed_order_sums_at_tile_edges(t, n_idx):
     assert (gk - rk).abs().max() <= 1 and (gk != rk).float().mean() <= 0.01
 
 
+@pytest.mark.parametrize("t,q_lora", [(64, 512), (127, 1536), (129, 1024), (256, 512), (257, 512), (512, 512), (513, 1024), (700, 512)])
+def test_fused_prolog_query_rows_at_tile_edges(t, q_lora):
+    """The launch that makes and finishes both queries from 64 tokens on, at the edges of its tiles of 128 and 256 tokens and
+    of the hidden-axis launch's: every query output against the sequential statement under the reference's rule."""
+    from oracle import lip_oracle as lo
+    from pypto_amd import lightning_indexer_prolog_quant_impl as lip_impl
+    from pypto_amd import mla_prolog_quant_impl as impl
+    from pypto_amd.synthetic import gen_indexer_prolog_inputs
+    impl.EXACT_ABSORB = lip_impl.EXACT_SUMS = False
+    kw = dict(h=128, q_lora_rank=q_lora)
+    mla = gen_mla_prolog_inputs(1, t, [t + 30], seed=t, n_heads=2, **kw)
+    lip = gen_indexer_prolog_inputs(1, t, [t + 30], seed=t + 1, n_heads=8, **kw)
+    ref = mo.mla_prolog_ref(*mla.input_tensors(), epsilon_cq=1e-5, epsilon_ckv=1e-5)
+    got = run_op(mla, (1e-5, 1e-5), prefill=True)
+    assert_reference_rule(got, ref, mla.cache_index.numpy(), f"t={t}")
+    dm, dl = mla.to(torch.device("cuda:0")), lip.to(torch.device("cuda:0"))
+    q_nope, q_rope, q_int8, q_scale, _ = run_fused(dm, dl, t, 2, 8, op=pypto_amd.mla_indexer_prolog_quant_p)
+    assert np.array_equal(q_nope.float().cpu().numpy(), got["query_nope"]) and np.array_equal(q_rope.float().cpu().numpy(), got["query_rope"])
+    lip.x, lip.cos_idx_rope, lip.sin_idx_rope, lip.k_cache_index = mla.token_x, mla.cos, mla.sin, mla.cache_index
+    lip.q_norm, lip.q_norm_scale = torch.from_numpy(got["q_norm"]), torch.from_numpy(got["q_norm_scale"]).reshape(-1, 1)
+    want = lo.indexer_prolog_ref(*lip.input_tensors())
+    assert np.abs(q_int8.cpu().numpy().astype(np.int32) - want["q_int8"].astype(np.int32)).max() <= 1
+    assert (np.abs(q_scale.float().cpu().numpy()[..., 0] - want["q_scale"].astype(np.float32)) > 2.5e-5).mean() <= 0.005
+
+
 @pytest.mark.parametrize("mode,shape", [("default", "small"), ("exact", "small"), ("matrix_cores", "small"), ("default", "t_512"),
                                         ("default", "t_11_idx_64"), ("exact", "t_11_idx_64"), ("default", "t_3_idx_32"),
                                         ("default", "t_40_idx_64"), ("exact", "t_40_idx_64"), ("default", "t_7_idx_64"),
