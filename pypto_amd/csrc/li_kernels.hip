@@ -146,14 +146,26 @@ __device__ __forceinline__ float mul_f16_f32_v(const uint32_t packed, const floa
     return r;
 }
 
-// x = fp16(relu(dot) / 2048) for two dots, packed.  v_fma_mixlo/mixhi_f16 scale in fp32 (exact: a power
-// of two) and round once to fp16; -|dot|/2048 rounds to a negative fp16 that the packed integer max
-// then clears, which equals clearing first.  scale = 2^-11 in a scalar register.
-__device__ __forceinline__ uint32_t relu_fp16_pair(const int d0, const int d1, const float scale)
+// sum + x * w for one half each of two packed fp16 pairs (the second wave-uniform), rounded once.  The product of two fp16
+// values is exact in fp32, so this is the rounded multiply followed by the rounded add of the definition.
+template <int HI>
+__device__ __forceinline__ void fma_f16_pair(float &sum, const uint32_t x, const uint32_t w)
 {
-    uint32_t packed;
-    asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(packed) : "v"((float)d0), "s"(scale));
-    asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(packed) : "v"((float)d1), "s"(scale));
+    if (HI)
+        asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "+v"(sum) : "v"(x), "s"(w));
+    else
+        asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel:[0,0,0] op_sel_hi:[1,1,0]" : "+v"(sum) : "v"(x), "s"(w));
+}
+
+// x = fp16(relu(dot) / 2048) for two dots, packed.  The integer accumulators start at the bit pattern of 4.0f (DOT_ZERO, an
+// operand the matrix instruction reads anyway), so that a sum's bits read as a float are 4 + dot * 2^-21 for dot >= 0 and
+// 4 + dot * 2^-22 below: times 1024 less 4096 is dot / 2048 exactly, or something negative, without a conversion.  The pair is
+// rounded once to fp16 (v_cvt_pk_f16_f32) and a packed integer max clears the negative ones.  (v_fma_mixlo/mixhi_f16, which
+// write half a register, issue at half the rate: 9.2 clocks against 5.3.)
+constexpr int DOT_ZERO = 0x40800000;
+__device__ __forceinline__ uint32_t relu_fp16_pair(const int d0, const int d1)
+{
+    const uint32_t packed = pack_f16x2(__builtin_fmaf(__int_as_float(d0), 1024.f, -4096.f), __builtin_fmaf(__int_as_float(d1), 1024.f, -4096.f));
     // relu on the bit patterns: a negative fp16 (and -0) is a negative 16-bit integer
     typedef __attribute__((ext_vector_type(2))) short s16x2;
     const s16x2 zero = {0, 0};
@@ -220,11 +232,13 @@ constexpr int SC_BUF_BYTES = SC_PAIR_BYTES + 256;   // + the 64 key scales (one 
 // a batch against a page in one matrix product (lightning_indexer_quant_impl.py:163-169, [S1*64, 128]); here
 // a "unit" is a pair of consecutive tokens of a sequence (the last unit of an odd s1 holds one), every staged
 // key row and scale serves both, and their per-head factors sit in LDS instead of scalar registers.
-template <int KDT, int VAR = 0, int NT = 1>
+// HW: query scales and weights are fp16, so the per-head factors are fp16 values, their products with x exact and the head
+// sum one instruction per head instead of two; the factors sit in scalar registers as packed pairs, for two tokens as well.
+template <int KDT, int VAR = 0, int NT = 1, bool HW = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void li_score_kernel(const LiParams p)
 {
     __shared__ __attribute__((aligned(16))) int8_t kstage[4][2][SC_BUF_BYTES];
-    __shared__ __attribute__((aligned(16))) float wsc_lds[NT > 1 ? 4 : 1][NT][LI_HEADS];
+    __shared__ __attribute__((aligned(16))) float wsc_lds[NT > 1 && !HW ? 4 : 1][NT][LI_HEADS];
     const int upb = (p.S1 + NT - 1) / NT;            // units per sequence
     const int nunits = p.B * upb;
     const int w = threadIdx.x >> 6;
@@ -361,7 +375,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
     // read as broadcasts, four heads at a time, along the head sum.
     // VAR = 1 keeps the fp16 query scales and weights of head pairs (2i, 2i+1) packed instead.
     static_assert(!(VAR && NT > 1), "the fp16 variant scores one token per wave");
-    float wsc[(VAR || NT > 1) ? 1 : LI_HEADS];
+    float wsc[(VAR || HW || NT > 1) ? 1 : LI_HEADS];
+    uint32_t wp[HW ? NT : 1][HW ? LI_HEADS / 2 : 1];             // HW: factors of heads 2i and 2i + 1
     uint32_t qs2[VAR ? LI_HEADS / 2 : 1], w2[VAR ? LI_HEADS / 2 : 1];
     if (VAR) {
         const uint32_t mq = reinterpret_cast<const uint32_t *>(p.q_scale)[(size_t)t * (LI_HEADS / 2) + (l & 31)];
@@ -370,6 +385,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
         for (int h = 0; h < LI_HEADS / 2; ++h) {
             qs2[h] = (uint32_t)__builtin_amdgcn_readlane((int)mq, h);
             w2[h] = (uint32_t)__builtin_amdgcn_readlane((int)mw, h);
+        }
+    } else if (HW) {
+#pragma unroll
+        for (int s = 0; s < NT; ++s) {
+            const size_t i0 = (size_t)(t + (s < nt ? s : 0)) * LI_HEADS + 2 * (l & 31);
+            const uint32_t mine = pack_f16x2(w_scale_of(p, i0), w_scale_of(p, i0 + 1));       // fp16 values: exact
+#pragma unroll
+            for (int h = 0; h < LI_HEADS / 2; ++h) wp[s][h] = (uint32_t)__builtin_amdgcn_readlane((int)mine, h);
         }
     } else if (NT > 1) {
 #pragma unroll
@@ -389,15 +412,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) koff[ks] = j * LI_DIM + (((4 * half + ks) ^ (j & 7)) << 4);
 
-    // One trip.  Requests complete in the order they were made, so "at most nine outstanding" (the
-    // nine of the following pair; the score store of the previous trip may or may not be among them)
-    // means that this trip's pair has landed.  Its operands and scale move to registers, which frees
-    // the buffer for the pair two ahead; then the pair is scored.
+    // One trip.  Requests and stores complete in the order they were made.  Behind this trip's pair there are the nine
+    // requests of the following pair and the two stores per token (scores, sample) of each of the last two trips -- every
+    // trip but the wave's last writes both -- and that many may be outstanding: a wait that counts the requests alone
+    // holds a wave up until half of the pair it has only just asked for has landed too.  The trip's operands and scale
+    // then move to registers, which frees the buffer for the pair two ahead, and the pair is scored.
+    auto wait_pair = [&](auto per_trip, const int pr) {
+        constexpr int ST = decltype(per_trip)::value;
+        if (pr + 1 < npair) {
+            if (pr >= 2) __builtin_amdgcn_s_waitcnt(vmcnt_imm(9 + 2 * ST));
+            else if (pr == 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(9 + ST));
+            else __builtin_amdgcn_s_waitcnt(vmcnt_imm(9));
+        } else {
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        }
+    };
     auto trip = [&](const int pr, const int buf) {
         const int8_t *src = &kstage[w][buf][0];
         i32x4 kx[4], ky[4];
-        if (pr + 1 < npair) __builtin_amdgcn_s_waitcnt(0x0F79);  // vmcnt(9)
-        else __builtin_amdgcn_s_waitcnt(0x0F70);                 // vmcnt(0)
+        if (NT > 1 && nt > 1) wait_pair(std::integral_constant<int, 4>{}, pr);
+        else wait_pair(std::integral_constant<int, 2>{}, pr);
         asm volatile("" ::: "memory");
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
@@ -426,7 +460,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
             constexpr int s = decltype(s_tag)::value;
             i32x16 ax0, ax1, ay0, ay1;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) { ax0[r] = 0; ax1[r] = 0; ay0[r] = 0; ay1[r] = 0; }
+            for (int r = 0; r < 16; ++r) ax0[r] = ax1[r] = ay0[r] = ay1[r] = VAR ? 0 : DOT_ZERO;
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
                 ax0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(qa[s][0][ks], kx[ks], ax0, 0, 0, 0);
@@ -438,10 +472,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
             uint32_t lo[2][8], hi[2][8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const uint32_t x0 = VAR ? fp16_pair(ax0[2 * i], ax0[2 * i + 1], scale) : relu_fp16_pair(ax0[2 * i], ax0[2 * i + 1], scale);
-                const uint32_t y0 = VAR ? fp16_pair(ay0[2 * i], ay0[2 * i + 1], scale) : relu_fp16_pair(ay0[2 * i], ay0[2 * i + 1], scale);
-                const uint32_t x1 = VAR ? fp16_pair(ax1[2 * i], ax1[2 * i + 1], scale) : relu_fp16_pair(ax1[2 * i], ax1[2 * i + 1], scale);
-                const uint32_t y1 = VAR ? fp16_pair(ay1[2 * i], ay1[2 * i + 1], scale) : relu_fp16_pair(ay1[2 * i], ay1[2 * i + 1], scale);
+                const uint32_t x0 = VAR ? fp16_pair(ax0[2 * i], ax0[2 * i + 1], scale) : relu_fp16_pair(ax0[2 * i], ax0[2 * i + 1]);
+                const uint32_t y0 = VAR ? fp16_pair(ay0[2 * i], ay0[2 * i + 1], scale) : relu_fp16_pair(ay0[2 * i], ay0[2 * i + 1]);
+                const uint32_t x1 = VAR ? fp16_pair(ax1[2 * i], ax1[2 * i + 1], scale) : relu_fp16_pair(ax1[2 * i], ax1[2 * i + 1]);
+                const uint32_t y1 = VAR ? fp16_pair(ay1[2 * i], ay1[2 * i + 1], scale) : relu_fp16_pair(ay1[2 * i], ay1[2 * i + 1]);
                 const auto s0 = __builtin_amdgcn_permlane32_swap(x0, y0, false, false);
                 const auto s1 = __builtin_amdgcn_permlane32_swap(x1, y1, false, false);
                 lo[0][i] = s0[0]; hi[0][i] = s0[1];
@@ -473,7 +507,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
                 if (sample_lane(pos, cur)) smp[pos >> 4] = sum;
                 return;
             }
-            if (NT > 1) {
+            if (HW) {
+#pragma unroll
+                for (int q = 0; q < 32; ++q) {                       // heads ascending, two per register
+                    const uint32_t x = q < 16 ? lo[q >> 3][q & 7] : hi[(q >> 3) & 1][q & 7];
+                    fma_f16_pair<0>(sum, x, wp[s][q]);
+                    fma_f16_pair<1>(sum, x, wp[s][q]);
+                }
+            } else if (NT > 1) {
                 // heads ascending: lo[0][0..7], lo[1][0..7], hi[0][0..7], hi[1][0..7], two heads per register
                 const f32x4 *wrow = reinterpret_cast<const f32x4 *>(&wsc_lds[w][s][0]);
 #pragma unroll
@@ -782,7 +823,7 @@ constexpr int SEL_CHUNK = 32 * SEL_THREADS;   // scores one trip of the row scan
 // range too long to stage) the general streaming select runs instead.
 __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p)
 {
-    __shared__ unsigned long long cand[SEL_CAP + 64];  // + one dump slot per lane
+    __shared__ uint32_t cand[SEL_CAP];                 // positions
     __shared__ unsigned long long stage[SEL_STAGE];    // also the sort buffer of the other paths
     __shared__ uint16_t sbucket[SEL_STAGE];            // bucket of every staged entry
     __shared__ uint32_t bcount[SEL_BUCKETS];
@@ -923,24 +964,26 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
     // it spread out too; anything beyond shares bucket 0
     const float bscale = smax - blo > 0.f ? (float)SEL_BUCKETS / (1.25f * (smax - blo)) : 0.f;
 
-    // ---- 2. candidates.  Wave w compacts the candidates among its keys into its own region of the
-    // list, cand[w*SEL_WAVE_CAP ...], so the waves share no counter.  A key costs a compare and an add
-    // to be counted and, branch-free, a compare, a select, an add and one LDS write of the raw
-    // (score bits, position) pair: a key that is no candidate goes to the lane's dump slot.  The
-    // order word is formed later, for the candidates only.  Wave-wide sums use DPP, not LDS.
+    // ---- 2. candidates.  Wave w compacts the positions of the candidates among its keys into its own region of the
+    // list, cand[w*SEL_WAVE_CAP ...], so the waves share no counter.  A key costs a compare and an add-with-carry that
+    // shifts the outcome into the lane's mask of its 32 keys; the few candidates (one key in twenty of a long row) are then
+    // picked out of the masks, a candidate of every lane per trip, and their scores fetched again below (out of the L2).
+    // (One LDS write per key, candidate or not, as before, took 14 to 17 of the kernel's 33 thousand clocks on 50 K keys.)
+    // Wave-wide sums use DPP, not LDS.
     uint32_t wave_count = 0;               // candidates of this wave so far (uniform)
     auto scan_chunk = [&](const int c0, auto full_tag) {
         constexpr bool FULL = decltype(full_tag)::value;          // the whole chunk lies inside the row
         const int i_base = c0 + 4 * tid;
-        uint32_t mine = 0;
+        uint32_t m = 0;                                           // key (u, c) is bit 31 - (4u + c)
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 const int i = i_base + 4 * u * SEL_THREADS + c;
-                mine += ((FULL || i < n) && v[u][c] >= pivot) ? 1u : 0u;
+                m = m + m + (((FULL || i < n) && v[u][c] >= pivot) ? 1u : 0u);
             }
         }
+        const uint32_t mine = (uint32_t)__popc(m);
         const uint32_t incl = wave_incl_scan(mine);
         const uint32_t wave_n = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
         if (wave_count + wave_n > (uint32_t)SEL_WAVE_CAP) {       // region overflow: the streaming path will run
@@ -949,16 +992,10 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
         }
         uint32_t slot = (uint32_t)(wv * SEL_WAVE_CAP) + wave_count + incl - mine;
         wave_count += wave_n;
-        const uint32_t dump = (uint32_t)(SEL_CAP + lane);
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const int i = i_base + 4 * u * SEL_THREADS + c;
-                const bool is_c = (FULL || i < n) && v[u][c] >= pivot;
-                cand[is_c ? slot : dump] = ((unsigned long long)(uint32_t)i << 32) | __float_as_uint(v[u][c]);
-                slot += is_c ? 1u : 0u;
-            }
+        while (m != 0u) {
+            const uint32_t q = (uint32_t)__clz(m);                // 4u + c
+            m &= 0x7fffffffu >> q;
+            cand[slot++] = (uint32_t)i_base + ((q >> 2) * (4u * SEL_THREADS) + (q & 3u));
         }
     };
     for (int c0 = 0; c0 < n; c0 += SEL_CHUNK) {
@@ -974,13 +1011,16 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
     // inside the bucket
     constexpr int CPT = SEL_WAVE_CAP / 64;
     unsigned long long ce[CPT];
-    uint32_t cb[CPT], cslot[CPT];
+    uint32_t cb[CPT], cslot[CPT], cpos[CPT];
+    float csc[CPT];
 #pragma unroll
     for (int u = 0; u < CPT; ++u) {
         const uint32_t j = (uint32_t)(u * 64 + lane);
-        const unsigned long long raw = cand[wv * SEL_WAVE_CAP + (j < wave_count ? j : 0u)];
-        ce[u] = j < wave_count ? order_word(__uint_as_float((uint32_t)raw), (uint32_t)(raw >> 32)) : 0ull;
+        cpos[u] = j < wave_count ? cand[wv * SEL_WAVE_CAP + j] : 0u;
+        csc[u] = srow[cpos[u]];
     }
+#pragma unroll
+    for (int u = 0; u < CPT; ++u) ce[u] = (uint32_t)(u * 64 + lane) < wave_count ? order_word(csc[u], cpos[u]) : 0ull;
 #pragma unroll
     for (int u = 0; u < CPT; ++u) {
         const uint32_t lin = (uint32_t)fmaxf((key_score((uint32_t)(ce[u] >> 32)) - blo) * bscale, 0.f);
@@ -1093,16 +1133,22 @@ hipError_t li_launch(const LiParams &p, hipStream_t stream)
         const unsigned gx = (unsigned)((p.score_stride + 4 * p.ppw * 64 - 1) / (4 * p.ppw * 64));
         grid = dim3(gx, (unsigned)nunits);
     }
+    const bool hw = p.q_dt == PTO_DT_FP16 && p.w_dt == PTO_DT_FP16;
+#define LI_SCORE(KDT)                                                                                                      \
+    do {                                                                                                                   \
+        if (nt == 2) {                                                                                                     \
+            if (hw) hipLaunchKernelGGL((li_score_kernel<KDT, 0, 2, true>), grid, block, 0, stream, p);                     \
+            else hipLaunchKernelGGL((li_score_kernel<KDT, 0, 2, false>), grid, block, 0, stream, p);                       \
+        } else {                                                                                                           \
+            if (hw) hipLaunchKernelGGL((li_score_kernel<KDT, 0, 1, true>), grid, block, 0, stream, p);                     \
+            else hipLaunchKernelGGL((li_score_kernel<KDT, 0, 1, false>), grid, block, 0, stream, p);                       \
+        }                                                                                                                  \
+    } while (0)
     if (p.variant == 1) hipLaunchKernelGGL((li_score_kernel<PTO_DT_FP16, 1>), grid, block, 0, stream, p);
-    else if (nt == 2) {
-        if (p.k_dt == PTO_DT_FP32) hipLaunchKernelGGL((li_score_kernel<PTO_DT_FP32, 0, 2>), grid, block, 0, stream, p);
-        else if (p.k_dt == PTO_DT_FP16) hipLaunchKernelGGL((li_score_kernel<PTO_DT_FP16, 0, 2>), grid, block, 0, stream, p);
-        else hipLaunchKernelGGL((li_score_kernel<PTO_DT_BF16, 0, 2>), grid, block, 0, stream, p);
-    } else {
-        if (p.k_dt == PTO_DT_FP32) hipLaunchKernelGGL(li_score_kernel<PTO_DT_FP32>, grid, block, 0, stream, p);
-        else if (p.k_dt == PTO_DT_FP16) hipLaunchKernelGGL(li_score_kernel<PTO_DT_FP16>, grid, block, 0, stream, p);
-        else hipLaunchKernelGGL(li_score_kernel<PTO_DT_BF16>, grid, block, 0, stream, p);
-    }
+    else if (p.k_dt == PTO_DT_FP32) LI_SCORE(PTO_DT_FP32);
+    else if (p.k_dt == PTO_DT_FP16) LI_SCORE(PTO_DT_FP16);
+    else LI_SCORE(PTO_DT_BF16);
+#undef LI_SCORE
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(li_select_kernel, dim3((unsigned)p.T), dim3(SEL_THREADS), 0, stream, p);

@@ -135,6 +135,23 @@ def test_token_pairs_share_a_key_pass(c_oracle, variant, b, s1):
     assert_exact(run_op(inp), oracle(inp, c_oracle), f"{variant} b={b} s1={s1}")
 
 
+@pytest.mark.parametrize("variant,b,s1", [("fp16", 28, 3), ("fp16", 2, 1), ("fp32", 2, 1)])
+def test_largest_dot_products(c_oracle, variant, b, s1):
+    """Queries and keys of -128 and 127 only, with runs of one value: dot products up to +-2^21, both ends of the range in which
+    the accumulators' bits are read as floats; with fp16 scales and weights the fused head sum, for a unit of one token too."""
+    g = torch.Generator().manual_seed(b)
+    act = [int(x) for x in torch.randint(2100, 20480, [b], generator=g)]
+    act[0] = 20480
+    inp = gen_indexer_inputs(b, s1, act, selected_count=2048, seed=5 + b, variant=variant)
+    inp.idx_query = torch.where(inp.idx_query < 0, -128, 127).to(torch.int8)
+    inp.idx_key_cache = torch.where(inp.idx_key_cache < 0, -128, 127).to(torch.int8)
+    inp.idx_query[:, ::3] = -128
+    inp.idx_query[:, 1::3] = 127
+    inp.idx_key_cache[:, ::7] = -128
+    inp.idx_key_cache[:, 1::7] = 127
+    assert_exact(run_op(inp), oracle(inp, c_oracle), f"{variant} b={b} s1={s1} extremes")
+
+
 @pytest.mark.parametrize("variant,b,s1", [("fp16", 260, 4), ("fp32", 260, 3)])
 def test_token_pairs_beyond_the_balanced_mapping(c_oracle, variant, b, s1):
     """Token pairs per key pass in the launch shape that takes one grid row per unit: more than 512 units (260
