@@ -131,6 +131,25 @@ __device__ __forceinline__ void both_halves(const float x, float &lo, float &hi)
 
 constexpr float RESCALE_TAU = 8.0f;   // log2 units: the reference max moves only when exceeded by 2^8
 
+// The bf16 cache with 128 heads in one workgroup (PIPE) divides the two products differently.  With a wave's 32 heads in both,
+// every wave reads the whole tile for each of them: 272 KiB of LDS per tile, about as long as the products take at the
+// ~128 B/clk the LDS sustains beside them.  Here the scores stay per head group, but of O^T wave w takes the value channels
+// 128*w .. +127 of all 128 heads (the same 256 accumulators): each V^T operand then serves four products, and the
+// probabilities go round through LDS (8 KiB per tile).  The products of tile n-1 against V run after the scores of tile n,
+// with tile n's softmax in their shadow, so a tile needs one barrier: three tile buffers, rows by LDS-DMA only (1040-byte
+// pitch; the rope part apart, 128-byte rows with 16-byte piece q of row r at q ^ ((r >> 1) & 7)).
+// Bound by the shader clock, which falls to 1.5-1.75 GHz under back-to-back products: 4096 rows over 4096 keys 1651 -> 1545 us,
+// 1247 with nothing but the products and barriers left in the loop; starting and ending a row (14 us of queries and results
+// per workgroup when every compute unit does it at once, 8-9 spread out) is another tenth.  Requests with scalar addresses: +1 %.
+constexpr int PT_PITCH = DN * 2 + 16;
+constexpr int PT_ROPE = KT * PT_PITCH;
+constexpr int PT_BYTES = PT_ROPE + KT * DR * 2;
+constexpr int PT_P = 3 * PT_BYTES;                 // two buffers of P^T: [k-step][head group][lane] 16 bytes
+constexpr int PT_P_BYTES = 8192;
+constexpr int PT_ALPHA = PT_P + 2 * PT_P_BYTES;    // two buffers: rescale factors of the 128 heads, then which groups have one
+constexpr int PT_ALPHA_BYTES = 128 * 4 + 16;
+constexpr int PT_POOL = PT_ALPHA + 2 * PT_ALPHA_BYTES;
+
 // QUANT: the latent part of a cache row is int8 with four fp32 scales and is de-quantised on the way into
 // LDS; otherwise it is bf16 already (1024 bytes) and travels cache -> LDS tile directly by LDS-DMA.
 // HG: groups of 32 heads in the workgroup, which always has four waves.  With HG = 4 a wave owns its 32 heads.  With fewer
@@ -162,7 +181,9 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
     constexpr int STG_SLOTS = 2;
     constexpr int STG_BASE = TILES_BYTES > WAVE_BYTES ? TILES_BYTES : WAVE_BYTES;   // above everything else in the pool
     constexpr int XCH_BASE = STG_BASE + (QUANT ? STG_SLOTS * STG_BYTES : 0);        // partial scores, 4 KiB per wave
-    constexpr int POOL_BYTES = XCH_BASE + (SP > 1 ? NW * 4096 : 0);
+    constexpr bool PIPE = HG == 4 && !QUANT;
+    constexpr int POOL_BYTES = PIPE ? PT_POOL : XCH_BASE + (SP > 1 ? NW * 4096 : 0);
+    static_assert(!PIPE || PT_P >= WAVE_BYTES, "query staging and epilogue fit the tile buffers");
     static_assert(STG_BASE % 16 == 0 && STG_BYTES % 16 == 0, "LDS-DMA destinations are 16-byte aligned");
     __shared__ __attribute__((aligned(16))) uint16_t pool[POOL_BYTES / 2];
     __shared__ int rows_lds[SFA_MAX_CHUNK + 3 * KT];
@@ -638,7 +659,25 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
     }
     land_q();
     __syncthreads();                       // every wave holds its Q^T fragments: the tile buffers are free
-    if (n_valid > 0) {
+    // PIPE: request i of the nine of this wave for tile kt, into tile buffer at LDS byte offset dst
+    auto pipe_row = [&](const int kt, const int i) {
+        const int *rtab = rows_lds + (kt - k_begin) + wu * 8;
+        return i < 8 ? rtab[i] : rtab[l >> 3];
+    };
+    auto pipe_request = [&](const int i, const int row, const uint32_t dst) {
+        const uint32_t base = (uint32_t)(uintptr_t)(lds_byte_t *)pool_b + dst;
+        if (i < 8) dma16(p.kn + (size_t)row * p.kn_pitch + 16 * l, base + (uint32_t)((wu * 8 + i) * PT_PITCH));
+        else dma16(p.kr + (size_t)row * p.kr_pitch + 16 * ((l & 7) ^ ((4 * wu + (l >> 4)) & 7)), base + PT_ROPE + 1024u * wu);
+    };
+    if (PIPE) {
+        if (n_valid > 0) {
+            int rows[9];
+#pragma unroll
+            for (int i = 0; i < 9; ++i) rows[i] = pipe_row(k_begin, i);
+#pragma unroll
+            for (int i = 0; i < 9; ++i) pipe_request(i, rows[i], 0);
+        }
+    } else if (n_valid > 0) {
         if (QUANT) {
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(DMA_PER_TILE));              // the first tile has landed
             asm volatile("" ::: "memory");
@@ -809,7 +848,170 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
         if (!QUANT) __builtin_amdgcn_s_waitcnt(0x0F70); // this wave's direct requests into the next tile have landed
         __syncthreads();
     };
-    {
+    if constexpr (PIPE) {
+        const int krow = tile_row_of(col);
+        // per-lane bases: score operand (rows of the latent part, then of the rope part), V^T operand, P^T
+        const uint32_t kbase = (uint32_t)(krow * PT_PITCH + 16 * half);
+        uint32_t rbase[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) rbase[e] = (uint32_t)(PT_ROPE + krow * (DR * 2) + 16 * ((2 * e + half) ^ ((krow >> 1) & 7)));
+        const uint32_t vbase = (uint32_t)((half + 4 * ((l & 15) >> 2)) * PT_PITCH + 32 * ((l >> 4) & 1) + 8 * (l & 3) + 256 * w);
+        f32x16 s;
+        u32x4 pk0, pk1;
+        float mx = 0.f, m_new = 0.f, alpha = 1.f, lsum = 0.f;
+        bool upd = false, rescale = false;
+        bf16x8 vf[2][4], pf[2];
+        auto load_v = [&](const uint32_t tile, const int kk, const int d) {
+            const uint16_t *a0 = reinterpret_cast<const uint16_t *>(pool_b + tile + vbase + (16 * kk) * PT_PITCH + 64 * d);
+            const s16x4 lo = lds_read_tr16(a0), hi = lds_read_tr16(a0 + PT_PITCH);       // (two rows on)
+            vf[kk][d] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        };
+        auto load_p = [&](const int pbuf, const int kk, const int hb) {
+            pf[hb & 1] = *reinterpret_cast<const bf16x8 *>(pool_b + PT_P + pbuf * PT_P_BYTES + ((kk * 4 + hb) * 64 + l) * 16);
+        };
+        // scores of the tile at `cur`; the next tile's requests and, if PV, the first operands of the products against V of the
+        // tile at `prev` ride along
+        auto scores = [&](auto pv_tag, const uint32_t cur, const uint32_t prev, const uint32_t next, const int kt, const int pbuf) {
+            constexpr bool PV = decltype(pv_tag)::value;
+            const uint8_t *kp = pool_b + cur + kbase;
+            auto read_k = [&](const int ks) {
+                return *reinterpret_cast<const bf16x8 *>(ks < 32 ? kp + 32 * ks : pool_b + cur + rbase[ks < 32 ? 0 : ks - 32]);
+            };
+            bf16x8 fa[8];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) fa[e] = read_k(e);
+            int row[2];
+#pragma unroll
+            for (int m = 0; m < KSTEPS; ++m) {
+                if (m == 0) s_mfma_first(s, fa[0], qf[0]);
+                else s_mfma(s, fa[m & 7], qf[m]);
+                __builtin_amdgcn_sched_barrier(0);
+                if (m + 4 < KSTEPS) fa[(m + 4) & 7] = read_k(m + 4);
+                if (m >= 2 && m < 11) pipe_request(m - 2, row[m & 1], next);
+                if (m < 9) row[m & 1] = pipe_row(kt + KT, m);
+                if (PV) {
+                    if (m >= 24 && m < 32 && (m & 1) == 0) load_v(prev, 0, (m - 24) >> 1);
+                    if (m == 33) load_p(pbuf, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        // the softmax of the scores in s, in 32 steps; step 31 leaves this wave's P^T in buffer `pbuf` and, where a running
+        // maximum moved past the threshold, the heads' rescale factors beside it
+        auto softmax_step = [&](const int q, const int kt, const int pbuf) {
+            if (q == 0) {
+                s_chain_done(s);
+                if (kt + KT > k_end) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        if (kt + tile_row_of(8 * (r >> 2) + 4 * half + (r & 3)) >= k_end) s[r] = -INFINITY;
+                }
+                mx = fmaxf(s[0], s[1]);
+            } else if (q < 4) {
+#pragma unroll
+                for (int e = 0; e < 2; ++e) mx = fmaxf(mx, fmaxf(s[4 * q - 2 + 2 * e], s[4 * q - 1 + 2 * e]));
+            } else if (q == 4) {
+                mx = fmaxf(mx, fmaxf(s[14], s[15]));
+            } else if (q == 5) {
+                float lo, hi;
+                both_halves(mx, lo, hi);
+                mx = fmaxf(lo, hi) * sc_log2;
+            } else if (q == 6) {
+                upd = mx > m_run + RESCALE_TAU;
+                m_new = upd ? mx : m_run;
+                alpha = upd ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.0f;
+                rescale = upd && l_run > 0.f;
+                m_run = m_new;
+                lsum = 0.f;
+            } else if (q < 23) {                              // one exponential per product
+                const int r = q - 7;
+                s[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], sc_log2, -m_new));
+                lsum += s[r];
+                if (r & 1) {
+                    if (r < 8) pk0[r >> 1] = pack_bf16x2(s[r - 1], s[r]);
+                    else pk1[(r - 8) >> 1] = pack_bf16x2(s[r - 1], s[r]);
+                }
+            } else if (q == 23) {
+                *reinterpret_cast<u32x4 *>(pool_b + PT_P + pbuf * PT_P_BYTES + (w * 64 + l) * 16) = pk0;
+            } else if (q == 24) {
+                *reinterpret_cast<u32x4 *>(pool_b + PT_P + pbuf * PT_P_BYTES + ((4 + w) * 64 + l) * 16) = pk1;
+            } else if (q == 25) {
+                float lo, hi;
+                both_halves(lsum, lo, hi);
+                l_run = l_run * alpha + (lo + hi);
+            } else if (q == 26) {
+                const bool any = __any(rescale);                                        // wave-uniform
+                uint8_t *a = pool_b + PT_ALPHA + pbuf * PT_ALPHA_BYTES;
+                if (any) reinterpret_cast<float *>(a)[32 * w + col] = rescale ? alpha : 1.0f;
+                reinterpret_cast<int *>(a + 512)[w] = any ? 1 : 0;
+            }
+        };
+        // O^T += V^T . P^T of the tile at `prev` (its P^T and factors in buffer pbuf); SM: with the softmax of tile kt beside it
+        auto values = [&](auto first_tag, auto sm_tag, const uint32_t prev, const int pbuf, const int kt) {
+            constexpr bool FIRST = decltype(first_tag)::value, SM = decltype(sm_tag)::value;
+            if (!FIRST) {
+                const i32x4 fl = *reinterpret_cast<const i32x4 *>(pool_b + PT_ALPHA + pbuf * PT_ALPHA_BYTES + 512);
+                const int any = __builtin_amdgcn_readfirstlane(fl[0] | fl[1] | fl[2] | fl[3]);
+                if (__builtin_expect(any, 0)) {              // rare
+                    mfma_to_valu_fence();
+#pragma unroll
+                    for (int hb = 0; hb < 4; ++hb) {
+                        if (__builtin_amdgcn_readfirstlane(fl[hb]) == 0) continue;
+                        const float a = reinterpret_cast<const float *>(pool_b + PT_ALPHA + pbuf * PT_ALPHA_BYTES)[32 * hb + col];
+                        AccLoop<0, 4>::scale(o + 4 * hb, a);
+                    }
+                    valu_to_mfma_fence();
+                }
+            }
+#pragma unroll
+            for (int mp = 0; mp < 32; ++mp) {
+                const int kk = mp >> 4, hb = (mp >> 2) & 3, d = mp & 3;
+                if (FIRST && kk == 0) acc_mfma_first(o[4 * hb + d], vf[0][d], pf[hb & 1]);
+                else acc_mfma(o[4 * hb + d], vf[kk][d], pf[hb & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+                if (d == 0 && (kk == 0 || hb < 3)) load_p(pbuf, hb < 3 ? kk : 1, (hb + 1) & 3);
+                if (kk == 0 && hb >= 2 && (d & 1)) load_v(prev, 1, 2 * (hb - 2) + (d >> 1));
+                if (SM && mp > 0) softmax_step(mp - 1, kt, pbuf ^ 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        auto turn = [&]() {                                   // the next tile has landed for every wave; this one's P^T is there
+            __builtin_amdgcn_s_waitcnt(0x0F70);
+            __syncthreads();
+        };
+        if (k_begin < k_end) {
+            uint32_t cur = 0, next = PT_BYTES, prev = 2 * PT_BYTES;
+            int pbuf = 0;                                     // of the tile at cur
+            scores(std::false_type{}, cur, prev, next, k_begin, 0);
+#pragma unroll
+            for (int q = 0; q < 30; ++q) softmax_step(q, k_begin, 0);
+            turn();
+            auto step = [&](auto first_tag, const int kt) {
+                const uint32_t t3 = prev;
+                prev = cur;
+                cur = next;
+                next = t3;
+                scores(std::true_type{}, cur, prev, next, kt, pbuf);
+                values(first_tag, std::true_type{}, prev, pbuf, kt);
+                pbuf ^= 1;
+                turn();
+            };
+            auto last = [&](auto first_tag) {                 // the products against V of the last tile
+#pragma unroll
+                for (int d = 0; d < 4; ++d) load_v(cur, 0, d);
+                load_p(pbuf, 0, 0);
+                values(first_tag, std::false_type{}, cur, pbuf, 0);
+            };
+            if (k_begin + KT < k_end) {
+                step(std::true_type{}, k_begin + KT);
+                for (int kt = k_begin + 2 * KT; kt < k_end; kt += KT) step(std::false_type{}, kt);
+                last(std::false_type{});
+            } else {
+                last(std::true_type{});
+            }
+        }
+        __syncthreads();                                      // every wave is done with the tile buffers
+    } else {
         if (k_begin < k_end) {
             tile_step(std::integral_constant<int, 0>{}, std::true_type{}, k_begin);
             if (k_begin + KT < k_end) tile_step(std::integral_constant<int, 1>{}, std::false_type{}, k_begin + KT);
@@ -833,9 +1035,17 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
         // of head h is stored at chunk c ^ h: the column-wise writes (32 heads, one chunk) and the
         // row-wise reads (two heads, 16 even or odd chunks each) both touch every bank once.
         uint8_t *stage = reinterpret_cast<uint8_t *>(pool) + w * (32 * 256);
-        const int head_base = hg * (32 * HG) + hgw * 32;
+        const int head_base = hg * (32 * HG) + (PIPE ? 0 : hgw * 32);
         const size_t prow_base = ((size_t)(t - 8 * p.whole_slots) * nsplit + sp) * p.NQ;    // split rows only
-        const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
+        float inv[PIPE ? 4 : 1];                          // of this lane's head in each head group (PIPE) or its own
+        inv[0] = l_run > 0.f ? 1.0f / l_run : 0.f;
+        if constexpr (PIPE) {
+            float *il = reinterpret_cast<float *>(pool_b + PT_ALPHA);
+            if (half == 0) il[32 * w + col] = inv[0];
+            __syncthreads();
+#pragma unroll
+            for (int hb = 0; hb < 4; ++hb) inv[hb] = il[32 * hb + col];
+        }
         // FINAL: bf16 result rows; otherwise fp16 partial of a key split (O / l of the split, merged by
         // the combine kernel with weights l * 2^(m - m_max); O / l is a convex combination of
         // de-quantised V rows, so it stays finite in fp16 as long as |int8 * scale| < 65504).
@@ -845,8 +1055,10 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
             constexpr bool FINAL = decltype(final_tag)::value;
             constexpr bool ALL = decltype(all_tag)::value;
             const int hsub = l >> 4, j = l & 15;          // on the way out: head 4*e + hsub, channels 8*j .. 8*j+7
-            uint16_t *dst0 = FINAL ? p.out + ((size_t)t * p.NQ + head_base + hsub) * DN + part * (32 * DVP) + 8 * j
-                                   : p.part_o + (prow_base + head_base + hsub) * DN + part * (32 * DVP) + 8 * j;
+            // chunk gq: 128 channels of the wave's heads, or (PIPE) the wave's 128 channels of head group gq
+            const int ch0 = PIPE ? 128 * w : part * (32 * DVP);
+            uint16_t *dst0 = FINAL ? p.out + ((size_t)t * p.NQ + head_base + hsub) * DN + ch0 + 8 * j
+                                   : p.part_o + (prow_base + head_base + hsub) * DN + ch0 + 8 * j;
 #pragma unroll
             for (int gq = 0; gq < DVP / 4; ++gq) {
 #pragma unroll
@@ -859,7 +1071,8 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
                         asm volatile("v_accvgpr_read_b32 %0, %4\n\tv_accvgpr_read_b32 %1, %5\n\tv_accvgpr_read_b32 %2, %6\n\tv_accvgpr_read_b32 %3, %7"
                                      : "=&v"(r0), "=&v"(r1), "=&v"(r2), "=&v"(r3)
                                      : "a"(acc[4 * q4]), "a"(acc[4 * q4 + 1]), "a"(acc[4 * q4 + 2]), "a"(acc[4 * q4 + 3]));
-                        const float v0 = r0 * inv, v1 = r1 * inv, v2 = r2 * inv, v3 = r3 * inv;
+                        const float iv = inv[PIPE ? gq : 0];
+                        const float v0 = r0 * iv, v1 = r1 * iv, v2 = r2 * iv, v3 = r3 * iv;
                         u32x2 pk;
                         pk[0] = FINAL ? pack_bf16x2(v0, v1) : pack_f16x2(v0, v1);
                         pk[1] = FINAL ? pack_bf16x2(v2, v3) : pack_f16x2(v2, v3);
@@ -885,13 +1098,13 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
                         const int hl = 4 * (e0 + e) + hsub;
                         asm volatile("" : "+v"(lo[e]), "+v"(hi[e]));
                         const u32x4 v = {lo[e][0], lo[e][1], hi[e][0], hi[e][1]};
-                        if (ALL || head_base + hl < p.NQ)
-                            *reinterpret_cast<u32x4 *>(dst0 + (size_t)(4 * (e0 + e)) * DN + 128 * gq) = v;
+                        if (ALL || head_base + hl + (PIPE ? 32 * gq : 0) < p.NQ)
+                            *reinterpret_cast<u32x4 *>(dst0 + (size_t)(4 * (e0 + e) + (PIPE ? 32 * gq : 0)) * DN + (PIPE ? 0 : 128 * gq)) = v;
                     }
                 }
             }
         };
-        const bool all_heads = head_base + 32 <= p.NQ;
+        const bool all_heads = head_base + (PIPE ? 128 : 32) <= p.NQ;
         if (nsplit == 1) {
             if (all_heads) drain(std::true_type{}, std::true_type{});
             else drain(std::true_type{}, std::false_type{});
