@@ -49,7 +49,8 @@ struct LipParams {
 constexpr int LIP_SUMS_DEFAULT = 0;        // the query rows' Hadamard sums on the matrix cores, everything else fixed-order
 constexpr int LIP_SUMS_EXACT = 1;          // every sum in its fixed order
 constexpr int LIP_SUMS_MATRIX_CORES = 2;   // the sums over the hidden axis on the matrix cores as well
-constexpr int LIP_MFMA_MIN_TOKENS = 64;
+constexpr int LIP_MFMA_MIN_TOKENS = 16;
+constexpr int LIP_UNSPLIT_MIN_TOKENS = 64;   // = QPROJ_PREFILL_TOKENS (prolog_common.h)
 constexpr int LIP_XM_MAX_SPLITS = 16;    // ranges of the hidden axis (partial sums per token) of the matrix-core form, at most
 
 __host__ __device__ inline bool lip_q_on_matrix_cores(const LipParams &p)
@@ -72,7 +73,8 @@ __host__ __device__ inline bool lip_x_group_width(const LipParams &p)
 __host__ __device__ inline bool lip_x_group_rows(const LipParams &p)
 {
     if (p.x_in_groups) return true;
-    return p.T >= LIP_MFMA_MIN_TOKENS && !lip_x_on_matrix_cores(p) && lip_x_group_width(p);
+    // (below 64 tokens with every sum in its fixed order the decode form's launch takes these sums and the projection together)
+    return (lip_q_on_matrix_cores(p) || p.T >= LIP_UNSPLIT_MIN_TOKENS) && !lip_x_on_matrix_cores(p) && lip_x_group_width(p);
 }
 // partial rows [T, LIP_XCOLS] the first launch leaves per token: the blocks of 64 of the fixed-order form, or the
 // ranges of the matrix-core form (enough of them for about 512 workgroups of 128 tokens x 128 columns: two per compute unit)

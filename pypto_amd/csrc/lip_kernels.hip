@@ -51,6 +51,7 @@
 namespace pto {
 namespace {
 
+static_assert(LIP_UNSPLIT_MIN_TOKENS == QPROJ_PREFILL_TOKENS, "the launcher and the last stage disagree about the projection's form");
 static_assert(LIP_KSPLIT == QPROJ_KSPLIT, "workspace sizing and the projection job disagree");
 
 // ---------------------------------------------------------------------------------------------
@@ -153,7 +154,7 @@ hipError_t lip_launch_linear(const LipParams &p, hipStream_t stream)
     const int tblocks = (p.T + 31) / 32;
     const bool unsplit = qproj_splits(p.T) == 1;      // prefill sizes: the query projection as a launch of its own
     const int q_jobs = unsplit ? 0 : p.n_heads * LIP_KSPLIT * tblocks;
-    if (unsplit && lip_q_on_matrix_cores(p)) {
+    if (lip_q_on_matrix_cores(p)) {
         if (x_done) return hipSuccess;                // the projection is part of the last launch
     } else if (unsplit) {
         if (p.q_lora % (32 * QPF_STEPS)) return hipErrorInvalidValue;

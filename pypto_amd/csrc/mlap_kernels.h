@@ -81,7 +81,9 @@ struct MlapRider {
 // the stages' prefill forms (matrix-core sums over the hidden axis, last stage per head and run of token blocks)
 __host__ __device__ inline bool mlap_prefill_forms(const MlapParams &p) { return p.T >= MLAP_MFMA_MIN_TOKENS && !p.absorb_exact; }
 // from PROLOG_PF_MIN_TOKENS tokens on the projection and the last stage are one launch (prolog_prefill.h)
-constexpr int PROLOG_PF_MIN_TOKENS = 64;
+// (as two launches and more, as before: 16 tokens 38.6 us per pass of the fused prolog, now 37.1; 32: 41.6, 39.1; 48: 48.2,
+// 41.6; 9 tokens the other way, 34.3 against 36.8)
+constexpr int PROLOG_PF_MIN_TOKENS = 16;
 __host__ __device__ inline bool mlap_fused_projection(const MlapParams &p) { return mlap_prefill_forms(p) && p.T >= PROLOG_PF_MIN_TOKENS; }
 // partial sums per output the int8 projection leaves: 1 = unsplit (de-quantised bf16), else QPROJ_KSPLIT_HOST int32 partials
 __host__ __device__ inline int mlap_qsplits(const MlapParams &p)
@@ -95,12 +97,10 @@ hipError_t mlap_launch(const MlapParams &p, hipStream_t stream);
 // all launches but the last (which from PROLOG_PF_MIN_TOKENS tokens on holds the projection too), and the number of
 // workgroups of the last (for the fused operator's last launch)
 // lip_rider (prefill forms only): the indexer prolog whose fixed-order sums over the hidden axis (left as group sums:
-// LipParams::x_in_groups) ride in this operator's first launch or, below 64 tokens and then with its split int8
-// projection, in the third
+// LipParams::x_in_groups) ride in this operator's first launch or, below PROLOG_PF_MIN_TOKENS tokens and then with its
+// split int8 projection, in the third
 struct LipParams;
 hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const MlapRider *rider = nullptr, const LipParams *lip_rider = nullptr);
-// whether the launches of `p` take such a rider
-inline bool mlap_takes_lip_rider(const MlapParams &p) { return mlap_prefill_forms(p); }
 int mlap_finish_wgs(const MlapParams &p);
 // the last launch alone; at prefill sizes (mlap_finish_is_prefill) it has a form of its own that the fused operator
 // launches beside, not inside, its own last launch

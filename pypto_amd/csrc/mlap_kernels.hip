@@ -35,11 +35,11 @@
 //                        instead (the rotated key allows no outlier under the reference's acceptance rule).
 //   mlap_mid_prefill_kernel    the middle stage as a wave per token and latent (64 tokens and more)
 //   qproj_prefill_kernel   the projection unsplit (prolog_common.h), a workgroup per tile over the whole reduction axis;
-//                        results leave de-quantised (up to 63 tokens, and in the fixed-order mode, which has
+//                        results leave de-quantised (up to 15 tokens, and in the fixed-order mode, which has
 //                        qproj_prefill256_kernel for more).
 //   mlap_finish_prefill_kernel   per (head, run of 32-token blocks): the head's whole w_uk staged once
-//                        (prolog_finish.h), absorb product on the matrix cores (up to 63 tokens).
-// From 64 tokens on the projection and the last stage are one launch (prolog_prefill.h).
+//                        (prolog_finish.h), absorb product on the matrix cores (up to 15 tokens).
+// From PROLOG_PF_MIN_TOKENS tokens on the projection and the last stage are one launch (prolog_prefill.h).
 #include <cstring>
 
 #include "mlap_kernels.h"
@@ -105,7 +105,7 @@ static_assert(XM_KC == MLAP_XBLOCK, "the workspace is sized in chunks of the hid
 // sequential sums), 64 columns each: the rope columns of w_dkv_kr at every size -- the reference's acceptance rule allows
 // the rotated key no outlier at all (deepseekv32_mla_prolog_quant.py:688: atol 1e-4, rtol 2^-7 per element, ratio 0), and
 // a sum that lands next to a bf16 rounding boundary in another order moves a small rotated value by more than that --
-// and, in the fused prolog from 64 tokens on, the indexer prolog's wk and w_proj.  They are short and follow the long workgroups of the
+// and, in the fused prolog from PROLOG_PF_MIN_TOKENS tokens on, the indexer prolog's wk and w_proj.  They are short and follow the long workgroups of the
 // other slabs, so they fill the launch's last round; two workgroups fit a compute unit.  (1000 tokens: 69 us here and 79
 // in a launch of the indexer's own before they shared it.)
 // TB: at most 32 * TB tokens (xm_small_body), 0 for tiles of 128 tokens (xm_body), XM_BIG for tiles of 256 (xb_body).
@@ -556,7 +556,7 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
     const int ngroups_fixed = ngroups;
     const int nslabs = p.q_lora / 128 + 5;
     if (rider != nullptr && !mlap_takes_rider(p)) return hipErrorInvalidValue;
-    if (lip_rider != nullptr && !mlap_takes_lip_rider(p)) return hipErrorInvalidValue;
+    if (lip_rider != nullptr && !mlap_takes_lip_rider(p, *lip_rider)) return hipErrorInvalidValue;
     LipParams lip;
     std::memset(&lip, 0, sizeof lip);
     if (lip_rider != nullptr) lip = *lip_rider;
@@ -585,7 +585,7 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
         }
         const int per_slab = ngroups * ttiles;
         const int wgs = big ? 8 * ((mslabs * ((p.T + XB_TOK - 1) / XB_TOK) * ngroups + 7) / 8) : 8 * ((mslabs >> 3) * per_slab + ((mslabs & 7) * per_slab + 7) / 8);   // the kernel's XCD-wise job order
-        const int sets = 1 + (lip_rider != nullptr && p.T >= QPROJ_PREFILL_TOKENS ? LIP_XF_SETS : 0);
+        const int sets = 1 + (lip_rider != nullptr && mlap_fused_projection(p) ? LIP_XF_SETS : 0);
         const dim3 g((unsigned)(wgs + xf_jobs(sets, ngroups_fixed, p.T)));
 #define XM_LAUNCH(TBV) hipLaunchKernelGGL(mlap_xlinear_mfma_kernel<TBV>, g, dim3(256), 0, stream, p, mslabs, ngroups, wgs, sets, ngroups_fixed, lip)
         if (p.T <= 32) XM_LAUNCH(1);
@@ -641,7 +641,7 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
     case 12: hipLaunchKernelGGL((qproj_prefill_kernel<TBV, 6>), gr, b, 0, stream, qp, njobs, qr, lip, ngroups_fixed, fixed_wgs); break;    \
     default: return hipErrorInvalidValue;                                                                    \
     }
-            if (tbk == 1) { QPF_RIDER(1) } else { QPF_RIDER(2) }
+            QPF_RIDER(1)                               // (fewer tokens than PROLOG_PF_MIN_TOKENS: one block)
 #undef QPF_RIDER
             return hipGetLastError();
         }

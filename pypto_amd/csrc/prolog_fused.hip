@@ -7,13 +7,14 @@
 // indexer's query rows, key row and weights (54 KB, eight waves) do not depend on each other and fit a compute
 // unit together, so they run side by side instead of one launch after the other.  Where the indexer prolog cannot
 // ride (other than 64 indexer heads) its first launch follows the MLA prolog's third.  From 9 tokens on the MLA
-// prolog's prefill forms take the indexer prolog's fixed-order sums along, up to 63 tokens its projection too (five
-// launches; four up to 32 tokens, where the two last stages share one); from 64 tokens on both projections and all that
-// follows them are one launch (three in all).
+// prolog's prefill forms take the indexer prolog's fixed-order sums along, up to 15 tokens its projection too (four
+// launches, the two last stages sharing one); from 16 tokens on both projections and all that follows them are one launch
+// (three in all).
 #include <cstring>
 
 #include "prolog_fused.h"
 #include "prolog_prefill.h"
+#include "lip_xjob.h"
 
 namespace pto {
 namespace {
@@ -111,18 +112,17 @@ hipError_t prolog_fused_launch(const MlapParams &pm, const LipParams &pl, hipStr
                            mla_wgs, q_wgs);
         return hipGetLastError();
     }
-    // From 9 tokens on the MLA prolog runs its prefill forms, which take the indexer prolog's fixed-order sums along in
-    // the first launch or, up to 63 tokens, in the third with its split projection (the third launch's workgroups leave
-    // half of every compute unit free); up to 32 tokens the finishing stages of the two halves share the last launch:
-    // four launches, five up to 63 tokens.
-    const bool lip_rides = mlap_takes_lip_rider(pm) && pl.T == pm.T && pl.h == pm.h && pl.q_lora == pm.q_lora && pl.x == pm.x &&
+    // From 9 tokens on the MLA prolog runs its prefill forms, which take the indexer prolog's fixed-order sums along: up to 15
+    // tokens in the third launch beside its split projection (that launch's workgroups leave half of every compute unit
+    // free) with the finishing stages of the two halves sharing the last; beyond, in the first.
+    const bool lip_rides = mlap_takes_lip_rider(pm, pl) && pl.T == pm.T && pl.h == pm.h && pl.q_lora == pm.q_lora && pl.x == pm.x &&
                            pl.q_norm == pm.q_norm && pl.q_norm_scale == pm.q_norm_scale && !lip_x_on_matrix_cores(pl) &&
                            lip_x_group_width(pl) && pl.n_heads <= LIP_MAX_HEADS;
     LipParams px = pl;
     if (lip_rides) px.x_in_groups = 1;
     hipError_t e = mlap_launch_front(pm, stream, nullptr, lip_rides ? &px : nullptr);
     if (e != hipSuccess) return e;
-    if (!lip_rides || px.T >= QPROJ_PREFILL_TOKENS) {
+    if (!lip_rides || mlap_fused_projection(pm)) {
         e = lip_launch_linear(px, stream);
         if (e != hipSuccess) return e;
     }
