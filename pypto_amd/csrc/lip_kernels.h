@@ -49,7 +49,7 @@ struct LipParams {
 constexpr int LIP_SUMS_DEFAULT = 0;        // the query rows' Hadamard sums on the matrix cores, everything else fixed-order
 constexpr int LIP_SUMS_EXACT = 1;          // every sum in its fixed order
 constexpr int LIP_SUMS_MATRIX_CORES = 2;   // the sums over the hidden axis on the matrix cores as well
-constexpr int LIP_MFMA_MIN_TOKENS = 16;
+constexpr int LIP_MFMA_MIN_TOKENS = 9;
 constexpr int LIP_UNSPLIT_MIN_TOKENS = 64;   // = QPROJ_PREFILL_TOKENS (prolog_common.h)
 constexpr int LIP_XM_MAX_SPLITS = 16;    // ranges of the hidden axis (partial sums per token) of the matrix-core form, at most
 

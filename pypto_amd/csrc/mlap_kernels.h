@@ -80,11 +80,10 @@ struct MlapRider {
 
 // the stages' prefill forms (matrix-core sums over the hidden axis, last stage per head and run of token blocks)
 __host__ __device__ inline bool mlap_prefill_forms(const MlapParams &p) { return p.T >= MLAP_MFMA_MIN_TOKENS && !p.absorb_exact; }
-// from PROLOG_PF_MIN_TOKENS tokens on the projection and the last stage are one launch (prolog_prefill.h)
-// (as two launches and more, as before: 16 tokens 38.6 us per pass of the fused prolog, now 37.1; 32: 41.6, 39.1; 48: 48.2,
-// 41.6; 9 tokens the other way, 34.3 against 36.8)
-constexpr int PROLOG_PF_MIN_TOKENS = 16;
-__host__ __device__ inline bool mlap_fused_projection(const MlapParams &p) { return mlap_prefill_forms(p) && p.T >= PROLOG_PF_MIN_TOKENS; }
+// unless every sum is to keep its fixed order the projection and the last stage are one launch (prolog_small.h up to
+// PROLOG_SMALL_TOKENS tokens, prolog_prefill.h beyond)
+constexpr int PROLOG_SMALL_TOKENS = 32;
+__host__ __device__ inline bool mlap_fused_projection(const MlapParams &p) { return !p.absorb_exact; }
 // partial sums per output the int8 projection leaves: 1 = unsplit (de-quantised bf16), else QPROJ_KSPLIT_HOST int32 partials
 __host__ __device__ inline int mlap_qsplits(const MlapParams &p)
 {

@@ -14,6 +14,7 @@
 
 #include "prolog_fused.h"
 #include "prolog_prefill.h"
+#include "prolog_small.h"
 #include "lip_xjob.h"
 
 namespace pto {
@@ -69,6 +70,18 @@ __global__ __launch_bounds__(256, 2) void prolog_prefill_kernel(const MlapParams
     else lip_finish_tokens_prefill_body(pl, wg - mla_wgs - lip_wgs, lds);
 }
 
+// The same for at most PROLOG_SMALL_TOKENS tokens (prolog_small.h), a workgroup per head.
+constexpr int PS_LDS = PSA_LDS > PSI_LDS ? PSA_LDS : PSI_LDS;
+static_assert(LIP_FINT_LDS <= PS_LDS, "the token workgroups fit");
+__global__ __launch_bounds__(256) void prolog_small_kernel(const MlapParams pm, const LipParams pl, const int mla_wgs, const int lip_wgs)
+{
+    __shared__ __attribute__((aligned(16))) uint8_t lds[PS_LDS];
+    const int wg = (int)blockIdx.x;
+    if (wg < mla_wgs) mlap_small_body(pm, wg, lds);
+    else if (wg < mla_wgs + lip_wgs) lip_small_body(pl, wg - mla_wgs, lds);
+    else lip_finish_tokens_prefill_body(pl, wg - mla_wgs - lip_wgs, lds);
+}
+
 }  // namespace
 
 hipError_t prolog_prefill_launch(const MlapParams *pm, const LipParams *pl, hipStream_t stream)
@@ -80,6 +93,11 @@ hipError_t prolog_prefill_launch(const MlapParams *pm, const LipParams *pl, hipS
     std::memset(&p, 0, sizeof p);
     if (pm) m = *pm;
     if (pl) p = *pl;
+    if (T <= PROLOG_SMALL_TOKENS) {
+        const int mla = pm ? m.n_heads : 0, lip = pl ? p.n_heads : 0, tok = pl ? (T + FINT_WAVES - 1) / FINT_WAVES : 0;
+        hipLaunchKernelGGL(prolog_small_kernel, dim3((unsigned)(mla + lip + tok)), dim3(256), 0, stream, m, p, mla, lip);
+        return hipGetLastError();
+    }
     // 256-token tiles take 12 % less time per (padded) token than 128-token ones where both fill the chip, which up to 256
     // tokens they do not (256 tokens: 79.6 us per pass against 77.5; 600: 150.4 against 140.3; 1000: 188.5 against 206.6)
     const bool small = T <= 256 || 100 * ((T + 127) / 128) <= 176 * ((T + 255) / 256);
@@ -106,6 +124,7 @@ hipError_t prolog_fused_launch(const MlapParams &pm, const LipParams &pl, hipStr
         if (e != hipSuccess) return e;
         LipParams pg = pl;
         pg.x_in_groups = 1;
+        if (mlap_fused_projection(pm)) return prolog_prefill_launch(&pm, &pg, stream);
         const int mla_wgs = mlap_finish_wgs(pm);
         const int q_wgs = lip_finish_query_wgs(pg);
         hipLaunchKernelGGL(prolog_fused_finish_kernel, dim3((unsigned)(mla_wgs + q_wgs + pg.T)), dim3(64 * FIN_WAVES), 0, stream, pm, pg,
@@ -126,7 +145,12 @@ hipError_t prolog_fused_launch(const MlapParams &pm, const LipParams &pl, hipStr
         e = lip_launch_linear(px, stream);
         if (e != hipSuccess) return e;
     }
-    if (mlap_fused_projection(pm) && lip_q_on_matrix_cores(px)) return prolog_prefill_launch(&pm, &px, stream);
+    if (mlap_fused_projection(pm)) {
+        if (lip_q_on_matrix_cores(px)) return prolog_prefill_launch(&pm, &px, stream);
+        e = mlap_launch_finish(pm, stream);
+        if (e != hipSuccess) return e;
+        return lip_launch_finish(px, stream);
+    }
     int per = 0, pf_wgs = 0;
     if (mlap_finish_is_prefill(pm)) mlap_finish_prefill_shape(pm, per, pf_wgs);
     // up to 32 tokens: one workgroup per head, the indexer half's take the other compute units (more would queue one

@@ -102,6 +102,29 @@ template <int XC, int TB> constexpr int PFA_LOOP_LDS = 2 * PFA_X<XC, TB> + 3 * P
 template <int XC, int TB> constexpr int PFA_LDS = PFA_LOOP_LDS<XC, TB> > PFA_Q<TB> ? PFA_LOOP_LDS<XC, TB> : PFA_Q<TB>;
 static_assert(PFA_RPITCH <= MLAP_NOPE * 2, "the rope rows fit where the nope operand goes");
 
+// Lane (row, e) of the rope rows at `rows` rotates pairs 4e .. 4e+3 of token t (channels 2j, 2j+1 are the partners j, 32 + j) and
+// stores them; rows of tokens past the end are read and dropped.
+__device__ __forceinline__ void pfa_rotate_rows(const MlapParams &p, const uint8_t *rows, const int row, const int t, const int head, const int e)
+{
+    const size_t tt = t < p.T ? t : p.T - 1;
+    const u32x4 x = *reinterpret_cast<const u32x4 *>(rows + row * PFA_RPITCH + 16 * e);
+    const u32x2 c0 = *reinterpret_cast<const u32x2 *>(p.cos + tt * MLAP_ROPE + 4 * e), c1 = *reinterpret_cast<const u32x2 *>(p.cos + tt * MLAP_ROPE + 32 + 4 * e);
+    const u32x2 s0 = *reinterpret_cast<const u32x2 *>(p.sin + tt * MLAP_ROPE + 4 * e), s1 = *reinterpret_cast<const u32x2 *>(p.sin + tt * MLAP_ROPE + 32 + 4 * e);
+    float r0[4], r1[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        auto at = [&](const u32x2 &q) { return __uint_as_float((j & 1) ? q[j >> 1] & 0xffff0000u : q[j >> 1] << 16); };
+        const float v0 = __uint_as_float(x[j] << 16), v1 = __uint_as_float(x[j] & 0xffff0000u);
+        r0[j] = __builtin_fmaf(v0, at(c0), (-v1) * at(s0));                   // products exact: one rounding
+        r1[j] = __builtin_fmaf(v1, at(c1), v0 * at(s1));
+    }
+    if (t < p.T) {
+        uint16_t *out = p.q_rope + (tt * p.n_heads + head) * MLAP_ROPE + 4 * e;
+        *reinterpret_cast<u32x2 *>(out) = u32x2{pack_bf16x2(r0[0], r0[1]), pack_bf16x2(r0[2], r0[3])};
+        *reinterpret_cast<u32x2 *>(out + 32) = u32x2{pack_bf16x2(r1[0], r1[1]), pack_bf16x2(r1[2], r1[3])};
+    }
+}
+
 template <int XC, int TB>
 __device__ __forceinline__ void mlap_prefill_body(const MlapParams &p, const int job, uint8_t *lds)
 {
@@ -204,23 +227,7 @@ __device__ __forceinline__ void mlap_prefill_body(const MlapParams &p, const int
 #pragma unroll
         for (int k = 0; k < 2 * TB; ++k) {
             const int tr = 8 * (2 * TB * w + k) + (l >> 3);
-            const size_t tt = token(tr);
-            const u32x4 x = *reinterpret_cast<const u32x4 *>(lds + tr * PFA_RPITCH + 16 * e);
-            const u32x2 c0 = *reinterpret_cast<const u32x2 *>(p.cos + tt * MLAP_ROPE + 4 * e), c1 = *reinterpret_cast<const u32x2 *>(p.cos + tt * MLAP_ROPE + 32 + 4 * e);
-            const u32x2 s0 = *reinterpret_cast<const u32x2 *>(p.sin + tt * MLAP_ROPE + 4 * e), s1 = *reinterpret_cast<const u32x2 *>(p.sin + tt * MLAP_ROPE + 32 + 4 * e);
-            float r0[4], r1[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                auto at = [&](const u32x2 &q) { return __uint_as_float((j & 1) ? q[j >> 1] & 0xffff0000u : q[j >> 1] << 16); };
-                const float v0 = __uint_as_float(x[j] << 16), v1 = __uint_as_float(x[j] & 0xffff0000u);
-                r0[j] = __builtin_fmaf(v0, at(c0), (-v1) * at(s0));                   // products exact: one rounding
-                r1[j] = __builtin_fmaf(v1, at(c1), v0 * at(s1));
-            }
-            if (t0 + tr < p.T) {
-                uint16_t *out = p.q_rope + (tt * p.n_heads + head) * MLAP_ROPE + 4 * e;
-                *reinterpret_cast<u32x2 *>(out) = u32x2{pack_bf16x2(r0[0], r0[1]), pack_bf16x2(r0[2], r0[3])};
-                *reinterpret_cast<u32x2 *>(out + 32) = u32x2{pack_bf16x2(r1[0], r1[1]), pack_bf16x2(r1[2], r1[3])};
-            }
+            pfa_rotate_rows(p, lds, tr, t0 + tr, head, e);
         }
         __syncthreads();
     }
