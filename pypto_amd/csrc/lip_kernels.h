@@ -45,11 +45,12 @@ struct LipParams {
                                  // operator's launch (the fused prolog); set by that launcher only
 };
 
-// How the fp32 sums are taken from LIP_MFMA_MIN_TOKENS tokens on (below that every sum has its fixed order):
+// How the fp32 sums are taken from LIP_MFMA_MIN_TOKENS tokens on (below that every sum has its fixed order, in every mode:
+// that is part of the interface):
 constexpr int LIP_SUMS_DEFAULT = 0;        // the query rows' Hadamard sums on the matrix cores, everything else fixed-order
 constexpr int LIP_SUMS_EXACT = 1;          // every sum in its fixed order
 constexpr int LIP_SUMS_MATRIX_CORES = 2;   // the sums over the hidden axis on the matrix cores as well
-constexpr int LIP_MFMA_MIN_TOKENS = 9;
+constexpr int LIP_MFMA_MIN_TOKENS = 64;
 constexpr int LIP_UNSPLIT_MIN_TOKENS = 64;   // = QPROJ_PREFILL_TOKENS (prolog_common.h)
 constexpr int LIP_XM_MAX_SPLITS = 16;    // ranges of the hidden axis (partial sums per token) of the matrix-core form, at most
 
@@ -57,7 +58,8 @@ __host__ __device__ inline bool lip_q_on_matrix_cores(const LipParams &p)
 {
     return p.T >= LIP_MFMA_MIN_TOKENS && p.sum_mode != LIP_SUMS_EXACT;
 }
-// (those rows are finished where the projection makes them: prolog_prefill.h)
+// (those rows are finished where the projection makes them: prolog_prefill.h.  In the fused prolog rows of fewer tokens are too,
+// with their sums in the fixed order: prolog_small.h and the FIXED form of prolog_prefill.h.)
 // the hidden-axis form needs w_proj rows made of whole 16-byte pieces
 __host__ __device__ inline bool lip_x_on_matrix_cores(const LipParams &p)
 {
@@ -73,8 +75,8 @@ __host__ __device__ inline bool lip_x_group_width(const LipParams &p)
 __host__ __device__ inline bool lip_x_group_rows(const LipParams &p)
 {
     if (p.x_in_groups) return true;
-    // (below 64 tokens with every sum in its fixed order the decode form's launch takes these sums and the projection together)
-    return (lip_q_on_matrix_cores(p) || p.T >= LIP_UNSPLIT_MIN_TOKENS) && !lip_x_on_matrix_cores(p) && lip_x_group_width(p);
+    // (below 64 tokens the decode form's launch takes these sums and the projection together)
+    return p.T >= LIP_UNSPLIT_MIN_TOKENS && !lip_x_on_matrix_cores(p) && lip_x_group_width(p);
 }
 // partial rows [T, LIP_XCOLS] the first launch leaves per token: the blocks of 64 of the fixed-order form, or the
 // ranges of the matrix-core form (enough of them for about 512 workgroups of 128 tokens x 128 columns: two per compute unit)

@@ -128,11 +128,7 @@ __device__ __forceinline__ XlSlab lip_xf_slab(const LipParams &p, const int set,
 
 }  // namespace
 
-// whether the launches of `p` take the indexer prolog's fixed-order sums along: with its split projection as well while the
-// attention query's projection is a launch of its own, alone where both queries are projected in the last launch
-inline bool mlap_takes_lip_rider(const MlapParams &p, const LipParams &lip)
-{
-    return mlap_prefill_forms(p) && (mlap_fused_projection(p) ? lip_q_on_matrix_cores(lip) || p.T >= QPROJ_PREFILL_TOKENS : !lip_q_on_matrix_cores(lip));
-}
+// whether the launches of `p` take the indexer prolog's fixed-order sums along
+inline bool mlap_takes_lip_rider(const MlapParams &p) { return mlap_prefill_forms(p); }
 
 }  // namespace pto

@@ -556,7 +556,7 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
     const int ngroups_fixed = ngroups;
     const int nslabs = p.q_lora / 128 + 5;
     if (rider != nullptr && !mlap_takes_rider(p)) return hipErrorInvalidValue;
-    if (lip_rider != nullptr && !mlap_takes_lip_rider(p, *lip_rider)) return hipErrorInvalidValue;
+    if (lip_rider != nullptr && !mlap_takes_lip_rider(p)) return hipErrorInvalidValue;
     LipParams lip;
     std::memset(&lip, 0, sizeof lip);
     if (lip_rider != nullptr) lip = *lip_rider;

@@ -367,6 +367,75 @@ __device__ __forceinline__ float lip_quant_rows(f32x16 (&c)[4], uint8_t *mine, c
     return deq;
 }
 
+// The same from the Hadamard product's operands, with its sums in their fixed order: 32 rows of rotated query channels (bf16,
+// HB_PITCH elements apart) times the matrix (plain rows), both in LDS, by a workgroup of four waves; the first T rows leave for
+// rows 0 .. T - 1 of q_int8 and q_scale at head `head`.  v_mfma_f32_16x16x1_4b_f32 multiplies one row of the matrix at a time, so
+// each of its results is one exact product added with one rounding (as in xlinear_fixed.h) and a chain of 128 is the sequential
+// sum.  Wave w makes columns 32*w .. +31: block b of the instruction is 16 of them (b / 2) x 16 rows (b % 2).
+// Bound: the matrix cores' fp32 rate, 128 x 32 clocks per wave.  (Fused prolog, 32 tokens: 42.3 us per pass; with the sums on the
+// vector ALU, a wave per row, 51.7; 16 tokens 39.8 and 41.9; 4 and 8 tokens the same.)
+// scratch: HB_SCRATCH bytes that nothing else of the workgroup uses.  The rows and the matrix have to be complete (barrier).
+constexpr int HB_PITCH = LIP_DIM + 8;
+constexpr int HB_SCRATCH = 32 * QFP_OPITCH + 4 * 32 * 4;
+__device__ __forceinline__ void lip_fixed_rows(const uint16_t *rows, const uint16_t *hmat, uint8_t *scratch, int8_t *q_int8, uint16_t *q_scale,
+                                               const int n_heads, const int head, const int T, const int w, const int l)
+{
+    const int i = l & 15, q = l >> 4;
+    f32x16 c;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) c[r] = 0.f;
+    const uint16_t *hp = hmat + 32 * w + 16 * (q >> 1) + i;
+    const uint16_t *ap = rows + (16 * (q & 1) + i) * HB_PITCH;
+#pragma unroll
+    for (int k0 = 0; k0 < LIP_DIM; k0 += 8) {
+        const u32x4 a = *reinterpret_cast<const u32x4 *>(ap + k0);
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            c = __builtin_amdgcn_mfma_f32_16x16x1f32(bf16_bits_to_f32(hp[(k0 + k) * LIP_DIM]),
+                                                     __uint_as_float((k & 1) ? a[k >> 1] & 0xffff0000u : a[k >> 1] << 16), c, 0, 0, 0);
+    }
+    // registers 4*b .. 4*b+3: columns 32*w + 16*(b / 2) + 4*q .. +3 of row 16*(b % 2) + i
+    float *mx = reinterpret_cast<float *>(scratch + 32 * QFP_OPITCH);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        float m = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int r = 4 * u + 8 * (e >> 2) + (e & 3);
+            c[r] = bf16_round_f32(c[r]);
+            m = fmaxf(m, fabsf(c[r]));
+        }
+        m = fmaxf(m, xor16_f32(m, l));
+        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+        m = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+        if (q == 0) mx[32 * w + 16 * u + i] = m;
+    }
+    __syncthreads();                                   // the four parts of every row's largest magnitude are there
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int row = 16 * u + i;
+        const float amax = fmaxf(fmaxf(mx[row], mx[32 + row]), fmaxf(mx[64 + row], mx[96 + row]));
+        float s = 0.f, deq = 0.f;
+        if (amax > 0.f) {
+            s = __fdiv_rn(127.0f, amax);
+            deq = __fdiv_rn(1.0f, s);
+        }
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            uint32_t v = 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v |= (uint32_t)((int)rintf(__fmul_rn(c[4 * u + 8 * g + j], s)) & 0xff) << (8 * j);
+            *reinterpret_cast<uint32_t *>(scratch + row * QFP_OPITCH + 32 * w + 16 * g + 4 * q) = v;
+        }
+        if (w == 0 && q == 0 && row < T) q_scale[(size_t)row * n_heads + head] = (uint16_t)(pack_f16x2(deq, 0.f) & 0xffffu);
+    }
+    __syncthreads();                                   // the int8 rows are complete
+    const int row = 8 * w + (l >> 3);
+    if (row < T)
+        *reinterpret_cast<u32x4 *>(q_int8 + ((size_t)row * n_heads + head) * LIP_DIM + 16 * (l & 7)) =
+            *reinterpret_cast<const u32x4 *>(scratch + row * QFP_OPITCH + 16 * (l & 7));
+}
+
 // ---------------------------------------------------------------------------------- MLA prolog
 constexpr int FIN_W_BYTES = MLAP_NOPE * 64 * 2;    // a wave's slice of w_uk[head]: 128 rows x 64 columns bf16
 constexpr int MLAP_FIN_LDS = 4 * FIN_W_BYTES + MLAP_XTOK * MLAP_NOPE * 4 + MLAP_XTOK * MLAP_NOPE * 2;   // 71 680 bytes

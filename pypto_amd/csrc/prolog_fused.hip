@@ -56,9 +56,10 @@ __global__ __launch_bounds__(64 * FIN_WAVES) void prolog_fused_finish_prefill_ke
 
 // Projections and last stages at prefill sizes (prolog_prefill.h): [0, mla_wgs) the attention query, then lip_wgs of the
 // indexer query, then the indexer's key rows and weights, a token per wave.  64 * TB tokens per workgroup of a head.
+// FIXED: the indexer query's Hadamard sums in their fixed order (fewer than LIP_MFMA_MIN_TOKENS tokens).
 template <int XC, int TB> constexpr int PF_LDS2 = PFA_LDS<XC, TB> > PFI_LDS<XC, TB / 2> ? PFA_LDS<XC, TB> : PFI_LDS<XC, TB / 2>;
 template <int XC, int TB> constexpr int PF_LDS = PF_LDS2<XC, TB> > LIP_FINT_LDS ? PF_LDS2<XC, TB> : LIP_FINT_LDS;
-template <int XC, int TB>
+template <int XC, int TB, bool FIXED>
 __global__ __launch_bounds__(256, 2) void prolog_prefill_kernel(const MlapParams pm, const LipParams pl, const int mla_wgs, const int lip_wgs)
 {
     static_assert(2 * PF_LDS<XC, TB> <= 160 * 1024, "two workgroups share a compute unit");
@@ -66,7 +67,7 @@ __global__ __launch_bounds__(256, 2) void prolog_prefill_kernel(const MlapParams
     __shared__ __attribute__((aligned(16))) uint8_t lds[PF_LDS<XC, TB>];
     const int wg = (int)blockIdx.x;
     if (wg < mla_wgs) mlap_prefill_body<XC, TB>(pm, q_prefill_job_of(wg, mla_wgs), lds);
-    else if (wg < mla_wgs + lip_wgs) lip_prefill_body<XC, TB / 2>(pl, q_prefill_job_of(wg - mla_wgs, lip_wgs), lds);
+    else if (wg < mla_wgs + lip_wgs) lip_prefill_body<XC, TB / 2, FIXED>(pl, q_prefill_job_of(wg - mla_wgs, lip_wgs), lds);
     else lip_finish_tokens_prefill_body(pl, wg - mla_wgs - lip_wgs, lds);
 }
 
@@ -107,8 +108,9 @@ hipError_t prolog_prefill_launch(const MlapParams *pm, const LipParams *pl, hipS
     const int lip_wgs = pl ? p.n_heads * tiles : 0;
     const int tok_wgs = pl ? (T + FINT_WAVES - 1) / FINT_WAVES : 0;
     const dim3 g((unsigned)(mla_wgs + lip_wgs + tok_wgs));
-    if (small) hipLaunchKernelGGL((prolog_prefill_kernel<2, 2>), g, dim3(256), 0, stream, m, p, mla_wgs, lip_wgs);
-    else hipLaunchKernelGGL((prolog_prefill_kernel<1, 4>), g, dim3(256), 0, stream, m, p, mla_wgs, lip_wgs);
+    if (T < LIP_MFMA_MIN_TOKENS) hipLaunchKernelGGL((prolog_prefill_kernel<2, 2, true>), g, dim3(256), 0, stream, m, p, mla_wgs, lip_wgs);
+    else if (small) hipLaunchKernelGGL((prolog_prefill_kernel<2, 2, false>), g, dim3(256), 0, stream, m, p, mla_wgs, lip_wgs);
+    else hipLaunchKernelGGL((prolog_prefill_kernel<1, 4, false>), g, dim3(256), 0, stream, m, p, mla_wgs, lip_wgs);
     return hipGetLastError();
 }
 
@@ -118,7 +120,7 @@ hipError_t prolog_fused_launch(const MlapParams &pm, const LipParams &pl, hipStr
     // axis are more column slabs of the MLA prolog's first launch and its int8 projection more jobs of the third
     // (MlapRider) -- so the pass is four launches: hidden-axis sums, latents, projections, one finish for both.
     if (mlap_takes_rider(pm) && pl.T == pm.T && pl.h == pm.h && pl.q_lora == pm.q_lora && pl.x == pm.x && pl.q_norm == pm.q_norm &&
-        pl.q_norm_scale == pm.q_norm_scale && pl.n_heads == 64 && !lip_q_on_matrix_cores(pl)) {
+        pl.q_norm_scale == pm.q_norm_scale && pl.n_heads == 64) {
         const MlapRider rd = {pl.wk, pl.w_proj, pl.xpart, pl.w_qb, pl.qpart, pl.n_heads};
         hipError_t e = mlap_launch_front(pm, stream, &rd);
         if (e != hipSuccess) return e;
@@ -131,22 +133,23 @@ hipError_t prolog_fused_launch(const MlapParams &pm, const LipParams &pl, hipStr
                            mla_wgs, q_wgs);
         return hipGetLastError();
     }
-    // From 9 tokens on the MLA prolog runs its prefill forms, which take the indexer prolog's fixed-order sums along: up to 15
-    // tokens in the third launch beside its split projection (that launch's workgroups leave half of every compute unit
-    // free) with the finishing stages of the two halves sharing the last; beyond, in the first.
-    const bool lip_rides = mlap_takes_lip_rider(pm, pl) && pl.T == pm.T && pl.h == pm.h && pl.q_lora == pm.q_lora && pl.x == pm.x &&
+    // From 9 tokens on the MLA prolog's prefill forms take the indexer prolog's fixed-order sums along in the first launch, and
+    // the last one makes and finishes both queries: three launches.  (On its own the indexer prolog keeps its two decode
+    // launches below 64 tokens: 9 tokens 14.1 us per pass against 20.6 as the sums and this last launch, 32: 18.2 and 23.7.)
+    const bool lip_rides = mlap_takes_lip_rider(pm) && pl.T == pm.T && pl.h == pm.h && pl.q_lora == pm.q_lora && pl.x == pm.x &&
                            pl.q_norm == pm.q_norm && pl.q_norm_scale == pm.q_norm_scale && !lip_x_on_matrix_cores(pl) &&
                            lip_x_group_width(pl) && pl.n_heads <= LIP_MAX_HEADS;
     LipParams px = pl;
     if (lip_rides) px.x_in_groups = 1;
     hipError_t e = mlap_launch_front(pm, stream, nullptr, lip_rides ? &px : nullptr);
     if (e != hipSuccess) return e;
-    if (!lip_rides || mlap_fused_projection(pm)) {
+    const bool joined = mlap_fused_projection(pm) && (lip_q_on_matrix_cores(px) || (lip_rides && px.T < LIP_MFMA_MIN_TOKENS));
+    if (!joined || !lip_rides) {
         e = lip_launch_linear(px, stream);
         if (e != hipSuccess) return e;
     }
+    if (joined) return prolog_prefill_launch(&pm, &px, stream);
     if (mlap_fused_projection(pm)) {
-        if (lip_q_on_matrix_cores(px)) return prolog_prefill_launch(&pm, &px, stream);
         e = mlap_launch_finish(pm, stream);
         if (e != hipSuccess) return e;
         return lip_launch_finish(px, stream);

@@ -215,15 +215,14 @@ __device__ __forceinline__ void mlap_small_body(const MlapParams &p, const int h
 
 // ------------------------------------------------------------------------------------------------- indexer query
 // Wave w projects columns 32*w .. +31; the rows then meet in LDS as bf16, a wave per row rotates them, and the Hadamard sums
-// are taken in their fixed order, a wave per row (exact), or on the matrix cores by the first wave for all rows at once.
+// are taken in their fixed order by all four waves (lip_fixed_rows).
 constexpr int PSI_SLOT = PF_KC * LIP_DIM;
 constexpr int PSI_SLOTS = 8;
-constexpr int PSI_HAD = PS_TOK;                        // the matrix: plain rows (exact), or 16-byte piece q of row r at q ^ 4*(r & 3)
+constexpr int PSI_HAD = PS_TOK;                        // the matrix, plain rows
 constexpr int PSI_RING = PSI_HAD + LIP_DIM * LIP_DIM * 2;
 constexpr int PSI_LDS = PSI_RING + PSI_SLOTS * PSI_SLOT;
-constexpr int PSI_APITCH = LIP_DIM + 8;                // elements between the rows of the operand (in the ring's place)
-constexpr int PSI_ROW = PSI_RING + 32 * PSI_APITCH * 2;// a wave's row as fp32 (exact), or the int8 rows on their way out
-static_assert(PSI_ROW + 4 * LIP_DIM * 4 <= PSI_LDS && PSI_ROW + 32 * QFP_OPITCH <= PSI_LDS, "the rows fit the ring's place");
+constexpr int PSI_SCRATCH = PSI_RING + 32 * HB_PITCH * 2;     // behind the rows, in the ring's place
+static_assert(PSI_SCRATCH + HB_SCRATCH <= PSI_LDS, "the rows fit the ring's place");
 static_assert(PSI_LDS <= 160 * 1024, "one workgroup fits a compute unit");
 
 __device__ __forceinline__ void lip_small_body(const LipParams &p, const int head, uint8_t *lds)
@@ -231,7 +230,6 @@ __device__ __forceinline__ void lip_small_body(const LipParams &p, const int hea
     const int l = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int half = l >> 5;
-    const bool exact = !lip_q_on_matrix_cores(p);
     const int ncols = p.n_heads * LIP_DIM;
     const int nch = p.q_lora / PF_KC;
     const uint32_t base = (uint32_t)(uintptr_t)(lds_byte_t *)lds;
@@ -270,7 +268,7 @@ __device__ __forceinline__ void lip_small_body(const LipParams &p, const int hea
         slot = slot == PSI_SLOTS - 1 ? 0 : slot + 1;
     }
     {   // the matrix, behind the last chunk's requests
-        const uint16_t *src = p.hq + (size_t)(32 * w + (l >> 4)) * LIP_DIM + 8 * ((l & 15) ^ (exact ? 0 : 4 * ((l >> 4) & 3)));
+        const uint16_t *src = p.hq + (size_t)(32 * w + (l >> 4)) * LIP_DIM + 8 * (l & 15);
 #pragma unroll 1
         for (int j = 0; j < 8; ++j) dma16(src + (size_t)4 * j * LIP_DIM, base + PSI_HAD + 1024 * (8 * w + j));
     }
@@ -290,63 +288,21 @@ __device__ __forceinline__ void lip_small_body(const LipParams &p, const int hea
             float f[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) f[j] = __fmul_rn(__fmul_rn((float)acc[4 * rg + j], ts), sc[rg][j]);
-            *reinterpret_cast<u32x2 *>(abf + tl * PSI_APITCH + 32 * w + 8 * rg + 4 * half) = u32x2{pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3])};
+            *reinterpret_cast<u32x2 *>(abf + tl * HB_PITCH + 32 * w + 8 * rg + 4 * half) = u32x2{pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3])};
         }
     }
     __syncthreads();                                   // the rows are complete
     const uint16_t *hmat = reinterpret_cast<const uint16_t *>(lds + PSI_HAD);
-    float *arow = reinterpret_cast<float *>(lds + PSI_ROW) + w * LIP_DIM;
     for (int t = w; t < p.T; t += 4) {
         const uint32_t rc = rope_coef(p.cos, t, l), rs = rope_coef(p.sin, t, l);
-        uint32_t *mine = reinterpret_cast<uint32_t *>(abf + t * PSI_APITCH + 2 * l);
+        uint32_t *mine = reinterpret_cast<uint32_t *>(abf + t * HB_PITCH + 2 * l);
         const uint32_t raw = *mine;
         float v0 = __uint_as_float(raw << 16), v1 = __uint_as_float(raw & 0xffff0000u);
         rope_pair(v0, v1, rc, rs, l);
-        if (exact) {
-            const f32x2 av = {v0, v1};
-            *reinterpret_cast<f32x2 *>(&arow[2 * l]) = av;         // the wave reads back what it wrote itself, in order
-            float y0, y1;
-            hadamard_pair(arow, hmat, l, y0, y1);
-            uint16_t sc;
-            const uint16_t q = quant_pair(y0, y1, sc);
-            reinterpret_cast<uint16_t *>(p.q_int8 + ((size_t)t * p.n_heads + head) * LIP_DIM)[l] = q;
-            if (l == 0) p.q_scale[(size_t)t * p.n_heads + head] = sc;
-        } else {
-            *mine = pack_bf16x2(v0, v1);
-        }
+        *mine = pack_bf16x2(v0, v1);
     }
-    if (exact) return;                                 // uniform
     __syncthreads();                                   // the rotated rows are complete
-    if (w != 0) return;
-    f32x16 cc[4];
-#pragma unroll
-    for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) cc[cb][r] = 0.f;
-    const uint16_t *at = abf + tl * PSI_APITCH + 4 * half;
-    const int arw = 4 * half + ((l & 15) >> 2);
-#pragma unroll
-    for (int ks = 0; ks < LIP_DIM / 16; ++ks) {
-        const u32x2 b0 = *reinterpret_cast<const u32x2 *>(at + 16 * ks), b1 = *reinterpret_cast<const u32x2 *>(at + 16 * ks + 8);
-        const u32x4 bq = {b0[0], b0[1], b1[0], b1[1]};
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb) {
-            const int piece = 4 * cb + 2 * ((l >> 4) & 1) + ((l & 3) >> 1);
-            const uint16_t *ap = reinterpret_cast<const uint16_t *>(lds + PSI_HAD + (16 * ks + arw) * 256 + 16 * (piece ^ (4 * ((l & 15) >> 2))) + 8 * (l & 1));
-            const s16x4 a0 = lds_read_tr16(ap), a1 = lds_read_tr16(ap + 8 * 128);
-            const s16x8 a = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
-            cc[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, bq), cc[cb], 0, 0, 0);
-        }
-    }
-    uint8_t *rows = lds + PSI_ROW;
-    const float deq = lip_quant_rows(cc, rows, l);
-    if (l < 32 && l < p.T) p.q_scale[(size_t)l * p.n_heads + head] = (uint16_t)(pack_f16x2(deq, 0.f) & 0xffffu);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int r = 8 * k + (l >> 3);
-        const u32x4 v = *reinterpret_cast<const u32x4 *>(rows + r * QFP_OPITCH + 16 * (l & 7));
-        if (r < p.T) *reinterpret_cast<u32x4 *>(p.q_int8 + ((size_t)r * p.n_heads + head) * LIP_DIM + 16 * (l & 7)) = v;
-    }
+    lip_fixed_rows(abf, hmat, lds + PSI_SCRATCH, p.q_int8, p.q_scale, p.n_heads, head, p.T, w, l);
 }
 
 }  // namespace

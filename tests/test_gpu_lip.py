@@ -206,3 +206,21 @@ def test_prolog_prefill_sizes_hidden_sums_on_matrix_cores(b, s1, act, kw):
     print(f"t={b * s1}: q_int8 off by one {float((dq != 0).mean()):.6f}, key entries off by one {float((gk != rk).mean()):.6f}, "
           f"key scales beyond 2.5e-5: {int((np.abs(gs - rs) > 2.5e-5).sum())} of {gs.size}, "
           f"weights beyond 2.5e-5: {int((np.abs(gw - rw) > 2.5e-5).sum())} of {gw.size}", flush=True)
+
+
+@pytest.mark.parametrize("mode", ["default", "matrix_cores"])
+@pytest.mark.parametrize("t,n_heads", [(1, 64), (8, 64), (9, 64), (16, 8), (16, 24), (31, 64), (32, 64), (33, 24), (33, 64), (63, 64)])
+def test_prolog_below_64_tokens_keeps_the_fixed_order_in_every_mode(t, n_heads, mode):
+    """Fewer than 64 tokens: every sum has its fixed order whatever the mode, so every output has the sequential statement's
+    bits -- at the edges of the forms (8 | 9, 32 | 33, 63), of a block of 16 or 32 rows, and with a head count (24) whose
+    w_proj rows are no power of two, which keeps the sums over the hidden axis in the decode form's launch."""
+    from pypto_amd import lightning_indexer_prolog_quant_impl as impl
+    impl.EXACT_SUMS = False
+    impl.MATRIX_CORE_HIDDEN_SUMS = mode == "matrix_cores"
+    try:
+        inp = gen_indexer_prolog_inputs(1, t, [t + 200], seed=100 + t, h=960, q_lora_rank=1536 if t % 2 else 512, n_heads=n_heads,
+                                        affine_ln=True)
+        got = run_op(inp)
+    finally:
+        impl.MATRIX_CORE_HIDDEN_SUMS = False
+    assert_exact(got, lo.indexer_prolog_ref(*inp.input_tensors()), f"t={t} n_heads={n_heads} {mode}")

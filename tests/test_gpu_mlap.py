@@ -270,6 +270,35 @@ def test_fused_prolog_query_rows_at_tile_edges(t, q_lora):
     assert (np.abs(q_scale.float().cpu().numpy()[..., 0] - want["q_scale"].astype(np.float32)) > 2.5e-5).mean() <= 0.005
 
 
+@pytest.mark.parametrize("t,n_idx,mode", [(8, 64, "default"), (9, 64, "default"), (16, 64, "default"), (31, 8, "default"),
+                                          (32, 64, "default"), (33, 64, "default"), (33, 24, "default"), (63, 64, "default"),
+                                          (9, 64, "exact"), (32, 64, "exact"), (63, 64, "exact"), (32, 64, "matrix_cores"),
+                                          (32, 64, "exact_absorb"), (33, 64, "exact_absorb"), (33, 24, "exact_absorb")])
+def test_fused_prolog_indexer_outputs_below_64_tokens_have_the_fixed_order_bits(t, n_idx, mode):
+    """The fused operator's indexer half below 64 tokens: from the query latent the MLA prolog makes (the standalone operator
+    gives the same one) every output has the sequential statement's bits in every mode of the sums."""
+    from oracle import lip_oracle as lo
+    from pypto_amd import lightning_indexer_prolog_quant_impl as lip_impl
+    from pypto_amd import mla_prolog_quant_impl as impl
+    from pypto_amd.synthetic import gen_indexer_prolog_inputs
+    impl.EXACT_ABSORB = mode == "exact_absorb"
+    lip_impl.EXACT_SUMS = mode == "exact"
+    lip_impl.MATRIX_CORE_HIDDEN_SUMS = mode == "matrix_cores"
+    kw = dict(h=960, q_lora_rank=512 if t % 2 else 1536)
+    mla = gen_mla_prolog_inputs(1, t, [t + 30], seed=t, n_heads=2, **kw)
+    lip = gen_indexer_prolog_inputs(1, t, [t + 30], seed=t + 1, n_heads=n_idx, **kw)
+    sep = run_op(mla, (1e-5, 1e-5))
+    dm, dl = mla.to(torch.device("cuda:0")), lip.to(torch.device("cuda:0"))
+    _, _, q_int8, q_scale, weights = run_fused(dm, dl, t, 2, n_idx)
+    lip.x, lip.cos_idx_rope, lip.sin_idx_rope, lip.k_cache_index = mla.token_x, mla.cos, mla.sin, mla.cache_index
+    lip.q_norm, lip.q_norm_scale = torch.from_numpy(sep["q_norm"]), torch.from_numpy(sep["q_norm_scale"]).reshape(-1, 1)
+    want = lo.indexer_prolog_ref(*lip.input_tensors())
+    for name, g in (("q_int8", q_int8), ("q_scale", q_scale[..., 0]), ("weights", weights), ("k_cache", dl.k_cache),
+                    ("k_cache_scale", dl.k_cache_scale)):
+        kind = np.uint8 if g.dtype == torch.int8 else np.uint16
+        assert np.array_equal(g.cpu().numpy().view(kind), want[name].view(kind)), name
+
+
 @pytest.mark.parametrize("mode,shape", [("default", "small"), ("exact", "small"), ("matrix_cores", "small"), ("default", "t_512"),
                                         ("default", "t_11_idx_64"), ("exact", "t_11_idx_64"), ("default", "t_3_idx_32"),
                                         ("default", "t_40_idx_64"), ("exact", "t_40_idx_64"), ("default", "t_7_idx_64"),
