@@ -92,6 +92,7 @@ struct SfaPlan {
     int hgroups;          // workgroups that share a row's heads
     int nsplit;
     int whole_slots;      // rows 0 .. 8 * whole_slots - 1 are not split
+    bool part_f32;        // partial results in fp32 instead of fp16
     size_t part_o_bytes;
     size_t part_ml_bytes;
     size_t predeq_bytes;  // the whole cache de-quantised once, behind the partial results (0: not worth it)
@@ -128,8 +129,8 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
     // (a size query on a host without a device plans for the 256 CUs of an MI355X; a launch there fails)
     const int cus = cu_count() > 0 ? cu_count() : 256;
     auto shares = [&](const int hg) { return (int)((a->nq + 32 * hg - 1) / (32 * hg)); };
-    auto partial_bytes = [&](const long long r, const int ns) {
-        return ns > 1 ? (size_t)r * ns * a->nq * (512 * sizeof(uint16_t) + 2 * sizeof(float)) : (size_t)0;
+    auto partial_bytes = [&](const long long r, const int ns, const bool f32 = false) {
+        return ns > 1 ? (size_t)r * ns * a->nq * (512 * (f32 ? sizeof(float) : sizeof(uint16_t)) + 2 * sizeof(float)) : (size_t)0;
     };
     // The schedule model, in microseconds: what a launch pair took over 1 to 128 rows x 16 to 128 heads x 1 to 64 splits
     // (fitted to within 10 %; neighbouring choices differ by less).  A compute unit holds one workgroup; a round of them
@@ -146,16 +147,42 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
     auto rounds = [&](const long long wgs) { return cus % 8 == 0 ? ((wgs + 7) / 8 + cus / 8 - 1) / (cus / 8) : (wgs + cus - 1) / cus; };
     const int hg_max = a->nq > 64 ? 4 : (a->nq > 32 ? 2 : 1);
     pl.head_groups = hg_max;
+    // A split row's partial results are fp16: one more rounding, to 11 bits, and a bf16 cache's values beyond 65504 become
+    // infinite, where a whole row goes from its fp32 accumulators straight to bf16.  So the launches whose partials are fp16 are a
+    // fixed set, and a launch outside of it that the model splits all the same leaves its partials in fp32.  The set: no
+    // split shorter than four tiles, rows dealt to the XCDs whole (row t on XCD t % 8), costs in tiles -- 3 per round around whole
+    // rows, 5.5 around split ones, the merge 1 and one per hundred partial rows.  (fp32 partials cost 0.25 us per MB they are
+    // larger by; only workgroups of one head group leave them.  16 heads, whole rows against fp32 partials: 50 rows of 256 keys
+    // 18.1 us and 14.7, 150 of 1024 58.7 and 52.3, 170 of 2048 109 and 88.6 -- as fp16 partials 12.8, 50.1 and 85.7.)
+    auto half_partials = [&]() {
+        const int sh = shares(hg_max), max_split = tiles / 4;
+        if (cus % 8 != 0) return max_split > 1 && rows * sh < cus;
+        const long long xcd_cus = cus / 8, xcd_rows = (rows + 7) / 8;
+        auto xcd_rounds = [&](const int s) { return (double)((xcd_rows * sh * s + xcd_cus - 1) / xcd_cus); };
+        const double whole = xcd_rounds(1) * (tiles + 3.0);
+        auto merge = [&](const long long r, const int s) { return 1.0 + 0.01 * (double)r * s * sh; };
+        for (int s = 2; s <= max_split && partial_bytes(rows, s) <= max_bytes; ++s)
+            if (xcd_rounds(s) * ((tiles + s - 1) / s + 5.5) + merge(rows, s) < whole) return true;
+        // full rounds of whole rows, and the rows left over in as many pieces as fill one more (below)
+        const long long per_round = xcd_cus / sh, full = per_round > 0 ? xcd_rows / per_round : 0;
+        const long long left = xcd_rows - full * per_round, rows_b = rows - 8 * full * per_round;
+        if (full < 1 || left < 1 || rows_b < 1) return false;
+        const int s = (int)(per_round / left < max_split ? per_round / left : max_split);
+        return s >= 2 && partial_bytes(rows_b, s) <= max_bytes &&
+               (double)full * (tiles + 3.0) + (tiles + s - 1) / s + 5.5 + merge(rows_b, s) < whole;
+    };
+    const bool f32 = a->num_splits == 0 && min_split == 1 && !half_partials();
     int ns = a->num_splits;
     double best = -1.0;
     if (ns == 0) {
         for (int hg = hg_max; hg >= 1; hg /= 2)
             // (of the split counts with equally long splits the smallest is the one to take)
-            for (int s = min_split, len = 0; s <= tiles; s = len > 1 ? (tiles + len - 2) / (len - 1) : tiles + 1) {
+            for (int s = min_split, len = 0; s <= (f32 ? (hg > 1 ? 1 : tiles < 8 ? tiles : 8) : tiles); s = len > 1 ? (tiles + len - 2) / (len - 1) : tiles + 1) {
                 len = (tiles + s - 1) / s;
                 const long long wgs = rows * shares(hg) * s;
-                if (s > min_split && (partial_bytes(rows, s) > max_bytes || wgs > 4ll * cus)) break;
-                const double cost = (double)rounds(wgs) * round_us(hg, s) + tail_us(hg, wgs, s);
+                if (s > min_split && (partial_bytes(rows, s, f32) > max_bytes || wgs > 4ll * cus)) break;
+                const double cost = (double)rounds(wgs) * round_us(hg, s) + tail_us(hg, wgs, s) +
+                                    (f32 ? 0.25e-6 * (double)(partial_bytes(rows, s, true) - partial_bytes(rows, s)) : 0.0);
                 if (best < 0.0 || cost < best) {
                     best = cost;
                     ns = s;
@@ -170,7 +197,7 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
     pl.nsplit = ns;
     pl.whole_slots = 0;
     long long split_rows = rows;
-    if (a->num_splits == 0 && min_split == 1 && cus % 8 == 0) {
+    if (a->num_splits == 0 && min_split == 1 && !f32 && cus % 8 == 0) {
         // More rows than compute units: the full rounds of whole rows first, then the rows left over dealt out in
         // as many pieces as fill one more round (300 rows on 256 CUs: 32 whole rows per XCD, the other five or
         // six in five pieces each), where that beats the best uniform split above.
@@ -195,9 +222,10 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
             }
         }
     }
+    pl.part_f32 = f32 && pl.nsplit > 1;
     if (pl.nsplit > 1) {
-        pl.part_o_bytes = (size_t)split_rows * pl.nsplit * a->nq * 512 * sizeof(uint16_t);
         pl.part_ml_bytes = (size_t)split_rows * pl.nsplit * a->nq * 2 * sizeof(float);
+        pl.part_o_bytes = partial_bytes(split_rows, pl.nsplit, f32) - pl.part_ml_bytes;
     } else {
         pl.part_o_bytes = pl.part_ml_bytes = 0;
     }
@@ -290,7 +318,7 @@ int sfa_enqueue(const PtoSfaQuantArgs *a, const int8_t *kn, int kn_pitch, const 
     p.bt = a->block_table;
     p.act = a->kv_act_seqs;
     p.out = static_cast<uint16_t *>(a->attention_out);
-    p.part_o = static_cast<uint16_t *>(a->workspace);
+    p.part_o = a->workspace;
     p.part_ml = pl.part_ml_bytes > 0 ? reinterpret_cast<float *>(static_cast<char *>(a->workspace) + pl.part_o_bytes) : nullptr;
     p.kv_rows = a->kv_rows;
     p.T = (int)(a->b * a->s1);
@@ -300,6 +328,7 @@ int sfa_enqueue(const PtoSfaQuantArgs *a, const int8_t *kn, int kn_pitch, const 
     p.bs = (int)a->block_size;
     p.maxblk = (int)a->max_blocknum_perbatch;
     p.nsplit = pl.nsplit;
+    p.part_f32 = pl.part_f32 ? 1 : 0;
     p.whole_slots = pl.whole_slots;
     p.hgroups = pl.hgroups;
     p.head_groups = pl.head_groups;

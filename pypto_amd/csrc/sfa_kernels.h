@@ -22,11 +22,12 @@ struct SfaParams {
     const int32_t *bt;        // [B, maxblk]
     const int32_t *act;       // [B]
     uint16_t *out;            // [T*NQ, 512] bf16
-    uint16_t *part_o;         // [split rows, nsplit, NQ, 512] fp16: O / l of each key split (nsplit > 1)
+    void *part_o;             // [split rows, nsplit, NQ, 512] fp16, or fp32 (part_f32): O / l of each key split (nsplit > 1)
     float *part_ml;           // [split rows, nsplit, NQ, 2]   reference max (log2 domain) and row sum of the split
     long long kv_rows;
     int T, S1, NQ, topk, bs, maxblk;
     int nsplit;               // key splits per query row, of the rows that are split
+    int part_f32;             // (with one head group per workgroup and at most eight splits)
     int whole_slots;          // rows 0 .. 8 * whole_slots - 1 are not split (one workgroup per row and head group): the
                               // full rounds of a launch of more rows than compute units; 0 = every row is split alike
     int hgroups;              // workgroups' shares of the heads per query row (32 * head_groups heads each)

@@ -1058,7 +1058,7 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
             // chunk gq: 128 channels of the wave's heads, or (PIPE) the wave's 128 channels of head group gq
             const int ch0 = PIPE ? 128 * w : part * (32 * DVP);
             uint16_t *dst0 = FINAL ? p.out + ((size_t)t * p.NQ + head_base + hsub) * DN + ch0 + 8 * j
-                                   : p.part_o + (prow_base + head_base + hsub) * DN + ch0 + 8 * j;
+                                   : static_cast<uint16_t *>(p.part_o) + (prow_base + head_base + hsub) * DN + ch0 + 8 * j;
 #pragma unroll
             for (int gq = 0; gq < DVP / 4; ++gq) {
 #pragma unroll
@@ -1104,8 +1104,38 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
                 }
             }
         };
+        // The partial as fp32: the wave's staging slice is 32 heads x 512 bytes, 16-byte chunk c (four channels) of head h at
+        // chunk c ^ h; half a wave writes 512 contiguous bytes of one head.
+        auto drain_f32 = [&]() {
+            static_assert(PIPE || NW * 32 * 512 <= WAVE_BYTES, "the slices fit the idle pool");
+            uint8_t *stage32 = reinterpret_cast<uint8_t *>(pool) + w * (32 * 512);
+            float *dst = static_cast<float *>(p.part_o) + (prow_base + head_base) * DN + part * (32 * DVP) + 4 * col;
+#pragma unroll
+            for (int gq = 0; gq < DVP / 4; ++gq) {
+#pragma unroll
+                for (int b4 = 0; b4 < 4; ++b4)
+#pragma unroll
+                    for (int q4 = 0; q4 < 4; ++q4) {
+                        const f32x16 &acc = o[4 * gq + b4];
+                        float r0, r1, r2, r3;
+                        asm volatile("v_accvgpr_read_b32 %0, %4\n\tv_accvgpr_read_b32 %1, %5\n\tv_accvgpr_read_b32 %2, %6\n\tv_accvgpr_read_b32 %3, %7"
+                                     : "=&v"(r0), "=&v"(r1), "=&v"(r2), "=&v"(r3)
+                                     : "a"(acc[4 * q4]), "a"(acc[4 * q4 + 1]), "a"(acc[4 * q4 + 2]), "a"(acc[4 * q4 + 3]));
+                        const f32x4 v = {r0 * inv[0], r1 * inv[0], r2 * inv[0], r3 * inv[0]};
+                        *reinterpret_cast<f32x4 *>(stage32 + col * 512 + 16 * ((8 * b4 + 2 * q4 + half) ^ col)) = v;
+                    }
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {            // (the wave reads back what it wrote itself, in order)
+                    const int hl = 2 * e + half;
+                    const f32x4 v = *reinterpret_cast<const f32x4 *>(stage32 + hl * 512 + 16 * (col ^ hl));
+                    if (head_base + hl < p.NQ) *reinterpret_cast<f32x4 *>(dst + (size_t)hl * DN + 128 * gq) = v;
+                }
+            }
+        };
         const bool all_heads = head_base + (PIPE ? 128 : 32) <= p.NQ;
-        if (nsplit == 1) {
+        if (HG == 1 && nsplit > 1 && p.part_f32) {
+            drain_f32();
+        } else if (nsplit == 1) {
             if (all_heads) drain(std::true_type{}, std::true_type{});
             else drain(std::true_type{}, std::false_type{});
         } else {
@@ -1120,7 +1150,7 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
 }
 
 // Merges the key splits of one query row: out = sum_s w_s O_s / sum_s w_s with w_s = l_s 2^(m_s - m)
-// and O_s the split's normalised fp16 partial (all zeros for an empty split, whose weight is zero).
+// and O_s the split's normalised partial, fp16 or fp32 (all zeros for an empty split, whose weight is zero).
 // One wave per (row, head), a lane per 8 value channels.  The (max, sum) pairs of a (row, head) are the
 // same for the whole wave and travel through the scalar cache; the NS 16-byte loads of a lane's partials
 // are all requested before the first of them is used.  The kernel moves bytes that were written
@@ -1128,7 +1158,7 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
 // smaller waves are faster than fewer waves with more loads each (2 or 4 (row, head) pairs per wave:
 // 8.2 and 10.2 us against 7.0 at 32 rows x 8 splits).  NS = 2, 4 or 8 splits are in flight at a time:
 // the smallest that covers the launch's splits.
-template <int NS>
+template <int NS, bool F32>
 __global__ __launch_bounds__(256) void sfa_combine_kernel(const SfaParams p)
 {
     const int lane = threadIdx.x & 63;
@@ -1139,13 +1169,15 @@ __global__ __launch_bounds__(256) void sfa_combine_kernel(const SfaParams p)
     const int ts = th / p.NQ, head = th - ts * p.NQ;
     const size_t prow0 = (size_t)ts * p.nsplit * p.NQ + head;      // split s: prow0 + s * NQ
     const f32x2 *ml = reinterpret_cast<const f32x2 *>(p.part_ml);
-    f16x8 hv[NS];
+    typedef typename std::conditional<F32, float, _Float16>::type P;
+    typedef __attribute__((ext_vector_type(8))) P P8;
+    P8 hv[NS];
     f32x2 v[NS];
 #pragma unroll
     for (int e = 0; e < NS; ++e) {
         const size_t prow = prow0 + (size_t)(e < p.nsplit ? e : p.nsplit - 1) * p.NQ;
         v[e] = ml[prow];
-        hv[e] = *reinterpret_cast<const f16x8 *>(p.part_o + prow * DN + 8 * lane);
+        hv[e] = *reinterpret_cast<const P8 *>(static_cast<const P *>(p.part_o) + prow * DN + 8 * lane);
     }
     float m = -INFINITY;
 #pragma unroll
@@ -1192,7 +1224,7 @@ __global__ __launch_bounds__(256) void sfa_combine_wide_kernel(const SfaParams p
         for (int e = 0; e < NS; ++e) {
             const size_t prow = prow0 + (size_t)(s0 + 4 * e < p.nsplit ? s0 + 4 * e : s0) * p.NQ;
             v[e] = ml[prow];
-            hv[e] = *reinterpret_cast<const f16x8 *>(p.part_o + prow * DN + 8 * lane);
+            hv[e] = *reinterpret_cast<const f16x8 *>(static_cast<const uint16_t *>(p.part_o) + prow * DN + 8 * lane);
         }
         float mn = m;
 #pragma unroll
@@ -1269,6 +1301,7 @@ hipError_t sfa_launch(const SfaParams &pa, hipStream_t stream)
     const int split_rows = p.T > 8 * p.whole_slots ? p.T - 8 * p.whole_slots : 0;
     p.xcd_pieces = (int)(((long long)split_rows * p.hgroups * p.nsplit + 7) / 8);
     const unsigned grid = (unsigned)(8 * (p.hgroups * p.whole_slots + p.xcd_pieces));
+    if (p.part_f32 && (p.head_groups > 1 || p.nsplit > 8)) return hipErrorInvalidValue;
 #define SFA_LAUNCH(Q)                                                                                                       \
     switch (p.head_groups) {                                                                                                \
     case 1: hipLaunchKernelGGL((sfa_decode_kernel<1, Q>), dim3(grid), dim3(256), 0, stream, p); break;                      \
@@ -1287,9 +1320,12 @@ hipError_t sfa_launch(const SfaParams &pa, hipStream_t stream)
         } else {
             // one wave per (row, head), four waves per workgroup
             const dim3 cgrid((unsigned)((n_th + 3) / 4));
-            if (p.nsplit <= 2) hipLaunchKernelGGL(sfa_combine_kernel<2>, cgrid, dim3(256), 0, stream, p);
-            else if (p.nsplit <= 4) hipLaunchKernelGGL(sfa_combine_kernel<4>, cgrid, dim3(256), 0, stream, p);
-            else hipLaunchKernelGGL(sfa_combine_kernel<8>, cgrid, dim3(256), 0, stream, p);
+#define SFA_COMBINE(F32)                                                                                                    \
+    if (p.nsplit <= 2) hipLaunchKernelGGL((sfa_combine_kernel<2, F32>), cgrid, dim3(256), 0, stream, p);                    \
+    else if (p.nsplit <= 4) hipLaunchKernelGGL((sfa_combine_kernel<4, F32>), cgrid, dim3(256), 0, stream, p);               \
+    else hipLaunchKernelGGL((sfa_combine_kernel<8, F32>), cgrid, dim3(256), 0, stream, p);
+            if (p.part_f32) { SFA_COMBINE(true) } else { SFA_COMBINE(false) }
+#undef SFA_COMBINE
         }
         e = hipGetLastError();
     }

@@ -163,3 +163,24 @@ def test_cache_out_overlapping_cache_in_is_refused():
     assert torch.equal(other, base[:32])
     with pytest.raises(ValueError, match="overlap"):
         copy_unless_same(base[8:40], base[:32], "k_int8")
+
+
+@pytest.mark.parametrize("nq,topk,rows", [
+    (128, 128, range(1, 20)), (128, 192, range(1, 20)), (128, 224, range(1, 20)), (64, 224, range(1, 40)), (16, 96, range(1, 80)),
+    (16, 128, range(1, 80)), (16, 224, range(1, 80)), (32, 256, range(25, 75)), (16, 256, range(281, 328)), (32, 320, range(75, 113)),
+    (64, 256, range(25, 40)), (128, 256, range(281, 284)), (16, 1024, range(129, 171)), (32, 768, range(129, 157)),
+    (16, 2048, range(169, 193)), (32, 1536, range(169, 193)), (64, 2048, range(169, 171)), (128, 2048, range(169, 171)),
+    (256, 2048, range(81, 86))])
+def test_attention_launches_without_half_precision_partials(nq, topk, rows):
+    """These launches (short selections at small batches, batches that just miss the next round of the chip) keep their rows
+    whole or leave the partial results of split rows in fp32, never in fp16."""
+    from pypto_amd import _C
+    for r in rows:
+        need = _C.sfa_quant_workspace_bytes(r, 1, nq, 1, topk, 128, 512, 1 << 30, 0.04, 0)
+        assert need in [0] + [r * s * nq * (512 * 4 + 8) for s in range(2, 9)], r
+
+
+@pytest.mark.parametrize("nq,topk,rows,splits", [(128, 2048, 1, 32), (128, 2048, 32, 8), (16, 256, 24, 4), (128, 256, 4, 8), (16, 2048, 168, 3)])
+def test_attention_launches_with_half_precision_partials(nq, topk, rows, splits):
+    from pypto_amd import _C
+    assert _C.sfa_quant_workspace_bytes(rows, 1, nq, 1, topk, 128, 512, 1 << 30, 0.04, 0) == rows * splits * nq * (512 * 2 + 8)

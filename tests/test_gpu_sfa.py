@@ -237,6 +237,57 @@ def test_bf16_latent_cache_branch(n_q, b, s1, act, topk):
     assert torch.equal(out.view(torch.int16), run_op(inp).view(torch.int16))
 
 
+@pytest.mark.parametrize("n_q,b,topk", [(128, 1, 128), (64, 5, 224), (16, 30, 256)])
+def test_bf16_latent_cache_beyond_the_range_of_fp16(n_q, b, topk):
+    """Launches outside of the set whose partial results are fp16 (short selections at small batches): latent values that fp16
+    does not hold come through.  The values are powers of two, so a weighted mean of them is within a few bf16 steps (2^-8
+    each) of one rounding of P and of the result."""
+    inp = gen_sfa_inputs(b, 1, n_q, [700] * b, topk=topk, seed=5)
+    dev = torch.device("cuda:0")
+    d = inp.to(dev)
+    kn = torch.full((inp.key_nope_2d.shape[0], 512), 2.0 ** 18, dtype=torch.bfloat16, device=dev)
+    kn[:, 1::2] = -2.0 ** 100
+    out = torch.zeros([b, 1, n_q, 512], dtype=torch.bfloat16, device=dev)
+    pypto_amd.sparse_flash_attention_quant_d(torch.zeros_like(d.query_nope), d.query_rope, kn, d.key_rope_2d, None, d.topk_indices,
+                                             d.block_table, d.kv_act_seqs, out, n_q, 1, inp.softmax_scale, topk, inp.block_size,
+                                             inp.max_blocknum_perbatch, None)
+    torch.cuda.synchronize()
+    o = out.double().cpu()
+    assert torch.isfinite(o).all()
+    assert ((o[..., 0::2] / 2.0 ** 18 - 1).abs().max() <= 3 * 2.0 ** -8) and ((o[..., 1::2] / -2.0 ** 100 - 1).abs().max() <= 3 * 2.0 ** -8)
+
+
+@pytest.mark.parametrize("n_q,b,s1,act,topk", [
+    (128, 1, 1, [3000], 128),                   # four head groups, splits of a tile or two
+    (128, 2, 1, [3000, 70], 97),                # a split with no keys
+    (20, 3, 2, [700, 90, 300], 128),            # part of a head group
+    (70, 1, 1, [33], 97),                       # a last group of six heads
+    (16, 40, 1, [300 + 11 * i for i in range(40)], 256),
+    (16, 33, 4, [600 + 11 * i for i in range(33)], 1024),
+])
+def test_single_precision_partials(n_q, b, s1, act, topk):
+    """Split launches outside of the set whose partials are fp16: both cache formats against the golden and the int8 cache's
+    result against that of whole rows (a rounding of P and of the result apart)."""
+    from oracle import sfa_oracle as so
+    inp = gen_sfa_inputs(b, s1, n_q, act, topk=topk, seed=61 + n_q)
+    from pypto_amd import _C
+    need = _C.sfa_quant_workspace_bytes(b, s1, n_q, 1, topk, inp.block_size, inp.max_blocknum_perbatch, 1 << 30, inp.softmax_scale, 0)
+    assert need in [b * s1 * s * n_q * (512 * 4 + 8) for s in range(2, 9)]
+    out = run_op(inp)
+    check(out, oracle(inp), f"fp32 partials nq={n_q} rows={b * s1} topk={topk}")
+    whole = run_op(inp, num_splits=1).float()
+    assert (out.float() - whole).abs().max() <= 3 * 2.0 ** -8 * whole.abs().max()
+    dev = torch.device("cuda:0")
+    d = inp.to(dev)
+    kn = so.dequant_kn(inp.key_nope_2d, inp.k_nope_scales).to(dev)
+    o2 = torch.full([b, s1, n_q, 512], float("nan"), dtype=torch.bfloat16, device=dev)
+    pypto_amd.sparse_flash_attention_quant_d(d.query_nope, d.query_rope, kn, d.key_rope_2d, None, d.topk_indices, d.block_table,
+                                             d.kv_act_seqs, o2, n_q, 1, inp.softmax_scale, topk, inp.block_size,
+                                             inp.max_blocknum_perbatch, None)
+    torch.cuda.synchronize()
+    check(o2.cpu(), oracle(inp), f"fp32 partials over a bf16 cache nq={n_q}")
+
+
 @pytest.mark.parametrize("scale", [-0.0416666679084301, 0.0, 0.25])
 def test_softmax_scale_of_any_sign(scale):
     """The kernel scales scores inside the exponent and wants a positive factor: a negative one moves its
