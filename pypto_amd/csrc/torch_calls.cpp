@@ -76,8 +76,10 @@ struct Call {
         ok = ok && t.scalar_type() == type && t.sizes() == c10::IntArrayRef(sizes.begin(), sizes.size());
         return t;
     }
-    // the address of a tensor that was checked
+    // the address of a tensor that was checked: ptr for what the kernels read, out for what they write (a tensor that shares
+    // its memory copy-on-write gets memory of its own here)
     template <typename T> T *ptr(const at::Tensor &t) { return ok ? static_cast<T *>(const_cast<void *>(t.const_data_ptr())) : nullptr; }
+    template <typename T> T *out(const at::Tensor &t) { return ok ? static_cast<T *>(t.mutable_data_ptr()) : nullptr; }
 
     int64_t integer(const int i)
     {
@@ -168,7 +170,7 @@ PyObject *sfa_call(PyObject *, PyObject *const *args, Py_ssize_t n)
         if (!c.ok) return declined();
         a.query_nope = c.ptr<void>(qn), a.query_rope = c.ptr<void>(qr), a.key_nope_2d = c.ptr<void>(kn), a.key_rope_2d = c.ptr<void>(kr);
         a.topk_indices = c.ptr<int32_t>(ti), a.block_table = c.ptr<int32_t>(bt), a.kv_act_seqs = c.ptr<int32_t>(act);
-        a.attention_out = c.ptr<void>(out);
+        a.attention_out = c.out<void>(out);
         return enqueue(c.device, a, pto_sfa_quant_workspace_bytes, quant ? pto_sfa_quant_launch : pto_sfa_bf16kv_launch);
     });
 }
@@ -195,7 +197,7 @@ PyObject *sa_antiquant_call(PyObject *, PyObject *const *args, Py_ssize_t n)
         if (!c.ok) return declined();
         a.query_nope = c.ptr<void>(qn), a.query_rope = c.ptr<void>(qr), a.nope_cache = c.ptr<void>(nc);
         a.topk_indices = c.ptr<int32_t>(ti), a.block_table = c.ptr<int32_t>(bt), a.kv_act_seqs = c.ptr<int32_t>(act);
-        a.attention_out = c.ptr<void>(out);
+        a.attention_out = c.out<void>(out);
         return enqueue(c.device, a, pto_sa_antiquant_workspace_bytes, pto_sa_antiquant_launch);
     });
 }
@@ -232,7 +234,7 @@ PyObject *li_decode_call(PyObject *, PyObject *const *args, Py_ssize_t n)
         a.q_scale_dtype = dtype_code(qs, c.ok), a.k_scale_dtype = dtype_code(ks, c.ok), a.weight_dtype = dtype_code(w, c.ok);
         if (!c.ok || (a.arith_variant != 0 && (qs.scalar_type() != FP16 || ks.scalar_type() != FP16 || w.scalar_type() != FP16))) return declined();
         a.idx_query = c.ptr<int8_t>(q), a.idx_query_scale = c.ptr<void>(qs), a.idx_key_cache = c.ptr<int8_t>(kc), a.idx_key_scale = c.ptr<void>(ks);
-        a.idx_weight = c.ptr<void>(w), a.act_seq_key = c.ptr<int32_t>(act), a.block_table = c.ptr<int32_t>(bt), a.topk_res = c.ptr<int32_t>(res);
+        a.idx_weight = c.ptr<void>(w), a.act_seq_key = c.ptr<int32_t>(act), a.block_table = c.ptr<int32_t>(bt), a.topk_res = c.out<int32_t>(res);
         return enqueue(c.device, a, pto_li_decode_workspace_bytes, pto_li_decode_launch);
     });
 }
@@ -241,7 +243,7 @@ PyObject *li_decode_call(PyObject *, PyObject *const *args, Py_ssize_t n)
 // out) and have to be the same memory.
 bool same_memory(Call &c, const at::Tensor &in, const at::Tensor &out)
 {
-    return c.ok && in.scalar_type() == out.scalar_type() && in.numel() == out.numel() && in.const_data_ptr() == out.const_data_ptr();
+    return c.ok && in.scalar_type() == out.scalar_type() && in.numel() == out.numel() && c.out<void>(out) == in.const_data_ptr();
 }
 
 // at: token_x, w_dq, w_uq_qr, dequant_scale, w_uk, w_dkv_kr, gamma_cq, gamma_ckv, cos, sin, cache_index, kv_cache,
@@ -258,7 +260,7 @@ bool mla_args(Call &c, const int (&at)[21], PtoMlaPrologQuantArgs &a)
         return false;
     if (!same_memory(c, c.tensor(at[11]), kvc) || !same_memory(c, c.tensor(at[12]), krc) || !same_memory(c, c.tensor(at[13]), ksc)) return false;
     a.token_x = c.ptr<void>(x), a.w_dq = c.ptr<void>(wdq), a.w_uk = c.ptr<void>(wuk);
-    a.kv_cache = c.ptr<int8_t>(kvc), a.kr_cache = c.ptr<void>(krc), a.k_scale_cache = c.ptr<float>(ksc);
+    a.kv_cache = c.out<int8_t>(kvc), a.kr_cache = c.out<void>(krc), a.k_scale_cache = c.out<float>(ksc);
     a.w_uq_qr = c.ptr<int8_t>(c.shaped(at[2], I8, {a.q_lora_rank, a.n_heads * 192}));
     a.dequant_scale = c.ptr<float>(c.of(at[3], FP32, a.n_heads * 192));
     a.w_dkv_kr = c.ptr<void>(c.shaped(at[5], BF16, {a.h, 576}));
@@ -268,11 +270,11 @@ bool mla_args(Call &c, const int (&at)[21], PtoMlaPrologQuantArgs &a)
     a.sin = c.ptr<void>(c.of(at[9], BF16, a.t * 64));
     a.cache_index = c.ptr<int64_t>(c.of(at[10], I64, a.t));
     if (at[14] >= 0) {
-        a.q_norm_out = c.ptr<int8_t>(c.of(at[14], I8, a.t * a.q_lora_rank));
-        a.q_norm_scale_out = c.ptr<float>(c.of(at[15], FP32, a.t));
+        a.q_norm_out = c.out<int8_t>(c.of(at[14], I8, a.t * a.q_lora_rank));
+        a.q_norm_scale_out = c.out<float>(c.of(at[15], FP32, a.t));
     }
-    a.query_nope_out = c.ptr<void>(c.of(at[16], BF16, a.t * a.n_heads * 512));
-    a.query_rope_out = c.ptr<void>(c.of(at[17], BF16, a.t * a.n_heads * 64));
+    a.query_nope_out = c.out<void>(c.of(at[16], BF16, a.t * a.n_heads * 512));
+    a.query_rope_out = c.out<void>(c.of(at[17], BF16, a.t * a.n_heads * 64));
     return c.ok;
 }
 
@@ -289,7 +291,7 @@ bool li_prolog_args(Call &c, const int (&at)[21], PtoLiPrologQuantArgs &a)
         return false;
     const at::Tensor &kc_in = c.of(at[13], I8);
     if (!same_memory(c, kc_in, kc) || kc_in.sizes() != kc.sizes() || !same_memory(c, c.tensor(at[14]), ks)) return false;
-    a.x = c.ptr<void>(x), a.w_qb = c.ptr<int8_t>(wqb), a.w_proj = c.ptr<void>(wp), a.k_cache = c.ptr<int8_t>(kc), a.k_cache_scale = c.ptr<void>(ks);
+    a.x = c.ptr<void>(x), a.w_qb = c.ptr<int8_t>(wqb), a.w_proj = c.ptr<void>(wp), a.k_cache = c.out<int8_t>(kc), a.k_cache_scale = c.out<void>(ks);
     if (at[1] >= 0) {
         a.q_norm = c.ptr<int8_t>(c.shaped(at[1], I8, {a.t, a.q_lora_rank}));
         a.q_norm_scale = c.ptr<float>(c.of(at[2], FP32, a.t));
@@ -303,9 +305,9 @@ bool li_prolog_args(Call &c, const int (&at)[21], PtoLiPrologQuantArgs &a)
     a.hadamard_q = c.ptr<void>(c.shaped(at[11], BF16, {128, 128}));
     a.hadamard_k = c.ptr<void>(c.shaped(at[12], BF16, {128, 128}));
     a.k_cache_index = c.ptr<int64_t>(c.of(at[15], I64, a.t));
-    a.q_int8 = c.ptr<int8_t>(c.of(at[16], I8, a.t * a.n_heads * 128));
-    a.q_scale = c.ptr<void>(c.of(at[17], FP16, a.t * a.n_heads));
-    a.weights = c.ptr<void>(c.of(at[20], FP16, a.t * a.n_heads));
+    a.q_int8 = c.out<int8_t>(c.of(at[16], I8, a.t * a.n_heads * 128));
+    a.q_scale = c.out<void>(c.of(at[17], FP16, a.t * a.n_heads));
+    a.weights = c.out<void>(c.of(at[20], FP16, a.t * a.n_heads));
     return c.ok;
 }
 
