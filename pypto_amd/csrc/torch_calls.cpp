@@ -106,6 +106,9 @@ struct Call {
 
 bool dims(const at::Tensor &t, const int64_t n) { return t.defined() && t.dim() == n; }
 
+// a count given as an argument: beyond this the library takes none of them, and the products below stay far from 64 bits
+bool count_ok(const int64_t v) { return v >= 1 && v <= (1ll << 24); }
+
 PyObject *declined() { Py_RETURN_FALSE; }
 
 PyObject *raise_status(const int rc)
@@ -157,7 +160,7 @@ PyObject *sfa_call(PyObject *, PyObject *const *args, Py_ssize_t n)
         const int64_t maxblk = c.integer(14);
         a.softmax_scale = static_cast<float>(c.real(11));
         const at::Tensor &qn = c.of(0, BF16), &kn = c.tensor(2), &bt = c.of(6, I32), &act = c.of(7, I32);
-        if (!c.ok || !dims(qn, 2) || !dims(kn, 2) || !dims(bt, 2) || !dims(act, 1) || a.nq < 1 || a.n_kv < 1) return declined();
+        if (!c.ok || !dims(qn, 2) || !dims(kn, 2) || !dims(bt, 2) || !dims(act, 1) || !count_ok(a.nq) || !count_ok(a.n_kv) || !count_ok(a.topk)) return declined();
         const bool quant = kn.scalar_type() == I8;
         a.b = act.size(0), a.kv_rows = kn.size(0);
         if (a.b < 1 || qn.size(1) != 512 || kn.size(1) != 512 || (!quant && kn.scalar_type() != BF16) || qn.size(0) % (a.b * a.nq) != 0 ||
@@ -187,7 +190,7 @@ PyObject *sa_antiquant_call(PyObject *, PyObject *const *args, Py_ssize_t n)
         const int64_t maxblk = c.integer(12);
         a.softmax_scale = static_cast<float>(c.real(9));
         const at::Tensor &qn = c.of(0, BF16), &nc = c.of(2, I8), &bt = c.of(4, I32), &act = c.of(5, I32);
-        if (!c.ok || !dims(qn, 2) || !dims(nc, 2) || !dims(bt, 2) || !dims(act, 1) || a.nq < 1 || a.n_kv < 1) return declined();
+        if (!c.ok || !dims(qn, 2) || !dims(nc, 2) || !dims(bt, 2) || !dims(act, 1) || !count_ok(a.nq) || !count_ok(a.n_kv) || !count_ok(a.topk)) return declined();
         a.b = act.size(0), a.kv_rows = nc.size(0);
         if (a.b < 1 || qn.size(1) != 512 || nc.size(1) != 656 || qn.size(0) % (a.b * a.nq) != 0 || bt.size(0) != a.b || bt.size(1) < maxblk)
             return declined();
@@ -227,7 +230,7 @@ PyObject *li_decode_call(PyObject *, PyObject *const *args, Py_ssize_t n)
         a.t = q.size(0), a.n_heads = q.size(1), a.head_dim = q.size(2), a.b = act.size(0);
         a.block_num = kc.size(0), a.block_size = kc.size(1), a.max_blocknum_perbatch = bt.size(1);
         if (a.b < 1 || kc.size(2) != 1 || kc.size(3) != a.head_dim || a.t % a.b != 0 || a.t / a.b > max_s1 || bt.size(0) != a.b ||
-            a.max_blocknum_perbatch * a.block_size > max_s2 || a.selected_count < 1)
+            a.max_blocknum_perbatch * a.block_size > max_s2 || !count_ok(a.selected_count))
             return declined();
         const at::Tensor &qs = c.tensor(1), &ks = c.tensor(3), &w = c.tensor(4), &res = c.of(7, I32, a.t * a.selected_count);
         if (!c.ok || qs.numel() != a.t * a.n_heads || w.numel() != a.t * a.n_heads || ks.numel() != a.block_num * a.block_size) return declined();

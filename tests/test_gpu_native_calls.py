@@ -110,3 +110,86 @@ def test_cache_out_that_is_a_lazy_clone_of_cache_in_is_another_cache(which):
         assert torch.equal(t.view(torch.uint8), b.view(torch.uint8))
     for i, w in zip(written, want):
         assert torch.equal(args[i].clone().view(torch.uint8), w.view(torch.uint8)), i
+
+
+def outcome(op, args):
+    try:
+        op(*args)
+    except Exception as e:                                           # noqa: BLE001 (whatever it raises is what is compared)
+        return type(e), str(e)
+    torch.cuda.synchronize()
+    return None
+
+
+NATIVE = ("sfa_call", "sa_antiquant_call", "li_decode_call", "mla_prolog_call", "li_prolog_call", "fused_prolog_call")
+
+
+@pytest.fixture
+def python_path():
+    """A call with the native path switched off."""
+    from pypto_amd import _native
+    C = _native.load()
+
+    def run(op, args):
+        with pytest.MonkeyPatch.context() as m:
+            for name in NATIVE:
+                m.setattr(C, name, lambda *a: False)
+            return outcome(op, args)
+    return run
+
+
+def other_type(t):
+    return t.to(torch.int64 if t.dtype != torch.int64 and not t.dtype.is_floating_point else torch.float64)
+
+
+def strided(t):
+    wide = torch.zeros([*t.shape, 2], dtype=t.dtype, device=t.device)
+    return wide[..., 0]
+
+
+MALFORMED = {"type": other_type, "host": lambda t: t.cpu(), "strided": strided, "short": lambda t: t[:-1].clone(),
+             "dimension": lambda t: t.unsqueeze(0), "none": lambda t: None, "list": lambda t: [1, 2]}
+
+
+@pytest.mark.parametrize("how", MALFORMED)
+@pytest.mark.parametrize("which", CALLS)
+def test_malformed_tensors_end_the_same_way_on_both_paths(which, how, python_path):
+    """Every tensor argument in turn, of the wrong type, device, stride or shape: refused with the same error by either path,
+    or (where only the number of elements counts) taken by both."""
+    op, args, _ = CALLS[which]()
+    refused = 0
+    for i, a in enumerate(args):
+        if not torch.is_tensor(a) or (how == "short" and which == "packed_attention_call" and i == 2):
+            continue                                                 # (a packed cache of one row fewer is another valid cache)
+        bad = list(args)
+        bad[i] = MALFORMED[how](a)
+        want = python_path(op, bad)
+        assert outcome(op, bad) == want, i
+        refused += want is not None
+    assert refused > 0
+
+
+BIG = 1 << 62
+MALFORMED_NUMBERS = {
+    "attention_call": [(9, v) for v in (0, -1, 7, BIG, 1 << 64, "x", None)] + [(10, v) for v in (0, 2, BIG)] +
+                      [(12, v) for v in (0, -1, 63, BIG, BIG + 16)] + [(13, v) for v in (0, -1, 1 << 40, BIG)] +
+                      [(14, v) for v in (1 << 20, BIG)] + [(11, v) for v in (float("nan"), float("inf"), 1e300, "x", None)],
+    "packed_attention_call": [(7, v) for v in (0, -1, 7, BIG, 1 << 64)] + [(8, v) for v in (0, 2, BIG)] +
+                             [(10, v) for v in (0, 63, BIG)] + [(11, v) for v in (0, 1 << 40)] + [(12, BIG), (9, float("nan"))],
+    "indexer_call": [(10, v) for v in (0, -1, 63, 4096, BIG, BIG + 64, "x", None)],
+    "mla_prolog_call": [(21, v) for v in (float("nan"), -1.0, "x", None)] + [(22, float("inf")), (23, "BSND")],
+    "fused_prolog_call": [(34, v) for v in (float("nan"), -1.0, "x", None)] + [(35, float("inf")), (36, "BSND")],
+}
+
+
+@pytest.mark.parametrize("which", MALFORMED_NUMBERS)
+def test_malformed_numbers_end_the_same_way_on_both_paths(which, python_path):
+    """Counts that are zero, negative, no divisor, or large enough that products of them would wrap; scalars that are not finite
+    or no numbers."""
+    op, args, _ = CALLS[which]()
+    for i, v in MALFORMED_NUMBERS[which]:
+        bad = list(args)
+        bad[i] = v
+        want = python_path(op, bad)
+        assert want is not None, (i, v)
+        assert outcome(op, bad) == want, (i, v)
