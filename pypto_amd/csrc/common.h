@@ -19,6 +19,10 @@ typedef __attribute__((ext_vector_type(4))) short s16x4;
 typedef __attribute__((ext_vector_type(8))) short s16x8;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+// the same for tensors of 16-bit elements that promise no more than their elements' alignment: one memory instruction
+// all the same, since gfx950 code runs in unaligned-access mode
+typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
 
 // two fp32 -> packed bf16 pair, round-to-nearest-even (v_cvt_pk_bf16_f32)
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi)

@@ -108,8 +108,8 @@ __device__ __forceinline__ void pfa_rotate_rows(const MlapParams &p, const uint8
 {
     const size_t tt = t < p.T ? t : p.T - 1;
     const u32x4 x = *reinterpret_cast<const u32x4 *>(rows + row * PFA_RPITCH + 16 * e);
-    const u32x2 c0 = *reinterpret_cast<const u32x2 *>(p.cos + tt * MLAP_ROPE + 4 * e), c1 = *reinterpret_cast<const u32x2 *>(p.cos + tt * MLAP_ROPE + 32 + 4 * e);
-    const u32x2 s0 = *reinterpret_cast<const u32x2 *>(p.sin + tt * MLAP_ROPE + 4 * e), s1 = *reinterpret_cast<const u32x2 *>(p.sin + tt * MLAP_ROPE + 32 + 4 * e);
+    const u32x2 c0 = *reinterpret_cast<const u32x2_a2 *>(p.cos + tt * MLAP_ROPE + 4 * e), c1 = *reinterpret_cast<const u32x2_a2 *>(p.cos + tt * MLAP_ROPE + 32 + 4 * e);
+    const u32x2 s0 = *reinterpret_cast<const u32x2_a2 *>(p.sin + tt * MLAP_ROPE + 4 * e), s1 = *reinterpret_cast<const u32x2_a2 *>(p.sin + tt * MLAP_ROPE + 32 + 4 * e);
     float r0[4], r1[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -120,8 +120,8 @@ __device__ __forceinline__ void pfa_rotate_rows(const MlapParams &p, const uint8
     }
     if (t < p.T) {
         uint16_t *out = p.q_rope + (tt * p.n_heads + head) * MLAP_ROPE + 4 * e;
-        *reinterpret_cast<u32x2 *>(out) = u32x2{pack_bf16x2(r0[0], r0[1]), pack_bf16x2(r0[2], r0[3])};
-        *reinterpret_cast<u32x2 *>(out + 32) = u32x2{pack_bf16x2(r1[0], r1[1]), pack_bf16x2(r1[2], r1[3])};
+        *reinterpret_cast<u32x2_a2 *>(out) = u32x2{pack_bf16x2(r0[0], r0[1]), pack_bf16x2(r0[2], r0[3])};
+        *reinterpret_cast<u32x2_a2 *>(out + 32) = u32x2{pack_bf16x2(r1[0], r1[1]), pack_bf16x2(r1[2], r1[3])};
     }
 }
 
@@ -286,7 +286,7 @@ __device__ __forceinline__ void mlap_prefill_body(const MlapParams &p, const int
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int t = tb0 + 8 * (r >> 2) + 4 * half + (r & 3);
-            if (t < p.T) *reinterpret_cast<u32x2 *>(dst + (size_t)t * p.n_heads * MLAP_KV) = u32x2{pack_bf16x2(c[0][r], c[1][r]), pack_bf16x2(c[2][r], c[3][r])};
+            if (t < p.T) *reinterpret_cast<u32x2_a2 *>(dst + (size_t)t * p.n_heads * MLAP_KV) = u32x2{pack_bf16x2(c[0][r], c[1][r]), pack_bf16x2(c[2][r], c[3][r])};
         }
     }
 }

@@ -208,7 +208,7 @@ __device__ __forceinline__ void mlap_small_body(const MlapParams &p, const int h
         const int t = 4 * k + (l >> 4);
         if (4 * k >= p.T) break;
         const u32x4 v = *reinterpret_cast<const u32x4 *>(stg + t * PSA_SPITCH + 16 * (l & 15));
-        if (t < p.T) *reinterpret_cast<u32x4 *>(p.q_nope + ((size_t)t * p.n_heads + head) * MLAP_KV + 128 * w + 8 * (l & 15)) = v;
+        if (t < p.T) *reinterpret_cast<u32x4_a2 *>(p.q_nope + ((size_t)t * p.n_heads + head) * MLAP_KV + 128 * w + 8 * (l & 15)) = v;
     }
     pfa_rotate_rows(p, lds, 8 * w + (l >> 3), 8 * w + (l >> 3), head, l & 7);
 }

@@ -198,6 +198,34 @@ def test_mla_prolog_feeds_the_attention_cache_layout():
         assert np.abs(deq.reshape(512)).max() > 0
 
 
+@pytest.mark.parametrize("t", [3, 20, 40, 70, 300])
+@pytest.mark.parametrize("exact", [False, True])
+def test_mla_prolog_query_outputs_and_rope_tables_at_odd_addresses(t, exact):
+    """query_nope_out, query_rope_out, cos and sin promise no more than a bf16 element's alignment: views that start one element
+    into their storage give the same bits in every form of the last launch."""
+    from pypto_amd import mla_prolog_quant_impl as impl
+    impl.EXACT_ABSORB = exact
+    inp = gen_mla_prolog_inputs(1, t, [t + 30], seed=t, h=128, q_lora_rank=512, n_heads=4)
+    want = run_op(inp, (1e-5, 1e-5))
+
+    def odd(v):
+        flat = torch.zeros(v.numel() + 1, dtype=v.dtype, device="cuda")
+        view = flat[1:].view(v.shape)
+        view.copy_(v)
+        assert view.data_ptr() % 4 == 2 and view.is_contiguous()
+        return view
+    d = inp.to(torch.device("cuda:0"))
+    args = list(d.input_tensors())
+    args[8], args[9] = odd(d.cos), odd(d.sin)
+    q_norm = torch.zeros([t, 512], dtype=torch.int8, device="cuda")
+    q_norm_scale = torch.zeros([t, 1], dtype=torch.float32, device="cuda")
+    q_nope, q_rope = odd(torch.zeros([t, 4, 512], dtype=torch.bfloat16)), odd(torch.zeros([t, 4, 64], dtype=torch.bfloat16))
+    pypto_amd.mla_prolog_quant_d(*args, q_norm, q_norm_scale, q_nope, q_rope, d.kv_cache, d.kr_cache, d.k_scale_cache, 1e-5, 1e-5)
+    torch.cuda.synchronize()
+    assert np.array_equal(q_nope.float().cpu().numpy(), want["query_nope"]) and np.array_equal(q_rope.float().cpu().numpy(), want["query_rope"])
+    assert np.array_equal(d.kr_cache.float().cpu().numpy(), want["kr_cache"])
+
+
 def run_fused(dm, dl, t, n, n_idx, op=None):
     """The fused operator on device inputs dm (MLA prolog) and dl (indexer prolog); caches updated in place."""
     dev = dm.token_x.device
