@@ -417,8 +417,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
     // trip but the wave's last writes both -- and that many may be outstanding: a wait that counts the requests alone
     // holds a wave up until half of the pair it has only just asked for has landed too.  The trip's operands and scale
     // then move to registers, which frees the buffer for the pair two ahead, and the pair is scored.
+    // (The wait itself orders nothing for the compiler: without the barrier in front of it a store of an earlier trip may move
+    // behind it, and the wait would then pass with the trip's own requests still on their way.)
     auto wait_pair = [&](auto per_trip, const int pr) {
         constexpr int ST = decltype(per_trip)::value;
+        asm volatile("" ::: "memory");
         if (pr + 1 < npair) {
             if (pr >= 2) __builtin_amdgcn_s_waitcnt(vmcnt_imm(9 + 2 * ST));
             else if (pr == 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(9 + ST));
