@@ -84,30 +84,23 @@ __host__ __device__ inline bool mlap_prefill_forms(const MlapParams &p) { return
 // PROLOG_SMALL_TOKENS tokens, prolog_prefill.h beyond)
 constexpr int PROLOG_SMALL_TOKENS = 32;
 __host__ __device__ inline bool mlap_fused_projection(const MlapParams &p) { return !p.absorb_exact; }
-// partial sums per output the int8 projection leaves: 1 = unsplit (de-quantised bf16), else QPROJ_KSPLIT_HOST int32 partials
-__host__ __device__ inline int mlap_qsplits(const MlapParams &p)
-{
-    return (mlap_prefill_forms(p) || p.T >= MLAP_UNSPLIT_MIN_TOKENS) ? 1 : QPROJ_KSPLIT_HOST;
-}
+// partial sums per output the int8 projection leaves where it is a launch of its own (absorb_exact): 1 = unsplit (de-quantised
+// bf16), else QPROJ_KSPLIT_HOST int32 partials
+__host__ __device__ inline int mlap_qsplits(const MlapParams &p) { return p.T >= MLAP_UNSPLIT_MIN_TOKENS ? 1 : QPROJ_KSPLIT_HOST; }
 // whether the launches of `p` take a rider at all: the decode forms only
-inline bool mlap_takes_rider(const MlapParams &p) { return !mlap_prefill_forms(p) && mlap_qsplits(p) != 1; }
+inline bool mlap_takes_rider(const MlapParams &p) { return !mlap_prefill_forms(p) && p.T < MLAP_UNSPLIT_MIN_TOKENS; }
 
 hipError_t mlap_launch(const MlapParams &p, hipStream_t stream);
-// all launches but the last (which from PROLOG_PF_MIN_TOKENS tokens on holds the projection too), and the number of
-// workgroups of the last (for the fused operator's last launch)
+// all launches but the last (which unless absorb_exact holds the projection too), and the number of workgroups of the last with
+// absorb_exact (for the fused operator's last launch)
 // lip_rider (prefill forms only): the indexer prolog whose fixed-order sums over the hidden axis (left as group sums:
-// LipParams::x_in_groups) ride in this operator's first launch or, below PROLOG_PF_MIN_TOKENS tokens and then with its
-// split int8 projection, in the third
+// LipParams::x_in_groups) ride in this operator's first launch
 struct LipParams;
 hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const MlapRider *rider = nullptr, const LipParams *lip_rider = nullptr);
 int mlap_finish_wgs(const MlapParams &p);
-// the last launch alone; at prefill sizes (mlap_finish_is_prefill) it has a form of its own that the fused operator
-// launches beside, not inside, its own last launch
+// the last launch alone
 hipError_t mlap_launch_finish(const MlapParams &p, hipStream_t stream);
-// projections and last stages of both prologs at prefill sizes, either of which may be absent (prolog_fused.hip)
+// projections and last stages of both prologs, either of which may be absent (prolog_fused.hip)
 hipError_t prolog_prefill_launch(const MlapParams *pm, const LipParams *pl, hipStream_t stream);
-bool mlap_finish_is_prefill(const MlapParams &p);
-// blocks of 32 tokens per workgroup and workgroups of that form's launch
-void mlap_finish_prefill_shape(const MlapParams &p, int &per, int &wgs);
 
 }  // namespace pto

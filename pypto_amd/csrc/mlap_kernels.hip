@@ -459,46 +459,12 @@ __global__ __launch_bounds__(128) void qproj_kernel(const QProj pa, const int nj
     }
 }
 
-// TB: token blocks per tile (prolog_common.h).  HS > 0: the fused prolog's riders.  The first fixed_wgs workgroups (a
-// multiple of eight) run the indexer prolog's fixed-order sums over the hidden axis, which nothing before the last launch
-// needs: in the first launch they would share compute units, and the matrix cores, with the workgroups every later
-// stage waits for (32 tokens: 16.3 us there against 12.7).  Workgroups past the launch's own run the indexer prolog's
-// split int8 projection (one job of a wave pair each, HS steps of 32 rows per half; the other two waves only keep the
-// barrier company), beside the tiles' workgroups (two workgroups fit a compute unit).
-template <int TB, int HS>
-__global__ __launch_bounds__(256) void qproj_prefill_kernel(const QProj p, const int njobs, const QProj rider, const LipParams lip,
-                                                            const int fixed_groups, const int fixed_wgs)
+// TB: token blocks per tile (prolog_common.h).
+template <int TB>
+__global__ __launch_bounds__(256) void qproj_prefill_kernel(const QProj p, const int njobs)
 {
-    constexpr int RIDER_LDS = HS > 0 ? (2 * lin_region_bytes<(HS > 0 ? HS : 1)>() > XF_LDS ? 2 * lin_region_bytes<(HS > 0 ? HS : 1)>() : XF_LDS) : 0;
-    constexpr int LDS = QPF_LDS > RIDER_LDS ? QPF_LDS : RIDER_LDS;
-    static_assert(2 * LDS <= 160 * 1024, "two workgroups share a compute unit");
-    __shared__ __attribute__((aligned(16))) uint8_t lds[LDS];
-    const int bid = (int)blockIdx.x - fixed_wgs;
-    if (HS > 0 && bid < 0) {
-        const XfJob j = xf_job((int)blockIdx.x, LIP_XF_SETS, fixed_groups, p.T);
-        if (j.g >= 0) xf_body(lip_xf_slab(lip, j.set, j.g), lip.x, lip.T, lip.h, j.g, j.t0, lds);
-        return;
-    }
-    if (HS > 0 && bid >= njobs) {
-        constexpr int H = HS > 0 ? HS : 1;
-        const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-        const int l = threadIdx.x & 63;
-        const int job = bid - njobs;
-        i32x16 acc[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][r] = 0;
-        uint8_t *region = lds + (w & 1) * lin_region_bytes<H>();
-        if (w < 2) {
-            q_half_job<H>(rider, region, job, w, acc);
-            if (w == 1) q_pair_park(region, l, acc);
-        }
-        __syncthreads();
-        if (w == 0) q_pair_store<H>(rider, lds, job, l, acc);
-        return;
-    }
-    q_prefill_body<TB>(p, q_prefill_job_of(bid, njobs), lds);
+    __shared__ __attribute__((aligned(16))) uint8_t lds[QPF_LDS];
+    q_prefill_body<TB>(p, q_prefill_job_of((int)blockIdx.x, njobs), lds);
 }
 
 __global__ __launch_bounds__(512) void qproj_prefill256_kernel(const QProj p, const int njobs)
@@ -515,35 +481,12 @@ __global__ __launch_bounds__(256) void mlap_finish_kernel(const MlapParams p)
     mlap_finish_body(p, (int)blockIdx.x, lds);
 }
 
-__global__ __launch_bounds__(64 * FINP_WAVES) void mlap_finish_prefill_kernel(const MlapParams p, const int per)
-{
-    __shared__ __attribute__((aligned(16))) uint8_t lds[MLAP_FINP_LDS];
-    mlap_finish_prefill_body(p, (int)blockIdx.x, per, lds);
-}
-
 }  // namespace
-
-bool mlap_finish_is_prefill(const MlapParams &p) { return mlap_prefill_forms(p); }
-
-void mlap_finish_prefill_shape(const MlapParams &p, int &per, int &wgs)
-{
-    // runs of up to 16 blocks of 32 tokens per workgroup, two runs at least so that 128 heads fill the chip
-    const int nblocks = (p.T + FINP_TOK - 1) / FINP_TOK;
-    per = (nblocks + 1) / 2;
-    per = per > 16 ? 16 : per;
-    wgs = p.n_heads * ((nblocks + per - 1) / per);
-}
 
 hipError_t mlap_launch_finish(const MlapParams &p, hipStream_t stream)
 {
     if (mlap_fused_projection(p)) return prolog_prefill_launch(&p, nullptr, stream);
-    if (mlap_finish_is_prefill(p)) {
-        int per, wgs;
-        mlap_finish_prefill_shape(p, per, wgs);
-        hipLaunchKernelGGL(mlap_finish_prefill_kernel, dim3((unsigned)wgs), dim3(64 * FINP_WAVES), 0, stream, p, per);
-    } else {
-        hipLaunchKernelGGL(mlap_finish_kernel, dim3((unsigned)mlap_finish_wgs(p)), dim3(256), 0, stream, p);
-    }
+    hipLaunchKernelGGL(mlap_finish_kernel, dim3((unsigned)mlap_finish_wgs(p)), dim3(256), 0, stream, p);
     return hipGetLastError();
 }
 
@@ -585,7 +528,7 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
         }
         const int per_slab = ngroups * ttiles;
         const int wgs = big ? 8 * ((mslabs * ((p.T + XB_TOK - 1) / XB_TOK) * ngroups + 7) / 8) : 8 * ((mslabs >> 3) * per_slab + ((mslabs & 7) * per_slab + 7) / 8);   // the kernel's XCD-wise job order
-        const int sets = 1 + (lip_rider != nullptr && mlap_fused_projection(p) ? LIP_XF_SETS : 0);
+        const int sets = 1 + (lip_rider != nullptr ? LIP_XF_SETS : 0);
         const dim3 g((unsigned)(wgs + xf_jobs(sets, ngroups_fixed, p.T)));
 #define XM_LAUNCH(TBV) hipLaunchKernelGGL(mlap_xlinear_mfma_kernel<TBV>, g, dim3(256), 0, stream, p, mslabs, ngroups, wgs, sets, ngroups_fixed, lip)
         if (p.T <= 32) XM_LAUNCH(1);
@@ -625,31 +568,8 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
         }
         const int njobs = q_prefill_jobs(qp);
         const dim3 g((unsigned)njobs), b(256);
-        const int tbk = q_prefill_token_blocks(p.T);
-        if (lip_rider != nullptr && p.T < QPROJ_PREFILL_TOKENS) {
-            // the indexer prolog's split projection rides along: one more workgroup per job of a wave pair
-            const LipParams &lp = *lip_rider;
-            const QProj qr = {lp.q_norm, lp.w_qb, lp.qpart, lp.T, lp.q_lora, lp.n_heads, lp.q_norm_scale, lp.w_qb_scale};
-            const int rjobs = lp.n_heads * QPROJ_KSPLIT * ((lp.T + 31) / 32);
-            const int fixed_wgs = xf_jobs(LIP_XF_SETS, ngroups_fixed, p.T);
-            const dim3 gr((unsigned)(fixed_wgs + njobs + rjobs));
-            const int steps = lp.q_lora / QPROJ_KSPLIT / 32;
-#define QPF_RIDER(TBV)                                                                                       \
-    switch (steps) {                                                                                         \
-    case 4: hipLaunchKernelGGL((qproj_prefill_kernel<TBV, 2>), gr, b, 0, stream, qp, njobs, qr, lip, ngroups_fixed, fixed_wgs); break;     \
-    case 8: hipLaunchKernelGGL((qproj_prefill_kernel<TBV, 4>), gr, b, 0, stream, qp, njobs, qr, lip, ngroups_fixed, fixed_wgs); break;     \
-    case 12: hipLaunchKernelGGL((qproj_prefill_kernel<TBV, 6>), gr, b, 0, stream, qp, njobs, qr, lip, ngroups_fixed, fixed_wgs); break;    \
-    default: return hipErrorInvalidValue;                                                                    \
-    }
-            QPF_RIDER(1)                               // (fewer tokens than PROLOG_PF_MIN_TOKENS: one block)
-#undef QPF_RIDER
-            return hipGetLastError();
-        }
-        switch (tbk) {
-        case 1: hipLaunchKernelGGL((qproj_prefill_kernel<1, 0>), g, b, 0, stream, qp, njobs, qp, lip, 0, 0); break;
-        case 2: hipLaunchKernelGGL((qproj_prefill_kernel<2, 0>), g, b, 0, stream, qp, njobs, qp, lip, 0, 0); break;
-        default: hipLaunchKernelGGL((qproj_prefill_kernel<4, 0>), g, b, 0, stream, qp, njobs, qp, lip, 0, 0);
-        }
+        if (q_prefill_token_blocks(p.T) == 2) hipLaunchKernelGGL(qproj_prefill_kernel<2>, g, b, 0, stream, qp, njobs);
+        else hipLaunchKernelGGL(qproj_prefill_kernel<4>, g, b, 0, stream, qp, njobs);
         return hipGetLastError();
     }
     const int qjobs_a = qp.nslabs * QPROJ_KSPLIT * ((p.T + 31) / 32);

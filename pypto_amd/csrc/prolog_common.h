@@ -273,18 +273,18 @@ constexpr int QPF_BUF = QPF_TILE + 4 * QPF_TOK;
 constexpr int QPF_LDS = 2 * QPF_BUF;                   // 64 KiB
 
 __host__ __device__ inline int q_prefill_jobs(const QProj &p) { return p.nslabs * ((p.T + 127) / 128); }
-// token blocks per tile of the form to take: a launch of one tile of one or two blocks has forms of its own
-__host__ __device__ inline int q_prefill_token_blocks(const int T) { return T <= 32 ? 1 : (T <= 64 ? 2 : 4); }
+// token blocks per tile of the form to take: a launch of one tile of two blocks has a form of its own
+__host__ __device__ inline int q_prefill_token_blocks(const int T) { return T <= 64 ? 2 : 4; }
 
 // job: the blocks of a slab are neighbours in the job order.
-// TB: blocks of 32 tokens the tile holds.  TB = 4 is the form described above.  A launch of at most 32 or 64 tokens
-// (one tile of TB = 1 or 2 blocks per slab) shares a token block among 4 / TB waves, each with TB of the four
-// 32-column products: a wave then issues 4 or 8 products per chunk instead of 16 on padding tokens, and the
-// kernel's time is its requests' and no longer a wave's products'.  Same integer sums, same conversion.
+// TB: blocks of 32 tokens the tile holds.  TB = 4 is the form described above.  A launch of 64 tokens (one tile of TB = 2 blocks per
+// slab) shares a token block between two waves, each with two of the four 32-column products: a wave then issues 8 products
+// per chunk instead of 16 on padding tokens, and the kernel's time is its requests' and no longer a wave's products'.
+// Same integer sums, same conversion.
 template <int TB = 4>
 __device__ __forceinline__ void q_prefill_body(const QProj &p, const int job, uint8_t *lds)
 {
-    static_assert(TB == 1 || TB == 2 || TB == 4, "token blocks per tile");
+    static_assert(TB == 2 || TB == 4, "token blocks per tile");
     constexpr int WPB = 4 / TB;                        // waves that share a token block
     const int l = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

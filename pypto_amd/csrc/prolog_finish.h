@@ -438,10 +438,11 @@ __device__ __forceinline__ void lip_fixed_rows(const uint16_t *rows, const uint1
 
 // ---------------------------------------------------------------------------------- MLA prolog
 constexpr int FIN_W_BYTES = MLAP_NOPE * 64 * 2;    // a wave's slice of w_uk[head]: 128 rows x 64 columns bf16
-constexpr int MLAP_FIN_LDS = 4 * FIN_W_BYTES + MLAP_XTOK * MLAP_NOPE * 4 + MLAP_XTOK * MLAP_NOPE * 2;   // 71 680 bytes
+constexpr int MLAP_FIN_LDS = 4 * FIN_W_BYTES + MLAP_XTOK * MLAP_NOPE * 4;   // 69 632 bytes
 
-// Workgroup (head, half of the 512 output columns, block of 8 tokens); wave w owns output columns
-// colbase + 64w + l.
+// The MLA prolog's last stage with every sum in its fixed order (absorb_exact; otherwise the projection's launch finishes its heads
+// itself: prolog_small.h, prolog_prefill.h).  Workgroup (head, half of the 512 output columns, block of 8 tokens); wave w
+// owns output columns colbase + 64w + l.
 // The work of workgroup wg of the last launch (256 threads), in MLAP_FIN_LDS bytes of LDS at lds.
 // workgroup barriers mlap_finish_body passes (every thread, unconditionally): a launch whose workgroups hold more
 // than this body's 256 threads lets the surplus waves pass as many and leave
@@ -450,7 +451,6 @@ __device__ __forceinline__ void mlap_finish_body(const MlapParams &p, const int 
 {
     uint8_t *wsl = lds;
     float(*arow)[MLAP_NOPE] = reinterpret_cast<float(*)[MLAP_NOPE]>(lds + 4 * FIN_W_BYTES);
-    uint16_t(*abf)[MLAP_NOPE] = reinterpret_cast<uint16_t(*)[MLAP_NOPE]>(lds + 4 * FIN_W_BYTES + MLAP_XTOK * MLAP_NOPE * 4);   // the same values as bf16 (they are bf16-valued)
     const int l = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int head = wg % p.n_heads;
@@ -481,7 +481,6 @@ __device__ __forceinline__ void mlap_finish_body(const MlapParams &p, const int 
             q_value2(p.qpart, mlap_qsplits(p), p.T, tt, ncols, col, ts, cs[0], cs[1], av0, av1);
             const f32x2 av = {av0, av1};
             *reinterpret_cast<f32x2 *>(&arow[tl][2 * l]) = av;
-            *reinterpret_cast<uint32_t *>(&abf[tl][2 * l]) = pack_bf16x2(av[0], av[1]);
         }
         // rope part (first half-workgroup only): lane l < 32 -> channels 2l, 2l+1 = rotation partners l, 32+l
         if (half == 0 && l < 32 && t < p.T) {
@@ -501,47 +500,6 @@ __device__ __forceinline__ void mlap_finish_body(const MlapParams &p, const int 
     VM_WAIT(0);
     __syncthreads();                                   // (counted in MLAP_FIN_BARRIERS)
 
-    if (!p.absorb_exact) {
-        // On the matrix cores: C^T[col][token] = sum_i W^T[col][i] a^T[i][token], v_mfma_f32_32x32x16_bf16 with
-        // A = the wave's slice of w_uk read transposed out of LDS (ds_read_b64_tr_b16: lane (col, half) gets rows
-        // 16ks + 4*half + 0..3 and 16ks + 8 + 4*half + 0..3 of its column), B = the tokens' query values in the same
-        // row order (lanes of tokens 8..31 repeat token 0; their results are not stored).  Two blocks of 32
-        // columns, eight contraction steps.  Lane (token, half) then holds columns 8*(r/4) + 4*half + r%4 of a block.
-        const uint16_t *wt = reinterpret_cast<const uint16_t *>(wsl + w * FIN_W_BYTES) +
-                             (4 * (l >> 5) + ((l & 15) >> 2)) * 64 + 16 * ((l >> 4) & 1) + 4 * (l & 3);
-        const int tok = (l & 31) < MLAP_XTOK ? (l & 31) : 0;
-        const uint16_t *at = &abf[tok][4 * (l >> 5)];
-        f32x16 c[2];
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) c[cb][r] = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < MLAP_NOPE / 16; ++ks) {
-            const u32x2 b0 = *reinterpret_cast<const u32x2 *>(at + 16 * ks);
-            const u32x2 b1 = *reinterpret_cast<const u32x2 *>(at + 16 * ks + 8);
-            const u32x4 bq = {b0[0], b0[1], b1[0], b1[1]};
-#pragma unroll
-            for (int cb = 0; cb < 2; ++cb) {
-                const s16x4 a0 = lds_read_tr16(wt + (16 * ks) * 64 + 32 * cb);
-                const s16x4 a1 = lds_read_tr16(wt + (16 * ks + 8) * 64 + 32 * cb);
-                const s16x8 a = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
-                c[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, bq), c[cb], 0, 0, 0);
-            }
-        }
-        const int t = t0 + (l & 31);
-        if ((l & 31) < MLAP_XTOK && t < p.T) {
-            uint16_t *dst = p.q_nope + ((size_t)t * p.n_heads + head) * MLAP_KV + colbase + 4 * (l >> 5);
-#pragma unroll
-            for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const u32x2 v = {pack_bf16x2(c[cb][4 * q], c[cb][4 * q + 1]), pack_bf16x2(c[cb][4 * q + 2], c[cb][4 * q + 3])};
-                    *reinterpret_cast<u32x2 *>(dst + 32 * cb + 8 * q) = v;
-                }
-        }
-        return;
-    }
     // out[t][colbase + 64w + l] = sum_i a[t][i] * w_uk[head][i][col], i ascending; 8 tokens at once.
     // Chunks of four rows are read one chunk ahead of the multiply-adds that consume them.
     const uint16_t *wl = reinterpret_cast<const uint16_t *>(wsl + w * FIN_W_BYTES) + l;
@@ -579,132 +537,6 @@ __device__ __forceinline__ void mlap_finish_body(const MlapParams &p, const int 
     for (int t = 0; t < MLAP_XTOK; ++t)
         if (t0 + t < p.T)
             p.q_nope[((size_t)(t0 + t) * p.n_heads + head) * MLAP_KV + colbase + l] = (uint16_t)(pack_bf16x2(acc[t], 0.f) & 0xffffu);
-}
-
-// ------------------------------------------------------------------------ MLA prolog, prefill sizes
-// The same last stage for MLAP_MFMA_MIN_TOKENS tokens and more with the absorb product on the matrix cores: one workgroup of eight
-// waves per (head, run of `per` blocks of 32 tokens).  The head's whole w_uk (128 x 512 bf16, 128 KiB) is staged
-// once, wave w keeping the slice of output columns 64w..64w+63 in the layout of the decode form; then per block:
-// wave w moves the query channels of tokens 4w..4w+3 (de-quantised bf16 already: the projection is unsplit at these
-// sizes) into one of two bf16 operand buffers and rotates and stores their rope part, the loads of the next block go out, one barrier, and
-// 16 products per wave give 32 tokens x 64 columns.  A weight slice is read once per `per` blocks instead of once
-// per 8 tokens; each output has the bits of the decode form (same products, same order).
-constexpr int FINP_TOK = 32;
-constexpr int FINP_WAVES = 8;
-constexpr int FINP_APITCH = MLAP_NOPE + 8;   // elements between operand rows: 272 bytes, so that the 32 rows of an operand read spread over the banks
-constexpr int FINP_SPITCH = 144;             // bytes between the rows of a wave's output staging area (8 tokens x 64 columns)
-constexpr int FINP_STAGE = 8 * FINP_SPITCH;
-constexpr int MLAP_FINP_LDS = FINP_WAVES * FIN_W_BYTES + 2 * FINP_TOK * FINP_APITCH * 2 + FINP_WAVES * FINP_STAGE;   // 157 696 bytes
-
-struct FinRaw {
-    uint32_t nope[4], rope[4];     // two bf16 values each: the unsplit projection leaves its results de-quantised
-    uint16_t c0[4], c1[4], s0[4], s1[4];
-};
-
-__device__ __forceinline__ void mlap_finish_prefill_body(const MlapParams &p, const int wg, const int per, uint8_t *lds)
-{
-    uint8_t *wsl = lds;
-    uint16_t(*abf)[FINP_TOK][FINP_APITCH] = reinterpret_cast<uint16_t(*)[FINP_TOK][FINP_APITCH]>(lds + FINP_WAVES * FIN_W_BYTES);
-    const int l = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int head = wg % p.n_heads;
-    const int nblocks = (p.T + FINP_TOK - 1) / FINP_TOK;
-    const int b0 = (wg / p.n_heads) * per;
-    const int b1 = b0 + per < nblocks ? b0 + per : nblocks;
-    const int ncols = p.n_heads * MLAP_QHEAD;
-    const int colbase = 64 * w;
-
-    {   // this wave's slice: rows of 128 bytes, pitch 1024 bytes: 8 lanes per row, 8 rows per request
-        const uint8_t *src = reinterpret_cast<const uint8_t *>(p.w_uk) + ((size_t)head * MLAP_NOPE + (l >> 3)) * (MLAP_KV * 2) +
-                             colbase * 2 + 16 * (l & 7);
-        const uint32_t dst = (uint32_t)(uintptr_t)(lds_byte_t *)(wsl + w * FIN_W_BYTES);
-#pragma unroll 1
-        for (int i = 0; i < MLAP_NOPE / 8; ++i) dma16(src + (size_t)i * 8 * MLAP_KV * 2, dst + 1024 * i);
-    }
-    // lane l: nope channels 2l, 2l+1; lanes < 32: rope channels 2l, 2l+1 (= rotation partners l, 32+l)
-    auto load = [&](FinRaw &r, const int blk) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int t = blk * FINP_TOK + 4 * w + u;
-            const int tt = t < p.T ? t : p.T - 1;
-            const uint16_t *row = reinterpret_cast<const uint16_t *>(p.qpart) + (size_t)tt * ncols + head * MLAP_QHEAD;
-            r.nope[u] = *reinterpret_cast<const uint32_t *>(row + 2 * l);
-            if (l < 32) {
-                r.rope[u] = *reinterpret_cast<const uint32_t *>(row + MLAP_NOPE + 2 * l);
-                r.c0[u] = p.cos[(size_t)tt * MLAP_ROPE + l];
-                r.c1[u] = p.cos[(size_t)tt * MLAP_ROPE + 32 + l];
-                r.s0[u] = p.sin[(size_t)tt * MLAP_ROPE + l];
-                r.s1[u] = p.sin[(size_t)tt * MLAP_ROPE + 32 + l];
-            }
-        }
-    };
-    FinRaw raw;
-    if (b0 < b1) load(raw, b0);
-    VM_WAIT(0);
-
-    const uint16_t *wt = reinterpret_cast<const uint16_t *>(wsl + w * FIN_W_BYTES) +
-                         (4 * (l >> 5) + ((l & 15) >> 2)) * 64 + 16 * ((l >> 4) & 1) + 4 * (l & 3);
-#pragma unroll 1
-    for (int blk = b0; blk < b1; ++blk) {
-        const int buf = (blk - b0) & 1;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int tl = 4 * w + u;
-            const int t = blk * FINP_TOK + tl;
-            *reinterpret_cast<uint32_t *>(&abf[buf][tl][2 * l]) = raw.nope[u];
-            if (l < 32 && t < p.T) {
-                const float v0 = __uint_as_float(raw.rope[u] << 16);
-                const float v1 = __uint_as_float(raw.rope[u] & 0xffff0000u);
-                const float r0 = __builtin_fmaf(v0, bf16_bits_to_f32(raw.c0[u]), (-v1) * bf16_bits_to_f32(raw.s0[u]));
-                const float r1 = __builtin_fmaf(v1, bf16_bits_to_f32(raw.c1[u]), v0 * bf16_bits_to_f32(raw.s1[u]));
-                uint16_t *out = p.q_rope + ((size_t)t * p.n_heads + head) * MLAP_ROPE;
-                out[l] = (uint16_t)(pack_bf16x2(r0, 0.f) & 0xffffu);
-                out[32 + l] = (uint16_t)(pack_bf16x2(r1, 0.f) & 0xffffu);
-            }
-        }
-        if (blk + 1 < b1) load(raw, blk + 1);
-        __syncthreads();                               // this block's operands are complete; the other buffer is free
-
-        const uint16_t *at = &abf[buf][l & 31][4 * (l >> 5)];
-        f32x16 c[2];
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) c[cb][r] = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < MLAP_NOPE / 16; ++ks) {
-            const u32x2 bq0 = *reinterpret_cast<const u32x2 *>(at + 16 * ks);
-            const u32x2 bq1 = *reinterpret_cast<const u32x2 *>(at + 16 * ks + 8);
-            const u32x4 bq = {bq0[0], bq0[1], bq1[0], bq1[1]};
-#pragma unroll
-            for (int cb = 0; cb < 2; ++cb) {
-                const s16x4 a0 = lds_read_tr16(wt + (16 * ks) * 64 + 32 * cb);
-                const s16x4 a1 = lds_read_tr16(wt + (16 * ks + 8) * 64 + 32 * cb);
-                const s16x8 a = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
-                c[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, bq), c[cb], 0, 0, 0);
-            }
-        }
-        // Lane (token, half) holds 8-byte fragments of its token's row; they leave through the wave's staging area,
-        // eight tokens at a time, as whole 128-byte rows (16 bytes per lane) -- scattered fragments cost the memory
-        // side several times their bytes.
-        uint8_t *stg = lds + FINP_WAVES * FIN_W_BYTES + 2 * FINP_TOK * FINP_APITCH * 2 + w * FINP_STAGE;
-#pragma unroll
-        for (int qt = 0; qt < 4; ++qt) {
-            if (((l & 31) >> 3) == qt) {
-                uint8_t *row = stg + (l & 7) * FINP_SPITCH + 8 * (l >> 5);
-#pragma unroll
-                for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const u32x2 v = {pack_bf16x2(c[cb][4 * q], c[cb][4 * q + 1]), pack_bf16x2(c[cb][4 * q + 2], c[cb][4 * q + 3])};
-                        *reinterpret_cast<u32x2 *>(row + 64 * cb + 16 * q) = v;
-                    }
-            }
-            const u32x4 v = *reinterpret_cast<const u32x4 *>(stg + (l >> 3) * FINP_SPITCH + 16 * (l & 7));
-            const int t = blk * FINP_TOK + 8 * qt + (l >> 3);
-            if (t < p.T) *reinterpret_cast<u32x4 *>(p.q_nope + ((size_t)t * p.n_heads + head) * MLAP_KV + colbase + 8 * (l & 7)) = v;
-        }
-    }
 }
 
 }  // namespace

@@ -40,20 +40,6 @@ __global__ __launch_bounds__(64 * FIN_WAVES) void prolog_fused_finish_kernel(con
     }
 }
 
-// The same for the MLA prolog's prefill form of its last stage (eight waves like the indexer prolog's, all of a
-// compute unit's LDS): between 9 and 32 tokens that form has one workgroup per head -- half of the compute
-// units -- and the indexer prolog's workgroups take the compute units it leaves, then the ones it frees, instead of
-// waiting for a launch of their own.
-constexpr int FUSED_FINP_LDS = MLAP_FINP_LDS > LIP_FIN_LDS ? MLAP_FINP_LDS : LIP_FIN_LDS;
-static_assert(FINP_WAVES == FIN_WAVES, "one block size for both bodies");
-__global__ __launch_bounds__(64 * FIN_WAVES) void prolog_fused_finish_prefill_kernel(const MlapParams pm, const int per, const LipParams pl,
-                                                                                     const int mla_wgs, const int q_wgs)
-{
-    __shared__ __attribute__((aligned(16))) uint8_t lds[FUSED_FINP_LDS];
-    if ((int)blockIdx.x < mla_wgs) mlap_finish_prefill_body(pm, (int)blockIdx.x, per, lds);
-    else lip_finish_body(pl, q_wgs, (int)blockIdx.x - mla_wgs, lds);
-}
-
 // Projections and last stages at prefill sizes (prolog_prefill.h): [0, mla_wgs) the attention query, then lip_wgs of the
 // indexer query, then the indexer's key rows and weights, a token per wave.  64 * TB tokens per workgroup of a head.
 // FIXED: the indexer query's Hadamard sums in their fixed order (fewer than LIP_MFMA_MIN_TOKENS tokens).
@@ -149,23 +135,7 @@ hipError_t prolog_fused_launch(const MlapParams &pm, const LipParams &pl, hipStr
         if (e != hipSuccess) return e;
     }
     if (joined) return prolog_prefill_launch(&pm, &px, stream);
-    if (mlap_fused_projection(pm)) {
-        e = mlap_launch_finish(pm, stream);
-        if (e != hipSuccess) return e;
-        return lip_launch_finish(px, stream);
-    }
-    int per = 0, pf_wgs = 0;
-    if (mlap_finish_is_prefill(pm)) mlap_finish_prefill_shape(pm, per, pf_wgs);
-    // up to 32 tokens: one workgroup per head, the indexer half's take the other compute units (more would queue one
-    // to a compute unit behind a full chip, slower than their own launch at two)
-    if (mlap_finish_is_prefill(pm) && !lip_q_on_matrix_cores(px) && pf_wgs <= 128) {
-        const int q_wgs = lip_finish_query_wgs(px);
-        hipLaunchKernelGGL(prolog_fused_finish_prefill_kernel, dim3((unsigned)(pf_wgs + q_wgs + px.T)), dim3(64 * FIN_WAVES), 0, stream, pm, per,
-                           px, pf_wgs, q_wgs);
-        return hipGetLastError();
-    }
-    if (mlap_finish_is_prefill(pm) || lip_q_on_matrix_cores(px)) {
-        // prefill sizes: the last stages have forms of their own (the attention query's: one workgroup per compute unit)
+    if (mlap_fused_projection(pm) || lip_q_on_matrix_cores(px)) {        // one half's last stage is part of its projection
         e = mlap_launch_finish(pm, stream);
         if (e != hipSuccess) return e;
         return lip_launch_finish(px, stream);

@@ -39,9 +39,6 @@ struct XlSlab {
     int out_pitch_hi = 0;
 };
 
-// row widths the staging handles (whole 16-byte pieces, a power of two of them per row)
-__host__ __device__ inline bool xl_width_ok(const int wbytes) { return wbytes >= 16 && wbytes <= 256 && (wbytes & (wbytes - 1)) == 0; }
-
 // group g of the hidden axis, tokens t0 .. t0 + 7 (rows past T - 1 repeat it and are not stored)
 __device__ __forceinline__ void xl_body(const XlSlab &sl, const uint16_t *x, const int T, const int h, const int g, const int t0, uint8_t *smem)
 {
