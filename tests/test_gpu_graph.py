@@ -116,25 +116,28 @@ def test_prologs_replays_match_eager(b, s1, act, ni):
             assert torch.equal(g_.view(torch.uint8), w_.view(torch.uint8)), f"replay {rep}: output {i} differs from the eager call"
 
 
-@pytest.mark.parametrize("b,s1,act", [(4, 2, [5000, 300, 129, 64]), (16, 2, [5000, 300, 129, 64] * 4)])
-def test_fused_prolog_operator_replays_match_the_two_operators_called_eagerly(b, s1, act):
-    """mla_indexer_prolog_quant_d (one library call, one workspace from torch's pool, the last launches of the two
-    halves merged) recorded once and replayed with new hidden states: every replay equals the two separate
-    operators called eagerly on the same inputs, bit for bit.  8 tokens: the decode forms' four launches; 32 tokens:
-    the MLA half's matrix-core forms with the indexer half's first launch riding in them."""
+@pytest.mark.parametrize("b,s1,act,n_idx", [(4, 2, [5000, 300, 129, 64], 4), (16, 2, [5000, 300, 129, 64] * 4, 4),
+                                             (4, 2, [5000, 300, 129, 64], 64), (16, 2, [5000, 300, 129, 64] * 4, 64),
+                                             (20, 2, [5000, 300, 129, 64] * 5, 64), (20, 4, [5000, 300, 129, 64] * 5, 64)])
+def test_fused_prolog_operator_replays_match_the_two_operators_called_eagerly(b, s1, act, n_idx):
+    """mla_indexer_prolog_quant_d (one library call, one workspace from torch's pool) recorded once and replayed with new hidden
+    states: every replay equals the two separate operators called eagerly on the same inputs, bit for bit.  With 64 indexer
+    heads three launches, the indexer half's work in the MLA half's: the fixed-order first launch (8 tokens) or the
+    matrix-core one, the last launch for up to 32 tokens, for up to 63 and beyond; with 4 heads the indexer half keeps
+    launches of its own."""
     from pypto_amd.synthetic import gen_indexer_prolog_inputs, gen_mla_prolog_inputs
     dev = torch.device(DEV)
     kw = dict(h=512, q_lora_rank=1536)
     mla = gen_mla_prolog_inputs(b, s1, act, seed=31, n_heads=8, **kw).to(dev)
-    lip = gen_indexer_prolog_inputs(b, s1, act, seed=32, n_heads=4, **kw).to(dev)
+    lip = gen_indexer_prolog_inputs(b, s1, act, seed=32, n_heads=n_idx, **kw).to(dev)
     t = b * s1
     caches = [mla.kv_cache, mla.kr_cache, mla.k_scale_cache, lip.k_cache, lip.k_cache_scale]
     base = [c.clone() for c in caches]
 
     def outputs():
         return (torch.zeros(t, 8, 512, dtype=torch.bfloat16, device=dev), torch.zeros(t, 8, 64, dtype=torch.bfloat16, device=dev),
-                torch.zeros(t, 4, 128, dtype=torch.int8, device=dev), torch.zeros(t, 4, 1, dtype=torch.float16, device=dev),
-                torch.zeros(t, 4, dtype=torch.float16, device=dev))
+                torch.zeros(t, n_idx, 128, dtype=torch.int8, device=dev), torch.zeros(t, n_idx, 1, dtype=torch.float16, device=dev),
+                torch.zeros(t, n_idx, dtype=torch.float16, device=dev))
 
     def fused(o):
         qnope, qrope, iq, iqs, iw = o
