@@ -415,8 +415,8 @@ int pto_mla_prolog_quant_launch(const PtoMlaPrologQuantArgs *args, void *hip_str
  *            workspace_bytes are ignored: taken from the MLA part and the common workspace.
  *   workspace  pto_mla_indexer_prolog_quant_workspace_bytes() bytes, 256-byte aligned: the
  *            intermediates, then the partial sums of the MLA half, then those of the indexer half.
- * Five kernels on the given stream, nothing else (the last launches of the two halves do not
- * depend on each other and run as one); errors as for the two operators.
+ * Three kernels on the given stream, nothing else (the indexer half's work rides in the MLA half's launches);
+ * up to six with fixed-order sums or with indexer head counts that cannot share them.  Errors as for the two operators.
  */
 typedef struct PtoMlaIndexerPrologQuantArgs {
     PtoMlaPrologQuantArgs mla;

@@ -15,10 +15,8 @@ constexpr int MLAP_MAX_XGROUPS = 32; // h <= 32 * 8 * 64 = 16384
 constexpr int MLAP_MAX_QLORA = 1536;
 constexpr int QPROJ_KSPLIT_HOST = 4; // partial sums of the int8 projection (prolog_common.h: QPROJ_KSPLIT)
 constexpr int MLAP_XTOK = 8;         // tokens per job of the first and of the last kernel
-constexpr int MLAP_MFMA_MIN_TOKENS = 9;    // from here on the stages take their prefill forms unless absorb_exact: the first launch
-                                           // sums on the matrix cores, the projection runs unsplit, the last stage walks token blocks
-                                           // per head (the decode forms work on 8 tokens at a time and their cost grows with every
-                                           // 8 tokens; those forms cost the same from 9 to 128 tokens, about what 8 tokens cost here)
+constexpr int MLAP_MFMA_MIN_TOKENS = 9;    // from here on the first launch sums on the matrix cores unless absorb_exact (the fixed-order
+                                           // form works on 8 tokens at a time and its cost grows with every 8 tokens)
 constexpr int MLAP_UNSPLIT_MIN_TOKENS = 64;   // with absorb_exact the projection still runs unsplit from here on
 // ranges of the hidden axis (partial sums per token) of that form, at most.  With a single token tile the sixteen
 // matrix-core slabs x 14 ranges and the rope columns' 32 workgroups are one workgroup per compute unit of an
@@ -78,7 +76,7 @@ struct MlapRider {
     int q_slabs;
 };
 
-// the stages' prefill forms (matrix-core sums over the hidden axis, last stage per head and run of token blocks)
+// whether the first launch sums on the matrix cores
 __host__ __device__ inline bool mlap_prefill_forms(const MlapParams &p) { return p.T >= MLAP_MFMA_MIN_TOKENS && !p.absorb_exact; }
 // unless every sum is to keep its fixed order the projection and the last stage are one launch (prolog_small.h up to
 // PROLOG_SMALL_TOKENS tokens, prolog_prefill.h beyond)

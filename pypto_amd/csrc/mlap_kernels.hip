@@ -12,34 +12,32 @@
 // sums against w_uk, and from MLAP_MFMA_MIN_TOKENS tokens on the sums over the hidden axis, run there as well
 // (MlapParams::absorb_exact = 0: the same exact products in the cores' own summation order).
 //
-// Four launches; below MLAP_MFMA_MIN_TOKENS tokens (decode):
+// Three launches -- sums over the hidden axis, latents, and one for the projection and everything behind it -- or, with every
+// sum in its fixed order (absorb_exact), four:
 //   mlap_xlinear_kernel  x . [w_dq | w_dkv_kr] (xlinear_fixed.h): one workgroup of eight waves per (slab of 128
 //                        columns, group of 512 hidden rows, 8 tokens); each wave takes a 64-row block (staged by
 //                        LDS-DMA, hidden states widened to fp32 in LDS), block sums meet in LDS and are
-//                        chained into the group sum.
+//                        chained into the group sum.  Below MLAP_MFMA_MIN_TOKENS tokens, and with absorb_exact.
+//   mlap_xlinear_mfma_kernel   the same sums on the matrix cores (xlinear_mfma.h): per workgroup a 128-column slab x
+//                        tokens x a range of the hidden axis, v_mfma_f32_32x32x16_bf16 with the row-major weight chunk as
+//                        the transposed operand.  The launch's last workgroups take the 64 rope columns of w_dkv_kr in
+//                        their fixed order instead (the rotated key allows no outlier under the reference's acceptance
+//                        rule), and the indexer prolog's sums with them in the fused operator.
 //   mlap_mid_kernel      per token: group sums chained, bf16, RMS norm (one wave per slab), per-token
 //                        int8 quantisation of the query latent; RMS norm and per-slab quantisation of
 //                        the key latent, rope of the key, scatter into the caches.
+//   mlap_mid_prefill_kernel    the same as a wave per token and latent (64 tokens and more)
+//   prolog_small_kernel, prolog_prefill_kernel (prolog_fused.hip)   a head's int8 projection, rope and product with w_uk
+// With absorb_exact instead of the last:
 //   qproj_kernel         int8 projection of the query latent (shared job code: LDS-DMA tile,
-//                        transposing 8-bit LDS reads, v_mfma_i32_32x32x32_i8), partial sums per quarter.
+//                        transposing 8-bit LDS reads, v_mfma_i32_32x32x32_i8), partial sums per quarter; from
+//                        MLAP_UNSPLIT_MIN_TOKENS tokens on qproj_prefill_kernel, qproj_prefill256_kernel (prolog_common.h):
+//                        unsplit, a workgroup per tile over the whole reduction axis, results de-quantised.
 //   mlap_finish_kernel   per (head, half of the 512 output columns, 8 tokens): partial sums added and
 //                        de-quantised, rope part rotated and stored, nope part times the head's w_uk
-//                        slice (staged in LDS by LDS-DMA): on the matrix cores, or one output column per lane.
-// For the fused operator the first and the third of these carry the lightning-indexer prolog's first stage along
+//                        slice (staged in LDS by LDS-DMA), one output column per lane.
+// For the fused operator the fixed-order first launch and qproj_kernel carry the lightning-indexer prolog's first stage along
 // (MlapRider in mlap_kernels.h: its hidden-axis sums have this prolog's fixed order, its projection this one's q_norm).
-// From MLAP_MFMA_MIN_TOKENS tokens on (prefill chunks) the stages take forms of their own:
-//   mlap_xlinear_mfma_kernel   the sums over the hidden axis on the matrix cores (xlinear_mfma.h) unless the fixed
-//                        order is asked for: per workgroup a 128-column slab x 128 tokens x a range of the hidden
-//                        axis, v_mfma_f32_32x32x16_bf16 with the row-major weight chunk as the transposed operand.
-//                        The launch's last workgroups take the 64 rope columns of w_dkv_kr in their fixed order
-//                        instead (the rotated key allows no outlier under the reference's acceptance rule).
-//   mlap_mid_prefill_kernel    the middle stage as a wave per token and latent (64 tokens and more)
-//   qproj_prefill_kernel   the projection unsplit (prolog_common.h), a workgroup per tile over the whole reduction axis;
-//                        results leave de-quantised (up to 15 tokens, and in the fixed-order mode, which has
-//                        qproj_prefill256_kernel for more).
-//   mlap_finish_prefill_kernel   per (head, run of 32-token blocks): the head's whole w_uk staged once
-//                        (prolog_finish.h), absorb product on the matrix cores (up to 15 tokens).
-// From PROLOG_PF_MIN_TOKENS tokens on the projection and the last stage are one launch (prolog_prefill.h).
 #include <cstring>
 
 #include "mlap_kernels.h"
@@ -105,7 +103,7 @@ static_assert(XM_KC == MLAP_XBLOCK, "the workspace is sized in chunks of the hid
 // sequential sums), 64 columns each: the rope columns of w_dkv_kr at every size -- the reference's acceptance rule allows
 // the rotated key no outlier at all (deepseekv32_mla_prolog_quant.py:688: atol 1e-4, rtol 2^-7 per element, ratio 0), and
 // a sum that lands next to a bf16 rounding boundary in another order moves a small rotated value by more than that --
-// and, in the fused prolog from PROLOG_PF_MIN_TOKENS tokens on, the indexer prolog's wk and w_proj.  They are short and follow the long workgroups of the
+// and, in the fused prolog, the indexer prolog's wk and w_proj.  They are short and follow the long workgroups of the
 // other slabs, so they fill the launch's last round; two workgroups fit a compute unit.  (1000 tokens: 69 us here and 79
 // in a launch of the indexer's own before they shared it.)
 // TB: at most 32 * TB tokens (xm_small_body), 0 for tiles of 128 tokens (xm_body), XM_BIG for tiles of 256 (xb_body).

@@ -1,6 +1,6 @@
-// The last launch of each of the two prologs (query rows finished: rope, Hadamard / absorb product,
-// quantisation; key row and head weights of the indexer) as device functions over an LDS pool, so that
-// the same code runs as a launch of its own and, for the fused operator, side by side in one launch.
+// What follows the projections of the two prologs (query rows: rope, Hadamard / absorb product, quantisation; key row and head
+// weights of the indexer) as device functions over an LDS pool, so that the same code runs as a launch of its own and, for the
+// fused operator, side by side in one launch.
 // Included by lip_kernels.hip, mlap_kernels.hip and prolog_fused.hip after prolog_common.h.
 #pragma once
 #include "lip_kernels.h"
@@ -264,7 +264,7 @@ __device__ __forceinline__ void lip_finish_body(const LipParams &p, const int q_
     }
 }
 
-// The key rows and weights at prefill sizes: a workgroup of FINT_WAVES waves takes FINT_WAVES tokens, one per wave (the
+// The key rows and weights where the queries are finished by their projection's launch: a workgroup of FINT_WAVES waves takes FINT_WAVES tokens, one per wave (the
 // matrix is staged once for all of them instead of once per token, and the rows are finished side by side instead of
 // by one wave per workgroup).  A wave adds its token's partial rows in registers, in the order of the form they come
 // in: group sums ascending, or blocks / ranges ascending into groups of eight and the groups ascending.

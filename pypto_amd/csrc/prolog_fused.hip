@@ -1,15 +1,17 @@
 // MLA prolog + lightning-indexer prolog as one operator (mla_indexer_prolog_quant_d/_p of the reference,
-// examples/models/deepseek_v32_exp/mla_indexer_prolog_quant_impl.py:141-256).  At decode sizes it is the MLA
-// prolog's four launches with the indexer prolog's work riding in them (MlapRider): hidden-axis sums (wk as one
-// more column slab, w_proj beside the rope columns of w_dkv_kr) -> norms and quantisation of the latents -> int8
-// projections of the attention query and of the indexer query, jobs of one kind -> ONE last launch for both: the
-// workgroups that finish the attention query (absorb product, 70 KB of LDS, four waves) and those that finish the
-// indexer's query rows, key row and weights (54 KB, eight waves) do not depend on each other and fit a compute
-// unit together, so they run side by side instead of one launch after the other.  Where the indexer prolog cannot
-// ride (other than 64 indexer heads) its first launch follows the MLA prolog's third.  From 9 tokens on the MLA
-// prolog's prefill forms take the indexer prolog's fixed-order sums along, up to 15 tokens its projection too (four
-// launches, the two last stages sharing one); from 16 tokens on both projections and all that follows them are one launch
-// (three in all).
+// examples/models/deepseek_v32_exp/mla_indexer_prolog_quant_impl.py:141-256).  Three launches, the MLA prolog's with the
+// indexer prolog's work in them:
+//   sums over the hidden axis   up to 8 tokens wk as one more column slab, w_proj beside the rope columns of w_dkv_kr
+//                        (MlapRider, 64 indexer heads); beyond, its fixed-order sums as further workgroups
+//   latents              norms and quantisation
+//   projections and everything behind them   a workgroup per head of either query (up to 32 tokens: prolog_small.h) or per head
+//                        and tile of tokens (prolog_prefill.h), and workgroups for the indexer's key rows and weights
+// With absorb_exact and fewer than 64 tokens the projections are a launch of their own (jobs of one kind), and the last one
+// finishes both queries from their partial sums: the workgroups that finish the attention query (absorb product, 68 KB of LDS,
+// four waves) and those that finish the indexer's query rows, key row and weights (54 KB, eight waves) do not depend on each
+// other and fit a compute unit together.  Where the indexer prolog cannot ride (other than 64 indexer heads up to 8 tokens or
+// with absorb_exact, w_proj rows that are no power of two of 16-byte pieces, sums over the hidden axis in the cores' order)
+// its own launches follow.
 #include <cstring>
 
 #include "prolog_fused.h"
@@ -102,9 +104,8 @@ hipError_t prolog_prefill_launch(const MlapParams *pm, const LipParams *pl, hipS
 
 hipError_t prolog_fused_launch(const MlapParams &pm, const LipParams &pl, hipStream_t stream)
 {
-    // Decode sizes: the indexer prolog's first launch has no work of a kind of its own -- its sums over the hidden
-    // axis are more column slabs of the MLA prolog's first launch and its int8 projection more jobs of the third
-    // (MlapRider) -- so the pass is four launches: hidden-axis sums, latents, projections, one finish for both.
+    // The fixed-order first launch: the indexer prolog's sums over the hidden axis are more column slabs of it and, with
+    // absorb_exact, its int8 projection more jobs of the third (MlapRider).
     if (mlap_takes_rider(pm) && pl.T == pm.T && pl.h == pm.h && pl.q_lora == pm.q_lora && pl.x == pm.x && pl.q_norm == pm.q_norm &&
         pl.q_norm_scale == pm.q_norm_scale && pl.n_heads == 64) {
         const MlapRider rd = {pl.wk, pl.w_proj, pl.xpart, pl.w_qb, pl.qpart, pl.n_heads};

@@ -1,4 +1,4 @@
-// The last stage of both prologs at prefill sizes, projection included: a head's int8 up-projection is finished where it is
+// The last launch of both prologs for more than 32 tokens, projection included: a head's int8 up-projection is finished where it is
 // made -- de-quantised out of the accumulators, rotated, and taken through the product with w_uk (attention query) or the
 // Hadamard matrix and quantised (indexer query) -- instead of going to memory as bf16 for a launch of its own.
 // Included by prolog_fused.hip after prolog_finish.h.

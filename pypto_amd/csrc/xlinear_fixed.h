@@ -1,7 +1,7 @@
 // Fixed-order sums over the hidden axis, one group of eight blocks of 64 rows per workgroup: x [T, h] bf16 times a
 // slab of columns of a row-major bf16 weight matrix.  Two forms: xl_body on the vector ALU, 8 tokens per workgroup (the
 // MLA prolog's fixed-order launches), and xf_body on the matrix cores, 32 tokens (the rope columns and the indexer
-// prolog's wk and w_proj from 9 or 64 tokens on); included after prolog_common.h.
+// prolog's wk and w_proj from 9 tokens on in the fused operator, from 64 on alone); included after prolog_common.h.
 //
 // Every product of two bf16 values is exact in fp32; a block is summed ascending from 0.0 by fp32 FMAs, the
 // workgroup's eight block sums (one per wave) meet in LDS and are added ascending into the group sum, which is all

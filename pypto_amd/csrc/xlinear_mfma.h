@@ -1,4 +1,4 @@
-// Sums over the hidden axis on the matrix cores, for prefill-sized token counts: x [T, h] bf16 times a slab of up
+// Sums over the hidden axis on the matrix cores, for 9 tokens and more: x [T, h] bf16 times a slab of up
 // to 128 columns of a row-major bf16 weight matrix, as partial sums over a range of the hidden axis.  Shared by the
 // MLA prolog (w_dq, w_dkv_kr) and the lightning-indexer prolog (wk, w_proj); included after prolog_common.h.
 //

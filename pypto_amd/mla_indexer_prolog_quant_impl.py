@@ -4,9 +4,9 @@ Same callables, argument names and order as ``mla_indexer_prolog_quant_d`` / ``m
 the reference example (examples/models/deepseek_v32_exp/mla_indexer_prolog_quant_impl.py:49-138, 141-256): the
 MLA prolog runs first; its int8 normalised query latent and that latent's scale -- intermediates the caller
 never sees (:218-219) -- are the indexer prolog's ``q_norm`` / ``q_norm_scale``; hidden states, rope tables and
-cache index are shared.  One launch call of the library (``pto_mla_indexer_prolog_quant_launch``: five kernels on the
-current stream, the last launches of the two halves merged into one) and one workspace, in which the two
-intermediates live; see the two operators'
+cache index are shared.  One launch call of the library (``pto_mla_indexer_prolog_quant_launch``: three kernels on the
+current stream, the indexer half's work in the MLA half's launches; up to six with fixed-order sums or with indexer head
+counts that cannot share them) and one workspace, in which the two intermediates live; see the two operators'
 modules for layouts and for what is built.  Returns ``None``.
 """
 from __future__ import annotations

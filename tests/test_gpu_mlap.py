@@ -275,7 +275,7 @@ def test_fused_prolog_fixed_order_sums_at_tile_edges(t, n_idx):
 
 @pytest.mark.parametrize("t,q_lora", [(64, 512), (127, 1536), (129, 1024), (256, 512), (257, 512), (512, 512), (513, 1024), (700, 512)])
 def test_fused_prolog_query_rows_at_tile_edges(t, q_lora):
-    """The launch that makes and finishes both queries from 64 tokens on, at the edges of its tiles of 128 and 256 tokens and
+    """The launch that makes and finishes both queries, from 64 tokens on (the Hadamard sums in the cores' order), at the edges of its tiles of 128 and 256 tokens and
     of the hidden-axis launch's: every query output against the sequential statement under the reference's rule."""
     from oracle import lip_oracle as lo
     from pypto_amd import lightning_indexer_prolog_quant_impl as lip_impl
@@ -332,14 +332,13 @@ def test_fused_prolog_indexer_outputs_below_64_tokens_have_the_fixed_order_bits(
                                         ("default", "t_40_idx_64"), ("exact", "t_40_idx_64"), ("default", "t_7_idx_64"),
                                         ("default", "t_32_idx_64")])
 def test_fused_prolog_at_prefill_size_equals_the_two_operators_chained(mode, shape):
-    """150 tokens (ragged last block of the token tiles): the fused operator's prefill-sized launches (unsplit int8
-    projections, the attention query's last stage per head and run of token blocks) against the MLA prolog and the
-    indexer prolog called one after the other on the same inputs, bit for bit, in each of the summation modes.
-    The two decode-sized shapes: with 64 indexer heads the indexer prolog's first stage rides in the MLA prolog's
+    """150 tokens (ragged last block of the token tiles): the fused operator against the MLA prolog and the indexer prolog
+    called one after the other on the same inputs, bit for bit, in each of the summation modes.
+    The decode-sized shapes: with 64 indexer heads the indexer prolog's first stage rides in the MLA prolog's
     launches (7 tokens by default; 11 in the exact mode: two token groups, the second ragged; 576 hidden channels: a
-    second, short group of blocks), with 32 heads it keeps its own launch.  At 40 tokens the MLA half takes its prefill forms by default
-    while the indexer half keeps its decode forms (in the exact mode both keep them, and the rider); at 32 and at 11
-    tokens the two last stages share a launch as well."""
+    second, short group of blocks), with 32 heads and 3 tokens it keeps its own launches.  From 9 tokens on (11, 32, 40) its sums ride
+    in the matrix-core launch by default and both queries are made and finished in the last one, in the form for up to 32
+    tokens or the one for more."""
     from pypto_amd import lightning_indexer_prolog_quant_impl as lip_impl
     from pypto_amd import mla_prolog_quant_impl as impl
     from pypto_amd.synthetic import gen_indexer_prolog_inputs
