@@ -173,7 +173,7 @@ def prolog_leg(torch, dev, pypto_amd, b=4, s1=2, calls=20, replays=10):
 
 
 def mla_prolog_leg(torch, dev, pypto_amd, b=4, s1=2, calls=10, replays=10):
-    """One MLA prolog pass = the four launches of mla_prolog_quant_d; timed like prolog_leg (HIP graph of `calls`
+    """One MLA prolog pass = the three launches of mla_prolog_quant_d; timed like prolog_leg (HIP graph of `calls`
     passes, each with its own copy of the four weight tensors: 10 x 85 MB exceeds the memory-side cache)."""
     from pypto_amd.synthetic import gen_mla_prolog_inputs
     d = gen_mla_prolog_inputs(b, s1, [4096] * b, seed=0).to(dev)
@@ -622,7 +622,7 @@ def main():
                      "frac": achieved_tflops / PEAK_BF16_TFLOPS,
                      "traffic": measured_traffic(TRAFFIC_FILE, "traffic_bytes_per_step", lib_version,
                                                  {"key_splits": key_splits}),
-                     "kernel": "sfa_decode_kernel<4>" + (f" + sfa_combine_kernel<{combine_ns}>" if key_splits > 1 else "") + " (one step)",
+                     "kernel": "sfa_decode_kernel<4, true>" + (f" + sfa_combine_kernel<{combine_ns}, false>" if key_splits > 1 else "") + " (one step)",
                      "key_splits": int(key_splits),
                      "launch_ms_avg": ev_avg_ms, "launch_ms_min": ev_min_ms, "launch_ms_avg_unsettled": ev_avg_ms_unsettled,
                      "frac_unsettled": flops / (ev_avg_ms_unsettled * 1e-3) / 1e12 / PEAK_BF16_TFLOPS, "flops_per_launch": flops},

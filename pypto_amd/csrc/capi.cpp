@@ -132,8 +132,10 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
     auto partial_bytes = [&](const long long r, const int ns, const bool f32 = false) {
         return ns > 1 ? (size_t)r * ns * a->nq * (512 * (f32 ? sizeof(float) : sizeof(uint16_t)) + 2 * sizeof(float)) : (size_t)0;
     };
-    // The schedule model, in microseconds: what a launch pair took over 1 to 128 rows x 16 to 128 heads x 1 to 64 splits
-    // (fitted to within 10 %; neighbouring choices differ by less).  A compute unit holds one workgroup; a round of them
+    // The schedule model, in microseconds: what a launch pair over an int8 cache took over 1 to 128 rows x 16 to 128 heads x 1 to
+    // 64 splits (fitted to within 10 %; neighbouring choices differ by less).  The same figures serve the other cache formats
+    // and every top-k: against the fastest of all head-group and split counts, both caches, 1 to 300 rows, 16 to 128 heads, the
+    // choice is within 5 % for top-k 1024 and 2048 but for a single row (up to 11 %, 64 splits where 32 are faster).  A compute unit holds one workgroup; a round of them
     // is as long as a split's tiles; starting, staging the query and the first tile and the merge launch are `fixed`, and
     // the partial results cost with the number of workgroups that write them.  Fewer head groups per workgroup make
     // a tile shorter, and the prologue, but the tiles of a row are de-quantised once per workgroup: that pays while the
@@ -440,7 +442,7 @@ extern "C" {
 
 const char *pto_last_error(void) { return g_err; }
 
-const char *pto_version(void) { return "0.6.0"; }
+const char *pto_version(void) { return "0.7.0"; }
 
 int pto_abi_revision(void) { return PTO_ABI_REVISION; }
 
