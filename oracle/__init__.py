@@ -1,7 +1,7 @@
 """CPU oracle for the quantized DeepSeek-V3.2 sparse-attention path.
 
 TEST INFRASTRUCTURE ONLY.  Nothing in the shipped package imports this
-directory; it is the checker used by ``tests/``, by ``__graft_entry__.smoke()``
+directory; it is the oracle used by ``tests/``, by ``__graft_entry__.smoke()``
 and by the ``cpu_baseline`` leg of ``bench.py``.  The product path is the HIP
 library under ``pypto_amd/csrc`` and fails loudly when that library is absent.
 

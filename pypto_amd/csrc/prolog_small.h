@@ -3,7 +3,7 @@
 // One workgroup of four waves per head and compute unit.  The launch's tokens lie in LDS whole; everything else of the LDS is a
 // ring of requests that never runs dry: chunks of 64 rows of the head's projection and, behind them without a gap, its w_uk,
 // sixteen rows at a time.  Bound: the rate at which 192 workgroups can draw weights out of memory with 80 KiB (attention
-// query) on their way each.  (Fused prolog, same box: 8 tokens as two launches with partial sums in between 40.7 us per pass,
+// query) on their way each.  (Fused prolog: 8 tokens as two launches with partial sums in between 40.7 us per pass,
 // so 34.2; 32 tokens with the 24 KiB in flight of the form for more tokens 44.2, so 42.5.)
 // Included by prolog_fused.hip after prolog_prefill.h.
 #pragma once

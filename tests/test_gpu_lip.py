@@ -121,7 +121,7 @@ def test_prolog_mtp_batch_t128():
 ])
 def test_prolog_reference_large_cases(b, s1, act, what):
     """The reference's "large" cases (deepseekv32_lightning_indexer_prolog_quant.py:470-509) at the model's
-    full projection sizes: the decode kernels walk the token blocks, so the bar stays bit-exact."""
+    full projection sizes: every sum in its fixed order, so the bar stays bit-exact."""
     inp = gen_indexer_prolog_inputs(b, s1, act, seed=b + s1)
     ref = lo.indexer_prolog_ref(*inp.input_tensors())
     assert_exact(run_op(inp), ref, what)
