@@ -93,7 +93,8 @@ struct SfaPlan {
     int nsplit;
     int whole_slots;      // rows 0 .. 8 * whole_slots - 1 are not split
     bool part_f32;        // partial results in fp32 instead of fp16
-    size_t part_o_bytes;
+    size_t scratch_bytes; // what a caller is asked for, for partial results: the launch uses as much or less
+    size_t part_o_bytes;  // what the launch uses of it
     size_t part_ml_bytes;
     size_t predeq_bytes;  // the whole cache de-quantised once, behind the partial results (0: not worth it)
     size_t predeq_offset; // where in the workspace
@@ -215,6 +216,7 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
                 const double cost = (double)full * round_us(hg_max, 1) + round_us(hg_max, sb) +
                                     tail_us(hg_max, rows_b * shares(hg_max) * sb, sb);
                 if (cost < best) {
+                    best = cost;
                     pl.head_groups = hg_max;
                     pl.hgroups = shares(hg_max);
                     pl.nsplit = sb;
@@ -225,24 +227,63 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
         }
     }
     pl.part_f32 = f32 && pl.nsplit > 1;
+    pl.scratch_bytes = partial_bytes(split_rows, pl.nsplit, f32);
+    // More than 32 heads: workgroups of 64 heads (sfa_slice_kernel) where they are the faster ones, within the bytes that a caller
+    // is asked for, which stay those of the division above.  In microseconds, fitted to an int8 cache, 1 to 128 rows, top-k 2048,
+    // 128 heads (measured: 32 rows 4 splits 32.3, 16 rows 8 splits 24.2, 4 rows 16 splits 18.8, 1 row 32 splits 13.5, against
+    // 35.0, 28.6, 20.0 and 14.1 as four groups and one group of 32 heads; 36 to 64 rows alike; 128 rows 97.1 against 95.0).
+    if (a->nq > 32 && a->num_splits == 0 && min_split == 1) {
+        const int sh = shares(2);
+        if (pl.head_groups == 2) best = -1.0;             // (two groups of 32 heads: that is this form, at another price)
+        auto slice_round_us = [&](const int s) {
+            const int len = (tiles + s - 1) / s;
+            return s == 1 ? 1.4 * len : (0.59 + 0.0175 * len) * len;
+        };
+        auto slice_tail_us = [&](const long long r, const int s) {
+            const double wgs = (double)(r * sh * s);
+            return s == 1 ? 6.0 : 13.2 + (s > 8 ? 0.056 * wgs - 3.5 : 0.02 * wgs);
+        };
+        auto take = [&](const double cost, const int s, const long long whole) {
+            if (best >= 0.0 && cost >= best) return;
+            best = cost;
+            pl.nsplit = s;
+            pl.head_groups = 2;
+            pl.hgroups = sh;
+            pl.whole_slots = (int)(whole / 8);
+            pl.part_f32 = false;
+            split_rows = rows - whole;
+        };
+        for (int s = 1, len = 0; s <= (f32 ? 1 : tiles); s = len > 1 ? (tiles + len - 2) / (len - 1) : tiles + 1) {
+            len = (tiles + s - 1) / s;
+            if (s > 1 && (partial_bytes(rows, s) > pl.scratch_bytes || rows * sh * s > 4ll * cus)) break;
+            const double n = (double)rounds(rows * sh * s);
+            take(n * slice_round_us(s) + (n - 1.0) * 7.0 + slice_tail_us(rows, s), s, 0);    // (a further round starts and ends too)
+        }
+        const long long per_round = cus / 8 / sh, full = per_round > 0 ? (rows + 7) / 8 / per_round : 0, rows_b = rows - 8 * full * per_round;
+        if (!f32 && cus % 8 == 0 && full >= 1 && rows_b >= 1) {            // full rounds of whole rows, the rows left over in pieces
+            int s = (int)(cus / (rows_b * sh));
+            s = s > tiles / 4 ? tiles / 4 : s;
+            while (s >= 2 && partial_bytes(rows_b, s) > pl.scratch_bytes) --s;
+            if (s >= 2) take((double)full * (slice_round_us(1) + 7.0) + slice_round_us(s) + slice_tail_us(rows_b, s), s, 8 * full * per_round);
+        }
+    }
+    pl.part_o_bytes = pl.part_ml_bytes = 0;
     if (pl.nsplit > 1) {
         pl.part_ml_bytes = (size_t)split_rows * pl.nsplit * a->nq * 2 * sizeof(float);
-        pl.part_o_bytes = partial_bytes(split_rows, pl.nsplit, f32) - pl.part_ml_bytes;
-    } else {
-        pl.part_o_bytes = pl.part_ml_bytes = 0;
+        pl.part_o_bytes = partial_bytes(split_rows, pl.nsplit, pl.part_f32) - pl.part_ml_bytes;
     }
     // A launch that selects every cache row many times over (a prefill chunk: thousands of query rows over a few
     // thousand keys) de-quantises the cache once into the workspace and attends over the bf16 rows -- the same
     // bits, since the kernel's bf16-cache form reads exactly what its int8 form converts to, without the per-tile
     // conversion (8 % at 4096 query rows over 4096 keys).  Only for caches that fit a modest workspace.
-    pl.predeq_offset = (pl.part_o_bytes + pl.part_ml_bytes + 255) / 256 * 256;
-    pl.predeq_bytes = 0;
     const size_t dq = (size_t)a->kv_rows * 512 * sizeof(uint16_t);
+    pl.predeq_offset = (pl.scratch_bytes + 255) / 256 * 256;
+    pl.predeq_bytes = 0;
     if (rows * a->topk >= 8 * a->kv_rows && dq <= SFA_PREDEQ_MAX_BYTES && pl.predeq_offset + dq <= max_bytes) pl.predeq_bytes = dq;
     return pl;
 }
 
-size_t sfa_ws_bytes(const SfaPlan &pl) { return pl.predeq_bytes ? pl.predeq_offset + pl.predeq_bytes : pl.part_o_bytes + pl.part_ml_bytes; }
+size_t sfa_ws_bytes(const SfaPlan &pl) { return pl.predeq_bytes ? pl.predeq_offset + pl.predeq_bytes : pl.scratch_bytes; }
 
 constexpr int PACKED_ROW_BYTES = 656;     // 512 int8 | 64 bf16 | 4 fp32
 
@@ -294,7 +335,7 @@ int sfa_enqueue(const PtoSfaQuantArgs *a, const int8_t *kn, int kn_pitch, const 
                 return fail(PTO_E_INVALID_ARG, "sfa: index, block-table and length pointers must be 4-byte aligned");
     }
     const bool predeq = pl.predeq_bytes != 0 && !kn_bf16;
-    const size_t need = predeq ? sfa_ws_bytes(pl) : pl.part_o_bytes + pl.part_ml_bytes;
+    const size_t need = predeq ? sfa_ws_bytes(pl) : pl.scratch_bytes;
     if (need > 0 && (!a->workspace || a->workspace_bytes < need))
         return fail(PTO_E_WORKSPACE, "sfa: workspace of %zu bytes required, %zu given", need, a->workspace ? a->workspace_bytes : (size_t)0);
     if (predeq) {

@@ -9,8 +9,8 @@
 // un-normalised, PV accumulates in fp32 over 512 dims and the result is divided by the fp32 row sum.
 //
 // Work decomposition: one workgroup of four waves = (query row, 32*HG heads, key split).  With HG = 4 each
-// wave owns 32 heads for both matrix products, so probabilities never leave registers (HG = 1 and 2: see the
-// kernel):
+// wave owns 32 heads for both matrix products, so probabilities never leave registers (HG = 1: see the
+// kernel; 64 heads and eight waves: sfa_slice.h):
 //   S^T[key][head] = K[key][:] . Q^T        v_mfma_f32_32x32x16_bf16, A = K tile rows from LDS,
 //                                            B = Q^T fragments resident in registers
 //   O^T[dv][head] += V^T[dv][key] . P^T     A = V^T read from the same LDS tile with the
@@ -152,16 +152,16 @@ constexpr int PT_POOL = PT_ALPHA + 2 * PT_ALPHA_BYTES;
 
 // QUANT: the latent part of a cache row is int8 with four fp32 scales and is de-quantised on the way into
 // LDS; otherwise it is bf16 already (1024 bytes) and travels cache -> LDS tile directly by LDS-DMA.
-// HG: groups of 32 heads in the workgroup, which always has four waves.  With HG = 4 a wave owns its 32 heads.  With fewer
-// groups the SP = 4 / HG waves ("parts") of a group share it: part q takes an SP-th of the score contraction and of the
-// value channels, the partial scores meet in LDS (one more barrier per tile) and every part does the softmax of the
-// group's heads for itself, on the same bits.  Bound by a wave's instruction stream (de-quantisation, LDS accesses), not
-// by the matrix cores: a tile takes 1.47 us with HG = 1, 1.58 with 2, 1.75 with 4.  (One wave per 32 heads and so one or
-// two waves per compute unit, as before: 40 rows x 64 heads over a bf16 cache 41.7 us, now 34.8; 4 rows x 16 heads over
-// 8 K keys 41.8, now 24.0.)
+// HG: groups of 32 heads in the workgroup, 1 or 4, which always has four waves (two groups: sfa_slice.h).  With HG = 4 a wave
+// owns its 32 heads.  With HG = 1 the SP = 4 waves ("parts") share the group: part q takes a quarter of the score contraction
+// and of the value channels, the partial scores meet in LDS (one more barrier per tile) and every part does the softmax of
+// the group's heads for itself, on the same bits.  Bound by a wave's instruction stream (de-quantisation, LDS accesses),
+// not by the matrix cores: a tile takes 1.47 us with HG = 1, 1.75 with 4.  (One wave per 32 heads and so one or two waves per
+// compute unit, as before: 4 rows x 16 heads over 8 K keys 41.8 us, now 24.0.)
 template <int HG, bool QUANT>
 __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
 {
+    static_assert(HG == 1 || HG == 4, "two groups of heads: sfa_slice_kernel");
     constexpr int NW = 4;
     constexpr int SP = NW / HG;
     constexpr int KSP = KSTEPS / SP;                                   // contraction steps of a part
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
     // conflict-free.  The cache address is a wave-uniform base plus a per-lane offset.  Heads past NQ
     // read the last head and are never stored.  The second pass stays in flight while the row table
     // below is built.
-    // (HG < 4: a wave holds a half or a quarter of its heads' fragments only, 18 or 9 loads straight from memory.)
+    // (HG = 1: a wave holds a quarter of its heads' fragments only, nine loads straight from memory.)
     bf16x8 qf[KSP];
     uint8_t *const qreg = reinterpret_cast<uint8_t *>(pool) + w * QREGION;
     const uint32_t qdst = (uint32_t)(uintptr_t)(lds_byte_t *)qreg;
@@ -736,7 +736,7 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
         }
         s_chain_done(s);
         if constexpr (SP > 1) {
-            // the parts' scores meet: own + neighbour's (+ the other pair's sum), the same bits in every part
+            // the parts' scores meet: own + neighbour's + the other pair's sum, the same bits in every part
             uint8_t *const xch = pool_b + XCH_BASE + 16 * l;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -748,14 +748,9 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const f32x4 a = theirs(part ^ 1, j);
-                f32x4 b = {0.f, 0.f, 0.f, 0.f};
-                if (SP == 4) {
-                    const f32x4 c = theirs(part ^ 2, j), d = theirs(part ^ 3, j);
+                const f32x4 c = theirs(part ^ 2, j), d = theirs(part ^ 3, j);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) b[e] = c[e] + d[e];
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) s[4 * j + e] = SP == 4 ? (s[4 * j + e] + a[e]) + b[e] : s[4 * j + e] + a[e];
+                for (int e = 0; e < 4; ++e) s[4 * j + e] = (s[4 * j + e] + a[e]) + (c[e] + d[e]);
             }
         }
 
@@ -1149,6 +1144,8 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
     }
 }
 
+#include "sfa_slice.h"
+
 // Merges the key splits of one query row: out = sum_s w_s O_s / sum_s w_s with w_s = l_s 2^(m_s - m)
 // and O_s the split's normalised partial, fp16 or fp32 (all zeros for an empty split, whose weight is zero).
 // One wave per (row, head), a lane per 8 value channels.  The (max, sum) pairs of a (row, head) are the
@@ -1302,14 +1299,16 @@ hipError_t sfa_launch(const SfaParams &pa, hipStream_t stream)
     p.xcd_pieces = (int)(((long long)split_rows * p.hgroups * p.nsplit + 7) / 8);
     const unsigned grid = (unsigned)(8 * (p.hgroups * p.whole_slots + p.xcd_pieces));
     if (p.part_f32 && (p.head_groups > 1 || p.nsplit > 8)) return hipErrorInvalidValue;
-#define SFA_LAUNCH(Q)                                                                                                       \
-    switch (p.head_groups) {                                                                                                \
-    case 1: hipLaunchKernelGGL((sfa_decode_kernel<1, Q>), dim3(grid), dim3(256), 0, stream, p); break;                      \
-    case 2: hipLaunchKernelGGL((sfa_decode_kernel<2, Q>), dim3(grid), dim3(256), 0, stream, p); break;                      \
-    default: hipLaunchKernelGGL((sfa_decode_kernel<4, Q>), dim3(grid), dim3(256), 0, stream, p); break;                     \
+    if (p.head_groups == 4) {
+        if (p.kn_bf16) hipLaunchKernelGGL((sfa_decode_kernel<4, false>), dim3(grid), dim3(256), 0, stream, p);
+        else hipLaunchKernelGGL((sfa_decode_kernel<4, true>), dim3(grid), dim3(256), 0, stream, p);
+    } else if (p.head_groups == 2) {
+        if (p.kn_bf16) hipLaunchKernelGGL((sfa_slice_kernel<false>), dim3(grid), dim3(512), 0, stream, p);
+        else hipLaunchKernelGGL((sfa_slice_kernel<true>), dim3(grid), dim3(512), 0, stream, p);
+    } else {
+        if (p.kn_bf16) hipLaunchKernelGGL((sfa_decode_kernel<1, false>), dim3(grid), dim3(256), 0, stream, p);
+        else hipLaunchKernelGGL((sfa_decode_kernel<1, true>), dim3(grid), dim3(256), 0, stream, p);
     }
-    if (p.kn_bf16) { SFA_LAUNCH(false) } else { SFA_LAUNCH(true) }
-#undef SFA_LAUNCH
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (p.nsplit > 1 && p.T > 8 * p.whole_slots) {
