@@ -89,6 +89,26 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v)
     return v;
 }
 
+// the same within each row of sixteen lanes, and the minimum and maximum of a row in all of its lanes
+__device__ __forceinline__ uint32_t row_incl_scan(uint32_t v)
+{
+    v += dpp_u32<0x111, 0xf>(0u, v);
+    v += dpp_u32<0x112, 0xf>(0u, v);
+    v += dpp_u32<0x114, 0xf>(0u, v);
+    v += dpp_u32<0x118, 0xf>(0u, v);
+    return v;
+}
+
+template <typename Op>
+__device__ __forceinline__ float row_reduce(float v, Op op)
+{
+    v = op(v, __uint_as_float(dpp_u32<0x128, 0xf>(0u, __float_as_uint(v))));     // row_ror: 8, 4, 2, 1
+    v = op(v, __uint_as_float(dpp_u32<0x124, 0xf>(0u, __float_as_uint(v))));
+    v = op(v, __uint_as_float(dpp_u32<0x122, 0xf>(0u, __float_as_uint(v))));
+    v = op(v, __uint_as_float(dpp_u32<0x121, 0xf>(0u, __float_as_uint(v))));
+    return v;
+}
+
 template <typename Op>
 __device__ __forceinline__ uint32_t wave_reduce_bits(uint32_t v, const uint32_t identity, Op op)
 {
@@ -803,7 +823,7 @@ __device__ __forceinline__ float key_score(const uint32_t key)
 }
 
 constexpr int SEL_SBINS = 1024;    // bins of the sample histogram
-constexpr int SEL_BUCKETS = 2048;  // buckets the candidates are spread over
+constexpr int SEL_BUCKETS = 8192;  // buckets the candidates are spread over, eight per thread
 constexpr int SEL_WAVE_CAP = SEL_CAP / SEL_WAVES;   // candidates one wave can compact
 constexpr int SEL_CHUNK = 32 * SEL_THREADS;   // scores one trip of the row scan holds in registers
 
@@ -816,12 +836,16 @@ constexpr int SEL_CHUNK = 32 * SEL_THREADS;   // scores one trip of the row scan
 //      least k and at most SEL_CAP scores of the row lie at or above it;
 //   2. one pass over the row (32 scores per thread in flight at once, requested before the sample is
 //      looked at) compacts the keys at or above the pivot into a candidate list;
-//   3. the candidates are spread over 2048 buckets linear in the score between the pivot and the
+//   3. the candidates are spread over 8192 buckets linear in the score between the pivot and the
 //      sample maximum, bucket 0 highest: bins follow the values instead of the float encoding, so
 //      the counters see few collisions and buckets stay short whatever the scale of the scores;
 //   4. a prefix sum over the bucket counts finds the bucket holding the k-th best key; the buckets
 //      down to it are staged contiguously and each is ordered by counting (a key's rank = the number
 //      of larger keys of its bucket).  Output slots below k are written straight to memory.
+// A chain of short phases: what each costs is the latency of its loads or the vector work of sixteen waves on four SIMDs, so work
+// that every wave would do alike is done by one (the pivot), or by a row of lanes (sums over the waves), and buckets are many
+// and short.  Clocks at 32 K scores: sample and minimum 5.9 K, pivot 1.9, scan 3.7 (the row arrives at 14-20 bytes per clock),
+// candidates 2.5, offsets 2.2, staging 1.7, ranking 3.5; 24.1 -> 21.3 K in all (pivot 5.1, ranking 4.7 before).
 // If the pivot misjudges the row (fewer than k candidates, more than the list holds, or a bucket
 // range too long to stage) the general streaming select runs instead.
 __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p)
@@ -829,13 +853,13 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
     __shared__ uint32_t cand[SEL_CAP];                 // positions
     __shared__ unsigned long long stage[SEL_STAGE];    // also the sort buffer of the other paths
     __shared__ uint16_t sbucket[SEL_STAGE];            // bucket of every staged entry
-    __shared__ uint32_t bcount[SEL_BUCKETS];
-    __shared__ uint32_t boff[SEL_BUCKETS];
+    __shared__ __attribute__((aligned(16))) uint32_t boff[SEL_BUCKETS + 4];   // counts, then first slots, of the buckets
     __shared__ uint32_t shist[SEL_SBINS];
     __shared__ uint32_t hist[256];                     // streaming path only
-    __shared__ uint32_t wave_tot[SEL_WAVES];
+    __shared__ uint32_t wave_tot[SEL_WAVES], wave_sum[SEL_WAVES];
     __shared__ float wave_mn[SEL_WAVES], wave_mx[SEL_WAVES];
-    __shared__ uint32_t sh_over, sh_tb;
+    __shared__ uint32_t sh_over, sh_pb, sh_tb, sh_stage;
+    static_assert(SEL_BUCKETS == 8 * SEL_THREADS && SEL_WAVES == 16, "eight buckets per thread, a wave per lane of a row");
 
     const int t = blockIdx.x;
     const int b = t / p.S1;
@@ -906,9 +930,11 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
     };
     f32x4 v[8], vn[8];
     load_chunk(0, v);
+    const uint32_t r0 = ((uint32_t)k * S + (uint32_t)n - 1u) / (uint32_t)n;
+    const uint32_t r = r0 + (uint32_t)(6.0f * __builtin_sqrtf((float)r0)) + 8u;
 
     for (int i = tid; i < SEL_SBINS; i += SEL_THREADS) shist[i] = 0u;
-    for (int i = tid; i < SEL_BUCKETS; i += SEL_THREADS) bcount[i] = 0u;
+    for (int i = tid; i < SEL_BUCKETS / 4; i += SEL_THREADS) reinterpret_cast<u32x4 *>(boff)[i] = u32x4{0u, 0u, 0u, 0u};
     if (tid == 0) sh_over = 0u;
     {
         float mn = __builtin_inff(), mx = -__builtin_inff();
@@ -920,11 +946,8 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
         if (lane == 0) { wave_mn[wv] = mn; wave_mx[wv] = mx; }
     }
     __syncthreads();
-    float smin = wave_mn[0], smax = wave_mx[0];
-#pragma unroll
-    for (int i = 1; i < SEL_WAVES; ++i) { smin = fminf(smin, wave_mn[i]); smax = fmaxf(smax, wave_mx[i]); }
-    const uint32_t r0 = ((uint32_t)k * S + (uint32_t)n - 1u) / (uint32_t)n;
-    const uint32_t r = r0 + (uint32_t)(6.0f * __builtin_sqrtf((float)r0)) + 8u;
+    const float smin = row_reduce(wave_mn[lane & 15], [](float x, float y) { return fminf(x, y); });
+    const float smax = row_reduce(wave_mx[lane & 15], [](float x, float y) { return fmaxf(x, y); });
     float pivot = -__builtin_inff();       // candidates: score >= pivot
     float blo = smin;                      // lower edge of the lowest bucket
     if (r < S) {
@@ -938,28 +961,27 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
             }
         }
         __syncthreads();
-        // every wave scans the 1024 bins from the top by itself (lane l owns the 16 bins below
-        // 1024 - 16*l): the bin in which the running count reaches r
-        uint32_t c[16];
-        uint32_t tot = 0;
-        {
+        // one wave scans the 1024 bins from the top (lane l owns the 16 bins below 1024 - 16*l): the bin in which the running
+        // count reaches r.  (Every wave by itself, without the barrier: 2.2 thousand clocks of vector work instead of 0.9.)
+        if (wv == 0) {
             const u32x4 *src = reinterpret_cast<const u32x4 *>(&shist[SEL_SBINS - 16 - 16 * lane]);
+            uint32_t tot = 0;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const u32x4 x = src[q];
-                c[4 * q] = x[0]; c[4 * q + 1] = x[1]; c[4 * q + 2] = x[2]; c[4 * q + 3] = x[3];
+                tot += (x[0] + x[1]) + (x[2] + x[3]);
             }
-#pragma unroll
-            for (int q = 0; q < 16; ++q) tot += c[q];
+            const uint32_t before = wave_incl_scan(tot) - tot;
+            // (found by exactly one lane: the sample holds S >= r scores); then the bin among its sixteen, a lane each
+            const int at = __ffsll((long long)__ballot(before < r && r <= before + tot)) - 1;
+            const uint32_t top = (uint32_t)(SEL_SBINS - 1 - 16 * at);
+            const uint32_t cnt = shist[top - (uint32_t)(lane & 15)];
+            const uint32_t incl = (uint32_t)__builtin_amdgcn_readlane((int)before, at) + row_incl_scan(cnt);
+            const int in = __ffsll((long long)__ballot(incl - cnt < r && r <= incl)) - 1;
+            if (lane == 0) sh_pb = top - (uint32_t)in;
         }
-        uint32_t before = wave_incl_scan(tot) - tot;
-        uint32_t pb = 0;                   // found by exactly one lane (the sample holds S >= r scores)
-#pragma unroll
-        for (int q = 15; q >= 0; --q) {
-            if (before < r && r <= before + c[q]) pb = (uint32_t)(SEL_SBINS - 16 - 16 * lane + q);
-            before += c[q];
-        }
-        pb = wave_max_u32(pb);
+        __syncthreads();
+        const uint32_t pb = sh_pb;
         pivot = smin + (float)pb * (range * (1.0f / (float)SEL_SBINS));
         blo = pivot;
     }
@@ -1020,55 +1042,64 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
     for (int u = 0; u < CPT; ++u) {
         const uint32_t j = (uint32_t)(u * 64 + lane);
         cpos[u] = j < wave_count ? cand[wv * SEL_WAVE_CAP + j] : 0u;
-        csc[u] = srow[cpos[u]];
+        csc[u] = (uint32_t)(u * 64) < wave_count ? srow[cpos[u]] : 0.f;             // (uniform: trips past the last are left out)
     }
-#pragma unroll
-    for (int u = 0; u < CPT; ++u) ce[u] = (uint32_t)(u * 64 + lane) < wave_count ? order_word(csc[u], cpos[u]) : 0ull;
 #pragma unroll
     for (int u = 0; u < CPT; ++u) {
-        const uint32_t lin = (uint32_t)fmaxf((key_score((uint32_t)(ce[u] >> 32)) - blo) * bscale, 0.f);
-        cb[u] = (uint32_t)SEL_BUCKETS - 1u - (lin < (uint32_t)SEL_BUCKETS ? lin : (uint32_t)SEL_BUCKETS - 1u);
+        ce[u] = 0ull;
+        cb[u] = (uint32_t)SEL_BUCKETS;                                              // none
         cslot[u] = 0u;
-        if ((uint32_t)(u * 64 + lane) < wave_count) cslot[u] = atomicAdd(&bcount[cb[u]], 1u);
+        if ((uint32_t)(u * 64 + lane) < wave_count) {
+            ce[u] = order_word(csc[u], cpos[u]);
+            const uint32_t lin = (uint32_t)fmaxf((key_score((uint32_t)(ce[u] >> 32)) - blo) * bscale, 0.f);
+            cb[u] = (uint32_t)SEL_BUCKETS - 1u - (lin < (uint32_t)SEL_BUCKETS ? lin : (uint32_t)SEL_BUCKETS - 1u);
+            cslot[u] = atomicAdd(&boff[cb[u]], 1u);
+        }
     }
     __syncthreads();
-    uint32_t n_cand = 0;
-#pragma unroll
-    for (int i = 0; i < SEL_WAVES; ++i) n_cand += wave_tot[i];
+    const uint32_t n_cand = (uint32_t)__builtin_amdgcn_readlane((int)row_incl_scan(wave_tot[lane & 15]), 15);
     if (sh_over != 0u || n_cand < (uint32_t)k) {
-        __syncthreads();                                         // wave_tot is reused below
         select_streaming(p, t, hist, stage);                     // uniform: the whole workgroup goes
         return;
     }
 
-    // ---- 4. bucket offsets (two buckets per thread) and the bucket holding the k-th best key
+    // ---- 4. bucket offsets (eight buckets per thread) and the bucket holding the k-th best key
     {
-        const uint32_t b0 = 2u * (uint32_t)tid;
-        const uint32_t c0 = bcount[b0], c1 = bcount[b0 + 1u];
-        const uint32_t tot = c0 + c1;
+        u32x4 *const mine = reinterpret_cast<u32x4 *>(boff) + 2 * tid;
+        u32x4 c[2];
+        c[0] = mine[0];
+        c[1] = mine[1];
+        const uint32_t tot = ((c[0][0] + c[0][1]) + (c[0][2] + c[0][3])) + ((c[1][0] + c[1][1]) + (c[1][2] + c[1][3]));
         const uint32_t incl = wave_incl_scan(tot);
-        __syncthreads();                                         // every wave has read the candidate counts
-        if (lane == 63) wave_tot[wv] = incl;
+        if (lane == 63) wave_sum[wv] = incl;
         __syncthreads();
-        uint32_t before = incl - tot;
+        const uint32_t of_wave = wave_sum[lane & 15];
+        uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)(row_incl_scan(of_wave) - of_wave), wv) + incl - tot;
+        const bool here = before < (uint32_t)k && (uint32_t)k <= before + tot;
 #pragma unroll
-        for (int i = 0; i < SEL_WAVES; ++i) before += i < wv ? wave_tot[i] : 0u;
-        boff[b0] = before;
-        boff[b0 + 1u] = before + c0;
-        if (before < (uint32_t)k && (uint32_t)k <= before + c0) sh_tb = b0;
-        else if (before + c0 < (uint32_t)k && (uint32_t)k <= before + tot) sh_tb = b0 + 1u;
+        for (int e = 0; e < 8; ++e) {
+            const uint32_t cnt = c[e >> 2][e & 3];
+            c[e >> 2][e & 3] = before;
+            if (here && before < (uint32_t)k && (uint32_t)k <= before + cnt) {
+                sh_tb = (uint32_t)(8 * tid + e);
+                sh_stage = before + cnt;
+            }
+            before += cnt;
+        }
+        mine[0] = c[0];
+        mine[1] = c[1];
+        if (tid == SEL_THREADS - 1) boff[SEL_BUCKETS] = before;
     }
     __syncthreads();
     const uint32_t tb = sh_tb;
-    const uint32_t n_stage = boff[tb] + bcount[tb];
+    const uint32_t n_stage = sh_stage;
     if (n_stage > (uint32_t)SEL_STAGE) {
-        __syncthreads();
         select_streaming(p, t, hist, stage);
         return;
     }
 #pragma unroll
     for (int u = 0; u < CPT; ++u) {
-        if ((uint32_t)(u * 64 + lane) < wave_count && cb[u] <= tb) {
+        if (cb[u] <= tb) {
             const uint32_t idx = boff[cb[u]] + cslot[u];
             stage[idx] = ce[u];
             sbucket[idx] = (uint16_t)cb[u];
@@ -1092,7 +1123,7 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
             e[q] = stage[ok ? i : 0u];
             const uint32_t bk = sbucket[ok ? i : 0u];
             beg[q] = boff[bk];
-            len[q] = ok ? bcount[bk] : 0u;
+            len[q] = ok ? boff[bk + 1u] - beg[q] : 0u;
             rank[q] = 0u;
             maxlen = len[q] > maxlen ? len[q] : maxlen;
         }

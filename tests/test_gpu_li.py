@@ -227,3 +227,18 @@ def test_fp16_dequant_variant_refuses_other_dtypes():
         pypto_amd.lightning_indexer_decode(*inp.operator_tensors(), None, None, 64, arith_variant="fp16_dequant")
     with pytest.raises(ValueError):
         pypto_amd.lightning_indexer_decode(*inp.operator_tensors(), None, None, 64, arith_variant="other")
+
+
+@pytest.mark.parametrize("k,act", [
+    (1, [1023, 1024, 1040, 2047]),               # 63 full groups of the sample (the general way), 64, 65, 127
+    (64, [65, 1025, 16383, 16385]),
+    (2047, [2048, 2049, 2064, 8193]),
+    (2048, [2049, 32767, 32769, 65537]),         # chunks of the row scan: one short of full, one key into the next
+])
+def test_row_lengths_of_the_select(c_oracle, k, act):
+    """Lengths at the edges of the sample, of the scan's chunks and of the selection itself; scores of both signs, many equal."""
+    inp = gen_indexer_inputs(len(act), 1, act, selected_count=k, seed=k, variant="fp16")
+    inp.idx_weight[1] = inp.idx_weight[1].sign() * 0.25
+    inp.idx_query[1] = inp.idx_query[1].sign()
+    inp.idx_key_cache[::3] = inp.idx_key_cache[0]
+    assert_exact(run_op(inp), oracle(inp, c_oracle), f"k={k} act={act}")
