@@ -229,7 +229,9 @@ constexpr int SC_BUF_BYTES = SC_PAIR_BYTES + 256;   // + the 64 key scales (one 
 //          global_load_lds: consecutive lanes fetch consecutive 16-byte chunks, so every request is a
 //          run of whole cache lines (loading the operand layout directly touches 32 lines with 32
 //          bytes each per instruction and is bound by the address unit).  Chunk c of row r lands at
-//          position c ^ (r & 7) of the row, which makes the operand reads below conflict-free.  The
+//          position c ^ ((r >> 1) & 7) of the row: the LDS serves sixteen lanes of an operand read at a time, two
+//          rows of 128 bytes span its banks, so any sixteen rows meet every bank once (with c ^ (r & 7) rows
+//          eight apart met in the same banks and every read took twice as long).  The
 //          pair after the current one is in flight while the current one is scored.
 //   MFMA   A = the token's 64 query heads as two 32-row operands (resident in registers), B = 32 key
 //          rows read from LDS in operand layout; four accumulators per trip.  With the head
@@ -335,13 +337,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
         run_row = pb * p.bs + (pos0 - page * p.bs);
     }
     // Requests pair pr into buffer buf: per block four instructions of eight rows each.  Lane l owns
-    // LDS slot l of an instruction's 1 KiB, i.e. row l/8 and position l%8, and fetches chunk
-    // (l%8) ^ (l/8) of that row; the instruction offset moves the cache address and the LDS address
+    // LDS slot l of an instruction's 1 KiB, i.e. row l/8 (of eight) and position l%8, and fetches chunk
+    // (l%8) ^ (row/2 % 8) of that row; the instruction offset moves the cache address and the LDS address
     // alike.  A ninth instruction stages the dword holding the scale of the key whose sum this lane
     // will hold (X_j on the lower half-wave, Y_j on the upper).  Every load of the loop is written as
     // assembly: the compiler then tracks none of them, and the explicit waits of the trips decide
     // alone how long requests stay outstanding (two pairs ahead).
-    const uint32_t lane_off = (uint32_t)((l >> 3) * LI_DIM + (((l & 7) ^ (l >> 3)) << 4));
+    const uint32_t lane_off = (uint32_t)((l >> 3) * LI_DIM + (((l & 7) ^ (l >> 4)) << 4));
+    const uint32_t lane_off4 = lane_off ^ 64u;       // rows 8..15 and 24..31
     const uint32_t lds_base = (uint32_t)__builtin_amdgcn_readfirstlane(
         (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) int8_t *)&kstage[w][0][0]);
     constexpr int KSZ = KDT == PTO_DT_FP32 ? 4 : 2;
@@ -350,20 +353,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
         const int8_t *gx = p.kcache + (size_t)rx * LI_DIM;
         const int8_t *gy = p.kcache + (size_t)ry * LI_DIM;
         const uint32_t dst = lds_base + (uint32_t)(buf * SC_BUF_BYTES);
-        asm volatile("s_mov_b32 m0, %2\n\t"
+        asm volatile("s_mov_b32 m0, %3\n\t"
                      "s_nop 0\n\t"
-                     "global_load_lds_dwordx4 %0, %1\n\t"
-                     "global_load_lds_dwordx4 %0, %1 offset:1024\n\t"
-                     "global_load_lds_dwordx4 %0, %1 offset:2048\n\t"
-                     "global_load_lds_dwordx4 %0, %1 offset:3072"
-                     :: "v"(lane_off), "s"(gx), "s"(dst) : "memory", "m0");
-        asm volatile("s_mov_b32 m0, %2\n\t"
+                     "global_load_lds_dwordx4 %0, %2\n\t"
+                     "global_load_lds_dwordx4 %1, %2 offset:1024\n\t"
+                     "global_load_lds_dwordx4 %0, %2 offset:2048\n\t"
+                     "global_load_lds_dwordx4 %1, %2 offset:3072"
+                     :: "v"(lane_off), "v"(lane_off4), "s"(gx), "s"(dst) : "memory", "m0");
+        asm volatile("s_mov_b32 m0, %3\n\t"
                      "s_nop 0\n\t"
-                     "global_load_lds_dwordx4 %0, %1\n\t"
-                     "global_load_lds_dwordx4 %0, %1 offset:1024\n\t"
-                     "global_load_lds_dwordx4 %0, %1 offset:2048\n\t"
-                     "global_load_lds_dwordx4 %0, %1 offset:3072"
-                     :: "v"(lane_off), "s"(gy), "s"(dst + 4096u) : "memory", "m0");
+                     "global_load_lds_dwordx4 %0, %2\n\t"
+                     "global_load_lds_dwordx4 %1, %2 offset:1024\n\t"
+                     "global_load_lds_dwordx4 %0, %2 offset:2048\n\t"
+                     "global_load_lds_dwordx4 %1, %2 offset:3072"
+                     :: "v"(lane_off), "v"(lane_off4), "s"(gy), "s"(dst + 4096u) : "memory", "m0");
         // the aligned dword that holds this lane's scale
         const uintptr_t sa = (reinterpret_cast<uintptr_t>(p.k_scale) + ((size_t)(half ? ry : rx) + j) * KSZ) & ~(uintptr_t)3;
         asm volatile("s_mov_b32 m0, %1\n\t"
@@ -430,7 +433,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
     // this lane's operand chunks of row j inside a staged block
     int koff[4];
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) koff[ks] = j * LI_DIM + (((4 * half + ks) ^ (j & 7)) << 4);
+    for (int ks = 0; ks < 4; ++ks) koff[ks] = j * LI_DIM + (((4 * half + ks) ^ ((j >> 1) & 7)) << 4);
 
     // One trip.  Requests and stores complete in the order they were made.  Behind this trip's pair there are the nine
     // requests of the following pair and the two stores per token (scores, sample) of each of the last two trips -- every
