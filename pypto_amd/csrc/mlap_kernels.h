@@ -18,9 +18,8 @@ constexpr int MLAP_XTOK = 8;         // tokens per job of the first and of the l
 constexpr int MLAP_MFMA_MIN_TOKENS = 9;    // from here on the first launch sums on the matrix cores unless absorb_exact (the fixed-order
                                            // form works on 8 tokens at a time and its cost grows with every 8 tokens)
 constexpr int MLAP_UNSPLIT_MIN_TOKENS = 64;   // with absorb_exact the projection still runs unsplit from here on
-// ranges of the hidden axis (partial sums per token) of that form, at most.  With a single token tile the sixteen
-// matrix-core slabs x 14 ranges and the rope columns' 32 workgroups are one workgroup per compute unit of an
-// MI355X, every one requesting weights from the start (8 ranges: 32 tokens 44.6 us per pass, 14: 40.9, 20 or 28: 43.3)
+// ranges of the hidden axis (partial sums per token) of the matrix-core form, at most (what a launch takes: mlap_launch_front);
+// the workspace is sized for it
 constexpr int MLAP_XM_MAX_SPLITS = 14;
 
 // rows [T, q_lora + 576] of partial sums over the hidden axis the workspace holds: the group sums of the

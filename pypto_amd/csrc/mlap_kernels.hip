@@ -503,29 +503,31 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
     if (lip_rider != nullptr) lip = *lip_rider;
     const MlapRider rd = rider != nullptr ? *rider : MlapRider{nullptr, nullptr, nullptr, nullptr, nullptr, 0};
     if (mlap_prefill_forms(p)) {
-        // prefill sizes: the sums over the hidden axis on the matrix cores, in as many ranges of the hidden axis
-        // (partial sums per token) as give about two workgroups per compute unit, MLAP_XM_MAX_SPLITS at most
+        // prefill sizes: the sums over the hidden axis on the matrix cores, in ranges of the hidden axis (partial sums per token)
         const int nchunks = p.h / XM_KC;
         const int ttiles = (p.T + XM_TOK - 1) / XM_TOK;
         const int cus = cu_count();
         if (cus <= 0) return hipErrorNoDevice;
-        ngroups = 2 * cus / (nslabs * ttiles);
-        ngroups = ngroups < 1 ? 1 : ngroups;
-        ngroups = ngroups > MLAP_XM_MAX_SPLITS ? MLAP_XM_MAX_SPLITS : ngroups;
         // every slab but the last, the rope columns, which keep their fixed-order sums
         const int mslabs = nslabs - 1;
-        ngroups = ngroups > nchunks ? nchunks : ngroups;
         const bool big = p.T > XM_TOK;       // 130 tokens: 60.9 us per pass, 66.7 with tiles of 128; 1500: 282 and 293; 4096: 700 and 724
-        if (big) {
-            // one workgroup per compute unit (the other half of each is for the fixed-order sums)
-            const int tiles = mslabs * ((p.T + XB_TOK - 1) / XB_TOK);
-            ngroups = cus / tiles;
-            ngroups = ngroups < 1 ? 1 : ngroups;
-            ngroups = ngroups > MLAP_XM_MAX_SPLITS ? MLAP_XM_MAX_SPLITS : ngroups;
-            ngroups = ngroups > nchunks ? nchunks : ngroups;
-        }
+        // As many ranges as make this many workgroups, in eighths of the compute units: the rest of the chip is for the
+        // fixed-order sums, and what does not fit beside them runs as a second round, nearly empty and as long as the first.
+        // Up to 64 tokens a compute unit holds one workgroup, and more ranges are more partial sums to write and read as well
+        // (fused prolog, 14 ranges and as it is: 9 tokens 38.9 and 33.6, 32: 42.4 and 37.0, 48: 47.3 and 42.4, 64: 52.9 and
+        // 45.2; MLA prolog alone, 32: 34.2 and 31.5).  128 tokens: 14 ranges 58.1, 12: 57.7 (alone, 100: 53.5 and 50.7); in
+        // tiles of 256 tokens, 192: 14 ranges 72.9, 12: 68.9; 256: 14 ranges 77.8, 10: 72.2 (alone 61.7 and 62.6); 400: 8 ranges
+        // 106.5, 6: 101.6, but alone, which has the same ranges to give the same bits, 77.2 and 80.7.
+        const int xtiles = big ? (p.T + XB_TOK - 1) / XB_TOK : ttiles;
+        int eighths = 8;
+        if (p.T <= 64) eighths = 4;
+        else if (xtiles == 1) eighths = p.T <= 192 ? 6 : 5;
+        ngroups = eighths * cus / (8 * mslabs * xtiles);
+        ngroups = ngroups < 1 ? 1 : ngroups;
+        ngroups = ngroups > MLAP_XM_MAX_SPLITS ? MLAP_XM_MAX_SPLITS : ngroups;
+        ngroups = ngroups > nchunks ? nchunks : ngroups;
         const int per_slab = ngroups * ttiles;
-        const int wgs = big ? 8 * ((mslabs * ((p.T + XB_TOK - 1) / XB_TOK) * ngroups + 7) / 8) : 8 * ((mslabs >> 3) * per_slab + ((mslabs & 7) * per_slab + 7) / 8);   // the kernel's XCD-wise job order
+        const int wgs = big ? 8 * ((mslabs * xtiles * ngroups + 7) / 8) : 8 * ((mslabs >> 3) * per_slab + ((mslabs & 7) * per_slab + 7) / 8);   // the kernel's XCD-wise job order
         const int sets = 1 + (lip_rider != nullptr ? LIP_XF_SETS : 0);
         const dim3 g((unsigned)(wgs + xf_jobs(sets, ngroups_fixed, p.T)));
 #define XM_LAUNCH(TBV) hipLaunchKernelGGL(mlap_xlinear_mfma_kernel<TBV>, g, dim3(256), 0, stream, p, mslabs, ngroups, wgs, sets, ngroups_fixed, lip)

@@ -173,6 +173,19 @@ def test_mla_prolog_prefill_t512_matrix_core_sums_default():
         print(f"t={b * s1}: q_norm entries off by one {float((dq != 0).mean()):.5f}, latent entries off by one {float((gk != rk).mean()):.5f}", flush=True)
 
 
+@pytest.mark.parametrize("t", [9, 32, 33, 64, 65, 128, 129, 192, 193, 256, 257])
+def test_mla_prolog_matrix_core_sums_at_the_edges_of_the_range_counts(t):
+    """The hidden axis is divided into as many ranges as the token count asks for: both sides of every line, at the model's
+    hidden size and query rank, against the launches that keep every sum in its fixed order."""
+    from pypto_amd import mla_prolog_quant_impl as impl
+    inp = gen_mla_prolog_inputs(1, t, [t], seed=t, n_heads=2)
+    ref = run_op(inp, (1e-5, 1e-5), prefill=True)
+    impl.EXACT_ABSORB = False
+    got = run_op(inp, (1e-5, 1e-5), prefill=True)
+    assert_reference_rule(got, ref, inp.cache_index.numpy(), f"t={t}")
+    assert np.array_equal(got["kr_cache"].view(np.uint32), ref["kr_cache"].view(np.uint32))
+
+
 def test_mla_prolog_separate_cache_output_skipped_indices_and_repeatability():
     inp = gen_mla_prolog_inputs(2, 2, [300, 129], seed=5, h=256, q_lora_rank=512, n_heads=4)
     inp.cache_index[1] = -1
