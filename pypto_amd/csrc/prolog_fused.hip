@@ -43,19 +43,22 @@ __global__ __launch_bounds__(64 * FIN_WAVES) void prolog_fused_finish_kernel(con
 }
 
 // Projections and last stages at prefill sizes (prolog_prefill.h): [0, mla_wgs) the attention query, then lip_wgs of the
-// indexer query, then the indexer's key rows and weights, a token per wave.  64 * TB tokens per workgroup of a head.
+// indexer query, then the indexer's key rows and weights, a token per wave.  64 * TB tokens per workgroup of a head of the
+// attention query, 128 * LTB of the indexer's.
 // FIXED: the indexer query's Hadamard sums in their fixed order (fewer than LIP_MFMA_MIN_TOKENS tokens).
-template <int XC, int TB> constexpr int PF_LDS2 = PFA_LDS<XC, TB> > PFI_LDS<XC, TB / 2> ? PFA_LDS<XC, TB> : PFI_LDS<XC, TB / 2>;
-template <int XC, int TB> constexpr int PF_LDS = PF_LDS2<XC, TB> > LIP_FINT_LDS ? PF_LDS2<XC, TB> : LIP_FINT_LDS;
-template <int XC, int TB, bool FIXED>
+constexpr int pf_xc(const int ltb) { return ltb == 1 ? 2 : 1; }
+template <int XC, int TB, int LTB>
+constexpr int PF_LDS2 = PFA_LDS<XC, TB> > PFI_LDS<pf_xc(LTB), LTB> ? PFA_LDS<XC, TB> : PFI_LDS<pf_xc(LTB), LTB>;
+template <int XC, int TB, int LTB> constexpr int PF_LDS = PF_LDS2<XC, TB, LTB> > LIP_FINT_LDS ? PF_LDS2<XC, TB, LTB> : LIP_FINT_LDS;
+template <int XC, int TB, int LTB, bool FIXED>
 __global__ __launch_bounds__(256, 2) void prolog_prefill_kernel(const MlapParams pm, const LipParams pl, const int mla_wgs, const int lip_wgs)
 {
-    static_assert(2 * PF_LDS<XC, TB> <= 160 * 1024, "two workgroups share a compute unit");
+    static_assert(2 * PF_LDS<XC, TB, LTB> <= 160 * 1024, "two workgroups share a compute unit");
     static_assert(FINT_WAVES == 4, "one block size for the three bodies");
-    __shared__ __attribute__((aligned(16))) uint8_t lds[PF_LDS<XC, TB>];
+    __shared__ __attribute__((aligned(16))) uint8_t lds[PF_LDS<XC, TB, LTB>];
     const int wg = (int)blockIdx.x;
     if (wg < mla_wgs) mlap_prefill_body<XC, TB>(pm, q_prefill_job_of(wg, mla_wgs), lds);
-    else if (wg < mla_wgs + lip_wgs) lip_prefill_body<XC, TB / 2, FIXED>(pl, q_prefill_job_of(wg - mla_wgs, lip_wgs), lds);
+    else if (wg < mla_wgs + lip_wgs) lip_prefill_body<pf_xc(LTB), LTB, FIXED>(pl, q_prefill_job_of(wg - mla_wgs, lip_wgs), lds);
     else lip_finish_tokens_prefill_body(pl, wg - mla_wgs - lip_wgs, lds);
 }
 
@@ -100,12 +103,19 @@ hipError_t prolog_prefill_launch(const MlapParams *pm, const LipParams *pl, hipS
     const int tok = small ? 128 : 256;
     const int tiles = (T + tok - 1) / tok;
     const int mla_wgs = pm ? m.n_heads * tiles : 0;
-    const int lip_wgs = pl ? p.n_heads * tiles : 0;
+    // Tiles of 256 tokens leave few workgroups at the first sizes that take them: there the indexer's half, whose workgroups are
+    // the shorter ones, is cut into tiles of 128.  The fused prolog with 256-token and 128-token tiles of the indexer's half:
+    // 390 tokens 104.3 us per pass and 101.8, 512: 116.6 and 108.0, 700: 151.2 and 147.1, 1024: 192.9 and 194.3, 2000: 356.7 and
+    // 360.9; the indexer prolog alone 400: 45.3 and 36.4, 512: 46.2 and 37.5, 1536: 85.5 and 84.4, 2000: 107.0 and 110.3.
+    const bool lip_small = small || tiles <= (pm ? 3 : 6);
+    const int lip_wgs = pl ? p.n_heads * (lip_small ? (T + 127) / 128 : tiles) : 0;
     const int tok_wgs = pl ? (T + FINT_WAVES - 1) / FINT_WAVES : 0;
     const dim3 g((unsigned)(mla_wgs + lip_wgs + tok_wgs));
-    if (T < LIP_MFMA_MIN_TOKENS) hipLaunchKernelGGL((prolog_prefill_kernel<2, 2, true>), g, dim3(256), 0, stream, m, p, mla_wgs, lip_wgs);
-    else if (small) hipLaunchKernelGGL((prolog_prefill_kernel<2, 2, false>), g, dim3(256), 0, stream, m, p, mla_wgs, lip_wgs);
-    else hipLaunchKernelGGL((prolog_prefill_kernel<1, 4, false>), g, dim3(256), 0, stream, m, p, mla_wgs, lip_wgs);
+    auto run = [&](auto *kernel) { hipLaunchKernelGGL(kernel, g, dim3(256), 0, stream, m, p, mla_wgs, lip_wgs); };
+    if (T < LIP_MFMA_MIN_TOKENS) run(prolog_prefill_kernel<2, 2, 1, true>);
+    else if (small) run(prolog_prefill_kernel<2, 2, 1, false>);
+    else if (lip_small) run(prolog_prefill_kernel<1, 4, 1, false>);
+    else run(prolog_prefill_kernel<1, 4, 2, false>);
     return hipGetLastError();
 }
 

@@ -311,6 +311,36 @@ def test_fused_prolog_query_rows_at_tile_edges(t, q_lora):
     assert (np.abs(q_scale.float().cpu().numpy()[..., 0] - want["q_scale"].astype(np.float32)) > 2.5e-5).mean() <= 0.005
 
 
+@pytest.mark.parametrize("t", [385, 511, 640, 768, 769, 1535, 1537])
+def test_indexer_query_rows_are_alike_in_tiles_of_128_and_256_tokens(t):
+    """The indexer query's tiles have 128 or 256 tokens by the number of tokens and by whether the attention query is made in the
+    same launch: the fused operator and the indexer prolog alone give the same bits at the edges of both rules, rows past the last
+    token stay as they are, and the rows meet the reference's rule."""
+    from oracle import lip_oracle as lo
+    from pypto_amd import lightning_indexer_prolog_quant_impl as lip_impl
+    from pypto_amd import mla_prolog_quant_impl as impl
+    from pypto_amd.synthetic import gen_indexer_prolog_inputs
+    impl.EXACT_ABSORB = lip_impl.EXACT_SUMS = False
+    kw = dict(h=128, q_lora_rank=512)
+    mla = gen_mla_prolog_inputs(1, t, [t + 30], seed=t, n_heads=2, **kw)
+    lip = gen_indexer_prolog_inputs(1, t, [t + 30], seed=t + 1, n_heads=8, **kw)
+    got = run_op(mla, (1e-5, 1e-5), prefill=True)
+    dm, dl = mla.to(torch.device("cuda:0")), lip.to(torch.device("cuda:0"))
+    _, _, q_int8, q_scale, weights = run_fused(dm, dl, t, 2, 8, op=pypto_amd.mla_indexer_prolog_quant_p)
+    lip.x, lip.cos_idx_rope, lip.sin_idx_rope, lip.k_cache_index = mla.token_x, mla.cos, mla.sin, mla.cache_index
+    lip.q_norm, lip.q_norm_scale = torch.from_numpy(got["q_norm"]), torch.from_numpy(got["q_norm_scale"]).reshape(-1, 1)
+    alone = [torch.full([t + 8] + list(v.shape[1:]), -7, dtype=v.dtype, device="cuda") for v in (q_int8, q_scale, weights)]
+    da = lip.to(torch.device("cuda:0"))
+    pypto_amd.lightning_indexer_prolog_quant(*da.input_tensors(), alone[0][:t], alone[1][:t], da.k_cache, da.k_cache_scale, alone[2][:t],
+                                             pypto_amd.IndexerPrologQuantAttr(eps=1e-6), pypto_amd.IndexerPrologQuantConfigs())
+    torch.cuda.synchronize()
+    for a, f in zip(alone, (q_int8, q_scale, weights)):
+        assert torch.equal(a[:t], f) and bool((a[t:] == -7).all())
+    want = lo.indexer_prolog_ref(*lip.input_tensors())
+    assert np.abs(q_int8.cpu().numpy().astype(np.int32) - want["q_int8"].astype(np.int32)).max() <= 1
+    assert (np.abs(q_scale.float().cpu().numpy()[..., 0] - want["q_scale"].astype(np.float32)) > 2.5e-5).mean() <= 0.005
+
+
 @pytest.mark.parametrize("t,n_idx,mode", [(8, 64, "default"), (9, 64, "default"), (16, 64, "default"), (31, 8, "default"),
                                           (32, 64, "default"), (33, 64, "default"), (33, 24, "default"), (63, 64, "default"),
                                           (9, 64, "exact"), (32, 64, "exact"), (63, 64, "exact"), (32, 64, "matrix_cores"),
