@@ -12,6 +12,7 @@ constexpr int MLAP_QHEAD = MLAP_NOPE + MLAP_ROPE;
 constexpr int MLAP_XBLOCK = 64;      // block length of the fixed-order sums over the hidden axis
 constexpr int MLAP_XGROUP = 8;       // block sums per group (one workgroup of the first kernel)
 constexpr int MLAP_MAX_XGROUPS = 32; // h <= 32 * 8 * 64 = 16384
+constexpr int MLAP_MIN_QLORA = 512;  // (512, 1024 or 1536)
 constexpr int MLAP_MAX_QLORA = 1536;
 constexpr int QPROJ_KSPLIT_HOST = 4; // partial sums of the int8 projection (prolog_common.h: QPROJ_KSPLIT)
 constexpr int MLAP_XTOK = 8;         // tokens per job of the first and of the last kernel
@@ -80,6 +81,13 @@ __host__ __device__ inline bool mlap_prefill_forms(const MlapParams &p) { return
 // unless every sum is to keep its fixed order the projection and the last stage are one launch (prolog_small.h up to
 // PROLOG_SMALL_TOKENS tokens, prolog_prefill.h beyond)
 constexpr int PROLOG_SMALL_TOKENS = 32;
+// Heads 2m and 2m + 1 are workgroups of the same XCD, eight apart: a head's rows of w_uq_qr are 192 bytes, a pair's three cache
+// lines, the middle one of which they share.  (With neighbours on different XCDs every such line crossed into two L2s, 81 MB
+// read for 67 MB of weights; fused prolog: 1 token 33.4 us per pass, now 32.5, 8 tokens 34.4 and 33.8, 16: 39.6 and 39.2.)
+__host__ __device__ inline int prolog_small_head(const int wg, const int n_heads)
+{
+    return (n_heads & 15) == 0 ? 2 * (8 * (wg >> 4) + (wg & 7)) + ((wg >> 3) & 1) : wg;
+}
 __host__ __device__ inline bool mlap_fused_projection(const MlapParams &p) { return !p.absorb_exact; }
 // partial sums per output the int8 projection leaves where it is a launch of its own (absorb_exact): 1 = unsplit (de-quantised
 // bf16), else QPROJ_KSPLIT_HOST int32 partials

@@ -197,6 +197,32 @@ __device__ __forceinline__ float slab_square_sum(const float v0, const float v1,
     return pair_tree_sum(__fmul_rn(__fmul_rn(v0, v0), coef), __fmul_rn(__fmul_rn(v1, v1), coef));
 }
 
+// Up to PROLOG_SMALL_TOKENS tokens the latents occupy 2 T compute units for the length of a few memory latencies, and the memory
+// idles.  Further workgroups of the launch, one per head, ask for the first rows of the head's projection weights, which the last
+// launch, bound by drawing weights, then finds in the L2 of the XCD it reads them on (workgroups go round the XCDs in both
+// launches, prolog_small_head).  The values are dropped.  512 rows are what arrives before the latents are done: fused prolog, 0 /
+// 256 / 512 / 768 rows: 8 tokens 34.6 / 33.6 / 32.9 / 33.6 us per pass, 32: 37.0 / 36.0 / 35.7 / 36.6; MLA prolog alone, 0 / 512:
+// 29.3 / 28.7 and 31.4 / 30.3.  Into the L2 of another XCD, so that only the memory-side cache helps: 8 tokens 34.4.  (The launch
+// for more than 32 tokens has two workgroups per compute unit to hide the same latencies: 48 tokens 42.6 / 42.8, 200: 68.3 / 68.4.)
+constexpr int MLAP_AHEAD_ROWS = 512;
+__device__ __forceinline__ void mlap_ask_ahead(const MlapParams &p, const int wg)
+{
+    if (wg < 0 || wg >= p.n_heads) return;
+    const int8_t *src = p.w_uqqr + (size_t)prolog_small_head(wg, p.n_heads) * MLAP_QHEAD;
+    constexpr int PIECES = MLAP_QHEAD / 64, N = MLAP_AHEAD_ROWS * PIECES / (64 * MID_WAVES);      // 64 bytes per lane
+    static_assert(N * 64 * MID_WAVES == MLAP_AHEAD_ROWS * PIECES && MLAP_AHEAD_ROWS <= MLAP_MIN_QLORA, "whole passes over rows that exist");
+    int v[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int piece = 64 * MID_WAVES * i + (int)threadIdx.x, row = piece / PIECES;
+        v[i] = *reinterpret_cast<const int *>(src + (size_t)row * p.n_heads * MLAP_QHEAD + 64 * (piece - PIECES * row));
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm volatile("" ::"v"(v[i]));
+}
+// workgroups of the latents' launch in front of those (a multiple of eight: the XCDs go round the same way)
+__host__ __device__ inline int mid_own_wgs(const int T) { return (2 * T + 7) / 8 * 8; }
+
 // Workgroup 2t: the query latent of token t (one wave per slab of 128 channels).  Workgroup 2t+1: its
 // key latent (waves 0..3) and key rope part (wave 4).
 // ngroups partial sums over the hidden axis per column, ngroups_rope for the 64 rope columns (which keep the fixed-order
@@ -205,6 +231,7 @@ __global__ __launch_bounds__(64 * MID_WAVES) void mlap_mid_kernel(const MlapPara
 {
     __shared__ float slabsum[MID_WAVES];
     __shared__ float slabmax[MID_WAVES];
+    if ((int)blockIdx.x >= 2 * p.T) return mlap_ask_ahead(p, (int)blockIdx.x - mid_own_wgs(p.T));
     const int l = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int t = blockIdx.x >> 1;
@@ -552,7 +579,9 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
         default: return hipErrorInvalidValue;
         }
     } else {
-        hipLaunchKernelGGL(mlap_mid_kernel, dim3((unsigned)(2 * p.T)), dim3(64 * MID_WAVES), 0, stream, p, ngroups, ngroups_fixed);
+        const bool ahead = mlap_fused_projection(p) && p.T <= PROLOG_SMALL_TOKENS;
+        const dim3 g((unsigned)(ahead ? mid_own_wgs(p.T) + p.n_heads : 2 * p.T));
+        hipLaunchKernelGGL(mlap_mid_kernel, g, dim3(64 * MID_WAVES), 0, stream, p, ngroups, ngroups_fixed);
     }
     e = hipGetLastError();
     if (e != hipSuccess || mlap_fused_projection(p)) return e;

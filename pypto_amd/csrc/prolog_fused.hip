@@ -63,20 +63,13 @@ __global__ __launch_bounds__(256, 2) void prolog_prefill_kernel(const MlapParams
 }
 
 // The same for at most PROLOG_SMALL_TOKENS tokens (prolog_small.h), a workgroup per head.
-// Heads 2m and 2m + 1 are workgroups of the same XCD, eight apart: a head's rows of w_uq_qr are 192 bytes, a pair's three cache
-// lines, the middle one of which they share.  (With neighbours on different XCDs every such line crossed into two L2s, 81 MB
-// read for 67 MB of weights; fused prolog: 1 token 33.4 us per pass, now 32.5, 8 tokens 34.4 and 33.8, 16: 39.6 and 39.2.)
-__device__ __forceinline__ int ps_head_of(const int wg, const int n_heads)
-{
-    return (n_heads & 15) == 0 ? 2 * (8 * (wg >> 4) + (wg & 7)) + ((wg >> 3) & 1) : wg;
-}
 constexpr int PS_LDS = PSA_LDS > PSI_LDS ? PSA_LDS : PSI_LDS;
 static_assert(LIP_FINT_LDS <= PS_LDS, "the token workgroups fit");
 __global__ __launch_bounds__(256) void prolog_small_kernel(const MlapParams pm, const LipParams pl, const int mla_wgs, const int lip_wgs)
 {
     __shared__ __attribute__((aligned(16))) uint8_t lds[PS_LDS];
     const int wg = (int)blockIdx.x;
-    if (wg < mla_wgs) mlap_small_body(pm, ps_head_of(wg, pm.n_heads), lds);
+    if (wg < mla_wgs) mlap_small_body(pm, prolog_small_head(wg, pm.n_heads), lds);
     else if (wg < mla_wgs + lip_wgs) lip_small_body(pl, wg - mla_wgs, lds);
     else lip_finish_tokens_prefill_body(pl, wg - mla_wgs - lip_wgs, lds);
 }
