@@ -368,72 +368,95 @@ __device__ __forceinline__ float lip_quant_rows(f32x16 (&c)[4], uint8_t *mine, c
 }
 
 // The same from the Hadamard product's operands, with its sums in their fixed order: 32 rows of rotated query channels (bf16,
-// HB_PITCH elements apart) times the matrix (plain rows), both in LDS, by a workgroup of four waves; the first T rows leave for
-// rows 0 .. T - 1 of q_int8 and q_scale at head `head`.  v_mfma_f32_16x16x1_4b_f32 multiplies one row of the matrix at a time, so
-// each of its results is one exact product added with one rounding (as in xlinear_fixed.h) and a chain of 128 is the sequential
-// sum.  Wave w makes columns 32*w .. +31: block b of the instruction is 16 of them (b / 2) x 16 rows (b % 2).
-// Bound: the matrix cores' fp32 rate, 128 x 32 clocks per wave.  (Fused prolog, 32 tokens: 42.3 us per pass; with the sums on the
-// vector ALU, a wave per row, 51.7; 16 tokens 39.8 and 41.9; 4 and 8 tokens the same.)
-// scratch: HB_SCRATCH bytes that nothing else of the workgroup uses.  The rows and the matrix have to be complete (barrier).
+// HB_PITCH elements apart) times the matrix (row r at 256 * r bytes, 16-byte piece q at q ^ 4*(r & 3)), both in LDS, by a workgroup
+// of four waves; the first T rows leave for rows 0 .. T - 1 of q_int8 and q_scale at head `head`.  v_mfma_f32_4x4x1_16b_f32
+// multiplies one row of the matrix at a time, so each of its results is one exact product added with one rounding (as in
+// xlinear_fixed.h) and a chain of 128 is the sequential sum.  Its sixteen blocks are 64 columns of the matrix (wave w: 64*(w & 1)
+// ..) and all take the same four rows: one register holds 16 channels of them, block k's lanes channel k, which the instruction
+// broadcasts.  A wave makes four rows up to 8 tokens, eight up to 16, else sixteen, as that many chains side by side.
+// Bound: the matrix cores' fp32 rate, 15 clocks per link and chain.  With the sums, by clock stamps: 8 tokens 2.2 us, 16: 2.7, 32: 3.9
+// (v_mfma_f32_16x16x1_4b_f32, whose chains are of 16 rows: 4.0 at any number of tokens); on the vector ALU, a wave per row, the
+// fused prolog took 9 us longer at 32 tokens.
 constexpr int HB_PITCH = LIP_DIM + 8;
-constexpr int HB_SCRATCH = 32 * QFP_OPITCH + 4 * 32 * 4;
+constexpr int HB_SCRATCH = 32 * HB_PITCH * 2;
+template <int G, int K>
+__device__ __forceinline__ void had_links(f32x4 (&c)[G], const float (&a)[G][LIP_DIM / 16], const int kk, const u32x2 (&h)[4])
+{
+    const uint32_t hw = h[K >> 2][(K >> 1) & 1];
+    const float hv = __uint_as_float((K & 1) ? hw & 0xffff0000u : hw << 16);
+#pragma unroll
+    for (int g = 0; g < G; ++g) c[g] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[g][kk], hv, c[g], 4, K, 0);
+    if constexpr (K < 15) had_links<G, K + 1>(c, a, kk, h);
+}
+// rows 4*G*(w / 2) .. +4*G-1, columns 64*(w & 1) .. +63 of the product, rounded to bf16, into out (HB_PITCH elements a row)
+template <int G>
+__device__ __forceinline__ void had_fixed_sums(const uint16_t *rows, const uint16_t *hmat, uint16_t *out, const int w, const int l)
+{
+    const int i = l & 15, q = l >> 4, row0 = 4 * G * (w >> 1);
+    f32x4 c[G];
+    float a[G][LIP_DIM / 16];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        c[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kk = 0; kk < LIP_DIM / 16; ++kk) a[g][kk] = bf16_bits_to_f32(rows[(row0 + 4 * g + (l & 3)) * HB_PITCH + 16 * kk + (l >> 2)]);
+    }
+    // a transposing read leaves lane i of sixteen column i of four rows
+    const uint16_t *hp = hmat + (i >> 2) * LIP_DIM + 8 * ((8 * (w & 1) + 2 * q + ((i & 3) >> 1)) ^ (4 * (i >> 2))) + 4 * (i & 1);
+#pragma unroll
+    for (int kk = 0; kk < LIP_DIM / 16; ++kk) {
+        u32x2 h[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) h[j] = __builtin_bit_cast(u32x2, lds_read_tr16(hp + (16 * kk + 4 * j) * LIP_DIM));
+        had_links<G, 0>(c, a, kk, h);
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            out[(row0 + 4 * g + r) * HB_PITCH + 64 * (w & 1) + l] = (uint16_t)(pack_bf16x2(c[g][r], 0.f) & 0xffffu);
+}
+// scratch: HB_SCRATCH bytes that nothing else of the workgroup uses.  The rows and the matrix have to be complete (barrier).
 __device__ __forceinline__ void lip_fixed_rows(const uint16_t *rows, const uint16_t *hmat, uint8_t *scratch, int8_t *q_int8, uint16_t *q_scale,
                                                const int n_heads, const int head, const int T, const int w, const int l)
 {
-    const int i = l & 15, q = l >> 4;
-    f32x16 c;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) c[r] = 0.f;
-    const uint16_t *hp = hmat + 32 * w + 16 * (q >> 1) + i;
-    const uint16_t *ap = rows + (16 * (q & 1) + i) * HB_PITCH;
-#pragma unroll
-    for (int k0 = 0; k0 < LIP_DIM; k0 += 8) {
-        const u32x4 a = *reinterpret_cast<const u32x4 *>(ap + k0);
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-            c = __builtin_amdgcn_mfma_f32_16x16x1f32(bf16_bits_to_f32(hp[(k0 + k) * LIP_DIM]),
-                                                     __uint_as_float((k & 1) ? a[k >> 1] & 0xffff0000u : a[k >> 1] << 16), c, 0, 0, 0);
-    }
-    // registers 4*b .. 4*b+3: columns 32*w + 16*(b / 2) + 4*q .. +3 of row 16*(b % 2) + i
-    float *mx = reinterpret_cast<float *>(scratch + 32 * QFP_OPITCH);
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-        float m = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int r = 4 * u + 8 * (e >> 2) + (e & 3);
-            c[r] = bf16_round_f32(c[r]);
-            m = fmaxf(m, fabsf(c[r]));
-        }
-        m = fmaxf(m, xor16_f32(m, l));
-        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
-        m = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-        if (q == 0) mx[32 * w + 16 * u + i] = m;
-    }
-    __syncthreads();                                   // the four parts of every row's largest magnitude are there
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-        const int row = 16 * u + i;
-        const float amax = fmaxf(fmaxf(mx[row], mx[32 + row]), fmaxf(mx[64 + row], mx[96 + row]));
-        float s = 0.f, deq = 0.f;
-        if (amax > 0.f) {
-            s = __fdiv_rn(127.0f, amax);
-            deq = __fdiv_rn(1.0f, s);
-        }
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            uint32_t v = 0;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) v |= (uint32_t)((int)rintf(__fmul_rn(c[4 * u + 8 * g + j], s)) & 0xff) << (8 * j);
-            *reinterpret_cast<uint32_t *>(scratch + row * QFP_OPITCH + 32 * w + 16 * g + 4 * q) = v;
-        }
-        if (w == 0 && q == 0 && row < T) q_scale[(size_t)row * n_heads + head] = (uint16_t)(pack_f16x2(deq, 0.f) & 0xffffu);
-    }
-    __syncthreads();                                   // the int8 rows are complete
+    uint16_t *out = reinterpret_cast<uint16_t *>(scratch);
+    if (T <= 8) had_fixed_sums<1>(rows, hmat, out, w, l);
+    else if (T <= 16) had_fixed_sums<2>(rows, hmat, out, w, l);
+    else had_fixed_sums<4>(rows, hmat, out, w, l);
+    __syncthreads();                                   // the product's rows are complete
+    if (8 * w >= T) return;
+    // eight lanes a row, sixteen columns each
     const int row = 8 * w + (l >> 3);
-    if (row < T)
-        *reinterpret_cast<u32x4 *>(q_int8 + ((size_t)row * n_heads + head) * LIP_DIM + 16 * (l & 7)) =
-            *reinterpret_cast<const u32x4 *>(scratch + row * QFP_OPITCH + 16 * (l & 7));
+    const uint16_t *src = out + row * HB_PITCH + 16 * (l & 7);
+    const u32x4 d[2] = {*reinterpret_cast<const u32x4 *>(src), *reinterpret_cast<const u32x4 *>(src + 8)};
+    float v[16], amax = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        const uint32_t x = d[e >> 3][(e & 7) >> 1];
+        v[e] = __uint_as_float((e & 1) ? x & 0xffff0000u : x << 16);
+        amax = fmaxf(amax, fabsf(v[e]));
+    }
+    amax = fmaxf(amax, dpp_f32<DPP_XOR1>(amax));
+    amax = fmaxf(amax, dpp_f32<DPP_XOR2>(amax));
+    amax = fmaxf(amax, dpp_f32<DPP_HALF_MIRROR>(amax));
+    float s = 0.f, deq = 0.f;
+    if (amax > 0.f) {
+        s = __fdiv_rn(127.0f, amax);
+        deq = __fdiv_rn(1.0f, s);
+    }
+    u32x4 o;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        uint32_t x = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x |= (uint32_t)((int)rintf(__fmul_rn(v[4 * g + j], s)) & 0xff) << (8 * j);
+        o[g] = x;
+    }
+    if (row < T) {
+        *reinterpret_cast<u32x4 *>(q_int8 + ((size_t)row * n_heads + head) * LIP_DIM + 16 * (l & 7)) = o;
+        if ((l & 7) == 0) q_scale[(size_t)row * n_heads + head] = (uint16_t)(pack_f16x2(deq, 0.f) & 0xffffu);
+    }
 }
 
 // ---------------------------------------------------------------------------------- MLA prolog

@@ -297,17 +297,17 @@ __device__ __forceinline__ void mlap_prefill_body(const MlapParams &p, const int
 // read is the accumulators' row order).  Weights: [head][64][128] per chunk, as q_build_a_tr reads them.  The matrix is
 // requested once the chunk buffers are free: row r at 256 * r, 16-byte piece q at q ^ 4*(r & 3).
 // FIXED (one tile of at most 64 tokens, the first two waves' blocks): the rotated rows meet in LDS and all four waves take the
-// Hadamard sums in their fixed order, a block of 32 rows at a time; the matrix then lies in plain rows.  (Fused prolog, 48
+// Hadamard sums in their fixed order, a block of 32 rows at a time.  (Fused prolog, 48
 // tokens: 46.9 us per pass; in the cores' own order, which the interface does not allow below 64 tokens, 46.3.)
 template <int TB> constexpr int PFI_TOK = 128 * TB;
 template <int XC, int TB> constexpr int PFI_X = PFI_TOK<TB> * PF_XPITCH<XC>;
 constexpr int PFI_W = PF_KC * LIP_DIM;
 constexpr int PFI_HAD = LIP_DIM * LIP_DIM * 2;
 template <int XC, int TB> constexpr int PFI_LOOP_LDS = 2 * PFI_X<XC, TB> + 3 * PFI_W;
-constexpr int PFI_FIN_LDS = PFI_HAD + 4 * 32 * QFP_OPITCH;
-template <int XC, int TB> constexpr int PFI_LDS = PFI_LOOP_LDS<XC, TB> > PFI_FIN_LDS ? PFI_LOOP_LDS<XC, TB> : PFI_FIN_LDS;
 constexpr int PFI_FIXED_TOK = 64;
 constexpr int PFI_FIXED_LDS = PFI_HAD + PFI_FIXED_TOK * HB_PITCH * 2 + HB_SCRATCH;
+constexpr int PFI_FIN_LDS = PFI_FIXED_LDS > PFI_HAD + 4 * 32 * QFP_OPITCH ? PFI_FIXED_LDS : PFI_HAD + 4 * 32 * QFP_OPITCH;
+template <int XC, int TB> constexpr int PFI_LDS = PFI_LOOP_LDS<XC, TB> > PFI_FIN_LDS ? PFI_LOOP_LDS<XC, TB> : PFI_FIN_LDS;
 
 template <int XC, int TB, bool FIXED>
 __device__ __forceinline__ void lip_prefill_body(const LipParams &p, const int job, uint8_t *lds)
@@ -360,7 +360,7 @@ __device__ __forceinline__ void lip_prefill_body(const LipParams &p, const int j
             });
     }
     {
-        const uint16_t *src = p.hq + (size_t)(4 * (8 * w) + (l >> 4)) * LIP_DIM + 8 * ((l & 15) ^ (FIXED ? 0 : 4 * ((l >> 4) & 3)));
+        const uint16_t *src = p.hq + (size_t)(4 * (8 * w) + (l >> 4)) * LIP_DIM + 8 * ((l & 15) ^ (4 * ((l >> 4) & 3)));
 #pragma unroll 1
         for (int j = 0; j < 8; ++j) dma16(src + (size_t)4 * j * LIP_DIM, base + 1024 * (8 * w + j));
     }
@@ -401,7 +401,7 @@ __device__ __forceinline__ void lip_prefill_body(const LipParams &p, const int j
         }
     }
     if constexpr (FIXED) {
-        static_assert(TB == 1 && PFI_FIXED_LDS <= PFI_LDS<XC, TB> && PFI_FIXED_TOK >= LIP_MFMA_MIN_TOKENS, "one tile of two blocks");
+        static_assert(TB == 1 && PFI_FIXED_TOK >= LIP_MFMA_MIN_TOKENS, "one tile of two blocks");
         uint16_t *rows = reinterpret_cast<uint16_t *>(lds + PFI_HAD);
         if (32 * w < PFI_FIXED_TOK) {
             // dword d of bq[0][ks]: channels 16*ks + 8*(d / 2) + 4*half + 2*(d % 2), +1 of row 32*w + l % 32
@@ -416,9 +416,11 @@ __device__ __forceinline__ void lip_prefill_body(const LipParams &p, const int j
         VM_WAIT(0);
         __syncthreads();                               // the rotated rows are complete, the matrix is staged
 #pragma unroll 1
-        for (int r0 = 0; r0 < p.T; r0 += 32)           // (a block's rows have left before the barriers of the next pass)
+        for (int r0 = 0; r0 < p.T; r0 += 32) {
+            if (r0) __syncthreads();                   // the last block's rows have left
             lip_fixed_rows(rows + r0 * HB_PITCH, reinterpret_cast<const uint16_t *>(lds), lds + PFI_HAD + PFI_FIXED_TOK * HB_PITCH * 2,
                            p.q_int8 + (size_t)r0 * p.n_heads * LIP_DIM, p.q_scale + (size_t)r0 * p.n_heads, p.n_heads, head, p.T - r0, w, l);
+        }
         return;
     }
     VM_WAIT(0);

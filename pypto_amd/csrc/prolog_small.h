@@ -2,9 +2,11 @@
 // prolog_prefill.h, in the form that fits a decode batch, where the weights -- 67 MB of them -- are all there is to wait for.
 // One workgroup of four waves per head and compute unit.  The launch's tokens lie in LDS whole; everything else of the LDS is a
 // ring of requests that never runs dry: chunks of 64 rows of the head's projection and, behind them without a gap, its w_uk,
-// sixteen rows at a time.  Bound: the rate at which 192 workgroups can draw weights out of memory with 80 KiB (attention
-// query) on their way each.  (Fused prolog: 8 tokens as two launches with partial sums in between 40.7 us per pass,
-// so 34.2; 32 tokens with the 24 KiB in flight of the form for more tokens 44.2, so 42.5.)
+// sixteen rows at a time.  Bound: memory, 54 MB in 10 us behind the first 2 (another 13 MB are in the L2: mlap_ask_ahead).  With
+// every chunk out of the L2 (timing only) an attention workgroup takes 8.1 us at 8 tokens and 9.0 at 32 instead of 13; with one
+// chunk between barriers, six blocks of columns as 2, 2, 1, 1 over the waves and 60 KiB on their way it took 9.6 and 10.8 (fused
+// prolog 8 tokens 33.0 us per pass, now 32.7, 32: 35.5 and 35.0).  (8 tokens as two launches with partial sums in between: 6 us
+// more.)
 // Included by prolog_fused.hip after prolog_prefill.h.
 #pragma once
 #include "prolog_prefill.h"
@@ -53,17 +55,23 @@ __device__ __forceinline__ i32x4 ps_token_operand(const uint8_t *tok, const int 
 }
 
 // ------------------------------------------------------------------------------------------------ attention query
-// Of the head's six blocks of 32 projected columns wave w makes w and, the first two waves, w + 4 (the rope channels).  Of the
-// product with w_uk each wave makes 128 columns, out of rows it has requested itself: that part of the ring needs no barriers.
-constexpr int PSA_SLOT = 16 * 1024;                    // 64 x 192 bytes of the projection, or 16 rows of w_uk: [wave][16][256 bytes]
-constexpr int PSA_SLOTS = 6;
+// Of the head's six blocks of 32 projected columns wave w makes w and, out of every second chunk, 4 + w % 2 (the rope channels: the
+// waves' sums are whole numbers and are added at the end).  Of the product with w_uk each wave makes 128 columns, out of rows it has requested itself: that part of the ring needs no barriers.
+constexpr int PSA_CHUNK = PF_KC * MLAP_QHEAD;          // 64 rows of 192 bytes of the projection
+constexpr int PSA_CHUNKS = 8;
+constexpr int PSA_STEP = 16 * 1024;                    // 16 rows of w_uk: [wave][16][256 bytes]
+constexpr int PSA_STEPS = 6;
 constexpr int PSA_RING = PS_TOK;
-constexpr int PSA_Q = PSA_RING + PSA_SLOTS * PSA_SLOT; // nope channels [token][256 bytes], 16-byte piece q at q ^ (t & 15)
+static_assert(PSA_CHUNKS * PSA_CHUNK == PSA_STEPS * PSA_STEP, "both go round the same ring");
+static_assert(MLAP_MIN_QLORA % (PF_KC * PSA_CHUNKS) == 0, "w_uk starts at the ring's start");
+constexpr int PSA_Q = PSA_RING + PSA_CHUNKS * PSA_CHUNK;   // nope channels [token][256 bytes], 16-byte piece q at q ^ (t & 15)
 constexpr int PSA_SC = PSA_Q + PROLOG_SMALL_TOKENS * MLAP_NOPE * 2;    // per wave: scales of the tokens, of its two blocks' columns
 constexpr int PSA_LDS = PSA_SC + 4 * 512;
 constexpr int PSA_SPITCH = 272;                        // bytes between the rows of a wave's output staging area
 // once the projection is made the tokens' place holds the rope rows and the staging areas
 static_assert(32 * PFA_RPITCH + 4 * 32 * PSA_SPITCH <= PS_TOK, "staging fits");
+constexpr int PSA_HALF = 16 * 1024;                    // and, before the staging areas, two waves' sums of the rope channels, 4 KB each
+static_assert(PSA_HALF >= 32 * PFA_RPITCH && PSA_HALF + 2 * 4096 <= PS_TOK, "behind the rope rows");
 static_assert(PSA_LDS <= 160 * 1024, "one workgroup fits a compute unit");
 
 __device__ __forceinline__ void mlap_small_body(const MlapParams &p, const int head, uint8_t *lds)
@@ -83,22 +91,23 @@ __device__ __forceinline__ void mlap_small_body(const MlapParams &p, const int h
     }
     // w_uk: rows 4j + l/16 of a chunk's sixteen, this wave's 128 columns; 16-byte piece q of row r at q ^ 4*(r & 3)
     const uint16_t *usrc = p.w_uk + ((size_t)head * MLAP_NOPE + (l >> 4)) * MLAP_KV + 128 * w + 8 * ((l & 15) ^ (4 * (l >> 4)));
-    auto request_w = [&](const int c, const int slot) {
+    auto request_w = [&](const int c) {
 #pragma unroll
-        for (int j = 0; j < 3; ++j) dma16(wsrc[j] + (size_t)c * PF_KC * ncols, base + PSA_RING + slot * PSA_SLOT + 1024 * (3 * w + j));
+        for (int j = 0; j < 3; ++j)
+            dma16(wsrc[j] + (size_t)c * PF_KC * ncols, base + PSA_RING + (c % PSA_CHUNKS) * PSA_CHUNK + 1024 * (3 * w + j));
     };
-    auto request_u = [&](const int ks, const int slot) {
+    auto request_u = [&](const int ks) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) dma16(usrc + (size_t)(16 * ks + 4 * j) * MLAP_KV, base + PSA_RING + slot * PSA_SLOT + 4096 * w + 1024 * j);
+        for (int j = 0; j < 4; ++j)
+            dma16(usrc + (size_t)(16 * ks + 4 * j) * MLAP_KV, base + PSA_RING + (ks % PSA_STEPS) * PSA_STEP + 4096 * w + 1024 * j);
     };
     const int tl = l & 31;
-    const bool two = w < 2;
     // (the scales too as requests: a load that the compiler tracks would wait for the whole ring)
     dma4(p.q_norm_scale + (tl < p.T ? tl : p.T - 1), base + PSA_SC + 512 * w);
-    dma4(p.w_qb_scale + head * MLAP_QHEAD + 32 * (two && half ? w + 4 : w) + tl, base + PSA_SC + 512 * w + 256);
+    dma4(p.w_qb_scale + head * MLAP_QHEAD + 32 * (half && w < 2 ? w + 4 : w) + tl, base + PSA_SC + 512 * w + 256);
     ps_request_tokens(p.q_norm, p.q_lora, p.T, base, w, l);
 #pragma unroll
-    for (int c = 0; c < PSA_SLOTS - 1; ++c) request_w(c, c);
+    for (int c = 0; c < PSA_CHUNKS; ++c) request_w(c);
 
     i32x16 acc[2];
 #pragma unroll
@@ -108,63 +117,90 @@ __device__ __forceinline__ void mlap_small_body(const MlapParams &p, const int h
     uint32_t aoff[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-        aoff[i] = PSA_RING + (16 * half + ((l & 15) >> 1)) * MLAP_QHEAD + 32 * ((w + 4 * (two ? i : 0)) ^ ((l >> 3) & 1)) + 16 * ((l >> 4) & 1) + 8 * (l & 1);
+        aoff[i] = PSA_RING + (16 * half + ((l & 15) >> 1)) * MLAP_QHEAD + 32 * ((i ? 4 + (w & 1) : w) ^ ((l >> 3) & 1)) + 16 * ((l >> 4) & 1) + 8 * (l & 1);
     typedef int v2i __attribute__((ext_vector_type(2)));
-    auto products = [&](const int c, const int slot) {
-#pragma unroll
-        for (int s = 0; s < PF_KC / 32; ++s) {
-            const i32x4 b = ps_token_operand(lds, p.q_lora, 2 * c + s, l);
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                if (i == 1 && !two) break;
-                const uint8_t *ap = lds + slot * PSA_SLOT + aoff[i] + s * 32 * MLAP_QHEAD;
-                const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i *)(lds_byte_t *)ap);
-                const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i *)(lds_byte_t *)(ap + 8 * MLAP_QHEAD));
-                const i32x4 a = {lo[0], lo[1], hi[0], hi[1]};
-                acc[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, acc[i], 0, 0, 0);
-            }
-        }
+    auto operand = [&](const int i, const int slot, const int s) {
+        const uint8_t *ap = lds + slot * PSA_CHUNK + aoff[i] + s * 32 * MLAP_QHEAD;
+        const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i *)(lds_byte_t *)ap);
+        const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i *)(lds_byte_t *)(ap + 8 * MLAP_QHEAD));
+        return i32x4{lo[0], lo[1], hi[0], hi[1]};
     };
-    auto next_slot = [](const int s) { return s == PSA_SLOTS - 1 ? 0 : s + 1; };
-    auto prev_slot = [](const int s) { return s == 0 ? PSA_SLOTS - 1 : s - 1; };
-    // chunk c is waited for with the four behind it outstanding, three requests each or, of w_uk, four
-    int c = 0, slot = 0;
-#pragma unroll 1
-    for (; c + PSA_SLOTS - 1 <= nch - 1; ++c) {
-        VM_WAIT(12);
-        __syncthreads();                               // chunk c has landed for every wave; every wave is done with chunk c - 1
-        request_w(c + PSA_SLOTS - 1, prev_slot(slot));
-        products(c, slot);
-        slot = next_slot(slot);
-    }
+    // chunks c and c + 1 (c even), for the rope block c + w / 2
+    auto products = [&](const int c) {
+        const int slot = c % PSA_CHUNKS;
+        i32x4 b[4], a[4], ar[2];
 #pragma unroll
-    for (int j = 0; j < PSA_SLOTS - 1; ++j, ++c) {     // c = nch - 5 + j: j chunks of w_uk behind it already
-        ps_wait(12 + j);
-        __syncthreads();
-        request_u(j, prev_slot(slot));
-        products(c, slot);
-        slot = next_slot(slot);
+        for (int s = 0; s < 4; ++s) {
+            b[s] = ps_token_operand(lds, p.q_lora, 2 * c + s, l);
+            a[s] = operand(0, slot + (s >> 1), s & 1);
+        }
+#pragma unroll
+        for (int s = 0; s < 2; ++s) ar[s] = operand(1, slot + (w >> 1), s);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[s], b[s], acc[0], 0, 0, 0);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ar[s], w >> 1 ? b[2 + s] : b[s], acc[1], 0, 0, 0);
+    };
+    // Two chunks between barriers.  Those of the next two turns, 12 requests, may be outstanding when they are waited for (at the
+    // start three turns'); the two behind them take the places of the last turn's.
+    VM_WAIT(18);
+    __syncthreads();
+    products(0);
+    int c = 2;
+#pragma unroll 1
+    for (; c <= nch - PSA_CHUNKS; c += 2) {
+        VM_WAIT(12);
+        __syncthreads();                               // chunks c, c + 1 have landed for every wave; every wave is done with c - 1
+        request_w(c + PSA_CHUNKS - 2);
+        request_w(c + PSA_CHUNKS - 1);
+        products(c);
     }
+    // the last six chunks: as 24, 48, 72 KiB of the ring become free, one, three, four of w_uk's 16 KiB steps follow
+    VM_WAIT(12);
+    __syncthreads();
+    request_u(0);
+    products(c);
+    VM_WAIT(10);
+    __syncthreads();
+    request_u(1);
+    request_u(2);
+    products(c + 2);
+    VM_WAIT(12);
+    __syncthreads();
+    request_u(3);
+    products(c + 4);
     __syncthreads();                                   // every wave is done with the projection's chunks and the tokens
+    request_u(4);
+    request_u(5);
+    if (w >= 2) {
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg)
+            *reinterpret_cast<i32x4 *>(lds + PSA_HALF + 4096 * (w - 2) + 1024 * rg + 16 * l) = i32x4{acc[1][4 * rg], acc[1][4 * rg + 1], acc[1][4 * rg + 2], acc[1][4 * rg + 3]};
+    }
     // registers 4*rg .. 4*rg+3 of a block: columns 8*rg + 4*half .. +3 of token l % 32
     const float *sc_lds = reinterpret_cast<const float *>(lds + PSA_SC + 512 * w);
     const float ts = sc_lds[tl];
+    auto dequantise = [&](const i32x16 &x, const int i, const int rg) {
+        const f32x4 sc = *reinterpret_cast<const f32x4 *>(sc_lds + 64 + 32 * i + 4 * half + 8 * rg);
+        float f[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        if (i == 1 && !two) break;
-        const float *cs = sc_lds + 64 + 32 * i + 4 * half;
+        for (int j = 0; j < 4; ++j) f[j] = __fmul_rn(__fmul_rn((float)x[4 * rg + j], ts), sc[j]);
+        return u32x2{pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3])};
+    };
+#pragma unroll
+    for (int rg = 0; rg < 4; ++rg)
+        *reinterpret_cast<u32x2 *>(lds + PSA_Q + tl * 256 + 16 * ((4 * w + rg) ^ (l & 15)) + 8 * half) = dequantise(acc[0], 0, rg);
+    __syncthreads();                                   // the nope operand and the other waves' sums of the rope channels are complete
+    if (w < 2) {
 #pragma unroll
         for (int rg = 0; rg < 4; ++rg) {
-            const f32x4 sc = *reinterpret_cast<const f32x4 *>(cs + 8 * rg);
-            float f[4];
+            const i32x4 other = *reinterpret_cast<const i32x4 *>(lds + PSA_HALF + 4096 * w + 1024 * rg + 16 * l);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) f[j] = __fmul_rn(__fmul_rn((float)acc[i][4 * rg + j], ts), sc[j]);
-            const u32x2 v = {pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3])};
-            if (i == 0) *reinterpret_cast<u32x2 *>(lds + PSA_Q + tl * 256 + 16 * ((4 * w + rg) ^ (l & 15)) + 8 * half) = v;
-            else *reinterpret_cast<u32x2 *>(lds + tl * PFA_RPITCH + 2 * (32 * w + 8 * rg + 4 * half)) = v;
+            for (int j = 0; j < 4; ++j) acc[1][4 * rg + j] += other[j];
+            *reinterpret_cast<u32x2 *>(lds + tl * PFA_RPITCH + 2 * (32 * w + 8 * rg + 4 * half)) = dequantise(acc[1], 1, rg);
         }
     }
-    __syncthreads();                                   // nope operand and rope rows are complete
+    __syncthreads();                                   // the rope rows are complete, their sums read
     f32x16 o[4];
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb)
@@ -173,26 +209,26 @@ __device__ __forceinline__ void mlap_small_body(const MlapParams &p, const int h
     const uint32_t uoff = PSA_RING + 4096 * w + (8 * half + ((l & 15) >> 2)) * 256 + 8 * (l & 1);
 #pragma unroll
     for (int ks = 0; ks < MLAP_NOPE / 16; ++ks) {
-        // steps ks + 1 .. ks + 4 are outstanding; the slot before this one is this wave's to fill again
-        if (ks <= 3) VM_WAIT(16);
+        // steps ks + 1 .. ks + 4, at first ks + 5, are outstanding; the place of the step before this one is this wave's to fill again
+        if (ks == 0) VM_WAIT(20);
+        else if (ks <= 3) VM_WAIT(16);
         else if (ks == 4) VM_WAIT(12);
         else if (ks == 5) VM_WAIT(8);
         else if (ks == 6) VM_WAIT(4);
         else VM_WAIT(0);
         asm volatile("" ::: "memory");
-        if (ks + PSA_SLOTS - 1 < MLAP_NOPE / 16) request_u(ks + PSA_SLOTS - 1, prev_slot(slot));
+        if (ks >= 1 && ks + PSA_STEPS - 1 < MLAP_NOPE / 16) request_u(ks + PSA_STEPS - 1);
         const bf16x8 b = *reinterpret_cast<const bf16x8 *>(lds + PSA_Q + tl * 256 + 16 * ((2 * ks + half) ^ (l & 15)));
 #pragma unroll
         for (int cb = 0; cb < 4; ++cb) {
             const int piece = 4 * cb + 2 * ((l >> 4) & 1) + ((l & 3) >> 1);
-            const uint16_t *ap = reinterpret_cast<const uint16_t *>(lds + slot * PSA_SLOT + uoff + 16 * (piece ^ (4 * ((l & 15) >> 2))));
+            const uint16_t *ap = reinterpret_cast<const uint16_t *>(lds + (ks % PSA_STEPS) * PSA_STEP + uoff + 16 * (piece ^ (4 * ((l & 15) >> 2))));
             const s16x4 lo = lds_read_tr16(ap), hi = lds_read_tr16(ap + 4 * 128);
             const s16x8 a = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
             o[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), b, o[cb], 0, 0, 0);
         }
         __builtin_amdgcn_s_waitcnt(0xC07F);            // lgkmcnt(0): the slot has been read
         asm volatile("" ::: "memory");
-        slot = next_slot(slot);
     }
     // lane (token, half) holds columns 8*(r/4) + 4*half + r%4 of each block: out through the staging area as 256-byte pieces of rows
     uint8_t *stg = lds + 32 * PFA_RPITCH + w * (32 * PSA_SPITCH);
@@ -218,7 +254,8 @@ __device__ __forceinline__ void mlap_small_body(const MlapParams &p, const int h
 // are taken in their fixed order by all four waves (lip_fixed_rows).
 constexpr int PSI_SLOT = PF_KC * LIP_DIM;
 constexpr int PSI_SLOTS = 8;
-constexpr int PSI_HAD = PS_TOK;                        // the matrix, plain rows
+constexpr int PSI_ROT = PROLOG_SMALL_TOKENS / 4;       // rows that a wave rotates
+constexpr int PSI_HAD = PS_TOK;                        // the matrix, row r at 256 * r, 16-byte piece q at q ^ 4*(r & 3)
 constexpr int PSI_RING = PSI_HAD + LIP_DIM * LIP_DIM * 2;
 constexpr int PSI_LDS = PSI_RING + PSI_SLOTS * PSI_SLOT;
 constexpr int PSI_SCRATCH = PSI_RING + 32 * HB_PITCH * 2;     // behind the rows, in the ring's place
@@ -241,14 +278,23 @@ __device__ __forceinline__ void lip_small_body(const LipParams &p, const int hea
 #pragma unroll
         for (int j = 0; j < 2; ++j) dma16(wsrc[j] + (size_t)c * PF_KC * ncols, base + PSI_RING + slot * PSI_SLOT + 1024 * (2 * w + j));
     };
-    ps_request_tokens(p.q_norm, p.q_lora, p.T, base, w, l);
-#pragma unroll
-    for (int c = 0; c < PSI_SLOTS - 1; ++c) request_w(c, c);
+    // (the loads that the compiler tracks come first: the waits below count the requests behind them)
     const int tl = l & 31;
     const float ts = p.q_norm_scale[tl < p.T ? tl : p.T - 1];
     f32x4 sc[4];
 #pragma unroll
     for (int rg = 0; rg < 4; ++rg) sc[rg] = *reinterpret_cast<const f32x4 *>(p.w_qb_scale + head * LIP_DIM + 32 * w + 8 * rg + 4 * half);
+    uint32_t rc[PSI_ROT], rs[PSI_ROT];                 // rotation factors of tokens w, w + 4, ..
+#pragma unroll
+    for (int k = 0; k < PSI_ROT; ++k) {
+        const int t = w + 4 * k < p.T ? w + 4 * k : p.T - 1;
+        rc[k] = rope_coef(p.cos, t, l);
+        rs[k] = rope_coef(p.sin, t, l);
+    }
+    asm volatile("" ::: "memory");
+    ps_request_tokens(p.q_norm, p.q_lora, p.T, base, w, l);
+#pragma unroll
+    for (int c = 0; c < PSI_SLOTS - 1; ++c) request_w(c, c);
     i32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0;
@@ -268,7 +314,7 @@ __device__ __forceinline__ void lip_small_body(const LipParams &p, const int hea
         slot = slot == PSI_SLOTS - 1 ? 0 : slot + 1;
     }
     {   // the matrix, behind the last chunk's requests
-        const uint16_t *src = p.hq + (size_t)(32 * w + (l >> 4)) * LIP_DIM + 8 * (l & 15);
+        const uint16_t *src = p.hq + (size_t)(32 * w + (l >> 4)) * LIP_DIM + 8 * ((l & 15) ^ (4 * (l >> 4)));
 #pragma unroll 1
         for (int j = 0; j < 8; ++j) dma16(src + (size_t)4 * j * LIP_DIM, base + PSI_HAD + 1024 * (8 * w + j));
     }
@@ -293,13 +339,18 @@ __device__ __forceinline__ void lip_small_body(const LipParams &p, const int hea
     }
     __syncthreads();                                   // the rows are complete
     const uint16_t *hmat = reinterpret_cast<const uint16_t *>(lds + PSI_HAD);
-    for (int t = w; t < p.T; t += 4) {
-        const uint32_t rc = rope_coef(p.cos, t, l), rs = rope_coef(p.sin, t, l);
-        uint32_t *mine = reinterpret_cast<uint32_t *>(abf + t * HB_PITCH + 2 * l);
-        const uint32_t raw = *mine;
-        float v0 = __uint_as_float(raw << 16), v1 = __uint_as_float(raw & 0xffff0000u);
-        rope_pair(v0, v1, rc, rs, l);
-        *mine = pack_bf16x2(v0, v1);
+#pragma unroll
+    for (int k0 = 0; k0 < PSI_ROT; k0 += 4) {          // (rows from T on are rotated along and dropped)
+        if (4 * k0 >= p.T) break;
+        uint32_t raw[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) raw[k] = *reinterpret_cast<const uint32_t *>(abf + (w + 4 * (k0 + k)) * HB_PITCH + 2 * l);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            float v0 = __uint_as_float(raw[k] << 16), v1 = __uint_as_float(raw[k] & 0xffff0000u);
+            rope_pair(v0, v1, rc[k0 + k], rs[k0 + k], l);
+            *reinterpret_cast<uint32_t *>(abf + (w + 4 * (k0 + k)) * HB_PITCH + 2 * l) = pack_bf16x2(v0, v1);
+        }
     }
     __syncthreads();                                   // the rotated rows are complete
     lip_fixed_rows(abf, hmat, lds + PSI_SCRATCH, p.q_int8, p.q_scale, p.n_heads, head, p.T, w, l);
