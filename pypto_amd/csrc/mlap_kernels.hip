@@ -99,25 +99,30 @@ __global__ __launch_bounds__(64 * XL_WAVES) void mlap_xlinear_kernel(const MlapP
 // one of nsplit ranges of the hidden axis, 128 tokens); the 64 rope columns are a narrow slab of their own.
 static_assert(XM_KC == MLAP_XBLOCK, "the workspace is sized in chunks of the hidden axis");
 
-// The workgroups past the first own_wgs take sums in their fixed order (xlinear_fixed.h, the matrix-core form of the
+// Further workgroups take sums in their fixed order (xlinear_fixed.h, the matrix-core form of the
 // sequential sums), 64 columns each: the rope columns of w_dkv_kr at every size -- the reference's acceptance rule allows
 // the rotated key no outlier at all (deepseekv32_mla_prolog_quant.py:688: atol 1e-4, rtol 2^-7 per element, ratio 0), and
 // a sum that lands next to a bf16 rounding boundary in another order moves a small rotated value by more than that --
 // and, in the fused prolog, the indexer prolog's wk and w_proj.  They are short and follow the long workgroups of the
 // other slabs, so they fill the launch's last round; two workgroups fit a compute unit.  (1000 tokens: 69 us here and 79
-// in a launch of the indexer's own before they shared it.)
+// in a launch of the indexer's own before they shared it.)  Up to 64 tokens all workgroups run at once and these are the longer
+// ones beside another workgroup, so they start first (fused prolog, 32 tokens: 37.4 us per pass, at the end of the launch 39.3;
+// 200 tokens 84.4, at the end 70.3).
 // TB: at most 32 * TB tokens (xm_small_body), 0 for tiles of 128 tokens (xm_body), XM_BIG for tiles of 256 (xb_body).
 constexpr int XM_BIG = 8;
 template <int TB> constexpr int XM_FORM_LDS = TB == 0 ? XM_LDS : (TB == XM_BIG ? XB_LDS : XMS_LDS<TB == 1 ? 1 : 2>);
 template <int TB> constexpr int XM_KERNEL_LDS = XM_FORM_LDS<TB> > XF_LDS ? XM_FORM_LDS<TB> : XF_LDS;
-static_assert(2 * XM_KERNEL_LDS<0> <= 160 * 1024, "two workgroups share a compute unit");
+static_assert(2 * XM_KERNEL_LDS<0> <= 160 * 1024 && 2 * XM_KERNEL_LDS<2> <= 160 * 1024, "two workgroups share a compute unit");
 template <int TB>
 __global__ __launch_bounds__(256) void mlap_xlinear_mfma_kernel(const MlapParams p, const int nslabs, const int nsplit, const int own_wgs,
                                                                 const int fixed_sets, const int fixed_groups, const LipParams lip)
 {
     __shared__ __attribute__((aligned(16))) uint8_t smem[XM_KERNEL_LDS<TB>];
-    if ((int)blockIdx.x >= own_wgs) {
-        const XfJob j = xf_job((int)blockIdx.x - own_wgs, fixed_sets, fixed_groups, p.T);
+    constexpr bool FIXED_FIRST = TB == 1 || TB == 2;
+    const int nfixed = (int)gridDim.x - own_wgs;                   // a multiple of eight, as own_wgs: the XCDs go round alike
+    const int fixed = (int)blockIdx.x - (FIXED_FIRST ? 0 : own_wgs), bid = (int)blockIdx.x - (FIXED_FIRST ? nfixed : 0);
+    if (FIXED_FIRST ? fixed < nfixed : fixed >= 0) {
+        const XfJob j = xf_job(fixed, fixed_sets, fixed_groups, p.T);
         if (j.g < 0) return;
         XlSlab sl;
         if (j.set == 0) {
@@ -133,7 +138,6 @@ __global__ __launch_bounds__(256) void mlap_xlinear_mfma_kernel(const MlapParams
         xf_body(sl, p.x, p.T, p.h, j.g, j.t0, smem);
         return;
     }
-    const int bid = (int)blockIdx.x;
     if constexpr (TB == XM_BIG) {
         // every XCD takes a run of the jobs in the order (range of h, token tile, slab): a range's weights and the hidden
         // states of a tile or two cross into its L2 once, chunk by chunk, as the run's workgroups walk the range together
@@ -329,9 +333,10 @@ __global__ __launch_bounds__(64 * MID_WAVES) void mlap_mid_kernel(const MlapPara
 // The same at prefill sizes, a wave per token and latent (waves 2t: the query latent, 2t + 1: the key latent and key rope):
 // no barriers, and the slabs' loads and reductions run side by side in one wave.  (The form above, a workgroup of twelve
 // waves per latent that waits for memory once and meets twice, is all latency once the chip has run out of room for more
-// workgroups: 1000 tokens 22.0 us.)
+// workgroups: 1000 tokens 22.0 us.  As long as 512 of them have room it is the faster one: 64 tokens 5.4 us and 9.4, fused prolog
+// 64 tokens 47.2 us per pass and 51.0, 128: 54.9 and 57.6, 256: 73.3 and 74.4.)
 constexpr int MIDP_WAVES = 4;
-constexpr int MIDP_MIN_TOKENS = 64;
+constexpr int MIDP_MIN_TOKENS = 257;
 
 // NS slabs of 128 columns at src (lane: columns 2l, 2l + 1 of each): the partial sums added ascending, rounded to bf16
 template <int NS>
@@ -538,18 +543,18 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
         // every slab but the last, the rope columns, which keep their fixed-order sums
         const int mslabs = nslabs - 1;
         const bool big = p.T > XM_TOK;       // 130 tokens: 60.9 us per pass, 66.7 with tiles of 128; 1500: 282 and 293; 4096: 700 and 724
-        // As many ranges as make this many workgroups, in eighths of the compute units: the rest of the chip is for the
-        // fixed-order sums, and what does not fit beside them runs as a second round, nearly empty and as long as the first.
-        // Up to 64 tokens a compute unit holds one workgroup, and more ranges are more partial sums to write and read as well
-        // (fused prolog, 14 ranges and as it is: 9 tokens 38.9 and 33.6, 32: 42.4 and 37.0, 48: 47.3 and 42.4, 64: 52.9 and
-        // 45.2; MLA prolog alone, 32: 34.2 and 31.5).  128 tokens: 14 ranges 58.1, 12: 57.7 (alone, 100: 53.5 and 50.7); in
-        // tiles of 256 tokens, 192: 14 ranges 72.9, 12: 68.9; 256: 14 ranges 77.8, 10: 72.2 (alone 61.7 and 62.6); 400: 8 ranges
-        // 106.5, 6: 101.6, but alone, which has the same ranges to give the same bits, 77.2 and 80.7.
+        // More than 64 tokens: as many ranges as make this many workgroups, in eighths of the compute units.  The rest of the chip
+        // is for the fixed-order sums, and what does not fit beside them runs as a second round, nearly empty and as long as the
+        // first.  (Fused prolog: 128 tokens, 14 ranges 58.1 us per pass, 12: 57.7 (alone, 100: 53.5 and 50.7); in tiles of 256
+        // tokens, 192: 14 ranges 72.9, 12: 68.9; 256: 14 ranges 77.8, 10: 72.2 (alone 61.7 and 62.6); 400: 8 ranges 106.5, 6:
+        // 101.6, but alone, which has the same ranges to give the same bits, 77.2 and 80.7.)
+        // Up to 64 tokens one int8 value of a token's latent that falls the other way is 9 % of its indexer query, so that the
+        // ranges, which the order of the sums depends on, stay what they are; two workgroups share a compute unit instead, and the
+        // fixed-order sums start first (one per compute unit, those last, so a second round: 9 tokens 39.1, now 32.2; 32: 42.5 and
+        // 36.4; 48: 47.3 and 43.3; 64: 52.9 and 44.8; two ranges per workgroup: 9 tokens 33.5, 32: 37.0, 48: 47.1, 64: 52.5).
         const int xtiles = big ? (p.T + XB_TOK - 1) / XB_TOK : ttiles;
-        int eighths = 8;
-        if (p.T <= 64) eighths = 4;
-        else if (xtiles == 1) eighths = p.T <= 192 ? 6 : 5;
-        ngroups = eighths * cus / (8 * mslabs * xtiles);
+        const int eighths = xtiles > 1 ? 8 : (p.T <= 192 ? 6 : 5);
+        ngroups = p.T <= 64 ? 2 * cus / nslabs : eighths * cus / (8 * mslabs * xtiles);
         ngroups = ngroups < 1 ? 1 : ngroups;
         ngroups = ngroups > MLAP_XM_MAX_SPLITS ? MLAP_XM_MAX_SPLITS : ngroups;
         ngroups = ngroups > nchunks ? nchunks : ngroups;

@@ -268,22 +268,23 @@ __device__ __forceinline__ void xb_body(const XmSlab &sl, const uint16_t *x, con
 }
 
 // ---------------------------------------------------------------------------------------------
-// The same for at most 32 * TB tokens (TB = 1 or 2), where the slab's weights are nearly all a workgroup reads and a
-// compute unit holds one workgroup: what counts is that every compute unit has its requests on their way from the start
-// and keeps them coming.  The staged tokens are the launch's own (the form above stages 128 rows whatever T is), which
-// leaves room for a ring of seven (six) chunks instead of two buffers, and one barrier per chunk.  At 32 tokens
-// (29 MB of weights) the launch takes 12.1 us; with the form above, at most two chunks in flight per compute unit, 14.1.
+// The same for at most 32 * TB tokens (TB = 1 or 2), where the slab's weights are nearly all a workgroup reads.  The staged tokens
+// are the launch's own (the form above stages 128 rows whatever T is), so two chunk buffers, the next chunk requested when the last
+// one is consumed, are a third of a compute unit's LDS and all workgroups of a launch run at once.  (With a ring of seven chunks and
+// one workgroup per compute unit the last workgroups were a second round.  More chunks on their way are slower all the same: they
+// are in the way of the fixed-order sums' requests, which the launch ends with.  Fused prolog, 2 / 3 / 4 chunk buffers: 9 tokens
+// 32.2 / 32.9 / 33.3 us per pass, 32: 36.4 / 37.0 / 37.6; MLA prolog alone, 2 / 3: 32 tokens 30.4 / 31.1, 64: 40.1 / 40.6; only the
+// fused prolog at 64 goes the other way, 44.8 / 44.6.)
 // Wave w takes token block w % TB and, of the slab's four blocks of 32 columns, the TB blocks from TB * (w / TB) on.
 template <int TB> constexpr int XMS_CHUNK = XM_W_BYTES + TB * 32 * XM_KC * 2;
-template <int TB> constexpr int XMS_RING = TB == 1 ? 7 : 6;
-template <int TB> constexpr int XMS_LDS = XMS_RING<TB> * XMS_CHUNK<TB>;      // 143 360, 147 456 bytes
+template <int TB> constexpr int XMS_LDS = 2 * XMS_CHUNK<TB>;                 // 40 960, 49 152 bytes
 
 template <int TB>
 __device__ __forceinline__ void xm_small_body(const XmSlab &sl, const uint16_t *x, const int T, const int h, const int c_begin, const int c_end,
                                               uint8_t *smem)
 {
     static_assert(TB == 1 || TB == 2, "token blocks");
-    constexpr int RING = XMS_RING<TB>, CHUNK = XMS_CHUNK<TB>, PER = 4 + TB;    // requests of a wave per chunk
+    constexpr int CHUNK = XMS_CHUNK<TB>;
     const int l = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tb = w % TB, cb0 = TB * (w / TB);
@@ -313,25 +314,13 @@ __device__ __forceinline__ void xm_small_body(const XmSlab &sl, const uint16_t *
 #pragma unroll
     for (int i = 0; i < TB; ++i) aoff[i] = (uint32_t)(arow * 256 + 16 * ((4 * (cb0 + i) + 2 * ((l >> 4) & 1) + ((l & 3) >> 1)) ^ aswz) + 8 * (l & 1));
     const int brow = 32 * tb + (l & 31), bswz = (brow >> 1) & 7;
-    const int n = c_end - c_begin;
-#pragma unroll 1
-    for (int c = 0; c < RING - 1 && c < n; ++c) request_chunk(c_begin + c, c);
+    if (c_begin < c_end) request_chunk(c_begin, 0);
     int buf = 0;
 #pragma unroll 1
-    for (int c = 0; c < n; ++c) {
-        // chunk c has landed when at most the younger chunks' requests are outstanding (uniform)
-        const int younger = n - 1 - c < RING - 2 ? n - 1 - c : RING - 2;
-        switch (younger) {
-        case 5: VM_WAIT(5 * PER); break;
-        case 4: VM_WAIT(4 * PER); break;
-        case 3: VM_WAIT(3 * PER); break;
-        case 2: VM_WAIT(2 * PER); break;
-        case 1: VM_WAIT(PER); break;
-        default: VM_WAIT(0); break;
-        }
-        static_assert(RING <= 7, "the cases above");
-        __syncthreads();                               // every wave's part has landed; every wave is done with chunk c - 1
-        if (c + RING - 1 < n) request_chunk(c_begin + c + RING - 1, buf == 0 ? RING - 1 : buf - 1);
+    for (int c = c_begin; c < c_end; ++c) {
+        VM_WAIT(0);
+        __syncthreads();                               // every wave's part of chunk c has landed; every wave is done with chunk c - 1
+        if (c + 1 < c_end) request_chunk(c + 1, buf ^ 1);
         const uint8_t *wb = smem + buf * CHUNK;
         const uint8_t *xb = wb + XM_W_BYTES;
 #pragma unroll
@@ -345,11 +334,12 @@ __device__ __forceinline__ void xm_small_body(const XmSlab &sl, const uint16_t *
                 acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[i], 0, 0, 0);
             }
         }
-        buf = buf + 1 == RING ? 0 : buf + 1;
+        buf ^= 1;
     }
-    __syncthreads();                                   // every wave is done with the last chunk: the ring becomes staging areas
+    __syncthreads();                                   // every wave is done with the last chunk: the buffers become staging areas
     // 32 tokens x 32 * TB columns per wave leave as whole row segments (as above)
     constexpr int SPITCH = 128 * TB + 16;
+    static_assert(4 * 32 * SPITCH <= XMS_LDS<TB>, "the staging areas reuse the chunk buffers");
     uint8_t *stg = smem + w * (32 * SPITCH);
 #pragma unroll
     for (int i = 0; i < TB; ++i)
