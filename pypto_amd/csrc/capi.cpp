@@ -230,18 +230,21 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
     pl.scratch_bytes = partial_bytes(split_rows, pl.nsplit, f32);
     // More than 32 heads: workgroups of 64 heads (sfa_slice_kernel) where they are the faster ones, within the bytes that a caller
     // is asked for, which stay those of the division above.  In microseconds, fitted to an int8 cache, 1 to 128 rows, top-k 2048,
-    // 128 heads (measured: 32 rows 4 splits 32.3, 16 rows 8 splits 24.2, 4 rows 16 splits 18.8, 1 row 32 splits 13.5, against
+    // 128 heads (measured: 32 rows 4 splits 32.3, 16 rows 8 splits 24.2, 4 rows 13 splits 18.4, 1 row 22 splits 14.0, against
     // 35.0, 28.6, 20.0 and 14.1 as four groups and one group of 32 heads; 36 to 64 rows alike; 128 rows 97.1 against 95.0).
+    // A tile of whole rows takes 1.13 with 128 workgroups, 1.2 with 192 and 1.45 with 256 (top-k 1024, 96 rows: 44.9, as four groups
+    // and two splits 49.4); partial results past one round's cost more (64 heads, 96 rows: 5 splits 58.8, 2 splits 51.8).
     if (a->nq > 32 && a->num_splits == 0 && min_split == 1) {
         const int sh = shares(2);
         if (pl.head_groups == 2) best = -1.0;             // (two groups of 32 heads: that is this form, at another price)
-        auto slice_round_us = [&](const int s) {
+        auto slice_round_us = [&](const int s, const long long wgs) {          // (of the launch: 256 and more fill the chip)
             const int len = (tiles + s - 1) / s;
-            return s == 1 ? 1.4 * len : (0.59 + 0.0175 * len) * len;
+            const double full = wgs < cus ? (double)wgs / cus : 1.0;
+            return s == 1 ? (1.1 + 0.35 * full * full * full * full) * len : (0.59 + 0.0175 * len) * len;
         };
         auto slice_tail_us = [&](const long long r, const int s) {
             const double wgs = (double)(r * sh * s);
-            return s == 1 ? 6.0 : 13.2 + (s > 8 ? 0.056 * wgs - 3.5 : 0.02 * wgs);
+            return s == 1 ? 6.0 : 13.2 + (s > 8 ? 0.056 * wgs - 3.5 : 0.02 * wgs + (wgs > cus ? 0.03 * (wgs - cus) : 0.0));
         };
         auto take = [&](const double cost, const int s, const long long whole) {
             if (best >= 0.0 && cost >= best) return;
@@ -257,14 +260,14 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
             len = (tiles + s - 1) / s;
             if (s > 1 && (partial_bytes(rows, s) > pl.scratch_bytes || rows * sh * s > 4ll * cus)) break;
             const double n = (double)rounds(rows * sh * s);
-            take(n * slice_round_us(s) + (n - 1.0) * 7.0 + slice_tail_us(rows, s), s, 0);    // (a further round starts and ends too)
+            take(n * slice_round_us(s, rows * sh * s) + (n - 1.0) * 7.0 + slice_tail_us(rows, s), s, 0);    // (a further round starts and ends too)
         }
         const long long per_round = cus / 8 / sh, full = per_round > 0 ? (rows + 7) / 8 / per_round : 0, rows_b = rows - 8 * full * per_round;
         if (!f32 && cus % 8 == 0 && full >= 1 && rows_b >= 1) {            // full rounds of whole rows, the rows left over in pieces
             int s = (int)(cus / (rows_b * sh));
             s = s > tiles / 4 ? tiles / 4 : s;
             while (s >= 2 && partial_bytes(rows_b, s) > pl.scratch_bytes) --s;
-            if (s >= 2) take((double)full * (slice_round_us(1) + 7.0) + slice_round_us(s) + slice_tail_us(rows_b, s), s, 8 * full * per_round);
+            if (s >= 2) take((double)full * (slice_round_us(1, cus) + 7.0) + slice_round_us(s, cus) + slice_tail_us(rows_b, s), s, 8 * full * per_round);
         }
     }
     pl.part_o_bytes = pl.part_ml_bytes = 0;
@@ -483,7 +486,7 @@ extern "C" {
 
 const char *pto_last_error(void) { return g_err; }
 
-const char *pto_version(void) { return "0.7.0"; }
+const char *pto_version(void) { return "0.8.0"; }
 
 int pto_abi_revision(void) { return PTO_ABI_REVISION; }
 
