@@ -90,6 +90,8 @@ hipError_t prolog_prefill_launch(const MlapParams *pm, const LipParams *pl, hipS
         hipLaunchKernelGGL(prolog_small_kernel, dim3((unsigned)(mla + lip + tok)), dim3(256), 0, stream, m, p, mla, lip);
         return hipGetLastError();
     }
+    // Up to 64 tokens the attention query's tiles have 64 (in tiles of 128, half and more of them padding: fused prolog 33 tokens 41.4
+    // us per pass, now 40.6, 48: 43.3 and 42.4, 64: 44.6 and 43.6; MLA prolog alone 33: 35.9 and 34.1, 64: 39.9 and 38.7).
     // 256-token tiles take 12 % less time per (padded) token than 128-token ones where both fill the chip, which up to 256
     // tokens they do not (256 tokens: 79.6 us per pass against 77.5; 600: 150.4 against 140.3; 1000: 188.5 against 206.6)
     const bool small = T <= 256 || 100 * ((T + 127) / 128) <= 176 * ((T + 255) / 256);
@@ -105,7 +107,8 @@ hipError_t prolog_prefill_launch(const MlapParams *pm, const LipParams *pl, hipS
     const int tok_wgs = pl ? (T + FINT_WAVES - 1) / FINT_WAVES : 0;
     const dim3 g((unsigned)(mla_wgs + lip_wgs + tok_wgs));
     auto run = [&](auto *kernel) { hipLaunchKernelGGL(kernel, g, dim3(256), 0, stream, m, p, mla_wgs, lip_wgs); };
-    if (T < LIP_MFMA_MIN_TOKENS) run(prolog_prefill_kernel<2, 2, 1, true>);
+    if (T < LIP_MFMA_MIN_TOKENS) run(prolog_prefill_kernel<2, 1, 1, true>);
+    else if (T <= PFA_TOK<1>) run(prolog_prefill_kernel<2, 1, 1, false>);
     else if (small) run(prolog_prefill_kernel<2, 2, 1, false>);
     else if (lip_small) run(prolog_prefill_kernel<1, 4, 1, false>);
     else run(prolog_prefill_kernel<1, 4, 2, false>);
