@@ -333,8 +333,8 @@ __global__ __launch_bounds__(64 * MID_WAVES) void mlap_mid_kernel(const MlapPara
 // The same at prefill sizes, a wave per token and latent (waves 2t: the query latent, 2t + 1: the key latent and key rope):
 // no barriers, and the slabs' loads and reductions run side by side in one wave.  (The form above, a workgroup of twelve
 // waves per latent that waits for memory once and meets twice, is all latency once the chip has run out of room for more
-// workgroups: 1000 tokens 22.0 us.  As long as 512 of them have room it is the faster one: 64 tokens 5.4 us and 9.4, fused prolog
-// 64 tokens 47.2 us per pass and 51.0, 128: 54.9 and 57.6, 256: 73.3 and 74.4.)
+// workgroups: 1000 tokens 22.0 us.  As long as 512 of them have room it is the faster one: 64 tokens 5.4 us and 9.4, 256: 8.0 and 9.0;
+// fused prolog, 64 tokens 43.2 us per pass and 47.1, 128: 54.0 and 57.2, 256: 70.6 and 72.3, but 300: 97.8 and 96.1.)
 constexpr int MIDP_WAVES = 4;
 constexpr int MIDP_MIN_TOKENS = 257;
 
@@ -550,8 +550,8 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
         // Up to 128 tokens one int8 value of a token's latent that falls the other way is 9 % of its indexer query, so that the
         // ranges, which the order of the sums depends on, stay what they are (12 ranges at 100 tokens: 53.1 and alone 47.4; 14: 52.4
         // and 49.9).  Up to 64 two workgroups share a compute unit, and the fixed-order sums start first (one per compute unit, those
-        // last, so a second round: 9 tokens 39.1, now 32.2; 32: 42.5 and 36.4; 48: 47.3 and 43.3; 64: 52.9 and 44.8; two ranges per
-        // workgroup: 9 tokens 33.5, 32: 37.0, 48: 47.1, 64: 52.5).
+        // last, so a second round: 9 tokens 39.1, in this form 32.2; 32: 42.5, 36.4; 48: 47.3, 43.3; 64: 52.9, 44.8, the last launch
+        // in tiles of 128 tokens; two ranges per workgroup: 9 tokens 33.5, 32: 37.0, 48: 47.1, 64: 52.5).
         const int xtiles = big ? (p.T + XB_TOK - 1) / XB_TOK : ttiles;
         const int eighths = xtiles > 1 ? 8 : (p.T <= 192 ? 6 : 5);
         ngroups = !big ? 2 * cus / nslabs : eighths * cus / (8 * mslabs * xtiles);
