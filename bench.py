@@ -86,6 +86,19 @@ def sfa_algorithmic_work(cur_seqs, n_heads=128):
     return byt, flops
 
 
+def attention_plan(C, *shape):
+    """(key splits, kernels) of one attention step over an int8 cache, by the plan of the library C for it."""
+    plan = C.sfa_quant_plan(*shape, 0)
+    heads, splits = plan["heads_per_workgroup"], plan["key_splits"]
+    names = "sfa_slice_kernel<true>" if heads == 64 else f"sfa_decode_kernel<{heads // 32}, true>"
+    if splits > 8:
+        names += f" + sfa_combine_wide_kernel<{4 if splits <= 16 else 8}>"
+    elif splits > 1:
+        in_flight, f32 = 2 if splits <= 2 else 4 if splits <= 4 else 8, plan["partial_element_bytes"] == 4
+        names += f" + sfa_combine_kernel<{in_flight}, {str(f32).lower()}>"
+    return splits, names
+
+
 def indexer_algorithmic_bytes(lengths, k_scale_bytes, k=2048):
     """Per query token over L keys: L*(128 + scale) + 64*128 query + 64*(scale+weight) + 4 per page + k*4 out."""
     return sum(L * (128 + k_scale_bytes) + 64 * 128 + 64 * 8 + 4 * math.ceil(L / 128) + k * 4 for L in lengths)
@@ -489,8 +502,8 @@ def main():
     from pypto_amd import _native
     C = _native.load()
     lib_version = C.version()
-    # the library's plan for this workload on 256 compute units: 64 heads and a quarter of the keys per workgroup, then a merge
-    key_splits = 4
+    key_splits, kernels = attention_plan(C, B, S1, NQ, 1, K, 128, int(sfa_d.block_table.shape[1]), int(sfa_d.key_nope_2d.shape[0]),
+                                         float(sfa.softmax_scale))
     achieved_tflops = flops / (ev_avg_ms * 1e-3) / 1e12
     achieved_gbs = byt / (ev_avg_ms * 1e-3) / 1e9
 
@@ -620,7 +633,7 @@ def main():
                      "frac": achieved_tflops / PEAK_BF16_TFLOPS,
                      "traffic": measured_traffic(TRAFFIC_FILE, "traffic_bytes_per_step", lib_version,
                                                  {"key_splits": key_splits}),
-                     "kernel": f"sfa_slice_kernel<true> + sfa_combine_kernel<{key_splits}, false> (one step)",
+                     "kernel": kernels + " (one step)",
                      "key_splits": key_splits,
                      "launch_ms_avg": ev_avg_ms, "launch_ms_min": ev_min_ms, "launch_ms_avg_unsettled": ev_avg_ms_unsettled,
                      "frac_unsettled": flops / (ev_avg_ms_unsettled * 1e-3) / 1e12 / PEAK_BF16_TFLOPS, "flops_per_launch": flops},

@@ -127,6 +127,19 @@ int pto_sfa_quant_workspace_bytes(const PtoSfaQuantArgs *args, size_t *bytes);
 int pto_sfa_quant_launch(const PtoSfaQuantArgs *args, void *hip_stream);
 
 /*
+ * How pto_sfa_quant_launch divides the work of such a call on the current device (on a host without one: of 256 compute
+ * units), for what times, counts or tests its launches.  No pointer of args is looked at and nothing is launched.
+ */
+typedef struct PtoSfaPlan {
+    int64_t heads_per_workgroup;   /* 32, 64 or 128 */
+    int64_t key_splits;            /* workgroups that share a split row's keys; 1: no row is split */
+    int64_t whole_rows;            /* rows at the front that are not split where the others are */
+    int64_t partial_element_bytes; /* 2 (fp16), 4 (fp32) or, where no row is split, 0 */
+    size_t partial_bytes;          /* what the partial results take of the workspace: at most what is asked for */
+} PtoSfaPlan;
+int pto_sfa_quant_plan(const PtoSfaQuantArgs *args, PtoSfaPlan *plan);
+
+/*
  * pto_sfa_quant_launch for callers that cannot allocate device memory (code under
  * HIP graph capture, serving loops, harnesses that forbid hipMalloc): it has no
  * counterpart in the reference.  The partial results of the key splits go to an
@@ -135,8 +148,8 @@ int pto_sfa_quant_launch(const PtoSfaQuantArgs *args, void *hip_stream);
  * are ignored.  Nothing is allocated or freed; the first call on a device looks
  * the array's device address up.  With num_splits = 0 the library takes the best
  * split count whose partial results fit the array (the decode shapes this library
- * is benchmarked on fit as they are: 32 rows x 8 splits and 128 rows x 2 splits of
- * 128 heads take 33.8 MB).  An explicit num_splits, or a top-k past what one
+ * is benchmarked on fit as they are: 32 rows and 128 rows of 128 heads ask for
+ * 33.8 MB).  An explicit num_splits, or a top-k past what one
  * workgroup holds, whose splits need more than the array holds is refused with
  * PTO_E_WORKSPACE.
  * All calls on one GPU share the array: calls whose execution may overlap (two

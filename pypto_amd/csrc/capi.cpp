@@ -500,6 +500,20 @@ int pto_sfa_quant_workspace_bytes(const PtoSfaQuantArgs *a, size_t *bytes)
     return PTO_OK;
 }
 
+int pto_sfa_quant_plan(const PtoSfaQuantArgs *a, PtoSfaPlan *plan)
+{
+    if (!plan) return fail(PTO_E_INVALID_ARG, "sfa: plan is NULL");
+    int rc = sfa_check(a);
+    if (rc != PTO_OK) return rc;
+    const SfaPlan pl = sfa_plan(a);
+    plan->heads_per_workgroup = 32 * pl.head_groups;
+    plan->key_splits = pl.nsplit;
+    plan->whole_rows = pl.nsplit > 1 ? 8 * (int64_t)pl.whole_slots : 0;
+    plan->partial_element_bytes = pl.nsplit > 1 ? (pl.part_f32 ? 4 : 2) : 0;
+    plan->partial_bytes = pl.part_o_bytes + pl.part_ml_bytes;
+    return PTO_OK;
+}
+
 int pto_sfa_quant_launch(const PtoSfaQuantArgs *a, void *hip_stream)
 {
     int rc = sfa_check(a);

@@ -113,6 +113,21 @@ PYBIND11_MODULE(_C, m)
               check(pto_sfa_quant_workspace_bytes(&a, &bytes));
               return bytes;
           });
+    m.def("sfa_quant_plan",
+          [](int64_t b, int64_t s1, int64_t nq, int64_t n_kv, int64_t topk, int64_t block_size,
+             int64_t max_blocknum_perbatch, int64_t kv_rows, double softmax_scale, int num_splits) {
+              PtoSfaQuantArgs a = sfa_args(0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, b, s1, nq, n_kv, topk, block_size,
+                                           max_blocknum_perbatch, kv_rows, softmax_scale, num_splits);
+              PtoSfaPlan plan{};
+              check(pto_sfa_quant_plan(&a, &plan));
+              py::dict d;
+              d["heads_per_workgroup"] = plan.heads_per_workgroup;
+              d["key_splits"] = plan.key_splits;
+              d["whole_rows"] = plan.whole_rows;
+              d["partial_element_bytes"] = plan.partial_element_bytes;
+              d["partial_bytes"] = plan.partial_bytes;
+              return d;
+          });
     m.def("sfa_quant_launch",
           [](std::uintptr_t query_nope, std::uintptr_t query_rope, std::uintptr_t key_nope_2d, std::uintptr_t key_rope_2d,
              std::uintptr_t k_nope_scales, std::uintptr_t topk_indices, std::uintptr_t block_table,

@@ -184,3 +184,37 @@ def test_attention_launches_without_half_precision_partials(nq, topk, rows):
 def test_attention_launches_with_half_precision_partials(nq, topk, rows, splits):
     from pypto_amd import _C
     assert _C.sfa_quant_workspace_bytes(rows, 1, nq, 1, topk, 128, 512, 1 << 30, 0.04, 0) == rows * splits * nq * (512 * 2 + 8)
+
+
+def attention_plan(rows, nq, topk, splits=0):
+    from pypto_amd import _C
+    args = (rows, 1, nq, 1, topk, 128, 512, 1 << 30, 0.04, splits)
+    return _C.sfa_quant_plan(*args), _C.sfa_quant_workspace_bytes(*args)
+
+
+@pytest.mark.parametrize("nq", [1, 16, 33, 64, 100, 128, 192])
+@pytest.mark.parametrize("topk", [1, 32, 200, 256, 768, 2048, 2049, 4096])
+def test_attention_plan_stays_within_the_bytes_a_caller_is_asked_for(nq, topk):
+    """A launch checks the workspace against the bytes asked for; what its plan lays out there is never more."""
+    for rows in [*range(1, 80), 127, 128, 129, 168, 200, 255, 256, 257, 283, 300, 513, 4096]:
+        plan, need = attention_plan(rows, nq, topk)
+        assert plan["heads_per_workgroup"] in (32, 64, 128) and 1 <= plan["key_splits"] <= (topk + 31) // 32
+        assert plan["key_splits"] * 2048 >= topk, rows                     # a split's keys fit a workgroup
+        split_rows = rows - plan["whole_rows"] if plan["key_splits"] > 1 else 0
+        assert plan["partial_bytes"] == split_rows * plan["key_splits"] * nq * (512 * plan["partial_element_bytes"] + 8) <= need, rows
+        assert plan["partial_element_bytes"] != 4 or plan["key_splits"] <= 8, rows
+
+
+@pytest.mark.parametrize("heads,splits,element,names", [
+    (64, 4, 2, "sfa_slice_kernel<true> + sfa_combine_kernel<4, false>"), (128, 1, 0, "sfa_decode_kernel<4, true>"),
+    (128, 7, 2, "sfa_decode_kernel<4, true> + sfa_combine_kernel<8, false>"), (32, 2, 4, "sfa_decode_kernel<1, true> + sfa_combine_kernel<2, true>"),
+    (64, 9, 2, "sfa_slice_kernel<true> + sfa_combine_wide_kernel<4>"), (32, 22, 2, "sfa_decode_kernel<1, true> + sfa_combine_wide_kernel<8>")])
+def test_benchmark_follows_the_plan_of_the_library(heads, splits, element, names):
+    """Split count and kernels in the benchmark's line are those of the plan, whatever it is: counter figures taken with another
+    one are then recognised as stale."""
+    from types import SimpleNamespace
+    import bench
+    plan = dict(heads_per_workgroup=heads, key_splits=splits, whole_rows=0, partial_element_bytes=element, partial_bytes=0)
+    assert bench.attention_plan(SimpleNamespace(sfa_quant_plan=lambda *a: plan), 32, 1) == (splits, names)
+    from pypto_amd import _C
+    assert bench.attention_plan(_C, 32, 1, 128, 1, 2048, 128, 512, 1 << 21, 0.04)[0] == _C.sfa_quant_plan(32, 1, 128, 1, 2048, 128, 512, 1 << 21, 0.04, 0)["key_splits"]
