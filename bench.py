@@ -24,8 +24,9 @@ timed region.  Prints ONE JSON line:
   cpu_baseline   the scalar C statement of the golden, all host threads, on a bounded sample of the
                  same batch; beside it the torch golden at configs[0] in its literal loop form and vectorised
 
-To keep a step from being served out of the 256 MB memory-side cache, steps rotate over ROT
-different selections (different indexer queries over the same caches).
+To keep a step from being served out of the 256 MB memory-side cache, attention steps rotate over ROT
+different selections (different indexer queries over the same caches), indexer passes over copies of their
+key cache, prolog passes over copies of their weights.
 """
 from __future__ import annotations
 
@@ -43,8 +44,9 @@ if ROOT not in sys.path:
 PEAK_BF16_TFLOPS = 2500.0
 PEAK_HBM_GBS = 8000.0
 ROT = 8
-SETTLE_STEPS = 1000   # untimed attention steps ahead of the caller's warm-up: about 40 ms of load, see main()
+SETTLE_STEPS = 1000   # untimed steps ahead of the timed ones (attention: of the caller's warm-up): 20 to 60 ms of load, see main()
 COPY_MIB = 256
+MEMORY_SIDE_CACHE = 256 << 20
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "sfa_decode_cfg2_hbm_traffic.md")
 LI_TRAFFIC_FILE = os.path.join(ROOT, "profiles", "indexer_hbm_traffic.md")
 
@@ -102,6 +104,13 @@ def attention_plan(C, *shape):
 def indexer_algorithmic_bytes(lengths, k_scale_bytes, k=2048):
     """Per query token over L keys: L*(128 + scale) + 64*128 query + 64*(scale+weight) + 4 per page + k*4 out."""
     return sum(L * (128 + k_scale_bytes) + 64 * 128 + 64 * 8 + 4 * math.ceil(L / 128) + k * 4 for L in lengths)
+
+
+def key_sets(cache, scale):
+    """An indexer's key cache and copies of it, enough of them that between two passes over one at least twice the memory-side
+    cache goes by, as in a decode step, where the other layers' caches and weights do."""
+    one = cache.numel() * cache.element_size() + scale.numel() * scale.element_size()
+    return [(cache, scale)] + [(cache.clone(), scale.clone()) for _ in range(-(-2 * MEMORY_SIDE_CACHE // one))]
 
 
 def time_events(fn, steps, warmup, torch):
@@ -524,38 +533,39 @@ def main():
     packed_same = bool(torch.equal(out.view(torch.int16), out_p.view(torch.int16)))
     del packed
 
-    # ------------------------------------------------------------------ indexer timings
+    # ------------------------------------------------------------------ indexer timings (at settled clocks too)
     res = torch.empty([B, 1, K], dtype=torch.int32, device=dev)
+    keys2 = key_sets(li_d.idx_key_cache, li_d.idx_key_scale)
 
     def li_step(i):
-        pypto_amd.lightning_indexer_decode(idx_queries[i % ROT], li_d.idx_query_scale, li_d.idx_key_cache,
-                                           li_d.idx_key_scale, li_d.idx_weight, li_d.act_seq_key, li_d.block_table,
-                                           res, None, None, K)
-    li2_avg_ms = time_batch(li_step, max(args.steps // 2, 40), 20, torch)
+        pypto_amd.lightning_indexer_decode(idx_queries[i % ROT], li_d.idx_query_scale, *keys2[i % len(keys2)], li_d.idx_weight,
+                                           li_d.act_seq_key, li_d.block_table, res, None, None, K)
+    li2_avg_ms = time_batch(li_step, max(args.steps // 2, 40), SETTLE_STEPS, torch)
     li2_bytes = indexer_algorithmic_bytes(lengths, 4)
+    del keys2
 
     li1 = gen_indexer_inputs(4, 1, config_lengths(1), selected_count=K, seed=1, variant="fp32").to(dev)
+    keys1 = key_sets(li1.idx_key_cache, li1.idx_key_scale)
 
     def li1_step(i):
-        pypto_amd.lightning_indexer_decode(li1.idx_query, li1.idx_query_scale, li1.idx_key_cache, li1.idx_key_scale,
-                                           li1.idx_weight, li1.act_seq_key, li1.block_table, li1.topk_res, None, None,
-                                           K)
-    li1_avg_ms = time_batch(li1_step, max(args.steps // 2, 40), 20, torch)
+        pypto_amd.lightning_indexer_decode(li1.idx_query, li1.idx_query_scale, *keys1[i % len(keys1)], li1.idx_weight,
+                                           li1.act_seq_key, li1.block_table, li1.topk_res, None, None, K)
+    li1_avg_ms = time_batch(li1_step, max(args.steps // 2, 40), SETTLE_STEPS, torch)
     li1_bytes = indexer_algorithmic_bytes(config_lengths(1), 4)
-    del li1
+    del li1, keys1
 
     # configs[3]'s indexer: B=64, two query tokens per sequence (the pair shares one pass over the keys)
     len3 = config_lengths(3, seed=3)
     li3 = gen_indexer_inputs(64, 2, len3, selected_count=K, seed=3, variant="fp32").to(dev)
+    keys3 = key_sets(li3.idx_key_cache, li3.idx_key_scale)
 
     def li3_step(i):
-        pypto_amd.lightning_indexer_decode(li3.idx_query, li3.idx_query_scale, li3.idx_key_cache, li3.idx_key_scale,
-                                           li3.idx_weight, li3.act_seq_key, li3.block_table, li3.topk_res, None, None,
-                                           K)
-    li3_avg_ms = time_batch(li3_step, max(args.steps // 4, 20), 10, torch)
+        pypto_amd.lightning_indexer_decode(li3.idx_query, li3.idx_query_scale, *keys3[i % len(keys3)], li3.idx_weight,
+                                           li3.act_seq_key, li3.block_table, li3.topk_res, None, None, K)
+    li3_avg_ms = time_batch(li3_step, max(args.steps // 4, 20), SETTLE_STEPS, torch)
     # per sequence: the keys once, two tokens' queries, factors and results
     li3_bytes = sum(L * (128 + 4) + 2 * (64 * 128 + 64 * 8 + K * 4) + 4 * math.ceil(L / 128) for L in len3)
-    del li3
+    del li3, keys3
 
     # ------------------------------------------------------------------ indexer prolog (projection stage)
     # the side legs must not cost the headline line: a failure there is reported in its field

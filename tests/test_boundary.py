@@ -218,3 +218,13 @@ def test_benchmark_follows_the_plan_of_the_library(heads, splits, element, names
     assert bench.attention_plan(SimpleNamespace(sfa_quant_plan=lambda *a: plan), 32, 1) == (splits, names)
     from pypto_amd import _C
     assert bench.attention_plan(_C, 32, 1, 128, 1, 2048, 128, 512, 1 << 21, 0.04)[0] == _C.sfa_quant_plan(32, 1, 128, 1, 2048, 128, 512, 1 << 21, 0.04, 0)["key_splits"]
+
+
+@pytest.mark.parametrize("pages", [1024, 8615, 40000])
+def test_benchmark_times_the_indexer_over_keys_that_are_in_no_cache(pages):
+    """Between two passes over one copy of the keys the benchmark reads more than the memory-side cache holds."""
+    import bench
+    sets = bench.key_sets(torch.empty([pages, 128, 1, 128], dtype=torch.int8, device="meta"), torch.empty([pages, 128, 1], device="meta"))
+    one = pages * 128 * (128 + 4)
+    assert all(k.shape == sets[0][0].shape and s.shape == sets[0][1].shape for k, s in sets)
+    assert bench.MEMORY_SIDE_CACHE == 256 << 20 and 2 * bench.MEMORY_SIDE_CACHE <= (len(sets) - 1) * one <= 2 * bench.MEMORY_SIDE_CACHE + one
