@@ -543,18 +543,19 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
         // every slab but the last, the rope columns, which keep their fixed-order sums
         const int mslabs = nslabs - 1;
         const bool big = p.T > XM_TOK;       // 130 tokens: 60.9 us per pass, 66.7 with tiles of 128; 1500: 282 and 293; 4096: 700 and 724
-        // Tiles of 256 tokens: as many ranges as make this many workgroups, in eighths of the compute units.  The rest of the chip
-        // is for the fixed-order sums, and what does not fit beside them runs as a second round, nearly empty and as long as the
-        // first.  (Fused prolog: 192 tokens, 14 ranges 72.9 us per pass, 12: 68.9; 256: 14 ranges 77.8, 10: 72.2 (alone 61.7 and
-        // 62.6); 400: 8 ranges 106.5, 6: 101.6, but alone, which has the same ranges to give the same bits, 77.2 and 80.7.)
-        // Up to 128 tokens one int8 value of a token's latent that falls the other way is 9 % of its indexer query, so that the
-        // ranges, which the order of the sums depends on, stay what they are (12 ranges at 100 tokens: 53.1 and alone 47.4; 14: 52.4
-        // and 49.9).  Up to 64 two workgroups share a compute unit, and the fixed-order sums start first (one per compute unit, those
+        // As many ranges as make two workgroups of 128 tokens or one of 256 per compute unit (the other half of each is for the
+        // fixed-order sums), MLAP_XM_MAX_SPLITS = 14 at most: that many up to 256 tokens, so that a token's latents do not depend
+        // on how many tokens the launch has.  Fewer ranges are longer fp32 chains, further from the 64-bit sums (relative error
+        // over 2048 columns of 7168 products: 14 ranges 1.44e-7, 12 1.52e-7, 10 1.63e-7, 8 1.80e-7), and one int8 value of a
+        // latent that falls the other way is 9 % of its token's indexer query.  They would leave the fixed-order sums more room
+        // beside them: fused prolog, 14 / 12 ranges: 129 tokens 60.0 / 60.5 us per pass, 192: 71.1 / 67.5; 14 / 10: 256 76.9 / 71.4
+        // (alone 61.1 / 62.5); 14 / 12: 100 52.4 / 53.1 (alone 49.9 / 47.4).  At 256 tokens the fourteen as two to a workgroup, one
+        // after the other, take 84.0, with the fixed-order sums first 83.7.
+        // Up to 64 tokens two workgroups share a compute unit, and the fixed-order sums start first (one per compute unit, those
         // last, so a second round: 9 tokens 39.1, in this form 32.2; 32: 42.5, 36.4; 48: 47.3, 43.3; 64: 52.9, 44.8, the last launch
         // in tiles of 128 tokens; two ranges per workgroup: 9 tokens 33.5, 32: 37.0, 48: 47.1, 64: 52.5).
         const int xtiles = big ? (p.T + XB_TOK - 1) / XB_TOK : ttiles;
-        const int eighths = xtiles > 1 ? 8 : (p.T <= 192 ? 6 : 5);
-        ngroups = !big ? 2 * cus / nslabs : eighths * cus / (8 * mslabs * xtiles);
+        ngroups = big ? cus / (mslabs * xtiles) : 2 * cus / nslabs;
         ngroups = ngroups < 1 ? 1 : ngroups;
         ngroups = ngroups > MLAP_XM_MAX_SPLITS ? MLAP_XM_MAX_SPLITS : ngroups;
         ngroups = ngroups > nchunks ? nchunks : ngroups;
