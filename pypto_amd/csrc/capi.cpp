@@ -135,12 +135,16 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
     };
     // The schedule model, in microseconds: what a launch pair over an int8 cache took over 1 to 128 rows x 16 to 128 heads x 1 to
     // 64 splits (fitted to within 10 %; neighbouring choices differ by less).  The same figures serve the other cache formats
-    // and every top-k: against the fastest of all head-group and split counts, both caches, 1 to 300 rows, 16 to 128 heads, the
-    // choice is within 5 % for top-k 1024 and 2048 but for a single row (up to 11 %, 64 splits where 32 are faster).  A compute unit holds one workgroup; a round of them
+    // and every top-k.  A compute unit holds one workgroup; a round of them
     // is as long as a split's tiles; starting, staging the query and the first tile and the merge launch are `fixed`, and
     // the partial results cost with the number of workgroups that write them.  Fewer head groups per workgroup make
     // a tile shorter, and the prologue, but the tiles of a row are de-quantised once per workgroup: that pays while the
     // chip is not full (128 heads, 1 row: 22.0 us as 16 splits of four groups, 14.3 as 32 splits of one; 4 rows: 22.5, 20.0).
+    // Two groups are priced as the form of four waves they had when the bytes a caller is asked for were settled (1.58 a tile,
+    // where sfa_slice_kernel takes 1.1 to 1.45): up to 2048 keys that price chooses nothing, the second model below does.  Beyond,
+    // where it is not asked, the choice is within 6 % of the fastest division from 64 rows on (128 heads; 64 heads: from 16 on)
+    // and dear for fewer (4096 keys of an int8 cache, 128 heads: 1 row 19.0 where 32 splits of 64 heads take 16.1, 4 rows 27.1 and
+    // 22.9, 16 rows 36.7 and 33.0).
     auto round_us = [&](const int hg, const int ns) { return (tiles + ns - 1) / ns * (hg == 4 ? 1.75 : (hg == 2 ? 1.58 : 1.47)); };
     auto tail_us = [&](const int hg, const long long wgs, const int ns) {
         if (ns == 1) return 6.0;
@@ -234,6 +238,10 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
     // 35.0, 28.6, 20.0 and 14.1 as four groups and one group of 32 heads; 36 to 64 rows alike; 128 rows 97.1 against 95.0).
     // A tile of whole rows takes 1.13 with 128 workgroups, 1.2 with 192 and 1.45 with 256 (top-k 1024, 96 rows: 44.9, as four groups
     // and two splits 49.4); partial results past one round's cost more (64 heads, 96 rows: 5 splits 58.8, 2 splits 51.8).
+    // Against the fastest of every form and split count, two rows and more, top-k 1024 and 2048, both caches, the choice is within
+    // 5 % in 104 of 108 shapes.  Where it is not: 128 rows of 128 heads over 1024 keys are priced 50.0 as two splits of four groups and
+    // 52.4 as whole rows of this form, and take 57.4 and 54.3 (bf16 cache 58.3 and 50.6).  A single row's 32 splits are priced 14.5
+    // and its 22 splits 14.1, and take 13.5 and 14.2.
     if (a->nq > 32 && a->num_splits == 0 && min_split == 1) {
         const int sh = shares(2);
         if (pl.head_groups == 2) best = -1.0;             // (two groups of 32 heads: that is this form, at another price)

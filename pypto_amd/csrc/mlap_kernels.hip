@@ -205,9 +205,10 @@ __device__ __forceinline__ float slab_square_sum(const float v0, const float v1,
 // idles.  Further workgroups of the launch, one per head, ask for the first rows of the head's projection weights, which the last
 // launch, bound by drawing weights, then finds in the L2 of the XCD it reads them on (workgroups go round the XCDs in both
 // launches, prolog_small_head).  The values are dropped.  512 rows are what arrives before the latents are done: fused prolog, 0 /
-// 256 / 512 / 768 rows: 8 tokens 34.6 / 33.6 / 32.9 / 33.6 us per pass, 32: 37.0 / 36.0 / 35.7 / 36.6; MLA prolog alone, 0 / 512:
-// 29.3 / 28.7 and 31.4 / 30.3.  Into the L2 of another XCD, so that only the memory-side cache helps: 8 tokens 34.4.  (The launch
-// for more than 32 tokens has two workgroups per compute unit to hide the same latencies: 48 tokens 42.6 / 42.8, 200: 68.3 / 68.4.)
+// 256 / 512 / 768 rows: 8 tokens 34.1 / 33.2 / 32.4 / 32.1 us per pass, 16: 35.3 / 34.3 / 33.4 / 33.6, 32: 38.1 / 37.2 / 36.5 / 36.6;
+// MLA prolog alone, 0 / 512: 8 tokens 27.9 / 27.4, 32: 31.1 / 29.9.  Into the L2 of another XCD, so that only the memory-side cache
+// helps, 8 tokens gain 0.3 us instead of 1.7.  (The launch for more than 32 tokens has two workgroups per compute unit to hide the
+// same latencies, and gained nothing at 48 and 200.)
 constexpr int MLAP_AHEAD_ROWS = 512;
 __device__ __forceinline__ void mlap_ask_ahead(const MlapParams &p, const int wg)
 {

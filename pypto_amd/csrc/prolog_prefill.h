@@ -297,8 +297,9 @@ __device__ __forceinline__ void mlap_prefill_body(const MlapParams &p, const int
 // read is the accumulators' row order).  Weights: [head][64][128] per chunk, as q_build_a_tr reads them.  The matrix is
 // requested once the chunk buffers are free: row r at 256 * r, 16-byte piece q at q ^ 4*(r & 3).
 // FIXED (one tile of at most 64 tokens, the first two waves' blocks): the rotated rows meet in LDS and all four waves take the
-// Hadamard sums in their fixed order, a block of 32 rows at a time.  (Fused prolog, 48
-// tokens: 46.9 us per pass; in the cores' own order, which the interface does not allow below 64 tokens, 46.3.)
+// Hadamard sums in their fixed order, a block of 32 rows at a time.  (Fused prolog, 33
+// tokens: 40.7 us per pass, 48: 42.4, 63: 43.7; in the cores' own order, which the interface does not allow below 64 tokens, 40.5,
+// 42.4 and 43.2.)
 template <int TB> constexpr int PFI_TOK = 128 * TB;
 template <int XC, int TB> constexpr int PFI_X = PFI_TOK<TB> * PF_XPITCH<XC>;
 constexpr int PFI_W = PF_KC * LIP_DIM;

@@ -5,7 +5,7 @@
 // sixteen rows at a time.  Bound: memory, 54 MB in 10 us behind the first 2 (another 13 MB are in the L2: mlap_ask_ahead).  With
 // every chunk out of the L2 (timing only) an attention workgroup takes 8.1 us at 8 tokens and 9.0 at 32 instead of 13; with one
 // chunk between barriers, six blocks of columns as 2, 2, 1, 1 over the waves and 60 KiB on their way it took 9.6 and 10.8 (fused
-// prolog 8 tokens 33.0 us per pass, now 32.7, 32: 35.5 and 35.0).  (8 tokens as two launches with partial sums in between: 6 us
+// prolog 8 tokens 32.6 us per pass, now 32.4, 16: 33.7 and 33.4, 32: 37.1 and 36.5).  (8 tokens as two launches with partial sums in between: 6 us
 // more.)
 // Included by prolog_fused.hip after prolog_prefill.h.
 #pragma once
