@@ -14,7 +14,7 @@ timed region.  Prints ONE JSON line:
                  "roofline_hbm" because the shape sits at the ridge of the two
   packed_cache   the same step through sparse_attention_antiquant_d (one 656-byte row per key)
   indexer        time of one lightning-indexer pass (score + select) on the same batch, on the
-                 indexer-only configuration (B=4, KV 32768) and on configs[3]'s batch (B=64, two query
+                 indexer-only batch (B=4, KV 32768) and on one with multi-token prediction (B=64, two query
                  tokens per sequence), with its HBM fraction and the counter-derived HBM traffic
   indexer_prolog time of one lightning-indexer prolog pass (projection stage) on the reference's enabled
                  case b=4, s1=2 (8 tokens, h=7168, q_lora_rank=1536), launches replayed from a HIP graph so
@@ -22,7 +22,8 @@ timed region.  Prints ONE JSON line:
   mla_prolog     the same for the MLA prolog (b=4, s=2, 128 heads; 85 MB of weights per pass, ten sets);
                  all three prolog legs also carry "batch_of_32": the same pass at the headline's 32 tokens
   cpu_baseline   the scalar C statement of the golden, all host threads, on a bounded sample of the
-                 same batch; beside it the torch golden at configs[0] in its literal loop form and vectorised
+                 same batch; beside it the torch golden on one sequence of 16 heads, in its literal loop form
+                 and vectorised
 
 To keep a step from being served out of the 256 MB memory-side cache, attention steps rotate over ROT
 different selections (different indexer queries over the same caches), indexer passes over copies of their
@@ -293,14 +294,14 @@ def fused_prolog_leg(torch, dev, pypto_amd, b=4, s1=2, calls=10, replays=10):
 
 
 def other_shapes_leg(torch, pypto_amd, dev):
-    """configs[3] and configs[4] through the same operators (parity of both is a GPU test): step time and the
-    fraction of the dense bf16 peak their algorithmic flops reach.  Row (b, s) attends
+    """64 sequences x 2 query tokens and a prefill chunk of 4096 tokens through the same operators (parity of both is
+    a GPU test): step time and the fraction of the dense bf16 peak their algorithmic flops reach.  Row (b, s) attends
     min(max(act[b] - S1 + 1 + s, 0), 2048) keys."""
     from pypto_amd.synthetic import config_lengths, gen_sfa_inputs
     res = []
     for name, b, s1, lengths, entry, steps in (
-            ("configs[3]: B=64 S_q=2 KV 4096-32768", 64, 2, config_lengths(3, seed=3), "d", 200),
-            ("configs[4]: B=1 S_q=4096 KV 4096 (row t sees min(t+1, 2048) keys)", 1, 4096, config_lengths(4), "p", 20)):
+            ("B=64 S_q=2 KV 4096-32768", 64, 2, config_lengths(3, seed=3), "d", 200),
+            ("B=1 S_q=4096 KV 4096 (row t sees min(t+1, 2048) keys)", 1, 4096, config_lengths(4), "p", 20)):
         inp = gen_sfa_inputs(b, s1, 128, lengths, topk=2048, seed=5).to(dev)
         out = torch.empty([b, s1, 128, 512], dtype=torch.bfloat16, device=dev)
         fn = pypto_amd.sparse_flash_attention_quant_d if entry == "d" else pypto_amd.sparse_flash_attention_quant_p
@@ -352,7 +353,7 @@ def prefill_prologs_leg(torch, pypto_amd, dev):
         return e0.elapsed_time(e1) / n * 1e3
     res = []
     from pypto_amd import mla_prolog_quant_impl as mla_impl
-    # the MLA prolog at the batch of configs[2] (32 sequences, one token each) in both summation modes -- the default
+    # the MLA prolog at the headline's batch (32 sequences, one token each) in both summation modes -- the default
     # takes the prefill forms from 9 tokens on, the exact mode keeps the decode forms up to 63 -- and at 512 tokens
     for b, s1, exact in ((32, 1, False), (32, 1, True), (1, 512, False)):
         d = gen_mla_prolog_inputs(b, s1, [4096] * b, seed=0).to(dev)
@@ -396,7 +397,7 @@ def main():
                          "(the calibration kernel of the counters), no timing, no JSON line")
     ap.add_argument("--seed", type=int, default=2)
     ap.add_argument("--other-shapes", action="store_true",
-                    help="also time configs[3] (B=64, two query tokens) and configs[4] (4096-token prefill chunk) "
+                    help="also time B=64 with two query tokens and a prefill chunk of 4096 tokens "
                          "and add them to the JSON line as 'other_shapes'")
     ap.add_argument("--prefill-prologs", action="store_true",
                     help="also time the MLA prolog at 512 tokens and the indexer prolog at 512 and 4096 tokens "
@@ -450,7 +451,7 @@ def main():
     if args.counter_run:
         for i in range(2 * ROT):
             sfa_step(i)
-        # the indexer on the same batch and on configs[1], for its kernels' counters
+        # the indexer on the same batch and on its own (B=4, KV 32768), for its kernels' counters
         res_c = torch.empty([B, 1, K], dtype=torch.int32, device=dev)
         li1_c = gen_indexer_inputs(4, 1, config_lengths(1), selected_count=K, seed=1, variant="fp32").to(dev)
         for i in range(ROT):
@@ -554,7 +555,7 @@ def main():
     li1_bytes = indexer_algorithmic_bytes(config_lengths(1), 4)
     del li1, keys1
 
-    # configs[3]'s indexer: B=64, two query tokens per sequence (the pair shares one pass over the keys)
+    # multi-token prediction: B=64, two query tokens per sequence (the pair shares one pass over the keys)
     len3 = config_lengths(3, seed=3)
     li3 = gen_indexer_inputs(64, 2, len3, selected_count=K, seed=3, variant="fp32").to(dev)
     keys3 = key_sets(li3.idx_key_cache, li3.idx_key_scale)
@@ -601,7 +602,7 @@ def main():
         cpu = {"value": reps * B / t_cpu, "unit": "tokens/s", "cores": nthreads, "kind": "port",
                "sample": f"the same batch of {B} sequences, {reps} passes of the scalar C golden (OpenMP over "
                          f"heads), {t_cpu:.1f} s"}
-        # configs[0] (B=1, 16 heads, top-k 256, the reference's own CPU-sized case) in the golden's literal form --
+        # the reference's own CPU-sized case (B=1, 16 heads, top-k 256) in the golden's literal form --
         # one Python iteration per selected key, as the reference gathers them
         # (deepseekv32_sparse_flash_attention_quant.py:215-228) -- and in the vectorised torch form of the same golden
         from oracle import sfa_oracle
@@ -618,7 +619,7 @@ def main():
                 t0c += time.perf_counter() - tc
                 n0 += 1
             forms[name] = {"tokens_per_s": n0 / t0c, "ms_per_call": t0c / n0 * 1e3, "calls": n0}
-        cpu["configs[0]_torch_golden"] = {"workload": "configs[0]: B=1 S_q=1 16 heads topk=256 KV 4096", "torch_threads": torch.get_num_threads(), **forms}
+        cpu["torch_golden"] = {"workload": "B=1 S_q=1 16 heads topk=256 KV 4096", "torch_threads": torch.get_num_threads(), **forms}
 
     line = {
         "metric": "sfa_decode_tokens_per_s",
@@ -635,7 +636,7 @@ def main():
         "vs_baseline": None,
         "dtype": "bf16",
         "data": "synthetic",
-        "config": {"workload": "configs[2]: SFA decode B=32 S_q=1 128 heads d=576/512 topk=2048 (from the indexer) "
+        "config": {"workload": "SFA decode B=32 S_q=1 128 heads d=576/512 topk=2048 (from the indexer) "
                                "int8 latent KV + 4 fp32 scales/token + bf16 rope, KV 8192-65536 paged bs=128, "
                                f"shuffled block table, {ROT} rotating selections",
                    "kv_rows": int(sfa.key_nope_2d.shape[0]), "sum_kv_len": int(sum(lengths))},
@@ -651,13 +652,13 @@ def main():
                          "frac": achieved_gbs / PEAK_HBM_GBS, "bytes_per_launch": byt},
         "packed_cache": {"operator": "sparse_attention_antiquant_d", "us_per_step": packed_avg_ms * 1e3,
                          "bit_identical_to_three_array_result": packed_same},
-        "indexer": {"configs[2]_us_per_step": li2_avg_ms * 1e3, "configs[2]_hbm_frac": li2_bytes / (li2_avg_ms * 1e-3) / 1e9 / PEAK_HBM_GBS,
-                    "configs[1]_us_per_step": li1_avg_ms * 1e3, "configs[1]_hbm_frac": li1_bytes / (li1_avg_ms * 1e-3) / 1e9 / PEAK_HBM_GBS,
-                    "bytes_configs[2]": li2_bytes, "bytes_configs[1]": li1_bytes,
-                    "traffic_configs[2]": measured_traffic(LI_TRAFFIC_FILE, "indexer_traffic_bytes_configs2", lib_version),
-                    "traffic_configs[1]": measured_traffic(LI_TRAFFIC_FILE, "indexer_traffic_bytes_configs1", lib_version),
-                    "configs[3]_us_per_step": li3_avg_ms * 1e3,
-                    "configs[3]_hbm_frac": li3_bytes / (li3_avg_ms * 1e-3) / 1e9 / PEAK_HBM_GBS, "bytes_configs[3]": li3_bytes,
+        "indexer": {"b32_us_per_step": li2_avg_ms * 1e3, "b32_hbm_frac": li2_bytes / (li2_avg_ms * 1e-3) / 1e9 / PEAK_HBM_GBS,
+                    "b4_us_per_step": li1_avg_ms * 1e3, "b4_hbm_frac": li1_bytes / (li1_avg_ms * 1e-3) / 1e9 / PEAK_HBM_GBS,
+                    "bytes_b32": li2_bytes, "bytes_b4": li1_bytes,
+                    "traffic_b32": measured_traffic(LI_TRAFFIC_FILE, "indexer_traffic_bytes_b32", lib_version),
+                    "traffic_b4": measured_traffic(LI_TRAFFIC_FILE, "indexer_traffic_bytes_b4", lib_version),
+                    "b64x2_us_per_step": li3_avg_ms * 1e3,
+                    "b64x2_hbm_frac": li3_bytes / (li3_avg_ms * 1e-3) / 1e9 / PEAK_HBM_GBS, "bytes_b64x2": li3_bytes,
                     "scale_dtype": "fp32", "weight_dtype": "bf16"},
         "indexer_prolog": prolog,
         "mla_prolog": mla_prolog,
