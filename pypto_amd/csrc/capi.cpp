@@ -494,7 +494,7 @@ extern "C" {
 
 const char *pto_last_error(void) { return g_err; }
 
-const char *pto_version(void) { return "0.8.0"; }
+const char *pto_version(void) { return "0.8.1"; }
 
 int pto_abi_revision(void) { return PTO_ABI_REVISION; }
 
