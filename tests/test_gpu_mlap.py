@@ -175,8 +175,8 @@ def test_mla_prolog_prefill_t512_matrix_core_sums_default():
 
 @pytest.mark.parametrize("t", [9, 32, 33, 64, 65, 128, 129, 192, 193, 256, 257])
 def test_mla_prolog_matrix_core_sums_at_the_edges_of_the_range_counts(t):
-    """The hidden axis is divided into as many ranges as the token count asks for: both sides of every line, at the model's
-    hidden size and query rank, against the launches that keep every sum in its fixed order."""
+    """The sums over the hidden axis have four forms by the token count, fourteen ranges up to 256 tokens and fewer beyond: both
+    sides of every line, at the model's hidden size and query rank, against the launches that keep every sum in its fixed order."""
     from pypto_amd import mla_prolog_quant_impl as impl
     inp = gen_mla_prolog_inputs(1, t, [t], seed=t, n_heads=2)
     ref = run_op(inp, (1e-5, 1e-5), prefill=True)
