@@ -41,24 +41,19 @@ namespace pto {
 namespace {
 
 
-__device__ __forceinline__ float load_scalar(const void *p, size_t i, int dt)
+// one scale or weight as it lies in memory, and its value: the conversion apart, so that several loads are on their way at once
+__device__ __forceinline__ uint32_t load_raw(const void *p, const size_t i, const int dt)
 {
-    if (dt == PTO_DT_FP32) return static_cast<const float *>(p)[i];
-    const uint16_t h = static_cast<const uint16_t *>(p)[i];
-    if (dt == PTO_DT_BF16) return bf16_bits_to_f32(h);
-    return (float)__builtin_bit_cast(_Float16, h);
+    return dt == PTO_DT_FP32 ? static_cast<const uint32_t *>(p)[i] : static_cast<const uint16_t *>(p)[i];
+}
+__device__ __forceinline__ float raw_to_f32(const uint32_t raw, const int dt)
+{
+    if (dt == PTO_DT_FP32) return __uint_as_float(raw);
+    return dt == PTO_DT_BF16 ? bf16_bits_to_f32((uint16_t)raw) : (float)__builtin_bit_cast(_Float16, (uint16_t)raw);
 }
 
-// w_scale[h] = fp16(q_scale * weight) when both are fp16 (one fp16 rounding of the exact product),
-// else the fp32 product
-__device__ __forceinline__ float w_scale_of(const LiParams &p, const size_t i)
-{
-    const float qs = load_scalar(p.q_scale, i, p.q_dt);
-    const float wt = load_scalar(p.weight, i, p.w_dt);
-    float prod = __fmul_rn(qs, wt);
-    if (p.q_dt == PTO_DT_FP16 && p.w_dt == PTO_DT_FP16) prod = (float)(_Float16)prod;
-    return prod;
-}
+// n / d for n < 2^18 and inv = 1 / d to one unit in the last place: (n + 1/2) / d is no nearer to an integer than 1 / (2 d)
+__device__ __forceinline__ int small_quotient(const int n, const float inv) { return (int)(((float)n + 0.5f) * inv); }
 
 // order-preserving image of a score: larger score <=> larger key; -0.0 and +0.0 map to one key
 __device__ __forceinline__ uint32_t score_key(const float x)
@@ -254,74 +249,117 @@ constexpr int SC_BUF_BYTES = SC_PAIR_BYTES + 256;   // + the 64 key scales (one 
 // a batch against a page in one matrix product (lightning_indexer_quant_impl.py:163-169, [S1*64, 128]); here
 // a "unit" is a pair of consecutive tokens of a sequence (the last unit of an odd s1 holds one), every staged
 // key row and scale serves both, and their per-head factors sit in LDS instead of scalar registers.
+// A workgroup of eight waves per compute unit, and nothing in front of the first requests that need not be there: as two workgroups of
+// four the second one's sequence lengths came back behind the first one's key rows (7 us, and it ended as much later), the
+// mapping took 2.3 us of divisions, and the queries, asked for behind two pairs of every wave, arrived behind 34 MB.  Kernel over
+// rotating key caches, before / now: 4 tokens x 32 K keys 10.5 / 6.8 us, 32 x 8-64 K 36.9 / 35.6, 64 pairs of tokens x 4-32 K 44.8 / 40.5.
 // HW: query scales and weights are fp16, so the per-head factors are fp16 values, their products with x exact and the head
 // sum one instruction per head instead of two; the factors sit in scalar registers as packed pairs, for two tokens as well.
 template <int KDT, int VAR = 0, int NT = 1, bool HW = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void li_score_kernel(const LiParams p)
+__global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void li_score_kernel(const LiParams p)
 {
-    __shared__ __attribute__((aligned(16))) int8_t kstage[4][2][SC_BUF_BYTES];
-    __shared__ __attribute__((aligned(16))) float wsc_lds[NT > 1 && !HW ? 4 : 1][NT][LI_HEADS];
+    __shared__ __attribute__((aligned(16))) int8_t kstage[LI_SCORE_WAVES][2][SC_BUF_BYTES];
+    __shared__ __attribute__((aligned(16))) float wsc_lds[NT > 1 && !HW ? LI_SCORE_WAVES : 1][NT][LI_HEADS];
+    static_assert(SC_PAIR_BYTES == LI_HEADS * LI_DIM, "a token's query is staged where a pair of key blocks goes later");
     const int upb = (p.S1 + NT - 1) / NT;            // units per sequence
     const int nunits = p.B * upb;
-    const int w = threadIdx.x >> 6;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l = threadIdx.x & 63;
     const int j = l & 31;
     const int half = l >> 5;
     const int cap = p.maxblk * p.bs;
-    int t, key0, ppw;
+    auto clamped = [&](const int n) { return n < 0 ? 0 : (n > cap ? cap : n); };
+    int unit, b, cur, key0, ppw;
     if (p.balanced) {
         // Balanced mapping (at most 512 query tokens): the launch has a fixed number of waves; every wave
         // reads all sequence lengths, sizes the runs so that the runs of all tokens just fill the
         // launch, and takes the gw-th run in token order.  Short and long sequences then cost the same
-        // number of trips per wave and the whole pass is one round of resident waves.
-        const int gw = blockIdx.x * 4 + w;
-        const int nwaves = gridDim.x * 4;
-        int pairs[8], total = 0;
+        // number of trips per wave and the whole pass is one round of resident waves.  (Nothing is on its way from memory
+        // meanwhile, so it is kept short: divisions by reciprocals, and for up to 64 units a single row of the unit table.)
+        const int gw = blockIdx.x * LI_SCORE_WAVES + w;
+        const int nwaves = gridDim.x * LI_SCORE_WAVES;
+        int found = -1, found_run = 0, found_seq = 0, found_len = 0;
+        auto balance = [&](auto rows_tag) __attribute__((always_inline)) {
+            constexpr int ROWS = decltype(rows_tag)::value;          // of 64 units
+            const float inv_upb = __builtin_amdgcn_rcpf((float)upb);
+            int seq[ROWS], len[ROWS], pairs[ROWS], total = 0;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int tt = l + 64 * i;
-            int c = tt < nunits ? p.act[tt / upb] : 0;
-            c = c < 0 ? 0 : (c > cap ? cap : c);
-            pairs[i] = (c + 63) >> 6;
-            total += pairs[i];
-        }
-        total = (int)wave_incl_scan((uint32_t)total);
-        total = __builtin_amdgcn_readlane(total, 63);
-        // every token may waste one run on rounding: plan for nwaves - T runs
-        ppw = (total + (nwaves - nunits) - 1) / (nwaves - nunits);
-        ppw = ppw < 1 ? 1 : (ppw > LI_MAX_PAIRS_PER_WAVE ? LI_MAX_PAIRS_PER_WAVE : ppw);
-        int base = 0;                     // runs of all tokens before row i of the token table
-        int found = -1;                   // token of this wave's run << 16 | run index... kept separately below
-        int found_run = 0;
+            for (int i = 0; i < ROWS; ++i) {
+                const int tt = l + 64 * i;
+                seq[i] = tt < nunits ? small_quotient(tt, inv_upb) : p.B - 1;
+                len[i] = p.act[seq[i]];
+            }
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int runs = (pairs[i] + ppw - 1) / ppw;
-            const int incl = (int)wave_incl_scan((uint32_t)runs);
-            const int start = base + incl - runs;
-            if (gw >= start && gw < start + runs) { found = l + 64 * i; found_run = gw - start; }
-            base += __builtin_amdgcn_readlane(incl, 63);
-        }
+            for (int i = 0; i < ROWS; ++i) {
+                len[i] = l + 64 * i < nunits ? clamped(len[i]) : 0;
+                pairs[i] = (len[i] + 63) >> 6;
+                total += pairs[i];
+            }
+            total = __builtin_amdgcn_readlane((int)wave_incl_scan((uint32_t)total), 63);
+            // the shortest run length whose runs fit the launch: every unit may waste one run on rounding
+            ppw = (int)((float)(total + nwaves - 1) * __builtin_amdgcn_rcpf((float)nwaves));
+            ppw = ppw < 1 ? 1 : (ppw > LI_MAX_PAIRS_PER_WAVE ? LI_MAX_PAIRS_PER_WAVE : ppw);
+            for (;;) {
+                const float inv_ppw = __builtin_amdgcn_rcpf((float)ppw);
+                int base = 0;                 // runs of all units before row i of the unit table
+#pragma unroll
+                for (int i = 0; i < ROWS; ++i) {
+                    const int runs = small_quotient(pairs[i] + ppw - 1, inv_ppw);
+                    const int incl = (int)wave_incl_scan((uint32_t)runs);
+                    const int run = gw - (base + incl - runs);
+                    if (run >= 0 && run < runs) {
+                        found = l + 64 * i;
+                        found_run = run;
+                        found_seq = seq[i];
+                        found_len = len[i];
+                    }
+                    base += __builtin_amdgcn_readlane(incl, 63);
+                }
+                if (base <= nwaves || ppw >= LI_MAX_PAIRS_PER_WAVE) break;
+                ++ppw;
+                found = -1;
+            }
+        };
+        if (nunits <= 64) balance(std::integral_constant<int, 1>{});
+        else balance(std::integral_constant<int, LI_MAX_BALANCED_TOKENS / 64>{});
         const unsigned long long hit = __ballot(found >= 0);
         if (hit == 0ull) return;          // more waves than runs
         const int src = __ffsll((long long)hit) - 1;
-        t = __builtin_amdgcn_readlane(found, src);
+        unit = __builtin_amdgcn_readlane(found, src);
+        b = __builtin_amdgcn_readlane(found_seq, src);
+        cur = __builtin_amdgcn_readlane(found_len, src);
         key0 = __builtin_amdgcn_readlane(found_run, src) * (ppw * 64);
     } else {
-        t = blockIdx.y;
+        unit = blockIdx.y;
         ppw = p.ppw;
-        key0 = (blockIdx.x * 4 + w) * (ppw * 64);
+        key0 = (blockIdx.x * LI_SCORE_WAVES + w) * (ppw * 64);
+        b = unit / upb;
+        cur = clamped(p.act[b]);
     }
-    // t is the unit's number up to here; from here on its first token
-    const int b = t / upb;
-    const int s_first = (t - b * upb) * NT;
+    const int s_first = (unit - b * upb) * NT;
     const int nt = p.S1 - s_first < NT ? p.S1 - s_first : NT;     // tokens of this unit (uniform)
-    t = b * p.S1 + s_first;
-    int cur = p.act[b];
-    cur = cur < 0 ? 0 : (cur > cap ? cap : cur);
+    const int t = b * p.S1 + s_first;                             // its first token
     if (key0 >= cur) return;
     int npair = (cur - key0 + 63) >> 6;
     npair = npair > ppw ? ppw : npair;
     const int last_blk = ((cur + 31) >> 5) - 1;                  // last 32-key block holding a valid key
+
+    // Per-head factors: lane l loads head l's (HW and VAR: lane i, 32 + i the packed pair of heads 2i and 2i + 1), in front of the
+    // block table's entry, so that one wait serves them all.
+    static_assert(!(VAR && NT > 1), "the fp16 variant scores one token per wave");
+    typedef uint32_t u32_a2 __attribute__((aligned(2)));
+    uint32_t raw_q[NT], raw_w[NT];
+#pragma unroll
+    for (int s = 0; s < NT; ++s) {
+        const size_t ts = (size_t)(t + (s < nt ? s : 0));         // a unit of one token takes that token twice
+        if (VAR || HW) {
+            raw_q[s] = reinterpret_cast<const u32_a2 *>(static_cast<const uint16_t *>(p.q_scale) + ts * LI_HEADS)[j];
+            raw_w[s] = reinterpret_cast<const u32_a2 *>(static_cast<const uint16_t *>(p.weight) + ts * LI_HEADS)[j];
+        } else {
+            raw_q[s] = load_raw(p.q_scale, ts * LI_HEADS + l, p.q_dt);
+            raw_w[s] = load_raw(p.weight, ts * LI_HEADS + l, p.w_dt);
+        }
+    }
 
     // First cache row of every 32-key block of this wave's run, looked up once: lane i holds the row of
     // block i of the run (32 consecutive positions never straddle a page; a run has at most 64 blocks;
@@ -335,6 +373,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
         int pb = p.bt[(size_t)b * p.maxblk + page];
         pb = pb < 0 ? 0 : (pb >= p.nblocks ? p.nblocks - 1 : pb);
         run_row = pb * p.bs + (pos0 - page * p.bs);
+        asm volatile("" ::"v"(run_row));      // waited for here, not behind the requests below, which the compiler does not count
     }
     // Requests pair pr into buffer buf: per block four instructions of eight rows each.  Lane l owns
     // LDS slot l of an instruction's 1 KiB, i.e. row l/8 (of eight) and position l%8, and fetches chunk
@@ -348,11 +387,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
     const uint32_t lds_base = (uint32_t)__builtin_amdgcn_readfirstlane(
         (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) int8_t *)&kstage[w][0][0]);
     constexpr int KSZ = KDT == PTO_DT_FP32 ? 4 : 2;
-    auto request_pair = [&](const int pr, const int buf) {
-        const int rx = __builtin_amdgcn_readlane(run_row, 2 * pr), ry = __builtin_amdgcn_readlane(run_row, 2 * pr + 1);
-        const int8_t *gx = p.kcache + (size_t)rx * LI_DIM;
-        const int8_t *gy = p.kcache + (size_t)ry * LI_DIM;
-        const uint32_t dst = lds_base + (uint32_t)(buf * SC_BUF_BYTES);
+    // two runs of 32 rows, at gx and gy, into 8 KiB of LDS
+    auto request_rows = [&](const int8_t *gx, const int8_t *gy, const uint32_t dst) {
         asm volatile("s_mov_b32 m0, %3\n\t"
                      "s_nop 0\n\t"
                      "global_load_lds_dwordx4 %0, %2\n\t"
@@ -367,6 +403,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
                      "global_load_lds_dwordx4 %0, %2 offset:2048\n\t"
                      "global_load_lds_dwordx4 %1, %2 offset:3072"
                      :: "v"(lane_off), "v"(lane_off4), "s"(gy), "s"(dst + 4096u) : "memory", "m0");
+    };
+    auto request_pair = [&](const int pr, const int buf) {
+        const int rx = __builtin_amdgcn_readlane(run_row, 2 * pr), ry = __builtin_amdgcn_readlane(run_row, 2 * pr + 1);
+        const uint32_t dst = lds_base + (uint32_t)(buf * SC_BUF_BYTES);
+        request_rows(p.kcache + (size_t)rx * LI_DIM, p.kcache + (size_t)ry * LI_DIM, dst);
         // the aligned dword that holds this lane's scale
         const uintptr_t sa = (reinterpret_cast<uintptr_t>(p.k_scale) + ((size_t)(half ? ry : rx) + j) * KSZ) & ~(uintptr_t)3;
         asm volatile("s_mov_b32 m0, %1\n\t"
@@ -374,54 +415,72 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
                      "global_load_lds_dword %0, off"
                      :: "v"(sa), "s"(dst + (uint32_t)SC_PAIR_BYTES) : "memory", "m0");
     };
-    request_pair(0, 0);
-    if (npair > 1) request_pair(1, 1);
 
     // A operands.  Row i of operand 0 is head 32*((i>>2)&1) + 4*(i>>3) + (i&3), operand 1 adds 16:
     // with the 32x32 accumulator layout (row = 8*(r/4) + 4*half + r%4) lane (key, half) then holds
     // heads 32*half + r in register r of accumulator 0 and heads 32*half + 16 + r in accumulator 1.
     // The contraction runs over 16-byte chunks in the order 4*half + ks (ks = 0..3).
+    // The queries travel through the pair buffers, in front of the first pairs: asked for behind them, as loads into registers,
+    // they arrive when both pairs of every wave have, and no third pair is asked for meanwhile.
     i32x4 qa[NT][2][4];
-#pragma unroll
-    for (int s = 0; s < NT; ++s) {
+    auto request_query = [&](const int s, const int buf) {
+        const int8_t *q0 = p.q + (size_t)(t + (s < nt ? s : 0)) * (LI_HEADS * LI_DIM);      // a unit of one token loads that token twice
+        request_rows(q0, q0 + 32 * LI_DIM, lds_base + (uint32_t)(buf * SC_BUF_BYTES));
+    };
+    auto read_query = [&](auto s_tag, const int buf) {
+        constexpr int s = decltype(s_tag)::value;
+        asm volatile("" ::: "memory");
         const int head0 = 32 * ((j >> 2) & 1) + 4 * (j >> 3) + (j & 3);
-        const int ts = t + (s < nt ? s : 0);                   // a unit of one token loads that token twice
-        const int8_t *q0 = p.q + ((size_t)ts * LI_HEADS + head0) * LI_DIM + 64 * half;
+        const int8_t *src = &kstage[w][buf][0];
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
-            qa[s][0][ks] = *reinterpret_cast<const i32x4 *>(q0 + 16 * ks);
-            qa[s][1][ks] = *reinterpret_cast<const i32x4 *>(q0 + 16 * LI_DIM + 16 * ks);
+            qa[s][0][ks] = *reinterpret_cast<const i32x4 *>(src + head0 * LI_DIM + (((4 * half + ks) ^ ((head0 >> 1) & 7)) << 4));
+            qa[s][1][ks] = *reinterpret_cast<const i32x4 *>(src + (head0 + 16) * LI_DIM + (((4 * half + ks) ^ ((head0 >> 1) & 7)) << 4));
         }
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0xC07F);                      // lgkmcnt(0): the buffer has been read
+    };
+    if (NT == 1) {
+        request_query(0, 1);
+        request_pair(0, 0);
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(9));
+        read_query(std::integral_constant<int, 0>{}, 1);
+    } else {
+        request_query(0, 0);
+        request_query(NT - 1, 1);
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(8));
+        read_query(std::integral_constant<int, 0>{}, 0);
+        request_pair(0, 0);
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(9));
+        read_query(std::integral_constant<int, NT - 1>{}, 1);
     }
-    // per-head factors: lane l computes head l's.  One token per wave: read back lane by lane they are
-    // wave-uniform and sit in scalar registers.  Two tokens: they go to this wave's rows of wsc_lds and are
-    // read as broadcasts, four heads at a time, along the head sum.
-    // VAR = 1 keeps the fp16 query scales and weights of head pairs (2i, 2i+1) packed instead.
-    static_assert(!(VAR && NT > 1), "the fp16 variant scores one token per wave");
+    if (npair > 1) request_pair(1, 1);
+
+    // The factors, wave-uniform.  One token per wave, or fp16 ones: read back lane by lane they sit in scalar registers.  Two
+    // tokens of other factors: they go to this wave's rows of wsc_lds and are read as broadcasts, four heads at a time, along
+    // the head sum.  VAR = 1 keeps the fp16 query scales and weights of head pairs (2i, 2i+1) packed instead.
     float wsc[(VAR || HW || NT > 1) ? 1 : LI_HEADS];
     uint32_t wp[HW ? NT : 1][HW ? LI_HEADS / 2 : 1];             // HW: factors of heads 2i and 2i + 1
     uint32_t qs2[VAR ? LI_HEADS / 2 : 1], w2[VAR ? LI_HEADS / 2 : 1];
     if (VAR) {
-        const uint32_t mq = reinterpret_cast<const uint32_t *>(p.q_scale)[(size_t)t * (LI_HEADS / 2) + (l & 31)];
-        const uint32_t mw = reinterpret_cast<const uint32_t *>(p.weight)[(size_t)t * (LI_HEADS / 2) + (l & 31)];
 #pragma unroll
         for (int h = 0; h < LI_HEADS / 2; ++h) {
-            qs2[h] = (uint32_t)__builtin_amdgcn_readlane((int)mq, h);
-            w2[h] = (uint32_t)__builtin_amdgcn_readlane((int)mw, h);
+            qs2[h] = (uint32_t)__builtin_amdgcn_readlane((int)raw_q[0], h);
+            w2[h] = (uint32_t)__builtin_amdgcn_readlane((int)raw_w[0], h);
         }
     } else if (HW) {
 #pragma unroll
         for (int s = 0; s < NT; ++s) {
-            const size_t i0 = (size_t)(t + (s < nt ? s : 0)) * LI_HEADS + 2 * (l & 31);
-            const uint32_t mine = pack_f16x2(w_scale_of(p, i0), w_scale_of(p, i0 + 1));       // fp16 values: exact
+            const f16x2 q2 = __builtin_bit_cast(f16x2, raw_q[s]), w2h = __builtin_bit_cast(f16x2, raw_w[s]);
+            const uint32_t mine = pack_f16x2(__fmul_rn((float)q2[0], (float)w2h[0]), __fmul_rn((float)q2[1], (float)w2h[1]));
 #pragma unroll
             for (int h = 0; h < LI_HEADS / 2; ++h) wp[s][h] = (uint32_t)__builtin_amdgcn_readlane((int)mine, h);
         }
     } else if (NT > 1) {
 #pragma unroll
-        for (int s = 0; s < NT; ++s) wsc_lds[w][s][l] = w_scale_of(p, (size_t)(t + (s < nt ? s : 0)) * LI_HEADS + l);
+        for (int s = 0; s < NT; ++s) wsc_lds[w][s][l] = __fmul_rn(raw_to_f32(raw_q[s], p.q_dt), raw_to_f32(raw_w[s], p.w_dt));
     } else {
-        const float mine = w_scale_of(p, (size_t)t * LI_HEADS + l);
+        const float mine = __fmul_rn(raw_to_f32(raw_q[0], p.q_dt), raw_to_f32(raw_w[0], p.w_dt));
 #pragma unroll
         for (int h = 0; h < LI_HEADS; ++h) wsc[h] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mine), h));
     }
@@ -1160,14 +1219,14 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_stream_kernel(const LiP
 
 hipError_t li_launch(const LiParams &p, hipStream_t stream)
 {
-    const dim3 block(256);
+    const dim3 block(64 * LI_SCORE_WAVES);
     const int nt = p.nt;
     const int nunits = p.B * ((p.S1 + nt - 1) / nt);
     dim3 grid;
     if (p.balanced) {
         grid = dim3((unsigned)p.score_wgs);
     } else {
-        const unsigned gx = (unsigned)((p.score_stride + 4 * p.ppw * 64 - 1) / (4 * p.ppw * 64));
+        const unsigned gx = (unsigned)((p.score_stride + LI_SCORE_WAVES * p.ppw * 64 - 1) / (LI_SCORE_WAVES * p.ppw * 64));
         grid = dim3(gx, (unsigned)nunits);
     }
     const bool hw = p.q_dt == PTO_DT_FP16 && p.w_dt == PTO_DT_FP16;
