@@ -253,6 +253,9 @@ constexpr int SC_BUF_BYTES = SC_PAIR_BYTES + 256;   // + the 64 key scales (one 
 // four the second one's sequence lengths came back behind the first one's key rows (7 us, and it ended as much later), the
 // mapping took 2.3 us of divisions, and the queries, asked for behind two pairs of every wave, arrived behind 34 MB.  Kernel over
 // rotating key caches, before / now: 4 tokens x 32 K keys 10.5 / 6.8 us, 32 x 8-64 K 36.9 / 35.6, 64 pairs of tokens x 4-32 K 44.8 / 40.5.
+// (Pairs of a workgroup's runs drawn by whichever wave comes first, so that its waves end together instead of up to 8 us apart: +-0.
+// Bound now: the first one by its bytes, 28.4 us with nothing but the requests and stores; the other by vector work and the
+// products beside it, two waves to a SIMD.)
 // HW: query scales and weights are fp16, so the per-head factors are fp16 values, their products with x exact and the head
 // sum one instruction per head instead of two; the factors sit in scalar registers as packed pairs, for two tokens as well.
 template <int KDT, int VAR = 0, int NT = 1, bool HW = false>
@@ -388,26 +391,32 @@ __global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_pe
         (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) int8_t *)&kstage[w][0][0]);
     constexpr int KSZ = KDT == PTO_DT_FP32 ? 4 : 2;
     // two runs of 32 rows, at gx and gy, into 8 KiB of LDS
-    auto request_rows = [&](const int8_t *gx, const int8_t *gy, const uint32_t dst) {
-        asm volatile("s_mov_b32 m0, %3\n\t"
-                     "s_nop 0\n\t"
-                     "global_load_lds_dwordx4 %0, %2\n\t"
-                     "global_load_lds_dwordx4 %1, %2 offset:1024\n\t"
-                     "global_load_lds_dwordx4 %0, %2 offset:2048\n\t"
-                     "global_load_lds_dwordx4 %1, %2 offset:3072"
-                     :: "v"(lane_off), "v"(lane_off4), "s"(gx), "s"(dst) : "memory", "m0");
-        asm volatile("s_mov_b32 m0, %3\n\t"
-                     "s_nop 0\n\t"
-                     "global_load_lds_dwordx4 %0, %2\n\t"
-                     "global_load_lds_dwordx4 %1, %2 offset:1024\n\t"
-                     "global_load_lds_dwordx4 %0, %2 offset:2048\n\t"
-                     "global_load_lds_dwordx4 %1, %2 offset:3072"
-                     :: "v"(lane_off), "v"(lane_off4), "s"(gy), "s"(dst + 4096u) : "memory", "m0");
+#define REQUEST_32_ROWS(HINT, G, DST)                                                              \
+    asm volatile("s_mov_b32 m0, %3\n\t"                                                            \
+                 "s_nop 0\n\t"                                                                     \
+                 "global_load_lds_dwordx4 %0, %2" HINT "\n\t"                                      \
+                 "global_load_lds_dwordx4 %1, %2 offset:1024" HINT "\n\t"                          \
+                 "global_load_lds_dwordx4 %0, %2 offset:2048" HINT "\n\t"                          \
+                 "global_load_lds_dwordx4 %1, %2 offset:3072" HINT                                 \
+                 :: "v"(lane_off), "v"(lane_off4), "s"(G), "s"(DST) : "memory", "m0")
+    auto request_rows = [&](const int8_t *gx, const int8_t *gy, const uint32_t dst, const bool once) {
+        if (once) {
+            REQUEST_32_ROWS(" nt", gx, dst);
+            REQUEST_32_ROWS(" nt", gy, dst + 4096u);
+        } else {
+            REQUEST_32_ROWS("", gx, dst);
+            REQUEST_32_ROWS("", gy, dst + 4096u);
+        }
     };
+#undef REQUEST_32_ROWS
+    // Keys that one unit alone reads are asked for without being kept (32 sequences of 8 to 64 K keys 35.2 us, so 31.4); with
+    // more units to a sequence the next one finds them in the caches (20 sequences of 20 to 60 K, four query tokens, 47.0; not
+    // kept 50.8; 4 of 60 to 120 K 32.0 and 36.9).
+    const bool read_once = upb == 1;
     auto request_pair = [&](const int pr, const int buf) {
         const int rx = __builtin_amdgcn_readlane(run_row, 2 * pr), ry = __builtin_amdgcn_readlane(run_row, 2 * pr + 1);
         const uint32_t dst = lds_base + (uint32_t)(buf * SC_BUF_BYTES);
-        request_rows(p.kcache + (size_t)rx * LI_DIM, p.kcache + (size_t)ry * LI_DIM, dst);
+        request_rows(p.kcache + (size_t)rx * LI_DIM, p.kcache + (size_t)ry * LI_DIM, dst, read_once);
         // the aligned dword that holds this lane's scale
         const uintptr_t sa = (reinterpret_cast<uintptr_t>(p.k_scale) + ((size_t)(half ? ry : rx) + j) * KSZ) & ~(uintptr_t)3;
         asm volatile("s_mov_b32 m0, %1\n\t"
@@ -425,7 +434,7 @@ __global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_pe
     i32x4 qa[NT][2][4];
     auto request_query = [&](const int s, const int buf) {
         const int8_t *q0 = p.q + (size_t)(t + (s < nt ? s : 0)) * (LI_HEADS * LI_DIM);      // a unit of one token loads that token twice
-        request_rows(q0, q0 + 32 * LI_DIM, lds_base + (uint32_t)(buf * SC_BUF_BYTES));
+        request_rows(q0, q0 + 32 * LI_DIM, lds_base + (uint32_t)(buf * SC_BUF_BYTES), false);
     };
     auto read_query = [&](auto s_tag, const int buf) {
         constexpr int s = decltype(s_tag)::value;
