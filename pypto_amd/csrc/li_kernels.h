@@ -31,6 +31,7 @@ struct LiParams {
     int ppw;                // 64-key block pairs per wave of the score kernel, <= LI_MAX_PAIRS_PER_WAVE
     int balanced;           // score kernel sizes its runs from the sequence lengths (units <= LI_MAX_BALANCED_TOKENS)
     int score_wgs;          // its launch size in workgroups when balanced
+    int round_waves;        // waves of one round of them, which the runs are sized for
     int nt;                 // query tokens of one sequence that a wave of the score kernel scores per key pass: 1 or 2
     int variant;            // 0: fp32 head factors applied after the ReLU; 1: fp16 scales applied before it (all tensors fp16)
 };

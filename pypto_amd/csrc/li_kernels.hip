@@ -280,7 +280,6 @@ __global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_pe
         // number of trips per wave and the whole pass is one round of resident waves.  (Nothing is on its way from memory
         // meanwhile, so it is kept short: divisions by reciprocals, and for up to 64 units a single row of the unit table.)
         const int gw = blockIdx.x * LI_SCORE_WAVES + w;
-        const int nwaves = gridDim.x * LI_SCORE_WAVES;
         int found = -1, found_run = 0, found_seq = 0, found_len = 0;
         auto balance = [&](auto rows_tag) __attribute__((always_inline)) {
             constexpr int ROWS = decltype(rows_tag)::value;          // of 64 units
@@ -299,6 +298,9 @@ __global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_pe
                 total += pairs[i];
             }
             total = __builtin_amdgcn_readlane((int)wave_incl_scan((uint32_t)total), 63);
+            // as few whole rounds as runs of the greatest length need (the launch has as many as the longest sequences would)
+            int nwaves = p.round_waves;
+            while (total > nwaves * LI_MAX_PAIRS_PER_WAVE && nwaves < (int)gridDim.x * LI_SCORE_WAVES) nwaves += p.round_waves;
             // the shortest run length whose runs fit the launch: every unit may waste one run on rounding
             ppw = (int)((float)(total + nwaves - 1) * __builtin_amdgcn_rcpf((float)nwaves));
             ppw = ppw < 1 ? 1 : (ppw > LI_MAX_PAIRS_PER_WAVE ? LI_MAX_PAIRS_PER_WAVE : ppw);

@@ -242,3 +242,31 @@ def test_row_lengths_of_the_select(c_oracle, k, act):
     inp.idx_query[1] = inp.idx_query[1].sign()
     inp.idx_key_cache[::3] = inp.idx_key_cache[0]
     assert_exact(run_op(inp), oracle(inp, c_oracle), f"k={k} act={act}")
+
+
+@pytest.mark.parametrize("b,s1,lo,hi,cap", [
+    (40, 1, 1, 3000, 131072),          # pages for far more keys than there are: a launch of more waves than one round
+    (18, 3, 20000, 131072, 131072),    # the same with runs of every length, and a unit of one token
+    (64, 1, 66000, 70000, 70016),      # more keys than a round of the longest runs holds
+])
+def test_indexer_launches_of_more_than_one_round(b, s1, lo, hi, cap):
+    """The rows of a batch whose runs are spread over all its sequences against the same rows scored one sequence at a time.  All
+    sequences read the same 2048 pages in orders of their own."""
+    g = torch.Generator().manual_seed(b)
+    dev, pages, k = torch.device("cuda:0"), 2048, 2048
+    act = torch.randint(lo, hi + 1, (b,), generator=g, dtype=torch.int32)
+    act[-1] = hi
+    table = torch.randint(0, pages, (b, cap // 128), generator=g, dtype=torch.int32).to(dev)
+    q = torch.randint(-127, 128, (b * s1, 64, 128), generator=g, dtype=torch.int8).to(dev)
+    qs = (torch.rand((b * s1, 64), generator=g) * 0.015 + 0.005).to(dev)
+    w = (torch.randn((b * s1, 64), generator=g) * 0.125).to(torch.bfloat16).to(dev)
+    keys = torch.randint(-127, 128, (pages, 128, 1, 128), generator=g, dtype=torch.int8).to(dev)
+    ks = (torch.rand((pages, 128, 1), generator=g) * 0.015 + 0.005).to(dev)
+    act = act.to(dev)
+    got = torch.full((b * s1, 1, k), -7, dtype=torch.int32, device=dev)
+    pypto_amd.lightning_indexer_decode(q, qs, keys, ks, w, act, table, got)
+    one = torch.full((s1, 1, k), -7, dtype=torch.int32, device=dev)
+    for i in range(b):
+        r = slice(i * s1, (i + 1) * s1)
+        pypto_amd.lightning_indexer_decode(q[r], qs[r], keys, ks, w[r], act[i:i + 1], table[i:i + 1].contiguous(), one)
+        assert torch.equal(got[r], one), i
