@@ -101,12 +101,12 @@ __global__ __launch_bounds__(256) void lip_qproj_prefill_kernel(const QProj p, c
 // The fixed-order sums over the hidden axis at prefill sizes (xlinear_fixed.h, the matrix-core form of the sequential
 // sums); only the group sums reach memory, an eighth of the rows the decode form leaves.
 static_assert(XL_BLOCK == LIP_XBLOCK && XL_GROUP == LIP_XGROUP, "the second launch adds groups of eight blocks of 64");
-__global__ __launch_bounds__(64 * XF_WAVES) void lip_xlinear_group_kernel(const LipParams p, const int ngroups)
+__global__ __launch_bounds__(64 * XF_WAVES, 2) void lip_xlinear_group_kernel(const LipParams p, const XfGrid fg)
 {
     __shared__ __attribute__((aligned(16))) uint8_t smem[XF_LDS];
-    const XfJob j = xf_job((int)blockIdx.x, LIP_XF_SETS, ngroups, p.T);
+    const XfJob j = xf_job((int)blockIdx.x, fg, p.T);
     if (j.g < 0) return;
-    xf_body(lip_xf_slab(p, j.set, j.g), p.x, p.T, p.h, j.g, j.t0, smem);
+    xf_body(lip_xf_slab(p, j.set, j.g), p.x, p.T, p.h, j.g, j.t0, fg.run, smem);
 }
 
 // The sums over the hidden axis on the matrix cores (xlinear_mfma.h): workgroup = (wk or w_proj, one of nsplit
@@ -181,7 +181,10 @@ hipError_t lip_launch_linear(const LipParams &p, hipStream_t stream)
     }
     if (lip_x_group_rows(p)) {
         const int ngroups = lip_xrows(p);
-        hipLaunchKernelGGL(lip_xlinear_group_kernel, dim3((unsigned)xf_jobs(LIP_XF_SETS, ngroups, p.T)), dim3(64 * XF_WAVES), 0, stream, p, ngroups);
+        const int cus = cu_count();
+        if (cus <= 0) return hipErrorNoDevice;
+        const XfGrid fg = {LIP_XF_SETS, ngroups, xf_run(LIP_XF_SETS * ngroups, p.T, 2 * cus)};
+        hipLaunchKernelGGL(lip_xlinear_group_kernel, dim3((unsigned)xf_jobs(fg, p.T)), dim3(64 * XF_WAVES), 0, stream, p, fg);
         return hipGetLastError();
     }
     const int xtok = lip_xtok(p.T);

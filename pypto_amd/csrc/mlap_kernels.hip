@@ -108,21 +108,21 @@ static_assert(XM_KC == MLAP_XBLOCK, "the workspace is sized in chunks of the hid
 // in a launch of the indexer's own before they shared it.)  Up to 64 tokens all workgroups run at once and these are the longer
 // ones beside another workgroup, so they start first (fused prolog, 32 tokens: 37.4 us per pass, at the end of the launch 39.3;
 // 200 tokens 84.4, at the end 70.3).
-// TB: at most 32 * TB tokens (xm_small_body), 0 for tiles of 128 tokens (xm_body), XM_BIG for tiles of 256 (xb_body).
+// TB: at most 32 * TB tokens (xm_small_body), 0 for tiles of 128 tokens x 128 columns (xm_body), XM_BIG for 128 x 256 (xb_body).
 constexpr int XM_BIG = 8;
 template <int TB> constexpr int XM_FORM_LDS = TB == 0 ? XM_LDS : (TB == XM_BIG ? XB_LDS : XMS_LDS<TB == 1 ? 1 : 2>);
 template <int TB> constexpr int XM_KERNEL_LDS = XM_FORM_LDS<TB> > XF_LDS ? XM_FORM_LDS<TB> : XF_LDS;
-static_assert(2 * XM_KERNEL_LDS<0> <= 160 * 1024 && 2 * XM_KERNEL_LDS<2> <= 160 * 1024, "two workgroups share a compute unit");
+static_assert(2 * XM_KERNEL_LDS<0> <= 160 * 1024 && 2 * XM_KERNEL_LDS<2> <= 160 * 1024 && 2 * XM_KERNEL_LDS<XM_BIG> <= 160 * 1024, "two workgroups share a compute unit");
 template <int TB>
-__global__ __launch_bounds__(256) void mlap_xlinear_mfma_kernel(const MlapParams p, const int nslabs, const int nsplit, const int own_wgs,
-                                                                const int fixed_sets, const int fixed_groups, const LipParams lip)
+__global__ __launch_bounds__(256, 2) void mlap_xlinear_mfma_kernel(const MlapParams p, const int nslabs, const int nsplit, const int own_wgs,
+                                                                const XfGrid fg, const LipParams lip)
 {
     __shared__ __attribute__((aligned(16))) uint8_t smem[XM_KERNEL_LDS<TB>];
     constexpr bool FIXED_FIRST = TB == 1 || TB == 2;
     const int nfixed = (int)gridDim.x - own_wgs;                   // a multiple of eight, as own_wgs: the XCDs go round alike
     const int fixed = (int)blockIdx.x - (FIXED_FIRST ? 0 : own_wgs), bid = (int)blockIdx.x - (FIXED_FIRST ? nfixed : 0);
     if (FIXED_FIRST ? fixed < nfixed : fixed >= 0) {
-        const XfJob j = xf_job(fixed, fixed_sets, fixed_groups, p.T);
+        const XfJob j = xf_job(fixed, fg, p.T);
         if (j.g < 0) return;
         XlSlab sl;
         if (j.set == 0) {
@@ -135,7 +135,7 @@ __global__ __launch_bounds__(256) void mlap_xlinear_mfma_kernel(const MlapParams
         } else {
             sl = lip_xf_slab(lip, j.set - 1, j.g);
         }
-        xf_body(sl, p.x, p.T, p.h, j.g, j.t0, smem);
+        xf_body(sl, p.x, p.T, p.h, j.g, j.t0, fg.run, smem);
         return;
     }
     if constexpr (TB == XM_BIG) {
@@ -145,15 +145,16 @@ __global__ __launch_bounds__(256) void mlap_xlinear_mfma_kernel(const MlapParams
         const int idx = (bid & 7) * (own_wgs >> 3) + (bid >> 3);
         if (idx >= nslabs * ttiles * nsplit) return;
         const int slab = idx % nslabs, sp = (idx / nslabs) / ttiles, t0 = ((idx / nslabs) % ttiles) * XB_TOK;
-        const int qslabs = p.q_lora / 128;
+        const int qslabs = p.q_lora / XB_COLS;
         const int nc = p.q_lora + MLAP_KV + MLAP_ROPE;
         XmSlab sl;
-        sl.w = slab < qslabs ? reinterpret_cast<const uint8_t *>(p.w_dq) + slab * 256 : reinterpret_cast<const uint8_t *>(p.w_dkvkr) + (slab - qslabs) * 256;
+        sl.w = slab < qslabs ? reinterpret_cast<const uint8_t *>(p.w_dq) + slab * (2 * XB_COLS)
+                             : reinterpret_cast<const uint8_t *>(p.w_dkvkr) + (slab - qslabs) * (2 * XB_COLS);
         sl.pitch = (slab < qslabs ? p.q_lora : MLAP_KV + MLAP_ROPE) * 2;
-        sl.pieces = 16;
-        sl.out = p.xpart + (size_t)sp * p.T * nc + slab * 128;
+        sl.pieces = 2 * XB_COLS / 16;
+        sl.out = p.xpart + (size_t)sp * p.T * nc + slab * XB_COLS;
         sl.out_pitch = nc;
-        const int nchunks = p.h / XB_KC;
+        const int nchunks = p.h / XM_KC;
         xb_body(sl, p.x, p.T, p.h, t0, (int)((long long)sp * nchunks / nsplit), (int)((long long)(sp + 1) * nchunks / nsplit), smem);
         return;
     } else {
@@ -542,9 +543,8 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
         const int cus = cu_count();
         if (cus <= 0) return hipErrorNoDevice;
         // every slab but the last, the rope columns, which keep their fixed-order sums
-        const int mslabs = nslabs - 1;
-        const bool big = p.T > XM_TOK;       // 130 tokens: 60.9 us per pass, 66.7 with tiles of 128; 1500: 282 and 293; 4096: 700 and 724
-        // As many ranges as make two workgroups of 128 tokens or one of 256 per compute unit (the other half of each is for the
+        const bool big = p.T > XM_TOK;
+        // As many ranges as make two workgroups of 128 x 128 or one of 128 x 256 per compute unit (the other half of each is for the
         // fixed-order sums), MLAP_XM_MAX_SPLITS = 14 at most: that many up to 256 tokens, so that a token's latents do not depend
         // on how many tokens the launch has.  Fewer ranges are longer fp32 chains, further from the 64-bit sums (relative error
         // over 2048 columns of 7168 products: 14 ranges 1.44e-7, 12 1.52e-7, 10 1.63e-7, 8 1.80e-7), and one int8 value of a
@@ -555,16 +555,17 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
         // Up to 64 tokens two workgroups share a compute unit, and the fixed-order sums start first (one per compute unit, those
         // last, so a second round: 9 tokens 39.1, in this form 32.2; 32: 42.5, 36.4; 48: 47.3, 43.3; 64: 52.9, 44.8, the last launch
         // in tiles of 128 tokens; two ranges per workgroup: 9 tokens 33.5, 32: 37.0, 48: 47.1, 64: 52.5).
-        const int xtiles = big ? (p.T + XB_TOK - 1) / XB_TOK : ttiles;
-        ngroups = big ? cus / (mslabs * xtiles) : 2 * cus / nslabs;
+        const int mslabs = (nslabs - 1) / (big ? XB_COLS / 128 : 1);
+        ngroups = big ? cus / (mslabs * ttiles) : 2 * cus / nslabs;
         ngroups = ngroups < 1 ? 1 : ngroups;
         ngroups = ngroups > MLAP_XM_MAX_SPLITS ? MLAP_XM_MAX_SPLITS : ngroups;
         ngroups = ngroups > nchunks ? nchunks : ngroups;
         const int per_slab = ngroups * ttiles;
-        const int wgs = big ? 8 * ((mslabs * xtiles * ngroups + 7) / 8) : 8 * ((mslabs >> 3) * per_slab + ((mslabs & 7) * per_slab + 7) / 8);   // the kernel's XCD-wise job order
+        const int wgs = big ? 8 * ((mslabs * per_slab + 7) / 8) : 8 * ((mslabs >> 3) * per_slab + ((mslabs & 7) * per_slab + 7) / 8);   // the kernel's XCD-wise job order
         const int sets = 1 + (lip_rider != nullptr ? LIP_XF_SETS : 0);
-        const dim3 g((unsigned)(wgs + xf_jobs(sets, ngroups_fixed, p.T)));
-#define XM_LAUNCH(TBV) hipLaunchKernelGGL(mlap_xlinear_mfma_kernel<TBV>, g, dim3(256), 0, stream, p, mslabs, ngroups, wgs, sets, ngroups_fixed, lip)
+        const XfGrid fg = {sets, ngroups_fixed, xf_run(sets * ngroups_fixed, p.T, 2 * cus - wgs)};
+        const dim3 g((unsigned)(wgs + xf_jobs(fg, p.T)));
+#define XM_LAUNCH(TBV) hipLaunchKernelGGL(mlap_xlinear_mfma_kernel<TBV>, g, dim3(256), 0, stream, p, mslabs, ngroups, wgs, fg, lip)
         if (p.T <= 32) XM_LAUNCH(1);
         else if (p.T <= 64) XM_LAUNCH(2);
         else if (big) XM_LAUNCH(XM_BIG);

@@ -523,5 +523,43 @@ __device__ __forceinline__ uint16_t quant_pair_amax(const float y0, const float 
     return 0;
 }
 
+// The chunk loop: tokens(s, buffer) requests chunks XC*s .. of the tokens (XR requests per wave), weights(c, slot) chunk c of the
+// weights (WR requests), products(c % XC, token buffer, slot) consumes chunk c.  nch is even.
+template <int XC, int XR, int WR, class Tokens, class Weights, class Products>
+__device__ __forceinline__ void staged_chunks(const int nch, const Tokens &tokens, const Weights &weights, const Products &products)
+{
+    tokens(0, 0);
+    weights(0, 0);
+    weights(1, 1);
+    int slot = 0;
+#pragma unroll 1
+    for (int c = 0; c < nch; c += XC) {
+        const int xb = (c / XC) & 1;
+        if (XC == 2 || c + 1 < nch) VM_WAIT(WR);       // everything but the weights of chunk c + 1
+        else VM_WAIT(0);
+        __syncthreads();                               // chunk c has landed for every wave; every wave is done with chunk c - 1
+        const int slot1 = slot == 2 ? 0 : slot + 1, slot2 = slot == 0 ? 2 : slot - 1;
+        if (XC == 2) {
+            if (c + 2 < nch) {
+                weights(c + 2, slot2);
+                tokens(c / 2 + 1, xb ^ 1);
+            }
+            products(0, xb, slot);
+            if (c + 2 < nch) VM_WAIT(WR + XR);
+            else VM_WAIT(0);
+            __syncthreads();
+            if (c + 3 < nch) weights(c + 3, slot);
+            products(1, xb, slot1);
+            slot = slot2;
+        } else {
+            if (c + 1 < nch) tokens(c + 1, xb ^ 1);
+            if (c + 2 < nch) weights(c + 2, slot2);
+            products(0, xb, slot);
+            slot = slot1;
+        }
+    }
+    __syncthreads();                                   // every wave is done with the last chunk
+}
+
 }  // namespace
 }  // namespace pto

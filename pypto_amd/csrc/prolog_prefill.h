@@ -47,44 +47,6 @@ struct PfTokens {
     }
 };
 
-// The chunk loop: tokens(s, buffer) requests chunks XC*s .. of the tokens (XR requests per wave), weights(c, slot) chunk c of the
-// weights (WR requests), products(c % XC, token buffer, slot) consumes chunk c.  nch is even.
-template <int XC, int XR, int WR, class Tokens, class Weights, class Products>
-__device__ __forceinline__ void pf_chunks(const int nch, const Tokens &tokens, const Weights &weights, const Products &products)
-{
-    tokens(0, 0);
-    weights(0, 0);
-    weights(1, 1);
-    int slot = 0;
-#pragma unroll 1
-    for (int c = 0; c < nch; c += XC) {
-        const int xb = (c / XC) & 1;
-        if (XC == 2 || c + 1 < nch) VM_WAIT(WR);       // everything but the weights of chunk c + 1
-        else VM_WAIT(0);
-        __syncthreads();                               // chunk c has landed for every wave; every wave is done with chunk c - 1
-        const int slot1 = slot == 2 ? 0 : slot + 1, slot2 = slot == 0 ? 2 : slot - 1;
-        if (XC == 2) {
-            if (c + 2 < nch) {
-                weights(c + 2, slot2);
-                tokens(c / 2 + 1, xb ^ 1);
-            }
-            products(0, xb, slot);
-            if (c + 2 < nch) VM_WAIT(WR + XR);
-            else VM_WAIT(0);
-            __syncthreads();
-            if (c + 3 < nch) weights(c + 3, slot);
-            products(1, xb, slot1);
-            slot = slot2;
-        } else {
-            if (c + 1 < nch) tokens(c + 1, xb ^ 1);
-            if (c + 2 < nch) weights(c + 2, slot2);
-            products(0, xb, slot);
-            slot = slot1;
-        }
-    }
-    __syncthreads();                                   // every wave is done with the last chunk
-}
-
 // ------------------------------------------------------------------------------------------------ attention query
 // Wave (wc, wt) holds columns 96*wc .. +95 of the head's 192 x TB blocks of 32 tokens (3 * TB accumulators).
 // Row r of a chunk of weights lies at 192 * r, its 32-byte block b at b ^ ((r >> 2) & 1): the eight consecutive rows of a
@@ -166,7 +128,7 @@ __device__ __forceinline__ void mlap_prefill_body(const MlapParams &p, const int
             aoff[i] = 2 * PFA_X<XC, TB> + (16 * half + ((l & 15) >> 1)) * MLAP_QHEAD + 32 * ((3 * wc + i) ^ ((l >> 3) & 1)) + 16 * ((l >> 4) & 1) + 8 * (l & 1);
         const uint32_t boff = (32 * TB * wt + (l & 31)) * PF_XPITCH<XC>;
         typedef int v2i __attribute__((ext_vector_type(2)));
-        pf_chunks<XC, XR, 3>(
+        staged_chunks<XC, XR, 3>(
             p.q_lora / PF_KC, [&](const int s, const int b) { xt.request(s, base + b * PFA_X<XC, TB> + 1024 * XR * w); },
             [&](const int c, const int slot) {
 #pragma unroll
@@ -339,7 +301,7 @@ __device__ __forceinline__ void lip_prefill_body(const LipParams &p, const int j
             wsrc[j] = p.w_qb + (size_t)(8 * (2 * w + j) + (l >> 3)) * ncols + head * LIP_DIM + 16 * ((l & 7) ^ q_tr_piece_swizzle(l >> 3));
         const size_t wstep = (size_t)PF_KC * ncols;
         const uint32_t boff = (32 * TB * w + (l & 31)) * PF_XPITCH<XC>;
-        pf_chunks<XC, XR, 2>(
+        staged_chunks<XC, XR, 2>(
             p.q_lora / PF_KC, [&](const int s, const int b) { xt.request(s, base + b * PFI_X<XC, TB> + 1024 * XR * w); },
             [&](const int c, const int slot) {
 #pragma unroll

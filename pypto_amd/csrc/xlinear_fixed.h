@@ -128,48 +128,64 @@ __device__ __forceinline__ void xl_body(const XlSlab &sl, const uint16_t *x, con
 // rounding -- an fp32 FMA -- and a chain of them is the sequential sum of the form above, bit for bit, whatever order
 // the cores have inside an instruction of more rows.  (Subnormal products and sums, signed zeros included: checked
 // against fmaf chains.)
-//   workgroup = (slab of up to 64 columns, group of 512 hidden rows, 32 tokens), four waves; wave w takes blocks 2w and
-//   2w + 1 of the group as the two independent products of the instruction (lanes 0..31 supply block 2w, lanes 32..63
-//   block 2w + 1).  Row i of the first operand is column 2i (accumulator 0) or 2i + 1 (accumulator 1) of the slab: one
-//   dword of LDS per lane and hidden row feeds both.  The hidden states go from memory to registers, 64 consecutive
-//   ones per lane.  The eight block sums meet in LDS and are chained ascending into the group sum.
-// Bound: the matrix cores' fp32 rate (64 clocks per instruction, 139 TFLOP/s reached by a bare loop); per two
-// instructions there are one LDS read and three conversions.  The multiply-add form of the vector ALU this replaced
-// (hidden states broadcast through DPP) ran at a quarter of that: 192 columns x 1000 tokens x 7168 rows took 79 us.
+//   workgroup = (slab of up to 64 columns, group of 512 hidden rows, a run of tiles of 32 tokens), four waves; wave w takes
+//   blocks 2w and 2w + 1 of the group as the two independent products of the instruction (lanes 0..31 supply block 2w, lanes
+//   32..63 block 2w + 1).  Row i of the first operand is column 2i (accumulator 0) or 2i + 1 (accumulator 1) of the slab: one
+//   dword per lane and hidden row feeds both, and all 64 of a block stay in registers for every tile.  A tile's hidden
+//   states are asked for as whole cache lines under the products of the tile before (a lane reading its own token's 128 bytes
+//   piece by piece takes 64 lines at a time, more than the waves of a compute unit find in its first cache again).  The
+//   eight block sums meet in LDS and are chained ascending into the group sum.
+// Bound: the matrix cores' fp32 rate: 64 clocks per instruction, 139 TFLOP/s reached by a bare loop; 4.8 us per tile and SIMD at
+// the clock that random operands leave.  256 columns x 4096 tokens x 7168 rows alone 162 us with the weights in LDS for one tile,
+// now 148 (112 TFLOP/s).  The multiply-add form of the vector ALU this replaced (hidden states broadcast through DPP) ran at a
+// quarter of the matrix cores' rate.
 constexpr int XF_TOK = 32;                                               // tokens per workgroup
 constexpr int XF_COLS = 64;                                              // columns per workgroup, at most
 constexpr int XF_WAVES = 4;
-constexpr int XF_BLOCK_PITCH = XL_BLOCK * 2 * XF_COLS + 128;             // a wave's second block lies 32 banks off the first
-constexpr int XF_STAGE = 2 * XF_BLOCK_PITCH;
 constexpr int XF_TOK_PITCH = XF_COLS * 4 + 16;                           // bytes between token rows of a block sum
 constexpr int XF_SUMS = XF_TOK * XF_TOK_PITCH;
-constexpr int XF_LDS = XF_WAVES * XF_STAGE > XL_GROUP * XF_SUMS ? XF_WAVES * XF_STAGE : XL_GROUP * XF_SUMS;   // 69 632 bytes
+constexpr int XF_LDS = XL_GROUP * XF_SUMS;                               // 69 632 bytes
 static_assert(XL_GROUP == 2 * XF_WAVES, "two blocks per wave");
 
 __host__ __device__ inline int xf_token_tiles(const int T) { return (T + XF_TOK - 1) / XF_TOK; }
 
-// The jobs of a launch: sets of columns x groups x token tiles.  Workgroups go round the eight XCDs; the sets of one
-// (group, tile) are consecutive workgroups of one XCD, so its hidden states cross into that L2 once.
-__host__ __device__ inline int xf_jobs(const int nsets, const int ngroups, const int T)
+// The jobs of a launch: sets of columns x groups x runs of token tiles.  Workgroups go round the eight XCDs; the sets of one
+// (group, run) are consecutive workgroups of one XCD, so its hidden states cross into that L2 once.
+struct XfGrid {
+    int nsets, ngroups, run;      // run: token tiles of a workgroup
+};
+__host__ __device__ inline int xf_jobs(const XfGrid &f, const int T)
 {
-    return 8 * nsets * ((ngroups * xf_token_tiles(T) + 7) / 8);
+    return 8 * f.nsets * ((f.ngroups * ((xf_token_tiles(T) + f.run - 1) / f.run) + 7) / 8);
+}
+// Token tiles of a workgroup where `cols` sets x groups share `free` places for workgroups beside the launch's other ones: two
+// where they make a single round and one more than a round and a third (fused prolog, 1 / 2 tiles: 130 tokens, a round in
+// either case, 58.3 / 63.1 us per pass, 200: 72.9 / 69.1, 256: 76.3 / 72.5, 400, two of them 1.5 rounds, 95.4 / 106.3; the
+// indexer prolog alone 400, one 1.07 rounds, 36.2 / 39.0, 512, 1.31 rounds, 39.3 / 41.3); beyond that two from 20 tiles on, for
+// which a workgroup keeps its weights (1 / 2: 1000 tokens 189.2 / 185.1, 1300 248.7 / 245.5, 4096 681.8 / 674.7).
+inline int xf_run(const int cols, const int T, const int free)
+{
+    const int tiles = xf_token_tiles(T);
+    if ((tiles + 1) / 2 * cols <= free) return 3 * tiles * cols > 4 * free ? 2 : 1;
+    return tiles < 20 ? 1 : 2;
 }
 struct XfJob {
     int set, g, t0;       // g < 0: padding of the job count
 };
-__device__ __forceinline__ XfJob xf_job(const int j, const int nsets, const int ngroups, const int T)
+__device__ __forceinline__ XfJob xf_job(const int j, const XfGrid &f, const int T)
 {
     const int q = j >> 3;
-    const int c = (q / nsets) * 8 + (j & 7);
+    const int c = (q / f.nsets) * 8 + (j & 7);
     XfJob r;
-    r.set = q % nsets;
-    r.g = c < ngroups * xf_token_tiles(T) ? c % ngroups : -1;
-    r.t0 = (c / ngroups) * XF_TOK;
+    r.set = q % f.nsets;
+    r.g = c < f.ngroups * ((xf_token_tiles(T) + f.run - 1) / f.run) ? c % f.ngroups : -1;
+    r.t0 = (c / f.ngroups) * f.run * XF_TOK;
     return r;
 }
 
-// group g of the hidden axis, tokens t0 .. t0 + 31 (rows past T - 1 repeat it and are not stored); sl.wbytes <= 128
-__device__ __forceinline__ void xf_body(const XlSlab &sl, const uint16_t *x, const int T, const int h, const int g, const int t0, uint8_t *smem)
+// group g of the hidden axis, `run` tiles of 32 tokens from t0 on (rows past T - 1 repeat it and are not stored); sl.wbytes <= 128
+__device__ __forceinline__ void xf_body(const XlSlab &sl, const uint16_t *x, const int T, const int h, const int g, const int t0, const int run,
+                                        uint8_t *smem)
 {
     typedef __attribute__((ext_vector_type(32))) float f32x32;
     const int l = threadIdx.x & 63;
@@ -178,79 +194,98 @@ __device__ __forceinline__ void xf_body(const XlSlab &sl, const uint16_t *x, con
     const int nblk = h / XL_BLOCK;
     const int nb = nblk - g * XL_GROUP < XL_GROUP ? nblk - g * XL_GROUP : XL_GROUP;
     const int wbytes = sl.wbytes;
-    f32x32 a0, a1;
+    const int tend = t0 + run * XF_TOK < T ? t0 + run * XF_TOK : T;
+    // a group's last wave may have one block only: both halves then work on it, and the second result is dropped; a wave
+    // without a block works on the group's first
+    const bool active = 2 * w < nb;
+    const int blk = active ? (half && 2 * w + 1 < nb ? 2 * w + 1 : 2 * w) : 0;
+    // the block's weights, a dword (columns 2i, 2i + 1) per row, and the hidden states of the tile's token
+    uint32_t wv[XL_BLOCK];
+    {
+        const uint8_t *row = sl.w + (size_t)g * (XL_GROUP * XL_BLOCK) * sl.pitch;         // (uniform)
+        const uint32_t off = (uint32_t)(blk * XL_BLOCK * sl.pitch + (4 * i < wbytes ? 4 * i : 0));
 #pragma unroll
-    for (int r = 0; r < 32; ++r) a0[r] = a1[r] = 0.f;
-    if (2 * w < nb) {
-        // a group's last wave may have one block only: both halves then work on it, and the second result is dropped
-        const int second = 2 * w + 1 < nb ? 2 * w + 1 : 2 * w;
-        uint8_t *region = smem + w * XF_STAGE;
-        {   // eight rows per request, 128 bytes apart in LDS (lanes past a narrow slab's row repeat its first piece)
-            const int piece = (l & 7) < (wbytes >> 4) ? l & 7 : 0;
-#pragma unroll 1
-            for (int b = 0; b < 2; ++b) {
-                const int k0 = (g * XL_GROUP + (b ? second : 2 * w)) * XL_BLOCK;
-                const uint8_t *src = sl.w + (size_t)(k0 + (l >> 3)) * sl.pitch + 16 * piece;
-                const uint32_t dst = (uint32_t)(uintptr_t)(lds_byte_t *)(region + b * XF_BLOCK_PITCH);
-#pragma unroll 1
-                for (int q = 0; q < XL_BLOCK / 8; ++q) dma16(src + (size_t)q * 8 * sl.pitch, dst + 1024 * q);
-            }
+        for (int k = 0; k < XL_BLOCK; ++k) wv[k] = *reinterpret_cast<const uint32_t *>(row + (size_t)k * sl.pitch + off);
+    }
+    // The hidden states: whole 128-byte rows of a block per eight lanes, put in order (a lane its token's) through the wave's own
+    // part of the LDS.
+    u32x4 xv[XL_BLOCK / 8], xn[XL_BLOCK / 8];
+    uint8_t *mine = smem + 2 * w * XF_SUMS;
+    const int blk1 = active && 2 * w + 1 < nb ? 2 * w + 1 : (active ? 2 * w : 0), blk0 = active ? 2 * w : 0;
+    auto load_x = [&](const int tile0) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int tl = tile0 + 8 * (q & 3) + (l >> 3), t = tl < T ? tl : T - 1;
+            xn[q] = *reinterpret_cast<const u32x4 *>(x + (size_t)t * h + (g * XL_GROUP + (q < 4 ? blk0 : blk1)) * XL_BLOCK + 8 * (l & 7));
         }
-        const int t = t0 + i < T ? t0 + i : T - 1;
-        const u32x4 *xp = reinterpret_cast<const u32x4 *>(x + (size_t)t * h + (g * XL_GROUP + (half ? second : 2 * w)) * XL_BLOCK);
-        u32x4 xv[XL_BLOCK / 8];
+    };
+    auto order_x = [&]() {
 #pragma unroll
-        for (int q = 0; q < XL_BLOCK / 8; ++q) xv[q] = xp[q];
-        VM_WAIT(0);
-        asm volatile("" ::: "memory");
-        const uint8_t *wl = region + half * XF_BLOCK_PITCH + 4 * i;
+        for (int q = 0; q < 8; ++q) {
+            const int row = 8 * q + (l >> 3);
+            *reinterpret_cast<u32x4 *>(mine + row * 128 + 16 * ((l & 7) ^ ((row >> 1) & 7))) = xn[q];
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) xv[q] = *reinterpret_cast<const u32x4 *>(mine + l * 128 + 16 * (q ^ ((l >> 1) & 7)));
+    };
+    load_x(t0);
+    order_x();
+#pragma unroll 1
+    for (int tile0 = t0; tile0 < tend; tile0 += XF_TOK) {
+        if (tile0 + XF_TOK < tend) load_x(tile0 + XF_TOK);
+        f32x32 a0, a1;
+#pragma unroll
+        for (int r = 0; r < 32; ++r) a0[r] = a1[r] = 0.f;
 #pragma unroll
         for (int k = 0; k < XL_BLOCK; ++k) {
-            const uint32_t wv = *reinterpret_cast<const uint32_t *>(wl + k * 2 * XF_COLS);
+            asm volatile("" : "+v"(wv[k]));                              // (widened here, not in front of the loop: registers)
             const uint32_t xw = xv[k >> 3][(k >> 1) & 3];
             const float xf = __uint_as_float((k & 1) ? xw & 0xffff0000u : xw << 16);
-            a0 = __builtin_amdgcn_mfma_f32_32x32x1f32(__uint_as_float(wv << 16), xf, a0, 0, 0, 0);
-            a1 = __builtin_amdgcn_mfma_f32_32x32x1f32(__uint_as_float(wv & 0xffff0000u), xf, a1, 0, 0, 0);
+            a0 = __builtin_amdgcn_mfma_f32_32x32x1f32(__uint_as_float(wv[k] << 16), xf, a0, 0, 0, 0);
+            a1 = __builtin_amdgcn_mfma_f32_32x32x1f32(__uint_as_float(wv[k] & 0xffff0000u), xf, a1, 0, 0, 0);
+            if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);           // (widened factors of a few rows at a time)
         }
-    }
-    __syncthreads();                                                     // every wave is done with its weights
-    if (2 * w < nb) {
-        // register 16*b + 4*q + j of lane (token, half) is row 8*q + 4*half + j of block b's product
+        if (active) {
+            // register 16*b + 4*q + j of lane (token, half) is row 8*q + 4*half + j of block b's product
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            uint8_t *row = smem + (2 * w + b) * XF_SUMS + i * XF_TOK_PITCH + 32 * half;
+            for (int b = 0; b < 2; ++b) {
+                uint8_t *row = smem + (2 * w + b) * XF_SUMS + i * XF_TOK_PITCH + 32 * half;
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
+                for (int q = 0; q < 4; ++q)
 #pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    const int r = 16 * b + 4 * q + 2 * e;
-                    const f32x4 v = {a0[r], a1[r], a0[r + 1], a1[r + 1]};
-                    *reinterpret_cast<f32x4 *>(row + 64 * q + 16 * e) = v;
-                }
-        }
-    }
-    __syncthreads();
-    {   // thread (token, eight columns) chains the block sums in ascending order
-        const int tl = threadIdx.x >> 3, c8 = 8 * (threadIdx.x & 7);
-        const int t = t0 + tl;
-        if (t < T && 2 * c8 < wbytes) {
-            float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            for (int b = 0; b < nb; ++b) {
-                const f32x4 *src = reinterpret_cast<const f32x4 *>(smem + b * XF_SUMS + tl * XF_TOK_PITCH + 4 * c8);
-#pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    const f32x4 v = src[e];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) s[4 * e + j] = __fadd_rn(s[4 * e + j], v[j]);
-                }
-            }
-            f32x4 *dst = reinterpret_cast<f32x4 *>(sl.out + (size_t)t * sl.out_pitch + c8);
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const f32x4 v = {s[4 * e], s[4 * e + 1], s[4 * e + 2], s[4 * e + 3]};
-                dst[e] = v;
+                    for (int e = 0; e < 2; ++e) {
+                        const int r = 16 * b + 4 * q + 2 * e;
+                        const f32x4 v = {a0[r], a1[r], a0[r + 1], a1[r + 1]};
+                        *reinterpret_cast<f32x4 *>(row + 64 * q + 16 * e) = v;
+                    }
             }
         }
+        __syncthreads();
+        {   // thread (token, eight columns) chains the block sums in ascending order
+            const int tl = threadIdx.x >> 3, c8 = 8 * (threadIdx.x & 7);
+            const int t = tile0 + tl;
+            if (t < T && 2 * c8 < wbytes) {
+                float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                for (int b = 0; b < nb; ++b) {
+                    const f32x4 *src = reinterpret_cast<const f32x4 *>(smem + b * XF_SUMS + tl * XF_TOK_PITCH + 4 * c8);
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        const f32x4 v = src[e];
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) s[4 * e + j] = __fadd_rn(s[4 * e + j], v[j]);
+                    }
+                }
+                f32x4 *dst = reinterpret_cast<f32x4 *>(sl.out + (size_t)t * sl.out_pitch + c8);
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const f32x4 v = {s[4 * e], s[4 * e + 1], s[4 * e + 2], s[4 * e + 3]};
+                    dst[e] = v;
+                }
+            }
+        }
+        if (tile0 + XF_TOK >= tend) break;
+        __syncthreads();                                                 // the sums have been read
+        order_x();
     }
 }
 

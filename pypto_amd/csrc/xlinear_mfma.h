@@ -162,45 +162,41 @@ __device__ __forceinline__ void xm_body(const XmSlab &sl, const uint16_t *x, con
 }
 
 // ---------------------------------------------------------------------------------------------
-// The same for tiles of 256 tokens: wave (wc, wt) holds columns 64*wc .. +63 x tokens 128*wt .. +127 (eight accumulators), so
-// a byte of LDS-DMA, which these launches are bound by, serves a third more products.  Chunks of 32 hidden rows in a ring of
-// three, two on their way while one is consumed, one barrier each.  The ring leaves room for a workgroup of the fixed-order
-// sums on the same compute unit: those keep the matrix cores busy and move next to nothing.
-constexpr int XB_TOK = 256;
-constexpr int XB_KC = 32;
-constexpr int XB_W_BYTES = XB_KC * 256;
-constexpr int XB_BUF = XB_W_BYTES + XB_TOK * XB_KC * 2;
-constexpr int XB_NBUF = 3;
-constexpr int XB_LDS = XB_NBUF * XB_BUF;
+// The same for more tokens: tiles of 128 tokens x 256 columns, wave w columns 64*w .. +63 of all the tokens (eight accumulators),
+// so a byte of LDS-DMA serves a third more products.  The tokens travel 64 hidden rows -- a whole cache line -- at a time into two
+// buffers, the slab 32 rows at a time into a ring of three: asked for 64 bytes of a row at a time, the second half of a line while
+// the first is on its way, hidden states come at 16 bytes per clock and compute unit, however many chunks are ahead and whether
+// they lie in the L2 or not (tiles of 256 tokens x 128 columns, as before: 4096 tokens alone 157 us, requests alone 153, products
+// alone 89; now 132 and 122, out of the L2 59: bound by the latency of the first miss of every line).  Half of a compute unit's
+// LDS: the other half is for the fixed-order sums, which keep the matrix cores busy and move next to nothing.
+// Fused prolog with both, before / now: 200 tokens 71.9 / 68.8 us per pass, 400 100.7 / 94.0, 1000 192.2 / 185.7, 4096 689 / 658.
+constexpr int XB_TOK = 128;
+constexpr int XB_COLS = 256;
+constexpr int XB_KC = 32;                        // hidden rows per chunk of the slab; the tokens take two chunks at a time
+constexpr int XB_W_BYTES = XB_KC * XB_COLS * 2;
+constexpr int XB_X_BYTES = XB_TOK * 2 * XB_KC * 2;
+constexpr int XB_LDS = 2 * XB_X_BYTES + 3 * XB_W_BYTES;                      // 81 920 bytes
 
-// hidden rows [XB_KC * c_begin, XB_KC * c_end), tokens t0 .. t0 + 255; the slab has all of its 128 columns
+// hidden rows [2 * XB_KC * c_begin, 2 * XB_KC * c_end), tokens t0 .. t0 + 127; sl.w, sl.out: column 0 of the 256
 __device__ __forceinline__ void xb_body(const XmSlab &sl, const uint16_t *x, const int T, const int h, const int t0, const int c_begin,
                                         const int c_end, uint8_t *smem)
 {
     const int l = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int half = l >> 5;
-    const int wc = w & 1, wt = w >> 1;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_byte_t *)smem;
-    // a wave's six requests of a chunk: two of the slab (four rows each), four of the tokens (sixteen rows of 64 bytes each,
-    // 16-byte piece q of token row t at q ^ ((t >> 2) & 3))
-    const uint8_t *wreq[2], *xreq[4];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) wreq[j] = sl.w + (size_t)(4 * (2 * w + j) + (l >> 4)) * sl.pitch + 16 * ((l & 15) ^ (4 * (l >> 4)));
+    // a wave's four requests of a chunk of the slab (two rows of 512 bytes each; 16-byte piece q of row r at q ^ 4*(r & 3)) and four
+    // of the tokens (eight rows of 128 bytes; piece q of token row t at q ^ ((t >> 1) & 7))
+    const uint8_t *wreq[4], *xreq[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const int tl = 16 * (4 * w + j) + (l >> 2);
+        const int row = 2 * (4 * w + j) + half;
+        wreq[j] = sl.w + (size_t)(2 * XB_KC * c_begin + row) * sl.pitch + 16 * ((l & 31) ^ (4 * (row & 3)));
+        const int tl = 8 * (4 * w + j) + (l >> 3);
         const int t = t0 + tl < T ? t0 + tl : T - 1;
-        xreq[j] = reinterpret_cast<const uint8_t *>(x) + (size_t)t * h * 2 + 16 * ((l & 3) ^ ((tl >> 2) & 3));
+        xreq[j] = reinterpret_cast<const uint8_t *>(x) + ((size_t)t * h + 2 * XB_KC * c_begin) * 2 + 16 * ((l & 7) ^ ((tl >> 1) & 7));
     }
     const size_t wstep = (size_t)XB_KC * sl.pitch;
-    auto request_chunk = [&](const int c, const int buf) {
-        const uint32_t dst = lds0 + (uint32_t)(buf * XB_BUF);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) dma16(wreq[j] + (size_t)c * wstep, dst + 1024u * (2 * w + j));
-#pragma unroll
-        for (int j = 0; j < 4; ++j) dma16(xreq[j] + (size_t)c * (XB_KC * 2), dst + XB_W_BYTES + 1024u * (4 * w + j));
-    };
     f32x16 acc[2][4];
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb)
@@ -208,42 +204,44 @@ __device__ __forceinline__ void xb_body(const XmSlab &sl, const uint16_t *x, con
         for (int tb = 0; tb < 4; ++tb)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[cb][tb][r] = 0.f;
+    // A: row 16*ks + 8*half + (l&15)>>2 (+4), column 64*w + 32*cb + 16*((l>>4)&1) + 4*(l&3)
     uint32_t aoff[2];
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb) {
-        const int piece = 8 * wc + 4 * cb + 2 * ((l >> 4) & 1) + ((l & 3) >> 1);
-        aoff[cb] = (uint32_t)((8 * half + ((l & 15) >> 2)) * 256 + 16 * (piece ^ (4 * ((l & 15) >> 2))) + 8 * (l & 1));
+        const int piece = 8 * w + 4 * cb + 2 * ((l >> 4) & 1) + ((l & 3) >> 1);
+        aoff[cb] = (uint32_t)(2 * XB_X_BYTES + (8 * half + ((l & 15) >> 2)) * (2 * XB_COLS) + 16 * (piece ^ (4 * ((l & 15) >> 2))) + 8 * (l & 1));
     }
-    const uint32_t boff = XB_W_BYTES + (128 * wt + (l & 31)) * (XB_KC * 2);
-    if (c_begin < c_end) request_chunk(c_begin, 0);
-    if (c_begin + 1 < c_end) request_chunk(c_begin + 1, 1);
-    int buf = 0;
-#pragma unroll 1
-    for (int c = c_begin; c < c_end; ++c) {
-        if (c + 1 < c_end) VM_WAIT(6);
-        else VM_WAIT(0);
-        __syncthreads();                                           // chunk c has landed; every wave is done with chunk c - 1
-        if (c + 2 < c_end) request_chunk(c + 2, buf == 0 ? 2 : buf - 1);
-        const uint8_t *bp = smem + buf * XB_BUF;
+    const uint32_t boff = (l & 31) * (4 * XB_KC);
+    const int bswz = (l >> 1) & 7;
+    staged_chunks<2, 4, 4>(
+        2 * (c_end - c_begin),
+        [&](const int s, const int b) {
 #pragma unroll
-        for (int ks = 0; ks < XB_KC / 16; ++ks) {
-            bf16x8 a[2];
+            for (int j = 0; j < 4; ++j) dma16(xreq[j] + (size_t)s * (4 * XB_KC), lds0 + b * XB_X_BYTES + 1024u * (4 * w + j));
+        },
+        [&](const int c, const int slot) {
 #pragma unroll
-            for (int cb = 0; cb < 2; ++cb) {
-                const uint16_t *ap = reinterpret_cast<const uint16_t *>(bp + aoff[cb] + 16 * ks * 256);
-                const s16x4 lo = lds_read_tr16(ap), hi = lds_read_tr16(ap + 4 * 128);
-                a[cb] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+            for (int j = 0; j < 4; ++j) dma16(wreq[j] + c * wstep, lds0 + 2 * XB_X_BYTES + slot * XB_W_BYTES + 1024u * (4 * w + j));
+        },
+        [&](const int odd, const int xb, const int slot) {
+            const uint8_t *wp = smem + slot * XB_W_BYTES, *xp = smem + xb * XB_X_BYTES + boff;
+#pragma unroll
+            for (int ks = 0; ks < XB_KC / 16; ++ks) {
+                bf16x8 a[2];
+#pragma unroll
+                for (int cb = 0; cb < 2; ++cb) {
+                    const uint16_t *ap = reinterpret_cast<const uint16_t *>(wp + aoff[cb] + 16 * ks * (2 * XB_COLS));
+                    const s16x4 lo = lds_read_tr16(ap), hi = lds_read_tr16(ap + 4 * XB_COLS);
+                    a[cb] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                }
+#pragma unroll
+                for (int tb = 0; tb < 4; ++tb) {
+                    const bf16x8 b = *reinterpret_cast<const bf16x8 *>(xp + 32 * tb * (4 * XB_KC) + 16 * ((4 * odd + 2 * ks + half) ^ bswz));
+#pragma unroll
+                    for (int cb = 0; cb < 2; ++cb) acc[cb][tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[cb], b, acc[cb][tb], 0, 0, 0);
+                }
             }
-#pragma unroll
-            for (int tb = 0; tb < 4; ++tb) {
-                const bf16x8 b = *reinterpret_cast<const bf16x8 *>(bp + boff + 32 * tb * (XB_KC * 2) + 16 * ((2 * ks + half) ^ ((l >> 2) & 3)));
-#pragma unroll
-                for (int cb = 0; cb < 2; ++cb) acc[cb][tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[cb], b, acc[cb][tb], 0, 0, 0);
-            }
-        }
-        buf = buf == 2 ? 0 : buf + 1;
-    }
-    __syncthreads();                                               // every wave is done with the last chunk
+        });
     static_assert(4 * 32 * XM_SPITCH <= XB_LDS, "the staging areas reuse the chunk buffers");
     uint8_t *stg = smem + w * (32 * XM_SPITCH);
 #pragma unroll
@@ -261,8 +259,8 @@ __device__ __forceinline__ void xb_body(const XmSlab &sl, const uint16_t *x, con
         for (int k = 0; k < 8; ++k) {
             const int r = 4 * k + (l >> 4);
             const f32x4 v = *reinterpret_cast<const f32x4 *>(stg + r * XM_SPITCH + 16 * (l & 15));
-            const int t = t0 + 128 * wt + 32 * tb + r;
-            if (t < T) *reinterpret_cast<f32x4 *>(sl.out + (size_t)t * sl.out_pitch + 64 * wc + 4 * (l & 15)) = v;
+            const int t = t0 + 32 * tb + r;
+            if (t < T) *reinterpret_cast<f32x4 *>(sl.out + (size_t)t * sl.out_pitch + 64 * w + 4 * (l & 15)) = v;
         }
     }
 }

@@ -619,3 +619,9 @@ def test_fused_entry_point_through_the_c_abi_keeps_the_intermediates_in_its_work
     # a workspace one byte short is refused, nothing is launched
     a.workspace_bytes = need.value - 1
     assert lib.pto_mla_indexer_prolog_quant_launch(ctypes.byref(a), None) == -2
+
+
+@pytest.mark.parametrize("t,n_idx", [(1500, 64), (2500, 8)])
+def test_fused_prolog_fixed_order_sums_of_several_tiles_per_workgroup(t, n_idx):
+    """The same where a workgroup takes two token tiles: an odd number of them, a ragged last one."""
+    test_fused_prolog_fixed_order_sums_at_tile_edges(t, n_idx)
