@@ -264,23 +264,23 @@ __device__ __forceinline__ void lip_finish_body(const LipParams &p, const int q_
     }
 }
 
-// The key rows and weights where the queries are finished by their projection's launch: a workgroup of FINT_WAVES waves takes FINT_WAVES tokens, one per wave (the
+// The key rows and weights where the queries are finished by their projection's launch: a workgroup of four or eight waves takes as many tokens, one per wave (the
 // matrix is staged once for all of them instead of once per token, and the rows are finished side by side instead of
 // by one wave per workgroup).  A wave adds its token's partial rows in registers, in the order of the form they come
 // in: group sums ascending, or blocks / ranges ascending into groups of eight and the groups ascending.
-constexpr int FINT_WAVES = 4;
-constexpr int LIP_FINT_LDS = LIP_DIM * LIP_DIM * 2 + FINT_WAVES * LIP_DIM * 4;
+template <int WAVES> constexpr int LIP_FINT_LDS = LIP_DIM * LIP_DIM * 2 + WAVES * LIP_DIM * 4;
 
+template <int WAVES>
 __device__ __forceinline__ void lip_finish_tokens_prefill_body(const LipParams &p, const int wg, uint8_t *lds)
 {
     uint16_t *hmat = reinterpret_cast<uint16_t *>(lds);
     float(*arow)[LIP_DIM] = reinterpret_cast<float(*)[LIP_DIM]>(lds + LIP_DIM * LIP_DIM * 2);
     const int l = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int t = wg * FINT_WAVES + w;
+    const int t = wg * WAVES + w;
     const bool live = t < p.T;
     const int tt = live ? t : p.T - 1;
-    stage_matrix<FINT_WAVES>(hmat, p.hk);
+    stage_matrix<WAVES>(hmat, p.hk);
     const bool pl = l < p.n_heads;
     const uint32_t rc = rope_coef(p.cos, tt, l), rs = rope_coef(p.sin, tt, l);
     const uint32_t gm = reinterpret_cast<const uint32_t *>(p.gamma)[l];

@@ -45,33 +45,34 @@ __global__ __launch_bounds__(64 * FIN_WAVES) void prolog_fused_finish_kernel(con
 // Projections and last stages at prefill sizes (prolog_prefill.h): [0, mla_wgs) the attention query, then lip_wgs of the
 // indexer query, then the indexer's key rows and weights, a token per wave.  64 * TB tokens per workgroup of a head of the
 // attention query, 128 * LTB of the indexer's.
+// HB: heads per workgroup of four waves each, which share the tokens.
 // FIXED: the indexer query's Hadamard sums in their fixed order (fewer than LIP_MFMA_MIN_TOKENS tokens).
-constexpr int pf_xc(const int ltb) { return ltb == 1 ? 2 : 1; }
-template <int XC, int TB, int LTB>
-constexpr int PF_LDS2 = PFA_LDS<XC, TB> > PFI_LDS<pf_xc(LTB), LTB> ? PFA_LDS<XC, TB> : PFI_LDS<pf_xc(LTB), LTB>;
-template <int XC, int TB, int LTB> constexpr int PF_LDS = PF_LDS2<XC, TB, LTB> > LIP_FINT_LDS ? PF_LDS2<XC, TB, LTB> : LIP_FINT_LDS;
-template <int XC, int TB, int LTB, bool FIXED>
-__global__ __launch_bounds__(256, 2) void prolog_prefill_kernel(const MlapParams pm, const LipParams pl, const int mla_wgs, const int lip_wgs)
+constexpr int pf_xc(const int ltb, const int hb) { return ltb == 1 || hb == 2 ? 2 : 1; }
+template <int XC, int TB, int LTB, int HB>
+constexpr int PF_LDS2 = PFA_LDS<XC, TB, HB> > PFI_LDS<pf_xc(LTB, HB), LTB, HB> ? PFA_LDS<XC, TB, HB> : PFI_LDS<pf_xc(LTB, HB), LTB, HB>;
+template <int XC, int TB, int LTB, int HB>
+constexpr int PF_LDS = PF_LDS2<XC, TB, LTB, HB> > LIP_FINT_LDS<4 * HB> ? PF_LDS2<XC, TB, LTB, HB> : LIP_FINT_LDS<4 * HB>;
+template <int XC, int TB, int LTB, int HB, bool FIXED>
+__global__ __launch_bounds__(256 * HB, 2) void prolog_prefill_kernel(const MlapParams pm, const LipParams pl, const int mla_wgs, const int lip_wgs)
 {
-    static_assert(2 * PF_LDS<XC, TB, LTB> <= 160 * 1024, "two workgroups share a compute unit");
-    static_assert(FINT_WAVES == 4, "one block size for the three bodies");
-    __shared__ __attribute__((aligned(16))) uint8_t lds[PF_LDS<XC, TB, LTB>];
+    static_assert(2 / HB * PF_LDS<XC, TB, LTB, HB> <= 160 * 1024, "eight waves share a compute unit");
+    __shared__ __attribute__((aligned(16))) uint8_t lds[PF_LDS<XC, TB, LTB, HB>];
     const int wg = (int)blockIdx.x;
-    if (wg < mla_wgs) mlap_prefill_body<XC, TB>(pm, q_prefill_job_of(wg, mla_wgs), lds);
-    else if (wg < mla_wgs + lip_wgs) lip_prefill_body<pf_xc(LTB), LTB, FIXED>(pl, q_prefill_job_of(wg - mla_wgs, lip_wgs), lds);
-    else lip_finish_tokens_prefill_body(pl, wg - mla_wgs - lip_wgs, lds);
+    if (wg < mla_wgs) mlap_prefill_body<XC, TB, HB>(pm, q_prefill_job_of(wg, mla_wgs), lds);
+    else if (wg < mla_wgs + lip_wgs) lip_prefill_body<pf_xc(LTB, HB), LTB, HB, FIXED>(pl, q_prefill_job_of(wg - mla_wgs, lip_wgs), lds);
+    else lip_finish_tokens_prefill_body<4 * HB>(pl, wg - mla_wgs - lip_wgs, lds);
 }
 
 // The same for at most PROLOG_SMALL_TOKENS tokens (prolog_small.h), a workgroup per head.
 constexpr int PS_LDS = PSA_LDS > PSI_LDS ? PSA_LDS : PSI_LDS;
-static_assert(LIP_FINT_LDS <= PS_LDS, "the token workgroups fit");
+static_assert(LIP_FINT_LDS<4> <= PS_LDS, "the token workgroups fit");
 __global__ __launch_bounds__(256) void prolog_small_kernel(const MlapParams pm, const LipParams pl, const int mla_wgs, const int lip_wgs)
 {
     __shared__ __attribute__((aligned(16))) uint8_t lds[PS_LDS];
     const int wg = (int)blockIdx.x;
     if (wg < mla_wgs) mlap_small_body(pm, prolog_small_head(wg, pm.n_heads), lds);
     else if (wg < mla_wgs + lip_wgs) lip_small_body(pl, wg - mla_wgs, lds);
-    else lip_finish_tokens_prefill_body(pl, wg - mla_wgs - lip_wgs, lds);
+    else lip_finish_tokens_prefill_body<4>(pl, wg - mla_wgs - lip_wgs, lds);
 }
 
 }  // namespace
@@ -86,32 +87,37 @@ hipError_t prolog_prefill_launch(const MlapParams *pm, const LipParams *pl, hipS
     if (pm) m = *pm;
     if (pl) p = *pl;
     if (T <= PROLOG_SMALL_TOKENS) {
-        const int mla = pm ? m.n_heads : 0, lip = pl ? p.n_heads : 0, tok = pl ? (T + FINT_WAVES - 1) / FINT_WAVES : 0;
+        const int mla = pm ? m.n_heads : 0, lip = pl ? p.n_heads : 0, tok = pl ? (T + 3) / 4 : 0;
         hipLaunchKernelGGL(prolog_small_kernel, dim3((unsigned)(mla + lip + tok)), dim3(256), 0, stream, m, p, mla, lip);
         return hipGetLastError();
     }
     // Up to 64 tokens the attention query's tiles have 64 (in tiles of 128, half and more of them padding: fused prolog 33 tokens 41.4
     // us per pass, now 40.6, 48: 43.3 and 42.4, 64: 44.6 and 43.6; MLA prolog alone 33: 35.9 and 34.1, 64: 39.9 and 38.7).
-    // 256-token tiles take 12 % less time per (padded) token than 128-token ones where both fill the chip, which up to 256
-    // tokens they do not (256 tokens: 79.6 us per pass against 77.5; 600: 150.4 against 140.3; 1000: 188.5 against 206.6)
-    const bool small = T <= 256 || 100 * ((T + 127) / 128) <= 176 * ((T + 255) / 256);
+    // Tiles of 256 tokens from 257 on (tiles of 128, 307 tokens 91.5 us per pass, now 85.4, 384: 99.3 and 90.7, 600: 132.4 and 131.4,
+    // 800: 165.0 and 160.5; 256 tokens the other way, 72.5 and 92.4: a tile per head leaves half of the chip's places empty).
+    const bool small = T <= 256;
     const int tok = small ? 128 : 256;
     const int tiles = (T + tok - 1) / tok;
-    const int mla_wgs = pm ? m.n_heads * tiles : 0;
-    // Tiles of 256 tokens leave few workgroups at the first sizes that take them: there the indexer's half, whose workgroups are
-    // the shorter ones, is cut into tiles of 128.  The fused prolog with 256-token and 128-token tiles of the indexer's half:
-    // 390 tokens 104.3 us per pass and 101.8, 512: 116.6 and 108.0, 700: 151.2 and 147.1, 1024: 192.9 and 194.3, 2000: 356.7 and
-    // 360.9; the indexer prolog alone 400: 45.3 and 36.4, 512: 46.2 and 37.5, 1536: 85.5 and 84.4, 2000: 107.0 and 110.3.
-    const bool lip_small = small || tiles <= (pm ? 3 : 6);
-    const int lip_wgs = pl ? p.n_heads * (lip_small ? (T + 127) / 128 : tiles) : 0;
-    const int tok_wgs = pl ? (T + FINT_WAVES - 1) / FINT_WAVES : 0;
+    // Two heads to a workgroup of eight waves, which then reads each token once and as whole cache lines, from four tiles on (one /
+    // two, on a fast card: 680 tokens 142.3 / 143.3 us per pass, 1000 185.3 / 177.2, 1300 251.1 / 238.1, 1500 273.2 / 259.1, 2112 375.6 /
+    // 365.3, 4096 662.9 / 659.9; on a slow one: 1000 196.1 / 194.9, 1300 265.9 / 258.8, 1500 288.5 / 276.8, 2112 397.1 / 399.2).
+    const int hb = pm && tiles >= 4 ? 2 : 1;
+    const int mla_wgs = pm ? m.n_heads / hb * tiles : 0;
+    // The indexer's half, whose workgroups are the shorter ones, is cut into tiles of 128 tokens up to six tiles of 256 (fused prolog,
+    // tiles of 256 / 128: 1000 tokens 195.9 / 187.6 us per pass, 1300 252.3 / 243.9, 1500 271.3 / 265.7, 1800 315.8 / 322.2, 4096 652.3 /
+    // 668.8; the indexer prolog alone 400: 45.3 / 36.4, 512: 46.2 / 37.5, 1536: 85.5 / 84.4, 2000: 107.0 / 110.3).
+    const bool lip_small = small || tiles <= 6;
+    const int lip_wgs = pl ? (p.n_heads + hb - 1) / hb * (lip_small ? (T + 127) / 128 : tiles) : 0;
+    const int tok_wgs = pl ? (T + 4 * hb - 1) / (4 * hb) : 0;
     const dim3 g((unsigned)(mla_wgs + lip_wgs + tok_wgs));
-    auto run = [&](auto *kernel) { hipLaunchKernelGGL(kernel, g, dim3(256), 0, stream, m, p, mla_wgs, lip_wgs); };
-    if (T < LIP_MFMA_MIN_TOKENS) run(prolog_prefill_kernel<2, 1, 1, true>);
-    else if (T <= PFA_TOK<1>) run(prolog_prefill_kernel<2, 1, 1, false>);
-    else if (small) run(prolog_prefill_kernel<2, 2, 1, false>);
-    else if (lip_small) run(prolog_prefill_kernel<1, 4, 1, false>);
-    else run(prolog_prefill_kernel<1, 4, 2, false>);
+    auto run = [&](auto *kernel) { hipLaunchKernelGGL(kernel, g, dim3(256 * hb), 0, stream, m, p, mla_wgs, lip_wgs); };
+    if (T < LIP_MFMA_MIN_TOKENS) run(prolog_prefill_kernel<2, 1, 1, 1, true>);
+    else if (T <= PFA_TOK<1>) run(prolog_prefill_kernel<2, 1, 1, 1, false>);
+    else if (small) run(prolog_prefill_kernel<2, 2, 1, 1, false>);
+    else if (hb == 2 && lip_small) run(prolog_prefill_kernel<2, 4, 1, 2, false>);
+    else if (hb == 2) run(prolog_prefill_kernel<2, 4, 2, 2, false>);
+    else if (lip_small) run(prolog_prefill_kernel<1, 4, 1, 1, false>);
+    else run(prolog_prefill_kernel<1, 4, 2, 1, false>);
     return hipGetLastError();
 }
 

@@ -3,15 +3,18 @@
 // Hadamard matrix and quantised (indexer query) -- instead of going to memory as bf16 for a launch of its own.
 // Included by prolog_fused.hip after prolog_finish.h.
 //
-// Both bodies are one workgroup of four waves per (head, tile of tokens), two workgroups to a compute unit.  The projection
-// walks the whole reduction axis in chunks of 64 rows (LDS-DMA, v_mfma_i32_32x32x32_i8 as in prolog_common.h), the weights in
-// a ring of three chunks, the tokens in two buffers.  The token tiles of a head run on one XCD, which reads its weights once.
-// Measured with parts left out (4096 tokens, attention query, 300 us): chunk loop 125, stores of q_nope 80 (7.5 TB/s),
-// absorb product 23-40, de-quantisation, rope and w_uk 45-70; they add up, two workgroups or one to the compute unit.
-// LDS-DMA out of the L2 runs at 31-36 TB/s where every cache line it touches is taken whole and at half of that in half
-// lines, which is why 128-token tiles take 128 bytes of a token row at a time (256-token tiles have no room for it).
-// Two heads and 256 tokens per workgroup of eight waves: 1000 tokens +5 %, 4096 -1.7 %, not kept.
-// As two launches with bf16 between them, as before, 1000 tokens took 281 us per pass, now 189; 4096: 906 and 686.
+// Both bodies are one workgroup of four waves per (head, tile of tokens), two workgroups to a compute unit, or of eight per (two
+// heads, tile).  The projection walks the whole reduction axis in chunks of 64 rows (LDS-DMA, v_mfma_i32_32x32x32_i8 as in
+// prolog_common.h), the weights in a ring of three chunks, the tokens in two buffers.  The token tiles of a head run on one XCD,
+// which reads its weights once.
+// Measured with parts left out (4096 tokens, attention query, one / two heads to a workgroup): in all 297 / 274 us, chunk loop 141 / 133,
+// of it requests and LDS reads 97 / 73; stores of q_nope 80 (6.7 TB/s), the rest of what follows the loop 78.  The parts add up: all
+// workgroups are in the same one at a time, and workgroups of either query taken in turn, or half of them started 30 us
+// late, change nothing at 4096 tokens and cost 8 % at 1000.  In the loop the matrix cores are busy 64 % of the clocks, at the
+// 1.77 GHz that is left then.
+// LDS-DMA out of the L2 runs at 31-36 TB/s where every cache line it touches is taken whole and at half of that in half lines:
+// a workgroup of 256 tokens and one head has room for 64 bytes of a token row at a time only, the others take 128.
+// As two launches with bf16 between them, as before, 1000 tokens took 281 us per pass, now 177 to 195; 4096: 906 and 652 to 700.
 #pragma once
 #include "prolog_finish.h"
 
@@ -48,20 +51,21 @@ struct PfTokens {
 };
 
 // ------------------------------------------------------------------------------------------------ attention query
-// Wave (wc, wt) holds columns 96*wc .. +95 of the head's 192 x TB blocks of 32 tokens (3 * TB accumulators).
-// Row r of a chunk of weights lies at 192 * r, its 32-byte block b at b ^ ((r >> 2) & 1): the eight consecutive rows of a
-// transposing read then fall on different banks.
+// Wave (wc, wt) of the 4 * HB holds columns 96*wc .. +95 of the HB heads' 192 each x TB blocks of 32 tokens (3 * TB accumulators).
+// Row r of a chunk of weights lies at 192 * HB * r, its 32-byte block b at b ^ ((r >> 2) & 1), two heads: b ^ ((r >> 1) & 3): the
+// eight consecutive rows of a transposing read then fall on different banks.
 // Then the rope channels meet in LDS as rows, are rotated and leave; then the tile's 128 nope channels become an operand
-// [token][256 bytes] in LDS, 16-byte piece q at q ^ (t & 15), with the channels of every 16 in the order the halves of a wave
-// want them (0-3 8-11 | 4-7 12-15); each wave takes 128 output columns with its part of w_uk in registers:
+// [head][token][256 bytes] in LDS, 16-byte piece q at q ^ (t & 15), with the channels of every 16 in the order the halves of a wave
+// want them (0-3 8-11 | 4-7 12-15); each wave takes 128 output columns of a head with its part of w_uk in registers:
 // lane n's columns are 4n .. 4n+3, so a row leaves as 256 contiguous bytes.
 template <int TB> constexpr int PFA_TOK = 64 * TB;
 template <int XC, int TB> constexpr int PFA_X = PFA_TOK<TB> * PF_XPITCH<XC>;
-constexpr int PFA_W = PF_KC * MLAP_QHEAD;
+template <int HB> constexpr int PFA_WPITCH = HB * MLAP_QHEAD;
+template <int HB> constexpr int PFA_W = PF_KC * PFA_WPITCH<HB>;
 constexpr int PFA_RPITCH = 144;                        // bytes between rope rows
-template <int TB> constexpr int PFA_Q = PFA_TOK<TB> * MLAP_NOPE * 2;
-template <int XC, int TB> constexpr int PFA_LOOP_LDS = 2 * PFA_X<XC, TB> + 3 * PFA_W;
-template <int XC, int TB> constexpr int PFA_LDS = PFA_LOOP_LDS<XC, TB> > PFA_Q<TB> ? PFA_LOOP_LDS<XC, TB> : PFA_Q<TB>;
+template <int TB, int HB> constexpr int PFA_Q = HB * PFA_TOK<TB> * MLAP_NOPE * 2;
+template <int XC, int TB, int HB> constexpr int PFA_LOOP_LDS = 2 * PFA_X<XC, TB> + 3 * PFA_W<HB>;
+template <int XC, int TB, int HB> constexpr int PFA_LDS = PFA_LOOP_LDS<XC, TB, HB> > PFA_Q<TB, HB> ? PFA_LOOP_LDS<XC, TB, HB> : PFA_Q<TB, HB>;
 static_assert(PFA_RPITCH <= MLAP_NOPE * 2, "the rope rows fit where the nope operand goes");
 
 // Lane (row, e) of the rope rows at `rows` rotates pairs 4e .. 4e+3 of token t (channels 2j, 2j+1 are the partners j, 32 + j) and
@@ -87,16 +91,16 @@ __device__ __forceinline__ void pfa_rotate_rows(const MlapParams &p, const uint8
     }
 }
 
-template <int XC, int TB>
+template <int XC, int TB, int HB>
 __device__ __forceinline__ void mlap_prefill_body(const MlapParams &p, const int job, uint8_t *lds)
 {
     const int l = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int half = l >> 5;
-    const int wc = w & 1, wt = w >> 1;
+    const int wc = w & (2 * HB - 1), wt = w / (2 * HB);
     const int ncols = p.n_heads * MLAP_QHEAD;
     const int ttiles = (p.T + PFA_TOK<TB> - 1) / PFA_TOK<TB>;
-    const int head = job / ttiles;
+    const int head0 = (job / ttiles) * HB;             // (their number is even)
     const int t0 = (job % ttiles) * PFA_TOK<TB>;
     const uint32_t base = (uint32_t)(uintptr_t)(lds_byte_t *)lds;
     auto token = [&](const int tl) { return t0 + tl < p.T ? t0 + tl : p.T - 1; };
@@ -112,38 +116,38 @@ __device__ __forceinline__ void mlap_prefill_body(const MlapParams &p, const int
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[tb][i][r] = 0;
     {
-        constexpr int XR = XC * TB;
-        constexpr int PPR = MLAP_QHEAD / 16;         // 16-byte pieces of a weight row
+        constexpr int XR = XC * TB / HB, WR = 3;
+        constexpr int PPR = PFA_WPITCH<HB> / 16;     // 16-byte pieces of a weight row
         const PfTokens<XC, XR> xt(p.q_norm, p.q_lora, p.T, t0, XR * w, l);
         const int8_t *wsrc[3];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             const int piece = 64 * (3 * w + j) + l, row = piece / PPR, pos = piece % PPR;
-            wsrc[j] = p.w_uqqr + (size_t)row * ncols + head * MLAP_QHEAD + 16 * (pos ^ (2 * ((row >> 2) & 1)));
+            wsrc[j] = p.w_uqqr + (size_t)row * ncols + head0 * MLAP_QHEAD + 16 * (pos ^ (2 * (HB == 1 ? (row >> 2) & 1 : (row >> 1) & 3)));
         }
         const size_t wstep = (size_t)PF_KC * ncols;
         uint32_t aoff[3];
 #pragma unroll
         for (int i = 0; i < 3; ++i)
-            aoff[i] = 2 * PFA_X<XC, TB> + (16 * half + ((l & 15) >> 1)) * MLAP_QHEAD + 32 * ((3 * wc + i) ^ ((l >> 3) & 1)) + 16 * ((l >> 4) & 1) + 8 * (l & 1);
+            aoff[i] = 2 * PFA_X<XC, TB> + (16 * half + ((l & 15) >> 1)) * PFA_WPITCH<HB> + 32 * ((3 * wc + i) ^ (HB == 1 ? (l >> 3) & 1 : (l >> 2) & 3)) + 16 * ((l >> 4) & 1) + 8 * (l & 1);
         const uint32_t boff = (32 * TB * wt + (l & 31)) * PF_XPITCH<XC>;
         typedef int v2i __attribute__((ext_vector_type(2)));
-        staged_chunks<XC, XR, 3>(
+        staged_chunks<XC, XR, WR>(
             p.q_lora / PF_KC, [&](const int s, const int b) { xt.request(s, base + b * PFA_X<XC, TB> + 1024 * XR * w); },
             [&](const int c, const int slot) {
 #pragma unroll
-                for (int j = 0; j < 3; ++j) dma16(wsrc[j] + c * wstep, base + 2 * PFA_X<XC, TB> + slot * PFA_W + 1024 * (3 * w + j));
+                for (int j = 0; j < 3; ++j) dma16(wsrc[j] + c * wstep, base + 2 * PFA_X<XC, TB> + slot * PFA_W<HB> + 1024 * (3 * w + j));
             },
             [&](const int odd, const int xb, const int slot) {
-                const uint8_t *wp = lds + slot * PFA_W, *xp = lds + xb * PFA_X<XC, TB> + boff;
+                const uint8_t *wp = lds + slot * PFA_W<HB>, *xp = lds + xb * PFA_X<XC, TB> + boff;
 #pragma unroll
                 for (int s = 0; s < PF_KC / 32; ++s) {
                     i32x4 a[3];
 #pragma unroll
                     for (int i = 0; i < 3; ++i) {
-                        const uint8_t *ap = wp + aoff[i] + s * 32 * MLAP_QHEAD;
+                        const uint8_t *ap = wp + aoff[i] + s * 32 * PFA_WPITCH<HB>;
                         const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i *)(lds_byte_t *)ap);
-                        const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i *)(lds_byte_t *)(ap + 8 * MLAP_QHEAD));
+                        const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i *)(lds_byte_t *)(ap + 8 * PFA_WPITCH<HB>));
                         a[i] = i32x4{lo[0], lo[1], hi[0], hi[1]};
                     }
 #pragma unroll
@@ -155,10 +159,11 @@ __device__ __forceinline__ void mlap_prefill_body(const MlapParams &p, const int
                 }
             });
     }
-    // registers 4*rg .. 4*rg+3 of product i: columns 96*wc + 32*i + 8*rg + 4*half .. +3 of token l % 32 of the block
+    // registers 4*rg .. 4*rg+3 of product i: columns 96*wc + 32*i + 8*rg + 4*half .. +3 (of the head: 96*part) of token l % 32 of the block
+    const int hh = wc >> 1, part = wc & 1;
     u32x2 pk[TB][3][4];
     {
-        const float *cs = p.w_qb_scale + head * MLAP_QHEAD + 96 * wc + 4 * half;
+        const float *cs = p.w_qb_scale + (head0 + hh) * MLAP_QHEAD + 96 * part + 4 * half;
 #pragma unroll
         for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -174,22 +179,22 @@ __device__ __forceinline__ void mlap_prefill_body(const MlapParams &p, const int
             }
     }
     {
-        if (wc == 1) {
+        if (part == 1) {
 #pragma unroll
             for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
                 for (int i = 1; i < 3; ++i)
 #pragma unroll
                     for (int rg = 0; rg < 4; ++rg)
-                        *reinterpret_cast<u32x2 *>(lds + (32 * (TB * wt + tb) + (l & 31)) * PFA_RPITCH + 2 * (32 * (i - 1) + 8 * rg + 4 * half)) = pk[tb][i][rg];
+                        *reinterpret_cast<u32x2 *>(lds + (PFA_TOK<TB> * hh + 32 * (TB * wt + tb) + (l & 31)) * PFA_RPITCH + 2 * (32 * (i - 1) + 8 * rg + 4 * half)) = pk[tb][i][rg];
         }
         __syncthreads();
-        // lane (token, e) rotates pairs 4e .. 4e+3 (channels 2j, 2j+1 are the partners j, 32 + j), eight tokens at a time
+        // lane (row, e) rotates pairs 4e .. 4e+3 (channels 2j, 2j+1 are the partners j, 32 + j), eight tokens at a time
         const int e = l & 7;
 #pragma unroll
         for (int k = 0; k < 2 * TB; ++k) {
-            const int tr = 8 * (2 * TB * w + k) + (l >> 3);
-            pfa_rotate_rows(p, lds, tr, t0 + tr, head, e);
+            const int row = 8 * (2 * TB * w + k) + (l >> 3);                                         // (a wave's rows are all of one head)
+            pfa_rotate_rows(p, lds, row, t0 + row - PFA_TOK<TB> * (w >> 2), head0 + (w >> 2), e);
         }
         __syncthreads();
     }
@@ -198,17 +203,17 @@ __device__ __forceinline__ void mlap_prefill_body(const MlapParams &p, const int
         const int tl = 32 * (TB * wt + tb) + (l & 31);
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-            if (wc == 1 && i > 0) break;
-            const int blk = 3 * wc + i;                // 32 nope channels
+            if (part == 1 && i > 0) break;
+            const int blk = 3 * part + i;                // 32 nope channels
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
                 const u32x4 o = {pk[tb][i][2 * k][0], pk[tb][i][2 * k][1], pk[tb][i][2 * k + 1][0], pk[tb][i][2 * k + 1][1]};
-                *reinterpret_cast<u32x4 *>(lds + tl * 256 + 16 * ((2 * (2 * blk + k) + half) ^ (l & 15))) = o;
+                *reinterpret_cast<u32x4 *>(lds + (PFA_TOK<TB> * hh + tl) * 256 + 16 * ((2 * (2 * blk + k) + half) ^ (l & 15))) = o;
             }
         }
     }
-    // w_uk[head], columns 128*w + 4n .. +3, every row: rows 16*ks + 4*half + {0..3, 8..11} are this half's part of step ks
-    const int col = 128 * w + 4 * (l & 31);
+    // w_uk of head w / 4, columns 128*(w % 4) + 4n .. +3, every row: rows 16*ks + 4*half + {0..3, 8..11} are this half's part of step ks
+    const int head = head0 + (w >> 2), col = 128 * (w & 3) + 4 * (l & 31);
     bf16x8 wf[MLAP_NOPE / 16][4];
     {
         const uint16_t *src = p.w_uk + (size_t)head * MLAP_NOPE * MLAP_KV + (size_t)(4 * half) * MLAP_KV + col;
@@ -229,6 +234,7 @@ __device__ __forceinline__ void mlap_prefill_body(const MlapParams &p, const int
     }
     __syncthreads();                                   // the operand of the second product is complete
     uint16_t *dst = p.q_nope + (size_t)head * MLAP_KV + col;
+    const uint8_t *operand = lds + (w >> 2) * (PFA_TOK<TB> * 256);
 #pragma unroll 1
     for (int blk = 0; blk < 2 * TB; ++blk) {
         const int tb0 = t0 + 32 * blk;
@@ -240,7 +246,7 @@ __device__ __forceinline__ void mlap_prefill_body(const MlapParams &p, const int
             for (int r = 0; r < 16; ++r) c[j][r] = 0.f;
 #pragma unroll
         for (int ks = 0; ks < MLAP_NOPE / 16; ++ks) {
-            const bf16x8 a = *reinterpret_cast<const bf16x8 *>(lds + (32 * blk + (l & 31)) * 256 + 16 * ((2 * ks + half) ^ (l & 15)));
+            const bf16x8 a = *reinterpret_cast<const bf16x8 *>(operand + (32 * blk + (l & 31)) * 256 + 16 * ((2 * ks + half) ^ (l & 15)));
 #pragma unroll
             for (int j = 0; j < 4; ++j) c[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, wf[ks][j], c[j], 0, 0, 0);
         }
@@ -266,21 +272,24 @@ template <int TB> constexpr int PFI_TOK = 128 * TB;
 template <int XC, int TB> constexpr int PFI_X = PFI_TOK<TB> * PF_XPITCH<XC>;
 constexpr int PFI_W = PF_KC * LIP_DIM;
 constexpr int PFI_HAD = LIP_DIM * LIP_DIM * 2;
-template <int XC, int TB> constexpr int PFI_LOOP_LDS = 2 * PFI_X<XC, TB> + 3 * PFI_W;
+template <int XC, int TB, int HB> constexpr int PFI_LOOP_LDS = 2 * PFI_X<XC, TB> + 3 * HB * PFI_W;
 constexpr int PFI_FIXED_TOK = 64;
 constexpr int PFI_FIXED_LDS = PFI_HAD + PFI_FIXED_TOK * HB_PITCH * 2 + HB_SCRATCH;
-constexpr int PFI_FIN_LDS = PFI_FIXED_LDS > PFI_HAD + 4 * 32 * QFP_OPITCH ? PFI_FIXED_LDS : PFI_HAD + 4 * 32 * QFP_OPITCH;
-template <int XC, int TB> constexpr int PFI_LDS = PFI_LOOP_LDS<XC, TB> > PFI_FIN_LDS ? PFI_LOOP_LDS<XC, TB> : PFI_FIN_LDS;
+template <int HB> constexpr int PFI_OUT_LDS = PFI_HAD + 4 * HB * 32 * QFP_OPITCH;
+template <int HB> constexpr int PFI_FIN_LDS = PFI_FIXED_LDS > PFI_OUT_LDS<HB> ? PFI_FIXED_LDS : PFI_OUT_LDS<HB>;
+template <int XC, int TB, int HB> constexpr int PFI_LDS = PFI_LOOP_LDS<XC, TB, HB> > PFI_FIN_LDS<HB> ? PFI_LOOP_LDS<XC, TB, HB> : PFI_FIN_LDS<HB>;
 
-template <int XC, int TB, bool FIXED>
+template <int XC, int TB, int HB, bool FIXED>
 __device__ __forceinline__ void lip_prefill_body(const LipParams &p, const int job, uint8_t *lds)
 {
     const int l = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int w8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int w = w8 & 3, hh = w8 >> 2;                // wave of the head's four
     const int half = l >> 5;
     const int ncols = p.n_heads * LIP_DIM;
     const int ttiles = (p.T + PFI_TOK<TB> - 1) / PFI_TOK<TB>;
-    const int head = job / ttiles;
+    const bool exists = (job / ttiles) * HB + hh < p.n_heads;      // (of an odd number of heads the last workgroups take one twice)
+    const int head = (job / ttiles) * HB + (exists ? hh : 0);
     const int t0 = (job % ttiles) * PFI_TOK<TB>;
     const uint32_t base = (uint32_t)(uintptr_t)(lds_byte_t *)lds;
     auto token = [&](const int tl) { return t0 + tl < p.T ? t0 + tl : p.T - 1; };
@@ -293,8 +302,8 @@ __device__ __forceinline__ void lip_prefill_body(const LipParams &p, const int j
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[tb][i][r] = 0;
     {
-        constexpr int XR = 2 * XC * TB;
-        const PfTokens<XC, XR> xt(p.q_norm, p.q_lora, p.T, t0, XR * w, l);
+        constexpr int XR = 2 * XC * TB / HB;
+        const PfTokens<XC, XR> xt(p.q_norm, p.q_lora, p.T, t0, XR * w8, l);
         const int8_t *wsrc[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j)
@@ -302,13 +311,13 @@ __device__ __forceinline__ void lip_prefill_body(const LipParams &p, const int j
         const size_t wstep = (size_t)PF_KC * ncols;
         const uint32_t boff = (32 * TB * w + (l & 31)) * PF_XPITCH<XC>;
         staged_chunks<XC, XR, 2>(
-            p.q_lora / PF_KC, [&](const int s, const int b) { xt.request(s, base + b * PFI_X<XC, TB> + 1024 * XR * w); },
+            p.q_lora / PF_KC, [&](const int s, const int b) { xt.request(s, base + b * PFI_X<XC, TB> + 1024 * XR * w8); },
             [&](const int c, const int slot) {
 #pragma unroll
-                for (int j = 0; j < 2; ++j) dma16(wsrc[j] + c * wstep, base + 2 * PFI_X<XC, TB> + slot * PFI_W + 1024 * (2 * w + j));
+                for (int j = 0; j < 2; ++j) dma16(wsrc[j] + c * wstep, base + 2 * PFI_X<XC, TB> + (slot * HB + hh) * PFI_W + 1024 * (2 * w + j));
             },
             [&](const int odd, const int xb, const int slot) {
-                const uint8_t *wp = lds + 2 * PFI_X<XC, TB> + slot * PFI_W, *xp = lds + xb * PFI_X<XC, TB> + boff;
+                const uint8_t *wp = lds + 2 * PFI_X<XC, TB> + (slot * HB + hh) * PFI_W, *xp = lds + xb * PFI_X<XC, TB> + boff;
 #pragma unroll
                 for (int s = 0; s < PF_KC / 32; ++s) {
                     i32x4 a[4];
@@ -323,9 +332,9 @@ __device__ __forceinline__ void lip_prefill_body(const LipParams &p, const int j
             });
     }
     {
-        const uint16_t *src = p.hq + (size_t)(4 * (8 * w) + (l >> 4)) * LIP_DIM + 8 * ((l & 15) ^ (4 * ((l >> 4) & 3)));
+        const uint16_t *src = p.hq + (size_t)(4 * (8 / HB * w8) + (l >> 4)) * LIP_DIM + 8 * ((l & 15) ^ (4 * ((l >> 4) & 3)));
 #pragma unroll 1
-        for (int j = 0; j < 8; ++j) dma16(src + (size_t)4 * j * LIP_DIM, base + 1024 * (8 * w + j));
+        for (int j = 0; j < 8 / HB; ++j) dma16(src + (size_t)4 * j * LIP_DIM, base + 1024 * (8 / HB * w8 + j));
     }
     const float *cs = p.w_qb_scale + head * LIP_DIM + 4 * half;
     bf16x8 bq[TB][LIP_DIM / 16];
@@ -364,7 +373,7 @@ __device__ __forceinline__ void lip_prefill_body(const LipParams &p, const int j
         }
     }
     if constexpr (FIXED) {
-        static_assert(TB == 1 && PFI_FIXED_TOK >= LIP_MFMA_MIN_TOKENS, "one tile of two blocks");
+        static_assert(TB == 1 && HB == 1 && PFI_FIXED_TOK >= LIP_MFMA_MIN_TOKENS, "one tile of two blocks");
         uint16_t *rows = reinterpret_cast<uint16_t *>(lds + PFI_HAD);
         if (32 * w < PFI_FIXED_TOK) {
             // dword d of bq[0][ks]: channels 16*ks + 8*(d / 2) + 4*half + 2*(d % 2), +1 of row 32*w + l % 32
@@ -388,7 +397,7 @@ __device__ __forceinline__ void lip_prefill_body(const LipParams &p, const int j
     }
     VM_WAIT(0);
     __syncthreads();                                   // the matrix is staged
-    uint8_t *mine = lds + PFI_HAD + w * (32 * QFP_OPITCH);
+    uint8_t *mine = lds + PFI_HAD + w8 * (32 * QFP_OPITCH);
     const int arow = 4 * half + ((l & 15) >> 2);
 #pragma unroll
     for (int tb = 0; tb < TB; ++tb) {
@@ -409,12 +418,12 @@ __device__ __forceinline__ void lip_prefill_body(const LipParams &p, const int j
             }
         const int tb0 = t0 + 32 * (TB * w + tb);
         const float deq = lip_quant_rows(c, mine, l);
-        if (l < 32 && tb0 + l < p.T) p.q_scale[(size_t)(tb0 + l) * p.n_heads + head] = (uint16_t)(pack_f16x2(deq, 0.f) & 0xffffu);
+        if (exists && l < 32 && tb0 + l < p.T) p.q_scale[(size_t)(tb0 + l) * p.n_heads + head] = (uint16_t)(pack_f16x2(deq, 0.f) & 0xffffu);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const int r = 8 * k + (l >> 3);
             const u32x4 v = *reinterpret_cast<const u32x4 *>(mine + r * QFP_OPITCH + 16 * (l & 7));
-            if (tb0 + r < p.T) *reinterpret_cast<u32x4 *>(p.q_int8 + ((size_t)(tb0 + r) * p.n_heads + head) * LIP_DIM + 16 * (l & 7)) = v;
+            if (exists && tb0 + r < p.T) *reinterpret_cast<u32x4 *>(p.q_int8 + ((size_t)(tb0 + r) * p.n_heads + head) * LIP_DIM + 16 * (l & 7)) = v;
         }
     }
 }

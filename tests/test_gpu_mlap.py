@@ -625,3 +625,28 @@ def test_fused_entry_point_through_the_c_abi_keeps_the_intermediates_in_its_work
 def test_fused_prolog_fixed_order_sums_of_several_tiles_per_workgroup(t, n_idx):
     """The same where a workgroup takes two token tiles: an odd number of them, a ragged last one."""
     test_fused_prolog_fixed_order_sums_at_tile_edges(t, n_idx)
+
+
+@pytest.mark.parametrize("t,n_heads,n_idx", [(769, 2, 8), (1024, 4, 5), (1537, 2, 3), (1793, 6, 16)])
+def test_fused_prolog_query_rows_with_two_heads_to_a_workgroup(t, n_heads, n_idx):
+    """From four tiles of 256 tokens on a workgroup makes two heads' queries: odd numbers of indexer heads (the last one's
+    second is then not there), a last tile of one token and a full one, the indexer's tiles of 128 and 256 tokens."""
+    from oracle import lip_oracle as lo
+    from pypto_amd import lightning_indexer_prolog_quant_impl as lip_impl
+    from pypto_amd import mla_prolog_quant_impl as impl
+    from pypto_amd.synthetic import gen_indexer_prolog_inputs
+    impl.EXACT_ABSORB = lip_impl.EXACT_SUMS = False
+    kw = dict(h=128, q_lora_rank=512)
+    mla = gen_mla_prolog_inputs(1, t, [t + 30], seed=t, n_heads=n_heads, **kw)
+    lip = gen_indexer_prolog_inputs(1, t, [t + 30], seed=t + 1, n_heads=n_idx, **kw)
+    ref = mo.mla_prolog_ref(*mla.input_tensors(), epsilon_cq=1e-5, epsilon_ckv=1e-5)
+    got = run_op(mla, (1e-5, 1e-5), prefill=True)
+    assert_reference_rule(got, ref, mla.cache_index.numpy(), f"t={t}")
+    dm, dl = mla.to(torch.device("cuda:0")), lip.to(torch.device("cuda:0"))
+    q_nope, q_rope, q_int8, q_scale, _ = run_fused(dm, dl, t, n_heads, n_idx, op=pypto_amd.mla_indexer_prolog_quant_p)
+    assert np.array_equal(q_nope.float().cpu().numpy(), got["query_nope"]) and np.array_equal(q_rope.float().cpu().numpy(), got["query_rope"])
+    lip.x, lip.cos_idx_rope, lip.sin_idx_rope, lip.k_cache_index = mla.token_x, mla.cos, mla.sin, mla.cache_index
+    lip.q_norm, lip.q_norm_scale = torch.from_numpy(got["q_norm"]), torch.from_numpy(got["q_norm_scale"]).reshape(-1, 1)
+    want = lo.indexer_prolog_ref(*lip.input_tensors())
+    assert np.abs(q_int8.cpu().numpy().astype(np.int32) - want["q_int8"].astype(np.int32)).max() <= 1
+    assert (np.abs(q_scale.float().cpu().numpy()[..., 0] - want["q_scale"].astype(np.float32)) > 2.5e-5).mean() <= 0.005
