@@ -411,7 +411,7 @@ int li_check(const PtoLiDecodeArgs *a)
         return fail(PTO_E_INVALID_ARG, "li: max_blocknum_perbatch * block_size exceeds %d", pto::LI_MAX_SEQ);
     if (a->t > (1ll << 20) || a->block_num > 0x7fffffffll || a->block_size > LI_MAX_SEQ_HOST || a->block_num * a->block_size > 0x7fffffffll)
         return fail(PTO_E_INVALID_ARG, "li: shape out of the supported range");
-    if (a->t > pto::LI_MAX_BALANCED_TOKENS && a->t > 65535)
+    if (a->t > 65535)
         return fail(PTO_E_INVALID_ARG, "li: at most 65535 query tokens per launch (got %lld)", (long long)a->t);
     if (a->arith_variant != 0 && a->arith_variant != 1) return fail(PTO_E_INVALID_ARG, "li: arith_variant must be 0 or 1");
     if (a->arith_variant == 1 &&
@@ -652,16 +652,18 @@ int pto_li_decode_launch(const PtoLiDecodeArgs *a, void *hip_stream)
     p.variant = a->arith_variant;
     {   // A wave pays three dependent memory latencies before its first pair, so runs are made as long
         // as still leaves every SIMD two rounds of two waves; at most 32 pairs (2048 keys) per wave.
-        // Two query tokens of a sequence share a key pass (half the key bytes, the same arithmetic) when
-        // there are two and the pass then still has several rounds of work for every resident wave; a
-        // small batch is bound by latency, not bytes, and keeps one token per wave for twice the waves.
+        // Two query tokens of a sequence share a wave's pass over a run of keys where they are an even number and the pass has
+        // several rounds of work for every resident wave.  Below, and with a token left over, units of one token are the
+        // faster ones: they read the same keys side by side anyway, and twice as many waves share the work more evenly (one / two
+        // tokens to a unit: 20 x 2 tokens of 5 to 60 K keys 36.0 / 40.0 us, 40 x 4 of 2 to 16 K 39.0 / 39.3, 18 x 2 of 20 to 130 K
+        // 65.5 / 65.0, 64 x 2 of 4 to 32 K 52.5 / 50.2, 18 x 4 of 20 to 130 K 104 / 99.6, but 18 x 3 84.0 / 100).
         int nt = 1;
-        if (p.S1 >= 2 && p.variant == 0) {
-            const long long pairs2 = (long long)p.B * ((p.S1 + 1) / 2) * ((p.score_stride + 63) / 64);
-            if (pairs2 >= 8ll * cu_count() * 8) nt = 2;
+        if (p.S1 % 2 == 0 && p.variant == 0) {
+            const long long pairs2 = (long long)p.B * (p.S1 / 2) * ((p.score_stride + 63) / 64);
+            if (pairs2 >= 12ll * cu_count() * 8) nt = 2;
         }
         p.nt = nt;
-        const long long units = (long long)p.B * ((p.S1 + nt - 1) / nt);    // token groups that share a key pass
+        const long long units = (long long)p.B * (p.S1 / nt);    // token groups that share a key pass
         const long long pairs = units * ((p.score_stride + 63) / 64);
         long long ppw = pairs / ((long long)cu_count() * 4 * 4);
         p.ppw = (int)(ppw < 1 ? 1 : (ppw > pto::LI_MAX_PAIRS_PER_WAVE ? pto::LI_MAX_PAIRS_PER_WAVE : ppw));
@@ -669,11 +671,12 @@ int pto_li_decode_launch(const PtoLiDecodeArgs *a, void *hip_stream)
         // per CU), more where the longest possible input would need them.  The kernel sizes the runs for as few whole rounds as
         // the actual lengths need (spread over all the launch's waves they left a few workgroups for a second round: 20 sequences
         // of 20 to 120 K keys, four tokens, 118 us, now 94).
-        p.balanced = units <= pto::LI_MAX_BALANCED_TOKENS;
+        p.balanced = p.B <= pto::LI_MAX_BALANCED_SEQS && units <= pto::LI_MAX_BALANCED_UNITS;
         p.round_waves = cu_count() * pto::LI_SCORE_WAVES;
         const long long need = (pairs + pto::LI_MAX_PAIRS_PER_WAVE - 1) / pto::LI_MAX_PAIRS_PER_WAVE + 2 * units;
         const long long rounds = (need + p.round_waves - 1) / p.round_waves;
-        p.score_wgs = (int)(rounds * cu_count());
+        p.unit_wgs = (int)((p.score_stride + pto::LI_SCORE_WAVES * p.ppw * 64 - 1) / (pto::LI_SCORE_WAVES * p.ppw * 64));
+        p.score_wgs = (int)(p.balanced ? rounds * cu_count() : units * p.unit_wgs);
     }
     hipError_t e = pto::li_launch(p, static_cast<hipStream_t>(hip_stream));
     if (e != hipSuccess) return fail(PTO_E_LAUNCH, "li: launch failed: %s", hipGetErrorString(e));

@@ -247,12 +247,12 @@ constexpr int SC_BUF_BYTES = SC_PAIR_BYTES + 256;   // + the 64 key scales (one 
 // the head's weight; the fp32 head sum (h ascending) is the score.  All three tensors are fp16 then.
 // NT = query tokens of one sequence a wave scores per key pass (1 or 2): the reference scores all s1 tokens of
 // a batch against a page in one matrix product (lightning_indexer_quant_impl.py:163-169, [S1*64, 128]); here
-// a "unit" is a pair of consecutive tokens of a sequence (the last unit of an odd s1 holds one), every staged
+// a "unit" is a pair of consecutive tokens of a sequence (s1 is even), every staged
 // key row and scale serves both, and their per-head factors sit in LDS instead of scalar registers.
 // A workgroup of eight waves per compute unit, and nothing in front of the first requests that need not be there: as two workgroups of
 // four the second one's sequence lengths came back behind the first one's key rows (7 us, and it ended as much later), the
 // mapping took 2.3 us of divisions, and the queries, asked for behind two pairs of every wave, arrived behind 34 MB.  Kernel over
-// rotating key caches, before / now: 4 tokens x 32 K keys 10.5 / 6.8 us, 32 x 8-64 K 36.9 / 35.6, 64 pairs of tokens x 4-32 K 44.8 / 40.5.
+// rotating key caches, before / now: 4 tokens x 32 K keys 10.5 / 6.8 us, 32 x 8-64 K 36.9 / 31.1, 64 pairs of tokens x 4-32 K 44.8 / 40.5.
 // (Pairs of a workgroup's runs drawn by whichever wave comes first, so that its waves end together instead of up to 8 us apart: +-0.
 // Bound now: the first one by its bytes, 28.4 us with nothing but the requests and stores; the other by vector work and the
 // products beside it, two waves to a SIMD.)
@@ -264,8 +264,7 @@ __global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_pe
     __shared__ __attribute__((aligned(16))) int8_t kstage[LI_SCORE_WAVES][2][SC_BUF_BYTES];
     __shared__ __attribute__((aligned(16))) float wsc_lds[NT > 1 && !HW ? LI_SCORE_WAVES : 1][NT][LI_HEADS];
     static_assert(SC_PAIR_BYTES == LI_HEADS * LI_DIM, "a token's query is staged where a pair of key blocks goes later");
-    const int upb = (p.S1 + NT - 1) / NT;            // units per sequence
-    const int nunits = p.B * upb;
+    const int upb = p.S1 / NT;                       // units per sequence (two tokens to a unit: S1 is even)
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l = threadIdx.x & 63;
     const int j = l & 31;
@@ -274,28 +273,27 @@ __global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_pe
     auto clamped = [&](const int n) { return n < 0 ? 0 : (n > cap ? cap : n); };
     int unit, b, cur, key0, ppw;
     if (p.balanced) {
-        // Balanced mapping (at most 512 query tokens): the launch has a fixed number of waves; every wave
-        // reads all sequence lengths, sizes the runs so that the runs of all tokens just fill the
-        // launch, and takes the gw-th run in token order.  Short and long sequences then cost the same
-        // number of trips per wave and the whole pass is one round of resident waves.  (Nothing is on its way from memory
-        // meanwhile, so it is kept short: divisions by reciprocals, and for up to 64 units a single row of the unit table.)
+        // Balanced mapping: the launch has a fixed number of waves; every wave reads all sequence lengths, sizes the runs so that
+        // the runs of all units just fill the launch, and takes the gw-th run.  Short and long sequences then cost the same number
+        // of trips per wave and the whole pass is one round of resident waves.  The units of a sequence take the same run side by
+        // side, mostly in one workgroup, so that its keys come from memory once: unit after unit, 4 x 2 tokens of 8 to 64 K keys took
+        // 23.8 us instead of 21.7, 20 x 3 49.3 instead of 42.9, two tokens to a unit either way.  (Nothing is on its way
+        // from memory meanwhile, so it is kept short: divisions by reciprocals, and for up to 64 sequences a single row of the table.)
         const int gw = blockIdx.x * LI_SCORE_WAVES + w;
-        int found = -1, found_run = 0, found_seq = 0, found_len = 0;
+        int found = -1, found_run = 0, found_len = 0;
         auto balance = [&](auto rows_tag) __attribute__((always_inline)) {
-            constexpr int ROWS = decltype(rows_tag)::value;          // of 64 units
-            const float inv_upb = __builtin_amdgcn_rcpf((float)upb);
-            int seq[ROWS], len[ROWS], pairs[ROWS], total = 0;
+            constexpr int ROWS = decltype(rows_tag)::value;          // of 64 sequences each
+            int len[ROWS], pairs[ROWS], total = 0;
 #pragma unroll
             for (int i = 0; i < ROWS; ++i) {
-                const int tt = l + 64 * i;
-                seq[i] = tt < nunits ? small_quotient(tt, inv_upb) : p.B - 1;
-                len[i] = p.act[seq[i]];
+                const int seq = l + 64 * i;
+                len[i] = p.act[seq < p.B ? seq : p.B - 1];
             }
 #pragma unroll
             for (int i = 0; i < ROWS; ++i) {
-                len[i] = l + 64 * i < nunits ? clamped(len[i]) : 0;
+                len[i] = l + 64 * i < p.B ? clamped(len[i]) : 0;
                 pairs[i] = (len[i] + 63) >> 6;
-                total += pairs[i];
+                total += pairs[i] * upb;
             }
             total = __builtin_amdgcn_readlane((int)wave_incl_scan((uint32_t)total), 63);
             // as few whole rounds as runs of the greatest length need (the launch has as many as the longest sequences would)
@@ -306,16 +304,15 @@ __global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_pe
             ppw = ppw < 1 ? 1 : (ppw > LI_MAX_PAIRS_PER_WAVE ? LI_MAX_PAIRS_PER_WAVE : ppw);
             for (;;) {
                 const float inv_ppw = __builtin_amdgcn_rcpf((float)ppw);
-                int base = 0;                 // runs of all units before row i of the unit table
+                int base = 0;                 // runs of all sequences before row i of the table
 #pragma unroll
                 for (int i = 0; i < ROWS; ++i) {
-                    const int runs = small_quotient(pairs[i] + ppw - 1, inv_ppw);
+                    const int runs = small_quotient(pairs[i] + ppw - 1, inv_ppw) * upb;
                     const int incl = (int)wave_incl_scan((uint32_t)runs);
                     const int run = gw - (base + incl - runs);
                     if (run >= 0 && run < runs) {
                         found = l + 64 * i;
                         found_run = run;
-                        found_seq = seq[i];
                         found_len = len[i];
                     }
                     base += __builtin_amdgcn_readlane(incl, 63);
@@ -325,25 +322,25 @@ __global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_pe
                 found = -1;
             }
         };
-        if (nunits <= 64) balance(std::integral_constant<int, 1>{});
-        else balance(std::integral_constant<int, LI_MAX_BALANCED_TOKENS / 64>{});
+        if (p.B <= 64) balance(std::integral_constant<int, 1>{});
+        else balance(std::integral_constant<int, LI_MAX_BALANCED_SEQS / 64>{});
         const unsigned long long hit = __ballot(found >= 0);
         if (hit == 0ull) return;          // more waves than runs
         const int src = __ffsll((long long)hit) - 1;
-        unit = __builtin_amdgcn_readlane(found, src);
-        b = __builtin_amdgcn_readlane(found_seq, src);
+        b = __builtin_amdgcn_readlane(found, src);
         cur = __builtin_amdgcn_readlane(found_len, src);
-        key0 = __builtin_amdgcn_readlane(found_run, src) * (ppw * 64);
+        const int of_seq = __builtin_amdgcn_readlane(found_run, src);
+        const int run = upb == 1 ? of_seq : __builtin_amdgcn_readfirstlane(small_quotient(of_seq, __builtin_amdgcn_rcpf((float)upb)));
+        unit = b * upb + of_seq - run * upb;
+        key0 = run * (ppw * 64);
     } else {
-        unit = blockIdx.y;
+        unit = (int)blockIdx.x / p.unit_wgs;
         ppw = p.ppw;
-        key0 = (blockIdx.x * LI_SCORE_WAVES + w) * (ppw * 64);
+        key0 = (((int)blockIdx.x - unit * p.unit_wgs) * LI_SCORE_WAVES + w) * (ppw * 64);
         b = unit / upb;
         cur = clamped(p.act[b]);
     }
-    const int s_first = (unit - b * upb) * NT;
-    const int nt = p.S1 - s_first < NT ? p.S1 - s_first : NT;     // tokens of this unit (uniform)
-    const int t = b * p.S1 + s_first;                             // its first token
+    const int t = b * p.S1 + (unit - b * upb) * NT;               // the unit's first token
     if (key0 >= cur) return;
     int npair = (cur - key0 + 63) >> 6;
     npair = npair > ppw ? ppw : npair;
@@ -356,7 +353,7 @@ __global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_pe
     uint32_t raw_q[NT], raw_w[NT];
 #pragma unroll
     for (int s = 0; s < NT; ++s) {
-        const size_t ts = (size_t)(t + (s < nt ? s : 0));         // a unit of one token takes that token twice
+        const size_t ts = (size_t)(t + s);
         if (VAR || HW) {
             raw_q[s] = reinterpret_cast<const u32_a2 *>(static_cast<const uint16_t *>(p.q_scale) + ts * LI_HEADS)[j];
             raw_w[s] = reinterpret_cast<const u32_a2 *>(static_cast<const uint16_t *>(p.weight) + ts * LI_HEADS)[j];
@@ -412,8 +409,8 @@ __global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_pe
     };
 #undef REQUEST_32_ROWS
     // Keys that one unit alone reads are asked for without being kept (32 sequences of 8 to 64 K keys 35.2 us, so 31.4); with
-    // more units to a sequence the next one finds them in the caches (20 sequences of 20 to 60 K, four query tokens, 47.0; not
-    // kept 50.8; 4 of 60 to 120 K 32.0 and 36.9).
+    // more units to a sequence the others find them in the caches (operator, 20 x 2 tokens of 5 to 60 K keys 35.9 us, not kept 39.7;
+    // 18 x 3 of 20 to 130 K 84.1 and 95.9).
     const bool read_once = upb == 1;
     auto request_pair = [&](const int pr, const int buf) {
         const int rx = __builtin_amdgcn_readlane(run_row, 2 * pr), ry = __builtin_amdgcn_readlane(run_row, 2 * pr + 1);
@@ -435,7 +432,7 @@ __global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_pe
     // they arrive when both pairs of every wave have, and no third pair is asked for meanwhile.
     i32x4 qa[NT][2][4];
     auto request_query = [&](const int s, const int buf) {
-        const int8_t *q0 = p.q + (size_t)(t + (s < nt ? s : 0)) * (LI_HEADS * LI_DIM);      // a unit of one token loads that token twice
+        const int8_t *q0 = p.q + (size_t)(t + s) * (LI_HEADS * LI_DIM);
         request_rows(q0, q0 + 32 * LI_DIM, lds_base + (uint32_t)(buf * SC_BUF_BYTES), false);
     };
     auto read_query = [&](auto s_tag, const int buf) {
@@ -526,8 +523,7 @@ __global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_pe
     auto trip = [&](const int pr, const int buf) {
         const int8_t *src = &kstage[w][buf][0];
         i32x4 kx[4], ky[4];
-        if (NT > 1 && nt > 1) wait_pair(std::integral_constant<int, 4>{}, pr);
-        else wait_pair(std::integral_constant<int, 2>{}, pr);
+        wait_pair(std::integral_constant<int, 2 * NT>{}, pr);
         asm volatile("" ::: "memory");
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
@@ -647,7 +643,7 @@ __global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_pe
             if (sample_lane(pos, cur)) smp[pos >> 4] = sc;
         };
         score_token(std::integral_constant<int, 0>{}, srow0, smp0);
-        if (NT > 1 && nt > 1)
+        if (NT > 1)
             score_token(std::integral_constant<int, NT - 1>{}, srow0 + p.score_stride, smp0 + p.score_stride / LI_SAMPLE_GROUP);
     };
     for (int pr = 0; pr < npair; pr += 2) {
@@ -1232,14 +1228,7 @@ hipError_t li_launch(const LiParams &p, hipStream_t stream)
 {
     const dim3 block(64 * LI_SCORE_WAVES);
     const int nt = p.nt;
-    const int nunits = p.B * ((p.S1 + nt - 1) / nt);
-    dim3 grid;
-    if (p.balanced) {
-        grid = dim3((unsigned)p.score_wgs);
-    } else {
-        const unsigned gx = (unsigned)((p.score_stride + LI_SCORE_WAVES * p.ppw * 64 - 1) / (LI_SCORE_WAVES * p.ppw * 64));
-        grid = dim3(gx, (unsigned)nunits);
-    }
+    const dim3 grid((unsigned)p.score_wgs);
     const bool hw = p.q_dt == PTO_DT_FP16 && p.w_dt == PTO_DT_FP16;
 #define LI_SCORE(KDT)                                                                                                      \
     do {                                                                                                                   \
