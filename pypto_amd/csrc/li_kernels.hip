@@ -862,22 +862,7 @@ __device__ void bitonic_sort_desc(unsigned long long *buf, const int width, cons
 constexpr int SEL_SAMPLE = 4096;   // most keys sampled from a row
 constexpr int SEL_CAP = 8192;      // candidates (keys above the pivot) the fast path holds in LDS
 constexpr int SEL_STAGE = 4096;    // entries of the buckets down to the one holding the k-th best
-constexpr int SEL_RANK_MAX = 512;  // rows of at most k keys: ordered by counting up to this length, else sorted
-
-// how many entries of list[beg, end) are larger than e; eight LDS reads in flight per round
-__device__ __forceinline__ uint32_t count_greater(const unsigned long long *list, const uint32_t beg, const uint32_t end,
-                                                  const unsigned long long e)
-{
-    uint32_t rank = 0;
-    for (uint32_t j0 = beg; j0 < end; j0 += 8) {
-        unsigned long long x[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) x[u] = list[j0 + u < end ? j0 + u : end - 1];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) rank += (j0 + u < end && x[u] > e) ? 1u : 0u;
-    }
-    return rank;
-}
+constexpr int SEL_COUNT_MAX = 128; // rows of at most k keys: most keys of a bucket that are ordered by counting
 
 // the 64-bit word whose descending order is (score descending, position ascending); never zero
 __device__ __forceinline__ unsigned long long order_word(const float score, const uint32_t pos)
@@ -945,191 +930,211 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
     const float *srow = p.scores + (size_t)t * p.score_stride;
     int32_t *out = p.topk_res + (size_t)t * k;
 
-    if (n <= k) {
-        // everything is selected; the tail of the output row is padding
-        for (int i = n + tid; i < k; i += SEL_THREADS) out[i] = -1;
-        if (n > SEL_RANK_MAX) {
-            int width = 64;
-            while (width < n) width <<= 1;
-            for (int i = tid; i < width; i += SEL_THREADS) stage[i] = i < n ? order_word(srow[i], (uint32_t)i) : 0ull;
-            __syncthreads();
-            bitonic_sort_desc(stage, width, tid);
-            for (int i = tid; i < n; i += SEL_THREADS) out[i] = (int32_t)(~(uint32_t)stage[i]);
-        } else {
-            for (int i = tid; i < n; i += SEL_THREADS) stage[i] = order_word(srow[i], (uint32_t)i);
-            __syncthreads();
-            for (int i = tid; i < n; i += SEL_THREADS) {
-                const unsigned long long e = stage[i];
-                out[count_greater(stage, 0u, (uint32_t)n, e)] = (int32_t)(~(uint32_t)e);
-            }
-        }
-        return;
-    }
-
-    // ---- 1. sample: the loads go out first, then the first chunk of the row, so that one memory
-    // latency covers both
-    // (the score kernel left one score of every 16 positions in a compact array; a row longer than
-    // 16 * SEL_SAMPLE takes every other one).  Rows with hardly any full group go the general way.
-    const uint32_t s_full = (uint32_t)n / (uint32_t)LI_SAMPLE_GROUP;
-    if (s_full < 64u) {
-        select_streaming(p, t, hist, stage);                     // uniform: the whole workgroup goes
-        return;
-    }
-    const uint32_t sstep = s_full > (uint32_t)SEL_SAMPLE ? 2u : 1u;
-    const uint32_t S = s_full / sstep;
-    constexpr int SPT = SEL_SAMPLE / SEL_THREADS;
-    const float *smp = p.sample + (size_t)t * (p.score_stride / LI_SAMPLE_GROUP);
-    float sx[SPT];
-    bool sval[SPT];
-#pragma unroll
-    for (int e = 0; e < SPT; ++e) {
-        const uint32_t i = (uint32_t)(tid + e * SEL_THREADS);
-        sval[e] = i < S;
-        sx[e] = smp[(sval[e] ? i : 0u) * sstep];
-    }
-    // the row as 16-byte vectors: thread tid holds vectors u*1024 + tid of a chunk.  The row buffer is
-    // score_stride (a multiple of 32) long, so whole vectors stay inside it.
-    const int last_vec = (int)(p.score_stride >> 2) - 1;
-    auto load_chunk = [&](const int c0, f32x4 (&v)[8]) {
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int vi = (c0 >> 2) + u * SEL_THREADS + tid;
-            v[u] = reinterpret_cast<const f32x4 *>(srow)[vi < last_vec ? vi : last_vec];
-        }
-    };
-    f32x4 v[8], vn[8];
-    load_chunk(0, v);
-    const uint32_t r0 = ((uint32_t)k * S + (uint32_t)n - 1u) / (uint32_t)n;
-    const uint32_t r = r0 + (uint32_t)(6.0f * __builtin_sqrtf((float)r0)) + 8u;
-
-    for (int i = tid; i < SEL_SBINS; i += SEL_THREADS) shist[i] = 0u;
-    for (int i = tid; i < SEL_BUCKETS / 4; i += SEL_THREADS) reinterpret_cast<u32x4 *>(boff)[i] = u32x4{0u, 0u, 0u, 0u};
-    if (tid == 0) sh_over = 0u;
-    {
-        float mn = __builtin_inff(), mx = -__builtin_inff();
-#pragma unroll
-        for (int e = 0; e < SPT; ++e)
-            if (sval[e]) { mn = fminf(mn, sx[e]); mx = fmaxf(mx, sx[e]); }
-        mn = wave_min(mn);
-        mx = wave_max(mx);
-        if (lane == 0) { wave_mn[wv] = mn; wave_mx[wv] = mx; }
-    }
-    __syncthreads();
-    const float smin = row_reduce(wave_mn[lane & 15], [](float x, float y) { return fminf(x, y); });
-    const float smax = row_reduce(wave_mx[lane & 15], [](float x, float y) { return fmaxf(x, y); });
-    float pivot = -__builtin_inff();       // candidates: score >= pivot
-    float blo = smin;                      // lower edge of the lowest bucket
-    if (r < S) {
-        const float range = smax - smin;
-        const float sscale = range > 0.f ? (float)SEL_SBINS / range : 0.f;
-#pragma unroll
-        for (int e = 0; e < SPT; ++e) {
-            if (sval[e]) {
-                const uint32_t sb = (uint32_t)fmaxf((sx[e] - smin) * sscale, 0.f);
-                atomicAdd(&shist[sb < (uint32_t)SEL_SBINS ? sb : (uint32_t)SEL_SBINS - 1u], 1u);
-            }
-        }
-        __syncthreads();
-        // one wave scans the 1024 bins from the top (lane l owns the 16 bins below 1024 - 16*l): the bin in which the running
-        // count reaches r.  (Every wave by itself, without the barrier: 2.2 thousand clocks of vector work instead of 0.9.)
-        if (wv == 0) {
-            const u32x4 *src = reinterpret_cast<const u32x4 *>(&shist[SEL_SBINS - 16 - 16 * lane]);
-            uint32_t tot = 0;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const u32x4 x = src[q];
-                tot += (x[0] + x[1]) + (x[2] + x[3]);
-            }
-            const uint32_t before = wave_incl_scan(tot) - tot;
-            // (found by exactly one lane: the sample holds S >= r scores); then the bin among its sixteen, a lane each
-            const int at = __ffsll((long long)__ballot(before < r && r <= before + tot)) - 1;
-            const uint32_t top = (uint32_t)(SEL_SBINS - 1 - 16 * at);
-            const uint32_t cnt = shist[top - (uint32_t)(lane & 15)];
-            const uint32_t incl = (uint32_t)__builtin_amdgcn_readlane((int)before, at) + row_incl_scan(cnt);
-            const int in = __ffsll((long long)__ballot(incl - cnt < r && r <= incl)) - 1;
-            if (lane == 0) sh_pb = top - (uint32_t)in;
-        }
-        __syncthreads();
-        const uint32_t pb = sh_pb;
-        pivot = smin + (float)pb * (range * (1.0f / (float)SEL_SBINS));
-        blo = pivot;
-    }
-    // the buckets reach a quarter of the range past the sample maximum, so that the few scores above
-    // it spread out too; anything beyond shares bucket 0
-    const float bscale = smax - blo > 0.f ? (float)SEL_BUCKETS / (1.25f * (smax - blo)) : 0.f;
-
-    // ---- 2. candidates.  Wave w compacts the positions of the candidates among its keys into its own region of the
-    // list, cand[w*SEL_WAVE_CAP ...], so the waves share no counter.  A key costs a compare and an add-with-carry that
-    // shifts the outcome into the lane's mask of its 32 keys; the few candidates (one key in twenty of a long row) are then
-    // picked out of the masks, a candidate of every lane per trip, and their scores fetched again below (out of the L2).
-    // (One LDS write per key, candidate or not, as before, took 14 to 17 of the kernel's 33 thousand clocks on 50 K keys.)
-    // Wave-wide sums use DPP, not LDS.
-    uint32_t wave_count = 0;               // candidates of this wave so far (uniform)
-    auto scan_chunk = [&](const int c0, auto full_tag) {
-        constexpr bool FULL = decltype(full_tag)::value;          // the whole chunk lies inside the row
-        const int i_base = c0 + 4 * tid;
-        uint32_t m = 0;                                           // key (u, c) is bit 31 - (4u + c)
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const int i = i_base + 4 * u * SEL_THREADS + c;
-                m = m + m + (((FULL || i < n) && v[u][c] >= pivot) ? 1u : 0u);
-            }
-        }
-        const uint32_t mine = (uint32_t)__popc(m);
-        const uint32_t incl = wave_incl_scan(mine);
-        const uint32_t wave_n = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-        if (wave_count + wave_n > (uint32_t)SEL_WAVE_CAP) {       // region overflow: the streaming path will run
-            if (lane == 0) sh_over = 1u;
-            return;
-        }
-        uint32_t slot = (uint32_t)(wv * SEL_WAVE_CAP) + wave_count + incl - mine;
-        wave_count += wave_n;
-        while (m != 0u) {
-            const uint32_t q = (uint32_t)__clz(m);                // 4u + c
-            m &= 0x7fffffffu >> q;
-            cand[slot++] = (uint32_t)i_base + ((q >> 2) * (4u * SEL_THREADS) + (q & 3u));
-        }
-    };
-    for (int c0 = 0; c0 < n; c0 += SEL_CHUNK) {
-        if (c0 + SEL_CHUNK < n) load_chunk(c0 + SEL_CHUNK, vn);
-        if (c0 + SEL_CHUNK <= n) scan_chunk(c0, std::true_type{});
-        else scan_chunk(c0, std::false_type{});
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = vn[u];
-    }
-    if (lane == 0) wave_tot[wv] = wave_count;
-
-    // ---- 3. bucket of every candidate of the wave's own region (up to eight per lane) and its slot
-    // inside the bucket
+    // everything is selected; the tail of the output row is padding
+    for (int i = n + tid; i < k; i += SEL_THREADS) out[i] = -1;
+    if (n == 0) return;
+    const int kk = n < k ? n : k;          // keys taken
     constexpr int CPT = SEL_WAVE_CAP / 64;
-    unsigned long long ce[CPT];
-    uint32_t cb[CPT], cslot[CPT], cpos[CPT];
-    float csc[CPT];
-#pragma unroll
-    for (int u = 0; u < CPT; ++u) {
-        const uint32_t j = (uint32_t)(u * 64 + lane);
-        cpos[u] = j < wave_count ? cand[wv * SEL_WAVE_CAP + j] : 0u;
-        csc[u] = (uint32_t)(u * 64) < wave_count ? srow[cpos[u]] : 0.f;             // (uniform: trips past the last are left out)
-    }
+    unsigned long long ce[CPT];            // this lane's candidates, their buckets and places in them
+    uint32_t cb[CPT], cslot[CPT];
+    // the workgroup's minimum and maximum
+    auto range_of = [&](const float mn, const float mx, float &lo, float &hi) __attribute__((always_inline)) {
+        const float a = wave_min(mn), b2 = wave_max(mx);
+        if (lane == 0) { wave_mn[wv] = a; wave_mx[wv] = b2; }
+        __syncthreads();
+        lo = row_reduce(wave_mn[lane & 15], [](float x, float y) { return fminf(x, y); });
+        hi = row_reduce(wave_mx[lane & 15], [](float x, float y) { return fmaxf(x, y); });
+    };
+    auto to_bucket = [&](const int u, const float score, const uint32_t pos, const float lo, const float scale) __attribute__((always_inline)) {
+        ce[u] = order_word(score, pos);
+        const uint32_t lin = (uint32_t)fmaxf((key_score((uint32_t)(ce[u] >> 32)) - lo) * scale, 0.f);
+        cb[u] = (uint32_t)SEL_BUCKETS - 1u - (lin < (uint32_t)SEL_BUCKETS ? lin : (uint32_t)SEL_BUCKETS - 1u);
+        cslot[u] = atomicAdd(&boff[cb[u]], 1u);
+    };
 #pragma unroll
     for (int u = 0; u < CPT; ++u) {
         ce[u] = 0ull;
-        cb[u] = (uint32_t)SEL_BUCKETS;                                              // none
+        cb[u] = (uint32_t)SEL_BUCKETS;     // none
         cslot[u] = 0u;
-        if ((uint32_t)(u * 64 + lane) < wave_count) {
-            ce[u] = order_word(csc[u], cpos[u]);
-            const uint32_t lin = (uint32_t)fmaxf((key_score((uint32_t)(ce[u] >> 32)) - blo) * bscale, 0.f);
-            cb[u] = (uint32_t)SEL_BUCKETS - 1u - (lin < (uint32_t)SEL_BUCKETS ? lin : (uint32_t)SEL_BUCKETS - 1u);
-            cslot[u] = atomicAdd(&boff[cb[u]], 1u);
-        }
     }
-    __syncthreads();
-    const uint32_t n_cand = (uint32_t)__builtin_amdgcn_readlane((int)row_incl_scan(wave_tot[lane & 15]), 15);
-    if (sh_over != 0u || n_cand < (uint32_t)k) {
-        select_streaming(p, t, hist, stage);                     // uniform: the whole workgroup goes
-        return;
+    // A row of at most k keys, two per thread: all of them go straight to the buckets, spread over their own range.  Where too
+    // many fall together (equal scores, one far from the rest, an infinite one), or one is not a number, they are sorted.
+    // (Always sorted beyond 512 keys and ordered by counting over the whole row up to there, as before, two sequences of 450
+    // keys took 24.3 us instead of 9.8, scores included, of 650 keys 18.5, of 1900 22.0 instead of 11.0.)
+    auto sort_row = [&]() {
+        int width = 64;
+        while (width < n) width <<= 1;
+        for (int i = tid; i < width; i += SEL_THREADS) stage[i] = i < n ? order_word(srow[i], (uint32_t)i) : 0ull;
+        __syncthreads();
+        bitonic_sort_desc(stage, width, tid);
+        for (int i = tid; i < n; i += SEL_THREADS) out[i] = (int32_t)(~(uint32_t)stage[i]);
+    };
+    if (n <= k) {
+        static_assert(LI_MAX_SELECT <= 2 * SEL_THREADS && CPT >= 2, "two keys per thread");
+        float x[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) x[e] = srow[tid + e * SEL_THREADS < n ? tid + e * SEL_THREADS : tid < n ? tid : 0];
+        for (int i = tid; i < SEL_BUCKETS / 4; i += SEL_THREADS) reinterpret_cast<u32x4 *>(boff)[i] = u32x4{0u, 0u, 0u, 0u};
+        if (tid == 0) sh_over = 0u;
+        float smin, smax;
+        range_of(fminf(x[0], x[1]), fmaxf(x[0], x[1]), smin, smax);
+        const float scale = smax - smin > 0.f ? (float)SEL_BUCKETS / (smax - smin) : 0.f;
+        if (!(x[0] == x[0]) || !(x[1] == x[1])) sh_over = 1u;
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+            if (tid + e * SEL_THREADS < n) to_bucket(e, x[e], (uint32_t)(tid + e * SEL_THREADS), smin, scale);
+        __syncthreads();
+    } else {
+        // ---- 1. sample: the loads go out first, then the first chunk of the row, so that one memory
+        // latency covers both
+        // (the score kernel left one score of every 16 positions in a compact array; a row longer than
+        // 16 * SEL_SAMPLE takes every other one).  Rows with hardly any full group go the general way.
+        const uint32_t s_full = (uint32_t)n / (uint32_t)LI_SAMPLE_GROUP;
+        if (s_full < 64u) {
+            select_streaming(p, t, hist, stage);                     // uniform: the whole workgroup goes
+            return;
+        }
+        const uint32_t sstep = s_full > (uint32_t)SEL_SAMPLE ? 2u : 1u;
+        const uint32_t S = s_full / sstep;
+        constexpr int SPT = SEL_SAMPLE / SEL_THREADS;
+        const float *smp = p.sample + (size_t)t * (p.score_stride / LI_SAMPLE_GROUP);
+        float sx[SPT];
+        bool sval[SPT];
+#pragma unroll
+        for (int e = 0; e < SPT; ++e) {
+            const uint32_t i = (uint32_t)(tid + e * SEL_THREADS);
+            sval[e] = i < S;
+            sx[e] = smp[(sval[e] ? i : 0u) * sstep];
+        }
+        // the row as 16-byte vectors: thread tid holds vectors u*1024 + tid of a chunk.  The row buffer is
+        // score_stride (a multiple of 32) long, so whole vectors stay inside it.
+        const int last_vec = (int)(p.score_stride >> 2) - 1;
+        auto load_chunk = [&](const int c0, f32x4 (&v)[8]) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int vi = (c0 >> 2) + u * SEL_THREADS + tid;
+                v[u] = reinterpret_cast<const f32x4 *>(srow)[vi < last_vec ? vi : last_vec];
+            }
+        };
+        f32x4 v[8], vn[8];
+        load_chunk(0, v);
+        const uint32_t r0 = ((uint32_t)k * S + (uint32_t)n - 1u) / (uint32_t)n;
+        const uint32_t r = r0 + (uint32_t)(6.0f * __builtin_sqrtf((float)r0)) + 8u;
+
+        for (int i = tid; i < SEL_SBINS; i += SEL_THREADS) shist[i] = 0u;
+        for (int i = tid; i < SEL_BUCKETS / 4; i += SEL_THREADS) reinterpret_cast<u32x4 *>(boff)[i] = u32x4{0u, 0u, 0u, 0u};
+        if (tid == 0) sh_over = 0u;
+        float smin, smax;
+        {
+            float mn = __builtin_inff(), mx = -__builtin_inff();
+#pragma unroll
+            for (int e = 0; e < SPT; ++e)
+                if (sval[e]) { mn = fminf(mn, sx[e]); mx = fmaxf(mx, sx[e]); }
+            range_of(mn, mx, smin, smax);
+        }
+        float pivot = -__builtin_inff();       // candidates: score >= pivot
+        float blo = smin;                      // lower edge of the lowest bucket
+        if (r < S) {
+            const float range = smax - smin;
+            const float sscale = range > 0.f ? (float)SEL_SBINS / range : 0.f;
+#pragma unroll
+            for (int e = 0; e < SPT; ++e) {
+                if (sval[e]) {
+                    const uint32_t sb = (uint32_t)fmaxf((sx[e] - smin) * sscale, 0.f);
+                    atomicAdd(&shist[sb < (uint32_t)SEL_SBINS ? sb : (uint32_t)SEL_SBINS - 1u], 1u);
+                }
+            }
+            __syncthreads();
+            // one wave scans the 1024 bins from the top (lane l owns the 16 bins below 1024 - 16*l): the bin in which the running
+            // count reaches r.  (Every wave by itself, without the barrier: 2.2 thousand clocks of vector work instead of 0.9.)
+            if (wv == 0) {
+                const u32x4 *src = reinterpret_cast<const u32x4 *>(&shist[SEL_SBINS - 16 - 16 * lane]);
+                uint32_t tot = 0;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const u32x4 x = src[q];
+                    tot += (x[0] + x[1]) + (x[2] + x[3]);
+                }
+                const uint32_t before = wave_incl_scan(tot) - tot;
+                // (found by exactly one lane: the sample holds S >= r scores); then the bin among its sixteen, a lane each
+                const int at = __ffsll((long long)__ballot(before < r && r <= before + tot)) - 1;
+                const uint32_t top = (uint32_t)(SEL_SBINS - 1 - 16 * at);
+                const uint32_t cnt = shist[top - (uint32_t)(lane & 15)];
+                const uint32_t incl = (uint32_t)__builtin_amdgcn_readlane((int)before, at) + row_incl_scan(cnt);
+                const int in = __ffsll((long long)__ballot(incl - cnt < r && r <= incl)) - 1;
+                if (lane == 0) sh_pb = top - (uint32_t)in;
+            }
+            __syncthreads();
+            const uint32_t pb = sh_pb;
+            pivot = smin + (float)pb * (range * (1.0f / (float)SEL_SBINS));
+            blo = pivot;
+        }
+        // the buckets reach a quarter of the range past the sample maximum, so that the few scores above
+        // it spread out too; anything beyond shares bucket 0
+        const float bscale = smax - blo > 0.f ? (float)SEL_BUCKETS / (1.25f * (smax - blo)) : 0.f;
+
+        // ---- 2. candidates.  Wave w compacts the positions of the candidates among its keys into its own region of the
+        // list, cand[w*SEL_WAVE_CAP ...], so the waves share no counter.  A key costs a compare and an add-with-carry that
+        // shifts the outcome into the lane's mask of its 32 keys; the few candidates (one key in twenty of a long row) are then
+        // picked out of the masks, a candidate of every lane per trip, and their scores fetched again below (out of the L2).
+        // (One LDS write per key, candidate or not, as before, took 14 to 17 of the kernel's 33 thousand clocks on 50 K keys.)
+        // Wave-wide sums use DPP, not LDS.
+        uint32_t wave_count = 0;               // candidates of this wave so far (uniform)
+        auto scan_chunk = [&](const int c0, auto full_tag) {
+            constexpr bool FULL = decltype(full_tag)::value;          // the whole chunk lies inside the row
+            const int i_base = c0 + 4 * tid;
+            uint32_t m = 0;                                           // key (u, c) is bit 31 - (4u + c)
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const int i = i_base + 4 * u * SEL_THREADS + c;
+                    m = m + m + (((FULL || i < n) && v[u][c] >= pivot) ? 1u : 0u);
+                }
+            }
+            const uint32_t mine = (uint32_t)__popc(m);
+            const uint32_t incl = wave_incl_scan(mine);
+            const uint32_t wave_n = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+            if (wave_count + wave_n > (uint32_t)SEL_WAVE_CAP) {       // region overflow: the streaming path will run
+                if (lane == 0) sh_over = 1u;
+                return;
+            }
+            uint32_t slot = (uint32_t)(wv * SEL_WAVE_CAP) + wave_count + incl - mine;
+            wave_count += wave_n;
+            while (m != 0u) {
+                const uint32_t q = (uint32_t)__clz(m);                // 4u + c
+                m &= 0x7fffffffu >> q;
+                cand[slot++] = (uint32_t)i_base + ((q >> 2) * (4u * SEL_THREADS) + (q & 3u));
+            }
+        };
+        for (int c0 = 0; c0 < n; c0 += SEL_CHUNK) {
+            if (c0 + SEL_CHUNK < n) load_chunk(c0 + SEL_CHUNK, vn);
+            if (c0 + SEL_CHUNK <= n) scan_chunk(c0, std::true_type{});
+            else scan_chunk(c0, std::false_type{});
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = vn[u];
+        }
+        if (lane == 0) wave_tot[wv] = wave_count;
+
+        // ---- 3. bucket of every candidate of the wave's own region (up to eight per lane) and its slot
+        // inside the bucket
+        uint32_t cpos[CPT];
+        float csc[CPT];
+#pragma unroll
+        for (int u = 0; u < CPT; ++u) {
+            const uint32_t j = (uint32_t)(u * 64 + lane);
+            cpos[u] = j < wave_count ? cand[wv * SEL_WAVE_CAP + j] : 0u;
+            csc[u] = (uint32_t)(u * 64) < wave_count ? srow[cpos[u]] : 0.f;             // (uniform: trips past the last are left out)
+        }
+#pragma unroll
+        for (int u = 0; u < CPT; ++u)
+            if ((uint32_t)(u * 64 + lane) < wave_count) to_bucket(u, csc[u], cpos[u], blo, bscale);
+        __syncthreads();
+        const uint32_t n_cand = (uint32_t)__builtin_amdgcn_readlane((int)row_incl_scan(wave_tot[lane & 15]), 15);
+        if (sh_over != 0u || n_cand < (uint32_t)k) {
+            select_streaming(p, t, hist, stage);                     // uniform: the whole workgroup goes
+            return;
+        }
     }
 
     // ---- 4. bucket offsets (eight buckets per thread) and the bucket holding the k-th best key
@@ -1144,12 +1149,14 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
         __syncthreads();
         const uint32_t of_wave = wave_sum[lane & 15];
         uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)(row_incl_scan(of_wave) - of_wave), wv) + incl - tot;
-        const bool here = before < (uint32_t)k && (uint32_t)k <= before + tot;
+        const bool here = before < (uint32_t)kk && (uint32_t)kk <= before + tot;
+        uint32_t longest = 0u;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const uint32_t cnt = c[e >> 2][e & 3];
             c[e >> 2][e & 3] = before;
-            if (here && before < (uint32_t)k && (uint32_t)k <= before + cnt) {
+            longest = longest > cnt ? longest : cnt;
+            if (here && before < (uint32_t)kk && (uint32_t)kk <= before + cnt) {
                 sh_tb = (uint32_t)(8 * tid + e);
                 sh_stage = before + cnt;
             }
@@ -1158,8 +1165,10 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
         mine[0] = c[0];
         mine[1] = c[1];
         if (tid == SEL_THREADS - 1) boff[SEL_BUCKETS] = before;
+        if (n <= k && longest > (uint32_t)SEL_COUNT_MAX) sh_over = 1u;
     }
     __syncthreads();
+    if (n <= k && sh_over != 0u) return sort_row();
     const uint32_t tb = sh_tb;
     const uint32_t n_stage = sh_stage;
     if (n_stage > (uint32_t)SEL_STAGE) {
@@ -1210,7 +1219,7 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             const uint32_t fin = beg[q] + rank[q];
-            if (i0 + (uint32_t)(q * SEL_THREADS + tid) < n_stage && fin < (uint32_t)k) out[fin] = (int32_t)(~(uint32_t)e[q]);
+            if (i0 + (uint32_t)(q * SEL_THREADS + tid) < n_stage && fin < (uint32_t)kk) out[fin] = (int32_t)(~(uint32_t)e[q]);
         }
     }
 }

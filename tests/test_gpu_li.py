@@ -272,3 +272,18 @@ def test_indexer_launches_of_more_than_one_round(b, s1, lo, hi, cap):
         r = slice(i * s1, (i + 1) * s1)
         pypto_amd.lightning_indexer_decode(q[r], qs[r], keys, ks, w[r], act[i:i + 1], table[i:i + 1].contiguous(), one)
         assert torch.equal(got[r], one), i
+
+
+@pytest.mark.parametrize("variant", ["fp16", "fp32"])
+@pytest.mark.parametrize("act,k", [([513, 512, 1000, 1023, 1024, 1025, 2047, 2048], 2048), ([600, 599, 513, 601, 20], 600),
+                                   ([1, 2, 3, 63, 64, 65, 100, 129, 450], 2048), ([1, 2, 1], 1)])
+def test_rows_of_at_most_k_keys_are_ordered_by_buckets_or_sorted(c_oracle, variant, act, k):
+    """Every key is taken: the order alone counts.  The last two rows have equal scores (all of them) and a score far from the
+    rest, so that nearly all keys fall into one bucket."""
+    act = act + [min(900, k), min(1500, k)]
+    inp = gen_indexer_inputs(len(act), 1, act, selected_count=k, seed=k, variant=variant)
+    inp.idx_weight[-2] = 0
+    pos = min(17, act[-1] - 1)
+    page = inp.block_table[-1].long()[pos // 128]
+    inp.idx_key_scale.reshape(-1)[page * 128 + pos % 128] = 60000.0
+    assert_exact(run_op(inp), oracle(inp, c_oracle), f"{variant} k={k}")
