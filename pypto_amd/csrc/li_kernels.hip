@@ -862,7 +862,8 @@ __device__ void bitonic_sort_desc(unsigned long long *buf, const int width, cons
 constexpr int SEL_SAMPLE = 4096;   // most keys sampled from a row
 constexpr int SEL_CAP = 8192;      // candidates (keys above the pivot) the fast path holds in LDS
 constexpr int SEL_STAGE = 4096;    // entries of the buckets down to the one holding the k-th best
-constexpr int SEL_COUNT_MAX = 128; // rows of at most k keys: most keys of a bucket that are ordered by counting
+constexpr int SEL_DIRECT = 8192;   // rows whose keys all go to the buckets
+constexpr int SEL_COUNT_MAX = 128; // of those: most keys of a bucket that are ordered by counting
 
 // the 64-bit word whose descending order is (score descending, position ascending); never zero
 __device__ __forceinline__ unsigned long long order_word(const float score, const uint32_t pos)
@@ -896,6 +897,7 @@ constexpr int SEL_CHUNK = 32 * SEL_THREADS;   // scores one trip of the row scan
 //   4. a prefix sum over the bucket counts finds the bucket holding the k-th best key; the buckets
 //      down to it are staged contiguously and each is ordered by counting (a key's rank = the number
 //      of larger keys of its bucket).  Output slots below k are written straight to memory.
+// Rows of up to SEL_DIRECT keys skip the first two: all their keys are candidates.
 // A chain of short phases: what each costs is the latency of its loads or the vector work of sixteen waves on four SIMDs, so work
 // that every wave would do alike is done by one (the pivot), or by a row of lanes (sums over the waves), and buckets are many
 // and short.  Clocks at 32 K scores: sample and minimum 5.9 K, pivot 1.9, scan 3.7 (the row arrives at 14-20 bytes per clock),
@@ -951,16 +953,51 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
         cb[u] = (uint32_t)SEL_BUCKETS - 1u - (lin < (uint32_t)SEL_BUCKETS ? lin : (uint32_t)SEL_BUCKETS - 1u);
         cslot[u] = atomicAdd(&boff[cb[u]], 1u);
     };
+    auto no_candidates = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < CPT; ++u) {
-        ce[u] = 0ull;
-        cb[u] = (uint32_t)SEL_BUCKETS;     // none
-        cslot[u] = 0u;
-    }
-    // A row of at most k keys, two per thread: all of them go straight to the buckets, spread over their own range.  Where too
-    // many fall together (equal scores, one far from the rest, an infinite one), or one is not a number, they are sorted.
-    // (Always sorted beyond 512 keys and ordered by counting over the whole row up to there, as before, two sequences of 450
-    // keys took 24.3 us instead of 9.8, scores included, of 650 keys 18.5, of 1900 22.0 instead of 11.0.)
+        for (int u = 0; u < CPT; ++u) {
+            ce[u] = 0ull;
+            cb[u] = (uint32_t)SEL_BUCKETS; // none
+            cslot[u] = 0u;
+        }
+    };
+    // ---- 4. bucket offsets (eight buckets per thread) and the bucket holding the k-th best key (sh_over: one of them is too long)
+    auto offsets = [&]() {
+        u32x4 *const mine = reinterpret_cast<u32x4 *>(boff) + 2 * tid;
+        u32x4 c[2];
+        c[0] = mine[0];
+        c[1] = mine[1];
+        const uint32_t tot = ((c[0][0] + c[0][1]) + (c[0][2] + c[0][3])) + ((c[1][0] + c[1][1]) + (c[1][2] + c[1][3]));
+        const uint32_t incl = wave_incl_scan(tot);
+        if (lane == 63) wave_sum[wv] = incl;
+        __syncthreads();
+        const uint32_t of_wave = wave_sum[lane & 15];
+        uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)(row_incl_scan(of_wave) - of_wave), wv) + incl - tot;
+        const bool here = before < (uint32_t)kk && (uint32_t)kk <= before + tot;
+        uint32_t longest = 0u;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const uint32_t cnt = c[e >> 2][e & 3];
+            c[e >> 2][e & 3] = before;
+            if (before < (uint32_t)kk && longest < cnt) longest = cnt;
+            if (here && before < (uint32_t)kk && (uint32_t)kk <= before + cnt) {
+                sh_tb = (uint32_t)(8 * tid + e);
+                sh_stage = before + cnt;
+            }
+            before += cnt;
+        }
+        mine[0] = c[0];
+        mine[1] = c[1];
+        if (tid == SEL_THREADS - 1) boff[SEL_BUCKETS] = before;
+        if (longest > (uint32_t)SEL_COUNT_MAX) sh_over = 1u;
+        __syncthreads();
+    };
+    // A short row, up to eight keys per thread: all of them go straight to the buckets, spread over their own range.  Where too
+    // many fall together (equal scores, one far from the rest, an infinite one), or one is not a number, a row of which every key
+    // is taken is sorted, and a longer one goes the way of the others.
+    // (Rows of at most k keys always sorted beyond 512 keys and ordered by counting over the whole row up to there, as before,
+    // two sequences of 450 keys took 24.3 us instead of 9.6, scores included, of 650 keys 18.5, of 1900 22.0 instead of 10.8.
+    // By way of a pivot, two of 2200 keys take 13.5, as here 11.2, of 4096 15.0 and 12.1, of 8100 15.1 and 13.4.)
     auto sort_row = [&]() {
         int width = 64;
         while (width < n) width <<= 1;
@@ -969,22 +1006,41 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
         bitonic_sort_desc(stage, width, tid);
         for (int i = tid; i < n; i += SEL_THREADS) out[i] = (int32_t)(~(uint32_t)stage[i]);
     };
-    if (n <= k) {
-        static_assert(LI_MAX_SELECT <= 2 * SEL_THREADS && CPT >= 2, "two keys per thread");
-        float x[2];
+    bool ordered = false;
+    if (n <= SEL_DIRECT) {
+        static_assert(LI_MAX_SELECT <= SEL_DIRECT && SEL_DIRECT <= CPT * SEL_THREADS, "a candidate's place for every key");
+        float x[CPT];
+        float mn = __builtin_inff(), mx = -__builtin_inff();
 #pragma unroll
-        for (int e = 0; e < 2; ++e) x[e] = srow[tid + e * SEL_THREADS < n ? tid + e * SEL_THREADS : tid < n ? tid : 0];
+        for (int e = 0; e < CPT; ++e) {
+            const int i = tid + e * SEL_THREADS;
+            x[e] = e * SEL_THREADS < n ? srow[i < n ? i : 0] : 0.f;
+        }
         for (int i = tid; i < SEL_BUCKETS / 4; i += SEL_THREADS) reinterpret_cast<u32x4 *>(boff)[i] = u32x4{0u, 0u, 0u, 0u};
         if (tid == 0) sh_over = 0u;
-        float smin, smax;
-        range_of(fminf(x[0], x[1]), fmaxf(x[0], x[1]), smin, smax);
-        const float scale = smax - smin > 0.f ? (float)SEL_BUCKETS / (smax - smin) : 0.f;
-        if (!(x[0] == x[0]) || !(x[1] == x[1])) sh_over = 1u;
+        bool odd = false;
 #pragma unroll
-        for (int e = 0; e < 2; ++e)
+        for (int e = 0; e < CPT; ++e)
+            if (e * SEL_THREADS < n) {
+                mn = fminf(mn, x[e]);
+                mx = fmaxf(mx, x[e]);
+                odd |= !(x[e] == x[e]);
+            }
+        float smin, smax;
+        range_of(mn, mx, smin, smax);
+        if (odd) sh_over = 1u;
+        const float scale = smax - smin > 0.f ? (float)SEL_BUCKETS / (smax - smin) : 0.f;
+        no_candidates();
+#pragma unroll
+        for (int e = 0; e < CPT; ++e)
             if (tid + e * SEL_THREADS < n) to_bucket(e, x[e], (uint32_t)(tid + e * SEL_THREADS), smin, scale);
         __syncthreads();
-    } else {
+        offsets();
+        ordered = sh_over == 0u;
+        if (!ordered && n <= k) return sort_row();
+        if (!ordered) __syncthreads();     // (everyone has seen it)
+    }
+    if (!ordered) {
         // ---- 1. sample: the loads go out first, then the first chunk of the row, so that one memory
         // latency covers both
         // (the score kernel left one score of every 16 positions in a compact array; a row longer than
@@ -1021,6 +1077,7 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
         const uint32_t r0 = ((uint32_t)k * S + (uint32_t)n - 1u) / (uint32_t)n;
         const uint32_t r = r0 + (uint32_t)(6.0f * __builtin_sqrtf((float)r0)) + 8u;
 
+        no_candidates();
         for (int i = tid; i < SEL_SBINS; i += SEL_THREADS) shist[i] = 0u;
         for (int i = tid; i < SEL_BUCKETS / 4; i += SEL_THREADS) reinterpret_cast<u32x4 *>(boff)[i] = u32x4{0u, 0u, 0u, 0u};
         if (tid == 0) sh_over = 0u;
@@ -1135,40 +1192,9 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
             select_streaming(p, t, hist, stage);                     // uniform: the whole workgroup goes
             return;
         }
+        offsets();
     }
 
-    // ---- 4. bucket offsets (eight buckets per thread) and the bucket holding the k-th best key
-    {
-        u32x4 *const mine = reinterpret_cast<u32x4 *>(boff) + 2 * tid;
-        u32x4 c[2];
-        c[0] = mine[0];
-        c[1] = mine[1];
-        const uint32_t tot = ((c[0][0] + c[0][1]) + (c[0][2] + c[0][3])) + ((c[1][0] + c[1][1]) + (c[1][2] + c[1][3]));
-        const uint32_t incl = wave_incl_scan(tot);
-        if (lane == 63) wave_sum[wv] = incl;
-        __syncthreads();
-        const uint32_t of_wave = wave_sum[lane & 15];
-        uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)(row_incl_scan(of_wave) - of_wave), wv) + incl - tot;
-        const bool here = before < (uint32_t)kk && (uint32_t)kk <= before + tot;
-        uint32_t longest = 0u;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const uint32_t cnt = c[e >> 2][e & 3];
-            c[e >> 2][e & 3] = before;
-            longest = longest > cnt ? longest : cnt;
-            if (here && before < (uint32_t)kk && (uint32_t)kk <= before + cnt) {
-                sh_tb = (uint32_t)(8 * tid + e);
-                sh_stage = before + cnt;
-            }
-            before += cnt;
-        }
-        mine[0] = c[0];
-        mine[1] = c[1];
-        if (tid == SEL_THREADS - 1) boff[SEL_BUCKETS] = before;
-        if (n <= k && longest > (uint32_t)SEL_COUNT_MAX) sh_over = 1u;
-    }
-    __syncthreads();
-    if (n <= k && sh_over != 0u) return sort_row();
     const uint32_t tb = sh_tb;
     const uint32_t n_stage = sh_stage;
     if (n_stage > (uint32_t)SEL_STAGE) {

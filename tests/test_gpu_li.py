@@ -275,12 +275,13 @@ def test_indexer_launches_of_more_than_one_round(b, s1, lo, hi, cap):
 
 
 @pytest.mark.parametrize("variant", ["fp16", "fp32"])
-@pytest.mark.parametrize("act,k", [([513, 512, 1000, 1023, 1024, 1025, 2047, 2048], 2048), ([600, 599, 513, 601, 20], 600),
-                                   ([1, 2, 3, 63, 64, 65, 100, 129, 450], 2048), ([1, 2, 1], 1)])
-def test_rows_of_at_most_k_keys_are_ordered_by_buckets_or_sorted(c_oracle, variant, act, k):
-    """Every key is taken: the order alone counts.  The last two rows have equal scores (all of them) and a score far from the
+@pytest.mark.parametrize("act,k,equal,far", [([513, 512, 1000, 1023, 1024, 1025, 2047, 2048], 2048, 900, 1500), ([600, 599, 513, 601, 20], 600, 600, 600),
+                                             ([1, 2, 3, 63, 64, 65, 100, 129, 450], 2048, 900, 1500), ([1, 2, 1], 1, 1, 1),
+                                             ([2049, 3000, 4096, 4097, 8191, 8192, 8193], 2048, 5000, 7000), ([1025, 7169, 9000], 1000, 8192, 1001)])
+def test_short_rows_are_ordered_by_buckets_or_another_way(c_oracle, variant, act, k, equal, far):
+    """All keys of a short row go to the buckets.  The last two rows have equal scores (all of them) and a score far from the
     rest, so that nearly all keys fall into one bucket."""
-    act = act + [min(900, k), min(1500, k)]
+    act = act + [equal, far]
     inp = gen_indexer_inputs(len(act), 1, act, selected_count=k, seed=k, variant=variant)
     inp.idx_weight[-2] = 0
     pos = min(17, act[-1] - 1)
