@@ -22,7 +22,8 @@ constexpr int XL_GROUP = 8;                                            // blocks
 constexpr int XL_TOK = 8;                                              // tokens per workgroup
 constexpr int XL_WAVES = XL_GROUP;                                     // one block per wave
 constexpr int XL_W_BYTES = XL_BLOCK * 256;                             // a block of one slab: 64 rows x 256 bytes
-constexpr int XL_REGION = XL_W_BYTES + XL_TOK * XL_BLOCK * 4;          // + the hidden states as fp32
+constexpr int XL_X_BYTES = XL_TOK * XL_BLOCK * 4;                      // the hidden states as fp32
+constexpr int XL_REGION = XL_W_BYTES + XL_X_BYTES + XL_TOK * XL_BLOCK * 2;   // + as they come
 constexpr int XL_LDS = XL_WAVES * XL_REGION;
 
 struct XlSlab {
@@ -58,6 +59,10 @@ __device__ __forceinline__ void xl_body(const XlSlab &sl, const uint16_t *x, con
     if (w < nb) {
         const int k0 = c * XL_BLOCK;
         const uint32_t wdst = (uint32_t)(uintptr_t)(lds_byte_t *)region;
+        {   // the hidden states first: lane l hidden states k0 + 8*(l%8) .. +7 of token t0 + l/8
+            const int t = t0 + (l >> 3);
+            dma16(x + (size_t)(t < T ? t : T - 1) * h + k0 + 8 * (l & 7), wdst + XL_W_BYTES + XL_X_BYTES);
+        }
         {   // rows of wbytes bytes: wbytes/16 lanes per row
             const int lpr = wbytes >> 4;
             const int rpi = 64 / lpr;                                     // rows per request
@@ -67,33 +72,50 @@ __device__ __forceinline__ void xl_body(const XlSlab &sl, const uint16_t *x, con
 #pragma unroll 1
             for (int i = 0; i < XL_BLOCK / rpi; ++i) dma16(src + (size_t)i * rpi * pitch, wdst + 1024 * i);
         }
+        if (wbytes == 256) VM_WAIT(16);                                   // everything but the sixteen requests of the weights
+        else VM_WAIT(0);
+        asm volatile("" ::: "memory");
+        {
+            const u32x4 xr = *reinterpret_cast<const u32x4 *>(region + XL_W_BYTES + XL_X_BYTES + 16 * l);
+            float *dst = xs + 8 * l;
 #pragma unroll
-        for (int u = 0; u < XL_TOK / 2; ++u) {   // lane l: hidden states k0 + 2*(l%32), +1 of token t0 + 2u + l/32
-            const int t = t0 + 2 * u + (l >> 5);
-            const int tt = t < T ? t : T - 1;
-            const uint32_t xv = reinterpret_cast<const uint32_t *>(x + (size_t)tt * h + k0)[l & 31];
-            f32x2 v = {__uint_as_float(xv << 16), __uint_as_float(xv & 0xffff0000u)};
-            *reinterpret_cast<f32x2 *>(xs + (2 * u + (l >> 5)) * XL_BLOCK + 2 * (l & 31)) = v;
-        }
-        VM_WAIT(0);
-        const int rowdw = wbytes >> 2;
-        const uint32_t *wl = reinterpret_cast<const uint32_t *>(region) + (l & (rowdw - 1));   // lanes past the slab's width repeat earlier ones
-#pragma unroll 2
-        for (int kk = 0; kk < XL_BLOCK; kk += 4) {
-            f32x4 xv[XL_TOK];
-#pragma unroll
-            for (int t = 0; t < XL_TOK; ++t) xv[t] = *reinterpret_cast<const f32x4 *>(xs + t * XL_BLOCK + kk);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t wv = wl[(kk + j) * rowdw];
-                const float w0 = __uint_as_float(wv << 16), w1 = __uint_as_float(wv & 0xffff0000u);
-#pragma unroll
-                for (int t = 0; t < XL_TOK; ++t) {
-                    a0[t] = __builtin_fmaf(xv[t][j], w0, a0[t]);
-                    a1[t] = __builtin_fmaf(xv[t][j], w1, a1[t]);
-                }
+            for (int q = 0; q < 2; ++q) {
+                const f32x4 v = {__uint_as_float(xr[2 * q] << 16), __uint_as_float(xr[2 * q] & 0xffff0000u),
+                                 __uint_as_float(xr[2 * q + 1] << 16), __uint_as_float(xr[2 * q + 1] & 0xffff0000u)};
+                *reinterpret_cast<f32x4 *>(dst + 4 * q) = v;
             }
         }
+        const int rowdw = wbytes >> 2;
+        const uint32_t *wl = reinterpret_cast<const uint32_t *>(region) + (l & (rowdw - 1));   // lanes past the slab's width repeat earlier ones
+        // Sixteen rows at a time, as they arrive (a whole slab's requests are of four rows each): the multiply-adds of a block
+        // take as long as half of the launch's bytes.
+        auto rows16 = [&](const int first) __attribute__((always_inline)) {
+            asm volatile("" ::: "memory");
+#pragma unroll 2
+            for (int kk = first; kk < first + 16; kk += 4) {
+                f32x4 xv[XL_TOK];
+#pragma unroll
+                for (int t = 0; t < XL_TOK; ++t) xv[t] = *reinterpret_cast<const f32x4 *>(xs + t * XL_BLOCK + kk);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t wv = wl[(kk + j) * rowdw];
+                    const float w0 = __uint_as_float(wv << 16), w1 = __uint_as_float(wv & 0xffff0000u);
+#pragma unroll
+                    for (int t = 0; t < XL_TOK; ++t) {
+                        a0[t] = __builtin_fmaf(xv[t][j], w0, a0[t]);
+                        a1[t] = __builtin_fmaf(xv[t][j], w1, a1[t]);
+                    }
+                }
+            }
+        };
+        VM_WAIT(12);                                                      // (narrower slabs have arrived)
+        rows16(0);
+        VM_WAIT(8);
+        rows16(16);
+        VM_WAIT(4);
+        rows16(32);
+        VM_WAIT(0);
+        rows16(48);
         // block sums into this wave's own (consumed) region: [8 tokens][128 columns]
         float *bs = reinterpret_cast<float *>(region);
 #pragma unroll
