@@ -327,9 +327,12 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
     // ahead unconditionally -- no per-key and no per-tile branches.
     //
     // The translation is a chain of two dependent loads (selected position, then its page in the block
-    // table) ahead of the gather itself.  When the table fits two entries per thread both loads travel
-    // as LDS-DMA requests between the Q^T passes, waited for by count, so that the chain runs beside
-    // the Q^T staging instead of after it; each lane handles the entries it requested itself.
+    // table) ahead of the gather itself.  Both travel as LDS-DMA requests between the Q^T passes, so that the chain runs beside
+    // the Q^T staging instead of after it; each lane handles the entries it requested itself.  When the table fits two entries
+    // per thread, positions and pages share its memory and are waited for by count; the pages of a longer one lie where the first
+    // tiles go later.  (A longer one entry by entry, position and then page, as before,
+    // cost a row 2 us and more: 4096 rows over 4096 keys 1561 us, now 1538, 1608 over 3848 806 and 778, 128 rows of 2048 selected keys
+    // 95.8 and 94.8.  Asking for PIPE's first tile beside the second Q^T pass: +-0.)
     constexpr int FAST_ENTRIES = 2 * NW * 64;
     static_assert(2 * FAST_ENTRIES <= SFA_MAX_CHUNK + 3 * KT, "positions and pages of the short table share its memory");
     auto padded = [](const int n) { return n > 0 ? (n + 2 * KT - 1) / (2 * KT) * (2 * KT) + 2 * KT : 0; };
@@ -351,6 +354,17 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
                  (uint32_t)(uintptr_t)(lds_byte_t *)(rows_lds + j * NW * 64 + wave_first));
         }
     };
+    // the same for a longer table, whose entries are whole waves
+    auto request_long = [&](const int kb, const int nv, const int np) {
+#pragma unroll 1
+        for (int i0 = wave_first; i0 < np; i0 += NW * 64) {
+            const int i = i0 + l;
+            dma4(p.topk_idx + (size_t)t * p.topk + kb + (i < nv ? i : 0), (uint32_t)(uintptr_t)(lds_byte_t *)(rows_lds + i0));
+        }
+    };
+    constexpr int PAGES_BASE = SP > 1 ? 0 : (QUANT ? STG_BASE : WAVE_BYTES);              // above the Q^T staging
+    static_assert(PAGES_BASE + (SFA_MAX_CHUNK + 2 * KT) * 4 <= POOL_BYTES, "the pages of a whole table fit");
+    int *const pages = reinterpret_cast<int *>(reinterpret_cast<uint8_t *>(pool) + PAGES_BASE);
     // A decoding row nearly always sees all topk selected keys.  The positions of this split are requested on
     // that assumption before the sequence length has arrived, which takes one memory latency out of the chain
     // length -> positions -> pages -> rows -> first tile; if the length says otherwise they are requested
@@ -360,6 +374,7 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
     const int nv_s = ke_s - kb_s;
     const bool fast_s = nv_s > 0 && padded(nv_s) <= FAST_ENTRIES;              // uniform
     if (fast_s) request_positions(kb_s, nv_s);
+    else if (nv_s > 0) request_long(kb_s, nv_s, padded(nv_s));
     if constexpr (SP == 1) request_q(0);                                      // 16 requests
     else load_q();
     int cur = act_b - p.S1 + 1 + s1i;
@@ -369,7 +384,7 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
     const int n_valid = k_end - k_begin;
     const int n_pad = padded(n_valid);
     const bool fast = n_valid > 0 && n_pad <= FAST_ENTRIES;                    // uniform
-    const bool as_assumed = fast_s && k_begin == kb_s && n_valid == nv_s;     // uniform
+    const bool as_assumed = nv_s > 0 && k_begin == kb_s && n_valid == nv_s;   // uniform
     if (fast) {
         if (as_assumed) {
             land_q();
@@ -387,7 +402,21 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
         }
         collect_q(0, std::integral_constant<int, 2>{});
     } else {
-        collect_q(0, std::integral_constant<int, 0>{});
+        if (n_valid > 0) {
+            if (as_assumed) {
+                land_q();
+                __builtin_amdgcn_s_waitcnt(vmcnt_imm(SP == 1 ? 16 : 0));      // the positions have landed
+            } else {
+                request_long(k_begin, n_valid, n_pad);
+                __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+            }
+            asm volatile("" ::: "memory");
+#pragma unroll 1
+            for (int i0 = wave_first; i0 < n_pad; i0 += NW * 64)
+                dma4(p.bt + (size_t)b * p.maxblk + block_of(rows_lds[i0 + l]), (uint32_t)(uintptr_t)(lds_byte_t *)(pages + i0));
+        }
+        if constexpr (SP > 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        collect_q(0, std::integral_constant<int, 0>{});                       // (and the pages)
     }
     if constexpr (SP == 1) request_q(1);                                      // 20 requests
     if (fast) {
@@ -399,10 +428,9 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
             rows_lds[i] = row_of(rows_lds[i], rows_lds[FAST_ENTRIES + i]);
         }
     } else {
-        for (int i = tid; i < n_pad; i += NW * 64) {
-            const int idx = p.topk_idx[(size_t)t * p.topk + k_begin + (i < n_valid ? i : 0)];
-            rows_lds[i] = row_of(idx, p.bt[(size_t)b * p.maxblk + block_of(idx)]);
-        }
+        asm volatile("" ::: "memory");
+#pragma unroll 1
+        for (int i = tid; i < n_pad; i += NW * 64) rows_lds[i] = row_of(rows_lds[i], pages[i]);
     }
 
     // the first tile's products start the accumulators from zero (acc_mfma_first); they are cleared beforehand
