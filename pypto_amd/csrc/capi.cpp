@@ -125,8 +125,14 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
 {
     SfaPlan pl;
     const long long rows = a->b * a->s1;
-    const int tiles = (int)((a->topk + pto::SFA_KEY_TILE - 1) / pto::SFA_KEY_TILE);
+    const int topk_tiles = (int)((a->topk + pto::SFA_KEY_TILE - 1) / pto::SFA_KEY_TILE);
     const int min_split = (int)((a->topk + pto::SFA_MAX_CHUNK - 1) / pto::SFA_MAX_CHUNK);
+    // A row has no more keys than its pages hold, whatever topk is, and is priced by those (147 rows of 32 heads over up to 374 keys,
+    // bf16 cache, 32.9 us by a topk of 2048, by three pages 24.0; 100 rows of 128 heads over up to 900 keys 42.3 and 38.5, 384 over up
+    // to 300 71.5 and 65.7; 2 rows over 900 keys, where more splits than they are priced at would be better, 12.5 and 13.5).  The
+    // launches whose partial results are fp16 stay the ones that topk gives.
+    const long long row_keys = a->max_blocknum_perbatch * a->block_size;
+    const int tiles = a->num_splits == 0 && min_split == 1 && row_keys < a->topk ? (int)((row_keys + pto::SFA_KEY_TILE - 1) / pto::SFA_KEY_TILE) : topk_tiles;
     // (a size query on a host without a device plans for the 256 CUs of an MI355X; a launch there fails)
     const int cus = cu_count() > 0 ? cu_count() : 256;
     auto shares = [&](const int hg) { return (int)((a->nq + 32 * hg - 1) / (32 * hg)); };
@@ -162,21 +168,21 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
     // larger by; only workgroups of one head group leave them.  16 heads, whole rows against fp32 partials: 50 rows of 256 keys
     // 18.1 us and 14.7, 150 of 1024 58.7 and 52.3, 170 of 2048 109 and 88.6 -- as fp16 partials 12.8, 50.1 and 85.7.)
     auto half_partials = [&]() {
-        const int sh = shares(hg_max), max_split = tiles / 4;
+        const int sh = shares(hg_max), max_split = topk_tiles / 4;
         if (cus % 8 != 0) return max_split > 1 && rows * sh < cus;
         const long long xcd_cus = cus / 8, xcd_rows = (rows + 7) / 8;
         auto xcd_rounds = [&](const int s) { return (double)((xcd_rows * sh * s + xcd_cus - 1) / xcd_cus); };
-        const double whole = xcd_rounds(1) * (tiles + 3.0);
+        const double whole = xcd_rounds(1) * (topk_tiles + 3.0);
         auto merge = [&](const long long r, const int s) { return 1.0 + 0.01 * (double)r * s * sh; };
         for (int s = 2; s <= max_split && partial_bytes(rows, s) <= max_bytes; ++s)
-            if (xcd_rounds(s) * ((tiles + s - 1) / s + 5.5) + merge(rows, s) < whole) return true;
+            if (xcd_rounds(s) * ((topk_tiles + s - 1) / s + 5.5) + merge(rows, s) < whole) return true;
         // full rounds of whole rows, and the rows left over in as many pieces as fill one more (below)
         const long long per_round = xcd_cus / sh, full = per_round > 0 ? xcd_rows / per_round : 0;
         const long long left = xcd_rows - full * per_round, rows_b = rows - 8 * full * per_round;
         if (full < 1 || left < 1 || rows_b < 1) return false;
         const int s = (int)(per_round / left < max_split ? per_round / left : max_split);
         return s >= 2 && partial_bytes(rows_b, s) <= max_bytes &&
-               (double)full * (tiles + 3.0) + (tiles + s - 1) / s + 5.5 + merge(rows_b, s) < whole;
+               (double)full * (topk_tiles + 3.0) + (topk_tiles + s - 1) / s + 5.5 + merge(rows_b, s) < whole;
     };
     const bool f32 = a->num_splits == 0 && min_split == 1 && !half_partials();
     int ns = a->num_splits;
