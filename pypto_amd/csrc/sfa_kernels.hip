@@ -369,18 +369,21 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
     // that assumption before the sequence length has arrived, which takes one memory latency out of the chain
     // length -> positions -> pages -> rows -> first tile; if the length says otherwise they are requested
     // again (same destinations; requests complete in order, so the later ones stand).
+    // (A row of a prefill chunk may see fewer, and the length is in the scalar cache after the first of them: it is waited for.)
+    auto seen_keys = [&]() {
+        const int n = act_b - p.S1 + 1 + s1i;
+        return n < 0 ? 0 : (n > p.topk ? p.topk : n);
+    };
     int kb_s, ke_s;
-    split_keys(p.topk, kb_s, ke_s);
+    split_keys(p.S1 > 8 ? seen_keys() : p.topk, kb_s, ke_s);
     const int nv_s = ke_s - kb_s;
     const bool fast_s = nv_s > 0 && padded(nv_s) <= FAST_ENTRIES;              // uniform
     if (fast_s) request_positions(kb_s, nv_s);
     else if (nv_s > 0) request_long(kb_s, nv_s, padded(nv_s));
     if constexpr (SP == 1) request_q(0);                                      // 16 requests
     else load_q();
-    int cur = act_b - p.S1 + 1 + s1i;
-    cur = cur < 0 ? 0 : (cur > p.topk ? p.topk : cur);
     int k_begin, k_end;
-    split_keys(cur, k_begin, k_end);
+    split_keys(seen_keys(), k_begin, k_end);
     const int n_valid = k_end - k_begin;
     const int n_pad = padded(n_valid);
     const bool fast = n_valid > 0 && n_pad <= FAST_ENTRIES;                    // uniform
