@@ -184,13 +184,19 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
         return s >= 2 && partial_bytes(rows_b, s) <= max_bytes &&
                (double)full * (topk_tiles + 3.0) + (topk_tiles + s - 1) / s + 5.5 + merge(rows_b, s) < whole;
     };
+    // The rows of a prefill chunk that begins less than a third of the most keys of a row into its sequence are of all lengths: more
+    // of them than a round holds stay whole and start longest first, and the launch ends evenly by itself (the last round's rows in
+    // pieces / whole: 300 rows over 300 keys 41.7 / 33.6 us, 563 over 563 84.3 / 75.3, 2000 over 2000 529 / 511; 800 over 1500, which
+    // begin 700 keys into it, 237 / 256, 1100 over 2000 404 / 415).
+    const bool ramp = a->num_splits == 0 && min_split == 1 && a->s1 > 8 && rows * shares(hg_max) > cus &&
+                      3 * (row_keys - a->s1) < (a->topk < row_keys ? a->topk : row_keys);
     const bool f32 = a->num_splits == 0 && min_split == 1 && !half_partials();
     int ns = a->num_splits;
     double best = -1.0;
     if (ns == 0) {
         for (int hg = hg_max; hg >= 1; hg /= 2)
             // (of the split counts with equally long splits the smallest is the one to take)
-            for (int s = min_split, len = 0; s <= (f32 ? (hg > 1 ? 1 : tiles < 8 ? tiles : 8) : tiles); s = len > 1 ? (tiles + len - 2) / (len - 1) : tiles + 1) {
+            for (int s = min_split, len = 0; s <= (ramp ? 1 : f32 ? (hg > 1 ? 1 : tiles < 8 ? tiles : 8) : tiles); s = len > 1 ? (tiles + len - 2) / (len - 1) : tiles + 1) {
                 len = (tiles + s - 1) / s;
                 const long long wgs = rows * shares(hg) * s;
                 if (s > min_split && (partial_bytes(rows, s, f32) > max_bytes || wgs > 4ll * cus)) break;
@@ -210,7 +216,7 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
     pl.nsplit = ns;
     pl.whole_slots = 0;
     long long split_rows = rows;
-    if (a->num_splits == 0 && min_split == 1 && !f32 && cus % 8 == 0) {
+    if (a->num_splits == 0 && min_split == 1 && !f32 && !ramp && cus % 8 == 0) {
         // More rows than compute units: the full rounds of whole rows first, then the rows left over dealt out in
         // as many pieces as fill one more round (300 rows on 256 CUs: 32 whole rows per XCD, the other five or
         // six in five pieces each), where that beats the best uniform split above.
@@ -270,14 +276,14 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
             pl.part_f32 = false;
             split_rows = rows - whole;
         };
-        for (int s = 1, len = 0; s <= (f32 ? 1 : tiles); s = len > 1 ? (tiles + len - 2) / (len - 1) : tiles + 1) {
+        for (int s = 1, len = 0; s <= (f32 || ramp ? 1 : tiles); s = len > 1 ? (tiles + len - 2) / (len - 1) : tiles + 1) {
             len = (tiles + s - 1) / s;
             if (s > 1 && (partial_bytes(rows, s) > pl.scratch_bytes || rows * sh * s > 4ll * cus)) break;
             const double n = (double)rounds(rows * sh * s);
             take(n * slice_round_us(s, rows * sh * s) + (n - 1.0) * 7.0 + slice_tail_us(rows, s), s, 0);    // (a further round starts and ends too)
         }
         const long long per_round = cus / 8 / sh, full = per_round > 0 ? (rows + 7) / 8 / per_round : 0, rows_b = rows - 8 * full * per_round;
-        if (!f32 && cus % 8 == 0 && full >= 1 && rows_b >= 1) {            // full rounds of whole rows, the rows left over in pieces
+        if (!f32 && !ramp && cus % 8 == 0 && full >= 1 && rows_b >= 1) {            // full rounds of whole rows, the rows left over in pieces
             int s = (int)(cus / (rows_b * sh));
             s = s > tiles / 4 ? tiles / 4 : s;
             while (s >= 2 && partial_bytes(rows_b, s) > pl.scratch_bytes) --s;

@@ -219,6 +219,9 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
         nsplit = p.nsplit;
     }
     if (t >= p.T) return;
+    // Rows of a prefill chunk see the more keys the later they are: the longest start first, so that the launch ends with short ones.
+    // (4096 rows over 4096 keys 1527 us, now 1496, 1000 over 1000 162.7 and 158.7, 655 over 655 94.8 and 88.3.)
+    if (p.S1 > 8 && p.nsplit == 1) t = p.T - 1 - t;
     const int hg = within / nsplit;
     const int sp = within % nsplit;
     const int b = t / p.S1;

@@ -87,6 +87,7 @@ __global__ __launch_bounds__(512) void sfa_slice_kernel(const SfaParams p)
         nsplit = p.nsplit;
     }
     if (t >= p.T) return;
+    if (p.S1 > 8 && p.nsplit == 1) t = p.T - 1 - t;        // (longest rows first)
     const int sp = within / p.hgroups;                     // the head shares of a split are neighbours: they gather the same rows
     const int hg = within - sp * p.hgroups;
     const int b = t / p.S1;

@@ -297,3 +297,19 @@ def test_softmax_scale_of_any_sign(scale):
     ref = oracle(inp)
     check(run_op(inp), ref, f"scale={scale}")
     check(run_op(inp, num_splits=4), ref, f"scale={scale}, 4 splits")
+
+
+@pytest.mark.parametrize("nq,act,topk", [(128, [600, 1500, 2048, 3000], 2048), (32, [513, 449, 2049, 900], 2048), (128, [577, 640, 100, 1], 640)])
+def test_long_tables_of_rows_that_see_fewer_keys_than_assumed(nq, act, topk):
+    """One workgroup per row: tables of more and of fewer than 512 entries, of rows that see all topk keys, as a decoding row is
+    assumed to, and fewer."""
+    inp = gen_sfa_inputs(len(act), 2, nq, act, topk=topk, seed=nq + topk)
+    check(run_op(inp, num_splits=1), oracle(inp), f"nq={nq} act={act} topk={topk}")
+
+
+@pytest.mark.parametrize("nq,b,s1,act", [(128, 1, 300, [300]), (64, 1, 270, [330]), (16, 1, 600, [601]), (128, 2, 140, [150, 190]), (128, 1, 270, [1300])])
+def test_prefill_rows_of_all_lengths_start_longest_first(nq, b, s1, act):
+    """More causal rows than a round of workgroups holds, whole, in every form; two sequences; and rows that begin far into their
+    sequence, the last of them in pieces."""
+    inp = gen_sfa_inputs(b, s1, nq, act, topk=512, seed=s1)
+    check(run_op(inp, entry="p"), oracle(inp), f"prefill nq={nq} s1={s1} act={act}")
