@@ -22,7 +22,8 @@
 //   li_select_kernel  one workgroup per query token, keys ordered by the strict word
 //                     (score image << 32 | ~position): a histogram of up to 4096 sampled scores (the
 //                     compact array the score kernel left) gives a pivot, one pass over the row
-//                     compacts the keys above it, those are spread over 2048 buckets linear in the
+//                     compacts the keys above it (a row of up to 8192 keys skips both: all its keys are
+//                     candidates), those are spread over 8192 buckets linear in the
 //                     score and ordered inside buckets by counting; select_streaming (radix select
 //                     over the row in memory + bitonic sort) is the capacity-free form it falls back to
 #include <type_traits>

@@ -1,14 +1,15 @@
 // Fixed-order sums over the hidden axis, one group of eight blocks of 64 rows per workgroup: x [T, h] bf16 times a
 // slab of columns of a row-major bf16 weight matrix.  Two forms: xl_body on the vector ALU, 8 tokens per workgroup (the
-// MLA prolog's fixed-order launches), and xf_body on the matrix cores, 32 tokens (the rope columns and the indexer
+// MLA prolog's fixed-order launches), and xf_body on the matrix cores, tiles of 32 tokens (the rope columns and the indexer
 // prolog's wk and w_proj from 9 tokens on in the fused operator, from 64 on alone); included after prolog_common.h.
 //
 // Every product of two bf16 values is exact in fp32; a block is summed ascending from 0.0 by fp32 FMAs, the
 // workgroup's eight block sums (one per wave) meet in LDS and are added ascending into the group sum, which is all
 // that reaches memory: out[t * out_pitch + column].  The caller adds the group sums ascending.
 //   workgroup = (slab, group of 512 hidden rows, 8 tokens), eight waves; wave w takes block 8*group + w: the block
-//   of the slab travels to the wave's LDS region by LDS-DMA, the hidden states are widened to fp32 on the way in,
-//   the product loop reads weights per lane (columns 2l, 2l+1) and the hidden states as broadcasts.
+//   of the slab travels to the wave's LDS region by LDS-DMA, behind its hidden states, which are widened to fp32 there
+//   meanwhile; the product loop takes sixteen rows at a time as they arrive, weights per lane (columns 2l, 2l+1) and hidden
+//   states as broadcasts (launch at 8 tokens 12.2 us with all rows waited for, now 11.3).
 #pragma once
 #include "prolog_common.h"
 
