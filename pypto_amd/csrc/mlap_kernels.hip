@@ -20,9 +20,9 @@
 //                        chained into the group sum.  Below MLAP_MFMA_MIN_TOKENS tokens, and with absorb_exact.
 //   mlap_xlinear_mfma_kernel   the same sums on the matrix cores (xlinear_mfma.h): per workgroup a 128-column slab x
 //                        tokens x a range of the hidden axis, v_mfma_f32_32x32x16_bf16 with the row-major weight chunk as
-//                        the transposed operand.  The launch's last workgroups take the 64 rope columns of w_dkv_kr in
-//                        their fixed order instead (the rotated key allows no outlier under the reference's acceptance
-//                        rule), and the indexer prolog's sums with them in the fused operator.
+//                        the transposed operand.  The launch's first workgroups (beyond 128 tokens its last) take the 64
+//                        rope columns of w_dkv_kr in their fixed order instead (the rotated key allows no outlier under the
+//                        reference's acceptance rule), and the indexer prolog's sums with them in the fused operator.
 //   mlap_mid_kernel      per token: group sums chained, bf16, RMS norm (one wave per slab), per-token
 //                        int8 quantisation of the query latent; RMS norm and per-slab quantisation of
 //                        the key latent, rope of the key, scatter into the caches.
@@ -118,7 +118,10 @@ __global__ __launch_bounds__(256, 2) void mlap_xlinear_mfma_kernel(const MlapPar
                                                                 const XfGrid fg, const LipParams lip)
 {
     __shared__ __attribute__((aligned(16))) uint8_t smem[XM_KERNEL_LDS<TB>];
-    constexpr bool FIXED_FIRST = TB == 1 || TB == 2;
+    // Up to 128 tokens the fixed-order sums, the longer chains, start first and the launch is one round (65 to 128 tokens, last / first:
+    // fused prolog, 72 tokens 48.1 / 46.9 us per pass, 100 52.3 / 50.4, 128 54.6 / 52.8, MLA prolog alone 128 52.4 / 50.4); beyond, where
+    // they fill more than the first places, they come last (first: 160 tokens 62.6 / 63.5, 300 90.3 / 96.1, 1000 187.9 / 203.3).
+    constexpr bool FIXED_FIRST = TB != XM_BIG;
     const int nfixed = (int)gridDim.x - own_wgs;                   // a multiple of eight, as own_wgs: the XCDs go round alike
     const int fixed = (int)blockIdx.x - (FIXED_FIRST ? 0 : own_wgs), bid = (int)blockIdx.x - (FIXED_FIRST ? nfixed : 0);
     if (FIXED_FIRST ? fixed < nfixed : fixed >= 0) {
@@ -551,7 +554,7 @@ hipError_t mlap_launch_front(const MlapParams &p, hipStream_t stream, const Mlap
         // latent that falls the other way is 9 % of its token's indexer query.  They would leave the fixed-order sums more room
         // beside them: fused prolog, 14 / 12 ranges: 129 tokens 60.0 / 60.5 us per pass, 192: 71.1 / 67.5; 14 / 10: 256 76.9 / 71.4
         // (alone 61.1 / 62.5); 14 / 12: 100 52.4 / 53.1 (alone 49.9 / 47.4).  At 256 tokens the fourteen as two to a workgroup, one
-        // after the other, take 84.0, with the fixed-order sums first 83.7.
+        // after the other, take 84.0.
         // Up to 64 tokens two workgroups share a compute unit, and the fixed-order sums start first (one per compute unit, those
         // last, so a second round: 9 tokens 39.1, in this form 32.2; 32: 42.5, 36.4; 48: 47.3, 43.3; 64: 52.9, 44.8, the last launch
         // in tiles of 128 tokens; two ranges per workgroup: 9 tokens 33.5, 32: 37.0, 48: 47.1, 64: 52.5).
