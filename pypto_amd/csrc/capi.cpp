@@ -92,6 +92,7 @@ struct SfaPlan {
     int hgroups;          // workgroups that share a row's heads
     int nsplit;
     int whole_slots;      // rows 0 .. 8 * whole_slots - 1 are not split
+    long long split_rows; // the others, or all of them
     bool part_f32;        // partial results in fp32 instead of fp16
     size_t scratch_bytes; // what a caller is asked for, for partial results: the launch uses as much or less
     size_t part_o_bytes;  // what the launch uses of it
@@ -119,89 +120,113 @@ int sfa_check(const PtoSfaQuantArgs *a)
     return PTO_OK;
 }
 
-// max_bytes: most bytes of partial results the caller can hold; the automatic choice (num_splits = 0) then takes the
-// best split count among those that fit (an explicit count is the caller's own business)
-SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
-{
-    SfaPlan pl;
-    const long long rows = a->b * a->s1;
-    const int topk_tiles = (int)((a->topk + pto::SFA_KEY_TILE - 1) / pto::SFA_KEY_TILE);
-    const int min_split = (int)((a->topk + pto::SFA_MAX_CHUNK - 1) / pto::SFA_MAX_CHUNK);
-    // A row has no more keys than its pages hold, whatever topk is, and is priced by those (147 rows of 32 heads over up to 374 keys,
-    // bf16 cache, 32.9 us by a topk of 2048, by three pages 24.0; 100 rows of 128 heads over up to 900 keys 42.3 and 38.5, 384 over up
-    // to 300 71.5 and 65.7; 2 rows over 900 keys, where more splits than they are priced at would be better, 12.5 and 13.5).  The
-    // launches whose partial results are fp16 stay the ones that topk gives.
-    const long long row_keys = a->max_blocknum_perbatch * a->block_size;
-    const int tiles = a->num_splits == 0 && min_split == 1 && row_keys < a->topk ? (int)((row_keys + pto::SFA_KEY_TILE - 1) / pto::SFA_KEY_TILE) : topk_tiles;
-    // (a size query on a host without a device plans for the 256 CUs of an MI355X; a launch there fails)
-    const int cus = cu_count() > 0 ? cu_count() : 256;
-    auto shares = [&](const int hg) { return (int)((a->nq + 32 * hg - 1) / (32 * hg)); };
-    auto partial_bytes = [&](const long long r, const int ns, const bool f32 = false) {
-        return ns > 1 ? (size_t)r * ns * a->nq * (512 * (f32 ? sizeof(float) : sizeof(uint16_t)) + 2 * sizeof(float)) : (size_t)0;
-    };
-    // The schedule model, in microseconds: what a launch pair over an int8 cache took over 1 to 128 rows x 16 to 128 heads x 1 to
-    // 64 splits (fitted to within 10 %; neighbouring choices differ by less).  The same figures serve the other cache formats
-    // and every top-k.  A compute unit holds one workgroup; a round of them
-    // is as long as a split's tiles; starting, staging the query and the first tile and the merge launch are `fixed`, and
-    // the partial results cost with the number of workgroups that write them.  Fewer head groups per workgroup make
-    // a tile shorter, and the prologue, but the tiles of a row are de-quantised once per workgroup: that pays while the
-    // chip is not full (128 heads, 1 row: 22.0 us as 16 splits of four groups, 14.3 as 32 splits of one; 4 rows: 22.5, 20.0).
-    // Two groups are priced as the form of four waves they had when the bytes a caller is asked for were settled (1.58 a tile,
-    // where sfa_slice_kernel takes 1.1 to 1.45): up to 2048 keys that price chooses nothing, the second model below does.  Beyond,
-    // where it is not asked, the choice is within 6 % of the fastest division from 64 rows on (128 heads; 64 heads: from 16 on)
-    // and dear for fewer (4096 keys of an int8 cache, 128 heads: 1 row 19.0 where 32 splits of 64 heads take 16.1, 4 rows 27.1 and
-    // 22.9, 16 rows 36.7 and 33.0).
-    auto round_us = [&](const int hg, const int ns) { return (tiles + ns - 1) / ns * (hg == 4 ? 1.75 : (hg == 2 ? 1.58 : 1.47)); };
-    auto tail_us = [&](const int hg, const long long wgs, const int ns) {
+// What dividing a call's rows over workgroups takes, in microseconds: what a launch pair over an int8 cache took over 1 to 128 rows x
+// 16 to 128 heads x 1 to 64 splits (fitted to within 10 %; neighbouring choices differ by less).  The same figures serve the other
+// cache formats and every number of keys.  A compute unit holds one workgroup; a round of them
+// is as long as a split's tiles; starting, staging the query and the first tile and the merge launch are `fixed`, and
+// the partial results cost with the number of workgroups that write them.  Fewer head groups per workgroup make
+// a tile shorter, and the prologue, but the tiles of a row are de-quantised once per workgroup: that pays while the
+// chip is not full (128 heads, 1 row: 22.0 us as 16 splits of four groups, 14.3 as 32 splits of one; 4 rows: 22.5, 20.0).
+// Two groups are priced as the form of four waves they had when the bytes a caller is asked for were settled (1.58 a tile,
+// where sfa_slice_kernel takes 1.1 to 1.45): up to 2048 keys that price chooses nothing, the second model below does.  Beyond,
+// where it is not asked, the choice is within 6 % of the fastest division from 64 rows on (128 heads; 64 heads: from 16 on)
+// and dear for fewer (4096 keys of an int8 cache, 128 heads: 1 row 19.0 where 32 splits of 64 heads take 16.1, 4 rows 27.1 and
+// 22.9, 16 rows 36.7 and 33.0).
+struct SfaPrices {
+    long long rows, nq;
+    int cus;
+    int tiles;            // of the longest row
+    bool f32;             // split rows leave fp32 partial results
+
+    int shares(const int hg) const { return (int)((nq + 32 * hg - 1) / (32 * hg)); }
+    int max_groups() const { return nq > 64 ? 4 : (nq > 32 ? 2 : 1); }
+    size_t partial_bytes(const long long r, const int ns, const bool fp32 = false) const
+    {
+        return ns > 1 ? (size_t)r * ns * nq * (512 * (fp32 ? sizeof(float) : sizeof(uint16_t)) + 2 * sizeof(float)) : (size_t)0;
+    }
+    long long rounds(const long long wgs) const { return cus % 8 == 0 ? ((wgs + 7) / 8 + cus / 8 - 1) / (cus / 8) : (wgs + cus - 1) / cus; }
+    int split_tiles(const int ns) const { return (tiles + ns - 1) / ns; }
+    // of the split counts with equally long splits the smallest is the one to take: the one behind ns
+    int next_splits(const int ns) const { return split_tiles(ns) > 1 ? (tiles + split_tiles(ns) - 2) / (split_tiles(ns) - 1) : tiles + 1; }
+
+    double round_us(const int hg, const int ns) const { return split_tiles(ns) * (hg == 4 ? 1.75 : (hg == 2 ? 1.58 : 1.47)); }
+    double tail_us(const int hg, const long long wgs, const int ns) const
+    {
         if (ns == 1) return 6.0;
         const double fixed = hg == 4 ? 10.5 : (hg == 2 ? 9.5 : 9.3), per_wg = hg == 4 ? 0.045 : (hg == 2 ? 0.032 : 0.018);
         return fixed + per_wg * (double)wgs + (ns > 8 ? (hg == 1 ? 0.5 : 1.5) : 0.0);       // (more than eight splits: the wide merge)
-    };
-    auto rounds = [&](const long long wgs) { return cus % 8 == 0 ? ((wgs + 7) / 8 + cus / 8 - 1) / (cus / 8) : (wgs + cus - 1) / cus; };
-    const int hg_max = a->nq > 64 ? 4 : (a->nq > 32 ? 2 : 1);
+    }
+    // every row in ns splits, or `full` rounds of whole rows and the rows_b left over in ns splits
+    double even(const int hg, const int ns) const
+    {
+        const long long wgs = rows * shares(hg) * ns;
+        return (double)rounds(wgs) * round_us(hg, ns) + tail_us(hg, wgs, ns) +
+               (f32 ? 0.25e-6 * (double)(partial_bytes(rows, ns, true) - partial_bytes(rows, ns)) : 0.0);
+    }
+    double mixed(const int hg, const int ns, const long long full, const long long rows_b) const
+    {
+        return (double)full * round_us(hg, 1) + round_us(hg, ns) + tail_us(hg, rows_b * shares(hg) * ns, ns);
+    }
+
+    // More than 32 heads: workgroups of 64 heads (sfa_slice_kernel).  Fitted to an int8 cache, 1 to 128 rows, top-k 2048,
+    // 128 heads (measured: 32 rows 4 splits 32.3, 16 rows 8 splits 24.2, 4 rows 13 splits 18.4, 1 row 22 splits 14.0, against
+    // 35.0, 28.6, 20.0 and 14.1 as four groups and one group of 32 heads; 36 to 64 rows alike; 128 rows 97.1 against 95.0).
+    // A tile of whole rows takes 1.13 with 128 workgroups, 1.2 with 192 and 1.45 with 256 (top-k 1024, 96 rows: 44.9, as four groups
+    // and two splits 49.4); partial results past one round's cost more (64 heads, 96 rows: 5 splits 58.8, 2 splits 51.8).
+    // Against the fastest of every form and split count, two rows and more, top-k 1024 and 2048, both caches, the choice is within
+    // 5 % in 104 of 108 shapes.  Where it is not: 128 rows of 128 heads over 1024 keys are priced 50.0 as two splits of four groups and
+    // 52.4 as whole rows of this form, and take 57.4 and 54.3 (bf16 cache 58.3 and 50.6).  A single row's 32 splits are priced 14.5
+    // and its 22 splits 14.1, and take 13.5 and 14.2.
+    double slice_round_us(const int ns, const long long wgs) const           // (wgs of the launch: 256 and more fill the chip)
+    {
+        const int len = split_tiles(ns);
+        const double full = wgs < cus ? (double)wgs / cus : 1.0;
+        return ns == 1 ? (1.1 + 0.35 * full * full * full * full) * len : (0.59 + 0.0175 * len) * len;
+    }
+    double slice_tail_us(const long long r, const int ns) const
+    {
+        const double wgs = (double)(r * shares(2) * ns);
+        return ns == 1 ? 6.0 : 13.2 + (ns > 8 ? 0.056 * wgs - 3.5 : 0.02 * wgs + (wgs > cus ? 0.03 * (wgs - cus) : 0.0));
+    }
+    double slice_even(const int ns) const
+    {
+        const long long wgs = rows * shares(2) * ns;
+        const double n = (double)rounds(wgs);
+        return n * slice_round_us(ns, wgs) + (n - 1.0) * 7.0 + slice_tail_us(rows, ns);     // (a further round starts and ends too)
+    }
+    double slice_mixed(const int ns, const long long full, const long long rows_b) const
+    {
+        return (double)full * (slice_round_us(1, cus) + 7.0) + slice_round_us(ns, cus) + slice_tail_us(rows_b, ns);
+    }
+
+    // of up to 2048 keys
+    double of(const SfaPlan &pl) const
+    {
+        const bool slice = nq > 32 && pl.head_groups == 2;
+        if (pl.whole_slots == 0) return slice ? slice_even(pl.nsplit) : even(pl.head_groups, pl.nsplit);
+        const long long full = pl.whole_slots / (cus / 8 / shares(pl.head_groups)), rows_b = rows - 8ll * pl.whole_slots;
+        return slice ? slice_mixed(pl.nsplit, full, rows_b) : mixed(pl.head_groups, pl.nsplit, full, rows_b);
+    }
+};
+
+// The cheapest division by these prices of those whose partial results fit max_bytes (an explicit num_splits is taken as it is); with
+// keep_whole of those that split no row.
+SfaPlan sfa_divide(const PtoSfaQuantArgs *a, const SfaPrices &m, const size_t max_bytes, const bool keep_whole)
+{
+    SfaPlan pl{};
+    const long long rows = m.rows;
+    const int cus = m.cus, tiles = m.tiles, hg_max = m.max_groups();
+    const bool f32 = m.f32;
+    const int min_split = (int)((a->topk + pto::SFA_MAX_CHUNK - 1) / pto::SFA_MAX_CHUNK);
+    const bool automatic = a->num_splits == 0 && min_split == 1;
     pl.head_groups = hg_max;
-    // A split row's partial results are fp16: one more rounding, to 11 bits, and a bf16 cache's values beyond 65504 become
-    // infinite, where a whole row goes from its fp32 accumulators straight to bf16.  So the launches whose partials are fp16 are a
-    // fixed set, and a launch outside of it that the model splits all the same leaves its partials in fp32.  The set: no
-    // split shorter than four tiles, rows dealt to the XCDs whole (row t on XCD t % 8), costs in tiles -- 3 per round around whole
-    // rows, 5.5 around split ones, the merge 1 and one per hundred partial rows.  (fp32 partials cost 0.25 us per MB they are
-    // larger by; only workgroups of one head group leave them.  16 heads, whole rows against fp32 partials: 50 rows of 256 keys
-    // 18.1 us and 14.7, 150 of 1024 58.7 and 52.3, 170 of 2048 109 and 88.6 -- as fp16 partials 12.8, 50.1 and 85.7.)
-    auto half_partials = [&]() {
-        const int sh = shares(hg_max), max_split = topk_tiles / 4;
-        if (cus % 8 != 0) return max_split > 1 && rows * sh < cus;
-        const long long xcd_cus = cus / 8, xcd_rows = (rows + 7) / 8;
-        auto xcd_rounds = [&](const int s) { return (double)((xcd_rows * sh * s + xcd_cus - 1) / xcd_cus); };
-        const double whole = xcd_rounds(1) * (topk_tiles + 3.0);
-        auto merge = [&](const long long r, const int s) { return 1.0 + 0.01 * (double)r * s * sh; };
-        for (int s = 2; s <= max_split && partial_bytes(rows, s) <= max_bytes; ++s)
-            if (xcd_rounds(s) * ((topk_tiles + s - 1) / s + 5.5) + merge(rows, s) < whole) return true;
-        // full rounds of whole rows, and the rows left over in as many pieces as fill one more (below)
-        const long long per_round = xcd_cus / sh, full = per_round > 0 ? xcd_rows / per_round : 0;
-        const long long left = xcd_rows - full * per_round, rows_b = rows - 8 * full * per_round;
-        if (full < 1 || left < 1 || rows_b < 1) return false;
-        const int s = (int)(per_round / left < max_split ? per_round / left : max_split);
-        return s >= 2 && partial_bytes(rows_b, s) <= max_bytes &&
-               (double)full * (topk_tiles + 3.0) + (topk_tiles + s - 1) / s + 5.5 + merge(rows_b, s) < whole;
-    };
-    // The rows of a prefill chunk that begins less than a third of the most keys of a row into its sequence are of all lengths: more
-    // of them than a round holds stay whole and start longest first, and the launch ends evenly by itself (the last round's rows in
-    // pieces / whole: 300 rows over 300 keys 41.7 / 33.6 us, 563 over 563 84.3 / 75.3, 2000 over 2000 529 / 511; 800 over 1500, which
-    // begin 700 keys into it, 237 / 256, 1100 over 2000 404 / 415).
-    const bool ramp = a->num_splits == 0 && min_split == 1 && a->s1 > 8 && rows * shares(hg_max) > cus &&
-                      3 * (row_keys - a->s1) < (a->topk < row_keys ? a->topk : row_keys);
-    const bool f32 = a->num_splits == 0 && min_split == 1 && !half_partials();
     int ns = a->num_splits;
     double best = -1.0;
     if (ns == 0) {
         for (int hg = hg_max; hg >= 1; hg /= 2)
-            // (of the split counts with equally long splits the smallest is the one to take)
-            for (int s = min_split, len = 0; s <= (ramp ? 1 : f32 ? (hg > 1 ? 1 : tiles < 8 ? tiles : 8) : tiles); s = len > 1 ? (tiles + len - 2) / (len - 1) : tiles + 1) {
-                len = (tiles + s - 1) / s;
-                const long long wgs = rows * shares(hg) * s;
-                if (s > min_split && (partial_bytes(rows, s, f32) > max_bytes || wgs > 4ll * cus)) break;
-                const double cost = (double)rounds(wgs) * round_us(hg, s) + tail_us(hg, wgs, s) +
-                                    (f32 ? 0.25e-6 * (double)(partial_bytes(rows, s, true) - partial_bytes(rows, s)) : 0.0);
+            for (int s = min_split; s <= (keep_whole ? 1 : f32 ? (hg > 1 ? 1 : tiles < 8 ? tiles : 8) : tiles); s = m.next_splits(s)) {
+                if (s > min_split && (m.partial_bytes(rows, s, f32) > max_bytes || rows * m.shares(hg) * s > 4ll * cus)) break;
+                const double cost = m.even(hg, s);
                 if (best < 0.0 || cost < best) {
                     best = cost;
                     ns = s;
@@ -212,60 +237,41 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
     ns = ns < min_split ? min_split : ns;
     ns = ns > tiles ? tiles : ns;
     ns = ns < 1 ? 1 : ns;
-    pl.hgroups = shares(pl.head_groups);
+    pl.hgroups = m.shares(pl.head_groups);
     pl.nsplit = ns;
-    pl.whole_slots = 0;
-    long long split_rows = rows;
-    if (a->num_splits == 0 && min_split == 1 && !f32 && !ramp && cus % 8 == 0) {
+    pl.split_rows = rows;
+    if (automatic && !f32 && !keep_whole && cus % 8 == 0) {
         // More rows than compute units: the full rounds of whole rows first, then the rows left over dealt out in
         // as many pieces as fill one more round (300 rows on 256 CUs: 32 whole rows per XCD, the other five or
         // six in five pieces each), where that beats the best uniform split above.
         const long long xcd_rows = (rows + 7) / 8;
-        const long long per_round = cus / 8 / shares(hg_max);                 // rows of an XCD that one round holds
+        const long long per_round = cus / 8 / m.shares(hg_max);               // rows of an XCD that one round holds
         const long long full = per_round > 0 ? xcd_rows / per_round : 0;
         const long long rows_b = rows - 8 * full * per_round;                 // rows 8 * whole_slots and up
         if (full >= 1 && rows_b >= 1) {
-            int sb = (int)(cus / (rows_b * shares(hg_max)));
+            int sb = (int)(cus / (rows_b * m.shares(hg_max)));
             const int max_split = tiles / 4 > 0 ? tiles / 4 : 1;              // (a last round shorter than four tiles is all prologue)
             sb = sb > max_split ? max_split : sb;
-            if (sb >= 2 && partial_bytes(rows_b, sb) <= max_bytes) {
-                const double cost = (double)full * round_us(hg_max, 1) + round_us(hg_max, sb) +
-                                    tail_us(hg_max, rows_b * shares(hg_max) * sb, sb);
+            if (sb >= 2 && m.partial_bytes(rows_b, sb) <= max_bytes) {
+                const double cost = m.mixed(hg_max, sb, full, rows_b);
                 if (cost < best) {
                     best = cost;
                     pl.head_groups = hg_max;
-                    pl.hgroups = shares(hg_max);
+                    pl.hgroups = m.shares(hg_max);
                     pl.nsplit = sb;
                     pl.whole_slots = (int)(full * per_round);
-                    split_rows = rows_b;
+                    pl.split_rows = rows_b;
                 }
             }
         }
     }
     pl.part_f32 = f32 && pl.nsplit > 1;
-    pl.scratch_bytes = partial_bytes(split_rows, pl.nsplit, f32);
-    // More than 32 heads: workgroups of 64 heads (sfa_slice_kernel) where they are the faster ones, within the bytes that a caller
-    // is asked for, which stay those of the division above.  In microseconds, fitted to an int8 cache, 1 to 128 rows, top-k 2048,
-    // 128 heads (measured: 32 rows 4 splits 32.3, 16 rows 8 splits 24.2, 4 rows 13 splits 18.4, 1 row 22 splits 14.0, against
-    // 35.0, 28.6, 20.0 and 14.1 as four groups and one group of 32 heads; 36 to 64 rows alike; 128 rows 97.1 against 95.0).
-    // A tile of whole rows takes 1.13 with 128 workgroups, 1.2 with 192 and 1.45 with 256 (top-k 1024, 96 rows: 44.9, as four groups
-    // and two splits 49.4); partial results past one round's cost more (64 heads, 96 rows: 5 splits 58.8, 2 splits 51.8).
-    // Against the fastest of every form and split count, two rows and more, top-k 1024 and 2048, both caches, the choice is within
-    // 5 % in 104 of 108 shapes.  Where it is not: 128 rows of 128 heads over 1024 keys are priced 50.0 as two splits of four groups and
-    // 52.4 as whole rows of this form, and take 57.4 and 54.3 (bf16 cache 58.3 and 50.6).  A single row's 32 splits are priced 14.5
-    // and its 22 splits 14.1, and take 13.5 and 14.2.
-    if (a->nq > 32 && a->num_splits == 0 && min_split == 1) {
-        const int sh = shares(2);
+    pl.scratch_bytes = m.partial_bytes(pl.split_rows, pl.nsplit, f32);
+    // Workgroups of 64 heads where they are the faster ones, within the bytes that a caller is asked for, which stay those of
+    // the division above.
+    if (a->nq > 32 && automatic) {
+        const int sh = m.shares(2);
         if (pl.head_groups == 2) best = -1.0;             // (two groups of 32 heads: that is this form, at another price)
-        auto slice_round_us = [&](const int s, const long long wgs) {          // (of the launch: 256 and more fill the chip)
-            const int len = (tiles + s - 1) / s;
-            const double full = wgs < cus ? (double)wgs / cus : 1.0;
-            return s == 1 ? (1.1 + 0.35 * full * full * full * full) * len : (0.59 + 0.0175 * len) * len;
-        };
-        auto slice_tail_us = [&](const long long r, const int s) {
-            const double wgs = (double)(r * sh * s);
-            return s == 1 ? 6.0 : 13.2 + (s > 8 ? 0.056 * wgs - 3.5 : 0.02 * wgs + (wgs > cus ? 0.03 * (wgs - cus) : 0.0));
-        };
         auto take = [&](const double cost, const int s, const long long whole) {
             if (best >= 0.0 && cost >= best) return;
             best = cost;
@@ -274,39 +280,112 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
             pl.hgroups = sh;
             pl.whole_slots = (int)(whole / 8);
             pl.part_f32 = false;
-            split_rows = rows - whole;
+            pl.split_rows = rows - whole;
         };
-        for (int s = 1, len = 0; s <= (f32 || ramp ? 1 : tiles); s = len > 1 ? (tiles + len - 2) / (len - 1) : tiles + 1) {
-            len = (tiles + s - 1) / s;
-            if (s > 1 && (partial_bytes(rows, s) > pl.scratch_bytes || rows * sh * s > 4ll * cus)) break;
-            const double n = (double)rounds(rows * sh * s);
-            take(n * slice_round_us(s, rows * sh * s) + (n - 1.0) * 7.0 + slice_tail_us(rows, s), s, 0);    // (a further round starts and ends too)
+        for (int s = 1; s <= (f32 || keep_whole ? 1 : tiles); s = m.next_splits(s)) {
+            if (s > 1 && (m.partial_bytes(rows, s) > pl.scratch_bytes || rows * sh * s > 4ll * cus)) break;
+            take(m.slice_even(s), s, 0);
         }
         const long long per_round = cus / 8 / sh, full = per_round > 0 ? (rows + 7) / 8 / per_round : 0, rows_b = rows - 8 * full * per_round;
-        if (!f32 && !ramp && cus % 8 == 0 && full >= 1 && rows_b >= 1) {            // full rounds of whole rows, the rows left over in pieces
+        if (!f32 && !keep_whole && cus % 8 == 0 && full >= 1 && rows_b >= 1) {            // full rounds of whole rows, the rows left over in pieces
             int s = (int)(cus / (rows_b * sh));
             s = s > tiles / 4 ? tiles / 4 : s;
-            while (s >= 2 && partial_bytes(rows_b, s) > pl.scratch_bytes) --s;
-            if (s >= 2) take((double)full * (slice_round_us(1, cus) + 7.0) + slice_round_us(s, cus) + slice_tail_us(rows_b, s), s, 8 * full * per_round);
+            while (s >= 2 && m.partial_bytes(rows_b, s) > pl.scratch_bytes) --s;
+            if (s >= 2) take(m.slice_mixed(s, full, rows_b), s, 8 * full * per_round);
         }
     }
+    return pl;
+}
+
+// max_bytes: most bytes of partial results the caller can hold; the automatic choice (num_splits = 0) then takes the
+// best split count among those that fit (an explicit count is the caller's own business)
+SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
+{
+    const long long rows = a->b * a->s1;
+    const int topk_tiles = (int)((a->topk + pto::SFA_KEY_TILE - 1) / pto::SFA_KEY_TILE);
+    // (a size query on a host without a device plans for the 256 CUs of an MI355X; a launch there fails)
+    const int cus = cu_count() > 0 ? cu_count() : 256;
+    SfaPrices m = {rows, a->nq, cus, topk_tiles, false};
+    const bool automatic = a->num_splits == 0 && a->topk <= pto::SFA_MAX_CHUNK;
+    // A split row's partial results are fp16: one more rounding, to 11 bits, and a bf16 cache's values beyond 65504 become
+    // infinite, where a whole row goes from its fp32 accumulators straight to bf16.  So the launches whose partials are fp16 are a
+    // fixed set, and a launch outside of it that the model splits all the same leaves its partials in fp32.  The set: no
+    // split shorter than four tiles, rows dealt to the XCDs whole (row t on XCD t % 8), costs in tiles -- 3 per round around whole
+    // rows, 5.5 around split ones, the merge 1 and one per hundred partial rows.  (fp32 partials cost 0.25 us per MB they are
+    // larger by; only workgroups of one head group leave them.  16 heads, whole rows against fp32 partials: 50 rows of 256 keys
+    // 18.1 us and 14.7, 150 of 1024 58.7 and 52.3, 170 of 2048 109 and 88.6 -- as fp16 partials 12.8, 50.1 and 85.7.)
+    auto half_partials = [&]() {
+        const int sh = m.shares(m.max_groups()), max_split = topk_tiles / 4;
+        if (cus % 8 != 0) return max_split > 1 && rows * sh < cus;
+        const long long xcd_cus = cus / 8, xcd_rows = (rows + 7) / 8;
+        auto xcd_rounds = [&](const int s) { return (double)((xcd_rows * sh * s + xcd_cus - 1) / xcd_cus); };
+        const double whole = xcd_rounds(1) * (topk_tiles + 3.0);
+        auto merge = [&](const long long r, const int s) { return 1.0 + 0.01 * (double)r * s * sh; };
+        for (int s = 2; s <= max_split && m.partial_bytes(rows, s) <= max_bytes; ++s)
+            if (xcd_rounds(s) * ((topk_tiles + s - 1) / s + 5.5) + merge(rows, s) < whole) return true;
+        // full rounds of whole rows, and the rows left over in as many pieces as fill one more (below)
+        const long long per_round = xcd_cus / sh, full = per_round > 0 ? xcd_rows / per_round : 0;
+        const long long left = xcd_rows - full * per_round, rows_b = rows - 8 * full * per_round;
+        if (full < 1 || left < 1 || rows_b < 1) return false;
+        const int s = (int)(per_round / left < max_split ? per_round / left : max_split);
+        return s >= 2 && m.partial_bytes(rows_b, s) <= max_bytes &&
+               (double)full * (topk_tiles + 3.0) + (topk_tiles + s - 1) / s + 5.5 + merge(rows_b, s) < whole;
+    };
+    m.f32 = automatic && !half_partials();
+    SfaPlan pl = sfa_divide(a, m, max_bytes, false);
+    const size_t scratch_bytes = pl.scratch_bytes;
+    // A row has no more keys than its pages hold, whatever topk is.
+    const long long row_keys = a->max_blocknum_perbatch * a->block_size;
+    if (automatic && row_keys < a->topk) m.tiles = (int)((row_keys + pto::SFA_KEY_TILE - 1) / pto::SFA_KEY_TILE);
+    // The rows of a prefill chunk that begins less than a third of the most keys of a row into its sequence are of all lengths: more
+    // of them than a round holds stay whole and start longest first, and the launch ends evenly by itself (the last round's rows in
+    // pieces / whole: 300 rows over 300 keys 41.7 / 33.6 us, 563 over 563 84.3 / 75.3, 2000 over 2000 529 / 511; 800 over 1500, which
+    // begin 700 keys into it, 237 / 256, 1100 over 2000 404 / 415).
+    if (automatic && a->s1 > 8 && rows * m.shares(m.max_groups()) > cus && 3 * (row_keys - a->s1) < (a->topk < row_keys ? a->topk : row_keys)) {
+        pl = sfa_divide(a, m, max_bytes, true);
+    } else if (m.tiles < topk_tiles) {
+        // Priced by the keys of its pages a call may be divided another way than by topk.  It is taken with no more splits than that, and
+        // where it holds no row's partial results in fewer bits: whole rows stay whole, fp32 partial results fp32.  And it has to
+        // be cheaper by what the prices are off by: nothing among up to eight splits of one form (24 rows of 64 heads over 384 keys,
+        // 8 splits 17.2 us, 4 splits 14.7), 7 % beyond, where splits are priced too dear (2 rows of 128 heads over 896 keys, 16 splits
+        // 12.5, 10 splits, 5 % cheaper by the prices, 13.6), unless half of the splits of 32 heads would be without a key (1 row of 16
+        // heads over 896, 64 splits 12.1, 28 splits 10.7), 5 % for whole rows of 64 heads and an eighth for others (128 rows of 128 heads
+        // over 384, 2 splits 34.7, whole 24.2; 128 rows of 16 heads over 256, 2 splits 21.2, whole, 10 % cheaper by the prices, 23.9).
+        // Over 903 pairs of divisions (1 to 500 rows, 16 to 128 heads, 128 to 1792 keys, all caches) the one taken is 5.4 % faster in
+        // the mean than that of topk, and 4 % slower at worst; the cheaper one by the prices alone is 11 % slower at worst.
+        const SfaPlan by_pages = sfa_divide(a, m, max_bytes, false);
+        const double was = m.of(pl), gain = (was - m.of(by_pages)) / was;
+        const bool few = pl.nsplit <= 8;
+        bool better;
+        if (by_pages.nsplit == 1) better = gain > (few && by_pages.head_groups == 2 ? 0.05 : 0.125);
+        else if (few && by_pages.head_groups == pl.head_groups) better = gain > 0.0;
+        else better = gain > 0.07 || (by_pages.head_groups == 1 && pl.nsplit >= 2 * by_pages.nsplit);
+        if (better && by_pages.nsplit <= pl.nsplit && by_pages.whole_slots == 0 && (pl.whole_slots == 0 || by_pages.nsplit == 1) &&
+            (by_pages.nsplit == 1 || by_pages.part_f32 == pl.part_f32))
+            pl = by_pages;
+    }
+    pl.predeq_offset = (pl.scratch_bytes + 255) / 256 * 256;
+    pl.scratch_bytes = scratch_bytes;                     // (asked for whatever the width of the block table)
     pl.part_o_bytes = pl.part_ml_bytes = 0;
     if (pl.nsplit > 1) {
-        pl.part_ml_bytes = (size_t)split_rows * pl.nsplit * a->nq * 2 * sizeof(float);
-        pl.part_o_bytes = partial_bytes(split_rows, pl.nsplit, pl.part_f32) - pl.part_ml_bytes;
+        pl.part_ml_bytes = (size_t)pl.split_rows * pl.nsplit * a->nq * 2 * sizeof(float);
+        pl.part_o_bytes = m.partial_bytes(pl.split_rows, pl.nsplit, pl.part_f32) - pl.part_ml_bytes;
     }
     // A launch that selects every cache row many times over (a prefill chunk: thousands of query rows over a few
     // thousand keys) de-quantises the cache once into the workspace and attends over the bf16 rows -- the same
     // bits, since the kernel's bf16-cache form reads exactly what its int8 form converts to, without the per-tile
     // conversion (8 % at 4096 query rows over 4096 keys).  Only for caches that fit a modest workspace.
     const size_t dq = (size_t)a->kv_rows * 512 * sizeof(uint16_t);
-    pl.predeq_offset = (pl.scratch_bytes + 255) / 256 * 256;
     pl.predeq_bytes = 0;
     if (rows * a->topk >= 8 * a->kv_rows && dq <= SFA_PREDEQ_MAX_BYTES && pl.predeq_offset + dq <= max_bytes) pl.predeq_bytes = dq;
     return pl;
 }
 
-size_t sfa_ws_bytes(const SfaPlan &pl) { return pl.predeq_bytes ? pl.predeq_offset + pl.predeq_bytes : pl.scratch_bytes; }
+size_t sfa_ws_bytes(const SfaPlan &pl)
+{
+    const size_t predeq = pl.predeq_bytes ? pl.predeq_offset + pl.predeq_bytes : 0;
+    return predeq > pl.scratch_bytes ? predeq : pl.scratch_bytes;
+}
 
 constexpr int PACKED_ROW_BYTES = 656;     // 512 int8 | 64 bf16 | 4 fp32
 

@@ -205,6 +205,24 @@ def test_attention_plan_stays_within_the_bytes_a_caller_is_asked_for(nq, topk):
         assert plan["partial_element_bytes"] != 4 or plan["key_splits"] <= 8, rows
 
 
+@pytest.mark.parametrize("nq,topk,rows,keys,block", [
+    (64, 2048, [167, 168], range(1664, 2048, 128), 128), (40, 2048, [167], [1984], 64), (64, 256, [10], range(160, 256, 16), 16),
+    (128, 256, [5], range(192, 256, 16), 16), (33, 2048, [168], [1920], 64), (128, 2048, [1, 2, 5, 33, 258, 300], range(128, 2048, 128), 128),
+    (16, 1024, [3, 24, 128, 170, 258], range(128, 1024, 128), 128), (32, 2048, [4, 100, 147, 170], range(128, 2048, 128), 128)])
+def test_short_block_tables_leave_no_row_fewer_bits(nq, topk, rows, keys, block):
+    """A call whose pages hold fewer keys than topk may be divided another way than by topk: in no more splits, whole rows still
+    whole, no partial result in fewer bits, and for the same workspace."""
+    from pypto_amd import _C
+    for r in rows:
+        for n in keys:
+            args = lambda pages: (r, 1, nq, 1, topk, block, pages, 1 << 30, 0.04, 0)  # noqa: E731
+            wide, short = _C.sfa_quant_plan(*args(topk // block)), _C.sfa_quant_plan(*args(n // block))
+            assert short["key_splits"] <= wide["key_splits"], (r, n)
+            assert short["key_splits"] == 1 or short["whole_rows"] == wide["whole_rows"], (r, n)
+            assert short["key_splits"] == 1 or short["partial_element_bytes"] == wide["partial_element_bytes"], (r, n)
+            assert short["partial_bytes"] <= _C.sfa_quant_workspace_bytes(*args(n // block)) == _C.sfa_quant_workspace_bytes(*args(topk // block)), (r, n)
+
+
 @pytest.mark.parametrize("heads,splits,element,names", [
     (64, 4, 2, "sfa_slice_kernel<true> + sfa_combine_kernel<4, false>"), (128, 1, 0, "sfa_decode_kernel<4, true>"),
     (128, 7, 2, "sfa_decode_kernel<4, true> + sfa_combine_kernel<8, false>"), (32, 2, 4, "sfa_decode_kernel<1, true> + sfa_combine_kernel<2, true>"),
