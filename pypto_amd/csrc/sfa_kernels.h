@@ -31,6 +31,7 @@ struct SfaParams {
     int whole_slots;          // rows 0 .. 8 * whole_slots - 1 are not split (one workgroup per row and head group): the
                               // full rounds of a launch of more rows than compute units; 0 = every row is split alike
     int hgroups;              // workgroups' shares of the heads per query row (32 * head_groups heads each)
+    int last_first;           // T - 1 where the rows of a launch of whole rows start with the last one, else 0 (set by sfa_launch)
     int head_groups;          // groups of 32 heads per workgroup: 1, 4, or 2 (sfa_slice_kernel)
     int xcd_pieces;           // workgroups of split rows per XCD (set by sfa_launch)
     float scale_log2;         // softmax_scale * log2(e)

@@ -209,6 +209,7 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
     int t, within, nsplit;
     if (slot < wslots) {
         t = (slot / p.hgroups) * 8 + xcd;
+        if (p.last_first != 0) t = t < p.T ? p.last_first - t : p.T;
         within = slot % p.hgroups;
         nsplit = 1;
     } else {
@@ -219,9 +220,6 @@ __global__ __launch_bounds__(256) void sfa_decode_kernel(const SfaParams p)
         nsplit = p.nsplit;
     }
     if (t >= p.T) return;
-    // Rows of a prefill chunk see the more keys the later they are: the longest start first, so that the launch ends with short ones.
-    // (4096 rows over 4096 keys 1527 us, now 1496, 1000 over 1000 162.7 and 158.7, 655 over 655 94.8 and 88.3.)
-    if (p.S1 > 8 && p.nsplit == 1) t = p.T - 1 - t;
     const int hg = within / nsplit;
     const int sp = within % nsplit;
     const int b = t / p.S1;
@@ -1329,6 +1327,11 @@ hipError_t sfa_launch(const SfaParams &pa, hipStream_t stream)
 {
     SfaParams p = pa;
     if (p.nsplit == 1) p.whole_slots = (p.T + 7) / 8;
+    // Rows of a prefill chunk see the more keys the later they are: the longest start first, so that the launch ends with short ones.
+    // (4096 rows over 4096 keys 1527 us, now 1496, 1000 over 1000 162.7 and 158.7, 655 over 655 94.8 and 88.3.  Decided here: from
+    // S1 and nsplit in the kernels, two more arguments in front of the first requests, 32 decode rows took 33.0 us, now 32.8, 36 of a
+    // bf16 cache 24.1 and 23.6, 86 of 1024 keys 41.5 and 40.2.)
+    p.last_first = p.S1 > 8 && p.nsplit == 1 ? p.T - 1 : 0;
     const int split_rows = p.T > 8 * p.whole_slots ? p.T - 8 * p.whole_slots : 0;
     p.xcd_pieces = (int)(((long long)split_rows * p.hgroups * p.nsplit + 7) / 8);
     const unsigned grid = (unsigned)(8 * (p.hgroups * p.whole_slots + p.xcd_pieces));

@@ -77,6 +77,7 @@ __global__ __launch_bounds__(512) void sfa_slice_kernel(const SfaParams p)
     int t, within, nsplit;
     if (slot < wslots) {
         t = (slot / p.hgroups) * 8 + xcd;
+        if (p.last_first != 0) t = t < p.T ? p.last_first - t : p.T;
         within = slot % p.hgroups;
         nsplit = 1;
     } else {
@@ -87,7 +88,6 @@ __global__ __launch_bounds__(512) void sfa_slice_kernel(const SfaParams p)
         nsplit = p.nsplit;
     }
     if (t >= p.T) return;
-    if (p.S1 > 8 && p.nsplit == 1) t = p.T - 1 - t;        // (longest rows first)
     const int sp = within / p.hgroups;                     // the head shares of a split are neighbours: they gather the same rows
     const int hg = within - sp * p.hgroups;
     const int b = t / p.S1;
