@@ -367,13 +367,15 @@ __global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_pe
     // First cache row of every 32-key block of this wave's run, looked up once: lane i holds the row of
     // block i of the run (32 consecutive positions never straddle a page; a run has at most 64 blocks;
     // blocks past the end of the sequence repeat the last valid block).
-    int run_row;
+    int run_row, page0, pb0;                  // (and the run's first page, in the table and in the cache)
     {
         int blk = (key0 >> 5) + l;
         blk = blk > last_blk ? last_blk : blk;
         const int pos0 = 32 * blk;
         const int page = pos0 / p.bs;
         int pb = p.bt[(size_t)b * p.maxblk + page];
+        page0 = __builtin_amdgcn_readfirstlane(page);
+        pb0 = __builtin_amdgcn_readfirstlane(pb);
         pb = pb < 0 ? 0 : (pb >= p.nblocks ? p.nblocks - 1 : pb);
         run_row = pb * p.bs + (pos0 - page * p.bs);
         asm volatile("" ::"v"(run_row));      // waited for here, not behind the requests below, which the compiler does not count
@@ -411,8 +413,17 @@ __global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_pe
 #undef REQUEST_32_ROWS
     // Keys that one unit alone reads are asked for without being kept (32 sequences of 8 to 64 K keys 35.2 us, so 31.4); with
     // more units to a sequence the others find them in the caches (operator, 20 x 2 tokens of 5 to 60 K keys 35.9 us, not kept 39.7;
-    // 18 x 3 of 20 to 130 K 84.1 and 95.9).
-    const bool read_once = upb == 1;
+    // 18 x 3 of 20 to 130 K 84.1 and 95.9).  So do other sequences that begin with the same pages: up to 16 of them are asked
+    // for the run's first page, in front of the queries and looked at with them, behind the first pair's requests (operator, 32
+    // sequences, 16 / 64 / 256 common pages: not kept 45.0 / 45.8 / 42.8 us, so 43.0 / 41.3 / 36.6; no common page 44.0 either way.  Asked for
+    // beside the sequence's own page, in front of all requests, that took 44.3; the first pair kept until the answer is there 44.6).
+    constexpr int SHARERS = 16;
+    const int sharers = p.B - 1 < SHARERS ? p.B - 1 : SHARERS;
+    bool read_once = upb == 1;
+    if (read_once) {
+        const int seq = l >= sharers ? b : (b + 1 + l < p.B ? b + 1 + l : b + 1 + l - p.B);
+        dma4(p.bt + (size_t)seq * p.maxblk + page0, lds_base + (uint32_t)(SC_BUF_BYTES + SC_PAIR_BYTES));       // where pair 1 has its scales
+    }
     auto request_pair = [&](const int pr, const int buf) {
         const int rx = __builtin_amdgcn_readlane(run_row, 2 * pr), ry = __builtin_amdgcn_readlane(run_row, 2 * pr + 1);
         const uint32_t dst = lds_base + (uint32_t)(buf * SC_BUF_BYTES);
@@ -446,6 +457,8 @@ __global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_pe
             qa[s][0][ks] = *reinterpret_cast<const i32x4 *>(src + head0 * LI_DIM + (((4 * half + ks) ^ ((head0 >> 1) & 7)) << 4));
             qa[s][1][ks] = *reinterpret_cast<const i32x4 *>(src + (head0 + 16) * LI_DIM + (((4 * half + ks) ^ ((head0 >> 1) & 7)) << 4));
         }
+        if (s == 0 && read_once)
+            read_once = __ballot(l < sharers && *reinterpret_cast<const int *>(&kstage[w][1][SC_PAIR_BYTES + 4 * l]) == pb0) == 0ull;
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_waitcnt(0xC07F);                      // lgkmcnt(0): the buffer has been read
     };

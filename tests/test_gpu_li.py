@@ -288,3 +288,18 @@ def test_short_rows_are_ordered_by_buckets_or_another_way(c_oracle, variant, act
     page = inp.block_table[-1].long()[pos // 128]
     inp.idx_key_scale.reshape(-1)[page * 128 + pos % 128] = 60000.0
     assert_exact(run_op(inp), oracle(inp, c_oracle), f"{variant} k={k}")
+
+
+@pytest.mark.parametrize("b,lengths,common", [(2, (3000, 5000), 16), (20, (300, 3000), 2), (40, (1, 2600), 20)])
+def test_sequences_with_common_pages(c_oracle, b, lengths, common):
+    """Sequences that begin with the same pages, all of them or every other one: their keys are kept in the caches, other ones not."""
+    from pypto_amd.synthetic import gen_block_table
+    g = torch.Generator().manual_seed(b)
+    act = [int(x) for x in torch.randint(lengths[0], lengths[1] + 1, [b], generator=g)]
+    num, table = gen_block_table(act, 128, g, shuffle=True, max_kv=lengths[1])
+    first = table[max(range(b), key=lambda i: act[i])].clone()
+    for i in range(0, b, 1 if b < 30 else 2):
+        n = min(common, (act[i] + 127) // 128)
+        table[i, :n] = first[:n]
+    inp = gen_indexer_inputs(b, 1, act, selected_count=500, seed=b, variant="fp32", block_table=table, block_num=num)
+    assert_exact(run_op(inp), oracle(inp, c_oracle), f"b={b} common={common}")
