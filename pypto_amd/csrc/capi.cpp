@@ -766,8 +766,9 @@ int pto_li_decode_launch(const PtoLiDecodeArgs *a, void *hip_stream)
         p.round_waves = cu_count() * pto::LI_SCORE_WAVES;
         const long long need = (pairs + pto::LI_MAX_PAIRS_PER_WAVE - 1) / pto::LI_MAX_PAIRS_PER_WAVE + 2 * units;
         const long long rounds = (need + p.round_waves - 1) / p.round_waves;
-        p.unit_wgs = (int)((p.score_stride + pto::LI_SCORE_WAVES * p.ppw * 64 - 1) / (pto::LI_SCORE_WAVES * p.ppw * 64));
-        p.score_wgs = (int)(p.balanced ? rounds * cu_count() : units * p.unit_wgs);
+        const long long runs = (p.score_stride + p.ppw * 64 - 1) / (p.ppw * 64);
+        p.seq_waves = (int)(p.S1 / nt * runs);
+        p.score_wgs = (int)(p.balanced ? rounds * cu_count() : (p.B * (long long)p.seq_waves + pto::LI_SCORE_WAVES - 1) / pto::LI_SCORE_WAVES);
     }
     hipError_t e = pto::li_launch(p, static_cast<hipStream_t>(hip_stream));
     if (e != hipSuccess) return fail(PTO_E_LAUNCH, "li: launch failed: %s", hipGetErrorString(e));

@@ -32,7 +32,7 @@ struct LiParams {
     int ppw;                // 64-key block pairs per wave of the score kernel, <= LI_MAX_PAIRS_PER_WAVE
     int balanced;           // score kernel sizes its runs from the sequence lengths (LI_MAX_BALANCED_SEQS, LI_MAX_BALANCED_UNITS)
     int score_wgs;          // its launch size in workgroups
-    int unit_wgs;           // of them per unit of query tokens when not balanced
+    int seq_waves;          // waves per sequence when not balanced
     int round_waves;        // waves of one round of them, which the runs are sized for
     int nt;                 // query tokens of one sequence that a wave of the score kernel scores per key pass: 1 or 2
     int variant;            // 0: fp32 head factors applied after the ReLU; 1: fp16 scales applied before it (all tensors fp16)

@@ -335,10 +335,17 @@ __global__ __launch_bounds__(64 * LI_SCORE_WAVES) __attribute__((amdgpu_waves_pe
         unit = b * upb + of_seq - run * upb;
         key0 = run * (ppw * 64);
     } else {
-        unit = (int)blockIdx.x / p.unit_wgs;
+        // runs of a fixed length, a sequence's units side by side here too and its waves next to the next one's (every unit in workgroups
+        // of its own: 520 x 3 tokens of 1 to 4 K keys 240 us, of 3 to 4 K 252, 1200 x 4 of up to 1.5 K 409, now 157, 176 and 227; every
+        // sequence in workgroups of its own 215, 261 and 267)
         ppw = p.ppw;
-        key0 = (((int)blockIdx.x - unit * p.unit_wgs) * LI_SCORE_WAVES + w) * (ppw * 64);
-        b = unit / upb;
+        const int gw = (int)blockIdx.x * LI_SCORE_WAVES + w;
+        b = gw / p.seq_waves;
+        if (b >= p.B) return;
+        const int of_seq = gw - b * p.seq_waves;
+        const int run = of_seq / upb;
+        unit = b * upb + of_seq - run * upb;
+        key0 = run * (ppw * 64);
         cur = clamped(p.act[b]);
     }
     const int t = b * p.S1 + (unit - b * upb) * NT;               // the unit's first token

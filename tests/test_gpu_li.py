@@ -250,6 +250,7 @@ def test_row_lengths_of_the_select(c_oracle, k, act):
     (64, 1, 66000, 70000, 70016),      # more keys than a round of the longest runs holds
     (300, 3, 1, 3000, 3072),           # more units than sequences in a row of the table, one token each
     (520, 4, 1, 3000, 3072),           # more sequences than the table holds: runs of a fixed length, two tokens to a unit
+    (521, 3, 1, 5000, 5120),           # the same, one token to a unit: the last workgroup is not full
 ])
 def test_indexer_launches_of_more_than_one_round(b, s1, lo, hi, cap):
     """The rows of a batch whose runs are spread over all its sequences against the same rows scored one sequence at a time.  All
