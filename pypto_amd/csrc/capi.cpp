@@ -751,7 +751,7 @@ int pto_li_decode_launch(const PtoLiDecodeArgs *a, void *hip_stream)
         int nt = 1;
         if (p.S1 % 2 == 0 && p.variant == 0) {
             const long long pairs2 = (long long)p.B * (p.S1 / 2) * ((p.score_stride + 63) / 64);
-            if (pairs2 >= 12ll * cu_count() * 8) nt = 2;
+            if (pairs2 >= (long long)pto::LI_PAIR_MIN * cu_count() * pto::LI_SCORE_WAVES) nt = 2;
         }
         p.nt = nt;
         const long long units = (long long)p.B * (p.S1 / nt);    // token groups that share a key pass

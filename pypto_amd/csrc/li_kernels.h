@@ -11,6 +11,7 @@ constexpr int LI_HEADS = 64;
 constexpr int LI_DIM = 128;
 constexpr int LI_MAX_BALANCED_SEQS = 512;  // most sequences, and
 constexpr int LI_MAX_BALANCED_UNITS = 2048; // units of query tokens, that the balanced run mapping of the score kernel handles
+constexpr int LI_PAIR_MIN = 12;            // key pairs of 64 per resident wave from which on two query tokens share a wave's pass over the keys
 constexpr int LI_SAMPLE_GROUP = 16;        // the score kernel leaves one sampled score per this many positions
 constexpr int LI_SCORE_WAVES = 8;          // waves per workgroup of the score kernel, one workgroup to a compute unit
 constexpr int LI_MAX_PAIRS_PER_WAVE = 32;  // a wave keeps one cache-row index per 32-key block of its run in a lane

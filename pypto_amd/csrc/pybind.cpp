@@ -13,6 +13,7 @@
 #include <string>
 
 #include "pypto_amd_sfa.h"
+#include "li_kernels.h"
 #include "torch_calls.h"
 
 namespace py = pybind11;
@@ -102,6 +103,11 @@ PYBIND11_MODULE(_C, m)
     m.attr("DT_FP32") = PTO_DT_FP32;
     m.attr("DT_BF16") = PTO_DT_BF16;
     if (pto::add_torch_calls(m.ptr()) != 0) throw py::error_already_set();
+    // how the indexer's score kernel is launched, for tests of its forms
+    m.attr("LI_PAIR_MIN") = pto::LI_PAIR_MIN;
+    m.attr("LI_SCORE_WAVES") = pto::LI_SCORE_WAVES;
+    m.attr("LI_MAX_BALANCED_SEQS") = pto::LI_MAX_BALANCED_SEQS;
+    m.attr("LI_MAX_BALANCED_UNITS") = pto::LI_MAX_BALANCED_UNITS;
     m.def("version", []() { return std::string(pto_version()); });
 
     m.def("sfa_quant_workspace_bytes",

@@ -107,42 +107,65 @@ def test_long_runs_wide_block_table(c_oracle):
     assert_exact(run_op(inp), oracle(inp, c_oracle), "wide block table")
 
 
-@pytest.mark.parametrize("b,s1", [
-    (100, 1),     # balanced run mapping, rows 1.. of the token table (tokens 64 and up)
-    (40, 4),      # the same with four query tokens per sequence
-    (130, 4),     # 520 tokens: past the balanced mapping, one grid row per token
+def score_launch(b, s1, width):
+    """(query tokens per unit, whether the runs are spread over all sequences) of the score kernel's launch over a block table of
+    `width` positions: the rule of pto_li_decode_launch."""
+    from pypto_amd import _C
+    waves = torch.cuda.get_device_properties(0).multi_processor_count * _C.LI_SCORE_WAVES
+    pairs = s1 % 2 == 0 and b * (s1 // 2) * ((width + 63) // 64) >= _C.LI_PAIR_MIN * waves
+    units = b * s1 // (2 if pairs else 1)
+    return 2 if pairs else 1, b <= _C.LI_MAX_BALANCED_SEQS and units <= _C.LI_MAX_BALANCED_UNITS
+
+
+def wide_inputs(b, s1, act, width, variant, k=2048, seed=0):
+    """Inputs whose block table has `width` positions, however short the sequences are."""
+    from pypto_amd.synthetic import gen_block_table
+    num, table = gen_block_table(act, 128, torch.Generator().manual_seed(seed), max_kv=width)
+    return gen_indexer_inputs(b, s1, act, selected_count=k, seed=seed + 1, variant=variant, block_table=table, block_num=num)
+
+
+@pytest.mark.parametrize("b,s1,balanced", [
+    (100, 1, True),     # runs spread over all sequences, rows 1.. of the table of sequences (64 and up)
+    (40, 4, True),      # the same with four query tokens per sequence
+    (130, 4, True),     # 520 query tokens
+    (515, 1, False),    # more sequences than the table holds: runs of a fixed length
+    (515, 3, False),
 ])
-def test_many_query_tokens_short_sequences(c_oracle, b, s1):
-    """More query tokens than one row of the score kernel's token table holds, and more than the balanced
-    mapping takes at all; short ragged sequences so the oracle stays cheap."""
+def test_many_query_tokens_short_sequences(c_oracle, b, s1, balanced):
+    """More sequences than one row of the score kernel's table holds, and more than the whole table; short ragged sequences so
+    the oracle stays cheap."""
     g = torch.Generator().manual_seed(1000 + b)
     act = [int(x) for x in torch.randint(s1, 700, [b], generator=g)]
     act[0], act[-1] = 699, s1                      # a long first and the shortest possible last sequence
     inp = gen_indexer_inputs(b, s1, act, selected_count=128, seed=b + s1, variant="fp16")
+    assert score_launch(b, s1, inp.block_table.shape[1] * 128) == (1, balanced)
     assert_exact(run_op(inp), oracle(inp, c_oracle), f"b={b} s1={s1}")
 
 
-@pytest.mark.parametrize("variant,b,s1", [("fp32", 28, 3), ("fp16", 28, 4)])
-def test_token_pairs_share_a_key_pass(c_oracle, variant, b, s1):
-    """Enough work for the launch to score two query tokens of a sequence per key pass (the reference scores
-    all s1 tokens against a page at once, lightning_indexer_quant_impl.py:163-169): an odd s1 leaves a unit of
-    one token, s1 = 4 makes two units per sequence; ragged lengths end inside runs and pairs."""
+@pytest.mark.parametrize("variant,b,s1,width,tokens", [
+    ("fp32", 28, 3, 0, 1), ("fp16", 28, 4, 0, 1),                      # an odd number of tokens, and too few keys: units of one token
+    ("fp32", 28, 4, 28160, 2), ("fp16", 28, 4, 28160, 2), ("fp16", 30, 2, 56320, 2)])
+def test_token_pairs_share_a_key_pass(c_oracle, variant, b, s1, width, tokens):
+    """Two query tokens of a sequence per key pass (the reference scores all s1 tokens against a page at once,
+    lightning_indexer_quant_impl.py:163-169) where the block table has room for enough keys: s1 = 4 makes two units per
+    sequence; ragged lengths end inside runs and pairs."""
     g = torch.Generator().manual_seed(300 + b)
     act = [int(x) for x in torch.randint(2100, 20480, [b], generator=g)]
     act[0], act[1] = 20480, 2049
-    inp = gen_indexer_inputs(b, s1, act, selected_count=2048, seed=b * s1, variant=variant)
-    assert inp.b * ((s1 + 1) // 2) * (inp.block_table.shape[1] * 128 // 64) >= 8 * 256 * 8, "shape too small for token pairs"
+    inp = wide_inputs(b, s1, act, max(width, 20480), variant, seed=b * s1)
+    assert score_launch(b, s1, inp.block_table.shape[1] * 128) == (tokens, True)
     assert_exact(run_op(inp), oracle(inp, c_oracle), f"{variant} b={b} s1={s1}")
 
 
-@pytest.mark.parametrize("variant,b,s1", [("fp16", 28, 3), ("fp16", 2, 1), ("fp32", 2, 1)])
-def test_largest_dot_products(c_oracle, variant, b, s1):
+@pytest.mark.parametrize("variant,b,s1,width", [("fp16", 28, 3, 0), ("fp16", 2, 1, 0), ("fp32", 2, 1, 0), ("fp16", 28, 4, 28160), ("fp32", 28, 4, 28160)])
+def test_largest_dot_products(c_oracle, variant, b, s1, width):
     """Queries and keys of -128 and 127 only, with runs of one value: dot products up to +-2^21, both ends of the range in which
-    the accumulators' bits are read as floats; with fp16 scales and weights the fused head sum, for a unit of one token too."""
+    the accumulators' bits are read as floats; with fp16 scales and weights the fused head sum; units of one token and of two."""
     g = torch.Generator().manual_seed(b)
     act = [int(x) for x in torch.randint(2100, 20480, [b], generator=g)]
     act[0] = 20480
-    inp = gen_indexer_inputs(b, s1, act, selected_count=2048, seed=5 + b, variant=variant)
+    inp = wide_inputs(b, s1, act, max(width, 20480), variant, seed=5 + b)
+    assert score_launch(b, s1, inp.block_table.shape[1] * 128)[0] == (2 if width else 1)
     inp.idx_query = torch.where(inp.idx_query < 0, -128, 127).to(torch.int8)
     inp.idx_key_cache = torch.where(inp.idx_key_cache < 0, -128, 127).to(torch.int8)
     inp.idx_query[:, ::3] = -128
@@ -152,19 +175,18 @@ def test_largest_dot_products(c_oracle, variant, b, s1):
     assert_exact(run_op(inp), oracle(inp, c_oracle), f"{variant} b={b} s1={s1} extremes")
 
 
-@pytest.mark.parametrize("variant,b,s1", [("fp16", 260, 4), ("fp32", 260, 3)])
-def test_token_pairs_beyond_the_balanced_mapping(c_oracle, variant, b, s1):
-    """Token pairs per key pass in the launch shape that takes one grid row per unit: more than 512 units (260
-    sequences of two units each) with enough keys for the pair form -- the far end of the operator's documented
-    decode range (b up to 128 with s1 up to 4 and long KV, examples/models/deepseek_v32_exp/README.md:6-24, and
-    past it).  The odd s1 leaves every sequence a unit of one token."""
+@pytest.mark.parametrize("variant,b,s1,width,tokens,balanced", [
+    ("fp16", 260, 4, 2304, 1, True), ("fp32", 260, 3, 2304, 1, True), ("fp16", 260, 4, 3072, 2, True),
+    ("fp16", 516, 4, 2304, 2, False), ("fp32", 516, 2, 3328, 2, False), ("fp16", 515, 2, 3328, 2, False)])
+def test_token_pairs_beyond_the_balanced_mapping(c_oracle, variant, b, s1, width, tokens, balanced):
+    """Token pairs per key pass among hundreds of sequences, with runs spread over all of them and, beyond 512, of a fixed length --
+    past the far end of the operator's documented decode range (b up to 128 with s1 up to 4 and long KV,
+    examples/models/deepseek_v32_exp/README.md:6-24)."""
     g = torch.Generator().manual_seed(500 + s1)
     act = [int(x) for x in torch.randint(s1, 2300, [b], generator=g)]
     act[0], act[1], act[-1] = 2300, 2049, s1
-    inp = gen_indexer_inputs(b, s1, act, selected_count=2048, seed=b + s1, variant=variant)
-    units = inp.b * ((s1 + 1) // 2)
-    assert units > 512, "shape must be past the balanced mapping"
-    assert units * (inp.block_table.shape[1] * 128 // 64) >= 8 * 256 * 8, "shape too small for token pairs"
+    inp = wide_inputs(b, s1, act, width, variant, seed=b + s1)
+    assert score_launch(b, s1, inp.block_table.shape[1] * 128) == (tokens, balanced)
     assert_exact(run_op(inp), oracle(inp, c_oracle), f"{variant} b={b} s1={s1}")
 
 
