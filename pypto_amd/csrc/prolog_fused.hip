@@ -101,7 +101,13 @@ hipError_t prolog_prefill_launch(const MlapParams *pm, const LipParams *pl, hipS
     // Two heads to a workgroup of eight waves, which then reads each token once and as whole cache lines, from four tiles on (one /
     // two, on a fast card: 680 tokens 142.3 / 143.3 us per pass, 1000 185.3 / 177.2, 1300 251.1 / 238.1, 1500 273.2 / 259.1, 2112 375.6 /
     // 365.3, 4096 662.9 / 659.9; on a slow one: 1000 196.1 / 194.9, 1300 265.9 / 258.8, 1500 288.5 / 276.8, 2112 397.1 / 399.2).
-    const int hb = pm && tiles >= 4 ? 2 : 1;
+    // The MLA prolog alone, with nothing behind them in the last round, takes them where that is two thirds full or more (one / two:
+    // 1000 tokens 129.3 / 124.2, 1025 156.4 / 167.2, 1280 178.9 / 190.1, 1536 198.6 / 204.4, 1792 229.7 / 222.3, 2500 326.7 / 331.3,
+    // 2816 359.5 / 351.5, 3500 420.4 / 428.5, 4096 492.4 / 466.6).
+    const int cus = cu_count();
+    if (cus <= 0) return hipErrorNoDevice;
+    const int last_round = pm ? m.n_heads / 2 * tiles % cus : 0;
+    const int hb = pm && tiles >= 4 && (pl || last_round == 0 || 3 * last_round >= 2 * cus) ? 2 : 1;
     const int mla_wgs = pm ? m.n_heads / hb * tiles : 0;
     // The indexer's half, whose workgroups are the shorter ones, is cut into tiles of 128 tokens up to six tiles of 256 (fused prolog,
     // tiles of 256 / 128: 1000 tokens 195.9 / 187.6 us per pass, 1300 252.3 / 243.9, 1500 271.3 / 265.7, 1800 315.8 / 322.2, 4096 652.3 /

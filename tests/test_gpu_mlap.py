@@ -650,3 +650,20 @@ def test_fused_prolog_query_rows_with_two_heads_to_a_workgroup(t, n_heads, n_idx
     want = lo.indexer_prolog_ref(*lip.input_tensors())
     assert np.abs(q_int8.cpu().numpy().astype(np.int32) - want["q_int8"].astype(np.int32)).max() <= 1
     assert (np.abs(q_scale.float().cpu().numpy()[..., 0] - want["q_scale"].astype(np.float32)) > 2.5e-5).mean() <= 0.005
+
+
+@pytest.mark.parametrize("t", [769, 1000])
+def test_query_rows_alone_with_two_heads_to_a_workgroup(t):
+    """128 heads at four tiles fill a round with two heads to a workgroup; two heads alone take workgroups of one.  The same bits."""
+    import dataclasses
+    from pypto_amd import mla_prolog_quant_impl as impl
+    impl.EXACT_ABSORB = False
+    mla = gen_mla_prolog_inputs(1, t, [t + 30], seed=t, n_heads=128, h=128, q_lora_rank=512)
+    got = run_op(mla, (1e-5, 1e-5), prefill=True)
+    for head in (0, 64, 126):
+        cols = slice(192 * head, 192 * (head + 2))
+        two = dataclasses.replace(mla, w_uq_qr=mla.w_uq_qr[:, cols].contiguous(), dequant_scale=mla.dequant_scale[cols].contiguous(),
+                                  w_uk=mla.w_uk[head:head + 2].contiguous())
+        part = run_op(two, (1e-5, 1e-5), prefill=True)
+        for name in ("query_nope", "query_rope"):
+            assert np.array_equal(part[name], got[name].reshape(t, 128, -1)[:, head:head + 2].reshape(part[name].shape)), (head, name)
