@@ -313,6 +313,33 @@ def test_short_rows_are_ordered_by_buckets_or_another_way(c_oracle, variant, act
     assert_exact(run_op(inp), oracle(inp, c_oracle), f"{variant} k={k}")
 
 
+def set_key_scale(inp, seq, positions, value):
+    for pos in positions:
+        inp.idx_key_scale.reshape(-1)[int(inp.block_table[seq, pos // 128]) * 128 + pos % 128] = value
+
+
+@pytest.mark.parametrize("k,act", [(2048, [40, 1500, 2048]), (2048, [2049, 3000, 8192, 8193, 20000]), (100, [129, 1025, 5000])])
+def test_select_with_infinite_scores(c_oracle, k, act):
+    """Some scores infinite, of either sign: no range spreads the others over buckets.  Equal ones in the order of their positions."""
+    inp = gen_indexer_inputs(len(act), 1, act, selected_count=k, seed=k + len(act), variant="fp32")
+    for i, n in enumerate(act):
+        set_key_scale(inp, i, range(3, n, 37), float("inf"))
+    assert_exact(run_op(inp), oracle(inp, c_oracle), f"k={k} act={act}")
+
+
+def test_select_of_every_key_with_scores_that_are_no_numbers(c_oracle):
+    """Rows of at most k keys: those whose score is not a number come first, in the order of their positions, then the others."""
+    act, bad = [65, 500, 1500, 2048], 41
+    inp = gen_indexer_inputs(len(act), 1, act, selected_count=2048, seed=9, variant="fp32")
+    want = oracle(inp, c_oracle)
+    for i, n in enumerate(act):
+        odd = list(range(5, n, bad))
+        set_key_scale(inp, i, odd, float("nan"))
+        rest = [x for x in want[i, 0, :n].tolist() if x not in odd]
+        want[i, 0, :n] = torch.tensor(odd + rest, dtype=torch.int32)
+    assert_exact(run_op(inp), want, "not a number")
+
+
 @pytest.mark.parametrize("b,lengths,common", [(2, (3000, 5000), 16), (20, (300, 3000), 2), (40, (1, 2600), 20)])
 def test_sequences_with_common_pages(c_oracle, b, lengths, common):
     """Sequences that begin with the same pages, all of them or every other one: their keys are kept in the caches, other ones not."""
