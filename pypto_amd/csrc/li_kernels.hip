@@ -1271,13 +1271,6 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
     }
 }
 
-__global__ __launch_bounds__(SEL_THREADS) void li_select_stream_kernel(const LiParams p)
-{
-    __shared__ uint32_t hist[256];
-    __shared__ unsigned long long sortbuf[LI_MAX_SELECT];
-    select_streaming(p, (int)blockIdx.x, hist, sortbuf);
-}
-
 }  // namespace
 
 hipError_t li_launch(const LiParams &p, hipStream_t stream)

@@ -186,7 +186,7 @@ __global__ __launch_bounds__(256, 2) void mlap_xlinear_mfma_kernel(const MlapPar
     XmSlab sl;
     sl.w = isq ? reinterpret_cast<const uint8_t *>(p.w_dq) + slab * 256 : reinterpret_cast<const uint8_t *>(p.w_dkvkr) + (slab - qslabs) * 256;
     sl.pitch = (isq ? p.q_lora : MLAP_KV + MLAP_ROPE) * 2;
-    sl.pieces = !isq && slab - qslabs == 4 ? 8 : 16;
+    sl.pieces = 16;                // (the narrow one, the rope columns, is not among them)
     sl.out = p.xpart + (size_t)sp * p.T * nc + slab * 128;
     sl.out_pitch = nc;
     const int nchunks = p.h / XM_KC;
