@@ -1018,7 +1018,10 @@ __global__ __launch_bounds__(SEL_THREADS) void li_select_kernel(const LiParams p
     // is taken is sorted, and a longer one goes the way of the others.
     // (Rows of at most k keys always sorted beyond 512 keys and ordered by counting over the whole row up to there, as before,
     // two sequences of 450 keys took 24.3 us instead of 9.6, scores included, of 650 keys 18.5, of 1900 22.0 instead of 10.8.
-    // By way of a pivot, two of 2200 keys take 13.5, as here 11.2, of 4096 15.0 and 12.1, of 8100 15.1 and 13.4.)
+    // By way of a pivot, two of 2200 keys take 13.5, as here 11.2, of 4096 15.0 and 12.1, of 8100 15.1 and 13.4.  A row that has to
+    // leave pays for both ways: four of 8000 equal scores 57.3 by the pivot alone, 66.3 here, with every thousandth score 10^6 times
+    // the others 43.4 and 52.2, of 1500 keys 22.0 and 23.4.  Scores crowd like that where one lies about eighty times as far out as the
+    // others among 8000 keys, three hundred times among 2048.)
     auto sort_row = [&]() {
         int width = 64;
         while (width < n) width <<= 1;

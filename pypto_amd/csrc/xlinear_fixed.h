@@ -162,7 +162,7 @@ __device__ __forceinline__ void xl_body(const XlSlab &sl, const uint16_t *x, con
 // the clock that random operands leave.  256 columns x 4096 tokens x 7168 rows alone 162 us with the weights in LDS for one tile,
 // now 148 (112 TFLOP/s).  The multiply-add form of the vector ALU this replaced (hidden states broadcast through DPP) ran at a
 // quarter of the matrix cores' rate.
-constexpr int XF_TOK = 32;                                               // tokens per workgroup
+constexpr int XF_TOK = 32;                                               // tokens per tile; a workgroup takes a run of tiles
 constexpr int XF_COLS = 64;                                              // columns per workgroup, at most
 constexpr int XF_WAVES = 4;
 constexpr int XF_TOK_PITCH = XF_COLS * 4 + 16;                           // bytes between token rows of a block sum
