@@ -341,7 +341,13 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
     // of them than a round holds stay whole and start longest first, and the launch ends evenly by itself (the last round's rows in
     // pieces / whole: 300 rows over 300 keys 41.7 / 33.6 us, 563 over 563 84.3 / 75.3, 2000 over 2000 529 / 511; 800 over 1500, which
     // begin 700 keys into it, 237 / 256, 1100 over 2000 404 / 415).
-    if (automatic && a->s1 > 8 && rows * m.shares(m.max_groups()) > cus && 3 * (row_keys - a->s1) < (a->topk < row_keys ? a->topk : row_keys)) {
+    // Of up to 32 heads, whose rows are the shorter ones, the less of a launch the last round is the fewer keys its rows may begin at
+    // (in pieces / whole: 300 over 361 34.4 / 26.7 us, 563 over 676 62.1 / 61.5, 800 over 881 92.0 / 87.6, over 1121 122.3 / 127.4, 1100
+    // over 1321 171.5 / 176.7, 1608 over 1930 341 / 352).
+    const long long before = row_keys - a->s1, most = a->topk < row_keys ? a->topk : row_keys;
+    const bool ramp = automatic && a->s1 > 8 && rows * m.shares(m.max_groups()) > cus && 3 * before < most &&
+                      (m.max_groups() > 1 || 8 * before * rows < 5 * most * cus);
+    if (ramp) {
         pl = sfa_divide(a, m, max_bytes, true);
     } else if (m.tiles < topk_tiles) {
         // Priced by the keys of its pages a call may be divided another way than by topk.  It is taken with no more splits than that, and
