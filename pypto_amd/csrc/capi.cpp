@@ -591,7 +591,7 @@ extern "C" {
 
 const char *pto_last_error(void) { return g_err; }
 
-const char *pto_version(void) { return "0.8.2"; }
+const char *pto_version(void) { return "0.8.3"; }
 
 int pto_abi_revision(void) { return PTO_ABI_REVISION; }
 
