@@ -94,25 +94,32 @@ hipError_t prolog_prefill_launch(const MlapParams *pm, const LipParams *pl, hipS
     // Up to 64 tokens the attention query's tiles have 64 (in tiles of 128, half and more of them padding: fused prolog 33 tokens 41.4
     // us per pass, now 40.6, 48: 43.3 and 42.4, 64: 44.6 and 43.6; MLA prolog alone 33: 35.9 and 34.1, 64: 39.9 and 38.7).
     // Tiles of 256 tokens from 257 on (tiles of 128, 307 tokens 91.5 us per pass, now 85.4, 384: 99.3 and 90.7, 600: 132.4 and 131.4,
-    // 800: 165.0 and 160.5; 256 tokens the other way, 72.5 and 92.4: a tile per head leaves half of the chip's places empty).
-    const bool small = T <= 256;
-    const int tok = small ? 128 : 256;
-    const int tiles = (T + tok - 1) / tok;
-    // Two heads to a workgroup of eight waves, which then reads each token once and as whole cache lines, from four tiles on (one /
-    // two, on a fast card: 680 tokens 142.3 / 143.3 us per pass, 1000 185.3 / 177.2, 1300 251.1 / 238.1, 1500 273.2 / 259.1, 2112 375.6 /
-    // 365.3, 4096 662.9 / 659.9; on a slow one: 1000 196.1 / 194.9, 1300 265.9 / 258.8, 1500 288.5 / 276.8, 2112 397.1 / 399.2).
-    // The MLA prolog alone, with nothing behind them in the last round, takes them where that is two thirds full or more (one / two:
-    // 1000 tokens 129.3 / 124.2, 1025 156.4 / 167.2, 1280 178.9 / 190.1, 1536 198.6 / 204.4, 1792 229.7 / 222.3, 2500 326.7 / 331.3,
-    // 2816 359.5 / 351.5, 3500 420.4 / 428.5, 4096 492.4 / 466.6).
+    // 800: 165.0 and 160.5; 256 tokens the other way, 72.5 and 92.4: a tile per head leaves half of the chip's places empty) -- but where few
+    // heads make workgroups for less than three quarters of the compute units, and the indexer's do not fill their places (tiles of
+    // 256 / 128: MLA prolog alone, 16 heads, 300 tokens 63.3 / 50.9, 1000 86.2 / 76.0, 64 heads 512 76.2 / 64.6, 600 79.7 / 80.0; fused, 32
+    // and 64 heads, 400 tokens 83.2 / 73.9, 769 113.6 / 120.0, 16 and 8 heads, 1000 tokens 114.5 / 104.2).
     const int cus = cu_count();
     if (cus <= 0) return hipErrorNoDevice;
-    const int last_round = pm ? m.n_heads / 2 * tiles % cus : 0;
-    const int hb = pm && tiles >= 4 && (pl || last_round == 0 || 3 * last_round >= 2 * cus) ? 2 : 1;
+    const int tiles128 = (T + 127) / 128, tiles256 = (T + 255) / 256;
+    const int mla256 = pm ? m.n_heads * tiles256 : 0;
+    const bool small = T <= 256 || (pm && 4 * mla256 < 3 * cus && mla256 + (pl ? p.n_heads * tiles128 : 0) <= 2 * cus);
+    const int tiles = small ? tiles128 : tiles256;
+    // Two heads to a workgroup of eight waves, which then reads each token once and as whole cache lines, from four tiles and 64 heads on,
+    // where they are for six tenths of the compute units or more (one / two, on a fast card: 680 tokens 142.3 / 143.3 us per pass, 1000
+    // 185.3 / 177.2, 1300 251.1 / 238.1, 1500 273.2 / 259.1, 2112 375.6 / 365.3, 4096 662.9 / 659.9; on a slow one: 1000 196.1 / 194.9, 1300
+    // 265.9 / 258.8, 1500 288.5 / 276.8, 2112 397.1 / 399.2; 64 heads 1300 tokens 192.7 / 187.0, with 32 of the indexer 800 121.7 / 130.3; 16
+    // heads 1000 126.6 / 140.6, 4096 396.0 / 399.7; 32 heads 1000 130.1 / 143.2, 3000 331.9 / 337.2).
+    // The MLA prolog alone, with nothing behind them, takes them where their last round is six tenths full or more (one / two: 600
+    // tokens 105.0 / 101.2, 1000 129.3 / 124.2, 1025 156.4 / 167.2, 1280 178.9 / 190.1, 1536 198.6 / 204.4, 1792 229.7 / 222.3, 2500 326.7 /
+    // 331.3, 2816 359.5 / 351.5, 3500 420.4 / 428.5, 4096 492.4 / 466.6; 64 heads 1000 99.6 / 113.3, 1152 127.8 / 122.6, 2500 242 / 259).
+    const int pairs = mla256 / 2, last_round = pairs % cus;
+    const bool two = pl ? tiles >= 4 && m.n_heads >= 64 && 5 * pairs >= 3 * cus : pairs > 0 && (last_round == 0 || 5 * last_round >= 3 * cus);
+    const int hb = pm && !small && two ? 2 : 1;
     const int mla_wgs = pm ? m.n_heads / hb * tiles : 0;
-    // The indexer's half, whose workgroups are the shorter ones, is cut into tiles of 128 tokens up to six tiles of 256 (fused prolog,
-    // tiles of 256 / 128: 1000 tokens 195.9 / 187.6 us per pass, 1300 252.3 / 243.9, 1500 271.3 / 265.7, 1800 315.8 / 322.2, 4096 652.3 /
+    // The indexer's half, whose workgroups are the shorter ones, is cut into tiles of 128 tokens up to six tiles of 256 of 64 heads (fused
+    // prolog, tiles of 256 / 128: 1000 tokens 195.9 / 187.6 us per pass, 1300 252.3 / 243.9, 1500 271.3 / 265.7, 1800 315.8 / 322.2, 4096 652.3 /
     // 668.8; the indexer prolog alone 400: 45.3 / 36.4, 512: 46.2 / 37.5, 1536: 85.5 / 84.4, 2000: 107.0 / 110.3).
-    const bool lip_small = small || tiles <= 6;
+    const bool lip_small = small || (pl && 2 * p.n_heads * tiles <= 3 * cus);
     const int lip_wgs = pl ? (p.n_heads + hb - 1) / hb * (lip_small ? (T + 127) / 128 : tiles) : 0;
     const int tok_wgs = pl ? (T + 4 * hb - 1) / (4 * hb) : 0;
     const dim3 g((unsigned)(mla_wgs + lip_wgs + tok_wgs));

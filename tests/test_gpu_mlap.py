@@ -352,7 +352,7 @@ def test_fused_prolog_fixed_order_sums_at_tile_edges(t, n_idx):
 
 @pytest.mark.parametrize("t,q_lora", [(64, 512), (127, 1536), (129, 1024), (256, 512), (257, 512), (512, 512), (513, 1024), (700, 512)])
 def test_fused_prolog_query_rows_at_tile_edges(t, q_lora):
-    """The launch that makes and finishes both queries, from 64 tokens on (the Hadamard sums in the cores' order), at the edges of its tiles of 128 and 256 tokens and
+    """The launch that makes and finishes both queries, from 64 tokens on (the Hadamard sums in the cores' order), at the edges of its tiles of 128 tokens and
     of the hidden-axis launch's: every query output against the sequential statement under the reference's rule."""
     from oracle import lip_oracle as lo
     from pypto_amd import lightning_indexer_prolog_quant_impl as lip_impl
@@ -376,10 +376,10 @@ def test_fused_prolog_query_rows_at_tile_edges(t, q_lora):
 
 
 @pytest.mark.parametrize("t", [385, 511, 640, 768, 769, 1535, 1537])
-def test_indexer_query_rows_are_alike_in_tiles_of_128_and_256_tokens(t):
-    """The indexer query's tiles have 128 or 256 tokens by the number of tokens and by whether the attention query is made in the
-    same launch: the fused operator and the indexer prolog alone give the same bits at the edges of both rules, rows past the last
-    token stay as they are, and the rows meet the reference's rule."""
+def test_indexer_query_rows_are_alike_fused_and_alone(t):
+    """The indexer query's tiles have 128 or 256 tokens by the numbers of tokens and heads (few heads: 128; many are tested below): the
+    fused operator and the indexer prolog alone give the same bits, rows past the last token stay as they are, and the rows meet the
+    reference's rule."""
     from oracle import lip_oracle as lo
     from pypto_amd import lightning_indexer_prolog_quant_impl as lip_impl
     from pypto_amd import mla_prolog_quant_impl as impl
@@ -628,9 +628,9 @@ def test_fused_prolog_fixed_order_sums_of_several_tiles_per_workgroup(t, n_idx):
 
 
 @pytest.mark.parametrize("t,n_heads,n_idx", [(769, 2, 8), (1024, 4, 5), (1537, 2, 3), (1793, 6, 16)])
-def test_fused_prolog_query_rows_with_two_heads_to_a_workgroup(t, n_heads, n_idx):
-    """From four tiles of 256 tokens on a workgroup makes two heads' queries: odd numbers of indexer heads (the last one's
-    second is then not there), a last tile of one token and a full one, the indexer's tiles of 128 and 256 tokens."""
+def test_fused_prolog_query_rows_of_few_heads(t, n_heads, n_idx):
+    """Few heads at sizes that many take in tiles of 256 tokens and two to a workgroup: odd numbers of indexer heads, a last tile of one
+    token and a full one."""
     from oracle import lip_oracle as lo
     from pypto_amd import lightning_indexer_prolog_quant_impl as lip_impl
     from pypto_amd import mla_prolog_quant_impl as impl
@@ -652,18 +652,56 @@ def test_fused_prolog_query_rows_with_two_heads_to_a_workgroup(t, n_heads, n_idx
     assert (np.abs(q_scale.float().cpu().numpy()[..., 0] - want["q_scale"].astype(np.float32)) > 2.5e-5).mean() <= 0.005
 
 
-@pytest.mark.parametrize("t", [769, 1000])
-def test_query_rows_alone_with_two_heads_to_a_workgroup(t):
-    """128 heads at four tiles fill a round with two heads to a workgroup; two heads alone take workgroups of one.  The same bits."""
+def head_rows(mla, head):
+    """query_nope and query_rope of heads head and head + 1 made by themselves, in tiles of 128 tokens and a head to a workgroup, and
+    the query latent with its scale."""
     import dataclasses
+    cols = slice(192 * head, 192 * (head + 2))
+    two = dataclasses.replace(mla, w_uq_qr=mla.w_uq_qr[:, cols].contiguous(), dequant_scale=mla.dequant_scale[cols].contiguous(),
+                              w_uk=mla.w_uk[head:head + 2].contiguous())
+    return run_op(two, (1e-5, 1e-5), prefill=True)
+
+
+@pytest.mark.parametrize("t,n_heads", [(257, 128), (600, 128), (769, 128), (1000, 128), (1281, 64)])
+def test_query_rows_of_many_heads_alone(t, n_heads):
+    """Many heads take tiles of 256 tokens and, where their last round is full enough, two to a workgroup; two heads alone do not.
+    The same bits."""
     from pypto_amd import mla_prolog_quant_impl as impl
     impl.EXACT_ABSORB = False
-    mla = gen_mla_prolog_inputs(1, t, [t + 30], seed=t, n_heads=128, h=128, q_lora_rank=512)
+    mla = gen_mla_prolog_inputs(1, t, [t + 30], seed=t, n_heads=n_heads, h=128, q_lora_rank=512)
     got = run_op(mla, (1e-5, 1e-5), prefill=True)
-    for head in (0, 64, 126):
-        cols = slice(192 * head, 192 * (head + 2))
-        two = dataclasses.replace(mla, w_uq_qr=mla.w_uq_qr[:, cols].contiguous(), dequant_scale=mla.dequant_scale[cols].contiguous(),
-                                  w_uk=mla.w_uk[head:head + 2].contiguous())
-        part = run_op(two, (1e-5, 1e-5), prefill=True)
+    for head in (0, n_heads // 2, n_heads - 2):
+        part = head_rows(mla, head)
         for name in ("query_nope", "query_rope"):
-            assert np.array_equal(part[name], got[name].reshape(t, 128, -1)[:, head:head + 2].reshape(part[name].shape)), (head, name)
+            assert np.array_equal(part[name], got[name].reshape(t, n_heads, -1)[:, head:head + 2].reshape(part[name].shape)), (head, name)
+
+
+@pytest.mark.parametrize("t,n_heads,n_idx", [(257, 128, 5), (512, 128, 8), (1025, 128, 3), (1281, 64, 5), (1793, 64, 64), (1793, 32, 64), (700, 16, 64)])
+def test_fused_query_rows_of_many_heads(t, n_heads, n_idx):
+    """The same in the fused operator, the indexer's queries too: tiles of 256 tokens, pairs of heads (an odd number of the indexer's,
+    whose last one's second is then not there) and the indexer's tiles of 128 and 256 tokens; and few heads beside many of the
+    indexer's.  The rows are those of two heads, and of up to eight of the indexer's, made by themselves."""
+    from pypto_amd import lightning_indexer_prolog_quant_impl as lip_impl
+    from pypto_amd import mla_prolog_quant_impl as impl
+    from pypto_amd.synthetic import gen_indexer_prolog_inputs
+    impl.EXACT_ABSORB = lip_impl.EXACT_SUMS = False
+    kw, dev = dict(h=128, q_lora_rank=512), torch.device("cuda:0")
+    mla = gen_mla_prolog_inputs(1, t, [t + 30], seed=t, n_heads=n_heads, **kw)
+    lip = gen_indexer_prolog_inputs(1, t, [t + 30], seed=t + 1, n_heads=n_idx, **kw)
+    dm, dl = mla.to(dev), lip.to(dev)
+    q_nope, q_rope, q_int8, q_scale, _ = run_fused(dm, dl, t, n_heads, n_idx, op=pypto_amd.mla_indexer_prolog_quant_p)
+    for head in (0, n_heads - 2):
+        part = head_rows(mla, head)
+        assert np.array_equal(part["query_nope"], q_nope[:, head:head + 2].float().cpu().numpy()), head
+        assert np.array_equal(part["query_rope"], q_rope[:, head:head + 2].float().cpu().numpy()), head
+    first = max(0, n_idx - 8)
+    n = n_idx - first
+    i8 = torch.zeros([t, n, 128], dtype=torch.int8, device=dev)
+    sc = torch.zeros([t, n, 1], dtype=torch.float16, device=dev)
+    pypto_amd.lightning_indexer_prolog_quant(
+        dm.token_x, torch.from_numpy(part["q_norm"]).to(dev), torch.from_numpy(part["q_norm_scale"]).reshape(-1, 1).to(dev),
+        dl.w_qb[:, first * 128:].contiguous(), dl.w_qb_scale[first * 128:].contiguous(), dl.wk, dl.w_proj[:, first:].contiguous(),
+        dl.ln_gamma_k, dl.ln_beta_k, dm.cos, dm.sin, dl.hadamard_q, dl.hadamard_k, dl.k_cache, dl.k_cache_scale, dm.cache_index, i8, sc,
+        dl.k_cache, dl.k_cache_scale, torch.zeros([t, n], dtype=torch.float16, device=dev))
+    torch.cuda.synchronize()
+    assert torch.equal(i8, q_int8[:, first:]) and torch.equal(sc, q_scale[:, first:])
