@@ -345,7 +345,8 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
     // (in pieces / whole: 300 over 361 34.4 / 26.7 us, 563 over 676 62.1 / 61.5, 800 over 881 92.0 / 87.6, over 1121 122.3 / 127.4, 1100
     // over 1321 171.5 / 176.7, 1608 over 1930 341 / 352).
     const long long before = row_keys - a->s1, most = a->topk < row_keys ? a->topk : row_keys;
-    const bool ramp = automatic && a->s1 > 8 && rows * m.shares(m.max_groups()) > cus && 3 * before < most &&
+    const bool ramp = automatic && pto::sfa_last_first(a->b, a->s1, a->nq, a->topk, row_keys, cus) &&
+                      rows * m.shares(m.max_groups()) > cus && 3 * before < most &&
                       (m.max_groups() > 1 || 8 * before * rows < 5 * most * cus);
     if (ramp) {
         pl = sfa_divide(a, m, max_bytes, true);

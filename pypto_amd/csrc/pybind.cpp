@@ -14,6 +14,7 @@
 
 #include "pypto_amd_sfa.h"
 #include "li_kernels.h"
+#include "sfa_kernels.h"
 #include "torch_calls.h"
 
 namespace py = pybind11;
@@ -119,6 +120,7 @@ PYBIND11_MODULE(_C, m)
               check(pto_sfa_quant_workspace_bytes(&a, &bytes));
               return bytes;
           });
+    m.def("sfa_last_first", &pto::sfa_last_first);
     m.def("sfa_quant_plan",
           [](int64_t b, int64_t s1, int64_t nq, int64_t n_kv, int64_t topk, int64_t block_size,
              int64_t max_blocknum_perbatch, int64_t kv_rows, double softmax_scale, int num_splits) {

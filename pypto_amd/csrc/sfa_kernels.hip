@@ -1327,11 +1327,11 @@ hipError_t sfa_launch(const SfaParams &pa, hipStream_t stream)
 {
     SfaParams p = pa;
     if (p.nsplit == 1) p.whole_slots = (p.T + 7) / 8;
-    // Rows of a prefill chunk see the more keys the later they are: the longest start first, so that the launch ends with short ones.
-    // (4096 rows over 4096 keys 1527 us, now 1496, 1000 over 1000 162.7 and 158.7, 655 over 655 94.8 and 88.3.  Decided here: from
-    // S1 and nsplit in the kernels, two more arguments in front of the first requests, 32 decode rows took 33.0 us, now 32.8, 36 of a
-    // bf16 cache 24.1 and 23.6, 86 of 1024 keys 41.5 and 40.2.)
-    p.last_first = p.S1 > 8 && p.nsplit == 1 ? p.T - 1 : 0;
+    // (Decided by the host: from S1 and nsplit in the kernels, two more arguments in front of the first requests, 32 decode rows took
+    // 33.0 us, now 32.8, 36 of a bf16 cache 24.1 and 23.6, 86 of 1024 keys 41.5 and 40.2.)
+    const int cus = cu_count();
+    if (cus <= 0) return hipErrorNoDevice;
+    p.last_first = p.nsplit == 1 && sfa_last_first(p.T / p.S1, p.S1, p.NQ, p.topk, (long long)p.maxblk * p.bs, cus) ? p.T - 1 : 0;
     const int split_rows = p.T > 8 * p.whole_slots ? p.T - 8 * p.whole_slots : 0;
     p.xcd_pieces = (int)(((long long)split_rows * p.hgroups * p.nsplit + 7) / 8);
     const unsigned grid = (unsigned)(8 * (p.hgroups * p.whole_slots + p.xcd_pieces));

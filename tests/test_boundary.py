@@ -223,6 +223,18 @@ def test_short_block_tables_leave_no_row_fewer_bits(nq, topk, rows, keys, block)
             assert short["partial_bytes"] <= _C.sfa_quant_workspace_bytes(*args(n // block)) == _C.sfa_quant_workspace_bytes(*args(topk // block)), (r, n)
 
 
+@pytest.mark.parametrize("b,s1,nq,topk,keys,last", [
+    (1, 8, 128, 2048, 2048, False), (1, 9, 128, 2048, 2048, True), (32, 1, 128, 2048, 65536, False),        # decoding rows; a chunk
+    (1, 4096, 128, 2048, 4096, True), (1, 1000, 64, 1024, 1024, True), (1, 300, 64, 512, 384, True),        # most rows still growing
+    (1, 2000, 128, 512, 2048, False), (1, 1219, 64, 256, 1280, False), (1, 1219, 64, 1024, 1664, False),    # most rows of full length
+    (1, 1219, 32, 256, 1280, True), (64, 16, 32, 512, 384, True),                                           # short rows of one group of heads
+    (8, 128, 64, 2048, 128, False), (2, 300, 64, 2048, 384, True), (5, 2000, 128, 2048, 2048, True)])       # several sequences
+def test_rows_that_a_launch_of_whole_rows_starts_with(b, s1, nq, topk, keys, last):
+    """Longest first where the launch then ends with short rows, and not where rows of full length would start together."""
+    from pypto_amd import _C
+    assert _C.sfa_last_first(b, s1, nq, topk, keys, 256) == last
+
+
 @pytest.mark.parametrize("heads,splits,element,names", [
     (64, 4, 2, "sfa_slice_kernel<true> + sfa_combine_kernel<4, false>"), (128, 1, 0, "sfa_decode_kernel<4, true>"),
     (128, 7, 2, "sfa_decode_kernel<4, true> + sfa_combine_kernel<8, false>"), (32, 2, 4, "sfa_decode_kernel<1, true> + sfa_combine_kernel<2, true>"),
