@@ -338,16 +338,26 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
     const long long row_keys = a->max_blocknum_perbatch * a->block_size;
     if (automatic && row_keys < a->topk) m.tiles = (int)((row_keys + pto::SFA_KEY_TILE - 1) / pto::SFA_KEY_TILE);
     // The rows of a prefill chunk that begins less than a third of the most keys of a row into its sequence are of all lengths: more
-    // of them than a round holds stay whole and start longest first, and the launch ends evenly by itself (the last round's rows in
-    // pieces / whole: 300 rows over 300 keys 41.7 / 33.6 us, 563 over 563 84.3 / 75.3, 2000 over 2000 529 / 511; 800 over 1500, which
+    // of them than a round holds may stay whole and start longest first (sfa_last_first), and the launch ends evenly by itself (the
+    // last round's rows in pieces / whole: 300 rows over 300 keys 41.7 / 33.6 us, 563 over 563 84.3 / 75.3; 800 over 1500, which
     // begin 700 keys into it, 237 / 256, 1100 over 2000 404 / 415).
+    // The more rounds there are, the less the last one costs, and in pieces it costs the less the fewer its rows are.  Behind the first
+    // round it has to be for 5/64 of a round per round before it, or 1/32 where most rows grow from short to long (128 heads, in pieces
+    // / whole: top-k 2048, 530 over 562 72.8 / 64.7, 800 over 800 114.9 / 104.9, 518 over 646 74.9 / 77.8, 1030 over 1094 178.1 / 183.8;
+    // top-k 512, 600 over 632 80.4 / 73.3, 518 over 582 63.4 / 67.5, 780 over 844 96.2 / 107.3, 1300 over 1300 189.0 / 211.9; 64 heads,
+    // top-k 1024, 2060 over 2260 276 / 297).  Over 438 such chunks (64 and 128 heads, top-k 512 to 2048, 262 to 4200 rows) the launch taken
+    // is 3.9 % faster than in pieces in the mean and 0.4 % slower at worst.
     // Of up to 32 heads, whose rows are the shorter ones, the less of a launch the last round is the fewer keys its rows may begin at
     // (in pieces / whole: 300 over 361 34.4 / 26.7 us, 563 over 676 62.1 / 61.5, 800 over 881 92.0 / 87.6, over 1121 122.3 / 127.4, 1100
     // over 1321 171.5 / 176.7, 1608 over 1930 341 / 352).
     const long long before = row_keys - a->s1, most = a->topk < row_keys ? a->topk : row_keys;
-    const bool ramp = automatic && pto::sfa_last_first(a->b, a->s1, a->nq, a->topk, row_keys, cus) &&
-                      rows * m.shares(m.max_groups()) > cus && 3 * before < most &&
-                      (m.max_groups() > 1 || 8 * before * rows < 5 * most * cus);
+    const long long wgs = rows * m.shares(m.max_groups()), round = wgs / cus, left = wgs % cus;
+    auto worth = [&]() {
+        if (m.max_groups() == 1) return 8 * before * rows < 5 * most * cus;
+        return round == 1 || 64 * left > 5 * round * cus ||
+               (32 * left > round * cus && 4 * before < most && 5 * pto::sfa_full_rows(a->s1, a->topk, row_keys) < a->s1);
+    };
+    const bool ramp = automatic && wgs > cus && 3 * before < most && pto::sfa_last_first(a->b, a->s1, a->nq, a->topk, row_keys, cus) && worth();
     if (ramp) {
         pl = sfa_divide(a, m, max_bytes, true);
     } else if (m.tiles < topk_tiles) {

@@ -235,6 +235,16 @@ def test_rows_that_a_launch_of_whole_rows_starts_with(b, s1, nq, topk, keys, las
     assert _C.sfa_last_first(b, s1, nq, topk, keys, 256) == last
 
 
+@pytest.mark.parametrize("s1,nq,topk,pages,whole", [
+    (300, 128, 2048, 3, True), (530, 64, 2048, 5, True), (800, 128, 2048, 7, True), (600, 64, 512, 5, True), (300, 16, 2048, 3, True),
+    (518, 128, 512, 5, False), (518, 64, 2048, 6, False), (780, 128, 512, 7, False), (1030, 64, 512, 9, False), (2060, 64, 1024, 18, False)])
+def test_chunks_whose_rows_stay_whole(s1, nq, topk, pages, whole):
+    """Rows of all lengths stay whole, unless what is left for a last round is little beside the rounds before it."""
+    from pypto_amd import _C
+    plan = _C.sfa_quant_plan(1, s1, nq, 1, topk, 128, pages, 1 << 14, 0.04, 0)
+    assert (plan["key_splits"] == 1) == whole, plan
+
+
 @pytest.mark.parametrize("heads,splits,element,names", [
     (64, 4, 2, "sfa_slice_kernel<true> + sfa_combine_kernel<4, false>"), (128, 1, 0, "sfa_decode_kernel<4, true>"),
     (128, 7, 2, "sfa_decode_kernel<4, true> + sfa_combine_kernel<8, false>"), (32, 2, 4, "sfa_decode_kernel<1, true> + sfa_combine_kernel<2, true>"),
