@@ -361,23 +361,30 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
     if (ramp) {
         pl = sfa_divide(a, m, max_bytes, true);
     } else if (m.tiles < topk_tiles) {
-        // Priced by the keys of its pages a call may be divided another way than by topk.  It is taken with no more splits than that, and
-        // where it holds no row's partial results in fewer bits: whole rows stay whole, fp32 partial results fp32.  And it has to
+        // Priced by the keys of its pages a call may be divided another way than by topk.  It is taken where it holds no row's
+        // partial results in fewer bits: whole rows stay whole, fp32 partial results fp32.  And it has to
         // be cheaper by what the prices are off by: nothing among up to eight splits of one form (24 rows of 64 heads over 384 keys,
         // 8 splits 17.2 us, 4 splits 14.7), 7 % beyond, where splits are priced too dear (2 rows of 128 heads over 896 keys, 16 splits
         // 12.5, 10 splits, 5 % cheaper by the prices, 13.6), unless half of the splits of 32 heads would be without a key (1 row of 16
         // heads over 896, 64 splits 12.1, 28 splits 10.7), 5 % for whole rows of 64 heads and an eighth for others (128 rows of 128 heads
         // over 384, 2 splits 34.7, whole 24.2; 128 rows of 16 heads over 256, 2 splits 21.2, whole, 10 % cheaper by the prices, 23.9).
+        // More splits have to fit the bytes asked for and to be cheaper at all where the wide merge runs either way, by 1.5 % where only they
+        // need it (64 heads: 5 rows over 768 keys, top-k 1024, 11 splits 14.2, 12 splits 13.4, 6 over 1792, top-k 2048, 13 splits 16.4, 14
+        // splits 15.9; 12 rows over 1920, 8 splits 20.8, 10 splits, 1.8 % cheaper by the prices, 20.7, over 1408, 9 splits, 0.7 %, 18.7
+        // and 19.0).
         // Over 903 pairs of divisions (1 to 500 rows, 16 to 128 heads, 128 to 1792 keys, all caches) the one taken is 5.4 % faster in
         // the mean than that of topk, and 4 % slower at worst; the cheaper one by the prices alone is 11 % slower at worst.
         const SfaPlan by_pages = sfa_divide(a, m, max_bytes, false);
         const double was = m.of(pl), gain = (was - m.of(by_pages)) / was;
         const bool few = pl.nsplit <= 8;
         bool better;
-        if (by_pages.nsplit == 1) better = gain > (few && by_pages.head_groups == 2 ? 0.05 : 0.125);
+        if (by_pages.nsplit > pl.nsplit)
+            better = pl.nsplit > 1 && gain > (few ? 0.015 : 0.0) &&
+                     m.partial_bytes(by_pages.split_rows, by_pages.nsplit, by_pages.part_f32) <= scratch_bytes;
+        else if (by_pages.nsplit == 1) better = gain > (few && by_pages.head_groups == 2 ? 0.05 : 0.125);
         else if (few && by_pages.head_groups == pl.head_groups) better = gain > 0.0;
         else better = gain > 0.07 || (by_pages.head_groups == 1 && pl.nsplit >= 2 * by_pages.nsplit);
-        if (better && by_pages.nsplit <= pl.nsplit && by_pages.whole_slots == 0 && (pl.whole_slots == 0 || by_pages.nsplit == 1) &&
+        if (better && by_pages.whole_slots == 0 && (pl.whole_slots == 0 || by_pages.nsplit == 1) &&
             (by_pages.nsplit == 1 || by_pages.part_f32 == pl.part_f32))
             pl = by_pages;
     }

@@ -210,7 +210,7 @@ def test_attention_plan_stays_within_the_bytes_a_caller_is_asked_for(nq, topk):
     (128, 256, [5], range(192, 256, 16), 16), (33, 2048, [168], [1920], 64), (128, 2048, [1, 2, 5, 33, 258, 300], range(128, 2048, 128), 128),
     (16, 1024, [3, 24, 128, 170, 258], range(128, 1024, 128), 128), (32, 2048, [4, 100, 147, 170], range(128, 2048, 128), 128)])
 def test_short_block_tables_leave_no_row_fewer_bits(nq, topk, rows, keys, block):
-    """A call whose pages hold fewer keys than topk may be divided another way than by topk: in no more splits, whole rows still
+    """A call whose pages hold fewer keys than topk may be divided another way than by topk: here in no more splits, whole rows still
     whole, no partial result in fewer bits, and for the same workspace."""
     from pypto_amd import _C
     for r in rows:
@@ -233,6 +233,16 @@ def test_rows_that_a_launch_of_whole_rows_starts_with(b, s1, nq, topk, keys, las
     """Longest first where the launch then ends with short rows, and not where rows of full length would start together."""
     from pypto_amd import _C
     assert _C.sfa_last_first(b, s1, nq, topk, keys, 256) == last
+
+
+@pytest.mark.parametrize("rows,nq,topk,pages,splits", [(5, 64, 1024, 6, 12), (6, 48, 2048, 14, 14), (3, 128, 2048, 14, 14), (6, 128, 2048, 15, 10), (12, 64, 2048, 11, 8)])
+def test_short_block_tables_in_more_splits(rows, nq, topk, pages, splits):
+    """More splits than by topk, where their price says so by enough, within the workspace that is asked for whatever the table."""
+    from pypto_amd import _C
+    args = lambda pages: (rows, 1, nq, 1, topk, 128, pages, 1 << 30, 0.04, 0)  # noqa: E731
+    wide, short = _C.sfa_quant_plan(*args(topk // 128)), _C.sfa_quant_plan(*args(pages))
+    assert short["key_splits"] == splits >= wide["key_splits"] and short["partial_element_bytes"] == wide["partial_element_bytes"]
+    assert short["partial_bytes"] <= _C.sfa_quant_workspace_bytes(*args(pages)) == _C.sfa_quant_workspace_bytes(*args(topk // 128))
 
 
 @pytest.mark.parametrize("s1,nq,topk,pages,whole", [
