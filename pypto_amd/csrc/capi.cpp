@@ -345,8 +345,9 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
     // round it has to be for 5/64 of a round per round before it, or 1/32 where most rows grow from short to long (128 heads, in pieces
     // / whole: top-k 2048, 530 over 562 72.8 / 64.7, 800 over 800 114.9 / 104.9, 518 over 646 74.9 / 77.8, 1030 over 1094 178.1 / 183.8;
     // top-k 512, 600 over 632 80.4 / 73.3, 518 over 582 63.4 / 67.5, 780 over 844 96.2 / 107.3, 1300 over 1300 189.0 / 211.9; 64 heads,
-    // top-k 1024, 2060 over 2260 276 / 297).  Over 438 such chunks (64 and 128 heads, top-k 512 to 2048, 262 to 4200 rows) the launch taken
-    // is 3.9 % faster than in pieces in the mean and 0.4 % slower at worst.
+    // top-k 1024, 2060 over 2260 276 / 297).  From five rounds of up to 2048 keys on it is the order that counts (128 heads, 2060 over
+    // 2060 555 / 545, 4100 over 4100 1552 / 1514).  Over 438 such chunks (64 and 128 heads, top-k 512 to 2048, 262 to 4200 rows) the
+    // launch taken is 3.9 % faster than in pieces in the mean and 2.1 % slower at worst (3120 over 3120 1036 / 1058).
     // Of up to 32 heads, whose rows are the shorter ones, the less of a launch the last round is the fewer keys its rows may begin at
     // (in pieces / whole: 300 over 361 34.4 / 26.7 us, 563 over 676 62.1 / 61.5, 800 over 881 92.0 / 87.6, over 1121 122.3 / 127.4, 1100
     // over 1321 171.5 / 176.7, 1608 over 1930 341 / 352).
@@ -354,7 +355,7 @@ SfaPlan sfa_plan(const PtoSfaQuantArgs *a, const size_t max_bytes = ~(size_t)0)
     const long long wgs = rows * m.shares(m.max_groups()), round = wgs / cus, left = wgs % cus;
     auto worth = [&]() {
         if (m.max_groups() == 1) return 8 * before * rows < 5 * most * cus;
-        return round == 1 || 64 * left > 5 * round * cus ||
+        return round == 1 || 64 * left > 5 * round * cus || (a->topk >= pto::SFA_MAX_CHUNK && round >= 5 && 5 * before < most) ||
                (32 * left > round * cus && 4 * before < most && 5 * pto::sfa_full_rows(a->s1, a->topk, row_keys) < a->s1);
     };
     const bool ramp = automatic && wgs > cus && 3 * before < most && pto::sfa_last_first(a->b, a->s1, a->nq, a->topk, row_keys, cus) && worth();

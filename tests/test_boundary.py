@@ -246,7 +246,7 @@ def test_short_block_tables_in_more_splits(rows, nq, topk, pages, splits):
 
 
 @pytest.mark.parametrize("s1,nq,topk,pages,whole", [
-    (300, 128, 2048, 3, True), (530, 64, 2048, 5, True), (800, 128, 2048, 7, True), (600, 64, 512, 5, True), (300, 16, 2048, 3, True),
+    (300, 128, 2048, 3, True), (530, 64, 2048, 5, True), (800, 128, 2048, 7, True), (600, 64, 512, 5, True), (300, 16, 2048, 3, True), (2338, 128, 2048, 20, True),
     (518, 128, 512, 5, False), (518, 64, 2048, 6, False), (780, 128, 512, 7, False), (1030, 64, 512, 9, False), (2060, 64, 1024, 18, False)])
 def test_chunks_whose_rows_stay_whole(s1, nq, topk, pages, whole):
     """Rows of all lengths stay whole, unless what is left for a last round is little beside the rounds before it."""
